@@ -1,0 +1,511 @@
+// Copies between host arrays and the resident device buffers: what the harness functions (run_kernel1/2, run_parallel,
+// run_fuse) and bfuse_upload / bfuse_download move.  The reference copies every tensor with a cudaMemcpy of pageable
+// memory (test-utils/test-suite-files/operation_cu.py:164-256).
+//
+// What bounds such a copy on this machine is the host, not the link: hipMemcpy of pageable memory reaches 18-30 GB/s
+// (10 GB/s into memory that was never touched, one thread taking every page fault) where the link takes 57 GB/s one way
+// and 96 GB/s both ways, and its small copies cost 12-60 us each.  So
+//   * a few hundred KB (kSmallBytes: where one thread's memcpy starts to show against a pipeline's start-up) are packed
+//     into a pinned arena by the calling thread and moved by ONE kernel launch over all tensors of the call
+//     (one launch, ~3 us of GPU time + the bytes, whatever the number of tensors);
+//   * anything larger goes through a ring of pinned slots: worker threads fill (or drain) slots while copy kernels move
+//     the ones that are ready, alternating between two streams so that one starts under the other's end (1 MiB chunks:
+//     56 GB/s; one stream 44, a copy engine 38);
+//   * host memory that came from host_buffer() is pinned and copied in place, with no slot and no thread in between.
+// run_fuse over 0.3 MB: 111 -> 56 us; run_parallel over 600 MB: 36 -> 10.4 ms (the link's floor: 6.4 up + what of the 4.4
+// down is not under it).  up() returns with the copied bytes on their way into place before anything launched later;
+// down_begin / down_finish leave the wait to the caller's own synchronisation.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <immintrin.h>
+#include <sched.h>
+
+#include <algorithm>
+#include <atomic>
+#include <chrono>
+#include <condition_variable>
+#include <cstdint>
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+namespace bfuse {
+
+struct CopySeg {
+    void* dev;
+    void* host;
+    size_t bytes;
+};
+
+constexpr int kMaxSegs = 2 * 4 + 1;   // two operands (or one result and the give-up counters) of every side
+
+struct SegList {
+    struct {
+        const unsigned char* src;
+        unsigned char* dst;
+        size_t bytes;
+    } s[kMaxSegs];
+    int n;
+};
+
+// All segments of one small transfer, device memory <-> pinned host memory, by one launch: consecutive lanes move
+// consecutive 16-byte words (one PCIe request per 64 bytes and more), every block strides over every segment.
+static __global__ __launch_bounds__(256) void copy_segments(SegList l)
+{
+    const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x, nt = (size_t)gridDim.x * 256;
+    for (int k = 0; k < l.n; ++k) {
+        const unsigned char* const src = l.s[k].src;
+        unsigned char* const dst = l.s[k].dst;
+        const size_t bytes = l.s[k].bytes;
+        const bool aligned = (((uintptr_t)src | (uintptr_t)dst) & 15) == 0;
+        const size_t words = aligned ? bytes / 16 : 0;
+        for (size_t i = t; i < words; i += nt) reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
+        for (size_t i = words * 16 + t; i < bytes; i += nt) dst[i] = src[i];
+    }
+}
+
+class HostCopy {
+public:
+    static constexpr size_t kSmallBytes = 512 << 10;
+    static constexpr size_t kArenaBytes = 2 << 20;          // per direction
+    static constexpr size_t kChunk = 2 << 20;               // a slot, at most one copy: 37 us of link time, long against a copy's start
+    static constexpr size_t kPiece = 256 << 10;             // what a thread moves at a time
+    static constexpr int kSlots = 8;                        // 16 MiB
+    static constexpr int kMaxWorkers = 6;                   // six threads copy 98 GB/s into pinned memory, four 76, one 31
+    static constexpr size_t kIdleLimit = 1ull << 30;        // pinned result buffers kept for the next result
+    static constexpr size_t kTotalLimit = 4ull << 30;       // pinned result buffers in existence
+
+    static HostCopy& get()
+    {
+        static HostCopy* h = new HostCopy;   // never destroyed: results may outlive every static of the program
+        return *h;
+    }
+
+    // Host -> device.  `busy`: something launched earlier may still be running (on any stream).
+    hipError_t up(const CopySeg* seg, int n, bool busy)
+    {
+        std::lock_guard<std::mutex> lock(call_);
+        hipError_t e = open();
+        if (e != hipSuccess) return e;
+        size_t total = 0;
+        for (int i = 0; i < n; ++i) total += seg[i].bytes;
+        if (total == 0) return hipSuccess;
+        if (total <= kSmallBytes) return up_small(seg, n, total);
+        if (busy && (e = hipDeviceSynchronize()) != hipSuccess) return e;   // the copy streams are ordered with no other
+        return pipeline(seg, n, true);
+    }
+
+    // Device -> host, in two steps around the caller's device synchronisation: begin() enqueues what can run behind the
+    // launches on `stream` (small results into the arena, results in pinned buffers in place), finish() puts the rest
+    // where it belongs.
+    struct Down {
+        CopySeg packed[kMaxSegs];     // arena -> host after the synchronisation (dev = where it lies in the arena)
+        CopySeg later[kMaxSegs];      // through the ring after the synchronisation
+        int n_packed = 0, n_later = 0;
+    };
+    hipError_t down_begin(const CopySeg* seg, int n, hipStream_t stream, Down& d)
+    {
+        std::lock_guard<std::mutex> lock(call_);
+        hipError_t e = open();
+        if (e != hipSuccess) return e;
+        size_t total = 0;
+        for (int i = 0; i < n; ++i) total += seg[i].bytes;
+        SegList l{};
+        for (int i = 0; i < n; ++i) {
+            if (seg[i].bytes == 0) continue;
+            if (total <= kSmallBytes) {
+                unsigned char* p = arena(out_, seg[i].bytes);
+                if (!p) return hipErrorOutOfMemory;   // cannot happen: the arena holds kArenaBytes / kSmallBytes calls between synchronisations
+                l.s[l.n++] = {static_cast<const unsigned char*>(seg[i].dev), p, seg[i].bytes};
+                d.packed[d.n_packed++] = {p, seg[i].host, seg[i].bytes};
+            } else if (pinned(seg[i].host, seg[i].bytes)) {
+                if ((e = hipMemcpyAsync(seg[i].host, seg[i].dev, seg[i].bytes, hipMemcpyDeviceToHost, stream)) != hipSuccess) return e;
+            } else {
+                d.later[d.n_later++] = seg[i];
+            }
+        }
+        return l.n ? launch(l, total, stream) : hipSuccess;
+    }
+    hipError_t down_finish(const Down& d)
+    {
+        std::lock_guard<std::mutex> lock(call_);
+        for (int i = 0; i < d.n_packed; ++i) memcpy(d.packed[i].host, d.packed[i].dev, d.packed[i].bytes);
+        return d.n_later ? pipeline(d.later, d.n_later, false) : hipSuccess;
+    }
+
+    // The device has been synchronised: nothing reads or writes the arenas any more.
+    void quiesced() { in_.used = out_.used = 0; }
+
+    // Pinned host memory for results: copied into by the engines themselves.  A released buffer is kept for the next
+    // request of its size (up to kIdleLimit bytes in all): pinning costs ~0.2 ms per MB.  nullptr: over the limit.
+    void* host_buffer(size_t bytes)
+    {
+        const size_t size = (bytes + (64 << 10) - 1) & ~(size_t)((64 << 10) - 1);
+        std::lock_guard<std::mutex> lock(pool_);
+        for (auto it = idle_.lower_bound(size); it != idle_.end() && it->first <= size + size / 8; ++it) {
+            void* p = it->second;
+            idle_bytes_ -= it->first;
+            bufs_[(uintptr_t)p].live = true;
+            idle_.erase(it);
+            return p;
+        }
+        if (total_bytes_ + size > kTotalLimit) trim(kTotalLimit > size ? kTotalLimit - size : 0);
+        if (total_bytes_ + size > kTotalLimit) return nullptr;
+        void* p = nullptr;
+        if (hipHostMalloc(&p, size, hipHostMallocPortable) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        bufs_[(uintptr_t)p] = {size, true};
+        total_bytes_ += size;
+        return p;
+    }
+    bool release(void* p)
+    {
+        std::lock_guard<std::mutex> lock(pool_);
+        auto it = bufs_.find((uintptr_t)p);
+        if (it == bufs_.end() || !it->second.live) return false;
+        it->second.live = false;
+        idle_.emplace(it->second.size, p);
+        idle_bytes_ += it->second.size;
+        if (idle_bytes_ > kIdleLimit) trim_idle(kIdleLimit);
+        return true;
+    }
+
+    // gives everything back that no caller holds (bfuse_shutdown)
+    void close()
+    {
+        std::lock_guard<std::mutex> lock(call_);
+        {
+            std::lock_guard<std::mutex> pool(pool_);
+            trim_idle(0);
+        }
+        if (device_ < 0) return;
+        stop_workers();
+        for (auto& ev : done_) (void)hipEventDestroy(ev);
+        for (auto& s : stream_) (void)hipStreamDestroy(s);
+        for (void* p : {(void*)ring_, (void*)in_.base, (void*)out_.base}) (void)hipHostFree(p);
+        ring_ = nullptr;
+        device_ = -1;
+    }
+
+private:
+    struct Arena {
+        unsigned char* base = nullptr;
+        size_t used = 0;
+    };
+    struct Buf {
+        size_t size;
+        bool live;
+    };
+
+    hipError_t open()
+    {
+        int dev = 0;
+        hipError_t e = hipGetDevice(&dev);
+        if (e != hipSuccess || dev == device_) return e;
+        if (!ring_) {
+            void* p[3] = {};
+            const size_t size[3] = {kChunk * kSlots, kArenaBytes, kArenaBytes};
+            for (int i = 0; i < 3; ++i)
+                if ((e = hipHostMalloc(&p[i], size[i], hipHostMallocPortable)) != hipSuccess) {
+                    for (int j = 0; j < i; ++j) (void)hipHostFree(p[j]);
+                    return e;
+                }
+            ring_ = static_cast<unsigned char*>(p[0]);
+            in_ = {static_cast<unsigned char*>(p[1]), 0};
+            out_ = {static_cast<unsigned char*>(p[2]), 0};
+            start_workers();
+        }
+        if (device_ >= 0) {   // another device was selected: streams and events belong to one
+            for (auto& ev : done_) (void)hipEventDestroy(ev);
+            for (auto& s : stream_) (void)hipStreamDestroy(s);
+            device_ = -1;
+        }
+        for (auto& s : stream_)
+            if ((e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking)) != hipSuccess) return e;
+        for (auto& ev : done_)
+            if ((e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return e;
+        device_ = dev;
+        return hipSuccess;
+    }
+
+    static unsigned char* arena(Arena& a, size_t bytes)
+    {
+        const size_t need = (bytes + 255) & ~(size_t)255;
+        if (a.used + need > kArenaBytes) return nullptr;
+        unsigned char* p = a.base + a.used;
+        a.used += need;
+        return p;
+    }
+    // 64 blocks: from 8 to 512 reach the link's rate on long copies; short ones want every request out at once
+    static hipError_t launch(const SegList& l, size_t total, hipStream_t stream)
+    {
+        const size_t blocks = std::min<size_t>(64, (total / 16 + 255) / 256 + 1);
+        hipLaunchKernelGGL(copy_segments, dim3((unsigned)blocks), dim3(256), 0, stream, l);
+        return hipGetLastError();
+    }
+
+    hipError_t up_small(const CopySeg* seg, int n, size_t total)
+    {
+        if (in_.used + total + 256 * (size_t)n > kArenaBytes) {
+            // earlier uploads may still be on their way out of the arena
+            hipError_t e = hipStreamSynchronize(nullptr);
+            if (e != hipSuccess) return e;
+            in_.used = 0;
+        }
+        SegList l{};
+        for (int i = 0; i < n; ++i) {
+            if (seg[i].bytes == 0) continue;
+            unsigned char* p = arena(in_, seg[i].bytes);
+            memcpy(p, seg[i].host, seg[i].bytes);
+            l.s[l.n++] = {p, static_cast<unsigned char*>(seg[i].dev), seg[i].bytes};
+        }
+        return launch(l, total, nullptr);
+    }
+
+    // ---- the ring ---------------------------------------------------------------------------------
+    struct Chunk {
+        unsigned char *dev, *host;
+        size_t bytes;
+        long first;                                   // number of its first piece
+        int pieces() const { return (int)((bytes + kPiece - 1) / kPiece); }
+    };
+    static void pause(unsigned& spins)
+    {
+        if (++spins < 512) _mm_pause();
+        else sched_yield();
+    }
+
+    // Chunks in order, each in pieces.  Up: the threads claim pieces and fill the slots; this thread sends every chunk
+    // whose slot is full and gives a slot back when its copy has ended.  Down: the other way round.  A piece is claimed
+    // only when it can be moved at once (its slot is free, or its chunk has landed), so no thread ever holds a claim
+    // that waits for another; this thread moves pieces too while it has nothing to send.
+    hipError_t pipeline(const CopySeg* seg, int n, bool up)
+    {
+        std::vector<Chunk> chunks;
+        long pieces = 0;
+        // half slots for a few MB, where the first chunk's way through the host shows (5 MB: 145 against 166 us);
+        // whole ones, with fewer starts, for more (10 MB: 260 against 300 us)
+        size_t total = 0;
+        for (int i = 0; i < n; ++i) total += seg[i].bytes;
+        const size_t chunk = total <= (8 << 20) ? kChunk / 2 : kChunk;
+        hipError_t e = hipSuccess;
+        for (int i = 0; i < n; ++i) {
+            if (up && pinned(seg[i].host, seg[i].bytes)) {
+                if ((e = hipMemcpyAsync(seg[i].dev, seg[i].host, seg[i].bytes, hipMemcpyHostToDevice, stream_[0])) != hipSuccess) return e;
+                continue;
+            }
+            for (size_t o = 0; o < seg[i].bytes; o += chunk) {
+                chunks.push_back({static_cast<unsigned char*>(seg[i].dev) + o, static_cast<unsigned char*>(seg[i].host) + o, std::min(chunk, seg[i].bytes - o), pieces});
+                pieces += chunks.back().pieces();
+            }
+        }
+        const long count = (long)chunks.size();
+        if (count) {
+            begin_job(chunks, up);
+            long sent = 0, ended = 0;          // copies enqueued / known to have ended
+            unsigned spins = 0;
+            while (ended < count && e == hipSuccess) {
+                const int slot = (int)(sent % kSlots);
+                // up: the chunk has been let into its slot and all of it is there.  down: what was in the slot has been drained
+                if (sent < count && (up ? sent < ended + kSlots && done(sent) : sent < kSlots || done(sent - kSlots))) {
+                    const Chunk& c = chunks[(size_t)sent];
+                    if (!up) left_[slot].store(c.pieces(), std::memory_order_relaxed);
+                    unsigned char* const s = ring_ + slot * kChunk;
+                    e = send(up ? s : c.dev, up ? c.dev : s, c.bytes, stream_[sent & 1]);
+                    if (e == hipSuccess) e = hipEventRecord(done_[slot], stream_[sent & 1]);
+                    ++sent;
+                    spins = 0;
+                    continue;
+                }
+                if (ended < sent) {
+                    const hipError_t q = hipEventQuery(done_[ended % kSlots]);
+                    if (q == hipSuccess) {
+                        // up: the slot takes the chunk kSlots further on.  down: the chunk can be drained
+                        const long i = up ? ended + kSlots : ended;
+                        if (up && i < count) left_[ended % kSlots].store(chunks[(size_t)i].pieces(), std::memory_order_relaxed);
+                        ++ended;
+                        if (i < count) go_.store(chunks[(size_t)i].first + chunks[(size_t)i].pieces(), std::memory_order_release);
+                        spins = 0;
+                        continue;
+                    }
+                    if (q != hipErrorNotReady) e = q;
+                }
+                if (!work()) pause(spins);
+            }
+            end_job();
+        }
+        for (auto& s : stream_) {
+            const hipError_t q = hipStreamSynchronize(s);
+            if (e == hipSuccess) e = q;
+        }
+        return e;
+    }
+
+    // whether every piece of chunk i, which is or was the last in its slot, has been moved
+    bool done(long i) const { return left_[i % kSlots].load(std::memory_order_acquire) == 0; }
+
+    // One copy of the ring: by a kernel, which starts sooner behind its predecessor than a copy engine does (1 MiB chunks,
+    // 128 MB: 48 against 46 GB/s up, 46 against 39 down); 32 workgroups fill the link and leave the chip to others.
+    static hipError_t send(const unsigned char* src, unsigned char* dst, size_t bytes, hipStream_t stream)
+    {
+        SegList l{};
+        l.n = 1;
+        l.s[0] = {src, dst, bytes};
+        hipLaunchKernelGGL(copy_segments, dim3(32), dim3(256), 0, stream, l);
+        return hipGetLastError();
+    }
+
+    void begin_job(const std::vector<Chunk>& c, bool up)
+    {
+        std::unique_lock<std::mutex> lock(job_);
+        idle_cv_.wait(lock, [this] { return active_ == 0; });
+        chunks_ = c.data();
+        count_ = (long)c.size();
+        up_ = up;
+        next_.store(0);
+        for (long i = 0; i < kSlots; ++i) left_[i].store(up && i < count_ ? c[(size_t)i].pieces() : 0);
+        go_.store(up ? c[(size_t)std::min<long>(count_, kSlots) - 1].first + c[(size_t)std::min<long>(count_, kSlots) - 1].pieces() : 0);
+        live_.store(true);
+        ++generation_;
+        if (asleep_) work_cv_.notify_all();
+    }
+    // every piece that may be moved has been, and nobody looks at the job any more
+    void end_job()
+    {
+        while (work()) {}
+        live_.store(false);
+        std::unique_lock<std::mutex> lock(job_);
+        idle_cv_.wait(lock, [this] { return active_ == 0; });
+        chunks_ = nullptr;                 // a worker that wakes up only now finds nothing
+    }
+
+    // into a slot: with stores that leave the lines in no cache, so that the link reads them from memory and not from
+    // whichever core wrote them (128 MB: 52 against 48 GB/s)
+    static void stream_copy(unsigned char* dst, const unsigned char* src, size_t bytes)
+    {
+        size_t i = 0;
+        for (; i + 64 <= bytes; i += 64)
+            for (size_t j = i; j < i + 64; j += 16)
+                _mm_stream_si128(reinterpret_cast<__m128i*>(dst + j), _mm_loadu_si128(reinterpret_cast<const __m128i*>(src + j)));
+        memcpy(dst + i, src + i, bytes - i);
+        _mm_sfence();
+    }
+
+    // moves one piece of the current job; false if none can be moved at the moment
+    bool work()
+    {
+        long i = next_.load(std::memory_order_relaxed);
+        do {
+            if (i >= go_.load(std::memory_order_acquire)) return false;
+        } while (!next_.compare_exchange_weak(i, i + 1));
+        const long c = std::upper_bound(chunks_, chunks_ + count_, i, [](long v, const Chunk& k) { return v < k.first; }) - chunks_ - 1;
+        const Chunk& k = chunks_[c];
+        const size_t at = (size_t)(i - k.first) * kPiece, len = std::min(kPiece, k.bytes - at);
+        const int slot = (int)(c % kSlots);
+        unsigned char* const s = ring_ + slot * kChunk + at;
+        if (up_) stream_copy(s, k.host + at, len);
+        else memcpy(k.host + at, s, len);
+        left_[slot].fetch_sub(1, std::memory_order_release);
+        return true;
+    }
+
+    // A worker that has just worked looks for the next job for a millisecond before it sleeps: waking a sleeping
+    // core takes longer (tens of microseconds each) than a transfer of a few MB.
+    void worker()
+    {
+        unsigned long seen = 0;
+        for (;;) {
+            const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
+            for (unsigned spins = 0; generation_.load(std::memory_order_acquire) == seen && std::chrono::steady_clock::now() < until;) pause(spins);
+            {
+                std::unique_lock<std::mutex> lock(job_);
+                if (!stop_ && generation_.load() == seen) {
+                    ++asleep_;
+                    work_cv_.wait(lock, [&] { return stop_ || generation_.load() != seen; });
+                    --asleep_;
+                }
+                if (stop_) return;
+                seen = generation_.load();
+                if (!chunks_) continue;
+                ++active_;
+            }
+            unsigned spins = 0;
+            while (live_.load(std::memory_order_acquire)) {
+                if (work()) spins = 0;
+                else pause(spins);
+            }
+            std::lock_guard<std::mutex> lock(job_);
+            if (--active_ == 0) idle_cv_.notify_all();
+        }
+    }
+    void start_workers()
+    {
+        cpu_set_t set;
+        int cores = sched_getaffinity(0, sizeof(set), &set) == 0 ? CPU_COUNT(&set) : 1;
+        stop_ = false;
+        for (int i = 0; i < std::min(kMaxWorkers, cores / 2); ++i) workers_.emplace_back([this] { worker(); });
+    }
+    void stop_workers()
+    {
+        {
+            std::lock_guard<std::mutex> lock(job_);
+            stop_ = true;
+        }
+        work_cv_.notify_all();
+        for (auto& t : workers_) t.join();
+        workers_.clear();
+    }
+
+    // ---- pinned result buffers ----------------------------------------------------------------------
+    bool pinned(const void* p, size_t bytes)
+    {
+        std::lock_guard<std::mutex> lock(pool_);
+        auto it = bufs_.upper_bound((uintptr_t)p);
+        if (it == bufs_.begin()) return false;
+        --it;
+        return (uintptr_t)p + bytes <= it->first + it->second.size;
+    }
+    void trim_idle(size_t limit)
+    {
+        while (idle_bytes_ > limit && !idle_.empty()) {
+            auto it = std::prev(idle_.end());
+            (void)hipHostFree(it->second);
+            bufs_.erase((uintptr_t)it->second);
+            idle_bytes_ -= it->first;
+            total_bytes_ -= it->first;
+            idle_.erase(it);
+        }
+    }
+    void trim(size_t limit) { trim_idle(total_bytes_ > limit ? (idle_bytes_ > total_bytes_ - limit ? idle_bytes_ - (total_bytes_ - limit) : 0) : idle_bytes_); }
+
+    std::mutex call_;                    // one transfer at a time
+    int device_ = -1;
+    unsigned char* ring_ = nullptr;
+    Arena in_, out_;
+    hipStream_t stream_[2] = {};
+    hipEvent_t done_[kSlots] = {};
+
+    std::mutex job_;
+    std::condition_variable work_cv_, idle_cv_;
+    std::vector<std::thread> workers_;
+    bool stop_ = false;
+    std::atomic<unsigned long> generation_{0};
+    int active_ = 0, asleep_ = 0;
+    const Chunk* chunks_ = nullptr;
+    long count_ = 0;
+    bool up_ = true;
+    std::atomic<bool> live_{false};
+    std::atomic<long> next_{0}, go_{0};  // pieces: the next one nobody has claimed, the end of those that can be moved
+    std::atomic<int> left_[kSlots] = {}; // pieces of the chunk in each slot that have not been moved yet
+
+    std::mutex pool_;
+    std::map<uintptr_t, Buf> bufs_;
+    std::multimap<size_t, void*> idle_;
+    size_t idle_bytes_ = 0, total_bytes_ = 0;
+};
+
+}  // namespace bfuse

@@ -18,6 +18,7 @@
 #include "../../include/bfuse_rt.h"
 #include "dispatch.h"
 #include "fuse.h"
+#include "host_copy.h"
 
 namespace bfuse {
 std::vector<KernelEntry>& registry()
@@ -105,6 +106,7 @@ struct EventList {
 // entry point performs it.
 std::vector<const void*> g_pending_fused;
 std::vector<int> g_pending_modules;
+bool g_busy = false;   // something has been enqueued since the last device synchronisation
 
 // ---- staging memory of bfuse_map_blocks_device_noalloc ----------------------------------------
 // A fixed device array (kernel and block index of up to kNoAllocMaxIds fused blocks) that lives as
@@ -247,6 +249,7 @@ int launch3(const void* func, const unsigned* grid, const unsigned* block, int i
 {
     Side& s = g.side[idx];
     void* args[3] = {&s.buf[0], &s.buf[1], &s.buf[2]};
+    g_busy = true;
     if (ev0 || ev1)
         HIP_TRY(hipExtLaunchKernel(func, d3(grid), d3(block), args, 0, stream, ev0, ev1, 0));
     else
@@ -267,6 +270,7 @@ int launch_fused(const void* func, const unsigned* grid, const unsigned* block, 
     bool known = false;
     for (const void* f : g_pending_fused) known = known || f == func;
     if (!known) g_pending_fused.push_back(func);
+    g_busy = true;
     if (ev0 || ev1)
         HIP_TRY(hipExtLaunchKernel(func, d3(grid), d3(block), args, 0, stream, ev0, ev1, 0));
     else
@@ -302,7 +306,10 @@ int sync_and_check()
         if (e != hipSuccess && rc == BFUSE_OK) rc = fail(BFUSE_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
         return e == hipSuccess;
     };
-    note_hip(hipDeviceSynchronize(), "hipDeviceSynchronize");
+    if (note_hip(hipDeviceSynchronize(), "hipDeviceSynchronize")) {
+        g_busy = false;
+        HostCopy::get().quiesced();
+    }
     note_hip(hipGetLastError(), "launch");
     // every counter is read (and thereby reset) even after an error above; the first error is the one returned
     for (const void* f : fused) {
@@ -484,6 +491,7 @@ int bfuse_shutdown(void)
             int rc2 = fini_side(i);
             if (rc2) return rc2;
         }
+    HostCopy::get().close();
     for (auto& m : modules())
         if (m) {
             HIP_TRY(hipModuleUnload(m));
@@ -871,6 +879,34 @@ int bfuse_finalize_side(int side)
     return fini_side(side - 1);
 }
 
+// The copies of the harness functions (host_copy.h): operands of a side up, results down.
+static int copy_up(const CopySeg* seg, int n, bool busy)
+{
+    HIP_TRY(HostCopy::get().up(seg, n, busy));
+    g_busy = true;   // a small upload is a launch
+    return BFUSE_OK;
+}
+static int upload_sides(const int* idx, const void* const (*src)[2], int n)
+{
+    CopySeg seg[kMaxSegs];
+    for (int k = 0; k < n; ++k)
+        for (int t = 0; t < 2; ++t) seg[2 * k + t] = {g.side[idx[k]].buf[t], const_cast<void*>(src[k][t]), g.side[idx[k]].bytes[t]};
+    return copy_up(seg, 2 * n, g_busy);
+}
+// waits for everything launched, then brings the results of `n` sides to the host; nothing is written there if a
+// barrier gave up, unless `always`
+static int download_sides(const int* idx, void* const* dst, int n, bool always)
+{
+    CopySeg seg[kMaxKernels];
+    for (int k = 0; k < n; ++k) seg[k] = {g.side[idx[k]].buf[2], dst[k], g.side[idx[k]].bytes[2]};
+    HostCopy::Down d;
+    HIP_TRY(HostCopy::get().down_begin(seg, n, nullptr, d));
+    const int rc = sync_and_check();
+    if (rc && !(always && rc == BFUSE_ERR_SYNC)) return rc;
+    HIP_TRY(HostCopy::get().down_finish(d));
+    return rc;
+}
+
 static int run_single(int idx, const void* I, const void* F, void* O, const int* Is, const int* Fs, const int* Os,
                       const void* func, const unsigned* grid, const unsigned* block)
 {
@@ -878,13 +914,10 @@ static int run_single(int idx, const void* I, const void* F, void* O, const int*
     if (!I || !F || !O) return fail(BFUSE_ERR_ARG, "null host buffer");
     if ((rc = check_shapes(idx, Is, Fs, Os))) return rc;
     if ((rc = validate_mode(idx == 0 ? BFUSE_MODE_KERNEL1 : BFUSE_MODE_KERNEL2, func, grid, block, nullptr, nullptr, nullptr))) return rc;
-    Side& s = g.side[idx];
-    HIP_TRY(hipMemcpy(s.buf[0], I, s.bytes[0], hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(s.buf[1], F, s.bytes[1], hipMemcpyHostToDevice));
+    const void* const src[1][2] = {{I, F}};
+    if ((rc = upload_sides(&idx, src, 1))) return rc;
     if ((rc = launch3(func, grid, block, idx, nullptr))) return rc;
-    if ((rc = sync_and_check())) return rc;
-    HIP_TRY(hipMemcpy(O, s.buf[2], s.bytes[2], hipMemcpyDeviceToHost));
-    return BFUSE_OK;
+    return download_sides(&idx, &O, 1, false);
 }
 
 int run_kernel1(const void* I, const void* F, void* O, const int* Is, const int* Fs, const int* Os,
@@ -899,24 +932,6 @@ int run_kernel2(const void* I, const void* F, void* O, const int* Is, const int*
     return run_single(1, I, F, O, Is, Fs, Os, (const void*)func, grid, block);
 }
 
-static int upload_both(const void* I1, const void* F1, const void* I2, const void* F2)
-{
-    Side &a = g.side[0], &b = g.side[1];
-    HIP_TRY(hipMemcpy(a.buf[0], I1, a.bytes[0], hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(a.buf[1], F1, a.bytes[1], hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(b.buf[0], I2, b.bytes[0], hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(b.buf[1], F2, b.bytes[1], hipMemcpyHostToDevice));
-    return BFUSE_OK;
-}
-
-static int download_both(void* O1, void* O2)
-{
-    Side &a = g.side[0], &b = g.side[1];
-    HIP_TRY(hipMemcpy(O1, a.buf[2], a.bytes[2], hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(O2, b.buf[2], b.bytes[2], hipMemcpyDeviceToHost));
-    return BFUSE_OK;
-}
-
 int run_parallel(const void* I1, const void* F1, void* O1, const void* I2, const void* F2, void* O2, const int* I1s,
                  const int* F1s, const int* O1s, const int* I2s, const int* F2s, const int* O2s,
                  bfuse_kernel3_fn func1, bfuse_kernel3_fn func2, const unsigned* g1, const unsigned* b1,
@@ -926,10 +941,29 @@ int run_parallel(const void* I1, const void* F1, void* O1, const void* I2, const
     if (!I1 || !F1 || !O1 || !I2 || !F2 || !O2) return fail(BFUSE_ERR_ARG, "null host buffer");
     if ((rc = check_shapes(0, I1s, F1s, O1s)) || (rc = check_shapes(1, I2s, F2s, O2s))) return rc;
     if ((rc = validate_mode(BFUSE_MODE_PARALLEL, (const void*)func1, g1, b1, (const void*)func2, g2, b2))) return rc;
-    if ((rc = upload_both(I1, F1, I2, F2))) return rc;
-    if ((rc = enqueue_mode(BFUSE_MODE_PARALLEL, (const void*)func1, g1, b1, (const void*)func2, g2, b2, nullptr))) return rc;
+    static constexpr int both[2] = {0, 1};
+    const void* const src[2][2] = {{I1, F1}, {I2, F2}};
+    void* const dst[2] = {O1, O2};
+    const Side &a = g.side[0], &b = g.side[1];
+    if (std::min(a.bytes[0] + a.bytes[1], b.bytes[0] + b.bytes[1]) <= HostCopy::kSmallBytes) {
+        if ((rc = upload_sides(both, src, 2))) return rc;
+        if ((rc = enqueue_mode(BFUSE_MODE_PARALLEL, (const void*)func1, g1, b1, (const void*)func2, g2, b2, nullptr))) return rc;
+        return download_sides(both, dst, 2, false);
+    }
+    // Long copies: each side runs through its own stream, so that side 1's kernel and the copy of its result (where it
+    // can be copied in place) run while side 2's operands come up -- the link carries 96 GB/s both ways, 57 one way.
+    // Side 2's copies wait for nothing: only this call's launches are under way, over other buffers.
+    HostCopy::Down d[2];
+    for (int k = 0; k < 2; ++k) {
+        const CopySeg up[2] = {{g.side[k].buf[0], const_cast<void*>(src[k][0]), g.side[k].bytes[0]}, {g.side[k].buf[1], const_cast<void*>(src[k][1]), g.side[k].bytes[1]}};
+        const CopySeg down = {g.side[k].buf[2], dst[k], g.side[k].bytes[2]};
+        if ((rc = copy_up(up, 2, k == 0 && g_busy))) return rc;
+        if ((rc = k == 0 ? launch3((const void*)func1, g1, b1, 0, a.stream) : launch3((const void*)func2, g2, b2, 1, b.stream))) return rc;
+        HIP_TRY(HostCopy::get().down_begin(&down, 1, g.side[k].stream, d[k]));
+    }
     if ((rc = sync_and_check())) return rc;
-    return download_both(O1, O2);
+    for (int k = 0; k < 2; ++k) HIP_TRY(HostCopy::get().down_finish(d[k]));
+    return BFUSE_OK;
 }
 
 int run_fuse(const void* I1, const void* F1, void* O1, const void* I2, const void* F2, void* O2, const int* I1s,
@@ -943,10 +977,12 @@ int run_fuse(const void* I1, const void* F1, void* O1, const void* I2, const voi
     if (!e || e->kind == kSingle) return fail(BFUSE_ERR_ARG, "func is not a fused kernel of this library");
     const int mode = e->kind == kHfuse ? BFUSE_MODE_HFUSE : BFUSE_MODE_BFUSE;
     if ((rc = validate_mode(mode, (const void*)func, grid, block, nullptr, nullptr, nullptr))) return rc;
-    if ((rc = upload_both(I1, F1, I2, F2))) return rc;
+    static constexpr int both[2] = {0, 1};
+    const void* const src[2][2] = {{I1, F1}, {I2, F2}};
+    void* const dst[2] = {O1, O2};
+    if ((rc = upload_sides(both, src, 2))) return rc;
     if ((rc = launch6((const void*)func, grid, block, nullptr))) return rc;
-    if ((rc = sync_and_check())) return rc;
-    return download_both(O1, O2);
+    return download_sides(both, dst, 2, false);
 }
 
 // ---- device-resident operation and timing -------------------------------------------------
@@ -956,9 +992,9 @@ int bfuse_upload(int side, const void* I, const void* F)
     Side& s = g.side[side - 1];
     if (!s.live) return fail(BFUSE_ERR_STATE, "kernel%d is not initialized", side);
     if (!I || !F) return fail(BFUSE_ERR_ARG, "null host buffer");
-    HIP_TRY(hipMemcpy(s.buf[0], I, s.bytes[0], hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(s.buf[1], F, s.bytes[1], hipMemcpyHostToDevice));
-    return BFUSE_OK;
+    const int idx = side - 1;
+    const void* const src[1][2] = {{I, F}};
+    return upload_sides(&idx, src, 1);
 }
 
 int bfuse_zero_output(int side)
@@ -966,6 +1002,7 @@ int bfuse_zero_output(int side)
     if (side < 1 || side > kMaxKernels) return fail(BFUSE_ERR_ARG, "side must be 1 .. %d", kMaxKernels);
     Side& s = g.side[side - 1];
     if (!s.live) return fail(BFUSE_ERR_STATE, "kernel%d is not initialized", side);
+    g_busy = true;
     HIP_TRY(hipMemset(s.buf[2], 0, s.bytes[2]));
     return BFUSE_OK;
 }
@@ -978,10 +1015,20 @@ int bfuse_download(int side, void* O)
     if (!O) return fail(BFUSE_ERR_ARG, "null host buffer");
     // the output is copied out even when a side barrier gave up (the caller may want to look at
     // it), but the call then reports BFUSE_ERR_SYNC
-    const int rc = sync_and_check();
-    if (rc && rc != BFUSE_ERR_SYNC) return rc;
-    HIP_TRY(hipMemcpy(O, s.buf[2], s.bytes[2], hipMemcpyDeviceToHost));
-    return rc;
+    const int idx = side - 1;
+    return download_sides(&idx, &O, 1, true);
+}
+
+void* bfuse_host_buffer(size_t bytes)
+{
+    if (!g.inited || bytes == 0) return nullptr;
+    return HostCopy::get().host_buffer(bytes);
+}
+
+int bfuse_host_buffer_release(void* p)
+{
+    if (!HostCopy::get().release(p)) return fail(BFUSE_ERR_ARG, "not a buffer of bfuse_host_buffer");
+    return BFUSE_OK;
 }
 
 int bfuse_upload_part(int side, int tensor, size_t offset, const void* src, size_t bytes)
@@ -993,8 +1040,8 @@ int bfuse_upload_part(int side, int tensor, size_t offset, const void* src, size
     if (!src) return fail(BFUSE_ERR_ARG, "null host buffer");
     if (offset > s.bytes[tensor] || bytes > s.bytes[tensor] - offset)
         return fail(BFUSE_ERR_ARG, "bytes %zu .. %zu are outside the tensor's %zu", offset, offset + bytes, s.bytes[tensor]);
-    if (bytes) HIP_TRY(hipMemcpy(static_cast<char*>(s.buf[tensor]) + offset, src, bytes, hipMemcpyHostToDevice));
-    return BFUSE_OK;
+    const CopySeg seg = {static_cast<char*>(s.buf[tensor]) + offset, const_cast<void*>(src), bytes};
+    return copy_up(&seg, 1, g_busy);
 }
 
 int bfuse_download_part(int side, size_t offset, void* dst, size_t bytes)
@@ -1005,9 +1052,12 @@ int bfuse_download_part(int side, size_t offset, void* dst, size_t bytes)
     if (!dst) return fail(BFUSE_ERR_ARG, "null host buffer");
     if (offset > s.bytes[2] || bytes > s.bytes[2] - offset)
         return fail(BFUSE_ERR_ARG, "bytes %zu .. %zu are outside the output's %zu", offset, offset + bytes, s.bytes[2]);
+    const CopySeg seg = {static_cast<char*>(s.buf[2]) + offset, dst, bytes};
+    HostCopy::Down d;
+    HIP_TRY(HostCopy::get().down_begin(&seg, 1, nullptr, d));
     const int rc = sync_and_check();
     if (rc && rc != BFUSE_ERR_SYNC) return rc;
-    if (bytes) HIP_TRY(hipMemcpy(dst, static_cast<const char*>(s.buf[2]) + offset, bytes, hipMemcpyDeviceToHost));
+    HIP_TRY(HostCopy::get().down_finish(d));
     return rc;
 }
 
@@ -1087,6 +1137,7 @@ int bfuse_fill_uniform_device(int side, int tensor, unsigned long long seed, flo
     size_t blocks = (n + 256 * 8 - 1) / (256 * 8);
     if (blocks > 16384) blocks = 16384;
     if (blocks < 1) blocks = 1;
+    g_busy = true;
     hipLaunchKernelGGL(fill_uniform_kernel, dim3((unsigned)blocks), dim3(256), 0, nullptr, s.buf[tensor], n, s.elem[tensor], seed, lo, hi);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipDeviceSynchronize());
@@ -1411,6 +1462,7 @@ int bfuse_module_launch(int id, const char* name, const unsigned* grid, const un
     bool known = false;
     for (int m : g_pending_modules) known = known || m == id;
     if (!known) g_pending_modules.push_back(id);
+    g_busy = true;
     HIP_TRY(hipExtModuleLaunchKernel(fn, grid[0] * block[0], grid[1] * block[1], grid[2] * block[2], block[0], block[1],
                                      block[2], 0, nullptr, args, nullptr, e0, e1, 0));
     if (us_out) {

@@ -4,6 +4,7 @@ finalize over numpy buffers, plus the device-resident launch and GPU-side timing
 """
 import ctypes as C
 import os
+import weakref
 from dataclasses import dataclass, replace
 from typing import List, Optional, Sequence
 
@@ -72,6 +73,23 @@ def _u3(v):
 
 _DT = {4: np.float32, 2: np.uint16, 1: np.uint8}
 
+# Results of at least this size are arrays over the library's pinned buffers, which the copy engines write in place
+# (57 GB/s; a new array of pageable memory takes 10-20 GB/s, most of it page faults).  Below, one memcpy out of the
+# library's arena is cheaper than the bookkeeping of a buffer (~5 us).
+PINNED_MIN_BYTES = 512 << 10
+
+
+def _result(shape, dtype) -> np.ndarray:
+    nbytes = int(np.prod(shape)) * np.dtype(dtype).itemsize
+    l = _lib.lib()
+    p = l.bfuse_host_buffer(nbytes) if nbytes >= PINNED_MIN_BYTES else None
+    if not p:      # small, or the library's limit of pinned memory is in use
+        return np.empty(shape, dtype)
+    buf = (C.c_byte * nbytes).from_address(p)
+    # the buffer goes back to the library with the last array over it (not at interpreter exit, when HIP is gone)
+    weakref.finalize(buf, l.bfuse_host_buffer_release, p).atexit = False
+    return np.frombuffer(buf, dtype).reshape(shape)
+
 
 class Operation:
     """One pair of sides with their device buffers (the reference keeps them in file-scope
@@ -119,7 +137,7 @@ class Operation:
 
     def empty_output(self, side):
         k = self.k[side]
-        return np.empty(tuple(d for d in k.shapes[2]), _DT[k.elem_bytes[2]])
+        return _result(k.shapes[2], _DT[k.elem_bytes[2]])
 
     def fused(self, kind: str, suffix: str = "") -> KernelHandle:
         return kernel_info(f"{self.k[0].name}_{self.k[1].name}_fused_{kind}{suffix}")
@@ -183,7 +201,7 @@ class Operation:
 
     def download_part(self, side: int, offset: int, count: int) -> np.ndarray:
         """`count` elements of the side's output, starting at element `offset`."""
-        O = np.empty(count, _DT[self.k[side].elem_bytes[2]])
+        O = _result((count,), _DT[self.k[side].elem_bytes[2]])
         _lib.check(self.l.bfuse_download_part(side + 1, offset * O.itemsize, O.ctypes.data, O.nbytes))
         return O
 
@@ -302,7 +320,7 @@ class GroupOperation:
 
     def download(self, side: int) -> np.ndarray:
         k = self.k[side]
-        O = np.empty(tuple(k.shapes[2]), _DT[k.elem_bytes[2]])
+        O = _result(k.shapes[2], _DT[k.elem_bytes[2]])
         _lib.check(self.l.bfuse_download(side + 1, O.ctypes.data))
         return O
 
@@ -388,7 +406,7 @@ class GenericOperation:
             _lib.check(self.l.bfuse_zero_output(side))
 
     def download(self, side: int) -> np.ndarray:
-        O = np.empty(self.nelem[side][2], np.float32)
+        O = _result((self.nelem[side][2],), np.float32)
         _lib.check(self.l.bfuse_download(side + 1, O.ctypes.data))
         return O
 

@@ -225,6 +225,14 @@ int bfuse_zero_output(int side);
 int bfuse_download(int side, void* O);
 int bfuse_synchronize(void);
 
+/* Pinned host memory for operands and results: the copies above move it in place, at the link's rate, where other host
+ * memory goes through a staging ring.  NULL before bfuse_init, or when the library already has its limit of such
+ * buffers (4 GiB) in existence: use ordinary memory then.  A released buffer is kept for the next request of its size
+ * (up to 1 GiB in all) and given back by bfuse_shutdown; a buffer stays valid until it is released, whatever happens to
+ * the operation.  Callable from any thread.  No counterpart in the reference. */
+void* bfuse_host_buffer(size_t bytes);
+int bfuse_host_buffer_release(void* buffer);
+
 /* The same for a part of a tensor: operands and results of several GB (the reference's benchmark.yaml runs every
  * operator at batch 1024) need not pass through one host array.  `tensor`: 0 = I, 1 = F; offsets and sizes in
  * bytes.  No counterpart in the reference, whose harness copies whole tensors (operation_cu.py:74-118). */
