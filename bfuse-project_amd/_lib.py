@@ -54,6 +54,11 @@ class LaunchDescC(C.Structure):
                 ("n_sides", C.c_int), ("sides", C.c_int * MAXK)]
 
 
+class LaunchArgsC(C.Structure):
+    _fields_ = [("mode", C.c_int), ("grid_a", C.c_uint * 3), ("block_a", C.c_uint * 3), ("grid_b", C.c_uint * 3), ("block_b", C.c_uint * 3),
+                ("func_a", C.c_void_p), ("func_b", C.c_void_p)]
+
+
 # every symbol include/bfuse_rt.h declares
 EXPORTS = [
     "bfuse_last_error", "bfuse_init", "bfuse_shutdown", "bfuse_device_info", "bfuse_device_memory",
@@ -62,7 +67,7 @@ EXPORTS = [
     "bfuse_kernel_count", "bfuse_kernel_at", "bfuse_kernel_find", "bfuse_load_kernels", "bfuse_kernel_op_type", "bfuse_kernel_op_lds",
     "bfuse_set_elem_bytes", "initialize_kernel1", "initialize_kernel2", "finalize_kernel1", "finalize_kernel2",
     "run_kernel1", "run_kernel2", "run_parallel", "run_fuse",
-    "bfuse_upload", "bfuse_zero_output", "bfuse_download", "bfuse_synchronize", "bfuse_launch",
+    "bfuse_upload", "bfuse_zero_output", "bfuse_download", "bfuse_synchronize", "bfuse_launch", "bfuse_launch_packed",
     "bfuse_host_buffer", "bfuse_host_buffer_release",
     "bfuse_upload_part", "bfuse_download_part", "bfuse_checksum_output", "bfuse_fill_uniform_device",
     "bfuse_time", "bfuse_time_batched", "bfuse_time_graph", "bfuse_module_load", "bfuse_module_unload", "bfuse_module_launch",
@@ -126,6 +131,7 @@ def lib():
         l.bfuse_checksum_output.argtypes = [C.c_int, C.c_size_t, vp]
         l.bfuse_fill_uniform_device.argtypes = [C.c_int, C.c_int, C.c_ulonglong, C.c_float, C.c_float]
         l.bfuse_launch.argtypes = [C.c_int, vp, up, up, vp, up, up]
+        l.bfuse_launch_packed.argtypes = [vp]
         fp = C.POINTER(C.c_float)
         l.bfuse_time.argtypes = [C.c_int, vp, up, up, vp, up, up, C.c_int, C.c_int, fp, fp, fp]
         l.bfuse_time_batched.argtypes = [C.c_int, vp, up, up, vp, up, up, C.c_int, C.c_int, fp]

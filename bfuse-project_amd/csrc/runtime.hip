@@ -13,6 +13,7 @@
 #include <cstring>
 #include <string>
 #include <map>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/bfuse_rt.h"
@@ -170,11 +171,46 @@ int check_shapes(int idx, const int* I, const int* F, const int* O)
 
 dim3 d3(const unsigned* v) { return dim3(v[0], v[1], v[2]); }
 
+// What a launch needs to know of a kernel, by its handle: its entry and the bytes each of its operators' tensors take.
+// Every launch is validated; looking this up by name in the registry (some 330 entries, a fused kernel's sides by string)
+// took 1.5 us of a launch that the runtime itself makes in 2.3.  Rebuilt when kernels have been added.
+struct Launchable {
+    const KernelEntry* e;
+    int n_sides;                               // operators it runs
+    const KernelEntry* side[kMaxKernels];      // their standalone kernels (nullptr: unknown)
+    size_t need[kMaxKernels][3];
+};
+const Launchable* launchable(const void* func)
+{
+    static std::unordered_map<const void*, Launchable> known;
+    static size_t built = 0;
+    const auto& r = registry();
+    if (built != r.size()) {
+        std::unordered_map<std::string, const KernelEntry*> single;
+        known.clear();
+        for (const auto& e : r)
+            if (e.kind == kSingle) single.emplace(e.name, &e);
+        for (const auto& e : r) {
+            Launchable l{};
+            l.e = &e;
+            l.n_sides = e.kind == kSingle ? 1 : e.n_sides;
+            for (int k = 0; k < l.n_sides; ++k) {
+                auto it = single.find(e.side[k]);
+                l.side[k] = e.kind == kSingle ? &e : it == single.end() ? nullptr : it->second;
+                for (int i = 0; l.side[k] && i < 3; ++i) l.need[k][i] = shape_bytes(l.side[k]->io[i].shape, l.side[k]->io[i].elem_bytes);
+            }
+            known.emplace(e.func, l);
+        }
+        built = r.size();
+    }
+    auto it = known.find(func);
+    return it == known.end() ? nullptr : &it->second;
+}
+
 const KernelEntry* entry_of(const void* func)
 {
-    for (const auto& e : registry())
-        if (e.func == func) return &e;
-    return nullptr;
+    const Launchable* l = launchable(func);
+    return l ? l->e : nullptr;
 }
 
 // The grid and block a caller passes must be the ones the kernel was built for: the bodies
@@ -212,33 +248,31 @@ int check_launch(const void* func, const unsigned* grid, const unsigned* block, 
     return BFUSE_OK;
 }
 
-// Buffers a single kernel touches must be at least as large as the shapes it was built for.
-int check_side_fits(const void* func, int idx)
+// Buffers an operator touches must be at least as large as the shapes its kernel was built for.
+int check_buffers(const Launchable& l, int k, int idx)
 {
-    const KernelEntry* e = entry_of(func);
-    if (!e || e->kind != kSingle) return BFUSE_OK;
     const Side& s = g.side[idx];
     if (!s.live) return fail(BFUSE_ERR_STATE, "kernel%d is not initialized", idx + 1);
-    for (int i = 0; i < 3; ++i) {
-        const size_t need = shape_bytes(e->io[i].shape, e->io[i].elem_bytes);
-        if (s.bytes[i] < need)
-            return fail(BFUSE_ERR_ARG, "%s needs %zu bytes for tensor %d, side %d holds %zu", e->name.c_str(), need, i,
+    for (int i = 0; i < 3; ++i)
+        if (s.bytes[i] < l.need[k][i])
+            return fail(BFUSE_ERR_ARG, "%s needs %zu bytes for tensor %d, side %d holds %zu", l.side[k]->name.c_str(), l.need[k][i], i,
                         idx + 1, s.bytes[i]);
-    }
     return BFUSE_OK;
+}
+int check_side_fits(const void* func, int idx)
+{
+    const Launchable* l = launchable(func);
+    return !l || l->e->kind != kSingle ? BFUSE_OK : check_buffers(*l, 0, idx);
 }
 
 // `sides` (0-based, one per operator of the fused kernel) or nullptr for sides 0, 1, ...
 int check_fused_fits(const void* func, const int* sides = nullptr)
 {
-    const KernelEntry* e = entry_of(func);
-    if (!e || e->kind == kSingle) return fail(BFUSE_ERR_ARG, "not a fused kernel");
-    for (int k = 0; k < e->n_sides; ++k) {
-        const KernelEntry* sk = nullptr;
-        for (const auto& c : registry())
-            if (c.kind == kSingle && c.name == e->side[k]) sk = &c;
-        if (!sk) return fail(BFUSE_ERR_ARG, "fused kernel %s names unknown side %s", e->name.c_str(), e->side[k].c_str());
-        int rc = check_side_fits(sk->func, sides ? sides[k] : k);
+    const Launchable* l = launchable(func);
+    if (!l || l->e->kind == kSingle) return fail(BFUSE_ERR_ARG, "not a fused kernel");
+    for (int k = 0; k < l->n_sides; ++k) {
+        if (!l->side[k]) return fail(BFUSE_ERR_ARG, "fused kernel %s names unknown side %s", l->e->name.c_str(), l->e->side[k].c_str());
+        int rc = check_buffers(*l, k, sides ? sides[k] : k);
         if (rc) return rc;
     }
     return BFUSE_OK;
@@ -1132,15 +1166,14 @@ int bfuse_fill_uniform_device(int side, int tensor, unsigned long long seed, flo
     if (tensor != 0 && tensor != 1) return fail(BFUSE_ERR_ARG, "tensor must be 0 (I) or 1 (F)");
     if (s.elem[tensor] != 4 && s.elem[tensor] != 2)
         return fail(BFUSE_ERR_ARG, "device fill writes fp32 or bf16 tensors, this one has %d-byte elements", s.elem[tensor]);
-    if (int rc = sync_and_check()) return rc;   // nothing launched earlier may still be reading the operand
     const size_t n = s.bytes[tensor] / (size_t)s.elem[tensor];
     size_t blocks = (n + 256 * 8 - 1) / (256 * 8);
     if (blocks > 16384) blocks = 16384;
     if (blocks < 1) blocks = 1;
     g_busy = true;
+    // on the default stream, in order with every launch: nothing has to be waited for
     hipLaunchKernelGGL(fill_uniform_kernel, dim3((unsigned)blocks), dim3(256), 0, nullptr, s.buf[tensor], n, s.elem[tensor], seed, lo, hi);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipDeviceSynchronize());
     return BFUSE_OK;
 }
 
@@ -1156,6 +1189,12 @@ int bfuse_launch(int mode, const void* fa, const unsigned* ga, const unsigned* b
     int rc;
     if ((rc = validate_mode(mode, fa, ga, ba, fb, gb, bb))) return rc;
     return enqueue_mode(mode, fa, ga, ba, fb, gb, bb, nullptr);
+}
+
+int bfuse_launch_packed(const bfuse_launch_args* a)
+{
+    if (!a) return fail(BFUSE_ERR_ARG, "null launch argument");
+    return bfuse_launch(a->mode, a->func_a, a->grid_a, a->block_a, a->func_b, a->grid_b, a->block_b);
 }
 
 int bfuse_time(int mode, const void* fa, const unsigned* ga, const unsigned* ba, const void* fb, const unsigned* gb,

@@ -3,6 +3,8 @@ operation_cu.py:123-256): initialize / run_kernel1 / run_kernel2 / run_parallel 
 finalize over numpy buffers, plus the device-resident launch and GPU-side timing entry points.
 """
 import ctypes as C
+import functools
+import math
 import os
 import weakref
 from dataclasses import dataclass, replace
@@ -74,13 +76,14 @@ def _u3(v):
 _DT = {4: np.float32, 2: np.uint16, 1: np.uint8}
 
 # Results of at least this size are arrays over the library's pinned buffers, which the copy engines write in place
-# (57 GB/s; a new array of pageable memory takes 10-20 GB/s, most of it page faults).  Below, one memcpy out of the
-# library's arena is cheaper than the bookkeeping of a buffer (~5 us).
-PINNED_MIN_BYTES = 512 << 10
+# (57 GB/s; memory that is new with every array takes 10-20 GB/s, most of it page faults).  Smaller ones come from
+# malloc's heap, which is not new, through the staging ring (35-45 GB/s): 32 MiB is the largest piece malloc keeps there,
+# and a program whose results are elsewhere sees it hand the memory of its own arrays back to the system more often.
+PINNED_MIN_BYTES = 32 << 20
 
 
 def _result(shape, dtype) -> np.ndarray:
-    nbytes = int(np.prod(shape)) * np.dtype(dtype).itemsize
+    nbytes = math.prod(shape) * np.dtype(dtype).itemsize
     l = _lib.lib()
     p = l.bfuse_host_buffer(nbytes) if nbytes >= PINNED_MIN_BYTES else None
     if not p:      # small, or the library's limit of pinned memory is in use
@@ -104,6 +107,7 @@ class Operation:
                 raise ValueError(f"{k.name} is a fused kernel; sides must be standalone kernels")
             _lib.check(self.l.bfuse_set_elem_bytes(side, *k.elem_bytes))
         self.shapes = [[_i4(s) for s in k.shapes] for k in self.k]
+        self._prepared = {}       # bfuse_launch_packed with its argument, by mode and fused kernel
         _lib.check(self.l.initialize_kernel1(*self.shapes[0]))
         try:
             _lib.check(self.l.initialize_kernel2(*self.shapes[1]))
@@ -130,7 +134,7 @@ class Operation:
         k = self.k[side]
         dt = _DT[k.elem_bytes[idx]]
         a = np.ascontiguousarray(arr, dtype=dt)
-        want = int(np.prod(k.shapes[idx]))
+        want = math.prod(k.shapes[idx])
         if a.size != want:
             raise ValueError(f"{k.name}: tensor {idx} has {a.size} elements, kernel expects {want}")
         return a
@@ -213,7 +217,7 @@ class Operation:
         """Device-side checksums of the side's output in chunks of `chunk_elems` elements: an array
         [chunks, 2] of uint64 that `checksum_of` reproduces on the host for expected contents."""
         k = self.k[side]
-        total = int(np.prod(k.shapes[2]))
+        total = math.prod(k.shapes[2])
         if chunk_elems < 1 or total % chunk_elems:
             raise ValueError(f"{k.name}: chunks of {chunk_elems} elements do not divide the output's {total}")
         sums = np.zeros((total // chunk_elems, 2), np.uint64)
@@ -237,7 +241,22 @@ class Operation:
         _lib.check(self.l.bfuse_set_sync_spin_limit(kernel.func, polls))
 
     def launch(self, mode: str, fused: Optional[KernelHandle] = None):
-        _lib.check(self.l.bfuse_launch(MODES[mode], *self._mode_args(mode, fused)))
+        # converting the arguments took 2 us of a launch that the runtime makes in 2.4: they are converted once
+        try:
+            call = self._prepared[mode, fused and (fused.func, fused.grid, fused.block)]
+        except KeyError:
+            call = self._prepare_launch(mode, fused)
+        rc = call()
+        if rc:
+            _lib.check(rc)
+
+    def _prepare_launch(self, mode, fused):
+        m = MODES[mode]
+        fa, ga, ba, fb, gb, bb = self._mode_args(mode, fused)
+        args = _lib.LaunchArgsC(m, ga, ba, gb or (0, 0, 0), bb or (0, 0, 0), fa, fb)
+        call = functools.partial(self.l.bfuse_launch_packed, C.cast(C.pointer(args), C.c_void_p))   # the pointer keeps `args` alive
+        self._prepared[mode, fused and (fused.func, fused.grid, fused.block)] = call
+        return call
 
     def synchronize(self):
         _lib.check(self.l.bfuse_synchronize())
@@ -276,6 +295,7 @@ class GroupOperation:
         if not 2 <= len(names) <= _lib.MAXK:
             raise ValueError(f"a group has 2 .. {_lib.MAXK} kernels")
         self.k = [kernel_info(n) for n in names]
+        self._prepared = {}       # launch lists by their kernels and sides, converted once
         self.live_sides = []
         try:
             for side, k in enumerate(self.k, 1):
@@ -310,8 +330,8 @@ class GroupOperation:
         k = self.k[side]
         a = [np.ascontiguousarray(x, dtype=_DT[k.elem_bytes[i]]) for i, x in enumerate((I, F))]
         for i in range(2):
-            if a[i].size != int(np.prod(k.shapes[i])):
-                raise ValueError(f"{k.name}: tensor {i} has {a[i].size} elements, kernel expects {int(np.prod(k.shapes[i]))}")
+            if a[i].size != math.prod(k.shapes[i]):
+                raise ValueError(f"{k.name}: tensor {i} has {a[i].size} elements, kernel expects {math.prod(k.shapes[i])}")
         _lib.check(self.l.bfuse_upload(side + 1, a[0].ctypes.data, a[1].ctypes.data))
 
     def zero_outputs(self):
@@ -326,6 +346,10 @@ class GroupOperation:
 
     def _descs(self, launches):
         """launches: [(KernelHandle, (side, ...)), ...] with 0-based sides; a standalone kernel takes one."""
+        key = tuple((k.func, k.grid, k.block, tuple(sides)) for k, sides in launches)
+        arr = self._prepared.get(key)
+        if arr is not None:
+            return arr
         arr = (_lib.LaunchDescC * len(launches))()
         for d, (k, sides) in zip(arr, launches):
             d.func = k.func
@@ -334,6 +358,7 @@ class GroupOperation:
             d.n_sides = len(sides)
             for i, sd in enumerate(sides):
                 d.sides[i] = sd + 1
+        self._prepared[key] = arr
         return arr
 
     def unfused(self):
@@ -365,7 +390,7 @@ class GenericOperation:
         if not 2 <= len(shapes) <= _lib.MAXK:
             raise ValueError(f"2 .. {_lib.MAXK} sides")
         self.shapes = [[_i4(s) for s in sh] for sh in shapes]
-        self.nelem = [[int(np.prod(s)) for s in sh] for sh in shapes]
+        self.nelem = [[math.prod(s) for s in sh] for sh in shapes]
         self.modules = []
         self.live_sides = []
         try:
