@@ -7,6 +7,7 @@
 #include "ops_ceiling.h"
 #include "ops_conv.h"
 #include "ops_conv_1x1.h"
+#include "ops_conv_tile.h"
 #include "ops_gemm_bf16.h"
 #include "ops_gemm_f32.h"
 #include "ops_gemm_f32_dma.h"
@@ -165,3 +166,19 @@ BFUSE_HFUSE_KERNEL(bgemm_f32_3x48x64x80, GemmS8, bias_relu_4096, BiasReluS)
 BFUSE_KERNEL(selftest_sync_a, SyncProbeA, ({{512, 1, 1, 1}, 4}), ({{512, 1, 1, 1}, 4}), ({{512, 1, 1, 1}, 4}))
 BFUSE_KERNEL(selftest_sync_b, SyncProbeB, ({{768, 1, 1, 1}, 4}), ({{768, 1, 1, 1}, 4}), ({{768, 1, 1, 1}, 4}))
 BFUSE_HFUSE_KERNEL(selftest_sync_a, SyncProbeA, selftest_sync_b, SyncProbeB)
+
+// The shared-tile convolution at the edges of its tiles (found by name only, so that nothing that walks the registry meets
+// them): tiles that run over several images, last tiles past the batch, strides, even and large filters, several channel
+// quads per stage, one stage and many.  <CI, CO, H, W, KH, KW, S, P, BM, 16-pixel blocks, stage channels, images, waves over BM>
+#define CONV_TILE_TEST(TAG, CI, CO, H, W, KH, KW, S, P, BM, PB, CPS, N, WM)                                        \
+    using ConvT_##TAG = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, CPS, N, WM>;                                \
+    BFUSE_KERNEL(selftest_conv_tile_##TAG, ConvT_##TAG, ({{N, CI, H, W}, 4}), ({{CO, CI, KH, KW}, 4}),             \
+                 ({{N, CO, (H - KH + 2 * P) / S + 1, (W - KW + 2 * P) / S + 1}, 4}))
+CONV_TILE_TEST(a, 16, 32, 5, 5, 3, 3, 1, 1, 32, 4, 4, 3, 1)         // 75 pixels of three images in two tiles of 64
+CONV_TILE_TEST(b, 32, 64, 9, 7, 3, 3, 2, 0, 32, 4, 8, 5, 2)         // stride 2, 60 pixels of five images in one tile, two quads a stage
+CONV_TILE_TEST(c, 16, 16, 11, 6, 5, 5, 1, 2, 16, 8, 4, 4, 1)        // 5 x 5, tiles of 128 over images of 66
+CONV_TILE_TEST(d, 16, 64, 20, 13, 3, 3, 4, 1, 64, 4, 4, 9, 2)       // stride 4, one window row per four image rows
+CONV_TILE_TEST(e, 48, 96, 8, 33, 3, 1, 1, 1, 96, 8, 4, 7, 2)        // 3 x 1 filter: an odd number of columns, twelve stages
+BFUSE_HFUSE_KERNEL(selftest_conv_tile_a, ConvT_a, bias_relu_4096, BiasReluS)
+BFUSE_BFUSE_KERNEL(selftest_conv_tile_b, ConvT_b, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
+BFUSE_HFUSE_KERNEL(selftest_conv_tile_c, ConvT_c, conv3x3_f32_32x12x12_32, ConvS2)

@@ -40,7 +40,8 @@ namespace bfuse {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
-template <int CI_, int CO_, int H_, int W_, int KH_, int KW_, int S_, int P_, int BM_, int PB_, int KS_, int NIMG_ = 1>
+// WM_ = 0: this form.  WM_ > 0 (ops_conv_tile.h): large tiles that the waves of a workgroup share.
+template <int CI_, int CO_, int H_, int W_, int KH_, int KW_, int S_, int P_, int BM_, int PB_, int KS_, int NIMG_ = 1, int WM_ = 0>
 struct ConvF32Lds {
     static constexpr bool MATRIX_CORES = true;   // the inner loop is a stream of MFMAs (what the fusion chooser asks)
     static constexpr int CI = CI_, CO = CO_, H = H_, W = W_, KH = KH_, KW = KW_, S = S_, P = P_, BM = BM_, PB = PB_, KS = KS_, NIMG = NIMG_;

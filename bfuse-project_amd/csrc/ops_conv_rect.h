@@ -26,6 +26,7 @@
 #include "dispatch.h"
 #include "ops_conv_1x1.h"
 #include "ops_conv_general.h"
+#include "ops_conv_tile.h"
 #include "wave.h"
 
 namespace bfuse {
@@ -370,7 +371,22 @@ struct ConvTiling {
     static constexpr int RESERVE = RECT && CI < 16 && (int)sizeof(typename staged::Smem) < 163840 / 12 - 1024
                                        ? 163840 / 12 - (int)sizeof(typename staged::Smem) : 0;
     using held = std::conditional_t<(RESERVE > 0), LdsReserve<staged, (RESERVE > 0 ? RESERVE : 1)>, staged>;
-    using type = std::conditional_t<STREAM, Conv1x1F32<CI, CO, H, W, S, stream_bm(), 4, NIMG>, held>;
+    // A batch with enough pixels for two workgroups per CU goes to the shared-tile form, with the largest tile whose
+    // part of each wave is at least twelve 16 x 16 blocks: measured at batch 1024 over the 3 x 3 and 5 x 5 layers it
+    // takes 0.40-0.82 of the time of the per-wave forms above (107-146 TFLOP/s against 52-115); with eight blocks per wave
+    // (32 x 64) 0.97-1.06.  96 channels before 128: 142 against 140 TFLOP/s on 288 -> 384; 64 x 256 pixels, one wave over
+    // the channels, against 64 x 128, two: 142 against 90.
+    static constexpr int tile_bm() { return CO % 96 == 0 ? 96 : CO % 128 == 0 ? 128 : CO % 160 == 0 ? 160 : CO % 64 == 0 ? 64 : CO % 48 == 0 ? 48 : CO % 80 == 0 ? 80 : CO % 32 == 0 ? 32 : 16; }
+    static constexpr int TBM = tile_bm(), TWM = TBM >= 96 ? 2 : 1, TPB = TBM >= 96 ? 8 : TBM >= 48 ? 16 : 32;
+    static constexpr bool tiled()
+    {
+        if constexpr (T > 1 && CI >= 16 && CI % 4 == 0 && KH >= S && TBM >= 32 && (long long)OHW * NIMG >= 512LL * 16 * TPB * TBM / CO)
+            return ConvF32Lds<CI, CO, H, W, KH, KW, S, P, TBM, TPB, 4, NIMG, TWM>::FITS;
+        return false;
+    }
+    template <bool TILED, class Else> struct pick { using type = Else; };
+    template <class Else> struct pick<true, Else> { using type = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, TBM, TPB, 4, NIMG, TWM>; };
+    using type = typename pick<tiled(), std::conditional_t<STREAM, Conv1x1F32<CI, CO, H, W, S, stream_bm(), 4, NIMG>, held>>::type;
 };
 template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int NIMG = 1>
 using ConvF32Auto = typename ConvTiling<CI, CO, H, W, KH, KW, S, P, NIMG>::type;
