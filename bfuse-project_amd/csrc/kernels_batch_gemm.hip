@@ -4,6 +4,7 @@
 #include "fuse.h"
 #include "ops_gemm_f32.h"
 #include "ops_gemm_f32_dma.h"
+#include "ops_gemm_tile.h"
 
 using namespace bfuse;
 
@@ -22,29 +23,30 @@ DENSE_F32(1024, 4096, 14336, 64, 128, 4)
 DENSE_F32(1024, 14336, 4096, 64, 128, 4)
 
 // C[b] = A[b] . B[b]^T, A [b, M, K], B [b, N, K]: <M, N, K, BM, BN, waves over K>
-#define BGEMM_F32(B, M, K, N, BM, BN, KS)                                                                        \
-    using Bgemm_##B##x##M##x##K##x##N = GemmF32<M, N, K, BM, BN, KS, kEpiNone, 2, 1, true, B>;                    \
+// Products whose rows and columns are whole tiles run on shared tiles (GemmTile): 128 x 128 in three buffers of 16 k
+// (1024 products 512 x 64 x 512: 0.46 -> 0.35 ms, 256 x 80 x 256: 0.140 -> 0.116), 256 x 64 with the waves over the rows
+// where there are 64 columns (512 x 512 x 64: 0.39 -> 0.31 ms).
+#define BGEMM_F32_TILE(B, M, K, N, BM, BN, WM, KS, NBUF)                                                         \
+    using Bgemm_##B##x##M##x##K##x##N = GemmTile<M, K, 1, N, 1, B, BM, BN, WM, KS, kRows, NBUF>;                  \
     BFUSE_KERNEL(bgemm_f32_##B##x##M##x##K##x##N, Bgemm_##B##x##M##x##K##x##N, ({{B, M, K, 1}, 4}), ({{B, N, K, 1}, 4}), ({{B, M, N, 1}, 4}))
-// the one-wave products reserve 32 KB of LDS per workgroup: four workgroups per CU, one wave per SIMD (see LdsReserve).
-// (128 x 64 tiles run the K <= 128 products 7-16 % faster alone, but their 300 registers make every kernel they are part
-// of a kernel of one wave per SIMD (GemmF32::MIN_WAVES_PER_EU): block-fused with them, the pairs of the reference's
-// tests/interleave_scheduler suite read 0.79 of the unfused time instead of 0.90.  The operators of a fusion library
-// stay good partners: 64 x 64.)
+// The others keep a tile per wave; the one-wave products reserve 32 KB of LDS per workgroup: four workgroups per CU, one
+// wave per SIMD (see LdsReserve).  (208 rows and columns: shared tiles of 128 would overlap by a quarter, 1.00-1.06x; 80
+// columns are no whole 64-column groups.)
 #define BGEMM_F32_RESERVE(B, M, K, N, BM, BN, KS, BYTES)                                                         \
     using Bgemm_##B##x##M##x##K##x##N = LdsReserve<GemmF32<M, N, K, BM, BN, KS, kEpiNone, 2, 1, true, B>, BYTES>; \
     BFUSE_KERNEL(bgemm_f32_##B##x##M##x##K##x##N, Bgemm_##B##x##M##x##K##x##N, ({{B, M, K, 1}, 4}), ({{B, N, K, 1}, 4}), ({{B, M, N, 1}, 4}))
-BGEMM_F32_RESERVE(1024, 512, 64, 512, 64, 64, 1, 32768)
-BGEMM_F32(1024, 512, 512, 64, 64, 64, 2)
-BGEMM_F32_RESERVE(1024, 512, 128, 512, 64, 64, 1, 32768)
-BGEMM_F32(1024, 512, 512, 128, 64, 64, 2)
-BGEMM_F32_RESERVE(1024, 256, 64, 256, 64, 64, 1, 32768)
-BGEMM_F32_RESERVE(1024, 256, 256, 64, 64, 64, 1, 32768)
-BGEMM_F32_RESERVE(1024, 256, 80, 256, 64, 64, 1, 32768)
+BGEMM_F32_TILE(1024, 512, 64, 512, 128, 128, 2, 16, 3)
+BGEMM_F32_TILE(1024, 512, 512, 64, 256, 64, 4, 32, 2)
+BGEMM_F32_TILE(1024, 512, 128, 512, 128, 128, 2, 16, 3)
+BGEMM_F32_TILE(1024, 512, 512, 128, 128, 128, 2, 16, 3)
+BGEMM_F32_TILE(1024, 256, 64, 256, 128, 128, 2, 16, 3)
+BGEMM_F32_TILE(1024, 256, 256, 64, 256, 64, 4, 32, 2)
+BGEMM_F32_TILE(1024, 256, 80, 256, 128, 128, 2, 16, 3)
 BGEMM_F32_RESERVE(1024, 256, 256, 80, 64, 80, 1, 32768)
 BGEMM_F32_RESERVE(1024, 208, 64, 208, 112, 64, 1, 32768)
 BGEMM_F32_RESERVE(1024, 208, 208, 64, 208, 32, 1, 32768)
 BGEMM_F32_RESERVE(1024, 208, 80, 208, 112, 64, 1, 32768)     // 208 = 112 + 96 rows, 3 x 64 + 16 columns: the last tiles overlap their neighbours
 BGEMM_F32_RESERVE(1024, 208, 208, 80, 64, 80, 1, 32768)
 // tests/interleave_scheduler/config/info.yaml: bgemm_6, bgemm_7
-BGEMM_F32_RESERVE(1024, 1024, 64, 512, 64, 64, 1, 32768)
-BGEMM_F32(1024, 1024, 512, 64, 64, 64, 2)
+BGEMM_F32_TILE(1024, 1024, 64, 512, 128, 128, 2, 16, 3)
+BGEMM_F32_TILE(1024, 1024, 512, 64, 256, 64, 4, 32, 2)

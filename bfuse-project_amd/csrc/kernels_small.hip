@@ -11,6 +11,7 @@
 #include "ops_gemm_bf16.h"
 #include "ops_gemm_f32.h"
 #include "ops_gemm_f32_dma.h"
+#include "ops_gemm_tile.h"
 #include "ops_layout.h"
 #include "ops_pool.h"
 #include "ops_rowwise.h"
@@ -182,3 +183,21 @@ CONV_TILE_TEST(e, 48, 96, 8, 33, 3, 1, 1, 1, 96, 8, 4, 7, 2)        // 3 x 1 fil
 BFUSE_HFUSE_KERNEL(selftest_conv_tile_a, ConvT_a, bias_relu_4096, BiasReluS)
 BFUSE_BFUSE_KERNEL(selftest_conv_tile_b, ConvT_b, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
 BFUSE_HFUSE_KERNEL(selftest_conv_tile_c, ConvT_c, conv3x3_f32_32x12x12_32, ConvS2)
+
+// The shared-tile product likewise: pixels of images that are no whole chunks, tiles over several images and past the batch,
+// strides, row and column tiles that overlap, fewer stages than buffers.
+// <M, K, H, W, S, images or products, BM, BN, waves over BM, k per stage, layout, buffers>
+#define CONV1_TILE_TEST(TAG, CI, CO, H, W, S, N, BM, BN, WM, KS, NBUF)                                              \
+    using GemmT_##TAG = SwapOperands<GemmTile<CO, CI, H, W, S, N, BM, BN, WM, KS, kPix, NBUF>>;                     \
+    BFUSE_KERNEL(selftest_gemm_tile_##TAG, GemmT_##TAG, ({{N, CI, H, W}, 4}), ({{CO, CI, 1, 1}, 4}), ({{N, CO, (H - 1) / S + 1, (W - 1) / S + 1}, 4}))
+#define BGEMM_TILE_TEST(TAG, B, M, K, N, BM, BN, WM, KS, NBUF)                                                     \
+    using GemmT_##TAG = GemmTile<M, K, 1, N, 1, B, BM, BN, WM, KS, kRows, NBUF>;                                   \
+    BFUSE_KERNEL(selftest_gemm_tile_##TAG, GemmT_##TAG, ({{B, M, K, 1}, 4}), ({{B, N, K, 1}, 4}), ({{B, M, N, 1}, 4}))
+CONV1_TILE_TEST(a, 16, 32, 5, 5, 1, 3, 32, 256, 1, 16, 3)        // one stage, three images of 25 pixels in one tile
+CONV1_TILE_TEST(b, 64, 80, 9, 9, 1, 5, 80, 256, 1, 32, 2)        // five images of 81 in two tiles, a row tile that is no whole round of loads
+CONV1_TILE_TEST(c, 48, 112, 9, 7, 2, 11, 96, 128, 2, 16, 3)      // stride 2 (20 pixels an image), row tiles that overlap
+CONV1_TILE_TEST(d, 32, 64, 8, 8, 1, 7, 64, 128, 2, 16, 4)        // fewer stages than buffers, whole chunks
+BGEMM_TILE_TEST(e, 3, 160, 48, 144, 128, 128, 2, 16, 3)          // row and column tiles that overlap
+BGEMM_TILE_TEST(f, 8, 64, 32, 64, 64, 64, 4, 32, 2)              // one stage, products dealt to the XCDs
+BFUSE_HFUSE_KERNEL(selftest_gemm_tile_c, GemmT_c, bias_relu_4096, BiasReluS)
+BFUSE_BFUSE_KERNEL(selftest_gemm_tile_e, GemmT_e, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)

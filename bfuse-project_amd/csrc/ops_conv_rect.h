@@ -27,6 +27,7 @@
 #include "ops_conv_1x1.h"
 #include "ops_conv_general.h"
 #include "ops_conv_tile.h"
+#include "ops_gemm_tile.h"
 #include "wave.h"
 
 namespace bfuse {
@@ -384,9 +385,16 @@ struct ConvTiling {
             return ConvF32Lds<CI, CO, H, W, KH, KW, S, P, TBM, TPB, 4, NIMG, TWM>::FITS;
         return false;
     }
-    template <bool TILED, class Else> struct pick { using type = Else; };
-    template <class Else> struct pick<true, Else> { using type = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, TBM, TPB, 4, NIMG, TWM>; };
-    using type = typename pick<tiled(), std::conditional_t<STREAM, Conv1x1F32<CI, CO, H, W, S, stream_bm(), 4, NIMG>, held>>::type;
+    // 1 x 1 filters likewise, as a matrix product (GemmTile): 1.02-1.28x of the streamed form at stride 1 (126-142 TFLOP/s on the
+    // layers of 768 and more channels, 4.0-5.1 TB/s on those of few), 1.4-1.9x at stride 2, where that one reads element
+    // by element.  Three buffers of 16 channels for 128-pixel tiles (134 against 124 TFLOP/s with two of 32 on 768 -> 192),
+    // two for 256-pixel ones, which are bound by memory and want more workgroups per CU.
+    static constexpr int GBM = CO % 96 != 0 && CO % 224 == 0 ? 224 : TBM, GWM = GBM >= 96 ? 2 : 1, GBN = GBM >= 96 ? 128 : 256;
+    static constexpr bool PRODUCT = T == 1 && P == 0 && CI % 16 == 0 && TBM >= 32 && (long long)((OHW + 3) / 4 * 4) * NIMG / GBN * (CO / GBM) >= 512;
+    template <int FORM, class Else> struct pick { using type = Else; };
+    template <class Else> struct pick<1, Else> { using type = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, TBM, TPB, 4, NIMG, TWM>; };
+    template <class Else> struct pick<2, Else> { using type = SwapOperands<GemmTile<CO, CI, H, W, S, NIMG, GBM, GBN, GWM, 16, kPix, GWM == 2 ? 3 : 2>>; };
+    using type = typename pick<PRODUCT ? 2 : tiled() ? 1 : 0, std::conditional_t<STREAM, Conv1x1F32<CI, CO, H, W, S, stream_bm(), 4, NIMG>, held>>::type;
 };
 template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int NIMG = 1>
 using ConvF32Auto = typename ConvTiling<CI, CO, H, W, KH, KW, S, P, NIMG>::type;

@@ -1,4 +1,5 @@
-"""The shared-tile convolution (csrc/ops_conv_tile.h) at the edges of its tiles, against the CPU oracle, alone and fused."""
+"""The shared-tile convolution and product (csrc/ops_conv_tile.h, ops_gemm_tile.h) at the edges of their tiles, against the
+CPU oracle (products: numpy in double), alone and fused."""
 import numpy as np
 import pytest
 
@@ -10,11 +11,8 @@ from tests import oracle_cases
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("tag,s,p,partner,kind,suffix", [
-    ("a", 1, 1, "bias_relu_4096", "hfuse", ""), ("b", 2, 0, "layernorm_8x256", "bfuse", "_c4"),
-    ("c", 1, 2, "conv3x3_f32_32x12x12_32", "hfuse", ""), ("d", 4, 1, "bias_relu_4096", None, ""), ("e", 1, 1, "bias_relu_4096", None, "")])
-def test_shared_tile_convolution_against_the_oracle_and_fused(tag, s, p, partner, kind, suffix):
-    with bf.Operation(f"selftest_conv_tile_{tag}", partner) as op:
+def _check(name, reference, partner, kind, suffix):
+    with bf.Operation(name, partner) as op:
         k, q = op.k
         x, w = fill_normal(3, int(np.prod(k.shapes[0])), 0, 1), fill_normal(4, int(np.prod(k.shapes[1])), 0, 0.1)
         x2, w2 = fill_normal(5, int(np.prod(q.shapes[0])), 0, 1), fill_normal(6, int(np.prod(q.shapes[1])), 0, 1)
@@ -23,10 +21,30 @@ def test_shared_tile_convolution_against_the_oracle_and_fused(tag, s, p, partner
         op.zero_outputs()
         op.launch("serial")
         y, y2 = op.download(0), op.download(1)
-        want = orf.conv2d(x.reshape(k.shapes[0]), w.reshape(k.shapes[1]), s=s, p=p)
-        assert y.shape == want.shape
+        want = reference(x.reshape(k.shapes[0]), w.reshape(k.shapes[1]))
+        assert y.size == want.size
         assert oracle_cases.rel_error(y.ravel(), want.ravel()) <= 1e-5
         if kind:
             op.zero_outputs()
             op.launch(kind, op.fused(kind, suffix))
             assert np.array_equal(op.download(0).view(np.uint32), y.view(np.uint32)) and np.array_equal(op.download(1).view(np.uint32), y2.view(np.uint32))
+
+
+@pytest.mark.parametrize("tag,s,p,partner,kind,suffix", [
+    ("a", 1, 1, "bias_relu_4096", "hfuse", ""), ("b", 2, 0, "layernorm_8x256", "bfuse", "_c4"),
+    ("c", 1, 2, "conv3x3_f32_32x12x12_32", "hfuse", ""), ("d", 4, 1, "bias_relu_4096", None, ""), ("e", 1, 1, "bias_relu_4096", None, "")])
+def test_shared_tile_convolution_against_the_oracle_and_fused(tag, s, p, partner, kind, suffix):
+    _check(f"selftest_conv_tile_{tag}", lambda x, w: orf.conv2d(x, w, s=s, p=p), partner, kind, suffix)
+
+
+@pytest.mark.parametrize("tag,s,partner,kind,suffix", [
+    ("a", 1, "bias_relu_4096", None, ""), ("b", 1, "bias_relu_4096", None, ""), ("c", 2, "bias_relu_4096", "hfuse", ""), ("d", 1, "bias_relu_4096", None, "")])
+def test_shared_tile_1x1_convolution_against_the_oracle_and_fused(tag, s, partner, kind, suffix):
+    _check(f"selftest_gemm_tile_{tag}", lambda x, w: orf.conv2d(x, w, s=s, p=0), partner, kind, suffix)
+
+
+@pytest.mark.parametrize("tag,partner,kind,suffix", [("e", "layernorm_8x256", "bfuse", "_c4"), ("f", "bias_relu_4096", None, "")])
+def test_shared_tile_batched_product_against_numpy_and_fused(tag, partner, kind, suffix):
+    def product(a, b):
+        return np.matmul(a[..., 0].astype(np.float64), b[..., 0].astype(np.float64).transpose(0, 2, 1)).astype(np.float32)
+    _check(f"selftest_gemm_tile_{tag}", product, partner, kind, suffix)
