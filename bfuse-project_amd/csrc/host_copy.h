@@ -9,8 +9,9 @@
 //     into a pinned arena by the calling thread and moved by ONE kernel launch over all tensors of the call
 //     (one launch, ~3 us of GPU time + the bytes, whatever the number of tensors);
 //   * anything larger goes through a ring of pinned slots: worker threads fill (or drain) slots while copy kernels move
-//     the ones that are ready, alternating between two streams so that one starts under the other's end (1 MiB chunks:
-//     56 GB/s; one stream 44, a copy engine 38);
+//     the ones that are ready, alternating between two streams so that one starts under the other's end, and report
+//     the end of a copy by a word in host memory (128 MB: 56 GB/s up, 53 down; with an event behind every copy 46 and
+//     47, with a copy engine 38);
 //   * host memory that came from host_buffer() is pinned and copied in place, with no slot and no thread in between.
 // run_fuse over 0.3 MB: 111 -> 56 us; run_parallel over 600 MB: 36 -> 10.4 ms (the link's floor: 6.4 up + what of the 4.4
 // down is not under it).  up() returns with the copied bytes on their way into place before anything launched later;
@@ -66,13 +67,47 @@ static __global__ __launch_bounds__(256) void copy_segments(SegList l)
     }
 }
 
+// One chunk of a long transfer.  Every block reports for itself: once its part is in place, whoever reads it next (the
+// host, or a kernel launched from now on), it writes `value` to its word of `flag`, which is host memory.  An event
+// would tell the same, but recording one holds the stream's next kernel up for 5 us and the host for 3.  Four words are
+// in flight per thread: fewer, fatter blocks keep the link as full and leave it less to switch between (128 MB up: 56
+// GB/s with 8 blocks, 53 with 16, 50 with 32, 45 with 64; down it is the other way round, 52, 53, 53, 54).
+static __global__ __launch_bounds__(256) void copy_chunk(const unsigned char* src, unsigned char* dst, size_t bytes, unsigned* flag, unsigned value)
+{
+    const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x, nt = (size_t)gridDim.x * 256;
+    const bool aligned = (((uintptr_t)src | (uintptr_t)dst) & 15) == 0;
+    const size_t words = aligned ? bytes / 16 : 0;
+    const uint4* const s = reinterpret_cast<const uint4*>(src);
+    uint4* const d = reinterpret_cast<uint4*>(dst);
+    size_t i = t;
+    for (; i + 3 * nt < words; i += 4 * nt) {
+        const uint4 a = s[i], b = s[i + nt], c = s[i + 2 * nt], e = s[i + 3 * nt];
+        d[i] = a;
+        d[i + nt] = b;
+        d[i + 2 * nt] = c;
+        d[i + 3 * nt] = e;
+    }
+    for (; i < words; i += nt) d[i] = s[i];
+    for (i = words * 16 + t; i < bytes; i += nt) dst[i] = src[i];
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // each wave's own stores have left it; the barrier alone does not wait for them
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __threadfence_system();
+        __hip_atomic_store(flag + blockIdx.x, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 class HostCopy {
 public:
     static constexpr size_t kSmallBytes = 512 << 10;
     static constexpr size_t kArenaBytes = 2 << 20;          // per direction
     static constexpr size_t kChunk = 2 << 20;               // a slot, at most one copy: 37 us of link time, long against a copy's start
-    static constexpr size_t kPiece = 256 << 10;             // what a thread moves at a time
+    static constexpr size_t kFirst = 256 << 10;             // the first copy of a transfer up, the last of one down
+    static constexpr size_t kPiece = 64 << 10;              // what a thread moves at a time: the first copy waits for four of them at once
     static constexpr int kSlots = 8;                        // 16 MiB
+    static constexpr int kUpBlocks = 8, kDownBlocks = 16;   // of copy_chunk
+    static constexpr int kFlagWords = 16;                   // a cache line of one word per block
+    static constexpr unsigned kQuietSpins = 100000;
     static constexpr int kMaxWorkers = 6;                   // six threads copy 98 GB/s into pinned memory, four 76, one 31
     static constexpr size_t kIdleLimit = 1ull << 30;        // pinned result buffers kept for the next result
     static constexpr size_t kTotalLimit = 4ull << 30;       // pinned result buffers in existence
@@ -136,7 +171,11 @@ public:
     }
 
     // The device has been synchronised: nothing reads or writes the arenas any more.
-    void quiesced() { in_.used = out_.used = 0; }
+    void quiesced()
+    {
+        in_.used = out_.used = 0;
+        unwaited_ = 0;
+    }
 
     // Pinned host memory for results: copied into by the engines themselves.  A released buffer is kept for the next
     // request of its size (up to kIdleLimit bytes in all): pinning costs ~0.2 ms per MB.  nullptr: over the limit.
@@ -184,9 +223,8 @@ public:
         }
         if (device_ < 0) return;
         stop_workers();
-        for (auto& ev : done_) (void)hipEventDestroy(ev);
         for (auto& s : stream_) (void)hipStreamDestroy(s);
-        for (void* p : {(void*)ring_, (void*)in_.base, (void*)out_.base}) (void)hipHostFree(p);
+        for (void* p : {(void*)ring_, (void*)in_.base, (void*)out_.base, (void*)flag_}) (void)hipHostFree(p);
         ring_ = nullptr;
         device_ = -1;
     }
@@ -207,9 +245,9 @@ private:
         hipError_t e = hipGetDevice(&dev);
         if (e != hipSuccess || dev == device_) return e;
         if (!ring_) {
-            void* p[3] = {};
-            const size_t size[3] = {kChunk * kSlots, kArenaBytes, kArenaBytes};
-            for (int i = 0; i < 3; ++i)
+            void* p[4] = {};
+            const size_t size[4] = {kChunk * kSlots, kArenaBytes, kArenaBytes, kSlots * kFlagWords * sizeof(unsigned)};
+            for (int i = 0; i < 4; ++i)
                 if ((e = hipHostMalloc(&p[i], size[i], hipHostMallocPortable)) != hipSuccess) {
                     for (int j = 0; j < i; ++j) (void)hipHostFree(p[j]);
                     return e;
@@ -217,17 +255,16 @@ private:
             ring_ = static_cast<unsigned char*>(p[0]);
             in_ = {static_cast<unsigned char*>(p[1]), 0};
             out_ = {static_cast<unsigned char*>(p[2]), 0};
+            flag_ = static_cast<unsigned*>(p[3]);
+            memset(flag_, 0, size[3]);
             start_workers();
         }
-        if (device_ >= 0) {   // another device was selected: streams and events belong to one
-            for (auto& ev : done_) (void)hipEventDestroy(ev);
+        if (device_ >= 0) {   // another device was selected: streams belong to one
             for (auto& s : stream_) (void)hipStreamDestroy(s);
             device_ = -1;
         }
         for (auto& s : stream_)
             if ((e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking)) != hipSuccess) return e;
-        for (auto& ev : done_)
-            if ((e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return e;
         device_ = dev;
         return hipSuccess;
     }
@@ -287,19 +324,28 @@ private:
     {
         std::vector<Chunk> chunks;
         long pieces = 0;
-        // half slots for a few MB, where the first chunk's way through the host shows (5 MB: 145 against 166 us);
-        // whole ones, with fewer starts, for more (10 MB: 260 against 300 us)
-        size_t total = 0;
-        for (int i = 0; i < n; ++i) total += seg[i].bytes;
-        const size_t chunk = total <= (8 << 20) ? kChunk / 2 : kChunk;
+        size_t rest = 0;
+        for (int i = 0; i < n; ++i) rest += seg[i].bytes;
+        // Up, the first chunk's way through the host is time in which nothing is on the link; down, the last one's:
+        // sizes double from kFirst, or halve to it (5 MB: 118 us up and 117 down against 152 and 136 in whole slots)
+        size_t ramp = kFirst;
         hipError_t e = hipSuccess;
+        bool wait = false;
         for (int i = 0; i < n; ++i) {
             if (up && pinned(seg[i].host, seg[i].bytes)) {
                 if ((e = hipMemcpyAsync(seg[i].dev, seg[i].host, seg[i].bytes, hipMemcpyHostToDevice, stream_[0])) != hipSuccess) return e;
+                wait = true;
                 continue;
             }
-            for (size_t o = 0; o < seg[i].bytes; o += chunk) {
-                chunks.push_back({static_cast<unsigned char*>(seg[i].dev) + o, static_cast<unsigned char*>(seg[i].host) + o, std::min(chunk, seg[i].bytes - o), pieces});
+            for (size_t o = 0, size; o < seg[i].bytes; o += size, rest -= size) {
+                if (up) {
+                    size = ramp;
+                    ramp = std::min(kChunk, 2 * ramp);
+                } else {
+                    size = std::min(kChunk, std::max(kFirst, (rest / 2 + kPiece - 1) / kPiece * kPiece));
+                }
+                size = std::min(size, seg[i].bytes - o);
+                chunks.push_back({static_cast<unsigned char*>(seg[i].dev) + o, static_cast<unsigned char*>(seg[i].host) + o, size, pieces});
                 pieces += chunks.back().pieces();
             }
         }
@@ -307,6 +353,8 @@ private:
         if (count) {
             begin_job(chunks, up);
             long sent = 0, ended = 0;          // copies enqueued / known to have ended
+            const unsigned base = value_;
+            value_ += (unsigned)count;
             unsigned spins = 0;
             while (ended < count && e == hipSuccess) {
                 const int slot = (int)(sent % kSlots);
@@ -315,15 +363,15 @@ private:
                     const Chunk& c = chunks[(size_t)sent];
                     if (!up) left_[slot].store(c.pieces(), std::memory_order_relaxed);
                     unsigned char* const s = ring_ + slot * kChunk;
-                    e = send(up ? s : c.dev, up ? c.dev : s, c.bytes, stream_[sent & 1]);
-                    if (e == hipSuccess) e = hipEventRecord(done_[slot], stream_[sent & 1]);
+                    hipLaunchKernelGGL(copy_chunk, dim3(up ? kUpBlocks : kDownBlocks), dim3(256), 0, stream_[sent & 1], up ? s : c.dev, up ? c.dev : s, c.bytes, flag_ + slot * kFlagWords,
+                                       base + (unsigned)sent);
+                    e = hipGetLastError();
                     ++sent;
                     spins = 0;
                     continue;
                 }
                 if (ended < sent) {
-                    const hipError_t q = hipEventQuery(done_[ended % kSlots]);
-                    if (q == hipSuccess) {
+                    if (landed((int)(ended % kSlots), up ? kUpBlocks : kDownBlocks, base + (unsigned)ended)) {
                         // up: the slot takes the chunk kSlots further on.  down: the chunk can be drained
                         const long i = up ? ended + kSlots : ended;
                         if (up && i < count) left_[ended % kSlots].store(chunks[(size_t)i].pieces(), std::memory_order_relaxed);
@@ -332,32 +380,41 @@ private:
                         spins = 0;
                         continue;
                     }
-                    if (q != hipErrorNotReady) e = q;
+                    // a copy that failed reports nothing: its stream says so, or says that it has nothing left to do
+                    if (spins > kQuietSpins) {
+                        const hipError_t q = hipStreamQuery(stream_[ended & 1]);
+                        if (q == hipSuccess && !landed((int)(ended % kSlots), up ? kUpBlocks : kDownBlocks, base + (unsigned)ended)) e = hipErrorUnknown;
+                        else if (q != hipSuccess && q != hipErrorNotReady) e = q;
+                        spins = 0;
+                    }
                 }
                 if (!work()) pause(spins);
             }
             end_job();
+            unwaited_ += count;
         }
-        for (auto& s : stream_) {
-            const hipError_t q = hipStreamSynchronize(s);
-            if (e == hipSuccess) e = q;
+        // The flags have said that everything is in place; the runtime, which keeps its record of a launch until the
+        // stream is waited for, is told now and then (a caller may upload for ever without synchronising).
+        if (wait || e != hipSuccess || unwaited_ > 1024) {
+            for (auto& s : stream_) {
+                const hipError_t q = hipStreamSynchronize(s);
+                if (e == hipSuccess) e = q;
+            }
+            unwaited_ = 0;
         }
         return e;
     }
 
+    // whether all blocks of the copy in this slot have reported
+    bool landed(int slot, int blocks, unsigned value) const
+    {
+        for (int b = 0; b < blocks; ++b)
+            if (__atomic_load_n(flag_ + slot * kFlagWords + b, __ATOMIC_ACQUIRE) != value) return false;
+        return true;
+    }
+
     // whether every piece of chunk i, which is or was the last in its slot, has been moved
     bool done(long i) const { return left_[i % kSlots].load(std::memory_order_acquire) == 0; }
-
-    // One copy of the ring: by a kernel, which starts sooner behind its predecessor than a copy engine does (1 MiB chunks,
-    // 128 MB: 48 against 46 GB/s up, 46 against 39 down); 32 workgroups fill the link and leave the chip to others.
-    static hipError_t send(const unsigned char* src, unsigned char* dst, size_t bytes, hipStream_t stream)
-    {
-        SegList l{};
-        l.n = 1;
-        l.s[0] = {src, dst, bytes};
-        hipLaunchKernelGGL(copy_segments, dim3(32), dim3(256), 0, stream, l);
-        return hipGetLastError();
-    }
 
     void begin_job(const std::vector<Chunk>& c, bool up)
     {
@@ -487,7 +544,9 @@ private:
     unsigned char* ring_ = nullptr;
     Arena in_, out_;
     hipStream_t stream_[2] = {};
-    hipEvent_t done_[kSlots] = {};
+    unsigned* flag_ = nullptr;           // kFlagWords of every slot
+    unsigned value_ = 1;                 // what the next copy reports
+    long unwaited_ = 0;                  // copies since the streams, or the device, were last waited for
 
     std::mutex job_;
     std::condition_variable work_cv_, idle_cv_;

@@ -19,7 +19,7 @@ def op():
         yield o
 
 
-@pytest.mark.parametrize("offset,count", [(0, 1), (3, 5), (1, SMALL), (0, SMALL + 1), (7, PIECE * 5 + 3), (0, 4 * CHUNK), (2, 4 * CHUNK + 1),
+@pytest.mark.parametrize("offset,count", [(0, 1), (3, 5), (1, SMALL), (0, SMALL + 1), (7, PIECE * 5 + 3), (0, 3 * PIECE), (4, 7 * PIECE + 1), (0, 4 * CHUNK), (2, 4 * CHUNK + 1),
                                           (0, RING), (5, RING + CHUNK + 1), (0, N)])
 def test_a_part_goes_up_and_comes_back_unchanged(op, offset, count):
     rng = np.random.default_rng(count)
@@ -35,6 +35,15 @@ def test_a_part_goes_up_and_comes_back_unchanged(op, offset, count):
     assert np.array_equal(pageable.view(np.uint32), x.view(np.uint32))
     rest = op.download_part(0, 0, zero.size)
     assert not rest[:offset].any() and not rest[offset + count:].any()
+
+
+def test_the_last_of_many_uploads_without_a_wait_is_what_stands(op):
+    count = SMALL + PIECE + 1
+    for k in range(700):
+        x = np.full(count, k, np.float32)
+        op.upload_part(0, 0, 0, x)
+    op.launch("kernel1")
+    assert np.array_equal(op.download_part(0, 0, count), x)
 
 
 def test_results_are_the_callers_own_and_may_be_operands(op):
