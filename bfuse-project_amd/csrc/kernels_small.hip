@@ -180,6 +180,8 @@ CONV_TILE_TEST(b, 32, 64, 9, 7, 3, 3, 2, 0, 32, 4, 8, 5, 2)         // stride 2,
 CONV_TILE_TEST(c, 16, 16, 11, 6, 5, 5, 1, 2, 16, 8, 4, 4, 1)        // 5 x 5, tiles of 128 over images of 66
 CONV_TILE_TEST(d, 16, 64, 20, 13, 3, 3, 4, 1, 64, 4, 4, 9, 2)       // stride 4, one window row per four image rows
 CONV_TILE_TEST(e, 48, 96, 8, 33, 3, 1, 1, 1, 96, 8, 4, 7, 2)        // 3 x 1 filter: an odd number of columns, twelve stages
+CONV_TILE_TEST(f, 16, 128, 7, 7, 3, 3, 1, 1, 128, 10, 4, 5, 2)      // 245 pixels in two tiles of 160, five blocks a wave
+CONV_TILE_TEST(g, 20, 48, 11, 11, 3, 3, 1, 1, 48, 20, 4, 3, 1)      // 363 pixels in two tiles of 320, an odd number of stages
 BFUSE_HFUSE_KERNEL(selftest_conv_tile_a, ConvT_a, bias_relu_4096, BiasReluS)
 BFUSE_BFUSE_KERNEL(selftest_conv_tile_b, ConvT_b, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
 BFUSE_HFUSE_KERNEL(selftest_conv_tile_c, ConvT_c, conv3x3_f32_32x12x12_32, ConvS2)

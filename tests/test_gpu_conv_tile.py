@@ -32,7 +32,8 @@ def _check(name, reference, partner, kind, suffix):
 
 @pytest.mark.parametrize("tag,s,p,partner,kind,suffix", [
     ("a", 1, 1, "bias_relu_4096", "hfuse", ""), ("b", 2, 0, "layernorm_8x256", "bfuse", "_c4"),
-    ("c", 1, 2, "conv3x3_f32_32x12x12_32", "hfuse", ""), ("d", 4, 1, "bias_relu_4096", None, ""), ("e", 1, 1, "bias_relu_4096", None, "")])
+    ("c", 1, 2, "conv3x3_f32_32x12x12_32", "hfuse", ""), ("d", 4, 1, "bias_relu_4096", None, ""), ("e", 1, 1, "bias_relu_4096", None, ""),
+    ("f", 1, 1, "bias_relu_4096", None, ""), ("g", 1, 1, "bias_relu_4096", None, "")])
 def test_shared_tile_convolution_against_the_oracle_and_fused(tag, s, p, partner, kind, suffix):
     _check(f"selftest_conv_tile_{tag}", lambda x, w: orf.conv2d(x, w, s=s, p=p), partner, kind, suffix)
 
