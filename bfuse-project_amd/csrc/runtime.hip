@@ -90,16 +90,61 @@ size_t shape_bytes(const int* s, int elem)
     return (size_t)s[0] * s[1] * s[2] * s[3] * (size_t)elem;
 }
 
-// device memory and events that an early return must not leak
+// device memory that an early return must not leak
 struct DevBuf {
     void* p = nullptr;
     ~DevBuf() { if (p) (void)hipFree(p); }
     template <class T> T* as() const { return static_cast<T*>(p); }
 };
+// Timing events that nobody uses at the moment: a timed repetition takes two to four, and creating and destroying one
+// costs 0.7 us.  Up to kMost of them are kept, all of one device, until bfuse_shutdown.
+class EventPool {
+public:
+    hipError_t take(hipEvent_t* e)
+    {
+        int dev = 0;
+        const hipError_t rc = hipGetDevice(&dev);
+        if (rc != hipSuccess) return rc;
+        std::lock_guard<std::mutex> lock(m_);
+        if (dev != device_) drop();
+        device_ = dev;
+        if (idle_.empty()) return hipEventCreate(e);
+        *e = idle_.back();
+        idle_.pop_back();
+        return hipSuccess;
+    }
+    void give(hipEvent_t e)
+    {
+        int dev = 0;
+        std::lock_guard<std::mutex> lock(m_);
+        if (hipGetDevice(&dev) == hipSuccess && dev == device_ && idle_.size() < kMost) idle_.push_back(e);
+        else (void)hipEventDestroy(e);
+    }
+    void clear()
+    {
+        std::lock_guard<std::mutex> lock(m_);
+        drop();
+    }
+
+private:
+    static constexpr size_t kMost = 512;
+    void drop()
+    {
+        for (auto e : idle_) (void)hipEventDestroy(e);
+        idle_.clear();
+    }
+    std::mutex m_;
+    std::vector<hipEvent_t> idle_;
+    int device_ = -1;
+};
+EventPool g_events;
+
+// The timing events of one call: taken one by one, given back when it ends.
 struct EventList {
     std::vector<hipEvent_t> v;
     explicit EventList(size_t n) : v(n, nullptr) {}
-    ~EventList() { for (auto e : v) if (e) (void)hipEventDestroy(e); }
+    ~EventList() { for (auto e : v) if (e) g_events.give(e); }
+    hipError_t create(size_t i) { return g_events.take(&v[i]); }
 };
 
 // Fused kernels launched since the last synchronisation whose side barriers can give up, and code
@@ -526,6 +571,7 @@ int bfuse_shutdown(void)
             if (rc2) return rc2;
         }
     HostCopy::get().close();
+    g_events.clear();
     for (auto& m : modules())
         if (m) {
             HIP_TRY(hipModuleUnload(m));
@@ -1211,14 +1257,18 @@ int bfuse_time(int mode, const void* fa, const unsigned* ga, const unsigned* ba,
     std::vector<hipEvent_t>& ev = evl.v;
     const int per = two ? 4 : 2;
     for (int r = 0; r < reps; ++r)
-        for (int j = 0; j < per; ++j) HIP_TRY(hipEventCreate(&ev[(size_t)r * 4 + j]));
+        for (int j = 0; j < per; ++j) HIP_TRY(evl.create((size_t)r * 4 + j));
     for (int r = 0; r < reps; ++r) {
         if ((rc = enqueue_mode(mode, fa, ga, ba, fb, gb, bb, &ev[(size_t)r * 4]))) return rc;
         // Two streams run ahead of each other: without a meeting point per repetition the short
         // kernel's stream would be hundreds of launches ahead and "first start -> last end" of
         // repetition r would span all of them.  The reference synchronises after every run_parallel
-        // (operation_cu.py:199-228).
-        if (mode == BFUSE_MODE_PARALLEL) HIP_TRY(hipDeviceSynchronize());
+        // (operation_cu.py:199-228).  The two ends are waited for, not the device with its other streams: 39 us a
+        // repetition instead of 56.
+        if (mode == BFUSE_MODE_PARALLEL) {
+            HIP_TRY(hipEventSynchronize(ev[(size_t)r * 4 + 1]));
+            HIP_TRY(hipEventSynchronize(ev[(size_t)r * 4 + 3]));
+        }
     }
     if ((rc = sync_and_check())) return rc;
     for (int r = 0; r < reps; ++r) {
@@ -1255,8 +1305,8 @@ int bfuse_time_batched(int mode, const void* fa, const unsigned* ga, const unsig
     HIP_TRY(hipDeviceSynchronize());
     EventList evl(2);
     hipEvent_t &e0 = evl.v[0], &e1 = evl.v[1];
-    HIP_TRY(hipEventCreate(&e0));
-    HIP_TRY(hipEventCreate(&e1));
+    HIP_TRY(evl.create(0));
+    HIP_TRY(evl.create(1));
     HIP_TRY(hipEventRecord(e0, nullptr));
     for (int r = 0; r < reps; ++r)
         if ((rc = enqueue_mode(mode, fa, ga, ba, fb, gb, bb, nullptr))) return rc;
@@ -1310,9 +1360,13 @@ int bfuse_time_graph(int mode, const void* fa, const unsigned* ga, const unsigne
     if ((rc = sync_and_check())) return rc;   // nothing of an earlier launch is pending when the capture starts
     hipStream_t s0 = g.side[mode == BFUSE_MODE_KERNEL2 ? 1 : 0].stream, s1 = g.side[1].stream;   // the legacy stream cannot be captured
     if (!s0 || (mode == BFUSE_MODE_PARALLEL && !s1)) return fail(BFUSE_ERR_STATE, "the side has no stream: initialize_kernel first");
-    EventList evl(4);
-    for (int i = 0; i < 2; ++i) HIP_TRY(hipEventCreateWithFlags(&evl.v[i], hipEventDisableTiming));   // fork, join
-    for (int i = 2; i < 4; ++i) HIP_TRY(hipEventCreate(&evl.v[i]));
+    EventList evl(2);
+    for (int i = 0; i < 2; ++i) HIP_TRY(evl.create(i));
+    struct Joints {   // fork and join: events that a capture has seen go into no pool
+        hipEvent_t v[2] = {};
+        ~Joints() { for (auto e : v) if (e) (void)hipEventDestroy(e); }
+    } joints;
+    for (auto& e : joints.v) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     struct Graph {
         hipGraph_t g = nullptr;
         hipGraphExec_t x = nullptr;
@@ -1323,19 +1377,19 @@ int bfuse_time_graph(int mode, const void* fa, const unsigned* ga, const unsigne
         }
     } gr;
     HIP_TRY(hipStreamBeginCapture(s0, hipStreamCaptureModeThreadLocal));
-    for (int c = 0; c < chain && rc == BFUSE_OK; ++c) rc = capture_mode(mode, fa, ga, ba, fb, gb, bb, s0, s1, evl.v[0], evl.v[1]);
+    for (int c = 0; c < chain && rc == BFUSE_OK; ++c) rc = capture_mode(mode, fa, ga, ba, fb, gb, bb, s0, s1, joints.v[0], joints.v[1]);
     const hipError_t ended = hipStreamEndCapture(s0, &gr.g);   // always: the stream must leave capture mode
     if (rc) return rc;
     HIP_TRY(ended);
     HIP_TRY(hipGraphInstantiate(&gr.x, gr.g, nullptr, nullptr, 0));
     HIP_TRY(hipGraphLaunch(gr.x, s0));
     if ((rc = sync_and_check())) return rc;
-    HIP_TRY(hipEventRecord(evl.v[2], s0));
+    HIP_TRY(hipEventRecord(evl.v[0], s0));
     for (int r = 0; r < reps; ++r) HIP_TRY(hipGraphLaunch(gr.x, s0));
-    HIP_TRY(hipEventRecord(evl.v[3], s0));
+    HIP_TRY(hipEventRecord(evl.v[1], s0));
     if ((rc = sync_and_check())) return rc;
     float ms = 0.f;
-    HIP_TRY(hipEventElapsedTime(&ms, evl.v[2], evl.v[3]));
+    HIP_TRY(hipEventElapsedTime(&ms, evl.v[0], evl.v[1]));
     *us_per_repetition = ms * 1000.f / ((float)reps * (float)chain);
     return BFUSE_OK;
 }
@@ -1397,7 +1451,7 @@ int bfuse_time_list(int n, const bfuse_launch_desc* launches, int warmup, int re
     HIP_TRY(hipDeviceSynchronize());
     if (us_each) {
         EventList evl((size_t)reps * 2 * n);
-        for (auto& e : evl.v) HIP_TRY(hipEventCreate(&e));
+        for (size_t i = 0; i < evl.v.size(); ++i) HIP_TRY(evl.create(i));
         for (int r = 0; r < reps; ++r)
             if ((rc = enqueue_list(n, launches, &evl.v[(size_t)r * 2 * n]))) return rc;
         if ((rc = sync_and_check())) return rc;
@@ -1413,8 +1467,8 @@ int bfuse_time_list(int n, const bfuse_launch_desc* launches, int warmup, int re
     }
     if (us_queued) {
         EventList evl(2);
-        HIP_TRY(hipEventCreate(&evl.v[0]));
-        HIP_TRY(hipEventCreate(&evl.v[1]));
+        HIP_TRY(evl.create(0));
+        HIP_TRY(evl.create(1));
         HIP_TRY(hipEventRecord(evl.v[0], nullptr));
         for (int r = 0; r < reps; ++r)
             if ((rc = enqueue_list(n, launches, nullptr))) return rc;
@@ -1495,8 +1549,8 @@ int bfuse_module_launch(int id, const char* name, const unsigned* grid, const un
     EventList evl(2);
     hipEvent_t &e0 = evl.v[0], &e1 = evl.v[1];
     if (us_out) {
-        HIP_TRY(hipEventCreate(&e0));
-        HIP_TRY(hipEventCreate(&e1));
+        HIP_TRY(evl.create(0));
+        HIP_TRY(evl.create(1));
     }
     bool known = false;
     for (int m : g_pending_modules) known = known || m == id;
