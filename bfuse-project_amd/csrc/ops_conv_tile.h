@@ -80,10 +80,11 @@ struct ConvF32Tile {
     static constexpr int NLB = (NPOS + 63) / 64;                     // wave-level loads per plane
     static constexpr int PLANE = NLB * 64;                            // words
     __host__ __device__ static constexpr int plane_bank(int q) { return S == 1 ? 16 * q : S == 2 ? 32 * (q / 2) + q % 2 : q; }
+    static constexpr int QUAD = 4 * PLANE + 64;                       // words of four planes: the last one's end is past the next quad's start otherwise
     static constexpr int A_CHUNKS = BM * CPS * T / 4;                // 16-byte chunks of the filter rows
     static constexpr int NLA = (A_CHUNKS + 63) / 64;
     static constexpr int A_BYTES = NLA * 1024;
-    static constexpr int B_BYTES = (CPS * PLANE + 64) * 4;
+    static constexpr int B_BYTES = CPS / 4 * QUAD * 4;
     static constexpr int BUF = (A_BYTES + B_BYTES + 255) / 256 * 256;
     static constexpr int NLA_W = (NLA + NWAVE - 1) / NWAVE;          // per wave
     static constexpr int PLANES_W = CPS / NWAVE;                     // planes a wave loads
@@ -138,7 +139,7 @@ struct ConvF32Tile {
         for (int k = 0; k < PLANES_W; ++k) {
             const int ci = k * NWAVE + c.wave;           // plane of the stage; quad k, channel `wave` of it
             const unsigned soff = (unsigned)(s * CPS + ci) * (unsigned)(HW * 4);
-            const unsigned plane = dst + A_BYTES + (unsigned)(ci * PLANE + plane_bank(c.wave)) * 4u;
+            const unsigned plane = dst + A_BYTES + (unsigned)(k * QUAD + c.wave * PLANE + plane_bank(c.wave)) * 4u;
 #pragma unroll
             for (int l = 0; l < NLB; ++l) dma_buffer_lds_b32(c.b_voff[l], c.rsrc, soff, plane + l * 256);
         }
@@ -227,7 +228,7 @@ struct ConvF32Tile {
                         a[(k + 1) & 1][tm] = *reinterpret_cast<const float*>(ap + (tm * 16 * CPS * T + c4 * 4 * T + tap) * 4);
 #pragma unroll
                     for (int tn = 0; tn < TN; ++tn)
-                        b[(k + 1) & 1][tn] = *reinterpret_cast<const float*>(bp[tn] + (c4 * 4 * PLANE + (tap / KW) * WPS + tap % KW) * 4);
+                        b[(k + 1) & 1][tn] = *reinterpret_cast<const float*>(bp[tn] + (c4 * QUAD + (tap / KW) * WPS + tap % KW) * 4);
                 }
 #pragma unroll
                 for (int tm = 0; tm < TM; ++tm)
