@@ -186,6 +186,12 @@ BFUSE_HFUSE_KERNEL(selftest_conv_tile_a, ConvT_a, bias_relu_4096, BiasReluS)
 BFUSE_BFUSE_KERNEL(selftest_conv_tile_b, ConvT_b, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
 BFUSE_HFUSE_KERNEL(selftest_conv_tile_c, ConvT_c, conv3x3_f32_32x12x12_32, ConvS2)
 
+// The dense product's long stages (16 k): an odd number of them, two waves over K.
+using GemmLong = GemmF32Dma<64, 96, 1056, 32, 48, 2>;
+static_assert(GemmLong::STAGE == 16);
+BFUSE_KERNEL(selftest_gemm_long, GemmLong, ({{64, 1056, 1, 1}, 4}), ({{1056, 96, 1, 1}, 4}), ({{64, 96, 1, 1}, 4}))
+BFUSE_HFUSE_KERNEL(selftest_gemm_long, GemmLong, bias_relu_4096, BiasReluS)
+
 // The shared-tile product likewise: pixels of images that are no whole chunks, tiles over several images and past the batch,
 // strides, row and column tiles that overlap, fewer stages than buffers.
 // <M, K, H, W, S, images or products, BM, BN, waves over BM, k per stage, layout, buffers>

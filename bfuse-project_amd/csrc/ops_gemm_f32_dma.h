@@ -24,13 +24,21 @@
 // s_waitcnt vmcnt(n) and for its own LDS reads with s_waitcnt lgkmcnt(0), both by hand (the
 // loads are asm, the compiler does not count them).
 //
-// Stage = 8 k.  Per wave and stage the ring slot holds A[BM][8] (rows of 32 bytes) followed by
+// Stage = 8 k (16: below).  Per wave and stage the ring slot holds A[BM][8] (rows of 32 bytes) followed by
 // B[8][BN].  Lane (i = lane % 16, kq = lane / 16) reads A[i][2kq], A[i][2kq+1] with one 64-bit
 // read and B[2kq+t][4i .. 4i+3] (t = 0, 1) with 128-bit reads; component e of a B vector feeds
 // accumulator block e of its 64-column group, so that block's column i is tile column 4i+e
 // and a lane ends up with four consecutive columns of a row (128-bit stores), as in GemmF32.
+//
+// A tile of at most six 16 x 16 blocks has 12 MFMAs per 8 k against 8 LDS reads and 3 loads (one of them half empty:
+// 8 rows of 48 columns are a load and a half): 108 TFLOP/s on 512 x 3072 x 768.  With stages of 16 k a lane reads its four
+// k of A at once, and 24 MFMAs share 14 reads and 5 loads: 22.4 -> 20.4 us there, launches back to back.  Not for a short
+// reduction, whose ramp a longer stage lengthens (K = 768, 192 a wave: 6.5 -> 6.8 us), nor for larger tiles (32 x 64:
+// 1.00x; 32 x 96: 0.94x, 32 x 144: 0.94x -- a third more registers and twice the LDS).  96-bit reads of the 48 columns: 25 us.
 #pragma once
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "dispatch.h"
 #include "ops_gemm_f32.h"
@@ -49,7 +57,8 @@ struct GemmF32Dma {
     static constexpr int G1 = (BN % 64) / 16;   // trailing 16-column groups
     static constexpr int NB = 4 * G4 + G1;      // accumulator blocks per row block
     static constexpr int KW = K / KS;           // k-range of one wave
-    static constexpr int STAGE = 8;
+    static constexpr int STAGE = BM * BN <= 32 * 48 && KW >= 512 && K % (16 * KS) == 0 ? 16 : 8;
+    static constexpr int KT = STAGE / 4;        // k-steps of a stage
     static constexpr int NSTAGE = KW / STAGE;
     static constexpr int A_BYTES = BM * STAGE * 4;
     static constexpr int B_BYTES = STAGE * BN * 4;
@@ -100,9 +109,9 @@ struct GemmF32Dma {
     }
 
     struct Frag {
-        f32x2 a[TM];
-        f32x4 b4[G4 > 0 ? G4 : 1][2];
-        float b1[G1 > 0 ? G1 : 1][2];
+        std::conditional_t<KT == 4, f32x4, f32x2> a[TM];
+        f32x4 b4[G4 > 0 ? G4 : 1][KT];
+        float b1[G1 > 0 ? G1 : 1][KT];
     };
     struct Ctx {
         // sources: a wave-uniform base (scalar registers) plus this lane's constant byte offset
@@ -117,9 +126,9 @@ struct GemmF32Dma {
     };
 
     // ---- one memory operation at a time, so that they can be dealt between the MFMAs ----------
-    static constexpr int NREADS = TM + 2 * (G4 + G1);     // LDS reads per stage
+    static constexpr int NREADS = TM + KT * (G4 + G1);    // LDS reads per stage
     static constexpr int NOPS = LPS + 1 + NREADS;         // loads, the wait for the next stage, its reads
-    static constexpr int NGROUPS = 2 * TM * (G4 + G1);    // MFMA groups per stage (4 MFMAs or 1)
+    static constexpr int NGROUPS = KT * TM * (G4 + G1);   // MFMA groups per stage (4 MFMAs or 1)
     static constexpr int OPS_PER_GROUP = (NOPS + NGROUPS - 3) / (NGROUPS - 2);   // leave the last two groups free
 
     template <int I>
@@ -147,12 +156,13 @@ struct GemmF32Dma {
 #if defined(__HIP_DEVICE_COMPILE__)
         constexpr int S0 = SLOT * STAGE_BYTES;
         if constexpr (J < TM) {
-            asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(f.a[J]) : "v"(c.a_base), "n"(S0 + J * 16 * 32));
-        } else if constexpr (J < TM + 2 * G4) {
-            constexpr int g = (J - TM) / 2, t = (J - TM) % 2;
+            if constexpr (KT == 4) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(f.a[J]) : "v"(c.a_base), "n"(S0 + J * 16 * STAGE * 4));
+            else asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(f.a[J]) : "v"(c.a_base), "n"(S0 + J * 16 * STAGE * 4));
+        } else if constexpr (J < TM + KT * G4) {
+            constexpr int g = (J - TM) / KT, t = (J - TM) % KT;
             asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(f.b4[g][t]) : "v"(c.b4_base), "n"(S0 + (t * BN + g * 64) * 4));
         } else {
-            constexpr int g = (J - TM - 2 * G4) / 2, t = (J - TM - 2 * G4) % 2;
+            constexpr int g = (J - TM - KT * G4) / KT, t = (J - TM - KT * G4) % KT;
             asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(f.b1[g][t]) : "v"(c.b1_base), "n"(S0 + (t * BN + G4 * 64 + g * 16) * 4));
         }
 #endif
@@ -176,11 +186,11 @@ struct GemmF32Dma {
 #pragma unroll
         for (int g = 0; g < G4; ++g)
 #pragma unroll
-            for (int t = 0; t < 2; ++t) asm volatile("" : "+v"(f.b4[g][t]));
+            for (int t = 0; t < KT; ++t) asm volatile("" : "+v"(f.b4[g][t]));
 #pragma unroll
         for (int g = 0; g < G1; ++g)
 #pragma unroll
-            for (int t = 0; t < 2; ++t) asm volatile("" : "+v"(f.b1[g][t]));
+            for (int t = 0; t < KT; ++t) asm volatile("" : "+v"(f.b1[g][t]));
 #endif
     }
 
@@ -289,11 +299,11 @@ struct GemmF32Dma {
         c.ring = (unsigned)(unsigned long long)(lds_u8*)sm.t + (unsigned)wave * WAVE_BYTES;
         c.a_ub = reinterpret_cast<const char*>(A + (size_t)m0 * K + kbeg);
         c.b_ub = reinterpret_cast<const char*>(B + (size_t)kbeg * N + n0);
-        // A slot: [BM][8] floats; a wave-level load covers 32 rows (two lanes per 32-byte row)
+        // A slot: [BM][STAGE] floats; a wave-level load covers 32 rows of 8 or 16 rows of 16 (two or four lanes per row)
 #pragma unroll
         for (int i = 0; i < A_LOADS; ++i)
-            c.a_voff[i] = (unsigned)((i * 32 + (lane >> 1)) * K + (lane & 1) * 4) * 4u;
-        // B slot: [8][BN] floats, 16-byte chunk ch = (row, ch % (BN/4))
+            c.a_voff[i] = (unsigned)(((i * 64 + lane) / KT) * K + (lane % KT) * 4) * 4u;
+        // B slot: [STAGE][BN] floats, 16-byte chunk ch = (row, ch % (BN/4))
 #pragma unroll
         for (int i = 0; i < B_LOADS; ++i) {
             // lanes past the end of a partial last load fetch the last chunk again; it lands in
@@ -303,9 +313,9 @@ struct GemmF32Dma {
             c.b_voff[i] = (unsigned)((ch / (BN / 4)) * N + (ch % (BN / 4)) * 4) * 4u;
         }
         const int base = (int)c.ring;
-        c.a_base = base + li * 32 + kq * 8;
-        c.b4_base = base + A_BYTES + (2 * kq * BN + 4 * li) * 4;
-        c.b1_base = base + A_BYTES + (2 * kq * BN + li) * 4;
+        c.a_base = base + li * (STAGE * 4) + kq * (KT * 4);
+        c.b4_base = base + A_BYTES + (KT * kq * BN + 4 * li) * 4;
+        c.b1_base = base + A_BYTES + (KT * kq * BN + li) * 4;
 
         f32x4 acc[TM][NB];
 #pragma unroll

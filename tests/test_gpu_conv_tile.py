@@ -1,5 +1,5 @@
-"""The shared-tile convolution and product (csrc/ops_conv_tile.h, ops_gemm_tile.h) at the edges of their tiles, against the
-CPU oracle (products: numpy in double), alone and fused."""
+"""The shared-tile convolution and product (csrc/ops_conv_tile.h, ops_gemm_tile.h) and the dense product's long stages
+(ops_gemm_f32_dma.h) at the edges of their tiles, against the CPU oracle (products: numpy in double), alone and fused."""
 import numpy as np
 import pytest
 
@@ -49,3 +49,8 @@ def test_shared_tile_batched_product_against_numpy_and_fused(tag, partner, kind,
     def product(a, b):
         return np.matmul(a[..., 0].astype(np.float64), b[..., 0].astype(np.float64).transpose(0, 2, 1)).astype(np.float32)
     _check(f"selftest_gemm_tile_{tag}", product, partner, kind, suffix)
+
+
+def test_long_stages_of_the_dense_product_against_numpy_and_fused():
+    _check("selftest_gemm_long", lambda a, b: (a[..., 0, 0].astype(np.float64) @ b[..., 0, 0].astype(np.float64)).astype(np.float32),
+           "bias_relu_4096", "hfuse", "")
