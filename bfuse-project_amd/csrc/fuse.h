@@ -394,6 +394,7 @@ struct KernelEntry {
     int pattern, p0, p1;    // bfuse: dispatch pattern and its parameters
     unsigned (*read_sync_timeouts)();  // device counter of GroupSync give-ups in this module (read and reset)
     int (*set_spin_limit)(unsigned);   // polls a side barrier of this module makes before it gives up (0 = ok)
+    int (*report_to)(unsigned*);       // the host word that side barriers of this module set when they give up (0 = ok)
     int (*set_plan)(const BlockPlan*); // bfuse_rt: per-kernel hook called when a plan is installed (0 = ok); the plan itself travels as a kernel argument
     const char* op_type = "";          // single: the operator's C++ type, spelled so that it can be compiled again
     int smem_bytes = -1;               // single: sizeof(Op::Smem), the LDS the operator's body declares
@@ -419,6 +420,7 @@ const char* op_type_name()
 struct ModuleHooks {
     unsigned (*read_sync_timeouts)();
     int (*set_spin_limit)(unsigned);
+    int (*report_to)(unsigned*);
 };
 
 std::vector<KernelEntry>& registry();
@@ -446,6 +448,7 @@ KernelEntry make_single_entry(const char* name, const void* func, TensorDesc i, 
     e.io[0] = i; e.io[1] = f; e.io[2] = o;
     e.read_sync_timeouts = hooks.read_sync_timeouts;
     e.set_spin_limit = hooks.set_spin_limit;
+    e.report_to = hooks.report_to;
     e.op_type = op_type_name<Op>();
     e.smem_bytes = (int)sizeof(typename Op::Smem);
     e.matrix_cores = UsesMatrixCores<Op>::value;
@@ -468,6 +471,7 @@ KernelEntry make_group_entry(const char* name, const void* func, int kind, std::
     e.pattern = pattern; e.p0 = p0; e.p1 = p1;
     e.read_sync_timeouts = hooks.read_sync_timeouts;
     e.set_spin_limit = hooks.set_spin_limit;
+    e.report_to = hooks.report_to;
     return e;
 }
 
@@ -493,7 +497,11 @@ KernelEntry make_fused_entry(const char* name, const void* func, int kind, const
     {                                                                                               \
         return hipMemcpyToSymbol(HIP_SYMBOL(bfuse::g_sync_spin_limit), &polls, sizeof(polls)) == hipSuccess ? 0 : -1; \
     }                                                                                               \
-    static const bfuse::ModuleHooks bfuse_module_hooks{&bfuse_module_read_sync_timeouts, &bfuse_module_set_spin_limit};
+    static int bfuse_module_report_to(unsigned* word)                                               \
+    {                                                                                               \
+        return hipMemcpyToSymbol(HIP_SYMBOL(bfuse::g_sync_gave_up), &word, sizeof(word)) == hipSuccess ? 0 : -1; \
+    }                                                                                               \
+    static const bfuse::ModuleHooks bfuse_module_hooks{&bfuse_module_read_sync_timeouts, &bfuse_module_set_spin_limit, &bfuse_module_report_to};
 
 namespace bfuse {
 // The waves per SIMD a kernel is compiled for (the register budget of its waves: 512 / waves): kMinWavesPerEu,

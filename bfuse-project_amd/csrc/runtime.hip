@@ -13,6 +13,8 @@
 #include <cstring>
 #include <string>
 #include <map>
+#include <mutex>
+#include <set>
 #include <unordered_map>
 #include <vector>
 
@@ -369,6 +371,34 @@ int launch6(const void* func, const unsigned* grid, const unsigned* block, hipSt
 const char* const kModuleSyncCounter = "bfuse_sync_timeouts";
 std::vector<hipModule_t>& modules();
 
+// Host memory that every module's side barriers set when they give up, for as long as the process lives: a kernel may
+// always still hold its address.
+unsigned* g_gave_up = nullptr;
+
+// Whether the kernels of e's module report to it on this device.  They are told so here, at the first synchronisation
+// after one of them was launched (the module is loaded then, and nothing is being captured); that one reads the counter.
+bool reports(const KernelEntry& e)
+{
+    static std::set<std::pair<int (*)(unsigned*), int>> told;
+    static std::mutex m;
+    int dev = 0;
+    if (!e.report_to || hipGetDevice(&dev) != hipSuccess) return false;
+    std::lock_guard<std::mutex> lock(m);
+    if (told.count({e.report_to, dev})) return true;
+    if (!g_gave_up) {
+        void* p = nullptr;
+        if (hipHostMalloc(&p, sizeof(unsigned), hipHostMallocPortable) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        g_gave_up = static_cast<unsigned*>(p);
+        *g_gave_up = 0;
+    }
+    if (e.report_to(g_gave_up) == 0) told.insert({e.report_to, dev});
+    else (void)hipGetLastError();
+    return false;
+}
+
 // Device synchronisation, launch errors, and the side barriers' give-up counters of everything
 // launched since the last call: a barrier that gave up let its side run on unsynchronised, so
 // outputs and timings of that launch are not to be trusted.
@@ -390,10 +420,17 @@ int sync_and_check()
         HostCopy::get().quiesced();
     }
     note_hip(hipGetLastError(), "launch");
-    // every counter is read (and thereby reset) even after an error above; the first error is the one returned
+    // every counter that may hold something is read (and thereby reset) even after an error above; the first error is the
+    // one returned
+    bool gave_up = true;
+    if (g_gave_up) {
+        gave_up = __atomic_load_n(g_gave_up, __ATOMIC_RELAXED) != 0;
+        if (gave_up) __atomic_store_n(g_gave_up, 0u, __ATOMIC_RELAXED);
+    }
     for (const void* f : fused) {
         const KernelEntry* e = entry_of(f);
         if (!e || !(e->kind == kHfuse || e->kind == kBfuseRt) || !e->read_sync_timeouts) continue;
+        if (reports(*e) && !gave_up) continue;
         const unsigned n = e->read_sync_timeouts();   // reads and resets
         if (n && rc == BFUSE_OK) rc = fail(BFUSE_ERR_SYNC, "%s: %u side-barrier waits gave up", e->name.c_str(), n);
     }

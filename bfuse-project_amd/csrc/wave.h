@@ -74,6 +74,9 @@ __device__ __forceinline__ unsigned int pack_bf16(float lo, float hi)
 // ---- synchronisation policies ---------------------------------------------------------
 // Counts waits that gave up (see GroupSync); read back by the host after a fused launch.
 static __device__ unsigned int g_sync_timeouts;
+// A word of host memory that is set along with it, once the library has put its address here: whether any counter is
+// worth reading, which costs the host a copy from the device (15 us).
+static __device__ unsigned int* g_sync_gave_up;
 
 // Whole-workgroup barrier: standalone kernels and block-fused kernels (each workgroup runs
 // one operator; waves outside the operator's thread range have already exited, and the
@@ -131,7 +134,10 @@ struct GroupSync {
         do {
             __builtin_amdgcn_s_sleep(1);
             if (++spins >= limit) {
-                if ((threadIdx.x & 63) == 0) atomicAdd(&g_sync_timeouts, 1u);
+                if ((threadIdx.x & 63) == 0) {
+                    atomicAdd(&g_sync_timeouts, 1u);
+                    if (unsigned int* const word = *(unsigned int* volatile*)&g_sync_gave_up) __hip_atomic_store(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                }
                 break;
             }
         } while (__hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < target);
