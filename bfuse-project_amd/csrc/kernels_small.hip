@@ -182,6 +182,7 @@ CONV_TILE_TEST(d, 16, 64, 20, 13, 3, 3, 4, 1, 64, 4, 4, 9, 2)       // stride 4,
 CONV_TILE_TEST(e, 48, 96, 8, 33, 3, 1, 1, 1, 96, 8, 4, 7, 2)        // 3 x 1 filter: an odd number of columns, twelve stages
 CONV_TILE_TEST(f, 16, 128, 7, 7, 3, 3, 1, 1, 128, 10, 4, 5, 2)      // 245 pixels in two tiles of 160, five blocks a wave
 CONV_TILE_TEST(g, 20, 48, 11, 11, 3, 3, 1, 1, 48, 20, 4, 3, 1)      // 363 pixels in two tiles of 320, an odd number of stages
+CONV_TILE_TEST(h, 64, 32, 9, 9, 3, 3, 1, 1, 32, 4, 4, 3, 1)         // sixteen stages, summed three at a time
 BFUSE_HFUSE_KERNEL(selftest_conv_tile_a, ConvT_a, bias_relu_4096, BiasReluS)
 BFUSE_BFUSE_KERNEL(selftest_conv_tile_b, ConvT_b, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
 BFUSE_HFUSE_KERNEL(selftest_conv_tile_c, ConvT_c, conv3x3_f32_32x12x12_32, ConvS2)
@@ -207,5 +208,6 @@ CONV1_TILE_TEST(c, 48, 112, 9, 7, 2, 11, 96, 128, 2, 16, 3)      // stride 2 (20
 CONV1_TILE_TEST(d, 32, 64, 8, 8, 1, 7, 64, 128, 2, 16, 4)        // fewer stages than buffers, whole chunks
 BGEMM_TILE_TEST(e, 3, 160, 48, 144, 128, 128, 2, 16, 3)          // row and column tiles that overlap
 BGEMM_TILE_TEST(f, 8, 64, 32, 64, 64, 64, 4, 32, 2)              // one stage, products dealt to the XCDs
+BGEMM_TILE_TEST(g, 2, 64, 512, 64, 64, 64, 4, 32, 3)             // two sums of 256 k
 BFUSE_HFUSE_KERNEL(selftest_gemm_tile_c, GemmT_c, bias_relu_4096, BiasReluS)
 BFUSE_BFUSE_KERNEL(selftest_gemm_tile_e, GemmT_e, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)

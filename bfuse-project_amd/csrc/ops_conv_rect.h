@@ -374,20 +374,20 @@ struct ConvTiling {
     using held = std::conditional_t<(RESERVE > 0), LdsReserve<staged, (RESERVE > 0 ? RESERVE : 1)>, staged>;
     // A batch with enough pixels for two workgroups per CU goes to the shared-tile form, with the largest tile whose
     // part of each wave is at least twelve 16 x 16 blocks: measured at batch 1024 over the 3 x 3 and 5 x 5 layers it
-    // takes 0.40-0.82 of the time of the per-wave forms above (107-146 TFLOP/s against 52-115); with eight blocks per wave
+    // takes 0.40-0.82 of the time of the per-wave forms above (107-142 TFLOP/s against 52-115); with eight blocks per wave
     // (32 x 64) 0.97-1.06.  96 channels before 128: 142 against 140 TFLOP/s on 288 -> 384; 64 x 256 pixels, one wave over
     // the channels, against 64 x 128, two: 142 against 90.
     static constexpr int tile_bm() { return CO % 96 == 0 ? 96 : CO % 128 == 0 ? 128 : CO % 160 == 0 ? 160 : CO % 64 == 0 ? 64 : CO % 48 == 0 ? 48 : CO % 80 == 0 ? 80 : CO % 32 == 0 ? 32 : 16; }
     // At stride 1 half the channels and twice the pixels: the patch of 256 consecutive pixels of a row or image has few more
     // rows than that of 128, the workgroup takes 32-38 KB of LDS instead of 42-48, and more of them share a CU (96 -> 96 on
-    // 35 x 35 143 against 139 TFLOP/s, 1.01-1.03x on six layers).  Not at stride 2, whose patch is four times the pixels
+    // 35 x 35 139 against 138 TFLOP/s, 1.00-1.01x on six layers).  Not at stride 2, whose patch is four times the pixels
     // (0.93-0.98x), nor on images so small that 256 pixels are several of them (8 x 8: 0.98x).
     static constexpr bool HALF = S == 1 && tile_bm() >= 96 && OHW >= 128;
     static constexpr int TBM = HALF ? tile_bm() / 2 : tile_bm(), TWM = TBM >= 96 ? 2 : 1, TPB0 = TBM >= 96 ? 8 : TBM >= 48 ? 16 : 32;
     // A quarter more pixels per tile where that leaves less of the last round idle.  A CU multiplies two workgroups' tiles in
     // the time of two, so a round is 256 tiles: 512 -> 512 channels on 7 x 7 is 6.13 rounds (7) of 128 pixels but 4.9 (5) of
     // 160: 142 against 127 TFLOP/s; 256 -> 256 on 14 x 14 145 against 140; 256 -> 512 on 14 x 14 at stride 2 132 against 121.
-    // A gain of two in a hundred by this count was 0.99-1.01x.
+    // A gain of two in a hundred by this count was 0.99-1.01x.  At most twenty blocks per wave: they take 160 registers.
     static constexpr double filled(int pb)
     {
         const long long tiles = ((long long)OHW * NIMG + 16 * pb - 1) / (16 * pb) * (CO / TBM);
@@ -397,7 +397,7 @@ struct ConvTiling {
     {
         if constexpr (T > 1 && CI >= 16 && CI % 4 == 0 && KH >= S && TBM >= 32 && (long long)OHW * NIMG >= 512LL * 16 * TPB0 * TBM / CO)
             return pb == TPB0 ? ConvF32Lds<CI, CO, H, W, KH, KW, S, P, TBM, TPB0, 4, NIMG, TWM>::FITS
-                              : ConvF32Lds<CI, CO, H, W, KH, KW, S, P, TBM, TPB0 / 4 * 5, 4, NIMG, TWM>::FITS;
+                              : TBM / 16 * (TPB0 / 4 * 5) <= 80 && ConvF32Lds<CI, CO, H, W, KH, KW, S, P, TBM, TPB0 / 4 * 5, 4, NIMG, TWM>::FITS;
         return false;
     }
     static constexpr int TPB = filled(TPB0 / 4 * 5) > 1.03 * filled(TPB0) && tiled(TPB0 / 4 * 5) ? TPB0 / 4 * 5 : TPB0;
@@ -406,7 +406,8 @@ struct ConvTiling {
     // by element.  Three buffers of 16 channels for 128-pixel tiles (134 against 124 TFLOP/s with two of 32 on 768 -> 192),
     // two for 256-pixel ones, which are bound by memory and want more workgroups per CU.
     static constexpr int GBM = CO % 96 != 0 && CO % 224 == 0 ? 224 : tile_bm(), GWM = GBM >= 96 ? 2 : 1, GBN = GBM >= 96 ? 128 : 256;
-    static constexpr bool PRODUCT = T == 1 && P == 0 && CI % 16 == 0 && tile_bm() >= 32 && (long long)((OHW + 3) / 4 * 4) * NIMG / GBN * (CO / GBM) >= 512;
+    // Only where the streamed form would do, which also keeps one sum over all channels.
+    static constexpr bool PRODUCT = STREAM && tile_bm() >= 32 && (long long)((OHW + 3) / 4 * 4) * NIMG / GBN * (CO / GBM) >= 512;
     template <int FORM, class Else> struct pick { using type = Else; };
     template <class Else> struct pick<1, Else> { using type = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, TBM, TPB, 4, NIMG, TWM>; };
     template <class Else> struct pick<2, Else> { using type = SwapOperands<GemmTile<CO, CI, H, W, S, NIMG, GBM, GBN, GWM, 16, kPix, GWM == 2 ? 3 : 2>>; };

@@ -2,6 +2,7 @@
 (ops_gemm_f32_dma.h) at the edges of their tiles, against the CPU oracle (products: numpy in double), alone and fused."""
 import numpy as np
 import pytest
+import torch
 
 import bfuse_project_amd as bf
 from bfuse_project_amd.operation import fill_normal
@@ -33,7 +34,7 @@ def _check(name, reference, partner, kind, suffix):
 @pytest.mark.parametrize("tag,s,p,partner,kind,suffix", [
     ("a", 1, 1, "bias_relu_4096", "hfuse", ""), ("b", 2, 0, "layernorm_8x256", "bfuse", "_c4"),
     ("c", 1, 2, "conv3x3_f32_32x12x12_32", "hfuse", ""), ("d", 4, 1, "bias_relu_4096", None, ""), ("e", 1, 1, "bias_relu_4096", None, ""),
-    ("f", 1, 1, "bias_relu_4096", None, ""), ("g", 1, 1, "bias_relu_4096", None, "")])
+    ("f", 1, 1, "bias_relu_4096", None, ""), ("g", 1, 1, "bias_relu_4096", None, ""), ("h", 1, 1, "bias_relu_4096", None, "")])
 def test_shared_tile_convolution_against_the_oracle_and_fused(tag, s, p, partner, kind, suffix):
     _check(f"selftest_conv_tile_{tag}", lambda x, w: orf.conv2d(x, w, s=s, p=p), partner, kind, suffix)
 
@@ -44,11 +45,29 @@ def test_shared_tile_1x1_convolution_against_the_oracle_and_fused(tag, s, partne
     _check(f"selftest_gemm_tile_{tag}", lambda x, w: orf.conv2d(x, w, s=s, p=0), partner, kind, suffix)
 
 
-@pytest.mark.parametrize("tag,partner,kind,suffix", [("e", "layernorm_8x256", "bfuse", "_c4"), ("f", "bias_relu_4096", None, "")])
+@pytest.mark.parametrize("tag,partner,kind,suffix", [("e", "layernorm_8x256", "bfuse", "_c4"), ("f", "bias_relu_4096", None, ""), ("g", "bias_relu_4096", None, "")])
 def test_shared_tile_batched_product_against_numpy_and_fused(tag, partner, kind, suffix):
     def product(a, b):
         return np.matmul(a[..., 0].astype(np.float64), b[..., 0].astype(np.float64).transpose(0, 2, 1)).astype(np.float32)
     _check(f"selftest_gemm_tile_{tag}", product, partner, kind, suffix)
+
+
+@pytest.mark.parametrize("name,steps,parts", [("selftest_conv_tile_h", 64 * 9 // 4, 16 / 3), ("selftest_gemm_tile_g", 512 // 4, 2)])
+def test_long_reductions_are_summed_in_parts(name, steps, parts):
+    """A sum of random terms that is rounded after each of `steps` steps, by at most u = 2^-24 of what it has grown to, is
+    off by at most u sqrt(steps / 2) of the result (2-norm); in `parts` equal parts by sqrt(parts) less.  (In one sum these
+    two are 3.0e-7 and 4.1e-7 off, the bounds are 2.2e-7 and 3.4e-7.)"""
+    with bf.Operation(name, "bias_relu_4096") as op:
+        k = op.k[0]
+        x, w = (fill_normal(7 + i, int(np.prod(k.shapes[i])), 0, 1).reshape(k.shapes[i]) for i in (0, 1))
+        op.upload(0, x, w)
+        op.launch("kernel1")
+        y = op.download(0).ravel().astype(np.float64)
+    if "conv" in name:
+        want = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(w).double(), padding=1).numpy()
+    else:
+        want = np.matmul(x[..., 0].astype(np.float64), w[..., 0].astype(np.float64).transpose(0, 2, 1))
+    assert np.linalg.norm(y - want.ravel()) <= 2.0 ** -24 * (steps / 2 / parts) ** 0.5 * np.linalg.norm(want)
 
 
 def test_long_stages_of_the_dense_product_against_numpy_and_fused():
