@@ -193,6 +193,10 @@ static_assert(GemmLong::STAGE == 16);
 BFUSE_KERNEL(selftest_gemm_long, GemmLong, ({{64, 1056, 1, 1}, 4}), ({{1056, 96, 1, 1}, 4}), ({{64, 96, 1, 1}, 4}))
 BFUSE_HFUSE_KERNEL(selftest_gemm_long, GemmLong, bias_relu_4096, BiasReluS)
 
+// The bf16 product's ring of four stages: eleven K-steps, eight of them in the rolled loop.
+using GemmRing4 = GemmBf16NTDma<128, 1024, 704, 64, 128, 4, 2, 2, 2, 2, 6>;
+BFUSE_KERNEL(selftest_gemm_ring4, GemmRing4, ({{128, 704, 1, 1}, 2}), ({{1024, 704, 1, 1}, 2}), ({{128, 1024, 1, 1}, 2}))
+
 // The shared-tile product likewise: pixels of images that are no whole chunks, tiles over several images and past the batch,
 // strides, row and column tiles that overlap, fewer stages than buffers.
 // <M, K, H, W, S, images or products, BM, BN, waves over BM, k per stage, layout, buffers>

@@ -23,10 +23,14 @@ using Dense2 = GemmF32Dma<512, 768, 3072, 32, 48, 4, kEpiNone, 2>;
 // dense_3: the QKV projection of pair 2
 using Dense3 = GemmF32Dma<512, 2304, 768, 32, 144, 4>;
 // dense_4 / dense_7 (Llama-3-8B, bf16, weights [N, K]): N = 4096 over 256 CUs leaves each a 64 x 128 tile: four
-// compute waves (2 x 2) of 32 x 64 and two producer waves, ring of three 64-k stages (72 KB), read-ahead of two
-// fragments, the next step's barrier before MFMA group 6 of 8
-using Dense4 = GemmBf16NTDma<512, 4096, 4096, 64, 128, 3, 2, 2, 2, 2, 6>;
-using Dense7 = GemmBf16NTDma<512, 4096, 14336, 64, 128, 3, 2, 2, 2, 2, 6>;
+// compute waves (2 x 2) of 32 x 64 and two producer waves, ring of four 64-k stages (96 KB), read-ahead of two
+// fragments, the next step's barrier before MFMA group 6 of 8.  A stage is 24 KB for 256 clocks of MFMAs: what bounds the
+// layer is how many bytes are under way, 72 KB with four stages.  Three: 71.9 against 67.0 us (K = 14336) and 23.8 against
+// 22.5, and although two workgroups of three stages fit a CU the fusions gain as well (with the norm 76.6 -> 71.6 and
+// 28.6 -> 26.3, with convolutions 1.04-1.05x).  Five and six stages are like four (66.8, 67.5; 22.5, 22.0), 128 x 128 tiles
+// on half the CUs 77.8 and 24.3.
+using Dense4 = GemmBf16NTDma<512, 4096, 4096, 64, 128, 4, 2, 2, 2, 2, 6>;
+using Dense7 = GemmBf16NTDma<512, 4096, 14336, 64, 128, 4, 2, 2, 2, 2, 6>;
 // dense_5: Llama-3-8B key / value projection, [512 x 4096] . [4096 x 1024]: 16 x 16 tiles of 32 x 64
 using Dense5 = GemmF32Dma<512, 1024, 4096, 32, 64, 4>;
 // dense_6: the gate projection of pair 5

@@ -1,11 +1,12 @@
-"""The shared-tile convolution and product (csrc/ops_conv_tile.h, ops_gemm_tile.h) and the dense product's long stages
-(ops_gemm_f32_dma.h) at the edges of their tiles, against the CPU oracle (products: numpy in double), alone and fused."""
+"""The shared-tile convolution and product (csrc/ops_conv_tile.h, ops_gemm_tile.h), the dense product's long stages
+(ops_gemm_f32_dma.h) and the bf16 product's ring of four (ops_gemm_bf16.h) at the edges of their tiles, against the CPU
+oracle (products: numpy in double), alone and fused."""
 import numpy as np
 import pytest
 import torch
 
 import bfuse_project_amd as bf
-from bfuse_project_amd.operation import fill_normal
+from bfuse_project_amd.operation import bf16_to_f32, f32_to_bf16, fill_normal
 from oracle import oracle as orf
 from tests import oracle_cases
 
@@ -73,3 +74,16 @@ def test_long_reductions_are_summed_in_parts(name, steps, parts):
 def test_long_stages_of_the_dense_product_against_numpy_and_fused():
     _check("selftest_gemm_long", lambda a, b: (a[..., 0, 0].astype(np.float64) @ b[..., 0, 0].astype(np.float64)).astype(np.float32),
            "bias_relu_4096", "hfuse", "")
+
+
+def test_ring_of_four_stages_of_the_bf16_product_against_numpy():
+    """Operands are bf16, sums fp32: what is left is the rounding of the result to eight bits (half a unit in the last place
+    is at most 2^-8 of it) and 1e-5 of the sum's size."""
+    with bf.Operation("selftest_gemm_ring4", "bias_relu_4096") as op:
+        k = op.k[0]
+        a, b = (f32_to_bf16(fill_normal(8 + i, int(np.prod(k.shapes[i])), 0, 1)) for i in (0, 1))
+        op.upload(0, a, b)
+        op.launch("kernel1")
+        y = bf16_to_f32(op.download(0)).reshape(128, 1024).astype(np.float64)
+    want = bf16_to_f32(a).reshape(128, 704).astype(np.float64) @ bf16_to_f32(b).reshape(1024, 704).astype(np.float64).T
+    assert np.all(np.abs(y - want) <= 2.0 ** -8 * np.abs(want) * (1 + 1e-5) + 1e-5 * np.sqrt(704))
