@@ -8,6 +8,7 @@
 #include "ops_gemm_bf16.h"
 #include "ops_gemm_f32.h"
 #include "ops_gemm_f32_dma.h"
+#include "ops_gemm_tile.h"
 #include "ops_rowwise.h"
 
 namespace bfuse {
@@ -39,14 +40,16 @@ using Dense6 = GemmBf16NTDma<512, 14336, 4096, 128, 224, 3, 4, 4, 2, 2, 11>;
 // Batched GEMMs of the attention layers (the reference's bgemm, scripts/configure_kernels.py:14-19,40-48:
 // C[b] = A[b] . B[b]^T with A [b, M, K] and B [b, N, K]): bgemm_0 / bgemm_1 are BERT's and GPT-2's scores and
 // context products (12 heads, sequence 512, head size 64), bgemm_2 / bgemm_3 Llama-3-8B's (32 heads, head size 128).
-// Operands go global -> VGPR in MFMA layout (both are contiguous along K); a short reduction (K = 64, 128) is
-// one wave's, a long one (K = 512) is split over two.
-// (tiles measured on bgemm_0 / bgemm_1: 64 x 64 one-wave 8.0 us, 32 x 64 8.3-9.0, 32 x 128 8.0, 16 x 64 10.1, 64 x 128 11.1;
-//  32 x 64 two-wave 9.7 us, 16 x 64 two-wave 11.3, four-wave 11.3, 16 x 32 10.1)
-using Bgemm0 = GemmF32<512, 512, 64, 64, 64, 1, kEpiNone, 2, 1, true, 12>;     // 8 x 8 tiles x 12 = 768 one-wave workgroups
+// Tiles of 64 rows shared by four waves (GemmTile), 512 workgroups and more: a wave per tile (64 x 64, operands straight
+// into registers) had one wave per SIMD at best to cover its loads.  bgemm_0 8.1 -> 7.3 us (128 x 64 tiles 8.3, 128 x 128
+// 8.8), bgemm_2 27.1 -> 23.3 (64 x 64 24.6 - 26.3, 128 x 128 23.4 - 23.8), bgemm_3 27.2 -> 21.4 (128 x 64 22.0, 64 x 128 21.8,
+// 128 x 128 36); fused with the dense layers 1.0-1.5x, with the causal softmax 13.8 -> 10.2.  Same bits as before.
+// bgemm_1 has 8 row tiles a product, too few of 64 rows (12.2 us): operands go global -> VGPR in MFMA layout, two waves
+// split K.  (32 x 64 two-wave 9.7 us, 16 x 64 two-wave 11.3, four-wave 11.3, 16 x 32 10.1)
+using Bgemm0 = GemmTile<512, 64, 1, 512, 1, 12, 64, 64, 4, 32, kRows, 2>;     // 8 x 8 tiles x 12 = 768 workgroups
 using Bgemm1 = GemmF32<512, 64, 512, 32, 64, 2, kEpiNone, 2, 1, true, 12>;     // 16 x 1 tiles x 12 = 192 two-wave workgroups
-using Bgemm2 = GemmF32<512, 512, 128, 64, 64, 1, kEpiNone, 2, 1, true, 32>;    // 2048 one-wave workgroups
-using Bgemm3 = GemmF32<512, 128, 512, 32, 64, 2, kEpiNone, 2, 1, true, 32>;    // 16 x 2 tiles x 32 = 1024 two-wave workgroups
+using Bgemm2 = GemmTile<512, 128, 1, 512, 1, 32, 64, 128, 2, 16, kRows, 3>;    // 8 x 4 tiles x 32 = 1024 workgroups
+using Bgemm3 = GemmTile<512, 512, 1, 128, 1, 32, 64, 64, 4, 32, kRows, 3>;    // 8 x 2 tiles x 32 = 512 workgroups
 
 // conv2d_1: the convolution of pair 3;  conv2d_4: 128 -> 128 channels on 28 x 28, 32 output channels x 16 pixels
 // per workgroup, four waves take two 16-channel groups each, 49 x 4 = 196 workgroups
@@ -60,22 +63,25 @@ using Dense6F32 = GemmF32Dma<512, 14336, 4096, 64, 128, 4>;
 using Dense7F32 = GemmF32Dma<512, 4096, 14336, 64, 128, 4>;
 
 // bgemm_4 .. bgemm_17 of llm.yaml (ViT / Swin / small-model attention products: 16 heads x 256 or 208 tokens with
-// head sizes 64 and 80, and single-head products of 512 / 768 / 1024 tokens).  208 = 13 x 16 and 80 = 5 x 16 are
-// whole 16-wide MFMA blocks: a 208-column tile is three 64-column groups and one of 16, an 80-column tile one of
-// each; reductions of 80 and 208 are five and thirteen 16-k stages of one wave.
-using Bgemm4 = GemmF32<256, 256, 64, 64, 64, 1, kEpiNone, 2, 1, true, 16>;      // 4 x 4 tiles x 16 = 256 one-wave workgroups
+// head sizes 64 and 80, and single-head products of 512 / 768 / 1024 tokens).  Scores (reductions of 64 and 80) run on
+// shared 64 x 64 tiles, four waves for each of 128 - 256 tiles where one wave had it before: 6.1 -> 3.8 us, 7.0 -> 4.4, with
+// 208 rows and columns (the last tiles overlap) 5.5 -> 3.6, 6.2 -> 4.3, one head of 1024 3.9 -> 3.3; the same bits.  Context
+// products have one column tile a product and too few row tiles for that (256 x 256 x 64: 6.8 against 4.3 us): 208 = 13 x 16
+// and 80 = 5 x 16 are whole 16-wide MFMA blocks, an 80-column tile is one 64-column group and one of 16; a reduction of 208 is
+// thirteen 16-k stages of one wave.
+using Bgemm4 = GemmTile<256, 64, 1, 256, 1, 16, 64, 64, 4, 32, kRows, 2>;      // 4 x 4 tiles x 16 = 256 workgroups
 using Bgemm5 = GemmF32<256, 64, 256, 16, 64, 2, kEpiNone, 2, 1, true, 16>;      // 16 x 1 x 16 = 256 two-wave workgroups
-using Bgemm6 = GemmF32<256, 256, 80, 64, 64, 1, kEpiNone, 2, 1, true, 16>;
+using Bgemm6 = GemmTile<256, 80, 1, 256, 1, 16, 64, 64, 4, 16, kRows, 2>;
 using Bgemm7 = GemmF32<256, 80, 256, 16, 80, 2, kEpiNone, 2, 1, true, 16>;
-using Bgemm8 = GemmF32<208, 208, 64, 16, 208, 1, kEpiNone, 2, 1, true, 16>;     // 13 x 1 x 16 = 208 one-wave workgroups
+using Bgemm8 = GemmTile<208, 64, 1, 208, 1, 16, 64, 64, 4, 32, kRows, 2>;      // 4 x 4 overlapping tiles x 16
 using Bgemm9 = GemmF32<208, 64, 208, 16, 64, 1, kEpiNone, 2, 1, true, 16>;
-using Bgemm10 = GemmF32<208, 208, 80, 16, 208, 1, kEpiNone, 2, 1, true, 16>;
+using Bgemm10 = GemmTile<208, 80, 1, 208, 1, 16, 64, 64, 4, 16, kRows, 2>;
 using Bgemm11 = GemmF32<208, 80, 208, 16, 80, 1, kEpiNone, 2, 1, true, 16>;
 using Bgemm12 = GemmF32<512, 256, 64, 16, 64, 1, kEpiNone, 2, 1, true, 1>;      // 32 x 4 = 128 one-wave workgroups
 using Bgemm13 = GemmF32<512, 64, 256, 16, 64, 4, kEpiNone, 2, 1, true, 1>;      // 32 four-wave workgroups
 using Bgemm14 = GemmF32<768, 384, 64, 16, 64, 1, kEpiNone, 2, 1, true, 1>;      // 48 x 6 = 288
 using Bgemm15 = GemmF32<768, 64, 384, 16, 64, 4, kEpiNone, 2, 1, true, 1>;      // 48 four-wave workgroups
-using Bgemm16 = GemmF32<1024, 512, 64, 32, 64, 1, kEpiNone, 2, 1, true, 1>;     // 32 x 8 = 256
+using Bgemm16 = GemmTile<1024, 64, 1, 512, 1, 1, 64, 64, 4, 32, kRows, 2>;      // 16 x 8 = 128
 using Bgemm17 = GemmF32<1024, 64, 512, 16, 64, 4, kEpiNone, 2, 1, true, 1>;     // 64 four-wave workgroups
 
 // The other ResNet-18 layers (test-utils/examples/resnet-18.yaml) on the general convolution:
