@@ -52,7 +52,8 @@ using Bgemm2 = GemmTile<512, 128, 1, 512, 1, 32, 64, 128, 2, 16, kRows, 3>;    /
 using Bgemm3 = GemmTile<512, 512, 1, 128, 1, 32, 64, 64, 4, 32, kRows, 3>;    // 8 x 2 tiles x 32 = 512 workgroups
 
 // conv2d_1: the convolution of pair 3;  conv2d_4: 128 -> 128 channels on 28 x 28, 32 output channels x 16 pixels
-// per workgroup, four waves take two 16-channel groups each, 49 x 4 = 196 workgroups
+// per workgroup, four waves take two 16-channel groups each, 49 x 4 = 196 workgroups (eight waves on 16 channels x 32 pixels:
+// 6.9 us alone against 8.9, but fused with the dense layers of two workgroups per CU 28.7 against 26.3)
 using Conv1 = Conv3x3F32Lds<64, 64, 56, 56, 16, 4, 4>;
 using Conv4 = Conv3x3F32Lds<128, 128, 28, 28, 32, 1, 4>;
 
@@ -86,15 +87,19 @@ using Bgemm17 = GemmF32<1024, 64, 512, 16, 64, 4, kEpiNone, 2, 1, true, 1>;     
 
 // The other ResNet-18 layers (test-utils/examples/resnet-18.yaml) on the general convolution:
 // <CI, CO, H, W, KH, KW, stride, padding, output channels per workgroup, 16-pixel blocks, waves>
+// One image has 128 - 208 tiles of 16 x 16 results and a reduction of 576 - 4608 for each: staging and the chain of MFMAs
+// of a wave are what takes the time, so the 3x3 layers of 128 channels and more split it over eight waves: 17.1 -> 14.7 us on
+// 7x7 (sixteen waves 14.5, but fused with the LayerNorm 16.4 against 14.9), 10.0 -> 8.9 on 14x14, 11.4 -> 9.9 and 6.8 -> 6.5 at
+// stride 2; fused with the LayerNorm 1.05-1.3x.  The 1x1 layers gain 1.1-1.2x alone and lose 0.74-0.84x fused: four waves.
 using Conv0 = ConvF32Rect<3, 64, 224, 224, 7, 7, 2, 3, 16, 4, 1>;         // 7x7 stride 2 on RGB: 4 x 16-pixel rectangles (13 x 37 patch instead of 9 x 230), 196 x 4 = 784 one-wave workgroups
 using Conv2 = SwapOperands<GemmF32<64, 3136, 64, 16, 64, 1>>;            // 1x1 stride 1 = Wt[64,64] . X[64,3136]: 4 x 49 = 196
-using Conv3 = ConvF32Lds<64, 128, 56, 56, 3, 3, 2, 1, 32, 1, 4>;          // 49 x 4 = 196 workgroups
+using Conv3 = ConvF32Lds<64, 128, 56, 56, 3, 3, 2, 1, 16, 2, 4>;          // 25 x 8 = 200 workgroups; 32 channels x 16 pixels 6.4 against 6.1 us, fused 10.8 against 8.0
 using Conv5 = ConvF32Lds<64, 128, 56, 56, 1, 1, 2, 0, 32, 1, 4>;
-using Conv6 = ConvF32Lds<128, 256, 28, 28, 3, 3, 2, 1, 16, 1, 4>;         // 13 x 16 = 208
-using Conv7 = ConvF32Lds<256, 256, 14, 14, 3, 3, 1, 1, 16, 1, 4>;
+using Conv6 = ConvF32Lds<128, 256, 28, 28, 3, 3, 2, 1, 16, 1, 8>;         // 13 x 16 = 208
+using Conv7 = ConvF32Lds<256, 256, 14, 14, 3, 3, 1, 1, 16, 1, 8>;
 using Conv8 = ConvF32Lds<128, 256, 28, 28, 1, 1, 2, 0, 16, 1, 4>;
-using Conv9 = ConvF32Lds<256, 512, 14, 14, 3, 3, 2, 1, 16, 1, 4>;         // 4 x 32 = 128
-using Conv10 = ConvF32Lds<512, 512, 7, 7, 3, 3, 1, 1, 16, 1, 4>;
+using Conv9 = ConvF32Lds<256, 512, 14, 14, 3, 3, 2, 1, 16, 1, 8>;         // 4 x 32 = 128
+using Conv10 = ConvF32Lds<512, 512, 7, 7, 3, 3, 1, 1, 16, 1, 8>;
 using Conv11 = ConvF32Lds<256, 512, 14, 14, 1, 1, 2, 0, 16, 1, 4>;
 
 // memory-bound partners
