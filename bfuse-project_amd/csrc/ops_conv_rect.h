@@ -386,7 +386,8 @@ struct ConvTiling {
     static constexpr int TBM = HALF ? tile_bm() / 2 : tile_bm(), TWM = TBM >= 96 ? 2 : 1, TPB0 = TBM >= 96 ? 8 : TBM >= 48 ? 16 : 32;
     // A quarter more pixels per tile where that leaves less of the last round idle.  A CU multiplies two workgroups' tiles in
     // the time of two, so a round is 256 tiles: 512 -> 512 channels on 7 x 7 is 6.13 rounds (7) of 128 pixels but 4.9 (5) of
-    // 160: 142 against 127 TFLOP/s; 256 -> 256 on 14 x 14 145 against 140; 256 -> 512 on 14 x 14 at stride 2 132 against 121.
+    // 160: 142 against 127 TFLOP/s; 256 -> 256 on 14 x 14 145 against 140; 256 -> 512 on 14 x 14 at stride 2 132 against 121.  (With one sum
+    // over the reduction; sums in parts take 0-5 % off both sides: 138 on 14 x 14.)
     // A gain of two in a hundred by this count was 0.99-1.01x.  At most twenty blocks per wave: they take 160 registers.
     static constexpr double filled(int pb)
     {
