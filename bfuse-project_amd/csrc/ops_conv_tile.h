@@ -95,8 +95,10 @@ struct ConvF32Tile {
     static constexpr int BUF = (A_BYTES + B_BYTES + 255) / 256 * 256;
     static constexpr int NLA_W = (NLA + NWAVE - 1) / NWAVE;          // per wave
     static constexpr int PLANES_W = CPS / NWAVE;                     // planes a wave loads
-    // fragment offsets are 16-bit immediates; two workgroups share a CU; a register per load of the patch
-    static constexpr bool FITS = A_BYTES + B_BYTES < 65536 && 4 * BUF <= 160 * 1024 && NLB <= 28;
+    // fragment offsets are 16-bit immediates; two workgroups share a CU; a register per load of the patch; the images of a tile
+    // are one buffer, whose size is 31 bits: an offset of 2^31 - 1 has to lie past its end
+    static constexpr bool FITS = A_BYTES + B_BYTES < 65536 && 4 * BUF <= 160 * 1024 && NLB <= 28 &&
+                                 (long long)(NIMAGES < NIMG ? NIMAGES : NIMG) * CI * HW * 4 < (1LL << 31);
 
     static constexpr Dims3 GRID{NPT * NCT, 1, 1};
     static constexpr Dims3 BLOCK{64 * NWAVE, 1, 1};
