@@ -408,11 +408,16 @@ struct ConvTiling {
     // two for 256-pixel ones, which are bound by memory and want more workgroups per CU.
     static constexpr int GBM = CO % 96 != 0 && CO % 224 == 0 ? 224 : tile_bm(), GWM = GBM >= 96 ? 2 : 1, GBN = GBM >= 96 ? 128 : 256;
     // Only where the streamed form would do, which also keeps one sum over all channels.
-    static constexpr bool PRODUCT = STREAM && tile_bm() >= 32 && (long long)((OHW + 3) / 4 * 4) * NIMG / GBN * (CO / GBM) >= 512;
+    using product = GemmTile<CO, CI, H, W, S, NIMG, GBM, GBN, GWM, 16, kPix, GWM == 2 ? 3 : 2>;
+    static constexpr bool is_product()
+    {
+        if constexpr (STREAM && tile_bm() >= 32 && (long long)((OHW + 3) / 4 * 4) * NIMG / GBN * (CO / GBM) >= 512) return product::FITS;
+        return false;
+    }
     template <int FORM, class Else> struct pick { using type = Else; };
     template <class Else> struct pick<1, Else> { using type = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, TBM, TPB, 4, NIMG, TWM>; };
-    template <class Else> struct pick<2, Else> { using type = SwapOperands<GemmTile<CO, CI, H, W, S, NIMG, GBM, GBN, GWM, 16, kPix, GWM == 2 ? 3 : 2>>; };
-    using type = typename pick<PRODUCT ? 2 : tiled(TPB) ? 1 : 0, std::conditional_t<STREAM, Conv1x1F32<CI, CO, H, W, S, stream_bm(), 4, NIMG>, held>>::type;
+    template <class Else> struct pick<2, Else> { using type = SwapOperands<product>; };
+    using type = typename pick<is_product() ? 2 : tiled(TPB) ? 1 : 0, std::conditional_t<STREAM, Conv1x1F32<CI, CO, H, W, S, stream_bm(), 4, NIMG>, held>>::type;
 };
 template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int NIMG = 1>
 using ConvF32Auto = typename ConvTiling<CI, CO, H, W, KH, KW, S, P, NIMG>::type;

@@ -67,7 +67,10 @@ struct GemmTile {
     static constexpr bool GATHER = LAYOUT == kPix && S > 1;
     static_assert(BM % (16 * WM) == 0 && BN % (64 * WN) == 0 && K % KS == 0 && (KS == 16 || KS == 32), "tile");
     static_assert(M >= BM && (LAYOUT == kPix || (W >= BN && H == 1 && S == 1)), "a tile is not larger than the problem");
-    static_assert(K % 4 == 0 && (long long)K * HW * 4 < (1LL << 31) && (long long)M * K * 4 < (1LL << 31), "sizes");
+    static constexpr int NIMAGES = LAYOUT == kRows ? 1 : (BN + OHWP - 2) / OHWP + 1;   // images a tile can touch
+    // The rows of a product, and the images of a tile, are addressed by 31 bits: columns past the batch (and past a strided
+    // image) are read through an offset of 2^31 - 1, which has to lie past the end of the buffer that the images are.
+    static constexpr bool FITS = (long long)M * K * 4 < (1LL << 31) && (long long)(NIMAGES < NIMG ? NIMAGES : NIMG) * K * HW * 4 < (1LL << 31);
 
     static constexpr int TILES = MT * NT;
     static constexpr Dims3 GRID{LAYOUT == kRows ? TILES * NIMG : TILES, 1, 1};
@@ -147,6 +150,7 @@ struct GemmTile {
     template <class Sync>
     __device__ static __forceinline__ void run(int vblock, int tid, Smem& sm, const void* I, const void* F, void* O, Sync sync)
     {
+        static_assert(FITS, "tile too large");
         static_assert(LAYOUT == kRows || 256 % BN == 0, "a load is whole planes");
         const float* __restrict__ A = static_cast<const float*>(I);
         const float* __restrict__ B = static_cast<const float*>(F);
@@ -195,7 +199,6 @@ struct GemmTile {
             }
         } else {
             n_lo = (int)(n0 / OHWP);
-            constexpr int NIMAGES = (BN + OHWP - 2) / OHWP + 1;
             const int images = NIMG - n_lo < NIMAGES ? NIMG - n_lo : NIMAGES;
             const unsigned long long base = (unsigned long long)(B + (size_t)n_lo * K * HW);
             c.rsrc = i32x4{(int)(unsigned)base, (int)(unsigned)(base >> 32), images * K * HW * 4, 0x00020000};   // raw buffer, 32-bit elements

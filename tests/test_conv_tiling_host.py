@@ -12,6 +12,8 @@ PROLOGUE = """
 using namespace bfuse;
 template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int BM, int BP, int WM, int CPS, int NIMG>
 std::true_type shared(const ConvF32Tile<CI, CO, H, W, KH, KW, S, P, BM, BP, WM, CPS, NIMG>*);
+template <int M, int K, int H, int W, int S, int NIMG, int BM, int BN, int WM, int KS, int LAYOUT, int NBUF>
+std::true_type shared(const GemmTile<M, K, H, W, S, NIMG, BM, BN, WM, KS, LAYOUT, NBUF>*);
 std::false_type shared(const void*);
 template <class Op> constexpr bool is_shared = decltype(shared(static_cast<const Op*>(nullptr)))::value;
 """
@@ -31,4 +33,14 @@ def test_images_of_a_tile_are_less_than_two_gigabytes(tmp_path):
         static_assert(!is_shared<ConvF32Auto<512, 64, 2200, 256, 3, 3, 1, 1, 4>>);    // two images of 1.15 GB
         static_assert(!is_shared<ConvF32Auto<512, 64, 2048, 256, 3, 3, 1, 1, 4>>);    // 2 GiB to the byte
         static_assert(is_shared<ConvF32Auto<512, 64, 2047, 256, 3, 3, 1, 1, 4>>);
+    """, tmp_path)
+
+
+def test_images_of_a_1x1_tile_are_less_than_two_gigabytes(tmp_path):
+    """Columns past the batch likewise; an image of 2 GiB by itself is no error."""
+    _compiles("""
+        static_assert(!is_shared<ConvF32Auto<512, 64, 2200, 256, 1, 1, 1, 0, 4>>);    // two images of 1.15 GB
+        static_assert(!is_shared<ConvF32Auto<512, 64, 2200, 256, 1, 1, 2, 0, 4>>);
+        static_assert(!is_shared<ConvF32Auto<512, 64, 2048, 512, 1, 1, 1, 0, 4>>);    // one of 2 GiB
+        static_assert(is_shared<ConvF32Auto<512, 64, 2047, 256, 1, 1, 1, 0, 4>>);
     """, tmp_path)
