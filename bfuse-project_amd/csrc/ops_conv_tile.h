@@ -62,24 +62,37 @@ struct ConvF32Tile {
     static constexpr int SUM_PARTS = CI / 16 % 4 == 0 ? 4 : CI / 16 % 2 == 0 ? 2 : 1;
     static constexpr int SUM = 3 * NS / (4 * SUM_PARTS) > 1 ? 3 * NS / (4 * SUM_PARTS) : 1;
     static constexpr long long NPIX = (long long)OHW * NIMG;
+    static constexpr long long TILES = (NPIX + BP - 1) / BP * (CO / BM);
     static constexpr int NPT = (int)((NPIX + BP - 1) / BP), NCT = CO / BM;
     static_assert(CI % CPS == 0 && CPS % 4 == 0 && CO % BM == 0 && BM % (16 * WM) == 0 && BP % (16 * WN) == 0, "channel tiling");
     static_assert((CI * T) % 4 == 0 && (CPS * T) % 4 == 0, "filter rows are whole 16-byte chunks");
-    static_assert((long long)NPT * NCT < (1LL << 31) && (long long)CI * HW * 4 < (1LL << 31), "sizes");
 
     // ---- the patch: the image rows under the tile's output rows, image after image, every column a window touches.
     // Image n's rows are HR virtual rows (its OH windows' rows -P .. ), one image after the other.
     static constexpr int HR = (OH - 1) * S + KH, WPS = (OW - 1) * S + KW;
-    static constexpr int patch_rows()        // the most virtual rows BP consecutive pixels of the batch span
+    static constexpr int MOST_LOADS = 28;                             // wave-level loads of a plane: a register each
+    // The virtual rows that the BP pixels of the tile starting at pixel a span: S for every output row, and where one image
+    // ends and the next begins KH - S more (windows of two images share no row; the least number of ends if that is negative).
+    static constexpr long long rows_from(long long a)
     {
-        int most = 0;
-        const long long period = NPT < 4 * OHW ? NPT : 4 * OHW;       // tile starts repeat after OHW tiles
-        for (long long t = 0; t < period; ++t) {
-            const long long a = t * BP % ((long long)OHW * 64), b = a + BP - 1;
-            const int rows = (int)((b / OHW * HR + b % OHW / OW * S) - (a / OHW * HR + a % OHW / OW * S)) + KH;
-            if (rows > most) most = rows;
+        return S * ((a % OW + BP - 1) / OW) + (KH - S) * (KH < S ? (BP - 1) / OHW : (a % OHW + BP - 1) / OHW) + KH;
+    }
+    // The most that any tile spans.  Rows depend on a tile's start within its output row, which comes round after at most OW
+    // tiles, and ends on the tiles that hold one, which are alike after at most BP images (tiles of more than an image: all
+    // of at most OHW different starts hold one).  Looking at these is exact and cheap; at all tiles of a large image it is
+    // beyond what a compiler evaluates (512 x 512 pixels).
+    static constexpr int patch_rows()
+    {
+        if (KH * WPS > 64 * MOST_LOADS) return KH;            // too wide to be staged at all: no need to look
+        long long most = 0;
+        const long long starts = BP > OHW ? OHW : OW;
+        for (long long t = 0; t < starts && t * BP < NPIX; ++t)
+            if (rows_from(t * BP) > most) most = rows_from(t * BP);
+        for (long long n = 1; n < NIMG && n <= BP; ++n) {
+            const long long a = (n * OHW - 1) / BP * BP;      // the tile that holds image n - 1's last pixel
+            if (rows_from(a) > most) most = rows_from(a);
         }
-        return most;
+        return (int)most;
     }
     static constexpr int NR = patch_rows();
     static constexpr int NIMAGES = (BP + OHW - 2) / OHW + 1;          // images a tile can touch
@@ -95,9 +108,9 @@ struct ConvF32Tile {
     static constexpr int BUF = (A_BYTES + B_BYTES + 255) / 256 * 256;
     static constexpr int NLA_W = (NLA + NWAVE - 1) / NWAVE;          // per wave
     static constexpr int PLANES_W = CPS / NWAVE;                     // planes a wave loads
-    // fragment offsets are 16-bit immediates; two workgroups share a CU; a register per load of the patch; the images of a tile
-    // are one buffer, whose size is 31 bits: an offset of 2^31 - 1 has to lie past its end
-    static constexpr bool FITS = A_BYTES + B_BYTES < 65536 && 4 * BUF <= 160 * 1024 && NLB <= 28 &&
+    // fragment offsets are 16-bit immediates; two workgroups share a CU; the images of a tile are one buffer, whose size is 31
+    // bits: an offset of 2^31 - 1 has to lie past its end
+    static constexpr bool FITS = A_BYTES + B_BYTES < 65536 && 4 * BUF <= 160 * 1024 && NLB <= MOST_LOADS && TILES < (1LL << 31) &&
                                  (long long)(NIMAGES < NIMG ? NIMAGES : NIMG) * CI * HW * 4 < (1LL << 31);
 
     static constexpr Dims3 GRID{NPT * NCT, 1, 1};

@@ -1,5 +1,6 @@
 """Which form a convolution gets (csrc/ops_conv_rect.h, ConvTiling) at the limits of the shared tiles, and that it gets one:
 a translation unit of static assertions, compiled for the host."""
+import math
 import os
 import subprocess
 
@@ -44,3 +45,42 @@ def test_images_of_a_1x1_tile_are_less_than_two_gigabytes(tmp_path):
         static_assert(!is_shared<ConvF32Auto<512, 64, 2048, 512, 1, 1, 1, 0, 4>>);    // one of 2 GiB
         static_assert(is_shared<ConvF32Auto<512, 64, 2047, 256, 1, 1, 1, 0, 4>>);
     """, tmp_path)
+
+
+def test_large_images_and_batches_compile(tmp_path):
+    """The rows of a patch come from a few of the batch's tiles: all of a large image's are more than a compiler evaluates.
+    Layers beyond the shared tiles' limits are no errors either."""
+    _compiles("""
+        static_assert(is_shared<ConvF32Auto<64, 64, 256, 256, 3, 3, 1, 1, 1024>> && is_shared<ConvF32Auto<64, 48, 256, 256, 3, 3, 1, 1, 1024>>);
+        static_assert(is_shared<ConvF32Auto<64, 96, 256, 256, 3, 3, 1, 1, 1024>> && is_shared<ConvF32Auto<64, 64, 512, 512, 3, 3, 1, 1, 256>>);
+        static_assert(sizeof(ConvF32Auto<64, 64, 1024, 1024, 3, 3, 1, 1, 64>::Smem) && sizeof(ConvF32Auto<32, 32, 512, 512, 3, 3, 1, 1, 512>::Smem));
+        static_assert(sizeof(ConvF32Auto<32, 64, 300, 300, 5, 5, 1, 2, 1024>::Smem) && sizeof(ConvF32Auto<64, 64, 224, 224, 3, 3, 1, 1, 1024>::Smem));
+        static_assert(!is_shared<ConvF32Auto<512, 64, 1024, 1024, 3, 3, 1, 1, 4>>);    // an image of 2 GiB
+        static_assert(!is_shared<ConvF32Auto<16, 32, 16, 65536, 3, 3, 1, 1, 16>>);     // three rows do not fit
+    """, tmp_path)
+
+
+def test_rows_of_a_patch_against_a_look_at_every_tile(tmp_path):
+    shapes = [(5, 5, 3, 1, 1, 64, 90), (9, 7, 3, 2, 0, 64, 50), (11, 6, 5, 1, 2, 128, 130), (7, 7, 3, 1, 1, 160, 170), (11, 11, 3, 1, 1, 320, 330), (14, 14, 3, 1, 1, 256, 70), (14, 14, 3, 1, 1, 160, 60),
+              (17, 17, 3, 2, 0, 128, 70), (35, 35, 3, 2, 1, 128, 40), (35, 35, 5, 1, 2, 256, 260), (56, 56, 3, 1, 1, 256, 8), (73, 73, 3, 1, 0, 256, 260), (147, 147, 3, 2, 1, 160, 41), (64, 64, 3, 1, 1, 512, 3),
+              (33, 50, 5, 3, 2, 96, 100), (300, 7, 3, 1, 1, 256, 30), (4, 300, 3, 1, 1, 256, 50), (16, 16, 3, 1, 1, 256, 9), (20, 13, 3, 4, 1, 64, 50), (21, 30, 3, 4, 1, 64, 40), (8, 8, 2, 2, 0, 64, 1)]
+    text = """
+        template <class C> constexpr bool rows_are_right(bool whole)   // `whole`: enough images that the batch's end shows nothing new
+        {
+            long long cut = 0, full = 0;
+            for (long long t = 0; t < C::NPT; ++t) {
+                const long long a = t * C::BP, b = a + C::BP - 1, c = b < C::NPIX ? b : C::NPIX - 1;
+                const long long first = a / C::OHW * C::HR + a % C::OHW / C::OW * C::S;
+                const long long r = b / C::OHW * C::HR + b % C::OHW / C::OW * C::S - first + C::KH, q = c / C::OHW * C::HR + c % C::OHW / C::OW * C::S - first + C::KH;
+                if (r > full) full = r;
+                if (q > cut) cut = q;
+            }
+            return whole && C::KH >= C::S ? C::NR == full : C::NR >= cut && (C::KH < C::S || C::NR <= full);
+        }
+    """
+    for h, w, k, s, p, bp, n in shapes:
+        pixels = ((h - k + 2 * p) // s + 1) * ((w - k + 2 * p) // s + 1)
+        for images in (1, 2, 3, n):
+            whole = (images - 1) * math.gcd(pixels, bp) >= bp          # every place that an image's end has in a tile comes up
+            text += f"static_assert(rows_are_right<ConvF32Tile<16, 32, {h}, {w}, {k}, {k}, {s}, {p}, 32, {bp}, {2 if bp % 32 == 0 else 1}, 4, {images}>>({'true' if whole else 'false'}));\n"
+    _compiles(text, tmp_path)
