@@ -51,6 +51,16 @@ struct SegList {
     int n;
 };
 
+// Bytes in front of the first 16-byte boundary.  Host memory that a copy kernel reads or writes is the library's own and is
+// chosen to lie like the device memory relative to such a boundary (see lie()): whatever a part's offset, all but up to 15
+// bytes at either end move as 16-byte words.  (48 MB at an offset of one float: 1.0 ms up and down; in single bytes, 64 of
+// them a wave's request, 15.2 up and 2.3 down.)
+static __device__ __forceinline__ size_t head_of(const void* p, size_t bytes)
+{
+    const size_t head = (16 - ((uintptr_t)p & 15)) & 15;
+    return head < bytes ? head : bytes;
+}
+
 // All segments of one small transfer, device memory <-> pinned host memory, by one launch: consecutive lanes move
 // consecutive 16-byte words (one PCIe request per 64 bytes and more), every block strides over every segment.
 static __global__ __launch_bounds__(256) void copy_segments(SegList l)
@@ -59,11 +69,9 @@ static __global__ __launch_bounds__(256) void copy_segments(SegList l)
     for (int k = 0; k < l.n; ++k) {
         const unsigned char* const src = l.s[k].src;
         unsigned char* const dst = l.s[k].dst;
-        const size_t bytes = l.s[k].bytes;
-        const bool aligned = (((uintptr_t)src | (uintptr_t)dst) & 15) == 0;
-        const size_t words = aligned ? bytes / 16 : 0;
-        for (size_t i = t; i < words; i += nt) reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
-        for (size_t i = words * 16 + t; i < bytes; i += nt) dst[i] = src[i];
+        const size_t bytes = l.s[k].bytes, head = head_of(dst, bytes), words = (bytes - head) / 16, ends = bytes - 16 * words;
+        for (size_t i = t; i < words; i += nt) reinterpret_cast<uint4*>(dst + head)[i] = reinterpret_cast<const uint4*>(src + head)[i];
+        for (size_t i = t; i < ends; i += nt) dst[i < head ? i : 16 * words + i] = src[i < head ? i : 16 * words + i];
     }
 }
 
@@ -75,10 +83,9 @@ static __global__ __launch_bounds__(256) void copy_segments(SegList l)
 static __global__ __launch_bounds__(256) void copy_chunk(const unsigned char* src, unsigned char* dst, size_t bytes, unsigned* flag, unsigned value)
 {
     const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x, nt = (size_t)gridDim.x * 256;
-    const bool aligned = (((uintptr_t)src | (uintptr_t)dst) & 15) == 0;
-    const size_t words = aligned ? bytes / 16 : 0;
-    const uint4* const s = reinterpret_cast<const uint4*>(src);
-    uint4* const d = reinterpret_cast<uint4*>(dst);
+    const size_t head = head_of(dst, bytes), words = (bytes - head) / 16, ends = bytes - 16 * words;
+    const uint4* const s = reinterpret_cast<const uint4*>(src + head);
+    uint4* const d = reinterpret_cast<uint4*>(dst + head);
     size_t i = t;
     for (; i + 3 * nt < words; i += 4 * nt) {
         const uint4 a = s[i], b = s[i + nt], c = s[i + 2 * nt], e = s[i + 3 * nt];
@@ -88,8 +95,10 @@ static __global__ __launch_bounds__(256) void copy_chunk(const unsigned char* sr
         d[i + 3 * nt] = e;
     }
     for (; i < words; i += nt) d[i] = s[i];
-    for (i = words * 16 + t; i < bytes; i += nt) dst[i] = src[i];
+    for (i = t; i < ends; i += nt) dst[i < head ? i : 16 * words + i] = src[i < head ? i : 16 * words + i];
+#if defined(__HIP_DEVICE_COMPILE__)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // each wave's own stores have left it; the barrier alone does not wait for them
+#endif
     __syncthreads();
     if (threadIdx.x == 0) {
         __threadfence_system();
@@ -105,6 +114,7 @@ public:
     static constexpr size_t kFirst = 256 << 10;             // the first copy of a transfer up, the last of one down
     static constexpr size_t kPiece = 64 << 10;              // what a thread moves at a time: the first copy waits for four of them at once
     static constexpr int kSlots = 8;                        // 16 MiB
+    static constexpr size_t kSlotBytes = kChunk + 64;       // a chunk, wherever it lies in its 16 bytes
     static constexpr int kUpBlocks = 8, kDownBlocks = 16;   // of copy_chunk
     static constexpr int kFlagWords = 16;                   // a cache line of one word per block
     static constexpr unsigned kQuietSpins = 100000;
@@ -151,7 +161,7 @@ public:
         for (int i = 0; i < n; ++i) {
             if (seg[i].bytes == 0) continue;
             if (total <= kSmallBytes) {
-                unsigned char* p = arena(out_, seg[i].bytes);
+                unsigned char* p = arena(out_, seg[i].bytes, seg[i].dev);
                 if (!p) return hipErrorOutOfMemory;   // cannot happen: the arena holds kArenaBytes / kSmallBytes calls between synchronisations
                 l.s[l.n++] = {static_cast<const unsigned char*>(seg[i].dev), p, seg[i].bytes};
                 d.packed[d.n_packed++] = {p, seg[i].host, seg[i].bytes};
@@ -246,7 +256,7 @@ private:
         if (e != hipSuccess || dev == device_) return e;
         if (!ring_) {
             void* p[4] = {};
-            const size_t size[4] = {kChunk * kSlots, kArenaBytes, kArenaBytes, kSlots * kFlagWords * sizeof(unsigned)};
+            const size_t size[4] = {kSlotBytes * kSlots, kArenaBytes, kArenaBytes, kSlots * kFlagWords * sizeof(unsigned)};
             for (int i = 0; i < 4; ++i)
                 if ((e = hipHostMalloc(&p[i], size[i], hipHostMallocPortable)) != hipSuccess) {
                     for (int j = 0; j < i; ++j) (void)hipHostFree(p[j]);
@@ -269,14 +279,17 @@ private:
         return hipSuccess;
     }
 
-    static unsigned char* arena(Arena& a, size_t bytes)
+    // p, which is on a 16-byte boundary, or as many bytes behind it as `dev` is behind one
+    static unsigned char* lie(unsigned char* p, const void* dev) { return p + ((uintptr_t)dev & 15); }
+    static unsigned char* arena(Arena& a, size_t bytes, const void* dev)
     {
-        const size_t need = (bytes + 255) & ~(size_t)255;
+        const size_t need = (bytes + 15 + 255) & ~(size_t)255;
         if (a.used + need > kArenaBytes) return nullptr;
         unsigned char* p = a.base + a.used;
         a.used += need;
-        return p;
+        return lie(p, dev);
     }
+    unsigned char* slot_of(long i, const void* dev) const { return lie(ring_ + (size_t)(i % kSlots) * kSlotBytes, dev); }
     // 64 blocks: from 8 to 512 reach the link's rate on long copies; short ones want every request out at once
     static hipError_t launch(const SegList& l, size_t total, hipStream_t stream)
     {
@@ -287,7 +300,7 @@ private:
 
     hipError_t up_small(const CopySeg* seg, int n, size_t total)
     {
-        if (in_.used + total + 256 * (size_t)n > kArenaBytes) {
+        if (in_.used + total + 270 * (size_t)n > kArenaBytes) {
             // earlier uploads may still be on their way out of the arena
             hipError_t e = hipStreamSynchronize(nullptr);
             if (e != hipSuccess) return e;
@@ -296,7 +309,7 @@ private:
         SegList l{};
         for (int i = 0; i < n; ++i) {
             if (seg[i].bytes == 0) continue;
-            unsigned char* p = arena(in_, seg[i].bytes);
+            unsigned char* p = arena(in_, seg[i].bytes, seg[i].dev);
             memcpy(p, seg[i].host, seg[i].bytes);
             l.s[l.n++] = {p, static_cast<unsigned char*>(seg[i].dev), seg[i].bytes};
         }
@@ -362,7 +375,7 @@ private:
                 if (sent < count && (up ? sent < ended + kSlots && done(sent) : sent < kSlots || done(sent - kSlots))) {
                     const Chunk& c = chunks[(size_t)sent];
                     if (!up) left_[slot].store(c.pieces(), std::memory_order_relaxed);
-                    unsigned char* const s = ring_ + slot * kChunk;
+                    unsigned char* const s = slot_of(sent, c.dev);
                     hipLaunchKernelGGL(copy_chunk, dim3(up ? kUpBlocks : kDownBlocks), dim3(256), 0, stream_[sent & 1], up ? s : c.dev, up ? c.dev : s, c.bytes, flag_ + slot * kFlagWords,
                                        base + (unsigned)sent);
                     e = hipGetLastError();
@@ -444,7 +457,8 @@ private:
     // whichever core wrote them (128 MB: 52 against 48 GB/s)
     static void stream_copy(unsigned char* dst, const unsigned char* src, size_t bytes)
     {
-        size_t i = 0;
+        size_t i = std::min(bytes, (size_t)(-(uintptr_t)dst & 15));
+        memcpy(dst, src, i);
         for (; i + 64 <= bytes; i += 64)
             for (size_t j = i; j < i + 64; j += 16)
                 _mm_stream_si128(reinterpret_cast<__m128i*>(dst + j), _mm_loadu_si128(reinterpret_cast<const __m128i*>(src + j)));
@@ -462,11 +476,10 @@ private:
         const long c = std::upper_bound(chunks_, chunks_ + count_, i, [](long v, const Chunk& k) { return v < k.first; }) - chunks_ - 1;
         const Chunk& k = chunks_[c];
         const size_t at = (size_t)(i - k.first) * kPiece, len = std::min(kPiece, k.bytes - at);
-        const int slot = (int)(c % kSlots);
-        unsigned char* const s = ring_ + slot * kChunk + at;
+        unsigned char* const s = slot_of(c, k.dev) + at;
         if (up_) stream_copy(s, k.host + at, len);
         else memcpy(k.host + at, s, len);
-        left_[slot].fetch_sub(1, std::memory_order_release);
+        left_[c % kSlots].fetch_sub(1, std::memory_order_release);
         return true;
     }
 
