@@ -144,8 +144,17 @@ public:
 
     // Device -> host, in two steps around the caller's device synchronisation: begin() enqueues what can run behind the
     // launches on `stream` (small results into the arena, results in pinned buffers in place), finish() puts the rest
-    // where it belongs.
+    // where it belongs.  A Down that is given up in between waits for what was enqueued: nothing is written into the
+    // caller's memory once the call that named it has returned.
     struct Down {
+        Down() = default;
+        Down(const Down&) = delete;
+        Down& operator=(const Down&) = delete;
+        ~Down()
+        {
+            if (open) (void)hipDeviceSynchronize();
+        }
+        bool open = false;            // between begin() and finish()
         CopySeg packed[kMaxSegs];     // arena -> host after the synchronisation (dev = where it lies in the arena)
         CopySeg later[kMaxSegs];      // through the ring after the synchronisation
         int n_packed = 0, n_later = 0;
@@ -157,6 +166,7 @@ public:
         if (e != hipSuccess) return e;
         size_t total = 0;
         for (int i = 0; i < n; ++i) total += seg[i].bytes;
+        d.open = true;
         SegList l{};
         for (int i = 0; i < n; ++i) {
             if (seg[i].bytes == 0) continue;
@@ -173,9 +183,10 @@ public:
         }
         return l.n ? launch(l, total, stream) : hipSuccess;
     }
-    hipError_t down_finish(const Down& d)
+    hipError_t down_finish(Down& d)
     {
         std::lock_guard<std::mutex> lock(call_);
+        d.open = false;
         for (int i = 0; i < d.n_packed; ++i) memcpy(d.packed[i].host, d.packed[i].dev, d.packed[i].bytes);
         return d.n_later ? pipeline(d.later, d.n_later, false) : hipSuccess;
     }
@@ -346,7 +357,7 @@ private:
         bool wait = false;
         for (int i = 0; i < n; ++i) {
             if (up && pinned(seg[i].host, seg[i].bytes)) {
-                if ((e = hipMemcpyAsync(seg[i].dev, seg[i].host, seg[i].bytes, hipMemcpyHostToDevice, stream_[0])) != hipSuccess) return e;
+                if ((e = hipMemcpyAsync(seg[i].dev, seg[i].host, seg[i].bytes, hipMemcpyHostToDevice, stream_[0])) != hipSuccess) break;
                 wait = true;
                 continue;
             }
@@ -363,7 +374,7 @@ private:
             }
         }
         const long count = (long)chunks.size();
-        if (count) {
+        if (count && e == hipSuccess) {
             begin_job(chunks, up);
             long sent = 0, ended = 0;          // copies enqueued / known to have ended
             const unsigned base = value_;

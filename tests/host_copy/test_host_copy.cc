@@ -49,10 +49,45 @@ static void unaligned()
             }
 }
 
+// Copies into a caller's pinned memory have ended when a transfer that failed is given up.
+static void given_up()
+{
+    const size_t n = HostCopy::kSmallBytes;
+    auto a = pattern(n, 1), b = pattern(n, 2);
+    auto* p = static_cast<unsigned char*>(hc().host_buffer(2 * n));
+    memset(p, 0, 2 * n);
+    const CopySeg seg[2] = {{a.data(), p, n}, {b.data(), p + n, n}};
+    {
+        HostCopy::Down d;
+        fake::fail_in["hipMemcpyAsync"] = 2;
+        CHECK(hc().down_begin(seg, 2, nullptr, d) == hipErrorUnknown);
+    }
+    CHECK(memcmp(p, a.data(), n) == 0);
+    memset(p, 0, n);
+    {
+        HostCopy::Down d;
+        CHECK(hc().down_begin(seg, 2, nullptr, d) == hipSuccess);   // and then an error between begin and finish
+    }
+    CHECK(memcmp(p, a.data(), n) == 0 && memcmp(p + n, b.data(), n) == 0);
+    const int waits = fake::device_waits;
+    {
+        HostCopy::Down d;
+        CHECK(hc().down_begin(seg, 2, nullptr, d) == hipSuccess && hipDeviceSynchronize() == hipSuccess && hc().down_finish(d) == hipSuccess);
+    }
+    CHECK(fake::device_waits == waits + 1);                         // none but the caller's own
+    // operands likewise
+    const CopySeg up[2] = {{a.data(), p, n}, {b.data(), p + n, n}};
+    memset(p, 5, n);
+    fake::fail_in["hipMemcpyAsync"] = 2;
+    CHECK(hc().up(up, 2, false) == hipErrorUnknown && a[0] == 5 && a[n - 1] == 5);
+    CHECK(hc().release(p));
+}
+
 int main(int argc, char** argv)
 {
     const std::string t = argc > 1 ? argv[1] : "";
     if (t == "unaligned") unaligned();
+    else if (t == "given_up") given_up();
     else return fprintf(stderr, "no test '%s'\n", t.c_str()), 2;
     hc().close();
     CHECK(fake::host.empty() && fake::streams.empty());
