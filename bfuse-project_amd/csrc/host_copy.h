@@ -152,9 +152,13 @@ public:
         Down& operator=(const Down&) = delete;
         ~Down()
         {
-            if (open) (void)hipDeviceSynchronize();
+            if (!open) return;
+            (void)hipDeviceSynchronize();
+            HostCopy& h = get();
+            std::lock_guard<std::mutex> lock(h.call_);
+            h.end(*this);
         }
-        bool open = false;            // between begin() and finish()
+        bool open = false;            // between begin() and finish(): its part of the arena is in use
         CopySeg packed[kMaxSegs];     // arena -> host after the synchronisation (dev = where it lies in the arena)
         CopySeg later[kMaxSegs];      // through the ring after the synchronisation
         int n_packed = 0, n_later = 0;
@@ -167,12 +171,12 @@ public:
         size_t total = 0;
         for (int i = 0; i < n; ++i) total += seg[i].bytes;
         d.open = true;
+        ++downs_;
         SegList l{};
         for (int i = 0; i < n; ++i) {
             if (seg[i].bytes == 0) continue;
-            if (total <= kSmallBytes) {
-                unsigned char* p = arena(out_, seg[i].bytes, seg[i].dev);
-                if (!p) return hipErrorOutOfMemory;   // cannot happen: the arena holds kArenaBytes / kSmallBytes calls between synchronisations
+            // (the arena holds kArenaBytes / kSmallBytes transfers: of more threads at once, the others take the ring)
+            if (unsigned char* p = total <= kSmallBytes ? arena(out_, seg[i].bytes, seg[i].dev) : nullptr) {
                 l.s[l.n++] = {static_cast<const unsigned char*>(seg[i].dev), p, seg[i].bytes};
                 d.packed[d.n_packed++] = {p, seg[i].host, seg[i].bytes};
             } else if (pinned(seg[i].host, seg[i].bytes)) {
@@ -186,16 +190,18 @@ public:
     hipError_t down_finish(Down& d)
     {
         std::lock_guard<std::mutex> lock(call_);
-        d.open = false;
         for (int i = 0; i < d.n_packed; ++i) memcpy(d.packed[i].host, d.packed[i].dev, d.packed[i].bytes);
+        end(d);
         return d.n_later ? pipeline(d.later, d.n_later, false) : hipSuccess;
     }
 
-    // The device has been synchronised: nothing reads or writes the arenas any more.
-    void quiesced()
+    // Around a device synchronisation: what was on its way out of the arena before it is not any more.  Another thread may
+    // be uploading meanwhile, and what it has launched since, or is about to, is waited for by a later one.
+    unsigned long wait_begins() const { return launched_.load(); }
+    void wait_ended(unsigned long begun)
     {
-        in_.used = out_.used = 0;
-        unwaited_ = 0;
+        unsigned long w = waited_.load();
+        while (w < begun && !waited_.compare_exchange_weak(w, begun)) {}
     }
 
     // Pinned host memory for results: copied into by the engines themselves.  A released buffer is kept for the next
@@ -309,8 +315,16 @@ private:
         return hipGetLastError();
     }
 
+    // a transfer down no longer uses the arena
+    void end(Down& d)
+    {
+        d.open = false;
+        if (--downs_ == 0) out_.used = 0;
+    }
+
     hipError_t up_small(const CopySeg* seg, int n, size_t total)
     {
+        if (waited_.load() >= launched_.load()) in_.used = 0;
         if (in_.used + total + 270 * (size_t)n > kArenaBytes) {
             // earlier uploads may still be on their way out of the arena
             hipError_t e = hipStreamSynchronize(nullptr);
@@ -324,7 +338,9 @@ private:
             memcpy(p, seg[i].host, seg[i].bytes);
             l.s[l.n++] = {p, static_cast<unsigned char*>(seg[i].dev), seg[i].bytes};
         }
-        return launch(l, total, nullptr);
+        const hipError_t e = launch(l, total, nullptr);
+        ++launched_;
+        return e;
     }
 
     // ---- the ring ---------------------------------------------------------------------------------
@@ -567,10 +583,12 @@ private:
     int device_ = -1;
     unsigned char* ring_ = nullptr;
     Arena in_, out_;
+    std::atomic<unsigned long> launched_{0}, waited_{0};   // uploads out of the arena / those known to have ended
+    int downs_ = 0;                      // transfers down that are between begin and finish
     hipStream_t stream_[2] = {};
     unsigned* flag_ = nullptr;           // kFlagWords of every slot
     unsigned value_ = 1;                 // what the next copy reports
-    long unwaited_ = 0;                  // copies since the streams, or the device, were last waited for
+    long unwaited_ = 0;                  // copies since the streams were last waited for
 
     std::mutex job_;
     std::condition_variable work_cv_, idle_cv_;

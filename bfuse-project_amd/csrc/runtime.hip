@@ -415,9 +415,10 @@ int sync_and_check()
         if (e != hipSuccess && rc == BFUSE_OK) rc = fail(BFUSE_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
         return e == hipSuccess;
     };
+    const unsigned long uploads = HostCopy::get().wait_begins();
     if (note_hip(hipDeviceSynchronize(), "hipDeviceSynchronize")) {
         g_busy = false;
-        HostCopy::get().quiesced();
+        HostCopy::get().wait_ended(uploads);
     }
     note_hip(hipGetLastError(), "launch");
     // every counter that may hold something is read (and thereby reset) even after an error above; the first error is the

@@ -40,13 +40,72 @@ static void unaligned()
                 std::vector<unsigned char> got(host_at + n + 1, 0x77);
                 seg.host = got.data() + host_at;
                 HostCopy::Down d;
-                CHECK(hc().down_begin(&seg, 1, nullptr, d) == hipSuccess && hipDeviceSynchronize() == hipSuccess);
-                hc().quiesced();
-                CHECK(hc().down_finish(d) == hipSuccess);
+                CHECK(hc().down_begin(&seg, 1, nullptr, d) == hipSuccess && hipDeviceSynchronize() == hipSuccess && hc().down_finish(d) == hipSuccess);
                 CHECK(memcmp(got.data() + host_at, src.data() + host_at, n) == 0 && got[host_at + n] == 0x77);
                 CHECK(alike && moved == 2 * n);
                 fake::seen = nullptr;
             }
+}
+
+// What one thread has in the arenas outlives another thread's synchronisation.
+static void arenas()
+{
+    fake::deferred = true;
+    std::vector<unsigned char> dev[3] = {std::vector<unsigned char>(1000), std::vector<unsigned char>(1000), std::vector<unsigned char>(9000)}, src[3];
+    auto up = [&](int i) {
+        src[i] = pattern(dev[i].size(), i);
+        const CopySeg seg = {dev[i].data(), src[i].data(), dev[i].size()};
+        CHECK(hc().up(&seg, 1, false) == hipSuccess);
+    };
+    // a thread starts to wait after upload 0; upload 1 comes before it has said that it did
+    up(0);
+    const unsigned long begun = hc().wait_begins();
+    CHECK(hipDeviceSynchronize() == hipSuccess);
+    up(1);
+    hc().wait_ended(begun);
+    up(2);
+    CHECK(hipDeviceSynchronize() == hipSuccess);
+    for (int i = 0; i < 3; ++i) CHECK(dev[i] == src[i]);
+    // a result that has landed is still there when another thread's results come and go
+    std::vector<unsigned char> got[3];
+    HostCopy::Down d[3];
+    auto begin = [&](int i) {
+        got[i].assign(dev[i].size(), 0);
+        const CopySeg seg = {dev[i].data(), got[i].data(), dev[i].size()};
+        CHECK(hc().down_begin(&seg, 1, nullptr, d[i]) == hipSuccess);
+    };
+    auto wait = [&] {
+        const unsigned long n = hc().wait_begins();
+        CHECK(hipDeviceSynchronize() == hipSuccess);
+        hc().wait_ended(n);
+    };
+    begin(0);
+    wait();
+    begin(1);
+    wait();
+    CHECK(hc().down_finish(d[1]) == hipSuccess);
+    begin(2);
+    wait();
+    CHECK(hc().down_finish(d[0]) == hipSuccess && hc().down_finish(d[2]) == hipSuccess);
+    for (int i = 0; i < 3; ++i) CHECK(got[i] == src[i]);
+    // more threads between begin and finish than the arena holds
+    constexpr int kMany = 2 * HostCopy::kArenaBytes / HostCopy::kSmallBytes;
+    std::vector<std::vector<unsigned char>> from, to(kMany, std::vector<unsigned char>(HostCopy::kSmallBytes));
+    HostCopy::Down many[kMany];
+    for (int i = 0; i < kMany; ++i) from.push_back(pattern(HostCopy::kSmallBytes, 7 * i));
+    for (int i = 0; i < kMany; ++i) {
+        const CopySeg seg = {from[i].data(), to[i].data(), HostCopy::kSmallBytes};
+        CHECK(hc().down_begin(&seg, 1, nullptr, many[i]) == hipSuccess);
+    }
+    wait();
+    for (int i = kMany; i-- > 0;) CHECK(hc().down_finish(many[i]) == hipSuccess && to[i] == from[i]);
+    // and the arena of uploads comes round when nobody ever waits
+    for (int i = 0; i < 30; ++i) {
+        const CopySeg seg = {to[0].data(), from[i % kMany].data(), HostCopy::kSmallBytes};
+        CHECK(hc().up(&seg, 1, false) == hipSuccess);
+    }
+    wait();
+    CHECK(to[0] == from[29 % kMany]);
 }
 
 // Copies into a caller's pinned memory have ended when a transfer that failed is given up.
@@ -87,6 +146,7 @@ int main(int argc, char** argv)
 {
     const std::string t = argc > 1 ? argv[1] : "";
     if (t == "unaligned") unaligned();
+    else if (t == "arenas") arenas();
     else if (t == "given_up") given_up();
     else return fprintf(stderr, "no test '%s'\n", t.c_str()), 2;
     hc().close();

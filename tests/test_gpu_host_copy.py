@@ -1,6 +1,8 @@
 """Copies between host arrays and the resident buffers: the packed path of small transfers, the staging ring at the edges
 of its pieces, chunks and slots, unaligned offsets, pageable and pinned destinations (oracle: the bytes themselves, through
 the library's device-to-device copy kernel)."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -60,3 +62,31 @@ def test_results_are_the_callers_own_and_may_be_operands(op):
     op.launch("kernel1")
     c = op.download(0)                                           # the released buffer serves again
     assert c.ctypes.data == address and np.array_equal(c, np.arange(N, dtype=np.float32).reshape(c.shape))
+
+
+def test_two_threads_each_with_a_side_of_its_own(op):
+    """Uploads, single-kernel launches and downloads of one thread are not disturbed by another's, which waits at times of
+    its own."""
+    failures = []
+
+    def work(side, mode, expect, sizes):
+        rng = np.random.default_rng(side)
+        try:
+            for k in range(200):
+                n = sizes[k % len(sizes)]
+                x = rng.standard_normal(n).astype(np.float32)
+                op.upload_part(side, 0, 0, x)
+                op.launch(mode)
+                got = op.download_part(side, 0, n)
+                if not np.array_equal(got, expect(x)):
+                    raise AssertionError(f"side {side}, repetition {k}, {n} floats")
+        except Exception as e:
+            failures.append(e)
+
+    op.upload_part(1, 1, 0, np.zeros(op.k[1].shapes[1][0], np.float32))
+    threads = [threading.Thread(target=work, args=a) for a in ((0, "kernel1", lambda x: x, (1000, 90000, 300000)), (1, "kernel2", lambda x: np.maximum(x, 0), (4096, 17, 2048)))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures, failures
