@@ -106,6 +106,23 @@ static __global__ __launch_bounds__(256) void copy_chunk(const unsigned char* sr
     }
 }
 
+// Whether something that was enqueued may still be running.  Work is counted once it has been enqueued, and a device
+// synchronisation covers what had been counted when it began: another thread's, in between, covers nothing of this one's.
+class InFlight {
+public:
+    void add() { ++added_; }
+    unsigned long wait_begins() const { return added_.load(); }
+    void wait_ended(unsigned long begun)
+    {
+        unsigned long w = waited_.load();
+        while (w < begun && !waited_.compare_exchange_weak(w, begun)) {}
+    }
+    bool any() const { return waited_.load() < added_.load(); }
+
+private:
+    std::atomic<unsigned long> added_{0}, waited_{0};
+};
+
 class HostCopy {
 public:
     static constexpr size_t kSmallBytes = 512 << 10;
@@ -197,12 +214,8 @@ public:
 
     // Around a device synchronisation: what was on its way out of the arena before it is not any more.  Another thread may
     // be uploading meanwhile, and what it has launched since, or is about to, is waited for by a later one.
-    unsigned long wait_begins() const { return launched_.load(); }
-    void wait_ended(unsigned long begun)
-    {
-        unsigned long w = waited_.load();
-        while (w < begun && !waited_.compare_exchange_weak(w, begun)) {}
-    }
+    unsigned long wait_begins() const { return small_ups_.wait_begins(); }
+    void wait_ended(unsigned long begun) { small_ups_.wait_ended(begun); }
 
     // Pinned host memory for results: copied into by the engines themselves.  A released buffer is kept for the next
     // request of its size (up to kIdleLimit bytes in all): pinning costs ~0.2 ms per MB.  nullptr: over the limit.
@@ -324,7 +337,7 @@ private:
 
     hipError_t up_small(const CopySeg* seg, int n, size_t total)
     {
-        if (waited_.load() >= launched_.load()) in_.used = 0;
+        if (!small_ups_.any()) in_.used = 0;
         if (in_.used + total + 270 * (size_t)n > kArenaBytes) {
             // earlier uploads may still be on their way out of the arena
             hipError_t e = hipStreamSynchronize(nullptr);
@@ -339,7 +352,7 @@ private:
             l.s[l.n++] = {p, static_cast<unsigned char*>(seg[i].dev), seg[i].bytes};
         }
         const hipError_t e = launch(l, total, nullptr);
-        ++launched_;
+        small_ups_.add();
         return e;
     }
 
@@ -583,7 +596,7 @@ private:
     int device_ = -1;
     unsigned char* ring_ = nullptr;
     Arena in_, out_;
-    std::atomic<unsigned long> launched_{0}, waited_{0};   // uploads out of the arena / those known to have ended
+    InFlight small_ups_;                 // uploads out of the arena
     int downs_ = 0;                      // transfers down that are between begin and finish
     hipStream_t stream_[2] = {};
     unsigned* flag_ = nullptr;           // kFlagWords of every slot

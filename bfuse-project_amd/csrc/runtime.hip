@@ -6,6 +6,7 @@
 
 #include <dlfcn.h>
 
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -154,7 +155,7 @@ struct EventList {
 // entry point performs it.
 std::vector<const void*> g_pending_fused;
 std::vector<int> g_pending_modules;
-bool g_busy = false;   // something has been enqueued since the last device synchronisation
+InFlight g_in_flight;   // everything enqueued on any stream
 
 // ---- staging memory of bfuse_map_blocks_device_noalloc ----------------------------------------
 // A fixed device array (kernel and block index of up to kNoAllocMaxIds fused blocks) that lives as
@@ -330,11 +331,11 @@ int launch3(const void* func, const unsigned* grid, const unsigned* block, int i
 {
     Side& s = g.side[idx];
     void* args[3] = {&s.buf[0], &s.buf[1], &s.buf[2]};
-    g_busy = true;
     if (ev0 || ev1)
         HIP_TRY(hipExtLaunchKernel(func, d3(grid), d3(block), args, 0, stream, ev0, ev1, 0));
     else
         HIP_TRY(hipLaunchKernel(func, d3(grid), d3(block), args, 0, stream));
+    g_in_flight.add();
     return BFUSE_OK;
 }
 
@@ -351,11 +352,11 @@ int launch_fused(const void* func, const unsigned* grid, const unsigned* block, 
     bool known = false;
     for (const void* f : g_pending_fused) known = known || f == func;
     if (!known) g_pending_fused.push_back(func);
-    g_busy = true;
     if (ev0 || ev1)
         HIP_TRY(hipExtLaunchKernel(func, d3(grid), d3(block), args, 0, stream, ev0, ev1, 0));
     else
         HIP_TRY(hipLaunchKernel(func, d3(grid), d3(block), args, 0, stream));
+    g_in_flight.add();
     return BFUSE_OK;
 }
 
@@ -415,9 +416,9 @@ int sync_and_check()
         if (e != hipSuccess && rc == BFUSE_OK) rc = fail(BFUSE_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
         return e == hipSuccess;
     };
-    const unsigned long uploads = HostCopy::get().wait_begins();
+    const unsigned long uploads = HostCopy::get().wait_begins(), launches = g_in_flight.wait_begins();
     if (note_hip(hipDeviceSynchronize(), "hipDeviceSynchronize")) {
-        g_busy = false;
+        g_in_flight.wait_ended(launches);
         HostCopy::get().wait_ended(uploads);
     }
     note_hip(hipGetLastError(), "launch");
@@ -1001,7 +1002,7 @@ int bfuse_finalize_side(int side)
 static int copy_up(const CopySeg* seg, int n, bool busy)
 {
     HIP_TRY(HostCopy::get().up(seg, n, busy));
-    g_busy = true;   // a small upload is a launch
+    g_in_flight.add();   // a small upload is a launch
     return BFUSE_OK;
 }
 static int upload_sides(const int* idx, const void* const (*src)[2], int n)
@@ -1009,7 +1010,7 @@ static int upload_sides(const int* idx, const void* const (*src)[2], int n)
     CopySeg seg[kMaxSegs];
     for (int k = 0; k < n; ++k)
         for (int t = 0; t < 2; ++t) seg[2 * k + t] = {g.side[idx[k]].buf[t], const_cast<void*>(src[k][t]), g.side[idx[k]].bytes[t]};
-    return copy_up(seg, 2 * n, g_busy);
+    return copy_up(seg, 2 * n, g_in_flight.any());
 }
 // waits for everything launched, then brings the results of `n` sides to the host; nothing is written there if a
 // barrier gave up, unless `always`
@@ -1075,7 +1076,7 @@ int run_parallel(const void* I1, const void* F1, void* O1, const void* I2, const
     for (int k = 0; k < 2; ++k) {
         const CopySeg up[2] = {{g.side[k].buf[0], const_cast<void*>(src[k][0]), g.side[k].bytes[0]}, {g.side[k].buf[1], const_cast<void*>(src[k][1]), g.side[k].bytes[1]}};
         const CopySeg down = {g.side[k].buf[2], dst[k], g.side[k].bytes[2]};
-        if ((rc = copy_up(up, 2, k == 0 && g_busy))) return rc;
+        if ((rc = copy_up(up, 2, k == 0 && g_in_flight.any()))) return rc;
         if ((rc = k == 0 ? launch3((const void*)func1, g1, b1, 0, a.stream) : launch3((const void*)func2, g2, b2, 1, b.stream))) return rc;
         HIP_TRY(HostCopy::get().down_begin(&down, 1, g.side[k].stream, d[k]));
     }
@@ -1120,8 +1121,8 @@ int bfuse_zero_output(int side)
     if (side < 1 || side > kMaxKernels) return fail(BFUSE_ERR_ARG, "side must be 1 .. %d", kMaxKernels);
     Side& s = g.side[side - 1];
     if (!s.live) return fail(BFUSE_ERR_STATE, "kernel%d is not initialized", side);
-    g_busy = true;
     HIP_TRY(hipMemset(s.buf[2], 0, s.bytes[2]));
+    g_in_flight.add();
     return BFUSE_OK;
 }
 
@@ -1159,7 +1160,7 @@ int bfuse_upload_part(int side, int tensor, size_t offset, const void* src, size
     if (offset > s.bytes[tensor] || bytes > s.bytes[tensor] - offset)
         return fail(BFUSE_ERR_ARG, "bytes %zu .. %zu are outside the tensor's %zu", offset, offset + bytes, s.bytes[tensor]);
     const CopySeg seg = {static_cast<char*>(s.buf[tensor]) + offset, const_cast<void*>(src), bytes};
-    return copy_up(&seg, 1, g_busy);
+    return copy_up(&seg, 1, g_in_flight.any());
 }
 
 int bfuse_download_part(int side, size_t offset, void* dst, size_t bytes)
@@ -1254,10 +1255,10 @@ int bfuse_fill_uniform_device(int side, int tensor, unsigned long long seed, flo
     size_t blocks = (n + 256 * 8 - 1) / (256 * 8);
     if (blocks > 16384) blocks = 16384;
     if (blocks < 1) blocks = 1;
-    g_busy = true;
     // on the default stream, in order with every launch: nothing has to be waited for
     hipLaunchKernelGGL(fill_uniform_kernel, dim3((unsigned)blocks), dim3(256), 0, nullptr, s.buf[tensor], n, s.elem[tensor], seed, lo, hi);
     HIP_TRY(hipGetLastError());
+    g_in_flight.add();
     return BFUSE_OK;
 }
 
@@ -1421,9 +1422,11 @@ int bfuse_time_graph(int mode, const void* fa, const unsigned* ga, const unsigne
     HIP_TRY(ended);
     HIP_TRY(hipGraphInstantiate(&gr.x, gr.g, nullptr, nullptr, 0));
     HIP_TRY(hipGraphLaunch(gr.x, s0));
+    g_in_flight.add();
     if ((rc = sync_and_check())) return rc;
     HIP_TRY(hipEventRecord(evl.v[0], s0));
     for (int r = 0; r < reps; ++r) HIP_TRY(hipGraphLaunch(gr.x, s0));
+    g_in_flight.add();
     HIP_TRY(hipEventRecord(evl.v[1], s0));
     if ((rc = sync_and_check())) return rc;
     float ms = 0.f;
@@ -1593,9 +1596,9 @@ int bfuse_module_launch(int id, const char* name, const unsigned* grid, const un
     bool known = false;
     for (int m : g_pending_modules) known = known || m == id;
     if (!known) g_pending_modules.push_back(id);
-    g_busy = true;
     HIP_TRY(hipExtModuleLaunchKernel(fn, grid[0] * block[0], grid[1] * block[1], grid[2] * block[2], block[0], block[1],
                                      block[2], 0, nullptr, args, nullptr, e0, e1, 0));
+    g_in_flight.add();
     if (us_out) {
         int rc = sync_and_check();
         if (rc) return rc;

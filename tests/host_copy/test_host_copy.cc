@@ -47,6 +47,23 @@ static void unaligned()
             }
 }
 
+// What is enqueued while another thread waits is still in flight behind that wait; a wait that began earlier takes nothing back.
+static void in_flight()
+{
+    InFlight f;
+    CHECK(!f.any());
+    f.add();
+    const unsigned long a = f.wait_begins();
+    f.add();
+    const unsigned long b = f.wait_begins();
+    f.wait_ended(a);
+    CHECK(f.any());
+    f.wait_ended(b);
+    CHECK(!f.any());
+    f.wait_ended(a);
+    CHECK(!f.any());
+}
+
 // What one thread has in the arenas outlives another thread's synchronisation.
 static void arenas()
 {
@@ -146,6 +163,7 @@ int main(int argc, char** argv)
 {
     const std::string t = argc > 1 ? argv[1] : "";
     if (t == "unaligned") unaligned();
+    else if (t == "in_flight") in_flight();
     else if (t == "arenas") arenas();
     else if (t == "given_up") given_up();
     else return fprintf(stderr, "no test '%s'\n", t.c_str()), 2;
