@@ -14,6 +14,7 @@
 #include <cstring>
 #include <string>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <set>
 #include <unordered_map>
@@ -221,38 +222,54 @@ dim3 d3(const unsigned* v) { return dim3(v[0], v[1], v[2]); }
 
 // What a launch needs to know of a kernel, by its handle: its entry and the bytes each of its operators' tensors take.
 // Every launch is validated; looking this up by name in the registry (some 330 entries, a fused kernel's sides by string)
-// took 1.5 us of a launch that the runtime itself makes in 2.3.  Rebuilt when kernels have been added.
+// took 1.5 us of a launch that the runtime itself makes in 2.3.  A table is never changed once a launch can see it: when
+// kernels have been added the next launch makes another (the old ones stay, one per module loaded, for who may be reading).
 struct Launchable {
     const KernelEntry* e;
     int n_sides;                               // operators it runs
     const KernelEntry* side[kMaxKernels];      // their standalone kernels (nullptr: unknown)
     size_t need[kMaxKernels][3];
 };
+struct LaunchTable {
+    size_t built;                              // registry entries it was made of
+    std::unordered_map<const void*, Launchable> known;
+};
+const LaunchTable& launch_table()
+{
+    static std::atomic<const LaunchTable*> current{nullptr};
+    const auto& r = registry();
+    const LaunchTable* t = current.load(std::memory_order_acquire);
+    if (t && t->built == r.size()) return *t;
+    static std::mutex m;
+    static std::vector<std::unique_ptr<LaunchTable>> all;
+    std::lock_guard<std::mutex> lock(m);
+    t = current.load(std::memory_order_acquire);
+    if (t && t->built == r.size()) return *t;
+    auto made = std::make_unique<LaunchTable>();
+    std::unordered_map<std::string, const KernelEntry*> single;
+    for (const auto& e : r)
+        if (e.kind == kSingle) single.emplace(e.name, &e);
+    for (const auto& e : r) {
+        Launchable l{};
+        l.e = &e;
+        l.n_sides = e.kind == kSingle ? 1 : e.n_sides;
+        for (int k = 0; k < l.n_sides; ++k) {
+            auto it = single.find(e.side[k]);
+            l.side[k] = e.kind == kSingle ? &e : it == single.end() ? nullptr : it->second;
+            for (int i = 0; l.side[k] && i < 3; ++i) l.need[k][i] = shape_bytes(l.side[k]->io[i].shape, l.side[k]->io[i].elem_bytes);
+        }
+        made->known.emplace(e.func, l);
+    }
+    made->built = r.size();
+    all.push_back(std::move(made));
+    current.store(all.back().get(), std::memory_order_release);
+    return *all.back();
+}
 const Launchable* launchable(const void* func)
 {
-    static std::unordered_map<const void*, Launchable> known;
-    static size_t built = 0;
-    const auto& r = registry();
-    if (built != r.size()) {
-        std::unordered_map<std::string, const KernelEntry*> single;
-        known.clear();
-        for (const auto& e : r)
-            if (e.kind == kSingle) single.emplace(e.name, &e);
-        for (const auto& e : r) {
-            Launchable l{};
-            l.e = &e;
-            l.n_sides = e.kind == kSingle ? 1 : e.n_sides;
-            for (int k = 0; k < l.n_sides; ++k) {
-                auto it = single.find(e.side[k]);
-                l.side[k] = e.kind == kSingle ? &e : it == single.end() ? nullptr : it->second;
-                for (int i = 0; l.side[k] && i < 3; ++i) l.need[k][i] = shape_bytes(l.side[k]->io[i].shape, l.side[k]->io[i].elem_bytes);
-            }
-            known.emplace(e.func, l);
-        }
-        built = r.size();
-    }
-    auto it = known.find(func);
-    return it == known.end() ? nullptr : &it->second;
+    const LaunchTable& t = launch_table();
+    auto it = t.known.find(func);
+    return it == t.known.end() ? nullptr : &it->second;
 }
 
 const KernelEntry* entry_of(const void* func)
