@@ -27,6 +27,7 @@
 #include <condition_variable>
 #include <cstdint>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <mutex>
 #include <thread>
@@ -156,7 +157,7 @@ public:
         if (total == 0) return hipSuccess;
         if (total <= kSmallBytes) return up_small(seg, n, total);
         if (busy && (e = hipDeviceSynchronize()) != hipSuccess) return e;   // the copy streams are ordered with no other
-        return pipeline(seg, n, true);
+        return pipeline_or_error(seg, n, true);
     }
 
     // Device -> host, in two steps around the caller's device synchronisation: begin() enqueues what can run behind the
@@ -209,7 +210,7 @@ public:
         std::lock_guard<std::mutex> lock(call_);
         for (int i = 0; i < d.n_packed; ++i) memcpy(d.packed[i].host, d.packed[i].dev, d.packed[i].bytes);
         end(d);
-        return d.n_later ? pipeline(d.later, d.n_later, false) : hipSuccess;
+        return d.n_later ? pipeline_or_error(d.later, d.n_later, false) : hipSuccess;
     }
 
     // Around a device synchronisation: what was on its way out of the arena before it is not any more.  Another thread may
@@ -237,7 +238,12 @@ public:
             (void)hipGetLastError();
             return nullptr;
         }
-        bufs_[(uintptr_t)p] = {size, true};
+        try {
+            bufs_[(uintptr_t)p] = {size, true};
+        } catch (const std::exception&) {
+            (void)hipHostFree(p);
+            return nullptr;
+        }
         total_bytes_ += size;
         return p;
     }
@@ -246,8 +252,15 @@ public:
         std::lock_guard<std::mutex> lock(pool_);
         auto it = bufs_.find((uintptr_t)p);
         if (it == bufs_.end() || !it->second.live) return false;
+        try {
+            idle_.emplace(it->second.size, p);
+        } catch (const std::exception&) {   // not kept, then
+            (void)hipHostFree(p);
+            total_bytes_ -= it->second.size;
+            bufs_.erase(it);
+            return true;
+        }
         it->second.live = false;
-        idle_.emplace(it->second.size, p);
         idle_bytes_ += it->second.size;
         if (idle_bytes_ > kIdleLimit) trim_idle(kIdleLimit);
         return true;
@@ -261,12 +274,11 @@ public:
             std::lock_guard<std::mutex> pool(pool_);
             trim_idle(0);
         }
-        if (device_ < 0) return;
+        drop_streams();
+        if (!ring_) return;
         stop_workers();
-        for (auto& s : stream_) (void)hipStreamDestroy(s);
         for (void* p : {(void*)ring_, (void*)in_.base, (void*)out_.base, (void*)flag_}) (void)hipHostFree(p);
         ring_ = nullptr;
-        device_ = -1;
     }
 
 private:
@@ -299,14 +311,23 @@ private:
             memset(flag_, 0, size[3]);
             start_workers();
         }
-        if (device_ >= 0) {   // another device was selected: streams belong to one
-            for (auto& s : stream_) (void)hipStreamDestroy(s);
-            device_ = -1;
-        }
-        for (auto& s : stream_)
-            if ((e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking)) != hipSuccess) return e;
+        hipStream_t made[2] = {};
+        for (auto& st : made)
+            if ((e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking)) != hipSuccess) {
+                if (made[0] && &st != made) (void)hipStreamDestroy(made[0]);
+                return e;   // the ring stays for the next call, or close()
+            }
+        drop_streams();     // another device was selected: streams belong to one
+        stream_[0] = made[0];
+        stream_[1] = made[1];
         device_ = dev;
         return hipSuccess;
+    }
+    void drop_streams()
+    {
+        if (device_ < 0) return;
+        for (auto& s : stream_) (void)hipStreamDestroy(s);
+        device_ = -1;
     }
 
     // p, which is on a 16-byte boundary, or as many bytes behind it as `dev` is behind one
@@ -369,6 +390,15 @@ private:
         else sched_yield();
     }
 
+    // The list of chunks is all that is allocated, before anything is enqueued: callers are entry points of C.
+    hipError_t pipeline_or_error(const CopySeg* seg, int n, bool up)
+    {
+        try {
+            return pipeline(seg, n, up);
+        } catch (const std::exception&) {
+            return hipErrorOutOfMemory;
+        }
+    }
     // Chunks in order, each in pieces.  Up: the threads claim pieces and fill the slots; this thread sends every chunk
     // whose slot is full and gives a slot back when its copy has ended.  Down: the other way round.  A piece is claimed
     // only when it can be moved at once (its slot is free, or its chunk has landed), so no thread ever holds a claim
@@ -376,18 +406,16 @@ private:
     hipError_t pipeline(const CopySeg* seg, int n, bool up)
     {
         std::vector<Chunk> chunks;
+        bool in_place[kMaxSegs] = {};
         long pieces = 0;
         size_t rest = 0;
         for (int i = 0; i < n; ++i) rest += seg[i].bytes;
         // Up, the first chunk's way through the host is time in which nothing is on the link; down, the last one's:
         // sizes double from kFirst, or halve to it (5 MB: 118 us up and 117 down against 152 and 136 in whole slots)
         size_t ramp = kFirst;
-        hipError_t e = hipSuccess;
-        bool wait = false;
         for (int i = 0; i < n; ++i) {
             if (up && pinned(seg[i].host, seg[i].bytes)) {
-                if ((e = hipMemcpyAsync(seg[i].dev, seg[i].host, seg[i].bytes, hipMemcpyHostToDevice, stream_[0])) != hipSuccess) break;
-                wait = true;
+                in_place[i] = true;
                 continue;
             }
             for (size_t o = 0, size; o < seg[i].bytes; o += size, rest -= size) {
@@ -402,6 +430,13 @@ private:
                 pieces += chunks.back().pieces();
             }
         }
+        hipError_t e = hipSuccess;
+        bool wait = false;
+        for (int i = 0; i < n && e == hipSuccess; ++i)
+            if (in_place[i]) {
+                e = hipMemcpyAsync(seg[i].dev, seg[i].host, seg[i].bytes, hipMemcpyHostToDevice, stream_[0]);
+                wait = true;
+            }
         const long count = (long)chunks.size();
         if (count && e == hipSuccess) {
             begin_job(chunks, up);
@@ -557,7 +592,12 @@ private:
         cpu_set_t set;
         int cores = sched_getaffinity(0, sizeof(set), &set) == 0 ? CPU_COUNT(&set) : 1;
         stop_ = false;
-        for (int i = 0; i < std::min(kMaxWorkers, cores / 2); ++i) workers_.emplace_back([this] { worker(); });
+        // fewer, or none, if the system gives no more: the thread that calls moves pieces too
+        try {
+            workers_.reserve(kMaxWorkers);
+            for (int i = 0; i < std::min(kMaxWorkers, cores / 2); ++i) workers_.emplace_back([this] { worker(); });
+        } catch (const std::exception&) {
+        }
     }
     void stop_workers()
     {

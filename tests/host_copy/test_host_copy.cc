@@ -1,5 +1,10 @@
 // host_copy.h over a stand-in for the HIP runtime (hip/hip_runtime.h beside this file): each test a name on the command line.
+#include <dlfcn.h>
+#include <pthread.h>
+
+#include <cerrno>
 #include <cstdio>
+#include <new>
 #include <string>
 
 #include "host_copy.h"
@@ -13,6 +18,22 @@ using namespace bfuse;
             exit(1);                                                    \
         }                                                               \
     } while (0)
+
+// allocations and threads that are to fail: the n-th from now
+static thread_local int new_fails_in = 0;
+static int thread_fails_in = 0;
+void* operator new(size_t n)
+{
+    if (new_fails_in > 0 && --new_fails_in == 0) throw std::bad_alloc();
+    return malloc(n);
+}
+void operator delete(void* p) noexcept { free(p); }
+void operator delete(void* p, size_t) noexcept { free(p); }
+extern "C" int pthread_create(pthread_t* t, const pthread_attr_t* a, void* (*f)(void*), void* arg)
+{
+    if (thread_fails_in > 0 && --thread_fails_in == 0) return EAGAIN;
+    return reinterpret_cast<decltype(&pthread_create)>(dlsym(RTLD_NEXT, "pthread_create"))(t, a, f, arg);
+}
 
 static HostCopy& hc() { return HostCopy::get(); }
 static std::vector<unsigned char> pattern(size_t n, unsigned seed)
@@ -159,6 +180,63 @@ static void given_up()
     CHECK(hc().release(p));
 }
 
+// Whatever fails while the first transfer sets up, the call says so, nothing is left behind, and the next one works.
+static void setup_fails()
+{
+    auto x = pattern(3 * HostCopy::kChunk, 3);
+    std::vector<unsigned char> dev(x.size());
+    const CopySeg seg = {dev.data(), x.data(), x.size()};
+    auto works = [&] {
+        std::fill(dev.begin(), dev.end(), 0);
+        CHECK(hc().up(&seg, 1, false) == hipSuccess && dev == x);
+    };
+    for (int n : {1, 2}) {
+        fake::fail_in["hipStreamCreateWithFlags"] = n;
+        CHECK(hc().up(&seg, 1, false) == hipErrorUnknown && fake::streams.empty());
+        hc().close();
+        CHECK(fake::host.empty());
+        fake::fail_in["hipStreamCreateWithFlags"] = n;
+        CHECK(hc().up(&seg, 1, false) == hipErrorUnknown);
+        works();
+        CHECK(fake::streams.size() == 2);
+        fake::device ^= 1;                                   // another device: the streams go over
+        fake::fail_in["hipStreamCreateWithFlags"] = n;
+        CHECK(hc().up(&seg, 1, false) == hipErrorUnknown && fake::streams.size() == 2);
+        works();
+        CHECK(fake::streams.size() == 2);
+        hc().close();
+    }
+    for (int n : {1, 2, 3, 4}) {
+        fake::fail_in["hipHostMalloc"] = n;
+        CHECK(hc().up(&seg, 1, false) == hipErrorOutOfMemory && fake::host.empty());
+    }
+    for (int n : {1, 2}) {
+        thread_fails_in = n;
+        works();
+        hc().close();
+    }
+    works();
+    for (int n : {1, 2, 3}) {
+        new_fails_in = n;
+        CHECK(hc().up(&seg, 1, false) == hipErrorOutOfMemory);
+        new_fails_in = 0;
+        works();
+        HostCopy::Down d;
+        std::vector<unsigned char> got(x.size());
+        const CopySeg back = {dev.data(), got.data(), got.size()};
+        CHECK(hc().down_begin(&back, 1, nullptr, d) == hipSuccess && hipDeviceSynchronize() == hipSuccess);
+        new_fails_in = n;
+        CHECK(hc().down_finish(d) == hipErrorOutOfMemory);
+        new_fails_in = 0;
+    }
+    const size_t pinned = fake::host.size();
+    new_fails_in = 2;                                        // the first is the stand-in's
+    CHECK(hc().host_buffer(1 << 20) == nullptr && fake::host.size() == pinned);
+    void* p = hc().host_buffer(1 << 20);
+    new_fails_in = 1;
+    CHECK(p && hc().release(p) && fake::host.size() == pinned && !hc().release(p));
+}
+
 int main(int argc, char** argv)
 {
     const std::string t = argc > 1 ? argv[1] : "";
@@ -166,6 +244,7 @@ int main(int argc, char** argv)
     else if (t == "in_flight") in_flight();
     else if (t == "arenas") arenas();
     else if (t == "given_up") given_up();
+    else if (t == "setup_fails") setup_fails();
     else return fprintf(stderr, "no test '%s'\n", t.c_str()), 2;
     hc().close();
     CHECK(fake::host.empty() && fake::streams.empty());

@@ -13,11 +13,11 @@ CSRC = os.path.join(os.path.dirname(HERE), "bfuse-project_amd", "csrc")
 def program(tmp_path_factory):
     exe = str(tmp_path_factory.mktemp("host_copy") / "test_host_copy")
     subprocess.run(["g++", "-O1", "-g", "-std=c++17", "-Wall", "-Wno-unused-function", "-pthread", "-I", os.path.join(HERE, "host_copy"), "-I", CSRC,
-                    os.path.join(HERE, "host_copy", "test_host_copy.cc"), "-o", exe], check=True)
+                    os.path.join(HERE, "host_copy", "test_host_copy.cc"), "-o", exe, "-ldl"], check=True)
     return exe
 
 
-@pytest.mark.parametrize("test", ["unaligned", "given_up", "arenas", "in_flight"])
+@pytest.mark.parametrize("test", ["unaligned", "given_up", "arenas", "in_flight", "setup_fails"])
 def test_host_copy(program, test):
     r = subprocess.run([program, test], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stderr
