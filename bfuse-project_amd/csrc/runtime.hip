@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <string>
 #include <map>
 #include <memory>
@@ -1081,14 +1082,21 @@ int run_parallel(const void* I1, const void* F1, void* O1, const void* I2, const
     const void* const src[2][2] = {{I1, F1}, {I2, F2}};
     void* const dst[2] = {O1, O2};
     const Side &a = g.side[0], &b = g.side[1];
-    if (std::min(a.bytes[0] + a.bytes[1], b.bytes[0] + b.bytes[1]) <= HostCopy::kSmallBytes) {
+    auto overlap = [](const void* p, size_t n, const void* q, size_t m) {
+        return std::less<>()(static_cast<const char*>(p), static_cast<const char*>(q) + m) && std::less<>()(static_cast<const char*>(q), static_cast<const char*>(p) + n);
+    };
+    // Operands of side 2 that lie in the memory of side 1's result are read before that is written: everything up, then
+    // everything down, as for small copies.
+    const bool in_turn = overlap(O1, a.bytes[2], I2, b.bytes[0]) || overlap(O1, a.bytes[2], F2, b.bytes[1]);
+    if (in_turn || std::min(a.bytes[0] + a.bytes[1], b.bytes[0] + b.bytes[1]) <= HostCopy::kSmallBytes) {
         if ((rc = upload_sides(both, src, 2))) return rc;
         if ((rc = enqueue_mode(BFUSE_MODE_PARALLEL, (const void*)func1, g1, b1, (const void*)func2, g2, b2, nullptr))) return rc;
         return download_sides(both, dst, 2, false);
     }
     // Long copies: each side runs through its own stream, so that side 1's kernel and the copy of its result (where it
     // can be copied in place) run while side 2's operands come up -- the link carries 96 GB/s both ways, 57 one way.
-    // Side 2's copies wait for nothing: only this call's launches are under way, over other buffers.
+    // Side 2's copies wait for nothing: only this call's launches are under way, over other buffers.  An error leaves by
+    // way of d's destructors, which wait for the copy of side 1's result.
     HostCopy::Down d[2];
     for (int k = 0; k < 2; ++k) {
         const CopySeg up[2] = {{g.side[k].buf[0], const_cast<void*>(src[k][0]), g.side[k].bytes[0]}, {g.side[k].buf[1], const_cast<void*>(src[k][1]), g.side[k].bytes[1]}};
