@@ -1030,8 +1030,8 @@ static int upload_sides(const int* idx, const void* const (*src)[2], int n)
         for (int t = 0; t < 2; ++t) seg[2 * k + t] = {g.side[idx[k]].buf[t], const_cast<void*>(src[k][t]), g.side[idx[k]].bytes[t]};
     return copy_up(seg, 2 * n, g_in_flight.any());
 }
-// waits for everything launched, then brings the results of `n` sides to the host; nothing is written there if a
-// barrier gave up, unless `always`
+// Waits for everything launched, then brings the results of `n` sides to the host.  If a barrier gave up nothing is written
+// there, unless `always` -- but into pinned buffers, whose copies run behind the launches, before anybody knows.
 static int download_sides(const int* idx, void* const* dst, int n, bool always)
 {
     CopySeg seg[kMaxKernels];

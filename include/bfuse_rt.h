@@ -229,7 +229,9 @@ int bfuse_synchronize(void);
  * memory goes through a staging ring.  NULL before bfuse_init, or when the library already has its limit of such
  * buffers (4 GiB) in existence: use ordinary memory then.  A released buffer is kept for the next request of its size
  * (up to 1 GiB in all) and given back by bfuse_shutdown; a buffer stays valid until it is released, whatever happens to
- * the operation.  Callable from any thread.  No counterpart in the reference. */
+ * the operation.  Copies into it run behind the launch: what a call that returns BFUSE_ERR_SYNC leaves in it is that
+ * launch's invalid result, where run_* leave other memory untouched.  Callable from any thread.  No counterpart in the
+ * reference. */
 void* bfuse_host_buffer(size_t bytes);
 int bfuse_host_buffer_release(void* buffer);
 
