@@ -169,20 +169,20 @@ BFUSE_KERNEL(selftest_sync_b, SyncProbeB, ({{768, 1, 1, 1}, 4}), ({{768, 1, 1, 1
 BFUSE_HFUSE_KERNEL(selftest_sync_a, SyncProbeA, selftest_sync_b, SyncProbeB)
 
 // The shared-tile convolution at the edges of its tiles (found by name only, so that nothing that walks the registry meets
-// them): tiles that run over several images, last tiles past the batch, strides, even and large filters, several channel
-// quads per stage, one stage and many.  <CI, CO, H, W, KH, KW, S, P, BM, 16-pixel blocks, stage channels, images, waves over BM>
-#define CONV_TILE_TEST(TAG, CI, CO, H, W, KH, KW, S, P, BM, PB, CPS, N, WM)                                        \
-    using ConvT_##TAG = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, CPS, N, WM>;                                \
+// them): tiles that run over several images, last tiles past the batch, strides, even and large filters, few stages and
+// many.  <CI, CO, H, W, KH, KW, S, P, BM, 16-pixel blocks, images, waves over BM>
+#define CONV_TILE_TEST(TAG, CI, CO, H, W, KH, KW, S, P, BM, PB, N, WM)                                             \
+    using ConvT_##TAG = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, 4, N, WM>;                                  \
     BFUSE_KERNEL(selftest_conv_tile_##TAG, ConvT_##TAG, ({{N, CI, H, W}, 4}), ({{CO, CI, KH, KW}, 4}),             \
                  ({{N, CO, (H - KH + 2 * P) / S + 1, (W - KW + 2 * P) / S + 1}, 4}))
-CONV_TILE_TEST(a, 16, 32, 5, 5, 3, 3, 1, 1, 32, 4, 4, 3, 1)         // 75 pixels of three images in two tiles of 64
-CONV_TILE_TEST(b, 32, 64, 9, 7, 3, 3, 2, 0, 32, 4, 8, 5, 2)         // stride 2, 60 pixels of five images in one tile, two quads a stage
-CONV_TILE_TEST(c, 16, 16, 11, 6, 5, 5, 1, 2, 16, 8, 4, 4, 1)        // 5 x 5, tiles of 128 over images of 66
-CONV_TILE_TEST(d, 16, 64, 20, 13, 3, 3, 4, 1, 64, 4, 4, 9, 2)       // stride 4, one window row per four image rows
-CONV_TILE_TEST(e, 48, 96, 8, 33, 3, 1, 1, 1, 96, 8, 4, 7, 2)        // 3 x 1 filter: an odd number of columns, twelve stages
-CONV_TILE_TEST(f, 16, 128, 7, 7, 3, 3, 1, 1, 128, 10, 4, 5, 2)      // 245 pixels in two tiles of 160, five blocks a wave
-CONV_TILE_TEST(g, 20, 48, 11, 11, 3, 3, 1, 1, 48, 20, 4, 3, 1)      // 363 pixels in two tiles of 320, an odd number of stages
-CONV_TILE_TEST(h, 64, 32, 9, 9, 3, 3, 1, 1, 32, 4, 4, 3, 1)         // sixteen stages, summed three at a time
+CONV_TILE_TEST(a, 16, 32, 5, 5, 3, 3, 1, 1, 32, 4, 3, 1)         // 75 pixels of three images in two tiles of 64
+CONV_TILE_TEST(b, 32, 64, 9, 7, 3, 3, 2, 0, 32, 4, 5, 2)         // stride 2, 60 pixels of five images in one tile
+CONV_TILE_TEST(c, 16, 16, 11, 6, 5, 5, 1, 2, 16, 8, 4, 1)        // 5 x 5, tiles of 128 over images of 66
+CONV_TILE_TEST(d, 16, 64, 20, 13, 3, 3, 4, 1, 64, 4, 9, 2)       // stride 4, one window row per four image rows
+CONV_TILE_TEST(e, 48, 96, 8, 33, 3, 1, 1, 1, 96, 8, 7, 2)        // 3 x 1 filter: an odd number of columns, twelve stages
+CONV_TILE_TEST(f, 16, 128, 7, 7, 3, 3, 1, 1, 128, 10, 5, 2)      // 245 pixels in two tiles of 160, five blocks a wave
+CONV_TILE_TEST(g, 20, 48, 11, 11, 3, 3, 1, 1, 48, 20, 3, 1)      // 363 pixels in two tiles of 320, an odd number of stages
+CONV_TILE_TEST(h, 64, 32, 9, 9, 3, 3, 1, 1, 32, 4, 3, 1)         // sixteen stages, summed three at a time
 BFUSE_HFUSE_KERNEL(selftest_conv_tile_a, ConvT_a, bias_relu_4096, BiasReluS)
 BFUSE_BFUSE_KERNEL(selftest_conv_tile_b, ConvT_b, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
 BFUSE_HFUSE_KERNEL(selftest_conv_tile_c, ConvT_c, conv3x3_f32_32x12x12_32, ConvS2)
@@ -209,7 +209,7 @@ BFUSE_KERNEL(selftest_gemm_ring4, GemmRing4, ({{128, 704, 1, 1}, 2}), ({{1024, 7
 CONV1_TILE_TEST(a, 16, 32, 5, 5, 1, 3, 32, 256, 1, 16, 3)        // one stage, three images of 25 pixels in one tile
 CONV1_TILE_TEST(b, 64, 80, 9, 9, 1, 5, 80, 256, 1, 32, 2)        // five images of 81 in two tiles, a row tile that is no whole round of loads
 CONV1_TILE_TEST(c, 48, 112, 9, 7, 2, 11, 96, 128, 2, 16, 3)      // stride 2 (20 pixels an image), row tiles that overlap
-CONV1_TILE_TEST(d, 32, 64, 8, 8, 1, 7, 64, 128, 2, 16, 4)        // fewer stages than buffers, whole chunks
+CONV1_TILE_TEST(d, 32, 64, 8, 8, 1, 7, 64, 128, 2, 16, 3)        // fewer stages than buffers, whole chunks
 BGEMM_TILE_TEST(e, 3, 160, 48, 144, 128, 128, 2, 16, 3)          // row and column tiles that overlap
 BGEMM_TILE_TEST(f, 8, 64, 32, 64, 64, 64, 4, 32, 2)              // one stage, products dealt to the XCDs
 BGEMM_TILE_TEST(g, 2, 64, 512, 64, 64, 64, 4, 32, 3)             // two sums of 256 k

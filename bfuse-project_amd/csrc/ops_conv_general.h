@@ -40,7 +40,7 @@ namespace bfuse {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
-// WM_ = 0: this form.  WM_ > 0 (ops_conv_tile.h): large tiles that the waves of a workgroup share.
+// WM_ = 0: this form.  WM_ = 1 or 2 (ops_conv_tile.h): large tiles that the waves of a workgroup share.
 template <int CI_, int CO_, int H_, int W_, int KH_, int KW_, int S_, int P_, int BM_, int PB_, int KS_, int NIMG_ = 1, int WM_ = 0>
 struct ConvF32Lds {
     static constexpr bool MATRIX_CORES = true;   // the inner loop is a stream of MFMAs (what the fusion chooser asks)
@@ -67,6 +67,7 @@ struct ConvF32Lds {
     static constexpr int NU = R * W / VW;               // staging units per channel
     static constexpr int NLD = (NU + LPC - 1) / LPC;    // wave-level loads per group
     static constexpr int NZ = (TILE_BYTES + 1023) / 1024;
+    static_assert(WM_ == 0, "shared tiles have stages of four channels and one or two waves over the output channels");
     static_assert(CG == 16 ? CI % 16 == 0 : CI <= 4, "input channels: a multiple of 16, or at most 4");
     static_assert(CO % BM == 0 && BM % 16 == 0 && NGROUP % KS == 0, "channel tiling");
     static_assert(((KH - 1) * WP + KW - 1) * 16 + (NQ - 1) * PLANE + 16 < 65536, "tap offsets are 16-bit immediates");

@@ -7,8 +7,8 @@
 // the 154 the matrix cores sustain.  Here
 //   * one workgroup of four waves owns BM output channels x BP consecutive pixels OF THE BATCH (a tile runs on into
 //     the next image: no ragged tiles but the batch's last), each wave a (BM / WM) x (BP / WN) part of it;
-//   * both operands of CPS input channels (a stage) are shared by the four waves: the filter rows, which are
-//     contiguous in memory ([CPS channels][T taps] per output channel), and the image patch, one plane per channel;
+//   * both operands of four input channels (a stage) are shared by the four waves: the filter rows, which are
+//     contiguous in memory ([4 channels][T taps] per output channel), and the image patch, one plane per channel;
 //   * both go from memory straight into LDS: the filter by 16-byte loads with a scalar base, the patch by 4-byte loads
 //     whose per-lane offset (which image element belongs at this position of the patch) does not change from stage to
 //     stage -- only a scalar offset moves on.  Padding and rows outside the image are lanes whose offset lies past the
@@ -16,9 +16,9 @@
 //   * two LDS buffers and one barrier per stage: the next stage lands while this one is multiplied (9 taps x 4
 //     channels of a 128 x 128 tile are 144 MFMAs = 4600 clocks per wave).
 //
-// A operand (rows = output channels) of tap t, channel quad c4: lane (i, q) reads A[i][(4 c4 + q) * T + t]: a row is
-// CPS * T words, for T = 9 the 64 lanes hit 64 banks.  B operand (columns = pixels): lane (i, q) reads plane
-// 4 c4 + q at the position of its pixel's window plus a compile-time offset per tap; the four planes start
+// A operand (rows = output channels) of tap t: lane (i, q) reads A[i][q * T + t]: a row is
+// 4 T words, for T = 9 the 64 lanes hit 64 banks.  B operand (columns = pixels): lane (i, q) reads plane
+// q at the position of its pixel's window plus a compile-time offset per tap; the four planes start
 // PLANE_BANK(q) banks apart so that lanes of different channels do not meet (stride 1: 16 consecutive words each;
 // stride 2: 16 even words of 32; more: a word in four).
 #pragma once
@@ -45,14 +45,15 @@ __device__ __forceinline__ void dma_buffer_lds_b32(unsigned voff, i32x4 rsrc, un
 #endif
 }
 
-template <int CI_, int CO_, int H_, int W_, int KH_, int KW_, int S_, int P_, int BM_, int BP_, int WM_, int CPS_, int NIMG_>
+template <int CI_, int CO_, int H_, int W_, int KH_, int KW_, int S_, int P_, int BM_, int BP_, int WM_, int NIMG_>
 struct ConvF32Tile {
     static constexpr bool MATRIX_CORES = true;   // the inner loop is a stream of MFMAs (what the fusion chooser asks)
-    static constexpr int CI = CI_, CO = CO_, H = H_, W = W_, KH = KH_, KW = KW_, S = S_, P = P_, BM = BM_, BP = BP_, WM = WM_, CPS = CPS_, NIMG = NIMG_;
+    static constexpr int CI = CI_, CO = CO_, H = H_, W = W_, KH = KH_, KW = KW_, S = S_, P = P_, BM = BM_, BP = BP_, WM = WM_, NIMG = NIMG_;
     static constexpr int OH = (H - KH + 2 * P) / S + 1, OW = (W - KW + 2 * P) / S + 1;
     static constexpr int HW = H * W, OHW = OH * OW, T = KH * KW;
     static constexpr int NWAVE = 4, WN = NWAVE / WM;
     static constexpr int TM = BM / WM / 16, TN = BP / WN / 16;      // 16 x 16 blocks of a wave
+    static constexpr int CPS = 4;                                   // channels of a stage: the four k of an MFMA, a plane per wave
     static constexpr int NS = CI / CPS;                             // stages
     // One accumulator over the whole reduction rounds after every four products of it: 256 -> 256 channels on 14 x 14 are
     // 5.8e-7 off (2-norm, against 64 bits) where the per-wave forms' four partial sums are 2.9e-7 off.  So the sum of every
@@ -64,8 +65,8 @@ struct ConvF32Tile {
     static constexpr long long NPIX = (long long)OHW * NIMG;
     static constexpr long long TILES = (NPIX + BP - 1) / BP * (CO / BM);
     static constexpr int NPT = (int)((NPIX + BP - 1) / BP), NCT = CO / BM;
-    static_assert(CI % CPS == 0 && CPS % 4 == 0 && CO % BM == 0 && BM % (16 * WM) == 0 && BP % (16 * WN) == 0, "channel tiling");
-    static_assert((CI * T) % 4 == 0 && (CPS * T) % 4 == 0, "filter rows are whole 16-byte chunks");
+    static_assert(CI % CPS == 0 && CPS == NWAVE && CO % BM == 0 && BM % (16 * WM) == 0 && BP % (16 * WN) == 0, "channel tiling");
+    static_assert((CI * T) % 4 == 0, "filter rows are whole 16-byte chunks");
 
     // ---- the patch: the image rows under the tile's output rows, image after image, every column a window touches.
     // Image n's rows are HR virtual rows (its OH windows' rows -P .. ), one image after the other.
@@ -100,14 +101,12 @@ struct ConvF32Tile {
     static constexpr int NLB = (NPOS + 63) / 64;                     // wave-level loads per plane
     static constexpr int PLANE = NLB * 64;                            // words
     __host__ __device__ static constexpr int plane_bank(int q) { return S == 1 ? 16 * q : S == 2 ? 32 * (q / 2) + q % 2 : q; }
-    static constexpr int QUAD = 4 * PLANE + 64;                       // words of four planes: the last one's end is past the next quad's start otherwise
     static constexpr int A_CHUNKS = BM * CPS * T / 4;                // 16-byte chunks of the filter rows
     static constexpr int NLA = (A_CHUNKS + 63) / 64;
     static constexpr int A_BYTES = NLA * 1024;
-    static constexpr int B_BYTES = CPS / 4 * QUAD * 4;
+    static constexpr int B_BYTES = (CPS * PLANE + 64) * 4;           // 64: the last plane starts up to 48 words late
     static constexpr int BUF = (A_BYTES + B_BYTES + 255) / 256 * 256;
     static constexpr int NLA_W = (NLA + NWAVE - 1) / NWAVE;          // per wave
-    static constexpr int PLANES_W = CPS / NWAVE;                     // planes a wave loads
     // fragment offsets are 16-bit immediates; two workgroups share a CU; the images of a tile are one buffer, whose size is 31
     // bits: an offset of 2^31 - 1 has to lie past its end
     static constexpr bool FITS = A_BYTES + B_BYTES < 65536 && 4 * BUF <= 160 * 1024 && NLB <= MOST_LOADS && TILES < (1LL << 31) &&
@@ -157,14 +156,10 @@ struct ConvF32Tile {
             const int l = j * NWAVE + c.wave;
             if (NLA % NWAVE == 0 || l < NLA) dma_load_lds_b128(c.a_voff[j], c.a_ub + (size_t)s * (CPS * T * 4), dst + l * 1024);
         }
+        const unsigned soff = (unsigned)(s * CPS + c.wave) * (unsigned)(HW * 4);
+        const unsigned plane = dst + A_BYTES + (unsigned)(c.wave * PLANE + plane_bank(c.wave)) * 4u;
 #pragma unroll
-        for (int k = 0; k < PLANES_W; ++k) {
-            const int ci = k * NWAVE + c.wave;           // plane of the stage; quad k, channel `wave` of it
-            const unsigned soff = (unsigned)(s * CPS + ci) * (unsigned)(HW * 4);
-            const unsigned plane = dst + A_BYTES + (unsigned)(k * QUAD + c.wave * PLANE + plane_bank(c.wave)) * 4u;
-#pragma unroll
-            for (int l = 0; l < NLB; ++l) dma_buffer_lds_b32(c.b_voff[l], c.rsrc, soff, plane + l * 256);
-        }
+        for (int l = 0; l < NLB; ++l) dma_buffer_lds_b32(c.b_voff[l], c.rsrc, soff, plane + l * 256);
     }
 
     template <class Sync>
@@ -237,30 +232,29 @@ struct ConvF32Tile {
             sync.raw();
             if (s + 1 < NS) issue(c, s + 1, (s + 1) & 1);
 
-            constexpr int NK = CPS / 4 * T;        // k-steps of the stage: (channel quad, tap)
             float a[2][TM], b[2][TN];
 #pragma unroll
             for (int tm = 0; tm < TM; ++tm) a[0][tm] = *reinterpret_cast<const float*>(ap + tm * 16 * CPS * T * 4);
 #pragma unroll
             for (int tn = 0; tn < TN; ++tn) b[0][tn] = *reinterpret_cast<const float*>(bp[tn]);
 #pragma unroll
-            for (int k = 0; k < NK; ++k) {
-                if (k + 1 < NK) {
-                    const int c4 = (k + 1) / T, tap = (k + 1) % T;
+            for (int tap = 0; tap < T; ++tap) {
+                if (tap + 1 < T) {
+                    const int next = tap + 1;
 #pragma unroll
                     for (int tm = 0; tm < TM; ++tm)
-                        a[(k + 1) & 1][tm] = *reinterpret_cast<const float*>(ap + (tm * 16 * CPS * T + c4 * 4 * T + tap) * 4);
+                        a[next & 1][tm] = *reinterpret_cast<const float*>(ap + (tm * 16 * CPS * T + next) * 4);
 #pragma unroll
                     for (int tn = 0; tn < TN; ++tn)
-                        b[(k + 1) & 1][tn] = *reinterpret_cast<const float*>(bp[tn] + (c4 * QUAD + (tap / KW) * WPS + tap % KW) * 4);
+                        b[next & 1][tn] = *reinterpret_cast<const float*>(bp[tn] + ((next / KW) * WPS + next % KW) * 4);
                 }
 #pragma unroll
                 for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
                     for (int tn = 0; tn < TN; ++tn)
-                        acc[tm][tn] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k & 1][tm], b[k & 1][tn], acc[tm][tn], 0, 0, 0);
-                // the next k-step's reads one by one between this one's MFMAs
-                if (k + 1 < NK) {
+                        acc[tm][tn] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[tap & 1][tm], b[tap & 1][tn], acc[tm][tn], 0, 0, 0);
+                // the next tap's reads one by one between this one's MFMAs
+                if (tap + 1 < T) {
 #pragma unroll
                     for (int r = 0; r < TM + TN; ++r) {
                         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                              // an LDS read
@@ -311,9 +305,9 @@ struct ConvF32Tile {
 
 // The shared-tile form under ConvF32Lds's name: WM_ waves over the output channels, KS_ is the stage's channels, PB_ counts
 // the workgroup's 16-pixel blocks as there.
-template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int BM, int PB, int KS, int NIMG>
-struct ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, KS, NIMG, 1> : ConvF32Tile<CI, CO, H, W, KH, KW, S, P, BM, 16 * PB, 1, KS, NIMG> {};
-template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int BM, int PB, int KS, int NIMG>
-struct ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, KS, NIMG, 2> : ConvF32Tile<CI, CO, H, W, KH, KW, S, P, BM, 16 * PB, 2, KS, NIMG> {};
+template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int BM, int PB, int NIMG>
+struct ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, 4, NIMG, 1> : ConvF32Tile<CI, CO, H, W, KH, KW, S, P, BM, 16 * PB, 1, NIMG> {};
+template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int BM, int PB, int NIMG>
+struct ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, 4, NIMG, 2> : ConvF32Tile<CI, CO, H, W, KH, KW, S, P, BM, 16 * PB, 2, NIMG> {};
 
 }  // namespace bfuse

@@ -84,7 +84,7 @@ struct GemmTile {
     static constexpr int B_BYTES = BN * KS * 4, BUF = A_BYTES + B_BYTES;
     static constexpr int B_W = (GATHER ? B_BYTES / 256 : B_BYTES / 1024) / NWAVE;
     static constexpr int LPS = A_W + B_W;
-    static_assert(BUF < 65536 && B_BYTES % (NWAVE * 1024) == 0 && (NBUF - 2) * LPS <= 63 && NBUF >= 2, "fragment offsets are 16-bit immediates");
+    static_assert(BUF < 65536 && B_BYTES % (NWAVE * 1024) == 0 && (NBUF - 2) * LPS <= 63 && (NBUF == 2 || NBUF == 3), "fragment offsets are 16-bit immediates");
     static constexpr int RC = KS / 4;                                            // 16-byte chunks of a row
 
     struct Smem {

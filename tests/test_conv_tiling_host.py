@@ -11,8 +11,8 @@ PROLOGUE = """
 #include "ops_conv_1x1.h"
 #include "ops_conv_rect.h"
 using namespace bfuse;
-template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int BM, int BP, int WM, int CPS, int NIMG>
-std::true_type shared(const ConvF32Tile<CI, CO, H, W, KH, KW, S, P, BM, BP, WM, CPS, NIMG>*);
+template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int BM, int BP, int WM, int NIMG>
+std::true_type shared(const ConvF32Tile<CI, CO, H, W, KH, KW, S, P, BM, BP, WM, NIMG>*);
 template <int M, int K, int H, int W, int S, int NIMG, int BM, int BN, int WM, int KS, int LAYOUT, int NBUF>
 std::true_type shared(const GemmTile<M, K, H, W, S, NIMG, BM, BN, WM, KS, LAYOUT, NBUF>*);
 std::false_type shared(const void*);
@@ -82,5 +82,5 @@ def test_rows_of_a_patch_against_a_look_at_every_tile(tmp_path):
         pixels = ((h - k + 2 * p) // s + 1) * ((w - k + 2 * p) // s + 1)
         for images in (1, 2, 3, n):
             whole = (images - 1) * math.gcd(pixels, bp) >= bp          # every place that an image's end has in a tile comes up
-            text += f"static_assert(rows_are_right<ConvF32Tile<16, 32, {h}, {w}, {k}, {k}, {s}, {p}, 32, {bp}, {2 if bp % 32 == 0 else 1}, 4, {images}>>({'true' if whole else 'false'}));\n"
+            text += f"static_assert(rows_are_right<ConvF32Tile<16, 32, {h}, {w}, {k}, {k}, {s}, {p}, 32, {bp}, {2 if bp % 32 == 0 else 1}, {images}>>({'true' if whole else 'false'}));\n"
     _compiles(text, tmp_path)
