@@ -13,7 +13,7 @@
 //     the end of a copy by a word in host memory (128 MB: 56 GB/s up, 53 down; with an event behind every copy 46 and
 //     47, with a copy engine 38);
 //   * host memory that came from host_buffer() is pinned and copied in place, with no slot and no thread in between.
-// run_fuse over 0.3 MB: 111 -> 56 us; run_parallel over 600 MB: 36 -> 10.4 ms (the link's floor: 6.4 up + what of the 4.4
+// run_fuse over 0.3 MB: 111 -> 44 us; run_parallel over 600 MB: 36 -> 8.6 ms (the link's floor: 6.4 up + what of the 4.4
 // down is not under it).  up() returns with the copied bytes on their way into place before anything launched later;
 // down_begin / down_finish leave the wait to the caller's own synchronisation.
 #pragma once
@@ -47,7 +47,7 @@ struct SegList {
     struct {
         const unsigned char* src;
         unsigned char* dst;
-        size_t bytes;
+        unsigned bytes;
     } s[kMaxSegs];
     int n;
 };
@@ -56,9 +56,9 @@ struct SegList {
 // chosen to lie like the device memory relative to such a boundary (see lie()): whatever a part's offset, all but up to 15
 // bytes at either end move as 16-byte words.  (48 MB at an offset of one float: 1.0 ms up and down; in single bytes, 64 of
 // them a wave's request, 15.2 up and 2.3 down.)
-static __device__ __forceinline__ size_t head_of(const void* p, size_t bytes)
+static __device__ __forceinline__ unsigned head_of(const void* p, unsigned bytes)
 {
-    const size_t head = (16 - ((uintptr_t)p & 15)) & 15;
+    const unsigned head = -(unsigned)(uintptr_t)p & 15;
     return head < bytes ? head : bytes;
 }
 
@@ -66,13 +66,13 @@ static __device__ __forceinline__ size_t head_of(const void* p, size_t bytes)
 // consecutive 16-byte words (one PCIe request per 64 bytes and more), every block strides over every segment.
 static __global__ __launch_bounds__(256) void copy_segments(SegList l)
 {
-    const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x, nt = (size_t)gridDim.x * 256;
+    const unsigned t = blockIdx.x * 256 + threadIdx.x, nt = gridDim.x * 256;
     for (int k = 0; k < l.n; ++k) {
         const unsigned char* const src = l.s[k].src;
         unsigned char* const dst = l.s[k].dst;
-        const size_t bytes = l.s[k].bytes, head = head_of(dst, bytes), words = (bytes - head) / 16, ends = bytes - 16 * words;
-        for (size_t i = t; i < words; i += nt) reinterpret_cast<uint4*>(dst + head)[i] = reinterpret_cast<const uint4*>(src + head)[i];
-        for (size_t i = t; i < ends; i += nt) dst[i < head ? i : 16 * words + i] = src[i < head ? i : 16 * words + i];
+        const unsigned bytes = l.s[k].bytes, head = head_of(dst, bytes), words = (bytes - head) / 16, ends = bytes - 16 * words;
+        for (unsigned i = t; i < words; i += nt) reinterpret_cast<uint4*>(dst + head)[i] = reinterpret_cast<const uint4*>(src + head)[i];
+        if (t < ends) dst[t < head ? t : 16 * words + t] = src[t < head ? t : 16 * words + t];
     }
 }
 
@@ -81,13 +81,13 @@ static __global__ __launch_bounds__(256) void copy_segments(SegList l)
 // would tell the same, but recording one holds the stream's next kernel up for 5 us and the host for 3.  Four words are
 // in flight per thread: fewer, fatter blocks keep the link as full and leave it less to switch between (128 MB up: 56
 // GB/s with 8 blocks, 53 with 16, 50 with 32, 45 with 64; down it is the other way round, 52, 53, 53, 54).
-static __global__ __launch_bounds__(256) void copy_chunk(const unsigned char* src, unsigned char* dst, size_t bytes, unsigned* flag, unsigned value)
+static __global__ __launch_bounds__(256) void copy_chunk(const unsigned char* src, unsigned char* dst, unsigned bytes, unsigned* flag, unsigned value)
 {
-    const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x, nt = (size_t)gridDim.x * 256;
-    const size_t head = head_of(dst, bytes), words = (bytes - head) / 16, ends = bytes - 16 * words;
+    const unsigned t = blockIdx.x * 256 + threadIdx.x, nt = gridDim.x * 256;
+    const unsigned head = head_of(dst, bytes), words = (bytes - head) / 16, ends = bytes - 16 * words;
     const uint4* const s = reinterpret_cast<const uint4*>(src + head);
     uint4* const d = reinterpret_cast<uint4*>(dst + head);
-    size_t i = t;
+    unsigned i = t;
     for (; i + 3 * nt < words; i += 4 * nt) {
         const uint4 a = s[i], b = s[i + nt], c = s[i + 2 * nt], e = s[i + 3 * nt];
         d[i] = a;
@@ -96,7 +96,7 @@ static __global__ __launch_bounds__(256) void copy_chunk(const unsigned char* sr
         d[i + 3 * nt] = e;
     }
     for (; i < words; i += nt) d[i] = s[i];
-    for (i = t; i < ends; i += nt) dst[i < head ? i : 16 * words + i] = src[i < head ? i : 16 * words + i];
+    if (t < ends) dst[t < head ? t : 16 * words + t] = src[t < head ? t : 16 * words + t];
 #if defined(__HIP_DEVICE_COMPILE__)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // each wave's own stores have left it; the barrier alone does not wait for them
 #endif
@@ -132,7 +132,6 @@ public:
     static constexpr size_t kFirst = 256 << 10;             // the first copy of a transfer up, the last of one down
     static constexpr size_t kPiece = 64 << 10;              // what a thread moves at a time: the first copy waits for four of them at once
     static constexpr int kSlots = 8;                        // 16 MiB
-    static constexpr size_t kSlotBytes = kChunk + 64;       // a chunk, wherever it lies in its 16 bytes
     static constexpr int kUpBlocks = 8, kDownBlocks = 16;   // of copy_chunk
     static constexpr int kFlagWords = 16;                   // a cache line of one word per block
     static constexpr unsigned kQuietSpins = 100000;
@@ -195,7 +194,7 @@ public:
             if (seg[i].bytes == 0) continue;
             // (the arena holds kArenaBytes / kSmallBytes transfers: of more threads at once, the others take the ring)
             if (unsigned char* p = total <= kSmallBytes ? arena(out_, seg[i].bytes, seg[i].dev) : nullptr) {
-                l.s[l.n++] = {static_cast<const unsigned char*>(seg[i].dev), p, seg[i].bytes};
+                l.s[l.n++] = {static_cast<const unsigned char*>(seg[i].dev), p, (unsigned)seg[i].bytes};
                 d.packed[d.n_packed++] = {p, seg[i].host, seg[i].bytes};
             } else if (pinned(seg[i].host, seg[i].bytes)) {
                 if ((e = hipMemcpyAsync(seg[i].host, seg[i].dev, seg[i].bytes, hipMemcpyDeviceToHost, stream)) != hipSuccess) return e;
@@ -298,7 +297,7 @@ private:
         if (e != hipSuccess || dev == device_) return e;
         if (!ring_) {
             void* p[4] = {};
-            const size_t size[4] = {kSlotBytes * kSlots, kArenaBytes, kArenaBytes, kSlots * kFlagWords * sizeof(unsigned)};
+            const size_t size[4] = {kChunk * kSlots, kArenaBytes, kArenaBytes, kSlots * kFlagWords * sizeof(unsigned)};
             for (int i = 0; i < 4; ++i)
                 if ((e = hipHostMalloc(&p[i], size[i], hipHostMallocPortable)) != hipSuccess) {
                     for (int j = 0; j < i; ++j) (void)hipHostFree(p[j]);
@@ -340,7 +339,7 @@ private:
         a.used += need;
         return lie(p, dev);
     }
-    unsigned char* slot_of(long i, const void* dev) const { return lie(ring_ + (size_t)(i % kSlots) * kSlotBytes, dev); }
+    unsigned char* slot_of(long i, const void* dev) const { return lie(ring_ + (size_t)(i % kSlots) * kChunk, dev); }
     // 64 blocks: from 8 to 512 reach the link's rate on long copies; short ones want every request out at once
     static hipError_t launch(const SegList& l, size_t total, hipStream_t stream)
     {
@@ -370,7 +369,7 @@ private:
             if (seg[i].bytes == 0) continue;
             unsigned char* p = arena(in_, seg[i].bytes, seg[i].dev);
             memcpy(p, seg[i].host, seg[i].bytes);
-            l.s[l.n++] = {p, static_cast<unsigned char*>(seg[i].dev), seg[i].bytes};
+            l.s[l.n++] = {p, static_cast<unsigned char*>(seg[i].dev), (unsigned)seg[i].bytes};
         }
         const hipError_t e = launch(l, total, nullptr);
         small_ups_.add();
@@ -414,16 +413,17 @@ private:
         // sizes double from kFirst, or halve to it (5 MB: 118 us up and 117 down against 152 and 136 in whole slots)
         size_t ramp = kFirst;
         for (int i = 0; i < n; ++i) {
+            const size_t most = ((uintptr_t)seg[i].dev & 15) ? kChunk - kPiece : kChunk;   // it starts up to 15 bytes into its slot
             if (up && pinned(seg[i].host, seg[i].bytes)) {
                 in_place[i] = true;
                 continue;
             }
             for (size_t o = 0, size; o < seg[i].bytes; o += size, rest -= size) {
                 if (up) {
-                    size = ramp;
+                    size = std::min(most, ramp);
                     ramp = std::min(kChunk, 2 * ramp);
                 } else {
-                    size = std::min(kChunk, std::max(kFirst, (rest / 2 + kPiece - 1) / kPiece * kPiece));
+                    size = std::min(most, std::max(kFirst, (rest / 2 + kPiece - 1) / kPiece * kPiece));
                 }
                 size = std::min(size, seg[i].bytes - o);
                 chunks.push_back({static_cast<unsigned char*>(seg[i].dev) + o, static_cast<unsigned char*>(seg[i].host) + o, size, pieces});
@@ -451,7 +451,7 @@ private:
                     const Chunk& c = chunks[(size_t)sent];
                     if (!up) left_[slot].store(c.pieces(), std::memory_order_relaxed);
                     unsigned char* const s = slot_of(sent, c.dev);
-                    hipLaunchKernelGGL(copy_chunk, dim3(up ? kUpBlocks : kDownBlocks), dim3(256), 0, stream_[sent & 1], up ? s : c.dev, up ? c.dev : s, c.bytes, flag_ + slot * kFlagWords,
+                    hipLaunchKernelGGL(copy_chunk, dim3(up ? kUpBlocks : kDownBlocks), dim3(256), 0, stream_[sent & 1], up ? s : c.dev, up ? c.dev : s, (unsigned)c.bytes, flag_ + slot * kFlagWords,
                                        base + (unsigned)sent);
                     e = hipGetLastError();
                     ++sent;

@@ -128,7 +128,7 @@ template <class F, class... A> void fake_run(F kernel, dim3 grid, dim3 block, A.
             kernel(args...);
         }
 }
-template <class F> void fake_launch(F kernel, dim3 grid, dim3 block, hipStream_t s, const unsigned char* src, unsigned char* dst, size_t bytes, unsigned* flag, unsigned value)
+template <class F> void fake_launch(F kernel, dim3 grid, dim3 block, hipStream_t s, const unsigned char* src, unsigned char* dst, unsigned bytes, unsigned* flag, unsigned value)
 {
     std::lock_guard<std::recursive_mutex> lock(fake::m);
     if (fake::seen) fake::seen(src, dst, bytes);
