@@ -146,6 +146,30 @@ static void arenas()
     CHECK(to[0] == from[29 % kMany]);
 }
 
+// Threads that move what is their own, small and long, and wait when they like.
+static void threads()
+{
+    fake::deferred = true;
+    std::vector<std::thread> all;
+    for (int id = 0; id < 4; ++id)
+        all.emplace_back([id] {
+            for (int k = 0; k < 60; ++k) {
+                const size_t n = k % 6 == 5 ? HostCopy::kSmallBytes + 7777 * id + 1 : 100 + 30000 * ((k + id) % 4);
+                std::vector<unsigned char> dev(n + 16), got(n);
+                const auto x = pattern(n, 100 * id + k);
+                const CopySeg up = {dev.data() + k % 16, const_cast<unsigned char*>(x.data()), n}, down = {dev.data() + k % 16, got.data(), n};
+                CHECK(hc().up(&up, 1, false) == hipSuccess);
+                HostCopy::Down d;
+                CHECK(hc().down_begin(&down, 1, nullptr, d) == hipSuccess);
+                const unsigned long begun = hc().wait_begins();
+                CHECK(hipDeviceSynchronize() == hipSuccess);
+                hc().wait_ended(begun);
+                CHECK(hc().down_finish(d) == hipSuccess && got == x);
+            }
+        });
+    for (auto& t : all) t.join();
+}
+
 // Copies into a caller's pinned memory have ended when a transfer that failed is given up.
 static void given_up()
 {
@@ -243,6 +267,7 @@ int main(int argc, char** argv)
     if (t == "unaligned") unaligned();
     else if (t == "in_flight") in_flight();
     else if (t == "arenas") arenas();
+    else if (t == "threads") threads();
     else if (t == "given_up") given_up();
     else if (t == "setup_fails") setup_fails();
     else return fprintf(stderr, "no test '%s'\n", t.c_str()), 2;

@@ -12,7 +12,7 @@ from bfuse_project_amd import _lib
 pytestmark = pytest.mark.gpu
 
 N = 16777216                     # floats of copy_f32_16777216
-SMALL, PIECE, CHUNK, RING = (512 << 10) // 4, (256 << 10) // 4, (2 << 20) // 4, (16 << 20) // 4
+SMALL, PIECE, FIRST, CHUNK, RING = (512 << 10) // 4, (64 << 10) // 4, (256 << 10) // 4, (2 << 20) // 4, (16 << 20) // 4
 
 
 @pytest.fixture(scope="module")
@@ -21,8 +21,8 @@ def op():
         yield o
 
 
-@pytest.mark.parametrize("offset,count", [(0, 1), (3, 5), (1, SMALL), (0, SMALL + 1), (7, PIECE * 5 + 3), (0, 3 * PIECE), (4, 7 * PIECE + 1), (0, 4 * CHUNK), (2, 4 * CHUNK + 1),
-                                          (0, RING), (5, RING + CHUNK + 1), (0, N)])
+@pytest.mark.parametrize("offset,count", [(0, 1), (3, 5), (1, SMALL), (0, SMALL + 1), (7, FIRST * 5 + 3), (0, 3 * FIRST), (4, 7 * FIRST + 1), (0, 9 * PIECE), (1, 9 * PIECE + 1),
+                                          (3, 13 * PIECE - 1), (0, 4 * CHUNK), (2, 4 * CHUNK + 1), (0, RING), (5, RING + CHUNK + 1), (0, N)])
 def test_a_part_goes_up_and_comes_back_unchanged(op, offset, count):
     rng = np.random.default_rng(count)
     x = rng.integers(0, 1 << 32, count, np.uint32).view(np.float32)
@@ -40,7 +40,7 @@ def test_a_part_goes_up_and_comes_back_unchanged(op, offset, count):
 
 
 def test_the_last_of_many_uploads_without_a_wait_is_what_stands(op):
-    count = SMALL + PIECE + 1
+    count = SMALL + FIRST + 1
     for k in range(700):
         x = np.full(count, k, np.float32)
         op.upload_part(0, 0, 0, x)

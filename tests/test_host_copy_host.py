@@ -17,7 +17,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("test", ["unaligned", "given_up", "arenas", "in_flight", "setup_fails"])
+@pytest.mark.parametrize("test", ["unaligned", "given_up", "arenas", "in_flight", "threads", "setup_fails"])
 def test_host_copy(program, test):
     r = subprocess.run([program, test], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stderr
