@@ -374,20 +374,20 @@ struct ConvTiling {
     using held = std::conditional_t<(RESERVE > 0), LdsReserve<staged, (RESERVE > 0 ? RESERVE : 1)>, staged>;
     // A batch with enough pixels for two workgroups per CU goes to the shared-tile form, with the largest tile whose
     // part of each wave is at least twelve 16 x 16 blocks: measured at batch 1024 over the 3 x 3 and 5 x 5 layers it
-    // takes 0.40-0.82 of the time of the per-wave forms above (107-142 TFLOP/s against 52-115); with eight blocks per wave
-    // (32 x 64) 0.97-1.06.  96 channels before 128: 142 against 140 TFLOP/s on 288 -> 384; 64 x 256 pixels, one wave over
-    // the channels, against 64 x 128, two: 142 against 90.
+    // takes 0.39-0.80 of the time of the per-wave forms above (108-146 TFLOP/s against 52-118); with eight blocks per wave
+    // (32 x 64) 1.04-1.08 at stride 1.  96 channels before 128: 141 against 139 TFLOP/s on 288 -> 384; 64 x 256 pixels, one
+    // wave over the channels, against 64 x 128, two: 136 against 88 on 64 -> 64 at 56 x 56.
     static constexpr int tile_bm() { return CO % 96 == 0 ? 96 : CO % 128 == 0 ? 128 : CO % 160 == 0 ? 160 : CO % 64 == 0 ? 64 : CO % 48 == 0 ? 48 : CO % 80 == 0 ? 80 : CO % 32 == 0 ? 32 : 16; }
     // At stride 1 half the channels and twice the pixels: the patch of 256 consecutive pixels of a row or image has few more
-    // rows than that of 128, the workgroup takes 32-38 KB of LDS instead of 42-48, and more of them share a CU (96 -> 96 on
-    // 35 x 35 139 against 138 TFLOP/s, 1.00-1.01x on six layers).  Not at stride 2, whose patch is four times the pixels
-    // (0.93-0.98x), nor on images so small that 256 pixels are several of them (8 x 8: 0.98x).
+    // rows than that of 128, the workgroup takes 32-38 KB of LDS instead of 42-48, and more of them share a CU (1.00-1.01x
+    // on six layers: 137 against 136 TFLOP/s for 256 -> 256 on 14 x 14, 137.4 against 137.2 for 96 -> 96 on 35 x 35).  Not at
+    // stride 2, whose patch is four times the pixels (0.95-1.00x), nor on images so small that 256 pixels are several of
+    // them (8 x 8: 0.99x).
     static constexpr bool HALF = S == 1 && tile_bm() >= 96 && OHW >= 128;
     static constexpr int TBM = HALF ? tile_bm() / 2 : tile_bm(), TWM = TBM >= 96 ? 2 : 1, TPB0 = TBM >= 96 ? 8 : TBM >= 48 ? 16 : 32;
     // A quarter more pixels per tile where that leaves less of the last round idle.  A CU multiplies two workgroups' tiles in
     // the time of two, so a round is 256 tiles: 512 -> 512 channels on 7 x 7 is 6.13 rounds (7) of 128 pixels but 4.9 (5) of
-    // 160: 142 against 127 TFLOP/s; 256 -> 256 on 14 x 14 145 against 140; 256 -> 512 on 14 x 14 at stride 2 132 against 121.  (With one sum
-    // over the reduction; sums in parts take 0-5 % off both sides: 138 on 14 x 14.)
+    // 160: 137 against 126 TFLOP/s; 256 -> 256 on 14 x 14 138 against 137; 256 -> 512 on 14 x 14 at stride 2 131 against 119.
     // A gain of two in a hundred by this count was 0.99-1.01x.  At most twenty blocks per wave: they take 160 registers.
     static constexpr double filled(int pb)
     {
@@ -402,7 +402,7 @@ struct ConvTiling {
         return false;
     }
     static constexpr int TPB = filled(TPB0 / 4 * 5) > 1.03 * filled(TPB0) && tiled(TPB0 / 4 * 5) ? TPB0 / 4 * 5 : TPB0;
-    // 1 x 1 filters likewise, as a matrix product (GemmTile): 1.02-1.28x of the streamed form at stride 1 (126-142 TFLOP/s on the
+    // 1 x 1 filters likewise, as a matrix product (GemmTile): 1.01-1.19x of the streamed form at stride 1 (119-145 TFLOP/s on the
     // layers of 768 and more channels, 4.0-5.1 TB/s on those of few), 1.4-1.9x at stride 2, where that one reads element
     // by element.  Three buffers of 16 channels for 128-pixel tiles (134 against 124 TFLOP/s with two of 32 on 768 -> 192),
     // two for 256-pixel ones, which are bound by memory and want more workgroups per CU.

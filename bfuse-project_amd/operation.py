@@ -77,7 +77,7 @@ _DT = {4: np.float32, 2: np.uint16, 1: np.uint8}
 
 # Results of at least this size are arrays over the library's pinned buffers, which the copy engines write in place
 # (57 GB/s; memory that is new with every array takes 10-20 GB/s, most of it page faults).  Smaller ones come from
-# malloc's heap, which is not new, through the staging ring (35-45 GB/s): 32 MiB is the largest piece malloc keeps there,
+# malloc's heap, which is not new, through the staging ring (44 GB/s for 5 MB, 53-56 for 128): 32 MiB is the largest piece malloc keeps there,
 # and a program whose results are elsewhere sees it hand the memory of its own arrays back to the system more often.
 PINNED_MIN_BYTES = 32 << 20
 
