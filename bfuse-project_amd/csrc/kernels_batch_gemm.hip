@@ -27,7 +27,7 @@ DENSE_F32(1024, 14336, 4096, 64, 128, 4)
 
 // C[b] = A[b] . B[b]^T, A [b, M, K], B [b, N, K]: <M, N, K, BM, BN, waves over K>
 // Products whose rows and columns are whole tiles run on shared tiles (GemmTile): 128 x 128 in three buffers of 16 k
-// (1024 products 512 x 64 x 512: 0.46-0.50 -> 0.38-0.42 ms from box to box, 256 x 80 x 256: 0.142 -> 0.122), 256 x 64 with the waves over the rows
+// (1024 products 512 x 64 x 512: 0.46-0.50 -> 0.38-0.42 ms from card to card, 256 x 80 x 256: 0.142 -> 0.122), 256 x 64 with the waves over the rows
 // where there are 64 columns (512 x 512 x 64: 0.41 -> 0.33 ms).
 #define BGEMM_F32_TILE(B, M, K, N, BM, BN, WM, KS, NBUF)                                                         \
     using Bgemm_##B##x##M##x##K##x##N = GemmTile<M, K, 1, N, 1, B, BM, BN, WM, KS, kRows, NBUF>;                  \
