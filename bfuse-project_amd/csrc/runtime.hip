@@ -434,11 +434,11 @@ int sync_and_check()
         if (e != hipSuccess && rc == BFUSE_OK) rc = fail(BFUSE_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
         return e == hipSuccess;
     };
-    const unsigned long uploads = HostCopy::get().wait_begins(), launches = g_in_flight.wait_begins();
-    if (note_hip(hipDeviceSynchronize(), "hipDeviceSynchronize")) {
-        g_in_flight.wait_ended(launches);
-        HostCopy::get().wait_ended(uploads);
-    }
+    HostCopy::get().wait_begins();
+    g_in_flight.wait_begins();
+    const bool waited = note_hip(hipDeviceSynchronize(), "hipDeviceSynchronize");
+    g_in_flight.wait_ended(waited);
+    HostCopy::get().wait_ended(waited);
     note_hip(hipGetLastError(), "launch");
     // every counter that may hold something is read (and thereby reset) even after an error above; the first error is the
     // one returned
