@@ -2,11 +2,13 @@
 // 1024 rows (dense: batch, in, out) and at 1024 independent products (bgemm: batch, M, K, N), fp32, with the
 // tilings of their 512-row / 16-product counterparts (model_ops.h) -- twice, or 64 times, the workgroups -- or with twice
 // the columns per tile, which is again a workgroup per CU and a better ratio of MFMAs to operand reads: 1024 x 3072 x 768
-// 44.4 -> 34.8 us (32 x 96 against 32 x 48), x 768 x 768 11.5 -> 10.8, 4096 x 1024 62.5 -> 60.2 (32 x 128 against 32 x 64),
-// 768 x 3072 37.4 -> 36.7 (32 x 128 against 32 x 96: three workgroups per CU).  64 x 144 for 768 x 2304: no gain.
+// 44.4 -> 34.8 us (32 x 96 against 32 x 48), x 768 x 768 11.5 -> 10.8, 4096 x 1024 62.5 -> 60.2 (32 x 128 against 32 x 64).
+// 64 x 144 for 768 x 2304: no gain.  The larger ones run on the bf16 matrix cores (ops_gemm_split.h has the figures): there the
+// tile is 128 x 128, 128 x 96 or 256 x 128, the largest that still gives every CU one, and those too small for 192 such tiles stay.
 #include "fuse.h"
 #include "ops_gemm_f32.h"
 #include "ops_gemm_f32_dma.h"
+#include "ops_gemm_split.h"
 #include "ops_gemm_tile.h"
 
 using namespace bfuse;
@@ -16,14 +18,18 @@ BFUSE_MODULE_PROLOGUE()
 #define DENSE_F32(M, K, N, ...)                                                                                  \
     using Dense_##M##x##K##x##N = GemmF32Dma<M, N, K, __VA_ARGS__>;                                               \
     BFUSE_KERNEL(gemm_f32_##M##x##K##x##N, Dense_##M##x##K##x##N, ({{M, K, 1, 1}, 4}), ({{K, N, 1, 1}, 4}), ({{M, N, 1, 1}, 4}))
+// <.., 16-row blocks of a wave, waves over the rows, over the columns, over K, columns>
+#define DENSE_SPLIT(M, K, N, ...)                                                                                \
+    using Dense_##M##x##K##x##N = GemmSplit<M, K, 1, N, 1, 1, __VA_ARGS__, kPix>;                                 \
+    BFUSE_KERNEL(gemm_f32_##M##x##K##x##N, Dense_##M##x##K##x##N, ({{M, K, 1, 1}, 4}), ({{K, N, 1, 1}, 4}), ({{M, N, 1, 1}, 4}))
 DENSE_F32(1024, 768, 768, 32, 96, 4)
-DENSE_F32(1024, 768, 3072, 32, 128, 4, kEpiNone, 2)
+DENSE_SPLIT(1024, 768, 3072, 2, 4, 1, 2, 96)
 DENSE_F32(1024, 3072, 768, 32, 96, 4)
 DENSE_F32(1024, 768, 2304, 32, 144, 4)
-DENSE_F32(1024, 4096, 4096, 64, 128, 4)
+DENSE_SPLIT(1024, 4096, 4096, 2, 4, 1, 2, 128)
 DENSE_F32(1024, 4096, 1024, 32, 128, 4)
-DENSE_F32(1024, 4096, 14336, 64, 128, 4)
-DENSE_F32(1024, 14336, 4096, 64, 128, 4)
+DENSE_SPLIT(1024, 4096, 14336, 2, 8, 1, 1, 128)
+DENSE_SPLIT(1024, 14336, 4096, 2, 4, 1, 2, 128)
 
 // C[b] = A[b] . B[b]^T, A [b, M, K], B [b, N, K]: <M, N, K, BM, BN, waves over K>
 // Products whose rows and columns are whole tiles run on shared tiles (GemmTile): 128 x 128 in three buffers of 16 k

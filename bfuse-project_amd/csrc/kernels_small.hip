@@ -11,6 +11,7 @@
 #include "ops_gemm_bf16.h"
 #include "ops_gemm_f32.h"
 #include "ops_gemm_f32_dma.h"
+#include "ops_gemm_split.h"
 #include "ops_gemm_tile.h"
 #include "ops_layout.h"
 #include "ops_pool.h"
@@ -215,3 +216,27 @@ BGEMM_TILE_TEST(f, 8, 64, 32, 64, 64, 64, 4, 32, 2)              // one stage, p
 BGEMM_TILE_TEST(g, 2, 64, 512, 64, 64, 64, 4, 32, 3)             // two sums of 256 k
 BFUSE_HFUSE_KERNEL(selftest_gemm_tile_c, GemmT_c, bias_relu_4096, BiasReluS)
 BFUSE_BFUSE_KERNEL(selftest_gemm_tile_e, GemmT_e, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
+
+// The product on the bf16 matrix cores: row tiles that overlap and columns past the end, odd and even numbers of stages, threads
+// that do a unit twice, a last stage of 8, 16 and 24 k, waves over the columns, groups of waves over K, images and strides.
+// <M, K, H, W, S, images or products, 16-row blocks of a wave, waves over rows, over columns, over K, columns, layout>
+#define DENSE_SPLIT_TEST(TAG, M, K, N, ...)                                                                        \
+    using GemmSp_##TAG = GemmSplit<M, K, 1, N, 1, 1, __VA_ARGS__, kPix>;                                             \
+    BFUSE_KERNEL(selftest_gemm_split_##TAG, GemmSp_##TAG, ({{M, K, 1, 1}, 4}), ({{K, N, 1, 1}, 4}), ({{M, N, 1, 1}, 4}))
+#define BGEMM_SPLIT_TEST(TAG, B, M, K, N, ...)                                                                     \
+    using GemmSp_##TAG = GemmSplit<M, K, 1, N, 1, B, __VA_ARGS__, kRows>;                                            \
+    BFUSE_KERNEL(selftest_gemm_split_##TAG, GemmSp_##TAG, ({{B, M, K, 1}, 4}), ({{B, N, K, 1}, 4}), ({{B, M, N, 1}, 4}))
+#define CONV1_SPLIT_TEST(TAG, CI, CO, H, W, S, N, ...)                                                             \
+    using GemmSp_##TAG = SwapOperands<GemmSplit<CO, CI, H, W, S, N, __VA_ARGS__, kPix>>;                             \
+    BFUSE_KERNEL(selftest_gemm_split_##TAG, GemmSp_##TAG, ({{N, CI, H, W}, 4}), ({{CO, CI, 1, 1}, 4}), ({{N, CO, (H - 1) / S + 1, (W - 1) / S + 1}, 4}))
+DENSE_SPLIT_TEST(a, 160, 96, 144, 2, 4, 1, 1, 64)
+DENSE_SPLIT_TEST(b, 128, 256, 96, 2, 4, 1, 2, 96)
+DENSE_SPLIT_TEST(c, 256, 64, 224, 2, 8, 1, 1, 112)
+DENSE_SPLIT_TEST(d, 64, 4096, 64, 2, 2, 1, 1, 64)
+BGEMM_SPLIT_TEST(e, 8, 64, 72, 80, 1, 2, 2, 1, 64)
+BGEMM_SPLIT_TEST(f, 3, 208, 208, 112, 1, 7, 1, 1, 112)
+CONV1_SPLIT_TEST(g, 48, 80, 9, 9, 1, 5, 1, 4, 2, 1, 128)
+CONV1_SPLIT_TEST(h, 56, 64, 9, 7, 2, 11, 2, 2, 1, 2, 96)
+BFUSE_BFUSE_KERNEL(selftest_gemm_split_a, GemmSp_a, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
+BFUSE_HFUSE_KERNEL(selftest_gemm_split_e, GemmSp_e, bias_relu_4096, BiasReluS)
+BFUSE_HFUSE_KERNEL(selftest_gemm_split_f, GemmSp_f, conv3x3_f32_32x12x12_32, ConvS2)

@@ -1,0 +1,357 @@
+// fp32 matrix product on the bf16 matrix cores: every operand as the sum of three bf16 (split.h), six MFMAs of 16 times the
+// fp32 rate for each of the fp32 ones they replace.
+//
+//   C[m][n] = sum_k A[m][k] * B(k, n)
+//
+// The fp32 forms (GemmF32Dma, GemmTile) run at 143 - 150 TFLOP/s on large products, the rate of the fp32 matrix instructions.
+// Six bf16 products at the 1.65 - 1.75 PFLOP/s that random operands leave the chip are 280 of these.  What stands in between is
+// taking the operands apart: 5.5 vector instructions an element, of which two go between two MFMAs of a wave almost for free
+// (17 -> 19 clocks) and more do not.  So the tile is as large as it can be (an element of A is used BN times, one of B BM times)
+// and every element is taken apart once in the workgroup:
+//   * a wave owns 16 TM rows of A alone and takes them apart in its registers: lane (i, q) loads A[i][8q .. 8q + 7], which is
+//     the MFMA's operand;
+//   * B is shared: a thread takes eight k of a column apart and writes them to LDS, [part][8-k octet][column][16 bytes], where
+//     the fragment reads of a wave are 256 consecutive bytes for each of its four octets: no bank is met twice;
+//   * three LDS buffers and one barrier per stage of 32 k.  While stage s is multiplied, the stage two ahead is taken apart and
+//     written and the A of the next one taken apart, dealt between the MFMAs; the loads are a stage ahead of that;
+//   * products with few tiles give two groups of waves the even and the odd stages (KG = 2): two waves per SIMD hide each
+//     other's waits, and the groups' sums meet in LDS at the end.
+// The operands of an MFMA are given in the order (B, A), so that a lane ends up with four consecutive columns of a row.
+//
+// The five small products are summed apart from the large one (`low`): what rounds the sum is then one addition per 32 k, and
+// 2-norm errors against 64 bits are below those of the fp32 forms: K = 4096 2.7e-7 (KG = 2) and 4.0e-7 (KG = 1) where GemmF32Dma
+// has 5.8e-7, 14336 5.3e-7 for 1.07e-6, 768 1.1e-7 for 2.5e-7.  What three bf16 cannot hold is multiplied again with the fp32 MFMAs
+// (see split.h): a wave whose results are not all finite, and the workgroup if a thread has met nothing but values below 2^-95.
+//
+// Measured (us, before = GemmF32Dma): 1024 x 4096 x 14336 805 -> 499 (241 TFLOP/s), 1024 x 14336 x 4096 798 -> 530, 1024 x 4096 x
+// 4096 232 -> 156, 512 x 4096 x 14336 461 -> 254, 512 x 4096 x 4096 119 -> 93, 1024 x 768 x 3072 37-41 -> 34.  Smaller tiles than
+// 64 x 64 a workgroup take more time than the fp32 forms: 1024 x 3072 x 768 63 (64 x 96 tiles) against 39.
+//
+// B comes in one of two layouts, as in GemmTile: kPix, planes of n for each k ([K, N] is one image of N pixels); kRows, rows
+// contiguous along k, NIMG independent products.  A row tile (kRows: also a column tile) that does not divide the problem starts
+// a tile before its end and writes the same bits as its neighbour.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <type_traits>
+
+#include "dispatch.h"
+#include "ops_gemm_tile.h"
+#include "split.h"
+#include "wave.h"
+
+namespace bfuse {
+
+// M, K, H, W, S, NIMG, LAYOUT: as in GemmTile.  TM 16-row blocks of a wave, WR waves over the rows and WN over the BN columns, KG
+// groups of such waves over the stages.
+template <int M_, int K_, int H_, int W_, int S_, int NIMG_, int TM_, int WR_, int WN_, int KG_, int BN_, int LAYOUT_>
+struct GemmSplit {
+    static constexpr bool MATRIX_CORES = true;   // the inner loop is a stream of MFMAs (what the fusion chooser asks)
+    static constexpr int M = M_, K = K_, H = H_, W = W_, S = S_, NIMG = NIMG_, TM = TM_, WR = WR_, WN = WN_, KG = KG_, BN = BN_, LAYOUT = LAYOUT_;
+    static constexpr int NWAVE = WR * WN * KG, THREADS = 64 * NWAVE, GT = 64 * WR * WN, BM = 16 * TM * WR, TN = BN / WN / 16;
+    static constexpr int NS = (K + 31) / 32, NIT = NS / KG, TAIL = K % 32;       // stages, those of a group, k of the last one if not 32
+    static constexpr int OH = (H - 1) / S + 1, OW = (W - 1) / S + 1, HW = H * W, OHW = OH * OW;
+    static constexpr int OHWP = (OHW + 3) / 4 * 4;                               // columns of an image, whole chunks of four
+    static constexpr int MT = (M + BM - 1) / BM;
+    static constexpr int NT = LAYOUT == kRows ? (W + BN - 1) / BN : (int)(((long long)OHWP * NIMG + BN - 1) / BN);
+    static constexpr int NIMAGES = LAYOUT == kRows ? 1 : (BN + OHWP - 2) / OHWP + 1;   // images a tile can touch
+    static constexpr int NUJ = (4 * BN + GT - 1) / GT;                           // units (a column's eight k) of a thread and stage
+    static_assert(BN % (16 * WN) == 0 && K % 8 == 0 && NS % KG == 0 && M >= BM && (LAYOUT == kPix || (W >= BN && H == 1 && S == 1)), "tile");
+    // 31-bit offsets; padding is read through one that lies past the buffer
+    static constexpr bool FITS = (long long)BM * K * 4 < (1LL << 31) && (long long)(NIMAGES < NIMG ? NIMAGES : NIMG) * K * HW * 4 < (1LL << 31);
+    static constexpr int PLANE = 4 * BN * 16, BUF = 3 * PLANE, NBUF = 3;
+    static constexpr int TILES = MT * NT;
+    static constexpr Dims3 GRID{LAYOUT == kRows ? TILES * NIMG : TILES, 1, 1};
+    static constexpr Dims3 BLOCK{THREADS, 1, 1};
+    static constexpr bool HAS_BARRIERS = true;
+    static constexpr bool LOOP_BARRIERS = true;
+    static constexpr int MIN_BARRIERS = NIT;
+    static constexpr int RED_BYTES = (KG - 1) * BM * BN * 4;                     // partial sums of the groups
+
+    struct Smem {
+        __attribute__((aligned(16))) unsigned char t[NBUF * KG * BUF > RED_BYTES ? NBUF * KG * BUF : RED_BYTES];
+        unsigned inexact;
+    };
+
+    // (column tile, row tile), dealt so that the row tiles of one column tile follow each other on one XCD
+    __device__ static __forceinline__ void tile_of(int vblock, int& nt, int& mt)
+    {
+        constexpr int PER_XCD = NT / 8;
+        constexpr int FULL = 8 * PER_XCD * MT;
+        if (vblock < FULL) {
+            const int xcd = vblock & 7, slot = vblock >> 3;
+            nt = xcd * PER_XCD + slot / MT;
+            mt = slot % MT;
+        } else {
+            const int rem = vblock - FULL;
+            nt = 8 * PER_XCD + rem / MT;
+            mt = rem % MT;
+        }
+    }
+
+    template <class Sync>
+    __device__ static __forceinline__ void run(int vblock, int tid, Smem& sm, const void* I, const void* F, void* O, Sync sync)
+    {
+        static_assert(FITS, "tile too large");
+        const float* A = static_cast<const float*>(I);
+        const float* B = static_cast<const float*>(F);
+        float* __restrict__ C = static_cast<float*>(O);
+        const int lane = tid & 63, li = lane & 15, kq = lane >> 4;
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const int g = wave / (WR * WN), w = wave % (WR * WN), wr = w / WN, wn = w % WN, gt = tid - g * GT;
+
+        int mt, nt;
+        if constexpr (LAYOUT == kRows) {
+            // whole products are dealt to the XCDs, so that the tiles of one share an L2
+            int batch = vblock / TILES, v = vblock % TILES;
+            if constexpr (NIMG % 8 == 0) {
+                const int xcd = vblock & 7, slot = vblock >> 3;
+                batch = (slot / TILES) * 8 + xcd;
+                v = slot % TILES;
+            }
+            mt = v / NT;
+            nt = v % NT;
+            A += (size_t)batch * M * K;
+            B += (size_t)batch * W * K;
+            C += (size_t)batch * M * W;
+        } else {
+            tile_of(vblock, nt, mt);
+        }
+        const int m0 = M % BM != 0 && mt == MT - 1 ? M - BM : mt * BM;
+        const long long n0 = LAYOUT == kRows && W % BN != 0 && nt == NT - 1 ? W - BN : (long long)nt * BN;
+        const int n_lo = LAYOUT == kRows ? 0 : (int)(n0 / OHWP);                 // kPix: first image of the tile
+        const int v0 = (int)(n0 - (long long)n_lo * OHWP);
+
+        // offset of B(0, column c of the tile); past the buffer if there is none
+        auto column = [&](int c) -> unsigned {
+            if constexpr (LAYOUT == kRows) return (unsigned)(c * K * 4);
+            const int v = v0 + c, img = v / OHWP, p = v % OHWP;
+            return p < OHW && n_lo + img < NIMG ? (unsigned)((img * K * HW + (p / OW) * S * W + (p % OW) * S) * 4) : 0x7fffffffu;
+        };
+        constexpr unsigned B_K = LAYOUT == kRows ? 4 : HW * 4;                   // bytes from one k of a column to the next
+        const auto ar = __builtin_amdgcn_make_buffer_rsrc((void*)(A + (size_t)m0 * K), 0, BM * K * 4, 0x00020000);
+        const auto br = __builtin_amdgcn_make_buffer_rsrc((void*)(LAYOUT == kRows ? B + (size_t)n0 * K : B + (size_t)n_lo * K * HW), 0,
+                                                          LAYOUT == kRows ? BN * K * 4 : (NIMG - n_lo < NIMAGES ? NIMG - n_lo : NIMAGES) * K * HW * 4, 0x00020000);
+        const unsigned a_voff = (unsigned)(((wr * TM * 16 + li) * K + 8 * kq) * 4);
+        unsigned b_voff[NUJ];
+        int b_lds[NUJ];
+#pragma unroll
+        for (int j = 0; j < NUJ; ++j) {
+            // threads past the last unit do one of the first ones again: the same values to the same place.  kRows: four lanes
+            // read 128 consecutive bytes of a row; kPix: 64 lanes 64 consecutive columns of a plane
+            const int u = (j * GT + gt) % (4 * BN), o = LAYOUT == kRows ? u & 3 : u / BN, c = LAYOUT == kRows ? u >> 2 : u % BN;
+            const unsigned v = column(c);
+            b_voff[j] = v == 0x7fffffffu ? v : v + 8 * o * B_K;
+            b_lds[j] = (o * BN + c) * 16;
+        }
+
+        f32x4 acc[TM][TN], low[TM][TN];
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+            for (int b = 0; b < TN; ++b) acc[tm][b] = low[tm][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+        f32x4 ra[TM][2];
+        float rb[NUJ][8];
+        auto load_a = [&](int tm, int s) {
+            const unsigned v = TAIL != 0 && s == NS - 1 && 8 * kq >= TAIL ? 0x7fffffffu : a_voff + tm * 16 * K * 4;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) ra[tm][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ar, v + h * 16, s * 128, 0));
+        };
+        auto load_b = [&](int j, int s) {
+            const unsigned v = TAIL != 0 && s == NS - 1 && b_lds[j] >= TAIL / 8 * BN * 16 ? 0x7fffffffu : b_voff[j];
+            if constexpr (LAYOUT == kRows) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const f32x4 f = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(br, v + h * 16, s * 128, 0));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) rb[j][4 * h + e] = f[e];
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) rb[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(br, v, (s * 32 + e) * B_K, 0));
+            }
+        };
+        shared_with_asm(sm.t);
+        unsigned char* const base = sm.t + g * NBUF * BUF;
+        const unsigned char* const fb = base + (kq * BN + wn * TN * 16 + li) * 16;
+        unsigned pa[2][TM][3][4], pb[3][4];
+        unsigned seen[NUJ + TM] = {};               // bits of the leading parts of each unit
+        if (tid == 0) sm.inexact = 0;
+        // Two of a unit's eight values: units 0 .. NUJ - 1 are this thread's of B, the others its rows of A.
+        auto convert = [&](int part, int to, int off) {
+            const int u = part / 4, j = part % 4;
+            if (u < NUJ) {
+                split2(rb[u][2 * j], rb[u][2 * j + 1], pb[0][j], pb[1][j], pb[2][j]);
+                if (j % 2 == 1) seen[u] |= pb[0][j - 1] | pb[0][j];
+                if (j == 3) {
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x4*>(base + off + q * PLANE + b_lds[u]) = u32x4{pb[q][0], pb[q][1], pb[q][2], pb[q][3]};
+                }
+            } else {
+                const int tm = u - NUJ;
+                unsigned(&p)[3][4] = pa[to][tm];
+                split2(ra[tm][j / 2][2 * (j % 2)], ra[tm][j / 2][2 * (j % 2) + 1], p[0][j], p[1][j], p[2][j]);
+                if (j % 2 == 1) seen[u] |= p[0][j - 1] | p[0][j];
+            }
+        };
+        constexpr int NPART = 4 * (NUJ + TM), VPM = (11 * NPART + 6 * TM * TN - 1) / (6 * TM * TN);
+        const auto stage_of = [&](int it) { return (it < NIT ? it : NIT - 1) * KG + g; };   // past the end: the last one again
+
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+#pragma unroll
+            for (int j = 0; j < NUJ; ++j) load_b(j, stage_of(i));
+            if (i == 0) {
+#pragma unroll
+                for (int tm = 0; tm < TM; ++tm) load_a(tm, g);
+            }
+#pragma unroll
+            for (int part = 0; part < 4 * NUJ; ++part) convert(part, 0, i * BUF);
+        }
+#pragma unroll
+        for (int j = 0; j < NUJ; ++j) load_b(j, stage_of(2));
+#pragma unroll
+        for (int part = 4 * NUJ; part < NPART; ++part) convert(part, 0, 0);
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm) load_a(tm, stage_of(1));
+        u32x4 fr[2][3];
+        auto read = [&](int set, int q, int b, int off) { fr[set][q] = *reinterpret_cast<const u32x4*>(fb + off + q * PLANE + b * 256); };
+        sync.raw();
+#pragma unroll
+        for (int q = 2; q >= 0; --q) read(0, q, 0, 0);
+        int off = 0, next = BUF, ahead = 2 * BUF;   // LDS offsets of this stage and the two after it
+        auto stage = [&](int it, auto from) {
+            constexpr int FROM = decltype(from)::value;
+            // Behind the barrier the next stage is in LDS whole, and nobody reads the one before this any more.
+            if (it > 0) sync.raw();
+#pragma unroll
+            for (int b = 0; b < TN; ++b) {
+                const int set = (b + FROM * (TN & 1)) & 1;
+#pragma unroll
+                for (int t = 0; t < SplitTerms::N; ++t) {
+#pragma unroll
+                    for (int tm = 0; tm < TM; ++tm) {
+                        f32x4& c = t + 1 < SplitTerms::N ? low[tm][b] : acc[tm][b];
+                        const unsigned(&p)[4] = pa[FROM][tm][SplitTerms::A[t]];
+                        c = mfma_bf16(fr[set][SplitTerms::B[t]], u32x4{p[0], p[1], p[2], p[3]}, c);
+                    }
+                    if (t == 0 || t == 2 || t == 4) read(set ^ 1, 2 - t / 2, b + 1 < TN ? b + 1 : 0, b + 1 < TN ? off : next);
+                }
+#pragma unroll
+                for (int part = 0; part < NPART; ++part)
+                    if (part * TN / NPART == b) {
+                        convert(part, FROM ^ 1, ahead);
+                        if (part % 4 == 3) {
+                            if (part / 4 < NUJ) load_b(part / 4, stage_of(it + 3));
+                            else load_a(part / 4 - NUJ, stage_of(it + 2));
+                        }
+                    }
+#pragma unroll
+                for (int t = 0; t < SplitTerms::N; ++t) {
+#pragma unroll
+                    for (int tm = 0; tm < TM; ++tm) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);     // an MFMA
+                        __builtin_amdgcn_sched_group_barrier(0x002, VPM, 0);   // vector instructions
+                    }
+                    if (t == 0 || t == 2 || t == 4) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // an LDS read
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            const int o = off;
+            off = next;
+            next = ahead;
+            ahead = o;
+        };
+#pragma unroll 1
+        for (int it = 0; it + 1 < NIT; it += 2) {
+            stage(it, std::integral_constant<int, 0>{});
+            stage(it + 1, std::integral_constant<int, 1>{});
+        }
+        if constexpr (NIT % 2 == 1) stage(NIT - 1, std::integral_constant<int, 0>{});
+
+        bool tiny = false;
+#pragma unroll
+        for (int u = 0; u < NUJ + TM; ++u) tiny |= split_tiny(seen[u]);
+        if (tiny) sm.inexact = 1;
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+            for (int b = 0; b < TN; ++b) acc[tm][b] += low[tm][b];
+        sync.raw();
+        bool again = sm.inexact != 0;
+        if constexpr (KG > 1) {
+            f32x4* const red = reinterpret_cast<f32x4*>(sm.t) + w * TM * TN * 64 + lane;
+            if (g > 0) {
+#pragma unroll
+                for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+                    for (int b = 0; b < TN; ++b) red[((g - 1) * WR * WN * TM * TN + tm * TN + b) * 64] = acc[tm][b];
+            }
+            sync.raw();
+            if (g > 0) return;
+#pragma unroll
+            for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+                for (int b = 0; b < TN; ++b)
+#pragma unroll
+                    for (int q = 1; q < KG; ++q) acc[tm][b] += red[((q - 1) * WR * WN * TM * TN + tm * TN + b) * 64];
+        }
+        float zero = 0.f;                           // or NaN
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+            for (int b = 0; b < TN; ++b)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) zero = __builtin_fmaf(acc[tm][b][v], 0.f, zero);
+        again |= __builtin_amdgcn_ballot_w64(zero != 0.f) != 0;
+        if (again) {
+#pragma unroll
+            for (int b = 0; b < TN; ++b) {
+                const unsigned c = column((wn * TN + b) * 16 + li), v = c == 0x7fffffffu ? c : c + kq * B_K;
+#pragma unroll
+                for (int tm = 0; tm < TM; ++tm) acc[tm][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+                for (int k = 0; k < K; k += 4) {
+                    const float bv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(br, v, k * B_K, 0));
+#pragma unroll
+                    for (int tm = 0; tm < TM; ++tm) {
+                        const float av = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ar, (((wr * TM + tm) * 16 + li) * K + kq) * 4, k * 4, 0));
+                        acc[tm][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv, av, acc[tm][b], 0, 0, 0);
+                    }
+                }
+            }
+        }
+        // lane (i, q): row i of a 16-row block, columns 4q .. 4q + 3 of each 16-column block
+#pragma unroll
+        for (int b = 0; b < TN; ++b) {
+            const int col = (wn * TN + b) * 16 + 4 * kq;
+            if constexpr (LAYOUT == kRows) {
+#pragma unroll
+                for (int tm = 0; tm < TM; ++tm) *reinterpret_cast<f32x4*>(C + (size_t)(m0 + (wr * TM + tm) * 16 + li) * W + n0 + col) = acc[tm][b];
+            } else {
+                const int vc = v0 + col, img = n_lo + vc / OHWP, p = vc % OHWP;
+                if (img < NIMG) {
+                    float* __restrict__ y = C + ((size_t)img * M + m0 + wr * TM * 16 + li) * OHW + p;
+                    const bool whole = OHW % 4 == 0 || p + 4 <= OHW;
+#pragma unroll
+                    for (int tm = 0; tm < TM; ++tm) {
+                        float* const d = y + (size_t)(tm * 16) * OHW;
+                        const f32x4 o = acc[tm][b];
+                        if constexpr (OHW % 4 == 0) {
+                            *reinterpret_cast<f32x4*>(d) = o;
+                        } else if (whole) {
+                            *reinterpret_cast<f32x4u*>(d) = f32x4u{o[0], o[1], o[2], o[3]};
+                        } else {
+#pragma unroll
+                            for (int e = 0; e < 3; ++e)
+                                if (p + e < OHW) d[e] = o[e];
+                        }
+                    }
+                }
+            }
+        }
+    }
+};
+
+}  // namespace bfuse

@@ -1,0 +1,101 @@
+"""fp32 products on the bf16 matrix cores (csrc/split.h, ops_gemm_split.h): the edges of tiles and stages against the oracle
+(products: numpy in double), alone and fused; their error against 64 bits; and operands that three bf16 cannot hold."""
+import numpy as np
+import pytest
+
+import bfuse_project_amd as bf
+from bfuse_project_amd.operation import fill_normal
+from oracle import oracle as orf
+from tests.test_gpu_conv_tile import _check
+
+pytestmark = pytest.mark.gpu
+
+
+def _product(a, b):
+    """[M, K] . [K, N], or [b, M, K] . [b, N, K]^T"""
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    return a[..., 0, 0] @ b[..., 0, 0] if a.shape[2] == 1 else np.matmul(a[..., 0], b[..., 0].transpose(0, 2, 1))
+
+
+@pytest.mark.parametrize("tag,partner,kind,suffix", [
+    ("a", "layernorm_8x256", "bfuse", "_c4"), ("b", "bias_relu_4096", None, ""), ("c", "bias_relu_4096", None, ""), ("d", "bias_relu_4096", None, ""),
+    ("e", "bias_relu_4096", "hfuse", ""), ("f", "conv3x3_f32_32x12x12_32", "hfuse", "")])
+def test_split_product_against_numpy_and_fused(tag, partner, kind, suffix):
+    _check(f"selftest_gemm_split_{tag}", lambda a, b: _product(a, b).astype(np.float32), partner, kind, suffix)
+
+
+@pytest.mark.parametrize("tag,s", [("g", 1), ("h", 2)])
+def test_split_1x1_convolution_against_the_oracle(tag, s):
+    _check(f"selftest_gemm_split_{tag}", lambda x, w: orf.conv2d(x, w, s=s, p=0), "bias_relu_4096", None, "")
+
+
+def _run(name, x, w):
+    with bf.Operation(name, "bias_relu_4096") as op:
+        op.upload(0, x, w)
+        op.zero_outputs()
+        op.launch("kernel1")
+        return op.download(0).reshape(op.k[0].shapes[2])
+
+
+def _operands(name):
+    with bf.Operation(name, "bias_relu_4096") as op:
+        k = op.k[0]
+    return [fill_normal(11 + i, int(np.prod(k.shapes[i])), 0, 1).reshape(k.shapes[i]) for i in (0, 1)]
+
+
+@pytest.mark.parametrize("tag,steps,groups", [("d", 4096 // 32, 1), ("b", 256 // 32, 2)])
+def test_split_product_is_closer_to_64_bits_than_one_fp32_sum(tag, steps, groups):
+    """One rounding of at most u = 2^-24 of what the sum has grown to for every 32 k: u sqrt(steps / 2) (2-norm), in two groups
+    sqrt(2) less and u for adding them; the products that are left out and the sum of the small ones add less than u / 2."""
+    name = f"selftest_gemm_split_{tag}"
+    x, w = _operands(name)
+    want = _product(x, w)
+    err = np.linalg.norm(_run(name, x, w).reshape(want.shape) - want) / np.linalg.norm(want)
+    assert err <= 2.0 ** -24 * ((steps / 2 / groups) ** 0.5 + 0.5 + (groups > 1))
+
+
+@pytest.mark.parametrize("tag", ["a", "b", "e"])
+@pytest.mark.parametrize("scale", [2.0 ** -100, 2.0 ** -118, 2.0 ** 100])
+def test_scaled_operands_keep_their_bits(tag, scale):
+    """A power of two on an operand is one on the result, however small the operand's own low bits become (whole operand, one
+    row or column among others, a column of zeros beside it)."""
+    name = f"selftest_gemm_split_{tag}"
+    x, w = _operands(name)
+    scale = np.float32(scale)
+    u = 2.0 ** -24 * x.shape[1] ** 0.5 * 2     # twice the bound of one sum rounded after every product
+    want = _product(x, w)
+    for a, b, f in ((x * scale, w, scale), (x, w * scale, scale)):
+        y = _run(name, a, b).reshape(want.shape).astype(np.float64) / float(f)
+        assert np.linalg.norm(y - want) <= u * np.linalg.norm(want)
+    a, rows = x.copy().reshape(-1, x.shape[-3] if x.shape[2] == 1 else x.shape[-2]), slice(3, None, 16)
+    a[rows] *= scale
+    a[5] = 0
+    a = a.reshape(x.shape)
+    want = _product(a, w)
+    y = _run(name, a, w).reshape(want.shape).astype(np.float64)
+    want, y = want.reshape(-1, want.shape[-1]), y.reshape(-1, want.shape[-1])
+    for r in range(want.shape[0]):
+        assert np.linalg.norm(y[r] - want[r]) <= u * np.linalg.norm(want[r]), r
+
+
+@pytest.mark.parametrize("tag", ["a", "b", "e"])
+def test_infinities_nan_and_the_largest_values(tag):
+    """What does not fit three bf16 gives what fp32 arithmetic gives: infinite where it is, NaN where it is, finite elsewhere."""
+    name = f"selftest_gemm_split_{tag}"
+    x, w = _operands(name)
+    x2 = x.reshape(-1, x.shape[1] if x.shape[2] == 1 else x.shape[2])      # rows
+    big = np.float32(3.4e38)
+    w = np.abs(w) + np.float32(0.5)
+    x2[2, 1], x2[4, 0], x2[4, 1], x2[7, 3] = np.inf, np.inf, -np.inf, np.nan
+    x2[9] = 0
+    x2[9, 2], x2[11, 4] = np.finfo(np.float32).min, big
+    if tag != "e":
+        w2 = w.reshape(w.shape[0], w.shape[1])
+        w2[2] = np.float32(0.5)                                            # 0.5 * the lowest value stays finite
+        w2[1, 5], w2[0, 6] = np.inf, np.nan
+    with np.errstate(all="ignore"):
+        want = _product(x, w).astype(np.float32).reshape(-1, _product(x, w).shape[-1])
+    y = _run(name, x, w).reshape(want.shape)
+    assert np.array_equal(np.isnan(y), np.isnan(want)) and np.array_equal(np.isposinf(y), np.isposinf(want)) and np.array_equal(np.isneginf(y), np.isneginf(want))
+    ok = np.isfinite(want)
+    assert ok.any() and np.all(np.abs(y[ok] - want[ok]) <= 1e-5 * np.maximum(np.abs(want[ok]), np.sqrt(np.float32(x2.shape[1]))))
