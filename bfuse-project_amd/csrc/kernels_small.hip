@@ -229,6 +229,15 @@ BFUSE_BFUSE_KERNEL(selftest_gemm_tile_e, GemmT_e, layernorm_8x256, LayerNormS, _
 #define CONV1_SPLIT_TEST(TAG, CI, CO, H, W, S, N, ...)                                                             \
     using GemmSp_##TAG = SwapOperands<GemmSplit<CO, CI, H, W, S, N, __VA_ARGS__, kPix>>;                             \
     BFUSE_KERNEL(selftest_gemm_split_##TAG, GemmSp_##TAG, ({{N, CI, H, W}, 4}), ({{CO, CI, 1, 1}, 4}), ({{N, CO, (H - 1) / S + 1, (W - 1) / S + 1}, 4}))
+// ... and convolutions: padding, strides, images of odd pixels, a last stage that runs past the window, 30 taps, even filters.
+#define CONV_SPLIT_TEST(TAG, CI, CO, H, W, KH, KW, S, P, N, ...)                                                    \
+    using GemmSp_##TAG = SwapOperands<GemmSplit<CO, CI * KH * KW, H, W, S, N, __VA_ARGS__, kPix, KH, KW, P>>;          \
+    BFUSE_KERNEL(selftest_gemm_split_##TAG, GemmSp_##TAG, ({{N, CI, H, W}, 4}), ({{CO, CI, KH, KW}, 4}),             \
+                 ({{N, CO, (H - KH + 2 * P) / S + 1, (W - KW + 2 * P) / S + 1}, 4}))
+CONV_SPLIT_TEST(i, 16, 64, 9, 7, 3, 3, 1, 1, 5, 2, 2, 1, 1, 64)
+CONV_SPLIT_TEST(j, 24, 48, 17, 17, 3, 3, 2, 0, 3, 1, 3, 1, 1, 128)
+CONV_SPLIT_TEST(k, 48, 32, 8, 12, 5, 5, 1, 2, 2, 1, 2, 2, 2, 64)
+CONV_SPLIT_TEST(l, 16, 80, 12, 10, 5, 6, 3, 2, 7, 1, 4, 1, 1, 64)
 DENSE_SPLIT_TEST(a, 160, 96, 144, 2, 4, 1, 1, 64)
 DENSE_SPLIT_TEST(b, 128, 256, 96, 2, 4, 1, 2, 96)
 DENSE_SPLIT_TEST(c, 256, 64, 224, 2, 8, 1, 1, 112)

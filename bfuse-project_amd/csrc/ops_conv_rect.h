@@ -27,6 +27,7 @@
 #include "ops_conv_1x1.h"
 #include "ops_conv_general.h"
 #include "ops_conv_tile.h"
+#include "ops_gemm_split.h"
 #include "ops_gemm_tile.h"
 #include "wave.h"
 
@@ -291,6 +292,13 @@ struct ConvF32Rect {
     }
 };
 
+// The product on the bf16 matrix cores under ConvF32Lds's name: BM output channels and 16 PB pixels of a workgroup of KS waves,
+// which split the channels.
+constexpr int kSplitForm = 32;
+template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int BM, int PB, int KS, int NIMG>
+struct ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, KS, NIMG, kSplitForm>
+    : SwapOperands<GemmSplit<CO, CI * KH * KW, H, W, S, NIMG, BM / 16 / KS, KS, 1, 1, 16 * PB, kPix, KH, KW, P>> {};
+
 // The tiling the library gives a convolution it has no hand-picked one for: as many output channels per
 // workgroup as keep the filter fragments of a wave within ~72 registers (the staged patch is shared by all
 // of them), 64 pixels (or the whole image when it has fewer), and as many waves over the channel groups as
@@ -414,10 +422,28 @@ struct ConvTiling {
         if constexpr (STREAM && tile_bm() >= 32 && (long long)((OHW + 3) / 4 * 4) * NIMG / GBN * (CO / GBM) >= 512) return product::FITS;
         return false;
     }
+    // Filters larger than 1 x 1 with many output channels: as a product on the bf16 matrix cores whose second operand is gathered
+    // from the images (GemmSplit).  The tile is the largest of 256 x 128 (eight waves), 128 x 128, 192 x 64 (four waves, two
+    // workgroups a CU) and 160 x 128 (ten waves of 16 rows) whose rows divide the channels, on at least two rounds over the CUs.
+    // Batch 1024, us, shared tiles before: 256 -> 256 on 14 x 14 1713 -> 1022 (128 x 128: 1115), 512 on 7 x 7 1730 -> 1178 (1191),
+    // 128 on 28 x 28 1693 -> 1133, 448 -> 384 on 8 x 8 1389 -> 906, 288 -> 384 at stride 2 4196 -> 2847 (192 x 128: 3123), 80 -> 192
+    // on 73 x 73 10257 -> 7642, 192 -> 320 at stride 2 521 -> 376 (128 x 128 on 2.5 tiles: 433).  Fewer channels give the
+    // gathered operand too few uses for what taking it apart costs: 64 -> 64 on 56 x 56 1740 against 1709-2330, 96 -> 96 on 35 x 35
+    // 1521 against 1345-1654.
+    static constexpr int SBM = CO % 256 == 0 ? 256 : CO % 128 == 0 ? 128 : CO % 192 == 0 ? 192 : 160;
+    using split = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, SBM, SBM == 192 ? 4 : 8, SBM == 256 ? 8 : SBM == 160 ? 10 : 4, NIMG, kSplitForm>;
+    static constexpr bool is_split()
+    {
+        // (the table of taps is made at compile time)
+        if constexpr (T > 1 && T < 31 && CI >= 16 && CI * T % 8 == 0 && CI * T <= 32768 && KH >= S && (CO % 128 == 0 || CO % 192 == 0 || CO % 160 == 0))
+            return split::FITS && split::TILES >= 512;
+        return false;
+    }
     template <int FORM, class Else> struct pick { using type = Else; };
+    template <class Else> struct pick<3, Else> { using type = split; };
     template <class Else> struct pick<1, Else> { using type = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, TBM, TPB, 4, NIMG, TWM>; };
     template <class Else> struct pick<2, Else> { using type = SwapOperands<product>; };
-    using type = typename pick<is_product() ? 2 : tiled(TPB) ? 1 : 0, std::conditional_t<STREAM, Conv1x1F32<CI, CO, H, W, S, stream_bm(), 4, NIMG>, held>>::type;
+    using type = typename pick<is_split() ? 3 : is_product() ? 2 : tiled(TPB) ? 1 : 0, std::conditional_t<STREAM, Conv1x1F32<CI, CO, H, W, S, stream_bm(), 4, NIMG>, held>>::type;
 };
 template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int NIMG = 1>
 using ConvF32Auto = typename ConvTiling<CI, CO, H, W, KH, KW, S, P, NIMG>::type;

@@ -28,7 +28,12 @@
 // 64 x 64 a workgroup take more time than the fp32 forms: 1024 x 3072 x 768 63 (64 x 96 tiles) against 39.
 //
 // B comes in one of two layouts, as in GemmTile: kPix, planes of n for each k ([K, N] is one image of N pixels); kRows, rows
-// contiguous along k, NIMG independent products.  A row tile (kRows: also a column tile) that does not divide the problem starts
+// contiguous along k, NIMG independent products.  With a filter of KH x KW taps (kPix) the product is a convolution: A holds the
+// filters as they lie in memory, k counts (channel, tap), and what a column loads for k is its window's element.  All lanes of a
+// load want the same k, so where the element lies from the window's first one comes from a table by a scalar load; padding is a
+// lane whose bit for that tap is set and which therefore reads past the buffer (two vector instructions a load).  Every element
+// is taken apart once for each tap it is under: 256 -> 256 channels on 14 x 14, batch 1024, 1713 -> 1022 us (232 TFLOP/s);
+// ConvTiling has the other layers and where the line to the shared tiles lies.  A row tile (kRows: also a column tile) that does not divide the problem starts
 // a tile before its end and writes the same bits as its neighbour.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -44,13 +49,14 @@ namespace bfuse {
 
 // M, K, H, W, S, NIMG, LAYOUT: as in GemmTile.  TM 16-row blocks of a wave, WR waves over the rows and WN over the BN columns, KG
 // groups of such waves over the stages.
-template <int M_, int K_, int H_, int W_, int S_, int NIMG_, int TM_, int WR_, int WN_, int KG_, int BN_, int LAYOUT_>
+template <int M_, int K_, int H_, int W_, int S_, int NIMG_, int TM_, int WR_, int WN_, int KG_, int BN_, int LAYOUT_, int KH_ = 1, int KW_ = 1, int P_ = 0>
 struct GemmSplit {
     static constexpr bool MATRIX_CORES = true;   // the inner loop is a stream of MFMAs (what the fusion chooser asks)
-    static constexpr int M = M_, K = K_, H = H_, W = W_, S = S_, NIMG = NIMG_, TM = TM_, WR = WR_, WN = WN_, KG = KG_, BN = BN_, LAYOUT = LAYOUT_;
+    static constexpr int M = M_, K = K_, H = H_, W = W_, S = S_, NIMG = NIMG_, TM = TM_, WR = WR_, WN = WN_, KG = KG_, BN = BN_, LAYOUT = LAYOUT_, KH = KH_, KW = KW_, P = P_;
+    static constexpr int T = KH * KW, CI = K / T;                                // kPix: taps, channels of the images
     static constexpr int NWAVE = WR * WN * KG, THREADS = 64 * NWAVE, GT = 64 * WR * WN, BM = 16 * TM * WR, TN = BN / WN / 16;
     static constexpr int NS = (K + 31) / 32, NIT = NS / KG, TAIL = K % 32;       // stages, those of a group, k of the last one if not 32
-    static constexpr int OH = (H - 1) / S + 1, OW = (W - 1) / S + 1, HW = H * W, OHW = OH * OW;
+    static constexpr int OH = (H - KH + 2 * P) / S + 1, OW = (W - KW + 2 * P) / S + 1, HW = H * W, OHW = OH * OW;
     static constexpr int OHWP = (OHW + 3) / 4 * 4;                               // columns of an image, whole chunks of four
     static constexpr int MT = (M + BM - 1) / BM;
     static constexpr int NT = LAYOUT == kRows ? (W + BN - 1) / BN : (int)(((long long)OHWP * NIMG + BN - 1) / BN);
@@ -58,7 +64,7 @@ struct GemmSplit {
     static constexpr int NUJ = (4 * BN + GT - 1) / GT;                           // units (a column's eight k) of a thread and stage
     static_assert(BN % (16 * WN) == 0 && K % 8 == 0 && NS % KG == 0 && M >= BM && (LAYOUT == kPix || (W >= BN && H == 1 && S == 1)), "tile");
     // 31-bit offsets; padding is read through one that lies past the buffer
-    static constexpr bool FITS = (long long)BM * K * 4 < (1LL << 31) && (long long)(NIMAGES < NIMG ? NIMAGES : NIMG) * K * HW * 4 < (1LL << 31);
+    static constexpr bool FITS = (long long)BM * K * 4 < (1LL << 31) && (long long)(NIMAGES < NIMG ? NIMAGES : NIMG) * CI * HW * 4 < (1LL << (T == 1 ? 31 : 29));
     static constexpr int PLANE = 4 * BN * 16, BUF = 3 * PLANE, NBUF = 3;
     static constexpr int TILES = MT * NT;
     static constexpr Dims3 GRID{LAYOUT == kRows ? TILES * NIMG : TILES, 1, 1};
@@ -72,6 +78,18 @@ struct GemmSplit {
         __attribute__((aligned(16))) unsigned char t[NBUF * KG * BUF > RED_BYTES ? NBUF * KG * BUF : RED_BYTES];
         unsigned inexact;
     };
+
+    // Filters larger than 1 x 1: where element k = (channel, row, column) of a window lies from its first one, in bytes, times
+    // eight, and the tap's number in the low five bits; past the last k a tap that no window has.
+    struct Taps {
+        unsigned at[T > 1 ? NS * 32 : 1];
+        constexpr Taps() : at{}
+        {
+            for (int k = 0; T > 1 && k < NS * 32; ++k) at[k] = k < K ? (unsigned)((k / T * HW + k % T / KW * W + k % KW) * 4) << 3 | (unsigned)(k % T) : 31u;
+        }
+    };
+    __device__ static constexpr Taps TAPS{};
+    static_assert(T == 1 || (LAYOUT == kPix && BN % 64 == 0 && T < 31 && K % T == 0), "a wave's units are one octet's");
 
     // (column tile, row tile), dealt so that the row tiles of one column tile follow each other on one XCD
     __device__ static __forceinline__ void tile_of(int vblock, int& nt, int& mt)
@@ -122,26 +140,35 @@ struct GemmSplit {
         const int n_lo = LAYOUT == kRows ? 0 : (int)(n0 / OHWP);                 // kPix: first image of the tile
         const int v0 = (int)(n0 - (long long)n_lo * OHWP);
 
-        // offset of B(0, column c of the tile); past the buffer if there is none
-        auto column = [&](int c) -> unsigned {
+        // Offset of B(0, column c of the tile); past the buffer if there is none.  Filters larger than 1 x 1: of its window's first
+        // element, counted from P rows and columns before the images; `outside` gets a bit for every tap that is in the padding.
+        auto column = [&](int c, unsigned& outside) -> unsigned {
             if constexpr (LAYOUT == kRows) return (unsigned)(c * K * 4);
-            const int v = v0 + c, img = v / OHWP, p = v % OHWP;
-            return p < OHW && n_lo + img < NIMG ? (unsigned)((img * K * HW + (p / OW) * S * W + (p % OW) * S) * 4) : 0x7fffffffu;
+            const int v = v0 + c, img = v / OHWP, p = v % OHWP, y = (p / OW) * S, x = (p % OW) * S;
+            const bool in = p < OHW && n_lo + img < NIMG;
+            outside = in ? 0x80000000u : ~0u;
+            if constexpr (P > 0)
+#pragma unroll
+                for (int t = 0; t < T; ++t)
+                    if (y + t / KW < P || y + t / KW >= H + P || x + t % KW < P || x + t % KW >= W + P) outside |= 1u << t;
+            return in ? (unsigned)((img * CI * HW + y * W + x) * 4) : 0x7fffffffu;
         };
         constexpr unsigned B_K = LAYOUT == kRows ? 4 : HW * 4;                   // bytes from one k of a column to the next
         const auto ar = __builtin_amdgcn_make_buffer_rsrc((void*)(A + (size_t)m0 * K), 0, BM * K * 4, 0x00020000);
-        const auto br = __builtin_amdgcn_make_buffer_rsrc((void*)(LAYOUT == kRows ? B + (size_t)n0 * K : B + (size_t)n_lo * K * HW), 0,
-                                                          LAYOUT == kRows ? BN * K * 4 : (NIMG - n_lo < NIMAGES ? NIMG - n_lo : NIMAGES) * K * HW * 4, 0x00020000);
+        const auto br = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)(LAYOUT == kRows ? B + (size_t)n0 * K : B + (size_t)n_lo * CI * HW - (P * W + P)), 0,
+            LAYOUT == kRows ? BN * K * 4 : ((NIMG - n_lo < NIMAGES ? NIMG - n_lo : NIMAGES) * CI * HW + P * W + P) * 4, 0x00020000);
         const unsigned a_voff = (unsigned)(((wr * TM * 16 + li) * K + 8 * kq) * 4);
-        unsigned b_voff[NUJ];
-        int b_lds[NUJ];
+        unsigned b_voff[NUJ], b_out[NUJ];
+        int b_lds[NUJ], b_k[NUJ];
 #pragma unroll
         for (int j = 0; j < NUJ; ++j) {
             // threads past the last unit do one of the first ones again: the same values to the same place.  kRows: four lanes
             // read 128 consecutive bytes of a row; kPix: 64 lanes 64 consecutive columns of a plane
             const int u = (j * GT + gt) % (4 * BN), o = LAYOUT == kRows ? u & 3 : u / BN, c = LAYOUT == kRows ? u >> 2 : u % BN;
-            const unsigned v = column(c);
-            b_voff[j] = v == 0x7fffffffu ? v : v + 8 * o * B_K;
+            const unsigned v = column(c, b_out[j]);
+            b_voff[j] = T > 1 || v == 0x7fffffffu ? v : v + 8 * o * B_K;
+            b_k[j] = T > 1 ? __builtin_amdgcn_readfirstlane(8 * o) : 0;
             b_lds[j] = (o * BN + c) * 16;
         }
 
@@ -159,13 +186,21 @@ struct GemmSplit {
             for (int h = 0; h < 2; ++h) ra[tm][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ar, v + h * 16, s * 128, 0));
         };
         auto load_b = [&](int j, int s) {
-            const unsigned v = TAIL != 0 && s == NS - 1 && b_lds[j] >= TAIL / 8 * BN * 16 ? 0x7fffffffu : b_voff[j];
+            const unsigned v = T == 1 && TAIL != 0 && s == NS - 1 && b_lds[j] >= TAIL / 8 * BN * 16 ? 0x7fffffffu : b_voff[j];
             if constexpr (LAYOUT == kRows) {
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     const f32x4 f = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(br, v + h * 16, s * 128, 0));
 #pragma unroll
                     for (int e = 0; e < 4; ++e) rb[j][4 * h + e] = f[e];
+                }
+            } else if constexpr (T > 1) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const unsigned at = TAPS.at[s * 32 + b_k[j] + e];
+                    // all ones (past the buffer) if this tap's bit is set; without padding only the last stage has such
+                    const unsigned o = P > 0 || TAIL != 0 ? (unsigned)__builtin_amdgcn_sbfe((int)b_out[j], at, 1) : 0u;
+                    rb[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(br, v | o, (at >> 5) * 4, 0));
                 }
             } else {
 #pragma unroll
@@ -308,12 +343,20 @@ struct GemmSplit {
         if (again) {
 #pragma unroll
             for (int b = 0; b < TN; ++b) {
-                const unsigned c = column((wn * TN + b) * 16 + li), v = c == 0x7fffffffu ? c : c + kq * B_K;
+                unsigned outside;
+                const unsigned c = column((wn * TN + b) * 16 + li, outside), v = T > 1 || c == 0x7fffffffu ? c : c + kq * B_K;
 #pragma unroll
                 for (int tm = 0; tm < TM; ++tm) acc[tm][b] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
                 for (int k = 0; k < K; k += 4) {
-                    const float bv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(br, v, k * B_K, 0));
+                    unsigned at = k * B_K, o = v;
+                    if constexpr (T > 1) {
+                        at = TAPS.at[k + kq];
+                        o |= (unsigned)__builtin_amdgcn_sbfe((int)outside, at, 1);
+                        if (o != ~0u) o += (at >> 5) * 4;
+                        at = 0;
+                    }
+                    const float bv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(br, o, at, 0));
 #pragma unroll
                     for (int tm = 0; tm < TM; ++tm) {
                         const float av = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ar, (((wr * TM + tm) * 16 + li) * K + kq) * 4, k * 4, 0));

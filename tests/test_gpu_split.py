@@ -2,6 +2,7 @@
 (products: numpy in double), alone and fused; their error against 64 bits; and operands that three bf16 cannot hold."""
 import numpy as np
 import pytest
+import torch
 
 import bfuse_project_amd as bf
 from bfuse_project_amd.operation import fill_normal
@@ -27,6 +28,30 @@ def test_split_product_against_numpy_and_fused(tag, partner, kind, suffix):
 @pytest.mark.parametrize("tag,s", [("g", 1), ("h", 2)])
 def test_split_1x1_convolution_against_the_oracle(tag, s):
     _check(f"selftest_gemm_split_{tag}", lambda x, w: orf.conv2d(x, w, s=s, p=0), "bias_relu_4096", None, "")
+
+
+@pytest.mark.parametrize("tag,s,p", [("i", 1, 1), ("j", 2, 0), ("k", 1, 2), ("l", 3, 2)])
+def test_split_convolution_against_the_oracle(tag, s, p):
+    _check(f"selftest_gemm_split_{tag}", lambda x, w: orf.conv2d(x, w, s=s, p=p), "bias_relu_4096", None, "")
+
+
+@pytest.mark.parametrize("tag,s,p", [("i", 1, 1), ("j", 2, 0)])
+def test_infinite_and_tiny_pixels_of_a_split_convolution(tag, s, p):
+    """An infinite, a NaN and a lowest value are in the windows that hold them and in no others (padding beside them is not
+    multiplied), an image of values below bf16's bits keeps its own."""
+    name = f"selftest_gemm_split_{tag}"
+    x, w = _operands(name)
+    w = np.abs(w) + np.float32(0.5)
+    x[0, 3, 0, 0], x[1, 5, 4, 3], x[1, 2, 0, 6], x[0, 7, 5, 5] = np.inf, np.nan, -np.inf, np.finfo(np.float32).min
+    x[2] *= np.float32(2.0 ** -118)
+    with np.errstate(all="ignore"):
+        want = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(w).double(), stride=s, padding=p).numpy()
+        f = want.astype(np.float32)
+    y = _run(name, x, w)
+    assert np.array_equal(np.isnan(y), np.isnan(f)) and np.array_equal(np.isposinf(y), np.isposinf(f)) and np.array_equal(np.isneginf(y), np.isneginf(f))
+    for n in range(x.shape[0]):
+        ok = np.isfinite(f[n])
+        assert ok.any() and np.linalg.norm((y[n][ok] - want[n][ok])) <= 1e-5 * np.linalg.norm(want[n][ok])
 
 
 def _run(name, x, w):
