@@ -439,11 +439,25 @@ struct ConvTiling {
             return split::FITS && split::TILES >= 512;
         return false;
     }
+    // 1 x 1 filters on 256 and more channels likewise, also on 224 x 128 tiles (seven waves).  us, GemmTile before: 768 -> 192 on
+    // 17 x 17 690 -> 534 (twelve waves of 16 rows 514, but no register is left beside twelve waves), 160 594 -> 464, 128 490 -> 344,
+    // 1280 -> 448 on 8 x 8 545 -> 374, 384 460 -> 311, 320 394 -> 293, 192 237 -> 179, 2048 -> 448 831 -> 584, 256 -> 256 on 56 x 56
+    // 3168 -> 2513, 256 -> 512 at stride 2 146 -> 121.  On fewer channels the tile's ends are too much of it: 128 -> 256 at stride 2
+    // 152 against 177, 64 -> 128 202 against 218; 64 output channels 394 against 383-410.
+    static constexpr int S1BM = CO % 256 == 0 ? 256 : CO % 128 == 0 ? 128 : CO % 224 == 0 ? 224 : CO % 192 == 0 ? 192 : 160;
+    static constexpr int S1WR = S1BM == 256 ? 8 : S1BM == 224 ? 7 : S1BM == 160 ? 10 : 4;
+    using split_product = GemmSplit<CO, CI, H, W, S, NIMG, S1BM / 16 / S1WR, S1WR, 1, 1, S1BM == 192 ? 64 : 128, kPix>;
+    static constexpr bool is_split_product()
+    {
+        if constexpr (STREAM && CI >= 256 && CO % S1BM == 0) return split_product::FITS && split_product::TILES >= 512;
+        return false;
+    }
     template <int FORM, class Else> struct pick { using type = Else; };
     template <class Else> struct pick<3, Else> { using type = split; };
+    template <class Else> struct pick<4, Else> { using type = SwapOperands<split_product>; };
     template <class Else> struct pick<1, Else> { using type = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, TBM, TPB, 4, NIMG, TWM>; };
     template <class Else> struct pick<2, Else> { using type = SwapOperands<product>; };
-    using type = typename pick<is_split() ? 3 : is_product() ? 2 : tiled(TPB) ? 1 : 0, std::conditional_t<STREAM, Conv1x1F32<CI, CO, H, W, S, stream_bm(), 4, NIMG>, held>>::type;
+    using type = typename pick<is_split() ? 3 : is_split_product() ? 4 : is_product() ? 2 : tiled(TPB) ? 1 : 0, std::conditional_t<STREAM, Conv1x1F32<CI, CO, H, W, S, stream_bm(), 4, NIMG>, held>>::type;
 };
 template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int NIMG = 1>
 using ConvF32Auto = typename ConvTiling<CI, CO, H, W, KH, KW, S, P, NIMG>::type;
