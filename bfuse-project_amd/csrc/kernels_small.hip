@@ -249,3 +249,14 @@ CONV1_SPLIT_TEST(h, 56, 64, 9, 7, 2, 11, 2, 2, 1, 2, 96)
 BFUSE_BFUSE_KERNEL(selftest_gemm_split_a, GemmSp_a, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
 BFUSE_HFUSE_KERNEL(selftest_gemm_split_e, GemmSp_e, bias_relu_4096, BiasReluS)
 BFUSE_HFUSE_KERNEL(selftest_gemm_split_f, GemmSp_f, conv3x3_f32_32x12x12_32, ConvS2)
+
+// The split-K product on the bf16 matrix cores: a trailing 16-column group and GELU in one round, two waves in two rounds, one stage.
+using GemmSpk_a = GemmF32Dma<64, 288, 256, 32, 144, 4, kEpiGeluTanh>;
+using GemmSpk_b = GemmF32Dma<96, 256, 192, 32, 128, 2, kEpiNone, 2>;
+using GemmSpk_c = GemmF32Dma<32, 384, 128, 32, 192, 4, kEpiNone, 2>;
+BFUSE_KERNEL(selftest_gemm_splitk_a, GemmSpk_a, ({{64, 256, 1, 1}, 4}), ({{256, 288, 1, 1}, 4}), ({{64, 288, 1, 1}, 4}))
+BFUSE_KERNEL(selftest_gemm_splitk_b, GemmSpk_b, ({{96, 192, 1, 1}, 4}), ({{192, 256, 1, 1}, 4}), ({{96, 256, 1, 1}, 4}))
+BFUSE_KERNEL(selftest_gemm_splitk_c, GemmSpk_c, ({{32, 128, 1, 1}, 4}), ({{128, 384, 1, 1}, 4}), ({{32, 384, 1, 1}, 4}))
+BFUSE_BFUSE_KERNEL(selftest_gemm_splitk_a, GemmSpk_a, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
+BFUSE_HFUSE_KERNEL(selftest_gemm_splitk_b, GemmSpk_b, bias_relu_4096, BiasReluS)
+BFUSE_HFUSE_KERNEL(selftest_gemm_splitk_b, GemmSpk_b, conv3x3_f32_32x12x12_32, ConvS2)

@@ -42,14 +42,16 @@
 
 #include "dispatch.h"
 #include "ops_gemm_f32.h"
+#include "ops_gemm_splitk.h"
 #include "wave.h"
 
 namespace bfuse {
 
+// The fp32 form of GemmF32Dma.
 // (One producer wave per k-range issuing the loads was tried: it has to meet its compute wave at a
 // workgroup barrier per K-stage, which costs about what the six loads per stage did -- no faster.)
 template <int M_, int N_, int K_, int BM_, int BN_, int KS_, int EPI_ = kEpiNone, int NSTG_ = 3>
-struct GemmF32Dma {
+struct GemmF32Ring {
     static constexpr bool MATRIX_CORES = true;   // the inner loop is a stream of MFMAs (what the fusion chooser asks)
     static constexpr int M = M_, N = N_, K = K_, BM = BM_, BN = BN_, KS = KS_, EPI = EPI_, NSTG = NSTG_;
     static constexpr int TM = BM / 16;
@@ -459,5 +461,20 @@ struct GemmF32Dma {
             C[(size_t)(m0 + tm * 16 + 4 * rg + v) * N + n0 + G4 * 64 + g * 16 + j] = epilogue(blk[v]);
     }
 };
+
+// Which of the two a product gets: the bf16 matrix cores (GemmSplitK) for tiles of at least 32 x 128, or of 32 x 96 where two
+// workgroups share a CU, whose every wave has whole stages of 32 k (its comment has both sides of the line); the fp32 ring for the
+// others.  NSTG is the stages of the ring; the split form's partial sums meet in rounds where all at once would take more LDS than it.
+template <int M, int N, int K, int BM, int BN, int KS, int EPI, int NSTG>
+struct GemmF32DmaForm {
+    static constexpr int RING = KS * NSTG * (BM * 32 + (8 * BN * 4 + 1023) / 1024 * 1024), FULL = KS * BM * BN * 4;
+    static constexpr bool SPLIT = K % (32 * KS) == 0 && KS > 1 && BM == 32 && BN % 16 == 0 && (long long)K * N * 4 < (1LL << 31) && (long long)BM * K * 4 < (1LL << 31) &&
+                                  (BN >= 128 || (BN >= 96 && (M / BM) * (N / BN) >= 512));
+    template <bool S, class = void> struct pick { using type = GemmF32Ring<M, N, K, BM, BN, KS, EPI, NSTG>; };
+    template <class X> struct pick<true, X> { using type = GemmSplitK<M, N, K, BM, BN, KS, EPI, FULL <= RING ? 1 : 2>; };
+    using type = typename pick<SPLIT>::type;
+};
+template <int M_, int N_, int K_, int BM_, int BN_, int KS_, int EPI_ = kEpiNone, int NSTG_ = 3>
+struct GemmF32Dma : GemmF32DmaForm<M_, N_, K_, BM_, BN_, KS_, EPI_, NSTG_>::type {};
 
 }  // namespace bfuse

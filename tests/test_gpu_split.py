@@ -1,4 +1,4 @@
-"""fp32 products on the bf16 matrix cores (csrc/split.h, ops_gemm_split.h): the edges of tiles and stages against the oracle
+"""fp32 products on the bf16 matrix cores (csrc/split.h, ops_gemm_split.h, ops_gemm_splitk.h): the edges of tiles and stages against the oracle
 (products: numpy in double), alone and fused; their error against 64 bits; and operands that three bf16 cannot hold."""
 import numpy as np
 import pytest
@@ -23,6 +23,16 @@ def _product(a, b):
     ("e", "bias_relu_4096", "hfuse", ""), ("f", "conv3x3_f32_32x12x12_32", "hfuse", "")])
 def test_split_product_against_numpy_and_fused(tag, partner, kind, suffix):
     _check(f"selftest_gemm_split_{tag}", lambda a, b: _product(a, b).astype(np.float32), partner, kind, suffix)
+
+
+def _gelu(x):
+    return 0.5 * x * (1 + np.tanh(0.797885 * (x + 0.044715 * x ** 3)))
+
+
+@pytest.mark.parametrize("tag,partner,kind,suffix", [
+    ("a", "layernorm_8x256", "bfuse", "_c4"), ("b", "bias_relu_4096", "hfuse", ""), ("b", "conv3x3_f32_32x12x12_32", "hfuse", ""), ("c", "bias_relu_4096", None, "")])
+def test_split_k_product_against_numpy_and_fused(tag, partner, kind, suffix):
+    _check(f"selftest_gemm_splitk_{tag}", lambda a, b: (_gelu if tag == "a" else np.asarray)(_product(a, b)).astype(np.float32), partner, kind, suffix)
 
 
 @pytest.mark.parametrize("tag,s", [("g", 1), ("h", 2)])
@@ -68,23 +78,24 @@ def _operands(name):
     return [fill_normal(11 + i, int(np.prod(k.shapes[i])), 0, 1).reshape(k.shapes[i]) for i in (0, 1)]
 
 
-@pytest.mark.parametrize("tag,steps,groups", [("d", 4096 // 32, 1), ("b", 256 // 32, 2)])
+@pytest.mark.parametrize("tag,steps,groups", [("_d", 4096 // 32, 1), ("_b", 256 // 32, 2), ("k_b", 6 * 192 // 32, 2), ("k_c", 6 * 128 // 32, 4)])
 def test_split_product_is_closer_to_64_bits_than_one_fp32_sum(tag, steps, groups):
     """One rounding of at most u = 2^-24 of what the sum has grown to for every 32 k: u sqrt(steps / 2) (2-norm), in two groups
-    sqrt(2) less and u for adding them; the products that are left out and the sum of the small ones add less than u / 2."""
-    name = f"selftest_gemm_split_{tag}"
+    sqrt(2) less and u for adding them; the products that are left out and the sum of the small ones add less than u / 2.  Split
+    over K (no sum of their own for the small ones) it is rounded six times for 32 k."""
+    name = f"selftest_gemm_split{tag}"
     x, w = _operands(name)
     want = _product(x, w)
     err = np.linalg.norm(_run(name, x, w).reshape(want.shape) - want) / np.linalg.norm(want)
     assert err <= 2.0 ** -24 * ((steps / 2 / groups) ** 0.5 + 0.5 + (groups > 1))
 
 
-@pytest.mark.parametrize("tag", ["a", "b", "e"])
+@pytest.mark.parametrize("tag", ["_a", "_b", "_e", "k_b", "k_c"])
 @pytest.mark.parametrize("scale", [2.0 ** -100, 2.0 ** -118, 2.0 ** 100])
 def test_scaled_operands_keep_their_bits(tag, scale):
     """A power of two on an operand is one on the result, however small the operand's own low bits become (whole operand, one
     row or column among others, a column of zeros beside it)."""
-    name = f"selftest_gemm_split_{tag}"
+    name = f"selftest_gemm_split{tag}"
     x, w = _operands(name)
     scale = np.float32(scale)
     u = 2.0 ** -24 * x.shape[1] ** 0.5 * 2     # twice the bound of one sum rounded after every product
@@ -103,10 +114,10 @@ def test_scaled_operands_keep_their_bits(tag, scale):
         assert np.linalg.norm(y[r] - want[r]) <= u * np.linalg.norm(want[r]), r
 
 
-@pytest.mark.parametrize("tag", ["a", "b", "e"])
+@pytest.mark.parametrize("tag", ["_a", "_b", "_e", "k_b", "k_c"])
 def test_infinities_nan_and_the_largest_values(tag):
     """What does not fit three bf16 gives what fp32 arithmetic gives: infinite where it is, NaN where it is, finite elsewhere."""
-    name = f"selftest_gemm_split_{tag}"
+    name = f"selftest_gemm_split{tag}"
     x, w = _operands(name)
     x2 = x.reshape(-1, x.shape[1] if x.shape[2] == 1 else x.shape[2])      # rows
     big = np.float32(3.4e38)
@@ -114,7 +125,7 @@ def test_infinities_nan_and_the_largest_values(tag):
     x2[2, 1], x2[4, 0], x2[4, 1], x2[7, 3] = np.inf, np.inf, -np.inf, np.nan
     x2[9] = 0
     x2[9, 2], x2[11, 4] = np.finfo(np.float32).min, big
-    if tag != "e":
+    if tag != "_e":
         w2 = w.reshape(w.shape[0], w.shape[1])
         w2[2] = np.float32(0.5)                                            # 0.5 * the lowest value stays finite
         w2[1, 5], w2[0, 6] = np.inf, np.nan
