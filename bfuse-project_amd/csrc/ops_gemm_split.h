@@ -48,12 +48,15 @@
 namespace bfuse {
 
 // M, K, H, W, S, NIMG, LAYOUT: as in GemmTile.  TM 16-row blocks of a wave, WR waves over the rows and WN over the BN columns, KG
-// groups of such waves over the stages.
-template <int M_, int K_, int H_, int W_, int S_, int NIMG_, int TM_, int WR_, int WN_, int KG_, int BN_, int LAYOUT_, int KH_ = 1, int KW_ = 1, int P_ = 0>
+// groups of such waves over the stages.  LEAN: one set of A's parts, taken apart at the top of the stage, instead of the next one's
+// beside this one's: 12 TM registers less for a stage that begins without MFMAs, which other workgroups of the CU fill.
+template <int M_, int K_, int H_, int W_, int S_, int NIMG_, int TM_, int WR_, int WN_, int KG_, int BN_, int LAYOUT_, int KH_ = 1, int KW_ = 1, int P_ = 0,
+          bool LEAN_ = (LAYOUT_ == kRows && K_ <= 256)>
 struct GemmSplit {
     static constexpr bool MATRIX_CORES = true;   // the inner loop is a stream of MFMAs (what the fusion chooser asks)
     static constexpr int M = M_, K = K_, H = H_, W = W_, S = S_, NIMG = NIMG_, TM = TM_, WR = WR_, WN = WN_, KG = KG_, BN = BN_, LAYOUT = LAYOUT_, KH = KH_, KW = KW_, P = P_;
     static constexpr int T = KH * KW, CI = K / T;                                // kPix: taps, channels of the images
+    static constexpr bool LEAN = LEAN_;
     static constexpr int NWAVE = WR * WN * KG, THREADS = 64 * NWAVE, GT = 64 * WR * WN, BM = 16 * TM * WR, TN = BN / WN / 16;
     static constexpr int NS = (K + 31) / 32, NIT = NS / KG, TAIL = K % 32;       // stages, those of a group, k of the last one if not 32
     static constexpr int OH = (H - KH + 2 * P) / S + 1, OW = (W - KW + 2 * P) / S + 1, HW = H * W, OHW = OH * OW;
@@ -210,7 +213,7 @@ struct GemmSplit {
         shared_with_asm(sm.t);
         unsigned char* const base = sm.t + g * NBUF * BUF;
         const unsigned char* const fb = base + (kq * BN + wn * TN * 16 + li) * 16;
-        unsigned pa[2][TM][3][4], pb[3][4];
+        unsigned pa[LEAN ? 1 : 2][TM][3][4], pb[3][4];
         unsigned seen[NUJ + TM] = {};               // bits of the leading parts of each unit
         if (tid == 0) sm.inexact = 0;
         // Two of a unit's eight values: units 0 .. NUJ - 1 are this thread's of B, the others its rows of A.
@@ -230,7 +233,7 @@ struct GemmSplit {
                 if (j % 2 == 1) seen[u] |= p[0][j - 1] | p[0][j];
             }
         };
-        constexpr int NPART = 4 * (NUJ + TM), VPM = (11 * NPART + 6 * TM * TN - 1) / (6 * TM * TN);
+        constexpr int NPART = 4 * (LEAN ? NUJ : NUJ + TM), VPM = (11 * NPART + 6 * TM * TN - 1) / (6 * TM * TN);
         const auto stage_of = [&](int it) { return (it < NIT ? it : NIT - 1) * KG + g; };   // past the end: the last one again
 
 #pragma unroll
@@ -246,10 +249,13 @@ struct GemmSplit {
         }
 #pragma unroll
         for (int j = 0; j < NUJ; ++j) load_b(j, stage_of(2));
+        auto convert_a = [&](int next) {
 #pragma unroll
-        for (int part = 4 * NUJ; part < NPART; ++part) convert(part, 0, 0);
+            for (int part = 4 * NUJ; part < 4 * (NUJ + TM); ++part) convert(part, 0, 0);
 #pragma unroll
-        for (int tm = 0; tm < TM; ++tm) load_a(tm, stage_of(1));
+            for (int tm = 0; tm < TM; ++tm) load_a(tm, stage_of(next));
+        };
+        if constexpr (!LEAN) convert_a(1);
         u32x4 fr[2][3];
         auto read = [&](int set, int q, int b, int off) { fr[set][q] = *reinterpret_cast<const u32x4*>(fb + off + q * PLANE + b * 256); };
         sync.raw();
@@ -260,6 +266,7 @@ struct GemmSplit {
             constexpr int FROM = decltype(from)::value;
             // Behind the barrier the next stage is in LDS whole, and nobody reads the one before this any more.
             if (it > 0) sync.raw();
+            if constexpr (LEAN) convert_a(it + 1);
 #pragma unroll
             for (int b = 0; b < TN; ++b) {
                 const int set = (b + FROM * (TN & 1)) & 1;
@@ -268,7 +275,7 @@ struct GemmSplit {
 #pragma unroll
                     for (int tm = 0; tm < TM; ++tm) {
                         f32x4& c = t + 1 < SplitTerms::N ? low[tm][b] : acc[tm][b];
-                        const unsigned(&p)[4] = pa[FROM][tm][SplitTerms::A[t]];
+                        const unsigned(&p)[4] = pa[LEAN ? 0 : FROM][tm][SplitTerms::A[t]];
                         c = mfma_bf16(fr[set][SplitTerms::B[t]], u32x4{p[0], p[1], p[2], p[3]}, c);
                     }
                     if (t == 0 || t == 2 || t == 4) read(set ^ 1, 2 - t / 2, b + 1 < TN ? b + 1 : 0, b + 1 < TN ? off : next);
@@ -276,7 +283,7 @@ struct GemmSplit {
 #pragma unroll
                 for (int part = 0; part < NPART; ++part)
                     if (part * TN / NPART == b) {
-                        convert(part, FROM ^ 1, ahead);
+                        convert(part, LEAN ? 0 : FROM ^ 1, ahead);
                         if (part % 4 == 3) {
                             if (part / 4 < NUJ) load_b(part / 4, stage_of(it + 3));
                             else load_a(part / 4 - NUJ, stage_of(it + 2));
