@@ -31,7 +31,8 @@ DENSE_SPLIT(1024, 4096, 14336, 2, 8, 1, 1, 128)
 DENSE_SPLIT(1024, 14336, 4096, 2, 4, 1, 2, 128)
 
 // C[b] = A[b] . B[b]^T, A [b, M, K], B [b, N, K]: <M, N, K, BM, BN, waves over K>
-// 256 x 80 x 256 runs on shared tiles (GemmTile), 128 x 128 in three buffers of 16 k: 0.142 -> 0.122 ms.
+// 512 x 64 x 512 and 256 x 80 x 256 run on shared tiles (GemmTile), 128 x 128 in three buffers of 16 k (0.46-0.50 -> 0.38-0.42 ms
+// from card to card, 0.142 -> 0.122).
 #define BGEMM_F32_TILE(B, M, K, N, BM, BN, WM, KS, NBUF)                                                         \
     using Bgemm_##B##x##M##x##K##x##N = GemmTile<M, K, 1, N, 1, B, BM, BN, WM, KS, kRows, NBUF>;                  \
     BFUSE_KERNEL(bgemm_f32_##B##x##M##x##K##x##N, Bgemm_##B##x##M##x##K##x##N, ({{B, M, K, 1}, 4}), ({{B, N, K, 1}, 4}), ({{B, M, N, 1}, 4}))
@@ -44,13 +45,13 @@ DENSE_SPLIT(1024, 14336, 4096, 2, 4, 1, 2, 128)
 // The bf16 matrix cores (ops_gemm_split.h), us, before (shared tiles; 80 columns a tile per wave) and now: 1024 products 512 x 512 x 128
 // 555 -> 420 on 128 x 128 tiles (256 x 128 of eight waves 408, which leave no room for a partner), 512 x 128 x 512 625 -> 545, 512 x
 // 512 x 64 334 -> 278, 1024 x 512 x 64 607 -> 536, 256 x 256 x 64 95.6 -> 87, 256 x 256 x 80 134 -> 100; with a reduction of 64, whose
-// tiles are mostly ends, 512 x 64 x 512 380 -> 356 and 256 x 64 x 256 99 -> 95 on 128 x 64 tiles (128 x 128 364 and 97), 1024 x 64 x 512
-// 708 -> 676 on 128 x 128 (128 x 64 717).  Not for 256 x 80 x 256 (121 against 122), nor for 208 x 208 x 64 (75.9 against 74); 208 x
+// tiles are mostly ends, 256 x 64 x 256 98 -> 94.5 on 128 x 64 tiles (128 x 128 97), 1024 x 64 x 512 705 -> 676 on 128 x 128 (128 x 64
+// 717).  Not for 512 x 64 x 512 (359-380 against 352-362 on 128 x 64), 256 x 80 x 256 (121 against 122), nor for 208 x 208 x 64 (75.9 against 74); 208 x
 // 64 x 208, x 80 x 208 and x 208 x 80 gain 1.1-1.2x on seven waves but keep the one-wave forms, which any operator can take beside it.
 #define BGEMM_F32_SPLIT(B, M, K, N, ...)                                                                         \
     using Bgemm_##B##x##M##x##K##x##N = GemmSplit<M, K, 1, N, 1, B, __VA_ARGS__, kRows>;                          \
     BFUSE_KERNEL(bgemm_f32_##B##x##M##x##K##x##N, Bgemm_##B##x##M##x##K##x##N, ({{B, M, K, 1}, 4}), ({{B, N, K, 1}, 4}), ({{B, M, N, 1}, 4}))
-BGEMM_F32_SPLIT(1024, 512, 64, 512, 2, 4, 1, 1, 64)
+BGEMM_F32_TILE(1024, 512, 64, 512, 128, 128, 2, 16, 3)
 BGEMM_F32_SPLIT(1024, 512, 512, 64, 2, 4, 1, 1, 64)
 BGEMM_F32_SPLIT(1024, 512, 128, 512, 2, 4, 1, 1, 128)
 BGEMM_F32_SPLIT(1024, 512, 512, 128, 2, 4, 1, 1, 128)

@@ -292,12 +292,23 @@ struct ConvF32Rect {
     }
 };
 
-// The product on the bf16 matrix cores under ConvF32Lds's name: BM output channels and 16 PB pixels of a workgroup of KS waves,
-// which split the channels.
+// The product on the bf16 matrix cores under ConvF32Lds's name: BM output channels and 16 PB pixels of the batch for a workgroup of
+// KS waves, which split the channels.  A shared tile like ConvF32Tile, whose place it takes: only what a workgroup does with it differs.
 constexpr int kSplitForm = 32;
 template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int BM, int PB, int KS, int NIMG>
-struct ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, KS, NIMG, kSplitForm>
-    : SwapOperands<GemmSplit<CO, CI * KH * KW, H, W, S, NIMG, BM / 16 / KS, KS, 1, 1, 16 * PB, kPix, KH, KW, P>> {};
+struct ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, KS, NIMG, kSplitForm> : ConvF32Tile<CI, CO, H, W, KH, KW, S, P, BM, 16 * PB, 1, NIMG> {
+    using Form = SwapOperands<GemmSplit<CO, CI * KH * KW, H, W, S, NIMG, BM / 16 / KS, KS, 1, 1, 16 * PB, kPix, KH, KW, P>>;
+    static constexpr long long TILES = Form::TILES;
+    static constexpr bool FITS = Form::FITS;
+    static constexpr Dims3 GRID = Form::GRID, BLOCK = Form::BLOCK;
+    static constexpr int THREADS = Form::THREADS, MIN_BARRIERS = Form::MIN_BARRIERS;
+    using Smem = typename Form::Smem;
+    template <class Sync>
+    __device__ static __forceinline__ void run(int vblock, int tid, Smem& sm, const void* I, const void* F, void* O, Sync sync)
+    {
+        Form::run(vblock, tid, sm, I, F, O, sync);
+    }
+};
 
 // The tiling the library gives a convolution it has no hand-picked one for: as many output channels per
 // workgroup as keep the filter fragments of a wave within ~72 registers (the staged patch is shared by all
@@ -422,20 +433,22 @@ struct ConvTiling {
         if constexpr (STREAM && tile_bm() >= 32 && (long long)((OHW + 3) / 4 * 4) * NIMG / GBN * (CO / GBM) >= 512) return product::FITS;
         return false;
     }
-    // Filters larger than 1 x 1 with many output channels: as a product on the bf16 matrix cores whose second operand is gathered
-    // from the images (GemmSplit).  The tile is the largest of 256 x 128 (eight waves), 128 x 128, 192 x 64 (four waves, two
-    // workgroups a CU) and 160 x 128 (ten waves of 16 rows) whose rows divide the channels, on at least two rounds over the CUs.
-    // Batch 1024, us, shared tiles before: 256 -> 256 on 14 x 14 1713 -> 1022 (128 x 128: 1115), 512 on 7 x 7 1730 -> 1178 (1191),
-    // 128 on 28 x 28 1693 -> 1133, 448 -> 384 on 8 x 8 1389 -> 906, 288 -> 384 at stride 2 4196 -> 2847 (192 x 128: 3123), 80 -> 192
-    // on 73 x 73 10257 -> 7642, 192 -> 320 at stride 2 521 -> 376 (128 x 128 on 2.5 tiles: 433).  Fewer channels give the
-    // gathered operand too few uses for what taking it apart costs: 64 -> 64 on 56 x 56 1740 against 1709-2330, 96 -> 96 on 35 x 35
-    // 1521 against 1345-1654.
-    static constexpr int SBM = CO % 256 == 0 ? 256 : CO % 128 == 0 ? 128 : CO % 192 == 0 ? 192 : 160;
-    using split = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, SBM, SBM == 192 ? 4 : 8, SBM == 256 ? 8 : SBM == 160 ? 10 : 4, NIMG, kSplitForm>;
+    // Filters larger than 1 x 1: as a product on the bf16 matrix cores whose second operand is gathered from the images (GemmSplit),
+    // on at least two rounds of tiles over the CUs.  The tile is the largest of 256 x 128 (eight waves), 128 x 128, 192 x 64 (four
+    // waves, two workgroups a CU), 160 x 128 (ten waves of 16 rows), 96 x 64 (two waves) and 64 x 128 (four of 16 rows) whose rows
+    // divide the channels.  Batch 1024, us, shared tiles before: 256 -> 256 on 14 x 14 1713 -> 1022 (128 x 128: 1115), 512 on 7 x 7
+    // 1730 -> 1178 (1191), 128 on 28 x 28 1693 -> 1133, 448 -> 384 on 8 x 8 1389 -> 906, 288 -> 384 at stride 2 4196 -> 2847 (192 x
+    // 128: 3123), 80 -> 192 on 73 x 73 10257 -> 7642, 192 -> 320 at stride 2 521 -> 376 (128 x 128 on 2.5 tiles: 433).  Few channels
+    // give the gathered operand few uses for what taking it apart costs: 96 -> 96 on 35 x 35 1521 -> 1237 (96 x 128 on four waves 1253,
+    // on six of 16 rows 1592), 64 -> 96 1057 -> 876, 64 -> 64 on 56 x 56 1740 -> 1620 (64 x 64 1659, 64 rows a wave 1912), 5 x 5 48 -> 64
+    // 1434 -> 1216, 32 -> 64 on 147 x 147 6838 -> 6219, 16 -> 64 at stride 4 1343 -> 932; but at stride 2, where a load of the gather
+    // touches twice the lines and the tile's patch was loaded once, 32 -> 64 on 147 x 147 1864 -> 1891.
+    static constexpr int SBM = CO % 256 == 0 ? 256 : CO % 128 == 0 ? 128 : CO % 192 == 0 ? 192 : CO % 160 == 0 ? 160 : CO % 96 == 0 ? 96 : 64;
+    using split = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, SBM, SBM == 192 || SBM == 96 ? 4 : 8, SBM == 256 ? 8 : SBM == 160 ? 10 : SBM == 96 ? 2 : 4, NIMG, kSplitForm>;
     static constexpr bool is_split()
     {
         // (the table of taps is made at compile time)
-        if constexpr (T > 1 && T < 31 && CI >= 16 && CI * T % 8 == 0 && CI * T <= 32768 && KH >= S && (CO % 128 == 0 || CO % 192 == 0 || CO % 160 == 0))
+        if constexpr (T > 1 && T < 31 && CI % 16 == 0 && CI * T <= 32768 && CO % SBM == 0 && !(SBM == 64 && S == 2))
             return split::FITS && split::TILES >= 512;
         return false;
     }
