@@ -8,7 +8,6 @@
 #include "ops_gemm_f32.h"
 #include "ops_gemm_f32_dma.h"
 #include "ops_gemm_split.h"
-#include "ops_gemm_tile.h"
 
 using namespace bfuse;
 
@@ -30,39 +29,33 @@ DENSE_F32(1024, 4096, 1024, 32, 128, 4)
 DENSE_SPLIT(1024, 4096, 14336, 2, 8, 1, 1, 128)
 DENSE_SPLIT(1024, 14336, 4096, 2, 4, 1, 2, 128)
 
-// C[b] = A[b] . B[b]^T, A [b, M, K], B [b, N, K]: <M, N, K, BM, BN, waves over K>
-// 512 x 64 x 512 and 256 x 80 x 256 run on shared tiles (GemmTile), 128 x 128 in three buffers of 16 k (0.46-0.50 -> 0.38-0.42 ms
-// from card to card, 0.142 -> 0.122).
-#define BGEMM_F32_TILE(B, M, K, N, BM, BN, WM, KS, NBUF)                                                         \
-    using Bgemm_##B##x##M##x##K##x##N = GemmTile<M, K, 1, N, 1, B, BM, BN, WM, KS, kRows, NBUF>;                  \
-    BFUSE_KERNEL(bgemm_f32_##B##x##M##x##K##x##N, Bgemm_##B##x##M##x##K##x##N, ({{B, M, K, 1}, 4}), ({{B, N, K, 1}, 4}), ({{B, M, N, 1}, 4}))
-// The others keep a tile per wave; the one-wave products reserve 32 KB of LDS per workgroup: four workgroups per CU, one
-// wave per SIMD (see LdsReserve).  (208 rows and columns: shared tiles of 128 would overlap by a quarter, 1.00-1.06x; 80
-// columns are no whole 64-column groups.)
+// C[b] = A[b] . B[b]^T, A [b, M, K], B [b, N, K].  Those of 208 rows: <M, N, K, BM, BN, waves over K>, a tile per wave; the one-wave
+// products reserve 32 KB of LDS per workgroup: four workgroups per CU, one wave per SIMD (see LdsReserve).
 #define BGEMM_F32_RESERVE(B, M, K, N, BM, BN, KS, BYTES)                                                         \
     using Bgemm_##B##x##M##x##K##x##N = LdsReserve<GemmF32<M, N, K, BM, BN, KS, kEpiNone, 2, 1, true, B>, BYTES>; \
     BFUSE_KERNEL(bgemm_f32_##B##x##M##x##K##x##N, Bgemm_##B##x##M##x##K##x##N, ({{B, M, K, 1}, 4}), ({{B, N, K, 1}, 4}), ({{B, M, N, 1}, 4}))
-// The bf16 matrix cores (ops_gemm_split.h), us, before (shared tiles; 80 columns a tile per wave) and now: 1024 products 512 x 512 x 128
-// 555 -> 420 on 128 x 128 tiles (256 x 128 of eight waves 408, which leave no room for a partner), 512 x 128 x 512 625 -> 545, 512 x
-// 512 x 64 334 -> 278, 1024 x 512 x 64 607 -> 536, 256 x 256 x 64 95.6 -> 87, 256 x 256 x 80 134 -> 100; with a reduction of 64, whose
-// tiles are mostly ends, 256 x 64 x 256 98 -> 94.5 on 128 x 64 tiles (128 x 128 97), 1024 x 64 x 512 705 -> 676 on 128 x 128 (128 x 64
-// 717).  Not for 512 x 64 x 512 (359-380 against 352-362 on 128 x 64), 256 x 80 x 256 (121 against 122), nor for 208 x 208 x 64 (75.9 against 74); 208 x
-// 64 x 208, x 80 x 208 and x 208 x 80 gain 1.1-1.2x on seven waves but keep the one-wave forms, which any operator can take beside it.
+// The bf16 matrix cores (ops_gemm_split.h): 128 x 64 tiles of 32-row waves for the long reductions, 128 x 128 of eight 16-row waves for
+// those of 64 - 128, which are mostly ends: 70 - 94 registers instead of 126 - 168, so that three workgroups a CU load, multiply and
+// store at different times.  us, fp32 matrix cores before and now: 1024 products 512 x 64 x 512 360 -> 303 (32-row waves 311-348), 512 x
+// 128 x 512 625 -> 465 (499), 256 x 64 x 256 98 -> 84 (94), 256 x 80 x 256 119 -> 107 (117), 1024 x 64 x 512 705 -> 609 (620), 256 x 256 x
+// 80 134 -> 95 (16-row waves; 32-row 99), 512 x 512 x 128 555 -> 419 (32-row, 128 x 128; 16-row 446), 512 x 512 x 64 334 -> 268 (293), 1024 x
+// 512 x 64 607 -> 518 (573), 256 x 256 x 64 95.6 -> 83 (88).  208 x 208 x 64 gains nothing (75.9 against 74); 208 x 64 x 208, x 80 x 208
+// and x 208 x 80 gain 1.1-1.4x on seven or thirteen waves but keep the one-wave forms, which any operator can take beside it.
 #define BGEMM_F32_SPLIT(B, M, K, N, ...)                                                                         \
     using Bgemm_##B##x##M##x##K##x##N = GemmSplit<M, K, 1, N, 1, B, __VA_ARGS__, kRows>;                          \
     BFUSE_KERNEL(bgemm_f32_##B##x##M##x##K##x##N, Bgemm_##B##x##M##x##K##x##N, ({{B, M, K, 1}, 4}), ({{B, N, K, 1}, 4}), ({{B, M, N, 1}, 4}))
-BGEMM_F32_TILE(1024, 512, 64, 512, 128, 128, 2, 16, 3)
+BGEMM_F32_SPLIT(1024, 512, 64, 512, 1, 8, 1, 1, 128)
 BGEMM_F32_SPLIT(1024, 512, 512, 64, 2, 4, 1, 1, 64)
-BGEMM_F32_SPLIT(1024, 512, 128, 512, 2, 4, 1, 1, 128)
+BGEMM_F32_SPLIT(1024, 512, 128, 512, 1, 8, 1, 1, 128)
 BGEMM_F32_SPLIT(1024, 512, 512, 128, 2, 4, 1, 1, 128)
-BGEMM_F32_SPLIT(1024, 256, 64, 256, 2, 4, 1, 1, 64)
+BGEMM_F32_SPLIT(1024, 256, 64, 256, 1, 8, 1, 1, 128)
 BGEMM_F32_SPLIT(1024, 256, 256, 64, 2, 4, 1, 1, 64)
-BGEMM_F32_TILE(1024, 256, 80, 256, 128, 128, 2, 16, 3)
-BGEMM_F32_SPLIT(1024, 256, 256, 80, 2, 4, 1, 1, 80)
+BGEMM_F32_SPLIT(1024, 256, 80, 256, 1, 8, 1, 1, 128)
+BGEMM_F32_SPLIT(1024, 256, 256, 80, 1, 8, 1, 1, 80)
 BGEMM_F32_RESERVE(1024, 208, 64, 208, 112, 64, 1, 32768)
 BGEMM_F32_RESERVE(1024, 208, 208, 64, 208, 32, 1, 32768)
 BGEMM_F32_RESERVE(1024, 208, 80, 208, 112, 64, 1, 32768)     // 208 = 112 + 96 rows, 3 x 64 + 16 columns: the last tiles overlap their neighbours
 BGEMM_F32_RESERVE(1024, 208, 208, 80, 64, 80, 1, 32768)
 // tests/interleave_scheduler/config/info.yaml: bgemm_6, bgemm_7
-BGEMM_F32_SPLIT(1024, 1024, 64, 512, 2, 4, 1, 1, 128)
+BGEMM_F32_SPLIT(1024, 1024, 64, 512, 1, 8, 1, 1, 128)
 BGEMM_F32_SPLIT(1024, 1024, 512, 64, 2, 4, 1, 1, 64)

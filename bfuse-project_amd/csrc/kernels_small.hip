@@ -244,6 +244,11 @@ DENSE_SPLIT_TEST(c, 256, 64, 224, 2, 8, 1, 1, 112)
 DENSE_SPLIT_TEST(d, 64, 4096, 64, 2, 2, 1, 1, 64)
 BGEMM_SPLIT_TEST(e, 8, 64, 72, 80, 1, 2, 2, 1, 64)
 BGEMM_SPLIT_TEST(f, 3, 208, 208, 112, 1, 7, 1, 1, 112)
+DENSE_SPLIT_TEST(m, 64, 256, 144, 2, 2, 1, 1, 144)               // two whole partial sums, and one and a half
+DENSE_SPLIT_TEST(n, 64, 192, 80, 2, 2, 1, 1, 80)
+BGEMM_SPLIT_TEST(o, 2, 64, 192, 64, 1, 4, 4, 1, 64)              // one block of columns a wave, partial sums of two stages and of four
+DENSE_SPLIT_TEST(p, 32, 288, 64, 1, 2, 2, 1, 32)
+BGEMM_SPLIT_TEST(q, 3, 48, 24, 32, 1, 3, 1, 1, 32)               // one stage, and that not whole
 CONV1_SPLIT_TEST(g, 48, 80, 9, 9, 1, 5, 1, 4, 2, 1, 128)
 CONV1_SPLIT_TEST(h, 56, 64, 9, 7, 2, 11, 2, 2, 1, 2, 96)
 BFUSE_BFUSE_KERNEL(selftest_gemm_split_a, GemmSp_a, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)

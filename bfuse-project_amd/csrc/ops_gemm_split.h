@@ -18,13 +18,21 @@
 //     other's waits, and the groups' sums meet in LDS at the end.
 // The operands of an MFMA are given in the order (B, A), so that a lane ends up with four consecutive columns of a row.
 //
-// The five small products are summed apart from the large one (`low`): what rounds the sum is then one addition per 32 k, and
-// 2-norm errors against 64 bits are below those of the fp32 forms: K = 4096 2.7e-7 (KG = 2) and 4.0e-7 (KG = 1) where GemmF32Dma
-// has 5.8e-7, 14336 5.3e-7 for 1.07e-6, 768 1.1e-7 for 2.5e-7.  What three bf16 cannot hold is multiplied again with the fp32 MFMAs
-// (see split.h): a wave whose results are not all finite, and the workgroup if a thread has met nothing but values below 2^-95.
+// What rounds the sum is one addition per partial sum of four stages (`part`; two where there are 9 - 20 of them), of which each
+// stage's MFMAs round only the small beginning: 2-norm errors against 64 bits, with the largest error over the result's root mean
+// square, are below those of the fp32 forms.  Reduction of 14336 2.2e-7, 1.1e-6 (GemmF32Dma 1.1e-6, 6.6e-6), 4096 1.9e-7, 1.5e-6 (5.8e-7,
+// 4.2e-6), 768 1.6e-7, 9.4e-7 (2.5e-7, 1.5e-6), 128 1.5e-7, 2.8e-6 (GemmTile 2.0e-7, 3.2e-6), 64 9.3e-8, 1.5e-6 (1.4e-7, 2.3e-6); 3 x 3
+// filters on 576 1.1e-7, 8.6e-7 (ConvF32Tile 1.4e-7, 1.0e-6; with four stages 1.5e-7, 1.2e-6), on 1152 1.7e-7, 1.1e-6 (1.9e-7, 1.5e-6).
+// (The five small products summed apart from the large one instead, two sets of registers as well, leave one addition per stage:
+// 1.0e-7 but 1.5e-6 on 576, 4.0e-7, 4.6e-6 on 4096; 1-3 % faster on large tiles, where the sums' additions take the place of other
+// vector work.)  What three bf16 cannot hold is multiplied again with the fp32 MFMAs (see split.h): a wave whose results are not
+// all finite, and the workgroup if a thread has met nothing but values below 2^-95.
 //
-// Measured (us, before = GemmF32Dma): 1024 x 4096 x 14336 805 -> 499 (241 TFLOP/s), 1024 x 14336 x 4096 798 -> 530, 1024 x 4096 x
-// 4096 232 -> 156, 512 x 4096 x 14336 461 -> 254, 512 x 4096 x 4096 119 -> 93, 1024 x 768 x 3072 37-41 -> 34.  Smaller tiles than
+// Reductions of up to four stages are one partial sum: no second set of accumulators, every stage compiled apart, and so nothing
+// loaded or taken apart past the last one (with two stages that was half of it): 512 x 128 x 512 545 -> 499 us.
+//
+// Measured (us, before = GemmF32Dma): 1024 x 4096 x 14336 805 -> 516 (233 TFLOP/s), 1024 x 14336 x 4096 798 -> 546, 1024 x 4096 x
+// 4096 232 -> 156, 512 x 4096 x 14336 461 -> 254, 512 x 4096 x 4096 119 -> 94, 1024 x 768 x 3072 37-41 -> 34.  Smaller tiles than
 // 64 x 64 a workgroup take more time than the fp32 forms: 1024 x 3072 x 768 63 (64 x 96 tiles) against 39.
 //
 // B comes in one of two layouts, as in GemmTile: kPix, planes of n for each k ([K, N] is one image of N pixels); kRows, rows
@@ -32,7 +40,7 @@
 // filters as they lie in memory, k counts (channel, tap), and what a column loads for k is its window's element.  All lanes of a
 // load want the same k, so where the element lies from the window's first one comes from a table by a scalar load; padding is a
 // lane whose bit for that tap is set and which therefore reads past the buffer (two vector instructions a load).  Every element
-// is taken apart once for each tap it is under: 256 -> 256 channels on 14 x 14, batch 1024, 1713 -> 1022 us (232 TFLOP/s);
+// is taken apart once for each tap it is under: 256 -> 256 channels on 14 x 14, batch 1024, 1713 -> 1035 us (229 TFLOP/s);
 // ConvTiling has the other layers and where the line to the shared tiles lies.  A row tile (kRows: also a column tile) that does not divide the problem starts
 // a tile before its end and writes the same bits as its neighbour.
 #pragma once
@@ -65,10 +73,15 @@ struct GemmSplit {
     static constexpr int NT = LAYOUT == kRows ? (W + BN - 1) / BN : (int)(((long long)OHWP * NIMG + BN - 1) / BN);
     static constexpr int NIMAGES = LAYOUT == kRows ? 1 : (BN + OHWP - 2) / OHWP + 1;   // images a tile can touch
     static constexpr int NUJ = (4 * BN + GT - 1) / GT;                           // units (a column's eight k) of a thread and stage
+    // a thread's units lie the same way apart for all threads (kRows: GT / 4 columns, kPix: GT / BN octets of one column), so that
+    // one address serves them all
+    static constexpr bool EVEN = 4 * BN % GT == 0 && GT % (LAYOUT == kRows ? 4 : BN) == 0;
+    static constexpr int NUB = EVEN ? 1 : NUJ;
     static_assert(BN % (16 * WN) == 0 && K % 8 == 0 && NS % KG == 0 && M >= BM && (LAYOUT == kPix || (W >= BN && H == 1 && S == 1)), "tile");
     // 31-bit offsets; padding is read through one that lies past the buffer
     static constexpr bool FITS = (long long)BM * K * 4 < (1LL << 31) && (long long)(NIMAGES < NIMG ? NIMAGES : NIMG) * CI * HW * 4 < (1LL << (T == 1 ? 31 : 29));
-    static constexpr int PLANE = 4 * BN * 16, BUF = 3 * PLANE, NBUF = 3;
+    static constexpr int PLANE = 4 * BN * 16, BUF = 3 * PLANE, NBUF = NIT < 3 ? NIT : 3;
+    static constexpr int SUMMED = NIT > 8 && NIT <= 20 ? 2 : 4;                     // stages of a partial sum (error and time: above)
     static constexpr int TILES = MT * NT;
     static constexpr Dims3 GRID{LAYOUT == kRows ? TILES * NIMG : TILES, 1, 1};
     static constexpr Dims3 BLOCK{THREADS, 1, 1};
@@ -162,10 +175,10 @@ struct GemmSplit {
             (void*)(LAYOUT == kRows ? B + (size_t)n0 * K : B + (size_t)n_lo * CI * HW - (P * W + P)), 0,
             LAYOUT == kRows ? BN * K * 4 : ((NIMG - n_lo < NIMAGES ? NIMG - n_lo : NIMAGES) * CI * HW + P * W + P) * 4, 0x00020000);
         const unsigned a_voff = (unsigned)(((wr * TM * 16 + li) * K + 8 * kq) * 4);
-        unsigned b_voff[NUJ], b_out[NUJ];
-        int b_lds[NUJ], b_k[NUJ];
+        unsigned b_voff[NUB], b_out[NUB];
+        int b_lds[NUB], b_k[NUB];
 #pragma unroll
-        for (int j = 0; j < NUJ; ++j) {
+        for (int j = 0; j < NUB; ++j) {
             // threads past the last unit do one of the first ones again: the same values to the same place.  kRows: four lanes
             // read 128 consecutive bytes of a row; kPix: 64 lanes 64 consecutive columns of a plane
             const int u = (j * GT + gt) % (4 * BN), o = LAYOUT == kRows ? u & 3 : u / BN, c = LAYOUT == kRows ? u >> 2 : u % BN;
@@ -175,39 +188,41 @@ struct GemmSplit {
             b_lds[j] = (o * BN + c) * 16;
         }
 
-        f32x4 acc[TM][TN], low[TM][TN];
+        f32x4 acc[TM][TN], part[TM][TN];            // the sum, and apart from it that of the last stages
 #pragma unroll
         for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
-            for (int b = 0; b < TN; ++b) acc[tm][b] = low[tm][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int b = 0; b < TN; ++b) acc[tm][b] = part[tm][b] = f32x4{0.f, 0.f, 0.f, 0.f};
 
         f32x4 ra[TM][2];
         float rb[NUJ][8];
         auto load_a = [&](int tm, int s) {
-            const unsigned v = TAIL != 0 && s == NS - 1 && 8 * kq >= TAIL ? 0x7fffffffu : a_voff + tm * 16 * K * 4;
+            const unsigned v = TAIL != 0 && s == NS - 1 && 8 * kq >= TAIL ? 0x7fffffffu : a_voff;
 #pragma unroll
-            for (int h = 0; h < 2; ++h) ra[tm][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ar, v + h * 16, s * 128, 0));
+            for (int h = 0; h < 2; ++h) ra[tm][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ar, v + (T > 1 ? 0 : h * 16), s * 128 + tm * 16 * K * 4 + (T > 1 ? h * 16 : 0), 0));
         };
+        auto lds_of = [&](int j) { return EVEN ? b_lds[0] + j * (LAYOUT == kRows ? GT / 4 : GT) * 16 : b_lds[j]; };
         auto load_b = [&](int j, int s) {
-            const unsigned v = T == 1 && TAIL != 0 && s == NS - 1 && b_lds[j] >= TAIL / 8 * BN * 16 ? 0x7fffffffu : b_voff[j];
+            const int i = EVEN ? 0 : j;
+            const unsigned v = T == 1 && TAIL != 0 && s == NS - 1 && lds_of(j) >= TAIL / 8 * BN * 16 ? 0x7fffffffu : b_voff[i];
             if constexpr (LAYOUT == kRows) {
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
-                    const f32x4 f = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(br, v + h * 16, s * 128, 0));
+                    const f32x4 f = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(br, v + h * 16, s * 128 + (EVEN ? j * (GT / 4) * K * 4 : 0), 0));
 #pragma unroll
                     for (int e = 0; e < 4; ++e) rb[j][4 * h + e] = f[e];
                 }
             } else if constexpr (T > 1) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    const unsigned at = TAPS.at[s * 32 + b_k[j] + e];
+                    const unsigned at = TAPS.at[s * 32 + b_k[i] + (EVEN ? 8 * j * (GT / BN) : 0) + e];
                     // all ones (past the buffer) if this tap's bit is set; without padding only the last stage has such
-                    const unsigned o = P > 0 || TAIL != 0 ? (unsigned)__builtin_amdgcn_sbfe((int)b_out[j], at, 1) : 0u;
+                    const unsigned o = P > 0 || TAIL != 0 ? (unsigned)__builtin_amdgcn_sbfe((int)b_out[i], at, 1) : 0u;
                     rb[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(br, v | o, (at >> 5) * 4, 0));
                 }
             } else {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) rb[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(br, v, (s * 32 + e) * B_K, 0));
+                for (int e = 0; e < 8; ++e) rb[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(br, v, (s * 32 + (EVEN ? 8 * j * (GT / BN) : 0) + e) * B_K, 0));
             }
         };
         shared_with_asm(sm.t);
@@ -219,12 +234,13 @@ struct GemmSplit {
         // Two of a unit's eight values: units 0 .. NUJ - 1 are this thread's of B, the others its rows of A.
         auto convert = [&](int part, int to, int off) {
             const int u = part / 4, j = part % 4;
+            if (j == 0) asm("" : "+v"(seen[u]));    // one bit pattern at a time: a tree over the stages keeps their parts in registers
             if (u < NUJ) {
                 split2(rb[u][2 * j], rb[u][2 * j + 1], pb[0][j], pb[1][j], pb[2][j]);
                 if (j % 2 == 1) seen[u] |= pb[0][j - 1] | pb[0][j];
                 if (j == 3) {
 #pragma unroll
-                    for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x4*>(base + off + q * PLANE + b_lds[u]) = u32x4{pb[q][0], pb[q][1], pb[q][2], pb[q][3]};
+                    for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x4*>(base + off + q * PLANE + lds_of(u)) = u32x4{pb[q][0], pb[q][1], pb[q][2], pb[q][3]};
                 }
             } else {
                 const int tm = u - NUJ;
@@ -233,11 +249,21 @@ struct GemmSplit {
                 if (j % 2 == 1) seen[u] |= p[0][j - 1] | p[0][j];
             }
         };
-        constexpr int NPART = 4 * (LEAN ? NUJ : NUJ + TM), VPM = (11 * NPART + 6 * TM * TN - 1) / (6 * TM * TN);
+        constexpr int NPART = 4 * (LEAN ? NUJ : NUJ + TM);
+        // A partial sum goes to the result between its last stage's MFMAs and the first ones of the next: every other block of columns,
+        // over the two stages (2 TN blocks) that this leaves, so that the additions too are dealt between MFMAs (1024 x 4096 x 4096 158 us;
+        // all in one stage 164).  Convolutions, whose padding takes registers, add a block right behind its last MFMAs (448 -> 384 channels
+        // is 17 registers short otherwise beside a partner in a thread-fused workgroup; alone 0-1 %), and keep one address of A's rows.
+        constexpr auto fold_at = [](int b) { return TN == 1 ? 0 : b == 0 ? 1 : T > 1 ? b + 1 : 2 * b; };
+        constexpr auto folded = [fold_at](int at) { int n = 0; for (int b = 0; b < TN; ++b) n += at == SUMMED - 1 ? fold_at(b) < TN : at == 0 && fold_at(b) >= TN; return n; };
+        auto fold = [&](int b) {
+#pragma unroll
+            for (int tm = 0; tm < TM; ++tm) acc[tm][b] += part[tm][b];
+        };
         const auto stage_of = [&](int it) { return (it < NIT ? it : NIT - 1) * KG + g; };   // past the end: the last one again
 
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < 2 && i < NIT; ++i) {
 #pragma unroll
             for (int j = 0; j < NUJ; ++j) load_b(j, stage_of(i));
             if (i == 0) {
@@ -247,26 +273,33 @@ struct GemmSplit {
 #pragma unroll
             for (int part = 0; part < 4 * NUJ; ++part) convert(part, 0, i * BUF);
         }
+        if constexpr (NIT > 2)
 #pragma unroll
-        for (int j = 0; j < NUJ; ++j) load_b(j, stage_of(2));
-        auto convert_a = [&](int next) {
+            for (int j = 0; j < NUJ; ++j) load_b(j, stage_of(2));
+        // A of the stage whose loads were the last; then those of stage `next`, if there is one
+        auto convert_a = [&](int next, bool more) {
 #pragma unroll
             for (int part = 4 * NUJ; part < 4 * (NUJ + TM); ++part) convert(part, 0, 0);
+            if (more)
 #pragma unroll
-            for (int tm = 0; tm < TM; ++tm) load_a(tm, stage_of(next));
+                for (int tm = 0; tm < TM; ++tm) load_a(tm, stage_of(next));
         };
-        if constexpr (!LEAN) convert_a(1);
+        if constexpr (!LEAN) convert_a(1, NIT > 1);
         u32x4 fr[2][3];
         auto read = [&](int set, int q, int b, int off) { fr[set][q] = *reinterpret_cast<const u32x4*>(fb + off + q * PLANE + b * 256); };
         sync.raw();
 #pragma unroll
         for (int q = 2; q >= 0; --q) read(0, q, 0, 0);
-        int off = 0, next = BUF, ahead = 2 * BUF;   // LDS offsets of this stage and the two after it
-        auto stage = [&](int it, auto from) {
-            constexpr int FROM = decltype(from)::value;
+        int off = 0, next = NIT > 1 ? BUF : 0, ahead = 2 * BUF;   // LDS offsets of this stage and the two after it
+        // `at`: which one of the SUMMED stages of a partial sum this is.
+        // `left`: how many stages follow, if those are less than three: nothing is loaded, taken apart or read past the last one.
+        auto stage = [&](int it, auto at, auto left) {
+            constexpr int AT = decltype(at)::value, FROM = AT % 2, LEFT = decltype(left)::value;
+            constexpr int FIRST = LEFT >= 2 ? 0 : 4 * NUJ, LAST = LEAN || LEFT >= 1 ? NPART : 4 * NUJ, N = LAST > FIRST ? LAST - FIRST : 0;
+            constexpr int VPM = (11 * N + (NIT > SUMMED ? 4 * TM * folded(AT) : 0) + 6 * TM * TN - 1) / (6 * TM * TN);
             // Behind the barrier the next stage is in LDS whole, and nobody reads the one before this any more.
             if (it > 0) sync.raw();
-            if constexpr (LEAN) convert_a(it + 1);
+            if constexpr (LEAN) convert_a(it + 1, LEFT >= 1);
 #pragma unroll
             for (int b = 0; b < TN; ++b) {
                 const int set = (b + FROM * (TN & 1)) & 1;
@@ -274,21 +307,27 @@ struct GemmSplit {
                 for (int t = 0; t < SplitTerms::N; ++t) {
 #pragma unroll
                     for (int tm = 0; tm < TM; ++tm) {
-                        f32x4& c = t + 1 < SplitTerms::N ? low[tm][b] : acc[tm][b];
                         const unsigned(&p)[4] = pa[LEAN ? 0 : FROM][tm][SplitTerms::A[t]];
-                        c = mfma_bf16(fr[set][SplitTerms::B[t]], u32x4{p[0], p[1], p[2], p[3]}, c);
+                        const f32x4 c = AT == 0 && t == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : part[tm][b];
+                        part[tm][b] = mfma_bf16(fr[set][SplitTerms::B[t]], u32x4{p[0], p[1], p[2], p[3]}, c);
                     }
-                    if (t == 0 || t == 2 || t == 4) read(set ^ 1, 2 - t / 2, b + 1 < TN ? b + 1 : 0, b + 1 < TN ? off : next);
+                    if ((b + 1 < TN || LEFT >= 1) && t % 2 == 0) read(set ^ 1, 2 - t / 2, b + 1 < TN ? b + 1 : 0, b + 1 < TN ? off : next);
                 }
 #pragma unroll
-                for (int part = 0; part < NPART; ++part)
-                    if (part * TN / NPART == b) {
-                        convert(part, LEAN ? 0 : FROM ^ 1, ahead);
-                        if (part % 4 == 3) {
-                            if (part / 4 < NUJ) load_b(part / 4, stage_of(it + 3));
-                            else load_a(part / 4 - NUJ, stage_of(it + 2));
+                for (int i = FIRST; i < FIRST + N; ++i)
+                    if ((i - FIRST) * TN / N == b) {
+                        convert(i, LEAN ? 0 : FROM ^ 1, ahead);
+                        if (i % 4 == 3) {
+                            if (i / 4 < NUJ && LEFT >= 3) load_b(i / 4, stage_of(it + 3));
+                            if (i / 4 >= NUJ && LEFT >= 2) load_a(i / 4 - NUJ, stage_of(it + 2));
                         }
                     }
+                if (NIT > SUMMED && (AT == 0 || AT == SUMMED - 1)) {
+                    const int when = AT == 0 ? TN + b : b;
+#pragma unroll
+                    for (int c = 0; c < TN; ++c)
+                        if (when == fold_at(c)) fold(c);
+                }
 #pragma unroll
                 for (int t = 0; t < SplitTerms::N; ++t) {
 #pragma unroll
@@ -296,7 +335,7 @@ struct GemmSplit {
                         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);     // an MFMA
                         __builtin_amdgcn_sched_group_barrier(0x002, VPM, 0);   // vector instructions
                     }
-                    if (t == 0 || t == 2 || t == 4) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // an LDS read
+                    if ((b + 1 < TN || LEFT >= 1) && t % 2 == 0) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // an LDS read
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -304,26 +343,35 @@ struct GemmSplit {
             off = next;
             next = ahead;
             ahead = o;
+            asm("" : "+s"(off), "+s"(next), "+s"(ahead));   // addresses are worked out anew: kept ones cost registers
         };
+        // N stages, the last of all if END
+        auto stages = [&](int it, auto n, auto end) {
+            constexpr int N = decltype(n)::value, END = decltype(end)::value ? 0 : 3;
+            if constexpr (N > 0) stage(it, std::integral_constant<int, 0>{}, std::integral_constant<int, END + N - 1>{});
+            if constexpr (N > 1) stage(it + 1, std::integral_constant<int, 1>{}, std::integral_constant<int, END + N - 2>{});
+            if constexpr (N > 2) stage(it + 2, std::integral_constant<int, 2>{}, std::integral_constant<int, END + N - 3>{});
+            if constexpr (N > 3) stage(it + 3, std::integral_constant<int, 3>{}, std::integral_constant<int, END + N - 4>{});
+        };
+        // the last ones apart; of large tiles only those that the loop leaves, the compiler runs out of registers otherwise
+        constexpr int REST = TM * TN <= 8 || NIT <= SUMMED ? (NIT - 1) % SUMMED + 1 : NIT % SUMMED;
 #pragma unroll 1
-        for (int it = 0; it + 1 < NIT; it += 2) {
-            stage(it, std::integral_constant<int, 0>{});
-            stage(it + 1, std::integral_constant<int, 1>{});
-        }
-        if constexpr (NIT % 2 == 1) stage(NIT - 1, std::integral_constant<int, 0>{});
+        for (int it = 0; it + SUMMED <= NIT - REST; it += SUMMED) stages(it, std::integral_constant<int, SUMMED>{}, std::false_type{});
+        stages(NIT - REST, std::integral_constant<int, REST>{}, std::true_type{});
+#pragma unroll
+        for (int b = 0; b < TN; ++b)
+            if (NIT <= SUMMED || NIT % SUMMED != 0 || fold_at(b) >= TN) fold(b);
 
+        // (the lane worked out again: three registers less in the loop)
+        const int el = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), ei = el & 15, eq = el >> 4;
         bool tiny = false;
 #pragma unroll
         for (int u = 0; u < NUJ + TM; ++u) tiny |= split_tiny(seen[u]);
         if (tiny) sm.inexact = 1;
-#pragma unroll
-        for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-            for (int b = 0; b < TN; ++b) acc[tm][b] += low[tm][b];
         sync.raw();
         bool again = sm.inexact != 0;
         if constexpr (KG > 1) {
-            f32x4* const red = reinterpret_cast<f32x4*>(sm.t) + w * TM * TN * 64 + lane;
+            f32x4* const red = reinterpret_cast<f32x4*>(sm.t) + w * TM * TN * 64 + el;
             if (g > 0) {
 #pragma unroll
                 for (int tm = 0; tm < TM; ++tm)
@@ -351,14 +399,14 @@ struct GemmSplit {
 #pragma unroll
             for (int b = 0; b < TN; ++b) {
                 unsigned outside;
-                const unsigned c = column((wn * TN + b) * 16 + li, outside), v = T > 1 || c == 0x7fffffffu ? c : c + kq * B_K;
+                const unsigned c = column((wn * TN + b) * 16 + ei, outside), v = T > 1 || c == 0x7fffffffu ? c : c + eq * B_K;
 #pragma unroll
                 for (int tm = 0; tm < TM; ++tm) acc[tm][b] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
                 for (int k = 0; k < K; k += 4) {
                     unsigned at = k * B_K, o = v;
                     if constexpr (T > 1) {
-                        at = TAPS.at[k + kq];
+                        at = TAPS.at[k + eq];
                         o |= (unsigned)__builtin_amdgcn_sbfe((int)outside, at, 1);
                         if (o != ~0u) o += (at >> 5) * 4;
                         at = 0;
@@ -366,7 +414,7 @@ struct GemmSplit {
                     const float bv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(br, o, at, 0));
 #pragma unroll
                     for (int tm = 0; tm < TM; ++tm) {
-                        const float av = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ar, (((wr * TM + tm) * 16 + li) * K + kq) * 4, k * 4, 0));
+                        const float av = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ar, (((wr * TM + tm) * 16 + ei) * K + eq) * 4, k * 4, 0));
                         acc[tm][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv, av, acc[tm][b], 0, 0, 0);
                     }
                 }
@@ -375,14 +423,14 @@ struct GemmSplit {
         // lane (i, q): row i of a 16-row block, columns 4q .. 4q + 3 of each 16-column block
 #pragma unroll
         for (int b = 0; b < TN; ++b) {
-            const int col = (wn * TN + b) * 16 + 4 * kq;
+            const int col = (wn * TN + b) * 16 + 4 * eq;
             if constexpr (LAYOUT == kRows) {
 #pragma unroll
-                for (int tm = 0; tm < TM; ++tm) *reinterpret_cast<f32x4*>(C + (size_t)(m0 + (wr * TM + tm) * 16 + li) * W + n0 + col) = acc[tm][b];
+                for (int tm = 0; tm < TM; ++tm) *reinterpret_cast<f32x4*>(C + (size_t)(m0 + (wr * TM + tm) * 16 + ei) * W + n0 + col) = acc[tm][b];
             } else {
                 const int vc = v0 + col, img = n_lo + vc / OHWP, p = vc % OHWP;
                 if (img < NIMG) {
-                    float* __restrict__ y = C + ((size_t)img * M + m0 + wr * TM * 16 + li) * OHW + p;
+                    float* __restrict__ y = C + ((size_t)img * M + m0 + wr * TM * 16 + ei) * OHW + p;
                     const bool whole = OHW % 4 == 0 || p + 4 <= OHW;
 #pragma unroll
                     for (int tm = 0; tm < TM; ++tm) {

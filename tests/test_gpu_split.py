@@ -20,7 +20,8 @@ def _product(a, b):
 
 @pytest.mark.parametrize("tag,partner,kind,suffix", [
     ("a", "layernorm_8x256", "bfuse", "_c4"), ("b", "bias_relu_4096", None, ""), ("c", "bias_relu_4096", None, ""), ("d", "bias_relu_4096", None, ""),
-    ("e", "bias_relu_4096", "hfuse", ""), ("f", "conv3x3_f32_32x12x12_32", "hfuse", "")])
+    ("e", "bias_relu_4096", "hfuse", ""), ("f", "conv3x3_f32_32x12x12_32", "hfuse", ""), ("m", "bias_relu_4096", None, ""), ("n", "bias_relu_4096", None, ""),
+    ("o", "bias_relu_4096", None, ""), ("p", "bias_relu_4096", None, ""), ("q", "bias_relu_4096", None, "")])
 def test_split_product_against_numpy_and_fused(tag, partner, kind, suffix):
     _check(f"selftest_gemm_split_{tag}", lambda a, b: _product(a, b).astype(np.float32), partner, kind, suffix)
 
@@ -78,11 +79,22 @@ def _operands(name):
     return [fill_normal(11 + i, int(np.prod(k.shapes[i])), 0, 1).reshape(k.shapes[i]) for i in (0, 1)]
 
 
-@pytest.mark.parametrize("tag,steps,groups", [("_d", 4096 // 32, 1), ("_b", 256 // 32, 2), ("k_b", 6 * 192 // 32, 2), ("k_c", 6 * 128 // 32, 4)])
+@pytest.mark.parametrize("tag,steps,groups", [("_d", 4096 // 32, 1), ("_m", 256 // 32, 1), ("_b", 256 // 32, 2)])
 def test_split_product_is_closer_to_64_bits_than_one_fp32_sum(tag, steps, groups):
-    """One rounding of at most u = 2^-24 of what the sum has grown to for every 32 k: u sqrt(steps / 2) (2-norm), in two groups
-    sqrt(2) less and u for adding them; the products that are left out and the sum of the small ones add less than u / 2.  Split
-    over K (no sum of their own for the small ones) it is rounded six times for 32 k."""
+    """A sum rounded r times on its way is off by at most u = 2^-24 of what it has grown to each time, u sqrt(r / 2) (2-norm).  A group
+    adds a partial sum every four steps of 32 k, r = steps / 4; those are rounded six times a step on sums of half of four steps,
+    24 steps / groups times 2 / (steps / groups) of the whole: 12 u^2 more.  The products left out add less than u / 2, adding
+    the groups u."""
+    name = f"selftest_gemm_split{tag}"
+    x, w = _operands(name)
+    want = _product(x, w)
+    err = np.linalg.norm(_run(name, x, w).reshape(want.shape) - want) / np.linalg.norm(want)
+    assert err <= 2.0 ** -24 * ((steps / groups / 8 + 12) ** 0.5 + 0.5 + (groups > 1))
+
+
+@pytest.mark.parametrize("tag,steps,groups", [("k_b", 6 * 192 // 32, 2), ("k_c", 6 * 128 // 32, 4)])
+def test_split_k_product_is_closer_to_64_bits_than_one_fp32_sum(tag, steps, groups):
+    """One sum a wave, rounded six times for 32 k, `groups` of which are added."""
     name = f"selftest_gemm_split{tag}"
     x, w = _operands(name)
     want = _product(x, w)
