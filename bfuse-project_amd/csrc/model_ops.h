@@ -41,21 +41,20 @@ using Dense6 = GemmBf16NTDma<512, 14336, 4096, 128, 224, 3, 4, 4, 2, 2, 11>;
 // Batched GEMMs of the attention layers (the reference's bgemm, scripts/configure_kernels.py:14-19,40-48:
 // C[b] = A[b] . B[b]^T with A [b, M, K] and B [b, N, K]): bgemm_0 / bgemm_1 are BERT's and GPT-2's scores and
 // context products (12 heads, sequence 512, head size 64), bgemm_2 / bgemm_3 Llama-3-8B's (32 heads, head size 128).
-// bgemm_0 runs on tiles of 64 rows shared by four waves (GemmTile): a wave per tile (64 x 64, operands straight into registers) had
-// one wave per SIMD at best to cover its loads, 8.1 us instead of 7.3 (128 x 64 tiles 8.3, 128 x 128 8.8), fused with the causal
-// softmax 13.8 instead of 10.2.  bgemm_1 has 8 row tiles a product, too few of 64 rows (12.2 us): operands go global -> VGPR in MFMA
-// layout, two waves split K.  (32 x 64 two-wave 9.7 us, 16 x 64 two-wave 11.3, four-wave 11.3, 16 x 32 10.1)
-// bgemm_2 and bgemm_3 run on the bf16 matrix cores (GemmSplit), on 128 x 64 tiles of four waves in as many registers as the twelve
-// waves a CU of a fused kernel with the bf16 gate projection leave.  us, GemmTile before, alone and fused with the 512 x 768 x 2304,
-// the bf16 4096 x 4096 and the bf16 4096 x 14336 layers:
-//   bgemm_2  21.5, 33.2, 45.4, 69.8 -> 19.0, 31.3, 43.3, 67.6; 128 x 128 tiles 18.6, 29.7, 39.0, but 250 registers
-//   bgemm_3  20.1, 33.0, 42.5, 67.3 -> 18.1, 28.1, 35.7, 61.3; not lean 16.8, 27.8, 34.8, but 174 registers; 64 x 64 18.6, 30.0, 40.8
-// bgemm_0 likewise gains alone (6.7) and loses fused (20.1 against 18.8, 27.9 against 27.2); bgemm_1 on 64 x 32 tiles gains (8.8
-// against 9.5; fused 19.4 against 21.5, 27.0 against 27.8), but beside the bf16 product's hand-counted reads the compiler then moves
-// registers in a way that the build's check refuses.
-using Bgemm0 = GemmTile<512, 64, 1, 512, 1, 12, 64, 64, 4, 32, kRows, 2>;     // 8 x 8 tiles x 12 = 768 workgroups
+// bgemm_1 has 8 row tiles a product, too few of 64 rows (12.2 us): operands go global -> VGPR in MFMA layout, two waves split K.
+// (32 x 64 two-wave 9.7 us, 16 x 64 two-wave 11.3, four-wave 11.3, 16 x 32 10.1.)  Split into bf16 (GemmSplit, 64 x 32 tiles) it takes
+// 8.0, but beside the bf16 product's hand-counted reads the compiler then moves registers in a way that the build's check refuses.
+// The others run on the bf16 matrix cores (GemmSplit).  us alone and fused with the fp32 768 x 768, 768 x 3072 and 768 x 2304 and the bf16
+// 4096 x 4096 and 4096 x 14336 layers, fp32 matrix cores (GemmTile) before:
+//   bgemm_0  6.8, 12.4, 25.3, 21.1, 27.4, 52.6 -> 6.2, 11.8, 23.7, 19.8, 27.6, 52.8, with the causal softmax 9.6 -> 8.5; 64 x 64 tiles of four
+//            16-row waves (lean 6.05, 11.6, 23.3, 19.4, but 27.6 and 53.3; 128 x 64 of 32-row waves 7.4)
+//   bgemm_2  21.4, 29.2, 42.4, 36.9, 46.1, 73.2 -> 17.4, 22.2, 39.6, 32.6, 37.7, 63.6; 128 x 128 tiles of eight 16-row waves (128 x 64 of four
+//            32-row waves 18.2, 24.1, 36.3, 29.7, 40.2, 65.1)
+//   bgemm_3  20.1 alone, 33.0, 42.5, 67.3 with the last three -> 18.1, 28.1, 35.7, 61.3; 128 x 64 tiles of four 32-row waves, lean: the twelve waves a CU of
+//            a fused kernel with the bf16 gate projection leave 168 registers (not lean 174)
+using Bgemm0 = GemmSplit<512, 64, 1, 512, 1, 12, 1, 4, 1, 1, 64, kRows, 1, 1, 0, false>;      // 8 x 8 tiles x 12 = 768 workgroups
 using Bgemm1 = GemmF32<512, 64, 512, 32, 64, 2, kEpiNone, 2, 1, true, 12>;     // 16 x 1 tiles x 12 = 192 two-wave workgroups
-using Bgemm2 = GemmSplit<512, 128, 1, 512, 1, 32, 2, 4, 1, 1, 64, kRows>;                     // 4 x 8 tiles x 32 = 1024
+using Bgemm2 = GemmSplit<512, 128, 1, 512, 1, 32, 1, 8, 1, 1, 128, kRows>;                    // 4 x 4 tiles x 32 = 512
 using Bgemm3 = GemmSplit<512, 512, 1, 128, 1, 32, 2, 4, 1, 1, 64, kRows, 1, 1, 0, true>;      // 4 x 2 tiles x 32 = 256
 
 // conv2d_1: the convolution of pair 3;  conv2d_4: 128 -> 128 channels on 28 x 28, 32 output channels x 16 pixels
