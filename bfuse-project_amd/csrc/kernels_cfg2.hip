@@ -10,7 +10,7 @@ using namespace bfuse;
 BFUSE_MODULE_PROLOGUE()
 
 // 32x144 tiles: 16 x 16 = 256 workgroups, exactly one per CU; four waves split K = 768;
-// operands staged through per-wave LDS rings by direct-to-LDS loads
+// operands go to registers and are taken apart for the bf16 matrix cores there (GemmSplitK)
 using GemmQkv = GemmF32Dma<512, 2304, 768, 32, 144, 4>;
 // one row per one-wave workgroup (512 workgroups): the finest cut hides best behind the GEMM
 using LnBert = LayerNorm<512, 768, 1, 1>;

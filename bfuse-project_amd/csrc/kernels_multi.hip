@@ -41,10 +41,9 @@ BFUSE_HFUSE3_KERNEL(conv3x3_f32_32x12x12_32, ConvS2, gemm_gelu_f32_96x128x192, G
 BFUSE_HFUSE4_KERNEL(conv3x3_f32_32x12x12_32, ConvS2, gemm_f32_128x160x192_d, GemmS5, layernorm_8x256, LayerNormS, bias_relu_4096, BiasReluS)
 
 // Full size: QKV projection 512x768x2304 (256 tiles, MFMA-bound), LayerNorm 512x768 and causal
-// softmax 12x512x512 (memory-bound), the kernels of pairs 2 and 4.  The GEMM runs here with a ring
-// of two stages: every workgroup of a block-fused kernel is charged the largest side's LDS, and
-// with 48 KB instead of 72 three workgroups fit a CU instead of two -- the GEMM alone is as fast
-// (16.0 us either way), the fused kernel 19.0 instead of 20.6 us.
+// softmax 12x512x512 (memory-bound), the kernels of pairs 2 and 4.  The GEMM's partial sums
+// meet here in two rounds: every workgroup of a block-fused kernel is charged the largest side's LDS, 37 KB
+// instead of 72.  The GEMM alone takes 15.4 us (14.4 in one round), the fused kernel 16.6-17.2 (on the fp32 ring 19.0).
 using GemmQkvS2 = GemmF32Dma<512, 2304, 768, 32, 144, 4, kEpiNone, 2>;
 using LnBert = LayerNorm<512, 768, 1, 1>;
 using Softmax4 = SoftmaxCausal<12, 512, 4, 1>;

@@ -56,8 +56,8 @@ using GemmS3 = GemmF32<32, 144, 256, 32, 144, 4>;                     // the 64+
 using GemmS7 = GemmF32<80, 112, 32, 32, 64, 1>;                        // tiles that do not divide the problem: rows 0, 32, 48 and columns 0, 48 (the last tiles overlap their neighbours)
 using GemmS8 = GemmF32<48, 80, 64, 32, 64, 2, kEpiNone, 2, 1, true, 3>;   // the same on three batched products with B [N, K] and two waves over K
 using GemmS9 = GemmF32<256, 64, 32, 128, 64, 1>;                       // 128 x 64 tiles: 32 accumulator blocks, a kernel of one wave per SIMD (MIN_WAVES_PER_EU), also when fused
-using GemmS5 = GemmF32Dma<128, 192, 160, 32, 96, 2>;                  // private LDS rings, two waves split K, ten 8-k stages each
-using GemmS6 = GemmF32Dma<64, 288, 192, 32, 144, 4, kEpiGeluTanh>;    // the 32x144 tile (partial last B load), four waves, GELU
+using GemmS5 = GemmF32Dma<128, 192, 160, 32, 96, 2>;                  // private LDS rings (GemmF32Ring), two waves split K, ten 8-k stages each
+using GemmS6 = GemmF32Dma<64, 288, 192, 32, 144, 4, kEpiGeluTanh>;    // the 32x144 tile on the ring (48 k a wave is no whole stage of GemmSplitK; partial last B load), four waves, GELU
 using BiasReluS = BiasRelu<4096, 64, 4>;
 using LayerNormS = LayerNorm<8, 256, 2, 1>;
 using SoftmaxS = SoftmaxCausal<2, 256, 2, 2, 2>;

@@ -436,12 +436,13 @@ struct ConvTiling {
     // Filters larger than 1 x 1: as a product on the bf16 matrix cores whose second operand is gathered from the images (GemmSplit),
     // on at least two rounds of tiles over the CUs.  The tile is the largest of 256 x 128 (eight waves), 128 x 128, 192 x 64 (four
     // waves, two workgroups a CU), 160 x 128 (ten waves of 16 rows), 96 x 64 (two waves) and 64 x 128 (four of 16 rows) whose rows
-    // divide the channels.  Batch 1024, us, shared tiles before: 256 -> 256 on 14 x 14 1713 -> 1022 (128 x 128: 1115), 512 on 7 x 7
-    // 1730 -> 1178 (1191), 128 on 28 x 28 1693 -> 1133, 448 -> 384 on 8 x 8 1389 -> 906, 288 -> 384 at stride 2 4196 -> 2847 (192 x
-    // 128: 3123), 80 -> 192 on 73 x 73 10257 -> 7642, 192 -> 320 at stride 2 521 -> 376 (128 x 128 on 2.5 tiles: 433).  Few channels
-    // give the gathered operand few uses for what taking it apart costs: 96 -> 96 on 35 x 35 1521 -> 1237 (96 x 128 on four waves 1253,
-    // on six of 16 rows 1592), 64 -> 96 1057 -> 876, 64 -> 64 on 56 x 56 1740 -> 1620 (64 x 64 1659, 64 rows a wave 1912), 5 x 5 48 -> 64
-    // 1434 -> 1216, 32 -> 64 on 147 x 147 6838 -> 6219, 16 -> 64 at stride 4 1343 -> 932; but at stride 2, where a load of the gather
+    // divide the channels.  Batch 1024, us, shared tiles before: 256 -> 256 on 14 x 14 1712 -> 1033 (128 x 128: 1.09x that), 512 on 7 x 7
+    // 1720 -> 1136, 128 on 28 x 28 1692 -> 1122, 448 -> 384 on 8 x 8 1381 -> 882 (192 x 64: 1.08x), 288 -> 384 at stride 2 4153 -> 2838
+    // (192 x 128 and x 64: 1.10x), 80 -> 192 on 73 x 73 10209 -> 7393, 192 -> 320 at stride 2 521 -> 378 (128 x 128 on 2.5 tiles: 433; five
+    // waves of 32 rows twice 477).  Few channels
+    // give the gathered operand few uses for what taking it apart costs: 96 -> 96 on 35 x 35 1506 -> 1169 (96 x 128 on four waves 1.01x,
+    // on six of 16 rows 1.3x), 64 -> 96 1056 -> 852, 64 -> 64 on 56 x 56 1740 -> 1504 (64 x 64 1.02x, 64 rows a wave 1.2x), 5 x 5 48 -> 64
+    // 1432 -> 1161, 32 -> 64 on 147 x 147 6802 -> 5938, 16 -> 64 at stride 4 1338 -> 865; but at stride 2, where a load of the gather
     // touches twice the lines and the tile's patch was loaded once, 32 -> 64 on 147 x 147 1864 -> 1891.
     static constexpr int SBM = CO % 256 == 0 ? 256 : CO % 128 == 0 ? 128 : CO % 192 == 0 ? 192 : CO % 160 == 0 ? 160 : CO % 96 == 0 ? 96 : 64;
     using split = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, SBM, SBM == 192 || SBM == 96 ? 4 : 8, SBM == 256 ? 8 : SBM == 160 ? 10 : SBM == 96 ? 2 : 4, NIMG, kSplitForm>;
@@ -453,9 +454,10 @@ struct ConvTiling {
         return false;
     }
     // 1 x 1 filters on 256 and more channels likewise, also on 224 x 128 tiles (seven waves).  us, GemmTile before: 768 -> 192 on
-    // 17 x 17 690 -> 534 (twelve waves of 16 rows 514, but no register is left beside twelve waves), 160 594 -> 464, 128 490 -> 344,
-    // 1280 -> 448 on 8 x 8 545 -> 374, 384 460 -> 311, 320 394 -> 293, 192 237 -> 179, 2048 -> 448 831 -> 584, 256 -> 256 on 56 x 56
-    // 3168 -> 2513, 256 -> 512 at stride 2 146 -> 121.  On fewer channels the tile's ends are too much of it: 128 -> 256 at stride 2
+    // 17 x 17 641 -> 525 (twelve waves of 16 rows 0.96x that, but no register is left beside twelve waves), 160 573 -> 447, 128 455 -> 344,
+    // 1280 -> 448 on 8 x 8 521 -> 378, 384 450 -> 314, 320 377 -> 292, 192 233 -> 179, 2048 -> 448 824 -> 582, 256 -> 256 on 56 x 56
+    // 3034 -> 2502, 256 -> 512 at stride 2 145 -> 121.  (160 rows are ten waves on four SIMDs, bound by their LDS reads: 155 TFLOP/s where 256 x
+    // 128 tiles have 207; five waves of 32 rows, 64 or 160 pixels, and lean ones are slower.)  On fewer channels the tile's ends are too much of it: 128 -> 256 at stride 2
     // 152 against 177, 64 -> 128 202 against 218; 64 output channels 394 against 383-410.
     static constexpr int S1BM = CO % 256 == 0 ? 256 : CO % 128 == 0 ? 128 : CO % 224 == 0 ? 224 : CO % 192 == 0 ? 192 : 160;
     static constexpr int S1WR = S1BM == 256 ? 8 : S1BM == 224 ? 7 : S1BM == 160 ? 10 : 4;

@@ -4,7 +4,8 @@
 // What bounded the per-wave form there: every wave staged a patch of its own through registers (address arithmetic,
 // predicated scattered LDS writes) for 16 - 64 output channels, so the same image patch was staged CO / BM times, and
 // tiles of 64 pixels per image leave a quarter of the lanes idle on 14 x 14 and 17 x 17 images.  37 - 110 TFLOP/s of
-// the 154 the matrix cores sustain.  Here
+// the 154 the matrix cores sustain.  (Most layers of a batch have since gone on to the bf16 matrix cores, GemmSplit; ConvTiling says which
+// stay: few workgroups, 64 output channels at stride 2, channel counts that its tiles do not divide.)  Here
 //   * one workgroup of four waves owns BM output channels x BP consecutive pixels OF THE BATCH (a tile runs on into
 //     the next image: no ragged tiles but the batch's last), each wave a (BM / WM) x (BP / WN) part of it;
 //   * both operands of four input channels (a stage) are shared by the four waves: the filter rows, which are

@@ -1,10 +1,10 @@
 // fp32 GEMM side, split-K with private LDS staging:  C[M,N] = A[M,K] . B[K,N] (+ optional
-// tanh-GELU).  Same arithmetic and the same decomposition as GemmF32 -- one workgroup per
+// tanh-GELU).  GemmF32Dma (at the end) is this form, GemmF32Ring, or for larger tiles GemmSplitK on the bf16 matrix cores.  Same arithmetic and the same decomposition as GemmF32 -- one workgroup per
 // BM x BN tile, its KS waves split K and each accumulates the whole tile over its own k-range,
 // partial tiles summed through LDS in wave order -- but the operands take another road:
 //
 //   GemmF32     global -> VGPR (global_load_dwordx4 in MFMA layout)
-//   GemmF32Dma  global -> LDS  (global_load_lds_dwordx4 into a ring PRIVATE to the wave)
+//   GemmF32Ring global -> LDS  (global_load_lds_dwordx4 into a ring PRIVATE to the wave)
 //                      -> VGPR (ds_read_b128 / b64 in MFMA layout)
 //
 // What the road buys is an inner loop made of MFMAs and almost nothing else.  Measured on

@@ -8,8 +8,10 @@
 // TFLOP/s, or 2 - 3.2 TB/s where the bytes count, of 154 and 4.7.  Here a workgroup stages BM rows of A and BN columns
 // of B for KS steps of k in LDS, memory -> LDS directly, in NBUF buffers (loads NBUF - 1 stages ahead) with one barrier
 // per stage: nothing but LDS reads and MFMAs in the loop, and two or more workgroups share a CU.  126 - 142 TFLOP/s where
-// the matrix cores bound it, 3.8 - 5.1 TB/s where memory does.  (A single dense product is better off on GemmF32Dma, 150
-// TFLOP/s against 131-143 here: with one or two tiles per CU there is no second workgroup to hide a stage's barrier.)
+// the matrix cores bound it, 3.8 - 5.1 TB/s where memory does.  Since GemmSplit took the
+// long reductions over (bf16 matrix cores, 160 - 240 TFLOP/s) it keeps products of few channels: 1 x 1 layers of fewer than 256, which
+// memory bounds or whose tiles are mostly ends, and the 16-head scores at batch 1.  (A single dense product is better off on
+// GemmF32Ring, 150 TFLOP/s against 131-143 here: with one or two tiles per CU no second workgroup hides a stage's barrier.)
 //
 // A rows are contiguous along k: [BM][KS] in LDS, 16-byte chunk c of row r at c ^ f(r) so that the 16 rows of a
 // fragment read spread over the banks.  Lane (i, q) reads A[i][16g + 4q .. +3] with one 128-bit read: element t is
