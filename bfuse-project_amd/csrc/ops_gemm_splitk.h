@@ -19,8 +19,8 @@
 // One sum over a wave's stages, rounded six times for every 32 k where the fp32 form rounds eight times: 2-norm errors against 64
 // bits 2.0e-7 (K = 768) and 4.9e-7 (4096) where that one has 2.5e-7 and 5.8e-7.
 //
-// What three bf16 cannot hold (split.h): a wave whose sums are not all finite, or that has met a row or column of nothing but
-// tiny values, hands over NaN.  Finite sums add up to NaN never, so all waves then see NaN in what they finish, and all multiply
+// What three bf16 cannot hold (split.h): a wave whose sums are not all finite, or that has met a value that is more than its
+// parts, hands over NaN.  Finite sums add up to NaN never, so all waves then see NaN in what they finish, and all multiply
 // their k-range again with the fp32 instructions.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -93,12 +93,13 @@ struct GemmSplitK {
             }
         };
         unsigned pa[TM][3][4], pb[2][3][4];
-        unsigned seen[TM + NB] = {};
+        unsigned left = 0;                                  // see split.h
         auto convert_a = [&](int tm) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) split2(ra[tm][j / 2][2 * (j % 2)], ra[tm][j / 2][2 * (j % 2) + 1], pa[tm][0][j], pa[tm][1][j], pa[tm][2][j]);
-            seen[tm] |= pa[tm][0][0] | pa[tm][0][1];
-            seen[tm] |= pa[tm][0][2] | pa[tm][0][3];
+            for (int j = 0; j < 4; ++j) {
+                split2(ra[tm][j / 2][2 * (j % 2)], ra[tm][j / 2][2 * (j % 2) + 1], pa[tm][0][j], pa[tm][1][j], pa[tm][2][j], left);
+                gather_left(left);
+            }
         };
         auto convert_b = [&](int b) {
             unsigned(&p)[3][4] = pb[b & 1];
@@ -106,10 +107,9 @@ struct GemmSplitK {
             for (int j = 0; j < 4; ++j) {
                 const float lo = b < 4 * G4 ? rb[b / 4 < G4 ? b / 4 : 0][2 * j][b % 4] : rt[b < 4 * G4 ? 0 : b - 4 * G4][2 * j];
                 const float hi = b < 4 * G4 ? rb[b / 4 < G4 ? b / 4 : 0][2 * j + 1][b % 4] : rt[b < 4 * G4 ? 0 : b - 4 * G4][2 * j + 1];
-                split2(lo, hi, p[0][j], p[1][j], p[2][j]);
+                split2(lo, hi, p[0][j], p[1][j], p[2][j], left);
+                gather_left(left);
             }
-            seen[TM + b] |= p[0][0] | p[0][1];
-            seen[TM + b] |= p[0][2] | p[0][3];
         };
         const auto group_of = [](int b) constexpr { return b < 4 * G4 ? b / 4 : G4 + b - 4 * G4; };
 
@@ -150,9 +150,6 @@ struct GemmSplitK {
             }
         }
 
-        bool tiny = false;
-#pragma unroll
-        for (int u = 0; u < TM + NB; ++u) tiny |= split_tiny(seen[u]);
         float zero = 0.f;                                   // or NaN
 #pragma unroll
         for (int tm = 0; tm < TM; ++tm)
@@ -160,7 +157,7 @@ struct GemmSplitK {
             for (int b = 0; b < NB; ++b)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) zero = __builtin_fmaf(acc[tm][b][v], 0.f, zero);
-        const float poison = __builtin_amdgcn_ballot_w64(tiny || zero != 0.f) != 0 ? __builtin_nanf("") : 0.f;
+        const float poison = __builtin_amdgcn_ballot_w64(split_inexact(left) || zero != 0.f) != 0 ? __builtin_nanf("") : 0.f;
 
         // component v of row block tm (row 4 rg + v of it) is unit 4 tm + v, finished by wave unit % KS
         unsigned char* const part = sm.t + lane * 16;

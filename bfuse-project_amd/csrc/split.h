@@ -9,9 +9,8 @@
 //   * infinities and NaN, and finite values whose nearest bf16 is infinite (2^128 - 2^119 and up): x - p0 is then infinite or NaN,
 //     and so is every result that x has a part in.  A kernel looks at its results and multiplies those that are not finite again
 //     with the fp32 instructions, so that what comes out is what fp32 arithmetic gives;
-//   * bits below 2^-133, bf16's smallest: those of values below 2^-109.  Beside a value of 2^-95 or more in the same row (column)
-//     they are 2^-38 of it.  A kernel ors the leading parts of what each thread takes apart; where some are not zero and all lie
-//     below 2^-95 (the three leading bits of every exponent zero) it does the tile again likewise.
+//   * bits below 2^-133, bf16's smallest: those of values below 2^-109.  What is left for p2 then has bits in its lower half,
+//     which is dropped.  A kernel ors all that was left for p2; if a lower half is not zero, it does the tile again likewise.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -32,14 +31,23 @@ __device__ __forceinline__ void shared_with_asm(const void* lds)
 #endif
 }
 
-// Two fp32 as three words of two bf16 each (lo in the low halves).
-__device__ __forceinline__ void split2(float lo, float hi, unsigned& p0, unsigned& p1, unsigned& p2)
+// Two fp32 as three words of two bf16 each (lo in the low halves).  `left` gets the bits of what is left for the last one.
+__device__ __forceinline__ void split2(float lo, float hi, unsigned& p0, unsigned& p1, unsigned& p2, unsigned& left)
 {
     p0 = pack_bf16(lo, hi);
     const float l1 = lo - __builtin_bit_cast(float, p0 << 16), h1 = hi - __builtin_bit_cast(float, p0 & 0xffff0000u);
     p1 = pack_bf16(l1, h1);
-    const float l2 = l1 - __builtin_bit_cast(float, p1 << 16), h2 = h1 - __builtin_bit_cast(float, p1 & 0xffff0000u);
-    p2 = __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, h2), __builtin_bit_cast(unsigned, l2), 0x07060302u);   // their upper halves
+    const unsigned l2 = __builtin_bit_cast(unsigned, l1 - __builtin_bit_cast(float, p1 << 16)), h2 = __builtin_bit_cast(unsigned, h1 - __builtin_bit_cast(float, p1 & 0xffff0000u));
+    p2 = __builtin_amdgcn_perm(h2, l2, 0x07060302u);   // their upper halves
+    left |= l2 | h2;
+}
+
+// One bit pattern at a time: a tree of ors over what is taken apart keeps all that was left in registers until its end.
+__device__ __forceinline__ void gather_left(unsigned& left)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("" : "+v"(left));
+#endif
 }
 
 __device__ __forceinline__ f32x4 mfma_bf16(u32x4 a, u32x4 b, f32x4 c)
@@ -47,10 +55,10 @@ __device__ __forceinline__ f32x4 mfma_bf16(u32x4 a, u32x4 b, f32x4 c)
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// Whether the values whose leading parts were or-ed into `seen` are all below 2^-95 without all being zero.
-__device__ __forceinline__ bool split_tiny(unsigned seen)
+// Whether one of the values taken apart is more than its three parts.
+__device__ __forceinline__ bool split_inexact(unsigned left)
 {
-    return (seen & 0x7fff7fffu) != 0 && (seen & 0x70007000u) == 0;
+    return (left & 0xffffu) != 0;
 }
 
 // The products (part A[t] of one operand, part B[t] of the other); all but the last are 2^-8 and less of it.  Part 2 of B is done

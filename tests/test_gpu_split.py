@@ -47,14 +47,16 @@ def test_split_convolution_against_the_oracle(tag, s, p):
 
 
 @pytest.mark.parametrize("tag,s,p", [("i", 1, 1), ("j", 2, 0)])
-def test_infinite_and_tiny_pixels_of_a_split_convolution(tag, s, p):
+@pytest.mark.parametrize("scale", [2.0 ** -118, 2.0 ** -140])
+def test_infinite_and_tiny_pixels_of_a_split_convolution(tag, s, p, scale):
     """An infinite, a NaN and a lowest value are in the windows that hold them and in no others (padding beside them is not
     multiplied), an image of values below bf16's bits keeps its own."""
     name = f"selftest_gemm_split_{tag}"
     x, w = _operands(name)
     w = np.abs(w) + np.float32(0.5)
     x[0, 3, 0, 0], x[1, 5, 4, 3], x[1, 2, 0, 6], x[0, 7, 5, 5] = np.inf, np.nan, -np.inf, np.finfo(np.float32).min
-    x[2] *= np.float32(2.0 ** -118)
+    x[2] *= np.float32(scale)
+    w *= np.float32(2.0 ** 60)
     with np.errstate(all="ignore"):
         want = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(w).double(), stride=s, padding=p).numpy()
         f = want.astype(np.float32)
@@ -124,6 +126,61 @@ def test_scaled_operands_keep_their_bits(tag, scale):
     want, y = want.reshape(-1, want.shape[-1]), y.reshape(-1, want.shape[-1])
     for r in range(want.shape[0]):
         assert np.linalg.norm(y[r] - want[r]) <= u * np.linalg.norm(want[r]), r
+
+
+@pytest.mark.parametrize("tag", ["_a", "_b", "_e", "k_b", "k_c"])
+@pytest.mark.parametrize("scale", [2.0 ** -112, 2.0 ** -125, 2.0 ** -136, 2.0 ** -145])
+def test_values_with_bits_below_the_parts_keep_them(tag, scale):
+    """Operands, or some rows of them, of which one bf16 part or all three are zero or hold less than the value (results are
+    ordinary numbers: the other operand is that much larger)."""
+    name = f"selftest_gemm_split{tag}"
+    x, w = _operands(name)
+    u = 2.0 ** -24 * x.shape[1 if x.shape[2] == 1 else 2] ** 0.5 * 2     # as above
+    big = np.float32(2.0 ** 90)
+    some = x.copy().reshape(-1, x.shape[-3] if x.shape[2] == 1 else x.shape[-2])
+    some[3::16] *= np.float32(scale)
+    for a, b in ((x * np.float32(scale), w * big), (x * big, w * np.float32(scale)), (some.reshape(x.shape), w * big)):
+        want = _product(a, b)
+        y = _run(name, a, b).reshape(want.shape).astype(np.float64)
+        want, y = want.reshape(-1, want.shape[-1]), y.reshape(-1, want.shape[-1])
+        for r in range(want.shape[0]):
+            assert np.linalg.norm(y[r] - want[r]) <= u * np.linalg.norm(want[r]), r
+
+
+def _one_hot(name, x, w, side, values):
+    """The operands with `side` replaced by one value a row (column) of the result, at k = row (column) modulo K, and what the
+    product then is: that value times the other operand's k."""
+    rows = x.shape[2] == 1                         # [M, K] . [K, N], or [b, M, K] . [b, N, K]^T
+    x, w = x.copy(), w.copy()
+    if side == 0:
+        x[...] = 0
+        m = x.shape[0 if rows else 1]
+        k = np.arange(m) % x.shape[1 if rows else 2]
+        if rows:
+            x[np.arange(m), k, 0, 0] = values[:m]
+        else:
+            x[:, np.arange(m), k, 0] = values[:m]
+    else:
+        w[...] = 0
+        n = w.shape[1]
+        k = np.arange(n) % w.shape[0 if rows else 2]
+        if rows:
+            w[k, np.arange(n), 0, 0] = values[:n]
+        else:
+            w[:, np.arange(n), k, 0] = values[:n]
+    return x, w, _product(x, w)
+
+
+@pytest.mark.parametrize("tag", ["_a", "_b", "_e", "k_b", "k_c"])
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** -112, 2.0 ** -120, 2.0 ** -126])
+@pytest.mark.parametrize("side", [0, 1])
+def test_a_product_with_a_permutation_is_exact(tag, scale, side):
+    """... whatever small values lie beside ordinary ones."""
+    name = f"selftest_gemm_split{tag}"
+    x, w = _operands(name)
+    (w if side == 0 else x).reshape(-1)[3::7] *= np.float32(scale)
+    x, w, want = _one_hot(name, x, w, side, np.ones(max(x.size, w.size), np.float32))
+    assert np.array_equal(_run(name, x, w).reshape(want.shape), want.astype(np.float32))
 
 
 @pytest.mark.parametrize("tag", ["_a", "_b", "_e", "k_b", "k_c"])
