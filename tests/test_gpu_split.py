@@ -184,6 +184,24 @@ def test_a_product_with_a_permutation_is_exact(tag, scale, side):
 
 
 @pytest.mark.parametrize("tag", ["_a", "_b", "_e", "k_b", "k_c"])
+@pytest.mark.parametrize("side", [0, 1])
+def test_sums_of_one_product(tag, side):
+    """One product of two values of 24 bits.  With u = 2^-24, of the product: its sum is rounded (u), after what the smaller partial
+    products came to has been cut off at half a unit of its last place (u); the two larger ones of the partial products that are
+    left out are u / 2 each at most; the five smaller ones, 2^-7 of the product together, are cut and rounded on their way."""
+    name = f"selftest_gemm_split{tag}"
+    x, w = _operands(name)
+    # the worst is near 1 + 2^-8, where the second part is half a bit of the first
+    near = fill_normal(5, x.size + w.size, 0, 1)
+    worst = (np.float32(1) + np.float32(2.0 ** -8) + np.arange(w.size + x.size, dtype=np.float32) % 512 * np.float32(2.0 ** -20)).astype(np.float32)
+    for values, other in ((near, near), (worst, worst)):
+        a, b = (x, other[: w.size].reshape(w.shape)) if side == 0 else (other[: x.size].reshape(x.shape), w)
+        a, b, want = _one_hot(name, a, b, side, values)
+        y = _run(name, a, b).reshape(want.shape)
+        assert np.all(np.abs(y - want) <= 2.0 ** -24 * (3 + 10 * 2.0 ** -7) * np.abs(want))
+
+
+@pytest.mark.parametrize("tag", ["_a", "_b", "_e", "k_b", "k_c"])
 def test_infinities_nan_and_the_largest_values(tag):
     """What does not fit three bf16 gives what fp32 arithmetic gives: infinite where it is, NaN where it is, finite elsewhere."""
     name = f"selftest_gemm_split{tag}"
