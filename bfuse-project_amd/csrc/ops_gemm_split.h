@@ -42,8 +42,8 @@
 // load want the same k, so where the element lies from the window's first one comes from a table by a scalar load; padding is a
 // lane whose bit for that tap is set and which therefore reads past the buffer (two vector instructions a load).  Every element
 // is taken apart once for each tap it is under: 256 -> 256 channels on 14 x 14, batch 1024, 1713 -> 1035 us (229 TFLOP/s);
-// ConvTiling has the other layers and where the line to the shared tiles lies.  A row tile (kRows: also a column tile) that does not divide the problem starts
-// a tile before its end and writes the same bits as its neighbour.
+// ConvTiling has the other layers and where the line to the shared tiles lies.  A row tile (kRows: also a column tile) that does not
+// divide the problem starts a tile before its end and leaves its neighbour's results to it: one of the two may be done again.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -417,12 +417,16 @@ struct GemmSplit {
             }
         }
         // lane (i, q): row i of a 16-row block, columns 4q .. 4q + 3 of each 16-column block
+        const auto own_row = [&](int m) { return M % BM == 0 || m >= mt * BM; };
 #pragma unroll
         for (int b = 0; b < TN; ++b) {
             const int col = (wn * TN + b) * 16 + 4 * eq;
             if constexpr (LAYOUT == kRows) {
 #pragma unroll
-                for (int tm = 0; tm < TM; ++tm) *reinterpret_cast<f32x4*>(C + (size_t)(m0 + (wr * TM + tm) * 16 + ei) * W + n0 + col) = acc[tm][b];
+                for (int tm = 0; tm < TM; ++tm) {
+                    const int m = m0 + (wr * TM + tm) * 16 + ei;
+                    if (own_row(m) && (W % BN == 0 || n0 + col >= nt * BN)) *reinterpret_cast<f32x4*>(C + (size_t)m * W + n0 + col) = acc[tm][b];
+                }
             } else {
                 const int vc = v0 + col, img = n_lo + vc / OHWP, p = vc % OHWP;
                 if (img < NIMG) {
@@ -430,6 +434,7 @@ struct GemmSplit {
                     const bool whole = OHW % 4 == 0 || p + 4 <= OHW;
 #pragma unroll
                     for (int tm = 0; tm < TM; ++tm) {
+                        if (!own_row(m0 + (wr * TM + tm) * 16 + ei)) continue;
                         float* const d = y + (size_t)(tm * 16) * OHW;
                         const f32x4 o = acc[tm][b];
                         if constexpr (OHW % 4 == 0) {

@@ -201,6 +201,22 @@ def test_sums_of_one_product(tag, side):
         assert np.all(np.abs(y - want) <= 2.0 ** -24 * (3 + 10 * 2.0 ** -7) * np.abs(want))
 
 
+@pytest.mark.parametrize("tag,side,at,kept", [("_a", 0, 150, 128), ("_f", 0, 200, 112), ("_e", 1, 79, 64)])
+def test_overlapping_tiles_leave_their_neighbours_results_to_them(tag, side, at, kept):
+    """A value that its parts do not hold in the last row (column) tile: that one is done again, and the rows (columns) before
+    the last tile's own keep their bits."""
+    name = f"selftest_gemm_split{tag}"
+    x, w = _operands(name)
+    k = np.s_[at, 2] if x.shape[2] == 1 else np.s_[:, at, 2]
+    out = []
+    for v in (0, 2.0 ** -120 * 1.2345678):
+        (x, w)[side][k] = v
+        out.append(_run(name, x, w).reshape(_product(x, w).shape))
+    a, b = (o[..., :kept, :] if side == 0 else o[..., :kept] for o in out)
+    assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    assert not np.array_equal(out[0], out[1])
+
+
 @pytest.mark.parametrize("tag", ["_a", "_b", "_e", "k_b", "k_c"])
 def test_infinities_nan_and_the_largest_values(tag):
     """What does not fit three bf16 gives what fp32 arithmetic gives: infinite where it is, NaN where it is, finite elsewhere."""
