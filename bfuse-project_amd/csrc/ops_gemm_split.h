@@ -27,7 +27,11 @@
 // 1.0e-7 but 1.5e-6 on 576, 4.0e-7, 4.6e-6 on 4096; 1-3 % faster on large tiles, where the sums' additions take the place of other
 // vector work.)  What three bf16 cannot hold is multiplied again with the fp32 MFMAs (see split.h): a wave whose results are not
 // all finite, and the workgroup if a thread has met a value that is more than its parts (the
-// ors that notice it take 0.2 % of the time in the mean, 2 % of 512 and 1024 x 4096 x 4096).
+// ors that notice it take 0.2 % of the time in the mean, 2 % of 512 and 1024 x 4096 x 4096).  That pass is bound by the fp32 MFMAs and
+// by loads that waves do not share; a tile takes 1.5 - 4 times what it took (us, no such value / one / one in every row of A;
+// in brackets with four dependent k at a time): 1024 x 4096 x 14336 655 / 1630 (7923) / 1740, 1024 x 4096 x 4096 171 / 463 (2573) /
+// 500, 512 x 512 x 128 of 32 heads 20 / 44 (185) / 49, 256 -> 256 on 14 x 14 1285 / 1282 (2957) / 4290 (18392), all on
+// uniform operands and a card that had been idle.
 //
 // Reductions of up to four stages are one partial sum: no second set of accumulators, every stage compiled apart, and so nothing
 // loaded or taken apart past the last one (with two stages that was half of it): 512 x 128 x 512 545 -> 499 us.
@@ -392,27 +396,88 @@ struct GemmSplit {
                 for (int v = 0; v < 4; ++v) zero = __builtin_fmaf(acc[tm][b][v], 0.f, zero);
         again |= __builtin_amdgcn_ballot_w64(zero != 0.f) != 0;
         if (again) {
+            // In ascending order of k, four an MFMA, as a sum that overflows wants it.
+            unsigned bo[TN], outside[TN];
 #pragma unroll
             for (int b = 0; b < TN; ++b) {
-                unsigned outside;
-                const unsigned c = column((wn * TN + b) * 16 + ei, outside), v = T > 1 || c == 0x7fffffffu ? c : c + eq * B_K;
+                const unsigned c = column((wn * TN + b) * 16 + ei, outside[b]);
+                bo[b] = LAYOUT == kRows ? c + eq * 16 : T > 1 || c == 0x7fffffffu ? c : c + eq * B_K;
+            }
 #pragma unroll
-                for (int tm = 0; tm < TM; ++tm) acc[tm][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+                for (int b = 0; b < TN; ++b) acc[tm][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (LAYOUT == kRows) {
+                // Rows on both sides: group q of 16 lanes loads k + 4q .. k + 4q + 3 and gets k + q, k + 4 + q, .. from the others.
 #pragma unroll 1
-                for (int k = 0; k < K; k += 4) {
-                    unsigned at = k * B_K, o = v;
-                    if constexpr (T > 1) {
-                        at = TAPS.at[k + eq];
-                        o |= (unsigned)__builtin_amdgcn_sbfe((int)outside, at, 1);
-                        if (o != ~0u) o += (at >> 5) * 4;
-                        at = 0;
-                    }
-                    const float bv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(br, o, at, 0));
+                for (int k = 0; k < K; k += 16) {
+                    const bool past = K % 16 != 0 && k + 4 * eq >= K;
+                    f32x4 a[TM], v[TN];
 #pragma unroll
-                    for (int tm = 0; tm < TM; ++tm) {
-                        const float av = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ar, (((wr * TM + tm) * 16 + ei) * K + eq) * 4, k * 4, 0));
-                        acc[tm][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv, av, acc[tm][b], 0, 0, 0);
+                    for (int tm = 0; tm < TM; ++tm)
+                        a[tm] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ar, past ? 0x7fffffffu : (unsigned)((((wr * TM + tm) * 16 + ei) * K + 4 * eq) * 4), k * 4, 0));
+#pragma unroll
+                    for (int b = 0; b < TN; ++b) v[b] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(br, past ? 0x7fffffffu : bo[b], k * 4, 0));
+#pragma unroll
+                    for (int tm = 0; tm < TM; ++tm) transpose_groups(a[tm]);
+#pragma unroll
+                    for (int b = 0; b < TN; ++b) transpose_groups(v[b]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int b = 0; b < TN; ++b)
+#pragma unroll
+                            for (int tm = 0; tm < TM; ++tm) acc[tm][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[b][e], a[tm][e], acc[tm][b], 0, 0, 0);
+                }
+            } else {
+                // Eight k at a time; the next eight are on their way meanwhile.
+                float na[2][TM], nb[2][TN];
+                auto fetch = [&](int k) {
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+#pragma unroll
+                        for (int tm = 0; tm < TM; ++tm)
+                            na[e][tm] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ar, (((wr * TM + tm) * 16 + ei) * K + eq + 4 * e) * 4, k * 4, 0));
+                    unsigned at[2];
+                    if constexpr (T > 1) {
+                        unsigned t[8];
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) t[e] = TAPS.at[k + e];
+#pragma unroll
+                        for (int e = 0; e < 2; ++e) at[e] = eq & 2 ? (eq & 1 ? t[4 * e + 3] : t[4 * e + 2]) : (eq & 1 ? t[4 * e + 1] : t[4 * e]);
                     }
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+#pragma unroll
+                        for (int b = 0; b < TN; ++b) {
+                            unsigned o = bo[b];
+                            if constexpr (T > 1) {
+                                o |= (unsigned)__builtin_amdgcn_sbfe((int)outside[b], at[e], 1);
+                                if (o != ~0u) o += (at[e] >> 5) * 4;
+                            }
+                            nb[e][b] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(br, o, T > 1 ? 0 : (k + 4 * e) * B_K, 0));
+                        }
+                };
+                fetch(0);
+#pragma unroll 1
+                for (int k = 0; k < K; k += 8) {
+                    float a[2][TM], v[2][TN];
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+#pragma unroll
+                        for (int tm = 0; tm < TM; ++tm) a[e][tm] = na[e][tm];
+#pragma unroll
+                        for (int b = 0; b < TN; ++b) v[e][b] = nb[e][b];
+                    }
+                    fetch(k + 8 < K ? k + 8 : k);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+#pragma unroll
+                        for (int b = 0; b < TN; ++b)
+#pragma unroll
+                            for (int tm = 0; tm < TM; ++tm) acc[tm][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][b], a[e][tm], acc[tm][b], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
             }
         }

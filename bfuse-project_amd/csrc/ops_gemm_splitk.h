@@ -21,7 +21,8 @@
 //
 // What three bf16 cannot hold (split.h): a wave whose sums are not all finite, or that has met a value that is more than its
 // parts, hands over NaN.  Finite sums add up to NaN never, so all waves then see NaN in what they finish, and all multiply
-// their k-range again with the fp32 instructions.
+// their k-range again with the fp32 instructions (512 x 768 x 2304: 16.6 us without such a value, 32-34 with; 39-41 with four
+// dependent k at a time).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -215,26 +216,49 @@ struct GemmSplitK {
                 for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
                     for (int b = 0; b < NB; ++b) acc[tm][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-                for (int k = 0; k < KW; k += 4) {
-                    float a[TM];
+                // Eight k at a time, in ascending order as a sum that overflows wants it; the next eight are on their way meanwhile.
+                float na[2][TM];
+                f32x4 nb[2][G4];
+                float nt[2][G1 > 0 ? G1 : 1];
+                auto fetch = [&](int k) {
 #pragma unroll
-                    for (int tm = 0; tm < TM; ++tm)
-                        a[tm] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ar, (unsigned)(((tm * 16 + li) * K + kq) * 4), k * 4, 0));
-#pragma unroll
-                    for (int g = 0; g < G4; ++g) {
-                        const f32x4 v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(br, (unsigned)((kq * N + g * 64 + 4 * li) * 4), k * (N * 4), 0));
+                    for (int e = 0; e < 2; ++e) {
 #pragma unroll
                         for (int tm = 0; tm < TM; ++tm)
+                            na[e][tm] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ar, (unsigned)(((tm * 16 + li) * K + kq + 4 * e) * 4), k * 4, 0));
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) acc[tm][4 * g + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[tm], v[e], acc[tm][4 * g + e], 0, 0, 0);
+                        for (int g = 0; g < G4; ++g)
+                            nb[e][g] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(br, (unsigned)((kq * N + g * 64 + 4 * li) * 4), (k + 4 * e) * (N * 4), 0));
+#pragma unroll
+                        for (int g = 0; g < G1; ++g)
+                            nt[e][g] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(br, (unsigned)((kq * N + G4 * 64 + g * 16 + li) * 4), (k + 4 * e) * (N * 4), 0));
                     }
+                };
+                fetch(0);
+#pragma unroll 1
+                for (int k = 0; k < KW; k += 8) {
+                    float a[2][TM];
+                    f32x4 v[2][G4];
+                    float w[2][G1 > 0 ? G1 : 1];
 #pragma unroll
-                    for (int g = 0; g < G1; ++g) {
-                        const float v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(br, (unsigned)((kq * N + G4 * 64 + g * 16 + li) * 4), k * (N * 4), 0));
+                    for (int e = 0; e < 2; ++e) {
 #pragma unroll
-                        for (int tm = 0; tm < TM; ++tm) acc[tm][4 * G4 + g] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[tm], v, acc[tm][4 * G4 + g], 0, 0, 0);
+                        for (int tm = 0; tm < TM; ++tm) a[e][tm] = na[e][tm];
+#pragma unroll
+                        for (int g = 0; g < G4; ++g) v[e][g] = nb[e][g];
+#pragma unroll
+                        for (int g = 0; g < G1; ++g) w[e][g] = nt[e][g];
                     }
+                    fetch(k + 8 < KW ? k + 8 : k);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+#pragma unroll
+                        for (int b = 0; b < NB; ++b)
+#pragma unroll
+                            for (int tm = 0; tm < TM; ++tm)
+                                acc[tm][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e][tm], b < 4 * G4 ? v[e][b / 4 < G4 ? b / 4 : 0][b % 4] : w[e][b < 4 * G4 ? 0 : b - 4 * G4], acc[tm][b], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
                 hand_over(0, 0.f);
                 sync();

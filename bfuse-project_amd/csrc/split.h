@@ -61,6 +61,17 @@ __device__ __forceinline__ f32x4 mfma_bf16(u32x4 a, u32x4 b, f32x4 c)
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
+// The four groups of 16 lanes as the rows of a matrix, the components as its columns: transposed.
+__device__ __forceinline__ void transpose_groups(f32x4& r)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    u32x4 u = __builtin_bit_cast(u32x4, r);
+    const u32x2 a = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(u[0], u[2], false, false)), b = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(u[1], u[3], false, false));
+    const u32x2 c = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false)), d = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false));
+    r = __builtin_bit_cast(f32x4, u32x4{c[0], c[1], d[0], d[1]});
+#endif
+}
+
 // Whether one of the values taken apart is more than its three parts.
 __device__ __forceinline__ bool split_inexact(unsigned left)
 {
