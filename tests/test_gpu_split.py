@@ -201,6 +201,28 @@ def test_sums_of_one_product(tag, side):
         assert np.all(np.abs(y - want) <= 2.0 ** -24 * (3 + 10 * 2.0 ** -7) * np.abs(want))
 
 
+@pytest.mark.parametrize("tag,partner,kind,suffix", [
+    ("_a", "layernorm_8x256", "bfuse", "_c4"), ("_e", "bias_relu_4096", "hfuse", ""), ("_f", "conv3x3_f32_32x12x12_32", "hfuse", ""),
+    ("k_a", "layernorm_8x256", "bfuse", "_c4"), ("k_b", "bias_relu_4096", "hfuse", ""), ("k_b", "conv3x3_f32_32x12x12_32", "hfuse", "")])
+@pytest.mark.parametrize("value", [2.0 ** -120 * 1.2345678, np.inf])
+def test_fused_kernels_multiply_again_where_the_parts_do_not_do(tag, partner, kind, suffix, value):
+    """One value that its parts do not hold: the tiles it is in are done again, with as many barriers as that takes, and fused
+    results are the unfused ones' bits."""
+    name = f"selftest_gemm_split{tag}"
+    x, w = _operands(name)
+    x.reshape(-1)[x.shape[1 if x.shape[2] == 1 else 2] + 2] = value
+    with bf.Operation(name, partner) as op:
+        P = [fill_normal(21 + i, int(np.prod(op.k[1].shapes[i])), 0, 1) for i in (0, 1)]
+        o1, o2 = op.run_kernel(0, x, w), op.run_kernel(1, *P)
+        f1, f2 = op.run_fuse(op.fused(kind, suffix), x, w, *P)
+    with np.errstate(all="ignore"):
+        want = (_gelu if tag == "k_a" else np.asarray)(_product(x, w))
+    o = o1.reshape(want.shape)
+    ok = np.isfinite(want)
+    assert np.array_equal(np.isfinite(o), ok) and np.linalg.norm(o[ok] - want[ok]) <= 1e-5 * np.linalg.norm(want[ok])
+    assert np.array_equal(o1.view(np.uint32), f1.view(np.uint32)) and np.array_equal(o2.view(np.uint32), f2.view(np.uint32))
+
+
 @pytest.mark.parametrize("tag,side,at,kept", [("_a", 0, 150, 128), ("_f", 0, 200, 112), ("_e", 1, 79, 64)])
 def test_overlapping_tiles_leave_their_neighbours_results_to_them(tag, side, at, kept):
     """A value that its parts do not hold in the last row (column) tile: that one is done again, and the rows (columns) before
