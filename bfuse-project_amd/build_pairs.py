@@ -18,6 +18,10 @@ checks (csrc/Makefile, target `module`).  `<suite>/config/modules.yaml` then nam
 
 Thread-level fusion is written only where it can work: both workgroups fit one (at most 1024 threads and
 160 KB of LDS together) and at most one side synchronises (config.choose_fusion's rule).
+
+A fused kernel whose sides need more registers than its workgroup leaves them is not built as it stands: if a side
+has more than 512 threads (three waves on a SIMD: 168 registers for both sides) it takes that side's form of fewer
+waves (Narrow: the same tiles, the same bits), and what then still does not fit is left out and named.
 """
 import argparse
 import os
@@ -167,9 +171,10 @@ def stale_units(hip_dir: str, types=None) -> List[str]:
     return out
 
 
-def drop_spilling(hip_dir: str) -> List[str]:
-    """Removes, from every pairs_*.hip whose last compilation reported spills, the kernels that spilled."""
-    dropped = []
+def _edit_spilling(hip_dir: str, edit) -> List[str]:
+    """Replaces the line of every kernel whose last compilation reported spills by `edit(name, line)`, where that is
+    another one; the names of these kernels."""
+    changed = []
     for f in sorted(os.listdir(hip_dir)):
         if not (f.startswith("pairs_") and f.endswith(".res")):
             continue
@@ -180,17 +185,35 @@ def drop_spilling(hip_dir: str) -> List[str]:
         src = os.path.join(hip_dir, f[:-4] + ".hip")
         with open(src) as fh:
             lines = fh.read().splitlines()
-        keep = []
+        out = []
         for line in lines:
             name = None if line.startswith("//") else _unit_kernel(line)
-            if name in bad:
-                dropped.append(name)
-                keep.append(f"// not built (does not fit the register file in this form): {name}")
-            else:
-                keep.append(line)
-        with open(src, "w") as fh:
-            fh.write("\n".join(keep) + "\n")
-    return dropped
+            out.append(edit(name, line) if name in bad else line)
+            if out[-1] != line:
+                changed.append(name)
+        if out != lines:
+            with open(src, "w") as fh:
+                fh.write("\n".join(out) + "\n")
+    return changed
+
+
+def narrow_spilling(hip_dir: str, registry: Dict[str, object]) -> List[str]:
+    """Gives every kernel whose last compilation reported spills its sides of more than 512 threads in their form of
+    fewer waves (csrc/wave.h, Narrow)."""
+    def edit(name, line):
+        macro, args = line.rstrip(")").split("(", 1)
+        a = [x.strip() for x in args.split(",")]
+        for i in (0, 2):
+            k = registry[a[i]]
+            if k.block[0] * k.block[1] * k.block[2] > 512 and not a[i + 1].startswith("Narrow<"):
+                a[i + 1] = f"Narrow<{a[i + 1]}>"
+        return f"{macro}({', '.join(a)})"
+    return _edit_spilling(hip_dir, edit)
+
+
+def drop_spilling(hip_dir: str) -> List[str]:
+    """Removes, from every pairs_*.hip whose last compilation reported spills, the kernels that spilled."""
+    return _edit_spilling(hip_dir, lambda name, line: f"// not built (does not fit the register file in this form): {name}")
 
 
 def suite_pairs(suite: str, triangular: bool = False) -> List[Tuple[str, str]]:
@@ -263,17 +286,19 @@ def build(suite: str, forms: str = "both", chunk: int = 256, only: Optional[Sequ
     if compile_:      # make decides what is out of date (new units, or headers of the library that changed)
         cmd = ["make", "-C", CSRC, f"MODDIR={os.path.abspath(hip)}", f"-j{jobs}", "-k", "module"]
         r = subprocess.run(cmd, capture_output=True, text=True)
-        if r.returncode != 0:
-            # A fused kernel that needs more registers than its launch bounds leave (a side that already fills the
-            # register file, thread-fused with another) fails the library's no-spill check: such kernels are taken
-            # out of their translation units and the build is run once more; anything else is an error.
-            dropped = drop_spilling(hip)
-            if not dropped:
-                raise RuntimeError(f"building {module} failed:\n{r.stdout[-3000:]}\n{r.stderr[-3000:]}")
+        # A fused kernel that needs more registers than its launch bounds leave (a side that already fills the
+        # register file, thread-fused with another) fails the library's no-spill check: its sides of many waves take
+        # their narrow form, then those that still spill are taken out of their translation units; anything else is
+        # an error.
+        if r.returncode != 0 and narrow_spilling(hip, registry):
             r = subprocess.run(cmd, capture_output=True, text=True)
-            if r.returncode != 0:
-                raise RuntimeError(f"building {module} failed:\n{r.stdout[-3000:]}\n{r.stderr[-3000:]}")
-            todo = [k for k in todo if k["name"] not in dropped]
+        if r.returncode != 0:
+            dropped = drop_spilling(hip)
+            if dropped:
+                r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError(f"building {module} failed:\n{r.stdout[-3000:]}\n{r.stderr[-3000:]}")
+        todo = [k for k in todo if k["name"] not in dropped]
         build_operators.name_module(suite, os.path.join("hip", "libbfuse_pairs.so"))
     return {"kernels": todo, "files": files, "module": module if compile_ else None, "dropped": dropped}
 

@@ -251,6 +251,8 @@ DENSE_SPLIT_TEST(p, 32, 288, 64, 1, 2, 2, 1, 32)
 BGEMM_SPLIT_TEST(q, 3, 48, 24, 32, 1, 3, 1, 1, 32)               // one stage, and that not whole
 CONV1_SPLIT_TEST(g, 48, 80, 9, 9, 1, 5, 1, 4, 2, 1, 128)
 CONV1_SPLIT_TEST(h, 56, 64, 9, 7, 2, 11, 2, 2, 1, 2, 96)
+CONV1_SPLIT_TEST(r, 64, 160, 9, 9, 1, 5, 1, 10, 1, 1, 128)       // ten waves, block-fused in the form of five
+BFUSE_BFUSE_KERNEL(selftest_gemm_split_r, Narrow<GemmSp_r>, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
 BFUSE_BFUSE_KERNEL(selftest_gemm_split_a, GemmSp_a, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
 BFUSE_HFUSE_KERNEL(selftest_gemm_split_e, GemmSp_e, bias_relu_4096, BiasReluS)
 BFUSE_HFUSE_KERNEL(selftest_gemm_split_f, GemmSp_f, conv3x3_f32_32x12x12_32, ConvS2)

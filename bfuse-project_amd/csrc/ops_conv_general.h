@@ -355,5 +355,9 @@ struct SwapOperands : Op {
         Op::run(vblock, tid, sm, F, I, O, sync);
     }
 };
+template <class Op>
+struct NarrowOf<SwapOperands<Op>> {
+    using type = SwapOperands<Narrow<Op>>;
+};
 
 }  // namespace bfuse

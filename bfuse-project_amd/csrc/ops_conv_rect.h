@@ -309,6 +309,10 @@ struct ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, KS, NIMG, kSplitForm> : Co
         Form::run(vblock, tid, sm, I, F, O, sync);
     }
 };
+template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int BM, int PB, int KS, int NIMG>
+struct NarrowOf<ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, KS, NIMG, kSplitForm>> {
+    using type = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, (KS > 8 && KS % 2 == 0 ? KS / 2 : KS), NIMG, kSplitForm>;
+};
 
 // The tiling the library gives a convolution it has no hand-picked one for: as many output channels per
 // workgroup as keep the filter fragments of a wave within ~72 registers (the staged patch is shared by all

@@ -369,7 +369,7 @@ struct GemmSplit {
         const int el = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), ei = el & 15, eq = el >> 4;
         if (split_inexact(left)) sm.inexact = 1;
         sync.raw();
-        bool again = sm.inexact != 0;
+        const bool again = sm.inexact != 0;
         if constexpr (KG > 1) {
             f32x4* const red = reinterpret_cast<f32x4*>(sm.t) + w * TM * TN * 64 + el;
             if (g > 0) {
@@ -387,16 +387,22 @@ struct GemmSplit {
 #pragma unroll
                     for (int q = 1; q < KG; ++q) acc[tm][b] += red[((q - 1) * WR * WN * TM * TN + tm * TN + b) * 64];
         }
-        float zero = 0.f;                           // or NaN
+        // Which 16-row blocks are done again: all of the tile's, or the wave's with a result that is not finite (by block, so that the
+        // bits do not depend on how many blocks a wave has).
+        bool redo[TM], any = false;
 #pragma unroll
-        for (int tm = 0; tm < TM; ++tm)
+        for (int tm = 0; tm < TM; ++tm) {
+            float zero = 0.f;                       // or NaN
 #pragma unroll
             for (int b = 0; b < TN; ++b)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) zero = __builtin_fmaf(acc[tm][b][v], 0.f, zero);
-        again |= __builtin_amdgcn_ballot_w64(zero != 0.f) != 0;
-        if (again) {
+            redo[tm] = again || __builtin_amdgcn_ballot_w64(zero != 0.f) != 0;
+            any |= redo[tm];
+        }
+        if (any) {
             // In ascending order of k, four an MFMA, as a sum that overflows wants it.
+            f32x4 re[TM][TN];
             unsigned bo[TN], outside[TN];
 #pragma unroll
             for (int b = 0; b < TN; ++b) {
@@ -406,7 +412,7 @@ struct GemmSplit {
 #pragma unroll
             for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
-                for (int b = 0; b < TN; ++b) acc[tm][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int b = 0; b < TN; ++b) re[tm][b] = f32x4{0.f, 0.f, 0.f, 0.f};
             if constexpr (LAYOUT == kRows) {
                 // Rows on both sides: group q of 16 lanes loads k + 4q .. k + 4q + 3 and gets k + q, k + 4 + q, .. from the others.
 #pragma unroll 1
@@ -427,7 +433,7 @@ struct GemmSplit {
 #pragma unroll
                         for (int b = 0; b < TN; ++b)
 #pragma unroll
-                            for (int tm = 0; tm < TM; ++tm) acc[tm][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[b][e], a[tm][e], acc[tm][b], 0, 0, 0);
+                            for (int tm = 0; tm < TM; ++tm) re[tm][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[b][e], a[tm][e], re[tm][b], 0, 0, 0);
                 }
             } else {
                 // Eight k at a time; the next eight are on their way meanwhile.
@@ -476,10 +482,15 @@ struct GemmSplit {
 #pragma unroll
                         for (int b = 0; b < TN; ++b)
 #pragma unroll
-                            for (int tm = 0; tm < TM; ++tm) acc[tm][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][b], a[e][tm], acc[tm][b], 0, 0, 0);
+                            for (int tm = 0; tm < TM; ++tm) re[tm][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][b], a[e][tm], re[tm][b], 0, 0, 0);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
+#pragma unroll
+            for (int tm = 0; tm < TM; ++tm)
+                if (redo[tm])
+#pragma unroll
+                    for (int b = 0; b < TN; ++b) acc[tm][b] = re[tm][b];
         }
         // lane (i, q): row i of a 16-row block, columns 4q .. 4q + 3 of each 16-column block
         const auto own_row = [&](int m) { return M % BM == 0 || m >= mt * BM; };
@@ -516,6 +527,14 @@ struct GemmSplit {
             }
         }
     }
+};
+
+// (see Narrow) us, ten waves and five, with twice the rows of a wave: 768 -> 160 channels on 17 x 17 460 and 514, 192 -> 320 at
+// stride 2 385 and 436, 1280 -> 320 on 8 x 8 296 and 324, 2048 -> 320 459 and 500.  (Eight waves of 80 x 32: the 3 x 3 layer spills.)
+template <int M, int K, int H, int W, int S, int NIMG, int TM, int WR, int WN, int KG, int BN, int LAYOUT, int KH, int KW, int P, bool LEAN>
+struct NarrowOf<GemmSplit<M, K, H, W, S, NIMG, TM, WR, WN, KG, BN, LAYOUT, KH, KW, P, LEAN>> {
+    static constexpr int HALVE = 64 * WR * WN * KG > 512 && WR % 2 == 0 ? 2 : 1;
+    using type = GemmSplit<M, K, H, W, S, NIMG, TM * HALVE, WR / HALVE, WN, KG, BN, LAYOUT, KH, KW, P, LEAN>;
 };
 
 }  // namespace bfuse

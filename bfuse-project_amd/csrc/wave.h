@@ -252,4 +252,14 @@ struct LdsReserve : Op {
     }
 };
 
+// An operator in at most 512 threads where it has such a form, otherwise itself: the same tiles, the same bits, slower alone.  A
+// workgroup of 512 threads has 256 registers a lane, one of 640 only 168, and the other side of a block-fused kernel has to do with as
+// many: more than half of the batch operators beside a ten-wave one do not.
+template <class Op>
+struct NarrowOf {
+    using type = Op;
+};
+template <class Op>
+using Narrow = typename NarrowOf<Op>::type;
+
 }  // namespace bfuse

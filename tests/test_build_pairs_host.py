@@ -1,7 +1,8 @@
 """build_pairs on the host: which fused kernels a suite lacks, the translation unit written for them, and the
-registry's own spelling of the operator types (no GPU, nothing compiled here -- the build step compiles the
-sample suite and the GPU tests run it)."""
+registry's own spelling of the operator types (no GPU; the build step compiles the sample suite and the GPU tests run it,
+here only the pairs of operators of more than 512 threads are compiled)."""
 import os
+import subprocess
 from types import SimpleNamespace as NS
 
 import pytest
@@ -100,3 +101,48 @@ def test_units_written_for_another_tiling_of_an_operator_are_found(tmp_path):
     assert build_pairs.stale_units(str(d), now) == ["pairs_0.hip"]
     assert build_pairs.stale_units(str(d), {"a": "bfuse::A<1>", "b": "bfuse::B<2>"}.__getitem__) == []
     assert build_pairs.stale_units(str(tmp_path / "none")) == []
+
+
+def test_kernels_that_spill_take_their_narrow_sides_and_are_left_out_only_then(tmp_path):
+    d = tmp_path / "hip"
+    d.mkdir()
+    reg = {k.name: k for k in (_k("a", 640, True), _k("b", 256, False), _k("c", 768, True))}
+    lines = ["using Side0 = bfuse::A<1, 2>;   // a", "BFUSE_BFUSE_KERNEL(a, Side0, b, Side1, _c256, bfuse::kChunked, 256, 1)", "BFUSE_BFUSE_RT_KERNEL(a, Side0, c, Side2)",
+             "BFUSE_HFUSE_KERNEL(b, Side1, b, Side1)", "BFUSE_BFUSE_KERNEL(c, Side2, b, Side1, _c256, bfuse::kChunked, 256, 1)"]
+    names = ["a_b_fused_bfuse_c256", "a_c_fused_bfuse_rt", "b_b_fused_hfuse"]
+    (d / "pairs_0.hip").write_text("\n".join(lines) + "\n")
+    (d / "pairs_0.res").write_text("".join(f"remark: Function Name: {n} [-R]\nremark:     ScratchSize [bytes/lane]: 8 [-R]\n" for n in names)
+                                   + "remark: Function Name: c_b_fused_bfuse_c256 [-R]\nremark:     ScratchSize [bytes/lane]: 0 [-R]\n")
+    assert build_pairs.narrow_spilling(str(d), reg) == names[:2]           # the third has no side of many waves
+    got = (d / "pairs_0.hip").read_text().splitlines()
+    assert got == [lines[0], "BFUSE_BFUSE_KERNEL(a, Narrow<Side0>, b, Side1, _c256, bfuse::kChunked, 256, 1)",
+                   "BFUSE_BFUSE_RT_KERNEL(a, Narrow<Side0>, c, Narrow<Side2>)", lines[3], lines[4]]
+    assert build_pairs.written(str(d)) == names + ["c_b_fused_bfuse_c256"]
+    assert build_pairs.narrow_spilling(str(d), reg) == []                  # narrow already
+    assert build_pairs.drop_spilling(str(d)) == names                      # spilled again: left out
+    assert [l for l in (d / "pairs_0.hip").read_text().splitlines() if l.startswith("BFUSE_")] == [lines[4]]
+
+
+def _suite_operators():
+    out = set()
+    for name in ("benchmark_batch1024", "inception_v3_batch1024", "interleave_scheduler_batch1024"):
+        doc = configure.load_user_config(os.path.join(ROOT, "bfuse-project_amd", "examples", f"{name}.yaml"))
+        out |= {k.name for k in configure.resolve(doc, {k.name: k for k in bf.list_kernels()}, None)[0].values()}
+    return sorted(out)
+
+
+@pytest.mark.parametrize("i", range(4))
+def test_no_block_fused_pair_of_the_batch_suites_is_left_out_for_registers(i, tmp_path):
+    """A side of at most 512 threads is compiled for 256 registers a lane, as many as a fused workgroup of two such sides has.  The
+    operators of more threads must have a form of fewer, and that must fit beside the partner that needs most."""
+    reg = {k.name: k for k in bf.list_kernels()}
+    wide = [n for n in _suite_operators() if reg[n].block[0] > 512]
+    assert len(wide) == 4
+    k = {"k1": wide[i], "k2": "bgemm_f32_1024x208x80x208", "form": "bfuse"}
+    k["name"] = f"{k['k1']}_{k['k2']}_fused_bfuse_c256"
+    src = build_pairs.source_text([k]).replace("Side0, ", "Narrow<Side0>, ") + "static_assert(Narrow<Side0>::THREADS <= 512 && Narrow<Side0>::GRID.size() == Side0::GRID.size());\n"
+    (tmp_path / "pairs_0.hip").write_text(src)
+    r = subprocess.run(["/opt/rocm/bin/hipcc", "--offload-arch=gfx950", "--cuda-device-only", "-O3", "-std=c++17", "-ffp-contract=off", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                        "-Rpass-analysis=kernel-resource-usage", "-I", build_pairs.CSRC, "-c", str(tmp_path / "pairs_0.hip"), "-o", str(tmp_path / "pairs_0.o")], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    assert f"Function Name: {k['name']}" in r.stderr and build_pairs.spilling_kernels(r.stderr) == []

@@ -36,9 +36,9 @@ def test_split_k_product_against_numpy_and_fused(tag, partner, kind, suffix):
     _check(f"selftest_gemm_splitk_{tag}", lambda a, b: (_gelu if tag == "a" else np.asarray)(_product(a, b)).astype(np.float32), partner, kind, suffix)
 
 
-@pytest.mark.parametrize("tag,s", [("g", 1), ("h", 2)])
-def test_split_1x1_convolution_against_the_oracle(tag, s):
-    _check(f"selftest_gemm_split_{tag}", lambda x, w: orf.conv2d(x, w, s=s, p=0), "bias_relu_4096", None, "")
+@pytest.mark.parametrize("tag,s,partner,kind,suffix", [("g", 1, "bias_relu_4096", None, ""), ("h", 2, "bias_relu_4096", None, ""), ("r", 1, "layernorm_8x256", "bfuse", "_c4")])
+def test_split_1x1_convolution_against_the_oracle(tag, s, partner, kind, suffix):
+    _check(f"selftest_gemm_split_{tag}", lambda x, w: orf.conv2d(x, w, s=s, p=0), partner, kind, suffix)
 
 
 @pytest.mark.parametrize("tag,s,p", [("i", 1, 1), ("j", 2, 0), ("k", 1, 2), ("l", 3, 2)])
@@ -221,6 +221,20 @@ def test_fused_kernels_multiply_again_where_the_parts_do_not_do(tag, partner, ki
     ok = np.isfinite(want)
     assert np.array_equal(np.isfinite(o), ok) and np.linalg.norm(o[ok] - want[ok]) <= 1e-5 * np.linalg.norm(want[ok])
     assert np.array_equal(o1.view(np.uint32), f1.view(np.uint32)) and np.array_equal(o2.view(np.uint32), f2.view(np.uint32))
+
+
+@pytest.mark.parametrize("side,value", [(0, 2.0 ** -120 * 1.2345678), (1, 2.0 ** -120 * 1.2345678), (0, np.inf), (1, np.inf)])
+def test_the_form_of_half_the_waves_does_the_same_results_again(side, value):
+    """Ten waves of 16 rows alone, five of 32 in the fused kernel: one image's pixel or one channel's weight that the parts do not hold."""
+    x, w = _operands("selftest_gemm_split_r")
+    (x, w)[side][(1, 5, 4, 3) if side == 0 else (19, 7, 0, 0)] = value
+    with bf.Operation("selftest_gemm_split_r", "layernorm_8x256") as op:
+        assert op.k[0].block[0] == 640 and op.fused("bfuse", "_c4").block[0] == 320
+        P = [fill_normal(21 + i, int(np.prod(op.k[1].shapes[i])), 0, 1) for i in (0, 1)]
+        o = op.run_kernel(0, x, w)
+        f = op.run_fuse(op.fused("bfuse", "_c4"), x, w, *P)[0]
+    assert np.isfinite(o).all() == np.isfinite(value) and np.isfinite(o).any()
+    assert np.array_equal(o.view(np.uint32), f.view(np.uint32))
 
 
 @pytest.mark.parametrize("tag,side,at,kept", [("_a", 0, 150, 128), ("_f", 0, 200, 112), ("_e", 1, 79, 64)])
