@@ -3,7 +3,8 @@
 // tilings of their 512-row / 16-product counterparts (model_ops.h) -- twice, or 64 times, the workgroups -- or with twice
 // the columns per tile, which is again a workgroup per CU and a better ratio of MFMAs to operand reads: 1024 x 3072 x 768
 // 44.4 -> 34.8 us (32 x 96 against 32 x 48), x 768 x 768 11.5 -> 10.8, 4096 x 1024 62.5 -> 60.2 (32 x 128 against 32 x 64).  The larger ones run on the bf16 matrix cores (ops_gemm_split.h has the figures): there the
-// tile is 128 x 128, 128 x 96 or 256 x 128, the largest that still gives every CU one, and those too small for 192 such tiles stay.
+// tile is 128 x 128, 128 x 96 or 256 x 128, the largest that still gives every CU one.  Those that have no 256 such tiles split K over the
+// waves of 32 x 96 - 32 x 144 tiles instead (GemmF32Dma): 1024 x 768 x 2304 24.8 us, on 192 tiles of 128 x 96 30.2.
 #include "fuse.h"
 #include "ops_gemm_f32.h"
 #include "ops_gemm_f32_dma.h"

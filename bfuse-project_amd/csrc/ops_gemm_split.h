@@ -4,8 +4,8 @@
 //   C[m][n] = sum_k A[m][k] * B(k, n)
 //
 // The fp32 forms (GemmF32Dma, GemmTile) run at 143 - 150 TFLOP/s on large products, the rate of the fp32 matrix instructions.
-// Six bf16 products at the 1.65 - 1.75 PFLOP/s that random operands leave the chip are 280 of these.  What stands in between is
-// taking the operands apart: 5.5 vector instructions an element, of which two go between two MFMAs of a wave almost for free
+// Six bf16 products at the 1.74 - 2.07 PFLOP/s that random operands leave the chip are 290 - 345 of these.  What stands in between is
+// taking the operands apart: six vector instructions an element, of which two go between two MFMAs of a wave almost for free
 // (17 -> 19 clocks) and more do not.  So the tile is as large as it can be (an element of A is used BN times, one of B BM times)
 // and every element is taken apart once in the workgroup:
 //   * a wave owns 16 TM rows of A alone and takes them apart in its registers: lane (i, q) loads A[i][8q .. 8q + 7], which is
@@ -19,15 +19,15 @@
 // The operands of an MFMA are given in the order (B, A), so that a lane ends up with four consecutive columns of a row.
 //
 // What rounds the sum is one addition per partial sum of four stages (`part`; two where there are 9 - 20 of them), of which each
-// stage's MFMAs round only the small beginning: 2-norm errors against 64 bits, with the largest error over the result's root mean
-// square, are below those of the fp32 forms.  Reduction of 14336 2.2e-7, 1.1e-6 (GemmF32Dma 1.1e-6, 6.6e-6), 4096 1.9e-7, 1.5e-6 (5.8e-7,
+// stage's MFMAs round only the small beginning: 2-norm errors against 64 bits are below those of the fp32 forms at every operator, the
+// largest error over the result's root mean square, given second here, at all but 64 -> 128 channels on 56 x 56 (1.28e-6 and 1.36e-6).  Reduction of 14336 2.2e-7, 1.1e-6 (GemmF32Dma 1.1e-6, 6.6e-6), 4096 1.9e-7, 1.5e-6 (5.8e-7,
 // 4.2e-6), 768 1.6e-7, 9.4e-7 (2.5e-7, 1.5e-6), 128 1.5e-7, 2.8e-6 (GemmTile 2.0e-7, 3.2e-6), 64 9.3e-8, 1.5e-6 (1.4e-7, 2.3e-6); 3 x 3
 // filters on 576 1.1e-7, 8.6e-7 (ConvF32Tile 1.4e-7, 1.0e-6; with four stages 1.5e-7, 1.2e-6), on 1152 1.7e-7, 1.1e-6 (1.9e-7, 1.5e-6).
 // (The five small products summed apart from the large one instead, two sets of registers as well, leave one addition per stage:
 // 1.0e-7 but 1.5e-6 on 576, 4.0e-7, 4.6e-6 on 4096; 1-3 % faster on large tiles, where the sums' additions take the place of other
 // vector work.)  What three bf16 cannot hold is multiplied again with the fp32 MFMAs (see split.h): a wave whose results are not
-// all finite, and the workgroup if a thread has met a value that is more than its parts (the
-// ors that notice it take 0.2 % of the time in the mean, 2 % of 512 and 1024 x 4096 x 4096).  That pass is bound by the fp32 MFMAs and
+// all finite, and the workgroup if a thread has met a value that is more than its parts (the ors
+// that notice it take 0.2 % of the time in the mean, 2 % of 512 and 1024 x 4096 x 4096).  That pass is bound by the fp32 MFMAs and
 // by loads that waves do not share; a tile takes 1.5 - 4 times what it took (us, no such value / one / one in every row of A;
 // in brackets with four dependent k at a time): 1024 x 4096 x 14336 655 / 1630 (7923) / 1740, 1024 x 4096 x 4096 171 / 463 (2573) /
 // 500, 512 x 512 x 128 of 32 heads 20 / 44 (185) / 49, 256 -> 256 on 14 x 14 1285 / 1282 (2957) / 4290 (18392), all on
@@ -36,16 +36,17 @@
 // Reductions of up to four stages are one partial sum: no second set of accumulators, every stage compiled apart, and so nothing
 // loaded or taken apart past the last one (with two stages that was half of it): 512 x 128 x 512 545 -> 499 us.
 //
-// Measured (us, before = GemmF32Dma): 1024 x 4096 x 14336 805 -> 516 (233 TFLOP/s), 1024 x 14336 x 4096 798 -> 546, 1024 x 4096 x
-// 4096 232 -> 156, 512 x 4096 x 14336 461 -> 254, 512 x 4096 x 4096 119 -> 94, 1024 x 768 x 3072 37-41 -> 34.  Smaller tiles than
-// 64 x 64 a workgroup take more time than the fp32 forms: 1024 x 3072 x 768 63 (64 x 96 tiles) against 39.
+// Measured (us, before = GemmF32Dma; uniform operands, two cards): 1024 x 4096 x 14336 828 -> 508-547 (220-237 TFLOP/s), 1024 x 14336 x
+// 4096 812 -> 539-569, 1024 x 4096 x 4096 236 -> 155-166, 512 x 4096 x 14336 460 -> 253-270, 512 x 4096 x 4096 118 -> 90-97, 1024 x 768 x
+// 3072 38 -> 30-31.  Smaller tiles than 64 x 64 a workgroup take more time than the fp32 forms: 1024 x 3072 x 768 63 (64 x 96
+// tiles) against 39.
 //
 // B comes in one of two layouts, as in GemmTile: kPix, planes of n for each k ([K, N] is one image of N pixels); kRows, rows
 // contiguous along k, NIMG independent products.  With a filter of KH x KW taps (kPix) the product is a convolution: A holds the
 // filters as they lie in memory, k counts (channel, tap), and what a column loads for k is its window's element.  All lanes of a
 // load want the same k, so where the element lies from the window's first one comes from a table by a scalar load; padding is a
 // lane whose bit for that tap is set and which therefore reads past the buffer (two vector instructions a load).  Every element
-// is taken apart once for each tap it is under: 256 -> 256 channels on 14 x 14, batch 1024, 1713 -> 1035 us (229 TFLOP/s);
+// is taken apart once for each tap it is under: 256 -> 256 channels on 14 x 14, batch 1024, 1715 -> 1047-1104 us (214-226 TFLOP/s);
 // ConvTiling has the other layers and where the line to the shared tiles lies.  A row tile (kRows: also a column tile) that does not
 // divide the problem starts a tile before its end and leaves its neighbour's results to it: one of the two may be done again.
 #pragma once

@@ -9,9 +9,9 @@
 // multiplied the next one is taken apart; what a group was loaded into takes its next stage as soon as the last block has been.
 //
 // What bounds it is the wave's issue: an MFMA takes 10 clocks of it (it lasts 16) and a vector instruction 4.4, and a 32 x 144 tile
-// has 108 of these and 506 of those a stage where the fp32 form has 144 MFMAs of 32.6: 3300 against 4700 clocks.  On tiles of fewer
-// uses for every element it is no faster: us, fp32 ring before, 32 x 144 512 x 768 x 2304 15.7 -> 13.7 and 1024 x 768 x 2304 32.6 ->
-// 28.4, 32 x 128 1024 x 4096 x 1024 62-65 -> 59, 32 x 96 two workgroups a CU 512 x 768 x 3072 20.8 -> 19.0; but 32 x 96 one
+// has 108 of these and 528 of those a stage where the fp32 form has 144 MFMAs of 32.6: 3400 against 4700 clocks.  On tiles of fewer
+// uses for every element it is no faster: us, fp32 ring before, 32 x 144 512 x 768 x 2304 15.9 -> 14.0-14.7 and 1024 x 768 x 2304 29.3 ->
+// 24.5-25.8, 32 x 128 1024 x 4096 x 1024 61 -> 52-56, 32 x 96 two workgroups a CU 512 x 768 x 3072 20.4 -> 18.4-19.2; but 32 x 96 one
 // workgroup a CU 1024 x 3072 x 768 39.2 -> 39.7, 32 x 64 512 x 4096 x 1024 37.0 -> 36.9, 32 x 48 512 x 3072 x 768 23.2 -> 23.6.  Fused:
 // with the LayerNorm 16.1 -> 14.1-14.5, with the softmax (32 x 96, GELU) 22.6 -> 22.0, with LayerNorm and softmax 19.2 -> 16.6-17.2, with the 56 x 56 convolution 19.9 -> 17.2.  Eight waves
 // of half the k (two a SIMD): 17.1 against 15.8; their partial tiles cost what their overlap gives.
