@@ -37,7 +37,7 @@ DENSE_SPLIT(1024, 14336, 4096, 2, 4, 1, 2, 128)
     BFUSE_KERNEL(bgemm_f32_##B##x##M##x##K##x##N, Bgemm_##B##x##M##x##K##x##N, ({{B, M, K, 1}, 4}), ({{B, N, K, 1}, 4}), ({{B, M, N, 1}, 4}))
 // The bf16 matrix cores (ops_gemm_split.h): 128 x 64 tiles of 32-row waves for the long reductions, 128 x 128 of eight 16-row waves for
 // those of 64 - 128, which are mostly ends: 70 - 94 registers instead of 126 - 168, so that three workgroups a CU load, multiply and
-// store at different times.  us, fp32 matrix cores before and now: 1024 products 512 x 64 x 512 360 -> 303 (32-row waves 311-348), 512 x
+// store at different times.  us on one card, fp32 matrix cores before and now: 1024 products 512 x 64 x 512 360 -> 303 (32-row waves 311-348), 512 x
 // 128 x 512 625 -> 465 (499), 256 x 64 x 256 98 -> 84 (94), 256 x 80 x 256 119 -> 107 (117), 1024 x 64 x 512 705 -> 609 (620), 256 x 256 x
 // 80 134 -> 95 (16-row waves; 32-row 99), 512 x 512 x 128 555 -> 419 (32-row, 128 x 128; 16-row 446), 512 x 512 x 64 334 -> 268 (293), 1024 x
 // 512 x 64 607 -> 518 (573), 256 x 256 x 64 95.6 -> 83 (88).  208 x 208 x 64 gains nothing (75.9 against 74); 208 x 64 x 208, x 80 x 208

@@ -440,7 +440,7 @@ struct ConvTiling {
     // Filters larger than 1 x 1: as a product on the bf16 matrix cores whose second operand is gathered from the images (GemmSplit),
     // on at least two rounds of tiles over the CUs.  The tile is the largest of 256 x 128 (eight waves), 128 x 128, 192 x 64 (four
     // waves, two workgroups a CU), 160 x 128 (ten waves of 16 rows), 96 x 64 (two waves) and 64 x 128 (four of 16 rows) whose rows
-    // divide the channels.  Batch 1024, us, shared tiles before: 256 -> 256 on 14 x 14 1712 -> 1033 (128 x 128: 1.09x that), 512 on 7 x 7
+    // divide the channels.  Batch 1024, us, shared tiles before (all on one card; others hold 0.93-1.00 of the clock): 256 -> 256 on 14 x 14 1712 -> 1033 (128 x 128: 1.09x that), 512 on 7 x 7
     // 1720 -> 1136, 128 on 28 x 28 1692 -> 1122, 448 -> 384 on 8 x 8 1381 -> 882 (192 x 64: 1.08x), 288 -> 384 at stride 2 4153 -> 2838
     // (192 x 128 and x 64: 1.10x), 80 -> 192 on 73 x 73 10209 -> 7393, 192 -> 320 at stride 2 521 -> 378 (128 x 128 on 2.5 tiles: 433; five
     // waves of 32 rows twice 477).  Few channels
