@@ -12,9 +12,8 @@ BFUSE_MODULE_PROLOGUE()
 // softmax: one row per wave, four-wave workgroups (1536 of them)
 using Softmax4 = SoftmaxCausal<12, 512, 4, 1>;
 // GEMM + GELU: 16 x 32 = 512 tiles of 32 x 96, two workgroups per CU, four waves split K = 768 on the bf16 matrix cores, their
-// sums meet in two rounds (24 KB).  196 registers: softmax workgroups run in the places of GEMM workgroups that are done,
-// not beside them; against the fp32 ring of two stages (90 registers, three beside two) 22.0 us against 22.6 fused, 19.4 against 20.7
-// alone.  (168 registers, three workgroups a CU, would spill 10-16.)
+// sums meet in two rounds (24 KB).  154 registers: three workgroups share a CU, so softmax workgroups run beside two of the GEMM's;
+// fused 20.0 us, 18.2 alone (with 196 registers and two workgroups a CU 22.0 and 19.3).
 using GemmFc = GemmF32Dma<512, 3072, 768, 32, 96, 4, kEpiGeluTanh, 2>;
 
 BFUSE_KERNEL(softmax_causal_12x512x512, Softmax4, ({{12, 512, 512, 1}, 4}), ({{1, 1, 1, 1}, 4}), ({{12, 512, 512, 1}, 4}))
@@ -27,7 +26,7 @@ BFUSE_BFUSE_KERNEL(softmax_causal_12x512x512, Softmax4, gemm_gelu_f32_512x768x30
 // the same pair with its dispatch plan as run-time data and persistent workgroups
 BFUSE_BFUSE_RT_KERNEL(softmax_causal_12x512x512, Softmax4, gemm_gelu_f32_512x768x3072, GemmFc)
 
-// alternative GEMM side: the sums meet in one round (48 KB; 19.35 us alone, 21.9 fused)
+// alternative GEMM side: the sums meet in one round (48 KB; 17.6 us alone, 21.0 fused)
 using GemmFcS3 = GemmF32Dma<512, 3072, 768, 32, 96, 4, kEpiGeluTanh, 3>;
 BFUSE_KERNEL(gemm_gelu_f32_512x768x3072_s3, GemmFcS3, ({{512, 768, 1, 1}, 4}), ({{768, 3072, 1, 1}, 4}), ({{512, 3072, 1, 1}, 4}))
 BFUSE_BFUSE_KERNEL(softmax_causal_12x512x512, Softmax4, gemm_gelu_f32_512x768x3072_s3, GemmFcS3, _c256, bfuse::kChunked, 256, 1)

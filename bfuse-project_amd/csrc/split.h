@@ -37,15 +37,21 @@ __device__ __forceinline__ void shared_with_asm(const void* lds)
 #endif
 }
 
-// Two fp32 as three words of two bf16 each (lo in the low halves).  `left` gets the bits of what is left for the last one.
-__device__ __forceinline__ void split2(float lo, float hi, unsigned& p0, unsigned& p1, unsigned& p2, unsigned& left)
+// What is left of two fp32 without their part 0, as words of parts 1 and 2 (lo in the low halves).  `left` gets the bits of what is
+// left for the last one.
+__device__ __forceinline__ void split2_left(float l1, float h1, unsigned& p1, unsigned& p2, unsigned& left)
 {
-    p0 = pack_bf16(lo, hi);
-    const float l1 = lo - __builtin_bit_cast(float, p0 << 16), h1 = hi - __builtin_bit_cast(float, p0 & 0xffff0000u);
     p1 = pack_bf16(l1, h1);
     const unsigned l2 = __builtin_bit_cast(unsigned, l1 - __builtin_bit_cast(float, p1 << 16)), h2 = __builtin_bit_cast(unsigned, h1 - __builtin_bit_cast(float, p1 & 0xffff0000u));
     p2 = __builtin_amdgcn_perm(h2, l2, 0x07060302u);   // their upper halves
     left |= l2 | h2;
+}
+
+// Two fp32 as three words of two bf16 each.
+__device__ __forceinline__ void split2(float lo, float hi, unsigned& p0, unsigned& p1, unsigned& p2, unsigned& left)
+{
+    p0 = pack_bf16(lo, hi);
+    split2_left(lo - __builtin_bit_cast(float, p0 << 16), hi - __builtin_bit_cast(float, p0 & 0xffff0000u), p1, p2, left);
 }
 
 // One bit pattern at a time: a tree of ors over what is taken apart keeps all that was left in registers until its end.
