@@ -399,7 +399,24 @@ struct KernelEntry {
     const char* op_type = "";          // single: the operator's C++ type, spelled so that it can be compiled again
     int smem_bytes = -1;               // single: sizeof(Op::Smem), the LDS the operator's body declares
     bool matrix_cores = false;         // single: the operator declares MATRIX_CORES (its inner loop is a stream of MFMAs)
+    const void* parts_func = nullptr;  // single: the kernel that takes operand `parts_operand` apart before a launch (see Prepares)
+    int parts_operand = -1;
+    unsigned parts_grid = 0, parts_block = 0;
+    size_t parts_bytes = 0;            // the workspace it writes, which the operator then gets in the operand's place
 };
+
+// An operator that wants one of its operands taken apart first (PARTS_OPERAND: 0 = I, 1 = F) declares a kernel for that (Parts):
+// PARTS_GRID workgroups of PARTS_THREADS, which write the PARTS_BYTES of a workspace.  Every launch of the operator, alone or
+// fused, is preceded by it on the same stream, and the operator gets the workspace in the operand's place.
+template <class Op, class = void>
+struct Prepares : std::false_type {};
+template <class Op>
+struct Prepares<Op, std::enable_if_t<(Op::PARTS_OPERAND >= 0)>> : std::true_type {};
+template <class Parts>
+static __global__ __launch_bounds__(Parts::PARTS_THREADS) void take_apart(const void* __restrict__ operand, void* __restrict__ parts)
+{
+    Parts::take_apart(operand, parts);
+}
 
 // The operator type as the compiler spells it, every template argument written out
 // ("bfuse::GemmF32Dma<512, 768, 768, 32, 48, 4, 0, 3>"): what a module of fused kernels built later for a
@@ -452,6 +469,13 @@ KernelEntry make_single_entry(const char* name, const void* func, TensorDesc i, 
     e.op_type = op_type_name<Op>();
     e.smem_bytes = (int)sizeof(typename Op::Smem);
     e.matrix_cores = UsesMatrixCores<Op>::value;
+    if constexpr (Prepares<Op>::value) {
+        e.parts_func = (const void*)&take_apart<typename Op::Parts>;
+        e.parts_operand = Op::PARTS_OPERAND;
+        e.parts_grid = Op::Parts::PARTS_GRID;
+        e.parts_block = Op::Parts::PARTS_THREADS;
+        e.parts_bytes = Op::Parts::PARTS_BYTES;
+    }
     return e;
 }
 

@@ -7,6 +7,7 @@
 #include "ops_ceiling.h"
 #include "ops_conv.h"
 #include "ops_conv_1x1.h"
+#include "ops_conv_split.h"
 #include "ops_conv_tile.h"
 #include "ops_gemm_bf16.h"
 #include "ops_gemm_f32.h"
@@ -256,6 +257,24 @@ BFUSE_BFUSE_KERNEL(selftest_gemm_split_r, Narrow<GemmSp_r>, layernorm_8x256, Lay
 BFUSE_BFUSE_KERNEL(selftest_gemm_split_a, GemmSp_a, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
 BFUSE_HFUSE_KERNEL(selftest_gemm_split_e, GemmSp_e, bias_relu_4096, BiasReluS)
 BFUSE_HFUSE_KERNEL(selftest_gemm_split_f, GemmSp_f, conv3x3_f32_32x12x12_32, ConvS2)
+
+// The convolution from a patch taken apart once: pixels that run on into the next images and past the batch, rectangles past an image's
+// edges with whole and with broken quads of pixels, one to four groups of channels, units that a thread does twice, two waves over the columns.
+// <CI, CO, H, W, padding, images, 16-row blocks of a wave, waves over rows, over columns, pixels, width>
+#define CONV_PATCH_TEST(TAG, CI, CO, H, W, P, N, ...)                                                              \
+    using ConvP_##TAG = SwapOperands<ConvSplit<CI, CO, H, W, 3, 3, 1, P, N, __VA_ARGS__>>;                          \
+    BFUSE_KERNEL(selftest_conv_split_##TAG, ConvP_##TAG, ({{N, CI, H, W}, 4}), ({{CO, CI, 3, 3}, 4}), ({{N, CO, H - 2 + 2 * P, W - 2 + 2 * P}, 4}))
+CONV_PATCH_TEST(a, 64, 64, 7, 7, 1, 5, 2, 2, 1, 96, 0)           // 245 pixels of five images in three tiles
+CONV_PATCH_TEST(b, 32, 96, 13, 15, 1, 2, 2, 3, 1, 144, 12)       // one group, rectangles of 12 x 12 on 13 x 15
+CONV_PATCH_TEST(c, 96, 256, 30, 18, 0, 2, 2, 4, 1, 112, 28)      // rectangles of 28 on 16 columns, two row tiles
+CONV_PATCH_TEST(d, 32, 32, 20, 33, 1, 2, 2, 1, 2, 224, 16)
+CONV_PATCH_TEST(e, 128, 128, 10, 10, 0, 4, 2, 4, 2, 224, 0)      // 256 pixels of four images
+CONV_PATCH_TEST(f, 64, 64, 9, 9, 2, 3, 2, 2, 1, 112, 16)         // padding of two
+CONV_PATCH_TEST(g, 96, 128, 5, 5, 1, 9, 2, 4, 1, 128, 0)         // a tile of six images
+BFUSE_BFUSE_KERNEL(selftest_conv_split_a, ConvP_a, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
+BFUSE_HFUSE_KERNEL(selftest_conv_split_b, ConvP_b, bias_relu_4096, BiasReluS)
+BFUSE_HFUSE_KERNEL(selftest_conv_split_d, ConvP_d, conv3x3_f32_32x12x12_32, ConvS2)
+BFUSE_BFUSE_RT_KERNEL(selftest_conv_split_f, ConvP_f, layernorm_8x256, LayerNormS)
 
 // The split-K product on the bf16 matrix cores: a trailing 16-column group and GELU in one round, two waves in two rounds, one stage.
 using GemmSpk_a = GemmF32Dma<64, 288, 256, 32, 144, 4, kEpiGeluTanh>;

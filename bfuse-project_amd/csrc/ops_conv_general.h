@@ -346,8 +346,13 @@ struct ConvF32Lds {
 
 // An operator with its first two operands exchanged: a 1x1 / stride 1 convolution is the product
 // Wt[CO, CI] . X[CI, H*W], i.e. a GEMM whose first operand is the convolution's SECOND (the weights).
+template <class Op, class = void>
+struct swapped_operand : std::integral_constant<int, -1> {};
+template <class Op>
+struct swapped_operand<Op, std::enable_if_t<(Op::PARTS_OPERAND >= 0)>> : std::integral_constant<int, 1 - Op::PARTS_OPERAND> {};
 template <class Op>
 struct SwapOperands : Op {
+    static constexpr int PARTS_OPERAND = swapped_operand<Op>::value;
     template <class Sync>
     __device__ static __forceinline__ void run(int vblock, int tid, typename Op::Smem& sm, const void* I, const void* F,
                                                void* O, Sync sync)

@@ -26,6 +26,7 @@
 #include "dispatch.h"
 #include "ops_conv_1x1.h"
 #include "ops_conv_general.h"
+#include "ops_conv_split.h"
 #include "ops_conv_tile.h"
 #include "ops_gemm_split.h"
 #include "ops_gemm_tile.h"
@@ -314,6 +315,26 @@ struct NarrowOf<ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, KS, NIMG, kSplitF
     using type = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, (KS > 8 && KS % 2 == 0 ? KS / 2 : KS), NIMG, kSplitForm>;
 };
 
+// The product from a patch taken apart once (ConvSplit) under that name as well: BM output channels, 32 a wave, and 16 PB pixels, TW wide
+// (0: that follow each other).  (The tile it derives from says only that this is a shared tile.)
+constexpr int kPatchForm = 33;
+template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int BM, int PB, int TW, int NIMG>
+struct ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, TW, NIMG, kPatchForm> : ConvF32Tile<CI, CO, H, W, KH, KW, S, P, BM, 128, 1, NIMG> {
+    using Form = SwapOperands<ConvSplit<CI, CO, H, W, KH, KW, S, P, NIMG, 2, BM / 32, (PB > 9 ? 2 : 1), 16 * PB, TW>>;
+    using Parts = typename Form::Parts;
+    static constexpr int PARTS_OPERAND = Form::PARTS_OPERAND;
+    static constexpr long long TILES = Form::TILES;
+    static constexpr bool FITS = Form::FITS;
+    static constexpr Dims3 GRID = Form::GRID, BLOCK = Form::BLOCK;
+    static constexpr int THREADS = Form::THREADS, MIN_BARRIERS = Form::MIN_BARRIERS;
+    using Smem = typename Form::Smem;
+    template <class Sync>
+    __device__ static __forceinline__ void run(int vblock, int tid, Smem& sm, const void* I, const void* F, void* O, Sync sync)
+    {
+        Form::run(vblock, tid, sm, I, F, O, sync);
+    }
+};
+
 // The tiling the library gives a convolution it has no hand-picked one for: as many output channels per
 // workgroup as keep the filter fragments of a wave within ~72 registers (the staged patch is shared by all
 // of them), 64 pixels (or the whole image when it has fewer), and as many waves over the channel groups as
@@ -440,7 +461,7 @@ struct ConvTiling {
     // Filters larger than 1 x 1: as a product on the bf16 matrix cores whose second operand is gathered from the images (GemmSplit),
     // on at least two rounds of tiles over the CUs.  The tile is the largest of 256 x 128 (eight waves), 128 x 128, 192 x 64 (four
     // waves, two workgroups a CU), 160 x 128 (ten waves of 16 rows), 96 x 64 (two waves) and 64 x 128 (four of 16 rows) whose rows
-    // divide the channels.  Batch 1024, us, shared tiles before (all on one card; others hold 0.93-1.00 of the clock): 256 -> 256 on 14 x 14 1712 -> 1033 (128 x 128: 1.09x that), 512 on 7 x 7
+    // divide the channels.  (Those at stride 1 have since gone on to the patch above, except channels that are no groups of 32.)  Batch 1024, us, shared tiles before (all on one card; others hold 0.93-1.00 of the clock): 256 -> 256 on 14 x 14 1712 -> 1033 (128 x 128: 1.09x that), 512 on 7 x 7
     // 1720 -> 1136, 128 on 28 x 28 1692 -> 1122, 448 -> 384 on 8 x 8 1381 -> 882 (192 x 64: 1.08x), 288 -> 384 at stride 2 4153 -> 2838
     // (192 x 128 and x 64: 1.10x), 80 -> 192 on 73 x 73 10209 -> 7393, 192 -> 320 at stride 2 521 -> 378 (128 x 128 on 2.5 tiles: 433; five
     // waves of 32 rows twice 477).  Few channels
@@ -456,6 +477,52 @@ struct ConvTiling {
         if constexpr (T > 1 && T < 31 && CI % 16 == 0 && CI * T <= 32768 && CO % SBM == 0 && !(SBM == 64 && S == 2))
             return split::FITS && split::TILES >= 512;
         return false;
+    }
+    // 3 x 3 filters at stride 1 on whole groups of 32 channels take the images apart once for all taps (ConvSplit, which has the figures: 0.71-0.92 of
+    // split's time on eleven layers, 0.75-0.89 on ten others from 14 x 14 to 14 x 300), where a tile of the most output channels up to 128 that divide theirs fits twice
+    // into a CU's LDS with at most 15 % of it outside the images: of 128, 112 or 96 consecutive pixels, 28 x 4, 16 x 7 and 12 x 12, the one that
+    // computes least besides.  Measured: 14 x 14 on 112 900 us, on 96 926; 7 x 7 on 96 972, on 112 (one tile a CU) 1062; 8 x 8 on 128 755, on 64 793; 35 x 35 on 12 x 12
+    // 702, on 12 x 8 760, on 36 x 4 806; 56 x 56 on 28 x 4 1242, on 16 x 8 1372; 147 x 147 on 16 x 7 4338, on 12 x 12 4424.  Where
+    // none of these does (26 x 26), eight waves on 224 consecutive pixels, one tile a CU (1718 against split's 1887; 28 x 4 of 16 % outside 1766).
+    // 32 output channels: two waves on 224 pixels.
+    static constexpr int QBM = CO % 128 == 0 ? 128 : CO % 96 == 0 ? 96 : CO % 64 == 0 ? 64 : 32;
+    template <int PB, int TW> using patch = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, QBM, PB, TW, NIMG, kPatchForm>;
+    // what a tile costs a pixel: those outside the image, and a sixteenth part of a wave's columns that every tile takes besides
+    template <int PB, int TW>
+    static constexpr double patch_cost()
+    {
+        using F = patch<PB, TW>;
+        if constexpr (F::FITS && (PB != 9 || CI <= 128)) {   // (nine blocks of columns take all registers there are)
+            const double pixels = 16.0 * PB * (double)F::TILES / (CO / QBM) / ((double)OHW * NIMG);
+            if (2 * (int)sizeof(typename F::Smem) <= 163840 && pixels <= 1.15) return pixels * (1 + 1.0 / (PB > 9 ? PB / 2 : PB));
+        }
+        return 1e9;
+    }
+    static constexpr int patch_form()     // 100 TW + PB, or 0
+    {
+        if constexpr (KH == 3 && KW == 3 && S == 1 && CI % 32 == 0 && CO % 32 == 0 && CI * T <= 32768 && (long long)OHW * NIMG >= 512LL * 128 * QBM / CO) {
+            if constexpr (QBM == 32) {
+                const int f[] = {14, 1614, 2814};
+                const double c[] = {patch_cost<14, 0>(), patch_cost<14, 16>(), patch_cost<14, 28>()};
+                return least(f, c);
+            } else {
+                const int f[] = {8, 7, 6, 2807, 1607, 1209};
+                const double c[] = {patch_cost<8, 0>(), patch_cost<7, 0>(), patch_cost<6, 0>(), patch_cost<7, 28>(), patch_cost<7, 16>(), patch_cost<9, 12>()};
+                const int best = least(f, c);
+                if constexpr (QBM == 128)
+                    if (best == 0 && patch<14, 0>::FITS) return 14;
+                return best;
+            }
+        }
+        return 0;
+    }
+    template <int N>
+    static constexpr int least(const int (&f)[N], const double (&c)[N])
+    {
+        int best = 0;
+        for (int i = 1; i < N; ++i)
+            if (c[i] < c[best]) best = i;
+        return c[best] < 1e8 ? f[best] : 0;
     }
     // 1 x 1 filters on 256 and more channels likewise, also on 224 x 128 tiles (seven waves).  us, GemmTile before: 768 -> 192 on
     // 17 x 17 641 -> 525 (twelve waves of 16 rows 0.96x that, but no register is left beside twelve waves), 160 573 -> 447, 128 455 -> 344,
@@ -473,10 +540,11 @@ struct ConvTiling {
     }
     template <int FORM, class Else> struct pick { using type = Else; };
     template <class Else> struct pick<3, Else> { using type = split; };
+    template <class Else> struct pick<5, Else> { using type = patch<patch_form() % 100, patch_form() / 100>; };
     template <class Else> struct pick<4, Else> { using type = SwapOperands<split_product>; };
     template <class Else> struct pick<1, Else> { using type = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, TBM, TPB, 4, NIMG, TWM>; };
     template <class Else> struct pick<2, Else> { using type = SwapOperands<product>; };
-    using type = typename pick<is_split() ? 3 : is_split_product() ? 4 : is_product() ? 2 : tiled(TPB) ? 1 : 0, std::conditional_t<STREAM, Conv1x1F32<CI, CO, H, W, S, stream_bm(), 4, NIMG>, held>>::type;
+    using type = typename pick<(patch_form() > 0) ? 5 : is_split() ? 3 : is_split_product() ? 4 : is_product() ? 2 : tiled(TPB) ? 1 : 0, std::conditional_t<STREAM, Conv1x1F32<CI, CO, H, W, S, stream_bm(), 4, NIMG>, held>>::type;
 };
 template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int NIMG = 1>
 using ConvF32Auto = typename ConvTiling<CI, CO, H, W, KH, KW, S, P, NIMG>::type;

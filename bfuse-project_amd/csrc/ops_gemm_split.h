@@ -46,8 +46,8 @@
 // filters as they lie in memory, k counts (channel, tap), and what a column loads for k is its window's element.  All lanes of a
 // load want the same k, so where the element lies from the window's first one comes from a table by a scalar load; padding is a
 // lane whose bit for that tap is set and which therefore reads past the buffer (two vector instructions a load).  Every element
-// is taken apart once for each tap it is under: 256 -> 256 channels on 14 x 14, batch 1024, 1715 -> 1047-1104 us (214-226 TFLOP/s);
-// ConvTiling has the other layers and where the line to the shared tiles lies.  A row tile (kRows: also a column tile) that does not
+// is taken apart once for each tap it is under: 256 -> 256 channels on 14 x 14, batch 1024, 1715 -> 1047-1104 us (214-226 TFLOP/s; 3 x 3 filters
+// at stride 1 do without that in ConvSplit, 901 us); ConvTiling has the other layers and where the line to the shared tiles lies.  A row tile (kRows: also a column tile) that does not
 // divide the problem starts a tile before its end and leaves its neighbour's results to it: one of the two may be done again.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -60,6 +60,58 @@
 #include "wave.h"
 
 namespace bfuse {
+
+// The parts of filters [M, K] of fp32, k = (channel, tap), as a kernel of its own leaves them in a workspace (Prepares, fuse.h) for one that
+// multiplies them (ConvSplit): taps are put behind the channels, 32 of which are a stage's k, stage (channels, tap); for every 16 rows and
+// stage the three parts one after the other, each as the MFMA's operand, 16 bytes a lane.  In front of them: where the filters
+// themselves lie, and a word for every 16 rows and 32 channels that is not zero if a value is more than its parts.
+// One wave takes a stage apart at a time; a lane's values are TAPS apart, so a wave's loads touch 16 rows, of which the other taps' then
+// come from the caches: 256 x 2304 in 5 us.
+template <int M, int K, int TAPS>
+struct SplitParts {
+    static_assert(M % 16 == 0 && K % (32 * TAPS) == 0, "parts");
+    static constexpr int PARTS_THREADS = 256;
+    static constexpr int STAGES = K / 32, CHUNKS = STAGES / TAPS;
+    static constexpr int BLOCK_BYTES = STAGES * 3072, HEAD = (64 + M / 16 * CHUNKS * 4 + 1023) / 1024 * 1024;
+    static constexpr unsigned PARTS_GRID = M / 16 * CHUNKS;
+    static constexpr size_t PARTS_BYTES = (size_t)HEAD + (size_t)(M / 16) * BLOCK_BYTES;
+
+    __device__ static __forceinline__ const void* source(const void* parts) { return *static_cast<const void* const*>(parts); }
+    __device__ static __forceinline__ const unsigned char* block(const void* parts, int b) { return static_cast<const unsigned char*>(parts) + HEAD + (size_t)b * BLOCK_BYTES; }
+    // Whether a value of 16-row blocks b .. b + n - 1 is more than its parts, some lane's share of that.
+    __device__ static __forceinline__ unsigned inexact(const void* parts, int b, int n, int lane)
+    {
+        const unsigned* const words = reinterpret_cast<const unsigned*>(static_cast<const unsigned char*>(parts) + 64) + b * CHUNKS;
+        unsigned any = 0;
+        for (int i = lane; i < n * CHUNKS; i += 64) any |= words[i];
+        return any;
+    }
+    __device__ static __forceinline__ void take_apart(const void* operand, void* parts)
+    {
+        const int b = blockIdx.x / CHUNKS, chunk = blockIdx.x % CHUNKS, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+        const float* const row = static_cast<const float*>(operand) + (size_t)(16 * b + (lane & 15)) * K;
+        __shared__ unsigned more;
+        if (threadIdx.x == 0) more = 0;
+        if (blockIdx.x == 0 && threadIdx.x == 0) *static_cast<const void**>(parts) = operand;
+        __syncthreads();
+        unsigned left = 0;
+        for (int s = chunk * TAPS + wave; s < (chunk + 1) * TAPS; s += PARTS_THREADS / 64) {
+            float x[8];
+            const int k = (chunk * 32 + (lane >> 4) * 8) * TAPS + s % TAPS;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = row[k + e * TAPS];
+            unsigned p[3][4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) split2(x[2 * j], x[2 * j + 1], p[0][j], p[1][j], p[2][j], left);
+            unsigned char* const to = static_cast<unsigned char*>(parts) + HEAD + (size_t)b * BLOCK_BYTES + (size_t)s * 3072 + lane * 16;
+#pragma unroll
+            for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x4*>(to + q * 1024) = u32x4{p[q][0], p[q][1], p[q][2], p[q][3]};
+        }
+        if (split_inexact(left)) more = 1;
+        __syncthreads();
+        if (threadIdx.x == 0) reinterpret_cast<unsigned*>(static_cast<unsigned char*>(parts) + 64)[b * CHUNKS + chunk] = more;
+    }
+};
 
 // M, K, H, W, S, NIMG, LAYOUT: as in GemmTile.  TM 16-row blocks of a wave, WR waves over the rows and WN over the BN columns, KG
 // groups of such waves over the stages.  LEAN: one set of A's parts, taken apart at the top of the stage, instead of the next one's
@@ -78,10 +130,13 @@ struct GemmSplit {
     static constexpr int MT = (M + BM - 1) / BM;
     static constexpr int NT = LAYOUT == kRows ? (W + BN - 1) / BN : (int)(((long long)OHWP * NIMG + BN - 1) / BN);
     static constexpr int NIMAGES = LAYOUT == kRows ? 1 : (BN + OHWP - 2) / OHWP + 1;   // images a tile can touch
-    static constexpr int NUJ = (4 * BN + GT - 1) / GT;                           // units (a column's eight k) of a thread and stage
-    // a thread's units lie the same way apart for all threads (kRows: GT / 4 columns, kPix: GT / BN octets of one column), so that
+    // Columns of an octet as the units (a column's eight k) are dealt to the threads: whole waves of them for filters larger than
+    // 1 x 1, a wave's units being one octet's.
+    static constexpr int BU = T > 1 ? (BN + 63) / 64 * 64 : BN;
+    static constexpr int NUJ = (4 * BU + GT - 1) / GT;                           // units of a thread and stage
+    // a thread's units lie the same way apart for all threads (kRows: GT / 4 columns, kPix: GT / BU octets of one column), so that
     // one address serves them all
-    static constexpr bool EVEN = 4 * BN % GT == 0 && GT % (LAYOUT == kRows ? 4 : BN) == 0;
+    static constexpr bool EVEN = 4 * BU % GT == 0 && GT % (LAYOUT == kRows ? 4 : BU) == 0;
     static constexpr int NUB = EVEN ? 1 : NUJ;
     static_assert(BN % (16 * WN) == 0 && K % 8 == 0 && NS % KG == 0 && M >= BM && (LAYOUT == kPix || (W >= BN && H == 1 && S == 1)), "tile");
     // 31-bit offsets; padding is read through one that lies past the buffer
@@ -111,9 +166,10 @@ struct GemmSplit {
         }
     };
     __device__ static constexpr Taps TAPS{};
-    static_assert(T == 1 || (LAYOUT == kPix && BN % 64 == 0 && T < 31 && K % T == 0), "a wave's units are one octet's");
+    static_assert(T == 1 || (LAYOUT == kPix && BN >= 64 && T < 31 && K % T == 0), "taps");
 
     // (column tile, row tile), dealt so that the row tiles of one column tile follow each other on one XCD
+    template <int NT = GemmSplit::NT>
     __device__ static __forceinline__ void tile_of(int vblock, int& nt, int& mt)
     {
         constexpr int PER_XCD = NT / 8;
@@ -127,6 +183,30 @@ struct GemmSplit {
             nt = 8 * PER_XCD + rem / MT;
             mt = rem % MT;
         }
+    }
+
+    static constexpr unsigned B_K = LAYOUT == kRows ? 4 : HW * 4;                   // bytes from one k of a column to the next
+    // Offset of B(0, column c of the tile); past the buffer if there is none.  Filters larger than 1 x 1: of its window's first
+    // element, counted from P rows and columns before the images; `outside` gets a bit for every tap that is in the padding.
+    // (n_lo, v0: the tile's first image and its first column in that one)
+    __device__ static __forceinline__ unsigned offset_of(int c, int v0, int n_lo, unsigned& outside)
+    {
+        if constexpr (LAYOUT == kRows) return (unsigned)(c * K * 4);
+        const int v = v0 + c, img = v / OHWP, p = v % OHWP, y = (p / OW) * S, x = (p % OW) * S;
+        const bool in = p < OHW && n_lo + img < NIMG;
+        outside = in ? 0x80000000u : ~0u;
+        if constexpr (P > 0)
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+                if (y + t / KW < P || y + t / KW >= H + P || x + t % KW < P || x + t % KW >= W + P) outside |= 1u << t;
+        return in ? (unsigned)((img * CI * HW + y * W + x) * 4) : 0x7fffffffu;
+    }
+    __device__ static __forceinline__ auto rows_of(const float* A, int m0) { return __builtin_amdgcn_make_buffer_rsrc((void*)(A + (size_t)m0 * K), 0, BM * K * 4, 0x00020000); }
+    __device__ static __forceinline__ auto columns_of(const float* B, long long n0, int n_lo)
+    {
+        return __builtin_amdgcn_make_buffer_rsrc(
+            (void*)(LAYOUT == kRows ? B + (size_t)n0 * K : B + (size_t)n_lo * CI * HW - (P * W + P)), 0,
+            LAYOUT == kRows ? BN * K * 4 : ((NIMG - n_lo < NIMAGES ? NIMG - n_lo : NIMAGES) * CI * HW + P * W + P) * 4, 0x00020000);
     }
 
     template <class Sync>
@@ -162,32 +242,18 @@ struct GemmSplit {
         const int n_lo = LAYOUT == kRows ? 0 : (int)(n0 / OHWP);                 // kPix: first image of the tile
         const int v0 = (int)(n0 - (long long)n_lo * OHWP);
 
-        // Offset of B(0, column c of the tile); past the buffer if there is none.  Filters larger than 1 x 1: of its window's first
-        // element, counted from P rows and columns before the images; `outside` gets a bit for every tap that is in the padding.
-        auto column = [&](int c, unsigned& outside) -> unsigned {
-            if constexpr (LAYOUT == kRows) return (unsigned)(c * K * 4);
-            const int v = v0 + c, img = v / OHWP, p = v % OHWP, y = (p / OW) * S, x = (p % OW) * S;
-            const bool in = p < OHW && n_lo + img < NIMG;
-            outside = in ? 0x80000000u : ~0u;
-            if constexpr (P > 0)
-#pragma unroll
-                for (int t = 0; t < T; ++t)
-                    if (y + t / KW < P || y + t / KW >= H + P || x + t % KW < P || x + t % KW >= W + P) outside |= 1u << t;
-            return in ? (unsigned)((img * CI * HW + y * W + x) * 4) : 0x7fffffffu;
-        };
-        constexpr unsigned B_K = LAYOUT == kRows ? 4 : HW * 4;                   // bytes from one k of a column to the next
-        const auto ar = __builtin_amdgcn_make_buffer_rsrc((void*)(A + (size_t)m0 * K), 0, BM * K * 4, 0x00020000);
-        const auto br = __builtin_amdgcn_make_buffer_rsrc(
-            (void*)(LAYOUT == kRows ? B + (size_t)n0 * K : B + (size_t)n_lo * CI * HW - (P * W + P)), 0,
-            LAYOUT == kRows ? BN * K * 4 : ((NIMG - n_lo < NIMAGES ? NIMG - n_lo : NIMAGES) * CI * HW + P * W + P) * 4, 0x00020000);
+        auto column = [&](int c, unsigned& outside) { return offset_of(c, v0, n_lo, outside); };
+        const auto ar = rows_of(A, m0);
+        const auto br = columns_of(B, n0, n_lo);
         const unsigned a_voff = (unsigned)(((wr * TM * 16 + li) * K + 8 * kq) * 4);
         unsigned b_voff[NUB], b_out[NUB];
         int b_lds[NUB], b_k[NUB];
 #pragma unroll
         for (int j = 0; j < NUB; ++j) {
-            // threads past the last unit do one of the first ones again: the same values to the same place.  kRows: four lanes
+            // threads past the last unit, or the last column of an octet, do another one again: the same values to the same place.  kRows: four lanes
             // read 128 consecutive bytes of a row; kPix: 64 lanes 64 consecutive columns of a plane
-            const int u = (j * GT + gt) % (4 * BN), o = LAYOUT == kRows ? u & 3 : u / BN, c = LAYOUT == kRows ? u >> 2 : u % BN;
+            const int u = (j * GT + gt) % (4 * BU), o = LAYOUT == kRows ? u & 3 : u / BU, cu = LAYOUT == kRows ? u >> 2 : u % BU;
+            const int c = BU > BN && cu >= BN ? cu - 64 : cu;
             const unsigned v = column(c, b_out[j]);
             b_voff[j] = T > 1 || v == 0x7fffffffu ? v : v + 8 * o * B_K;
             b_k[j] = T > 1 ? __builtin_amdgcn_readfirstlane(8 * o) : 0;
@@ -207,7 +273,7 @@ struct GemmSplit {
 #pragma unroll
             for (int h = 0; h < 2; ++h) ra[tm][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ar, v + (T > 1 ? 0 : h * 16), s * 128 + tm * 16 * K * 4 + (T > 1 ? h * 16 : 0), 0));
         };
-        auto lds_of = [&](int j) { return EVEN ? b_lds[0] + j * (LAYOUT == kRows ? GT / 4 : GT) * 16 : b_lds[j]; };
+        auto lds_of = [&](int j) { return EVEN ? b_lds[0] + j * (LAYOUT == kRows ? GT / 4 : GT / BU * BN) * 16 : b_lds[j]; };
         auto load_b = [&](int j, int s) {
             const int i = EVEN ? 0 : j;
             const unsigned v = T == 1 && TAIL != 0 && s == NS - 1 && lds_of(j) >= TAIL / 8 * BN * 16 ? 0x7fffffffu : b_voff[i];
@@ -221,14 +287,14 @@ struct GemmSplit {
             } else if constexpr (T > 1) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    const unsigned at = TAPS.at[s * 32 + b_k[i] + (EVEN ? 8 * j * (GT / BN) : 0) + e];
+                    const unsigned at = TAPS.at[s * 32 + b_k[i] + (EVEN ? 8 * j * (GT / BU) : 0) + e];
                     // all ones (past the buffer) if this tap's bit is set; without padding only the last stage has such
                     const unsigned o = P > 0 || TAIL != 0 ? (unsigned)__builtin_amdgcn_sbfe((int)b_out[i], at, 1) : 0u;
                     rb[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(br, v | o, (at >> 5) * 4, 0));
                 }
             } else {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) rb[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(br, v, (s * 32 + (EVEN ? 8 * j * (GT / BN) : 0) + e) * B_K, 0));
+                for (int e = 0; e < 8; ++e) rb[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(br, v, (s * 32 + (EVEN ? 8 * j * (GT / BU) : 0) + e) * B_K, 0));
             }
         };
         shared_with_asm(sm.t);
@@ -388,6 +454,25 @@ struct GemmSplit {
 #pragma unroll
                     for (int q = 1; q < KG; ++q) acc[tm][b] += red[((q - 1) * WR * WN * TM * TN + tm * TN + b) * 64];
         }
+        finish(acc, again, A, B, C, m0, mt, n0, nt, n_lo, wr, wn, ei, eq, column, [&](int col, int& img, int& p) { return quad_at(v0 + col, n_lo, img, p); });
+    }
+
+    // kPix: the image and pixel of column v counted from image n_lo, and how many of it and the next three are one image's.
+    __device__ static __forceinline__ int quad_at(int v, int n_lo, int& img, int& p)
+    {
+        img = n_lo + v / OHWP;
+        p = v % OHWP;
+        return img >= NIMG ? 0 : OHW - p < 4 ? OHW - p : 4;
+    }
+
+    // What follows the sums of a wave: the results that three parts do not give are done again, and all are stored.
+    // offset(c, outside): as offset_of, for column c of the tile; quad(c, img, p): as quad_at; QUADS: four columns are one image's and aligned.
+    template <bool QUADS = OHW % 4 == 0, class Offset, class Quad>
+    __device__ static __forceinline__ void finish(f32x4 (&acc)[TM][TN], bool again, const float* A, const float* B, float* __restrict__ C, int m0, int mt, long long n0, int nt, int n_lo,
+                                                  int wr, int wn, int ei, int eq, Offset offset, Quad quad)
+    {
+        const auto ar = rows_of(A, m0);
+        const auto br = columns_of(B, n0, n_lo);
         // Which 16-row blocks are done again: all of the tile's, or the wave's with a result that is not finite (by block, so that the
         // bits do not depend on how many blocks a wave has).
         bool redo[TM], any = false;
@@ -407,7 +492,7 @@ struct GemmSplit {
             unsigned bo[TN], outside[TN];
 #pragma unroll
             for (int b = 0; b < TN; ++b) {
-                const unsigned c = column((wn * TN + b) * 16 + ei, outside[b]);
+                const unsigned c = offset((wn * TN + b) * 16 + ei, outside[b]);
                 bo[b] = LAYOUT == kRows ? c + eq * 16 : T > 1 || c == 0x7fffffffu ? c : c + eq * B_K;
             }
 #pragma unroll
@@ -505,23 +590,23 @@ struct GemmSplit {
                     if (own_row(m) && (W % BN == 0 || n0 + col >= nt * BN)) *reinterpret_cast<f32x4*>(C + (size_t)m * W + n0 + col) = acc[tm][b];
                 }
             } else {
-                const int vc = v0 + col, img = n_lo + vc / OHWP, p = vc % OHWP;
-                if (img < NIMG) {
+                int img, p;
+                const int n = quad(col, img, p);
+                if (n > 0) {
                     float* __restrict__ y = C + ((size_t)img * M + m0 + wr * TM * 16 + ei) * OHW + p;
-                    const bool whole = OHW % 4 == 0 || p + 4 <= OHW;
 #pragma unroll
                     for (int tm = 0; tm < TM; ++tm) {
                         if (!own_row(m0 + (wr * TM + tm) * 16 + ei)) continue;
                         float* const d = y + (size_t)(tm * 16) * OHW;
                         const f32x4 o = acc[tm][b];
-                        if constexpr (OHW % 4 == 0) {
+                        if constexpr (QUADS) {
                             *reinterpret_cast<f32x4*>(d) = o;
-                        } else if (whole) {
+                        } else if (n == 4) {
                             *reinterpret_cast<f32x4u*>(d) = f32x4u{o[0], o[1], o[2], o[3]};
                         } else {
 #pragma unroll
                             for (int e = 0; e < 3; ++e)
-                                if (p + e < OHW) d[e] = o[e];
+                                if (e < n) d[e] = o[e];
                         }
                     }
                 }

@@ -78,6 +78,8 @@ struct Side {
     size_t bytes[3] = {0, 0, 0};
     int elem[3] = {4, 4, 4};
     hipStream_t stream = nullptr;                // S1 / S2
+    void* parts = nullptr;                       // workspace of operators that want an operand taken apart: made for the first of them,
+    size_t parts_bytes = 0;                      // never smaller again while the side lives
     bool live = false;
 };
 
@@ -200,6 +202,11 @@ int fini_side(int idx)
     Side& s = g.side[idx];
     if (!s.live) return fail(BFUSE_ERR_STATE, "kernel%d is not initialized", idx + 1);
     HIP_TRY(hipStreamDestroy(s.stream));
+    if (s.parts) {
+        HIP_TRY(hipFree(s.parts));
+        s.parts = nullptr;
+        s.parts_bytes = 0;
+    }
     for (int i = 2; i >= 0; --i) {
         HIP_TRY(hipFree(s.buf[i]));
         s.buf[i] = nullptr;
@@ -314,15 +321,24 @@ int check_launch(const void* func, const unsigned* grid, const unsigned* block, 
     return BFUSE_OK;
 }
 
-// Buffers an operator touches must be at least as large as the shapes its kernel was built for.
+// Buffers an operator touches must be at least as large as the shapes its kernel was built for.  The workspace for an operand that is
+// taken apart is made here, by the first check of such an operator and so before any of its launches is enqueued or captured.
 int check_buffers(const Launchable& l, int k, int idx)
 {
-    const Side& s = g.side[idx];
+    Side& s = g.side[idx];
     if (!s.live) return fail(BFUSE_ERR_STATE, "kernel%d is not initialized", idx + 1);
     for (int i = 0; i < 3; ++i)
         if (s.bytes[i] < l.need[k][i])
             return fail(BFUSE_ERR_ARG, "%s needs %zu bytes for tensor %d, side %d holds %zu", l.side[k]->name.c_str(), l.need[k][i], i,
                         idx + 1, s.bytes[i]);
+    if (const size_t need = l.side[k]->parts_bytes; need > s.parts_bytes) {
+        DevBuf made;
+        HIP_TRY(hipMalloc(&made.p, need));
+        if (s.parts) HIP_TRY(hipFree(s.parts));   // waits for the launches that use it
+        s.parts = made.p;
+        made.p = nullptr;
+        s.parts_bytes = need;
+    }
     return BFUSE_OK;
 }
 int check_side_fits(const void* func, int idx)
@@ -344,11 +360,30 @@ int check_fused_fits(const void* func, const int* sides = nullptr)
     return BFUSE_OK;
 }
 
+// Takes an operand of this operator apart if it wants that, and puts the workspace in the operand's place among its three arguments.
+// The first kernel of a launch records its start event.
+int launch_parts(const KernelEntry* e, int idx, void** args, hipStream_t stream, hipEvent_t& ev0)
+{
+    if (!e || !e->parts_func) return BFUSE_OK;
+    Side& s = g.side[idx];
+    void* own[2] = {args[e->parts_operand], &s.parts};
+    if (ev0)
+        HIP_TRY(hipExtLaunchKernel(e->parts_func, dim3(e->parts_grid), dim3(e->parts_block), own, 0, stream, ev0, nullptr, 0));
+    else
+        HIP_TRY(hipLaunchKernel(e->parts_func, dim3(e->parts_grid), dim3(e->parts_block), own, 0, stream));
+    g_in_flight.add();
+    ev0 = nullptr;
+    args[e->parts_operand] = &s.parts;
+    return BFUSE_OK;
+}
+
 int launch3(const void* func, const unsigned* grid, const unsigned* block, int idx, hipStream_t stream,
             hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr)
 {
     Side& s = g.side[idx];
     void* args[3] = {&s.buf[0], &s.buf[1], &s.buf[2]};
+    if (s.parts)   // (a side that has had such an operator)
+        if (int rc = launch_parts(entry_of(func), idx, args, stream, ev0)) return rc;
     if (ev0 || ev1)
         HIP_TRY(hipExtLaunchKernel(func, d3(grid), d3(block), args, 0, stream, ev0, ev1, 0));
     else
@@ -364,6 +399,9 @@ int launch_fused(const void* func, const unsigned* grid, const unsigned* block, 
     void* args[3 * kMaxKernels + 1] = {};
     for (int k = 0; k < n; ++k)
         for (int i = 0; i < 3; ++i) args[3 * k + i] = &g.side[sides[k]].buf[i];
+    for (int k = 0; k < n; ++k)
+        if (g.side[sides[k]].parts)
+            if (int rc = launch_parts(launchable(func)->side[k], sides[k], args + 3 * k, stream, ev0)) return rc;
     // a run-time-plan kernel takes its installed plan by value as its last argument
     auto it = installed_plans().find(func);
     if (it != installed_plans().end()) args[3 * n] = &it->second;

@@ -84,3 +84,41 @@ def test_rows_of_a_patch_against_a_look_at_every_tile(tmp_path):
             whole = (images - 1) * math.gcd(pixels, bp) >= bp          # every place that an image's end has in a tile comes up
             text += f"static_assert(rows_are_right<ConvF32Tile<16, 32, {h}, {w}, {k}, {k}, {s}, {p}, 32, {bp}, {2 if bp % 32 == 0 else 1}, {images}>>({'true' if whole else 'false'}));\n"
     _compiles(text, tmp_path)
+
+
+def test_places_of_a_patch_against_a_look_at_every_tile(tmp_path):
+    """ConvSplit: every window of every tile lies inside its patch, whatever place of an image it begins at, and what the patch
+    takes for that place is the images' element there (or padding)."""
+    text = """
+        template <class C> constexpr bool places_are_right()
+        {
+            for (int nt = 0; nt < C::NT; ++nt) {
+                const long long n0 = (long long)nt * C::BN;
+                const int n_lo = C::TW > 0 ? nt / (C::TX * C::TY) : (int)(n0 / C::OHWP), v0 = C::TW > 0 ? 0 : (int)(n0 % C::OHWP);
+                const int ty = C::TW > 0 ? nt / C::TX % C::TY * C::TH : 0, tx = C::TW > 0 ? nt % C::TX * C::TW : 0;
+                const int r0 = C::TW > 0 ? ty * C::S : v0 / C::OW * C::S, x0 = tx * C::S;
+                for (int c = 0; c < C::BN; ++c) {
+                    const int v = v0 + c, img = C::TW > 0 ? 0 : v / C::OHWP, p = C::TW > 0 ? 0 : v % C::OHWP;
+                    const int y = C::TW > 0 ? ty + c / (C::TW > 0 ? C::TW : 1) : p / C::OW, x = C::TW > 0 ? tx + c % (C::TW > 0 ? C::TW : 1) : p % C::OW;
+                    if (n_lo + img >= C::NIMG || y >= C::OHW / C::OW || x >= C::OW) continue;
+                    const int base = (img * C::PH + y * C::S - r0) * C::PW + x * C::S - x0;
+                    for (int t = 0; t < C::T; t += C::T - 1) {
+                        const int place = base + t / C::KW * C::PW + t % C::KW, row = r0 + place / C::PW, i = C::TW > 0 ? 0 : row / C::PH;
+                        if (base < 0 || place >= C::SLOTS || i >= C::NIMAGES || i != img || row - i * C::PH != y * C::S + t / C::KW || x0 + place % C::PW != x * C::S + t % C::KW) return false;
+                    }
+                    if (C::TW > 0 && base != c / (C::TW > 0 ? C::TW : 1) * C::S * C::PW + c % (C::TW > 0 ? C::TW : 1) * C::S) return false;
+                }
+            }
+            return true;
+        }
+    """
+    for h, w, p, bn, tw, n in [(5, 5, 1, 128, 0, 20), (7, 7, 1, 96, 0, 27), (7, 7, 1, 112, 0, 29), (8, 8, 1, 128, 0, 7), (9, 6, 0, 96, 0, 30), (13, 15, 1, 112, 0, 9), (14, 14, 1, 112, 0, 9), (16, 16, 1, 128, 0, 3),
+                               (11, 10, 2, 224, 0, 9), (28, 28, 0, 224, 0, 5), (20, 33, 1, 224, 16, 2), (13, 15, 1, 144, 12, 2), (30, 18, 0, 112, 28, 2), (9, 9, 2, 112, 16, 2), (14, 60, 1, 112, 28, 1)]:
+        text += f"static_assert(places_are_right<ConvSplit<64, 128, {h}, {w}, 3, 3, 1, {p}, {n}, 2, 4, {2 if bn > 144 else 1}, {bn}, {tw}>>());\n"
+    text += """
+        static_assert(ConvTiling<256, 256, 14, 14, 3, 3, 1, 1, 1024>::patch_form() == 7 && ConvTiling<64, 64, 56, 56, 3, 3, 1, 1, 1024>::patch_form() == 2807);
+        static_assert(ConvTiling<96, 96, 35, 35, 3, 3, 1, 1, 1024>::patch_form() == 1209 && ConvTiling<128, 256, 28, 28, 3, 3, 1, 0, 1024>::patch_form() == 14);
+        static_assert(ConvTiling<48, 64, 56, 56, 3, 3, 1, 1, 1024>::patch_form() == 0 && ConvTiling<64, 64, 56, 56, 3, 3, 2, 1, 1024>::patch_form() == 0);   // half a group; stride 2
+        static_assert(ConvTiling<256, 256, 14, 14, 3, 3, 1, 1, 64>::patch_form() == 0 && ConvTiling<64, 64, 56, 56, 5, 5, 1, 2, 1024>::patch_form() == 0);   // few tiles; 25 taps
+    """
+    _compiles(text, tmp_path)

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import bfuse_project_amd as bf
+from bfuse_project_amd import patterns
 from bfuse_project_amd.operation import fill_normal
 from oracle import oracle as orf
 from tests.test_gpu_conv_tile import _check
@@ -274,3 +275,87 @@ def test_infinities_nan_and_the_largest_values(tag):
     assert np.array_equal(np.isnan(y), np.isnan(want)) and np.array_equal(np.isposinf(y), np.isposinf(want)) and np.array_equal(np.isneginf(y), np.isneginf(want))
     ok = np.isfinite(want)
     assert ok.any() and np.all(np.abs(y[ok] - want[ok]) <= 1e-5 * np.maximum(np.abs(want[ok]), np.sqrt(np.float32(x2.shape[1]))))
+
+
+CONV_PATCHES = [("a", 1), ("b", 1), ("c", 0), ("d", 1), ("e", 0), ("f", 2), ("g", 1)]
+
+
+@pytest.mark.parametrize("tag,p", CONV_PATCHES)
+def test_convolution_from_a_patch_against_the_oracle_and_fused(tag, p):
+    partner, kind, suffix = {"a": ("layernorm_8x256", "bfuse", "_c4"), "b": ("bias_relu_4096", "hfuse", ""),
+                             "d": ("conv3x3_f32_32x12x12_32", "hfuse", "")}.get(tag, ("bias_relu_4096", None, ""))
+    _check(f"selftest_conv_split_{tag}", lambda x, w: orf.conv2d(x, w, s=1, p=p), partner, kind, suffix)
+
+
+@pytest.mark.parametrize("tag,p", CONV_PATCHES)
+@pytest.mark.parametrize("where", ["image", "filter"])
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** -118, 2.0 ** -140])
+def test_values_that_parts_do_not_hold_in_a_patch_or_its_filters(tag, p, where, scale):
+    """Infinite, NaN and lowest values are in the results that have them in their window (padding and places beside an image
+    are not multiplied), and values below bf16's bits keep theirs: what fp32 arithmetic gives."""
+    name = f"selftest_conv_split_{tag}"
+    x, w = _operands(name)
+    w = np.abs(w) + np.float32(0.5)
+    if where == "image":
+        x[0, 3, 0, 0], x[1, 5, 4, 3], x[-1, 2, 0, 4], x[0, 7, 4, 4] = np.inf, np.nan, -np.inf, np.finfo(np.float32).min
+        x[1] *= np.float32(scale)
+    else:
+        x = np.abs(x) + np.float32(0.5)
+        w[17, 3, 1, 1], w[1, 5, 0, 2], w[-1, 2, 2, 0] = np.inf, np.nan, np.finfo(np.float32).min
+        w[2] *= np.float32(scale)
+    (w if where == "image" else x)[...] *= np.float32(2.0 ** 60)
+    with np.errstate(all="ignore"):
+        want = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(w).double(), padding=p).numpy()
+        f = want.astype(np.float32)
+    y = _run(name, x, w)
+    assert np.array_equal(np.isnan(y), np.isnan(f)) and np.array_equal(np.isposinf(y), np.isposinf(f)) and np.array_equal(np.isneginf(y), np.isneginf(f))
+    u = 2.0 ** -24 * (9 * x.shape[1]) ** 0.5 * 2     # twice the bound of one sum rounded after every product
+    for part in [(n, slice(None)) for n in range(x.shape[0])] + [(slice(None), m) for m in range(w.shape[0])]:
+        ok = np.isfinite(f[part]) & (np.abs(want[part]) < 2.0 ** 120)      # (the lowest value's products drown the others)
+        assert np.linalg.norm(y[part][ok] - want[part][ok]) <= u * np.linalg.norm(want[part][ok])
+
+
+@pytest.mark.parametrize("tag,channels", [("a", 64), ("c", 96), ("e", 128), ("g", 96)])
+def test_convolution_from_a_patch_is_closer_to_64_bits_than_one_fp32_sum(tag, channels):
+    """As the products: partial sums of n taps of 32 channels are each rounded 6 n times while they grow, and added once; n is two or three."""
+    name = f"selftest_conv_split_{tag}"
+    x, w = _operands(name)
+    p = dict(CONV_PATCHES)[tag]
+    want = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(w).double(), padding=p).numpy()
+    err = np.linalg.norm(_run(name, x, w) - want) / np.linalg.norm(want)
+    steps = channels // 32 * 9
+    assert err <= 2.0 ** -24 * ((steps / 4 + 9) ** 0.5 + 0.5)
+
+
+def test_filters_are_taken_apart_for_every_launch_and_side():
+    """The parts are the launch's own filters': new ones, two sides at once on two streams, replays of a graph, a plan at run time."""
+    name = "selftest_conv_split_a"
+    with bf.Operation(name, name) as op:
+        k = op.k[0]
+        X = [fill_normal(31 + i, int(np.prod(k.shapes[0])), 0, 1) for i in range(2)]
+        W = [fill_normal(41 + i, int(np.prod(k.shapes[1])), 0, 1) for i in range(2)]
+        want = [[op.run_kernel(0, x, w) for w in W] for x in X]
+        assert np.array_equal(op.run_kernel(0, X[0], W[0]), want[0][0])
+        for a, b in ((0, 1), (1, 0)):
+            y0, y1 = op.run_parallel(X[0], W[a], X[1], W[b])
+            assert np.array_equal(y0, want[0][a]) and np.array_equal(y1, want[1][b])
+        for rnd in range(3):
+            op.upload(0, X[0], W[rnd % 2])
+            op.upload(1, X[1], W[1])
+            for mode in ("parallel", "serial", "kernel1"):
+                op.zero_outputs()
+                assert op.time_graph(mode, chain=2, reps=2) > 0
+                assert np.array_equal(op.download(0), want[0][rnd % 2]) and (mode == "kernel1" or np.array_equal(op.download(1), want[1][1]))
+                assert (op.time(mode, warmup=1, reps=2)[0] > 0).all()
+        P = [fill_normal(21 + i, 8 * 256 if i == 0 else 512, 0, 1) for i in (0, 1)]
+    with bf.Operation(name, "layernorm_8x256") as op:
+        for w in (0, 1):
+            assert np.array_equal(op.run_fuse(op.fused("bfuse", "_c4"), X[0], W[w], *P)[0], want[0][w])
+    with bf.Operation("selftest_conv_split_f", "layernorm_8x256") as op:
+        k = op.k[0]
+        x, W = fill_normal(31, int(np.prod(k.shapes[0])), 0, 1), [fill_normal(41 + i, int(np.prod(k.shapes[1])), 0, 1) for i in range(2)]
+        dims = [patterns.LaunchDims(tuple(q.grid), tuple(q.block)) for q in op.k]
+        rt = op.set_plan(op.fused_rt(), patterns.plan_blocks("ranges", dims), 2)
+        for w in W:
+            y = op.run_kernel(0, x, w)
+            assert np.array_equal(op.run_fuse(rt, x, w, *P)[0], y)
