@@ -3,7 +3,7 @@
 // tilings of their 512-row / 16-product counterparts (model_ops.h) -- twice, or 64 times, the workgroups -- or with twice
 // the columns per tile, which is again a workgroup per CU and a better ratio of MFMAs to operand reads: 1024 x 3072 x 768
 // 44.4 -> 34.8 us (32 x 96 against 32 x 48), x 768 x 768 11.5 -> 10.8, 4096 x 1024 62.5 -> 60.2 (32 x 128 against 32 x 64).  The larger ones run on the bf16 matrix cores (ops_gemm_split.h has the figures): there the
-// tile is 128 x 128, 128 x 96 or 256 x 128, the largest that still gives every CU one.  Those that have no 256 such tiles split K over the
+// tile is 128 x 128, 128 x 96 or 256 x 112 (two whole rounds for 14336 columns; 128 are one and three quarters), the largest that still gives every CU one.  Those that have no 256 such tiles split K over the
 // waves of 32 x 96 - 32 x 144 tiles instead (GemmF32Dma): 1024 x 768 x 2304 24.8 us, on 192 tiles of 128 x 96 30.2.
 #include "fuse.h"
 #include "ops_gemm_f32.h"
@@ -19,16 +19,16 @@ BFUSE_MODULE_PROLOGUE()
     BFUSE_KERNEL(gemm_f32_##M##x##K##x##N, Dense_##M##x##K##x##N, ({{M, K, 1, 1}, 4}), ({{K, N, 1, 1}, 4}), ({{M, N, 1, 1}, 4}))
 // <.., 16-row blocks of a wave, waves over the rows, over the columns, over K, columns>
 #define DENSE_SPLIT(M, K, N, ...)                                                                                \
-    using Dense_##M##x##K##x##N = GemmSplit<M, K, 1, N, 1, 1, __VA_ARGS__, kPix>;                                 \
+    using Dense_##M##x##K##x##N = GemmSplit<M, K, 1, N, 1, 1, __VA_ARGS__>;                                       \
     BFUSE_KERNEL(gemm_f32_##M##x##K##x##N, Dense_##M##x##K##x##N, ({{M, K, 1, 1}, 4}), ({{K, N, 1, 1}, 4}), ({{M, N, 1, 1}, 4}))
 DENSE_F32(1024, 768, 768, 32, 96, 4)
-DENSE_SPLIT(1024, 768, 3072, 2, 4, 1, 2, 96)
+DENSE_SPLIT(1024, 768, 3072, 2, 4, 1, 2, 96, kPix)
 DENSE_F32(1024, 3072, 768, 32, 96, 4)
 DENSE_F32(1024, 768, 2304, 32, 144, 4)
-DENSE_SPLIT(1024, 4096, 4096, 2, 4, 1, 2, 128)
+DENSE_SPLIT(1024, 4096, 4096, 2, 4, 1, 2, 128, kPix)
 DENSE_F32(1024, 4096, 1024, 32, 128, 4)
-DENSE_SPLIT(1024, 4096, 14336, 2, 8, 1, 1, 128)
-DENSE_SPLIT(1024, 14336, 4096, 2, 4, 1, 2, 128)
+DENSE_SPLIT(1024, 4096, 14336, 2, 8, 1, 1, 112, kPix, 1, 1, 0, false, true)
+DENSE_SPLIT(1024, 14336, 4096, 2, 4, 1, 2, 128, kPix)
 
 // C[b] = A[b] . B[b]^T, A [b, M, K], B [b, N, K].  Those of 208 rows: <M, N, K, BM, BN, waves over K>, a tile per wave; the one-wave
 // products reserve 32 KB of LDS per workgroup: four workgroups per CU, one wave per SIMD (see LdsReserve).

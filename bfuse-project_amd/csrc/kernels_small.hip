@@ -258,6 +258,23 @@ BFUSE_BFUSE_KERNEL(selftest_gemm_split_a, GemmSp_a, layernorm_8x256, LayerNormS,
 BFUSE_HFUSE_KERNEL(selftest_gemm_split_e, GemmSp_e, bias_relu_4096, BiasReluS)
 BFUSE_HFUSE_KERNEL(selftest_gemm_split_f, GemmSp_f, conv3x3_f32_32x12x12_32, ConvS2)
 
+// The same products with the first operand taken apart before: _p of a, b, h, i, j, l and r, and a dense one with a last stage of eight k.
+#define PARTS_TEST(TAG, OP, I, F, O)                                                                               \
+    using GemmSpP_##TAG = OP;                                                                                       \
+    BFUSE_KERNEL(selftest_gemm_split_##TAG##_p, GemmSpP_##TAG, (I), (F), (O))
+#define DIMS4(...) {{__VA_ARGS__}, 4}
+#define PARTS_OF(...) GemmSplit<__VA_ARGS__, false, true>
+DENSE_SPLIT_TEST(s, 160, 104, 144, 2, 4, 1, 1, 64)
+PARTS_TEST(s, PARTS_OF(160, 104, 1, 144, 1, 1, 2, 4, 1, 1, 64, kPix, 1, 1, 0), DIMS4(160, 104, 1, 1), DIMS4(104, 144, 1, 1), DIMS4(160, 144, 1, 1))
+PARTS_TEST(a, PARTS_OF(160, 96, 1, 144, 1, 1, 2, 4, 1, 1, 64, kPix, 1, 1, 0), DIMS4(160, 96, 1, 1), DIMS4(96, 144, 1, 1), DIMS4(160, 144, 1, 1))
+PARTS_TEST(b, PARTS_OF(128, 256, 1, 96, 1, 1, 2, 4, 1, 2, 96, kPix, 1, 1, 0), DIMS4(128, 256, 1, 1), DIMS4(256, 96, 1, 1), DIMS4(128, 96, 1, 1))
+PARTS_TEST(h, SwapOperands<PARTS_OF(64, 56, 9, 7, 2, 11, 2, 2, 1, 2, 96, kPix, 1, 1, 0)>, DIMS4(11, 56, 9, 7), DIMS4(64, 56, 1, 1), DIMS4(11, 64, 5, 4))
+PARTS_TEST(i, SwapOperands<PARTS_OF(64, 144, 9, 7, 1, 5, 2, 2, 1, 1, 64, kPix, 3, 3, 1)>, DIMS4(5, 16, 9, 7), DIMS4(64, 16, 3, 3), DIMS4(5, 64, 9, 7))
+PARTS_TEST(j, SwapOperands<PARTS_OF(48, 216, 17, 17, 2, 3, 1, 3, 1, 1, 128, kPix, 3, 3, 0)>, DIMS4(3, 24, 17, 17), DIMS4(48, 24, 3, 3), DIMS4(3, 48, 8, 8))
+PARTS_TEST(l, SwapOperands<PARTS_OF(80, 480, 12, 10, 3, 7, 1, 4, 1, 1, 112, kPix, 5, 6, 2)>, DIMS4(7, 16, 12, 10), DIMS4(80, 16, 5, 6), DIMS4(7, 80, 4, 3))
+PARTS_TEST(r, SwapOperands<PARTS_OF(160, 64, 9, 9, 1, 5, 1, 10, 1, 1, 128, kPix, 1, 1, 0)>, DIMS4(5, 64, 9, 9), DIMS4(160, 64, 1, 1), DIMS4(5, 160, 9, 9))
+BFUSE_BFUSE_KERNEL(selftest_gemm_split_r_p, Narrow<GemmSpP_r>, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
+
 // The convolution from a patch taken apart once: pixels that run on into the next images and past the batch, rectangles past an image's
 // edges with whole and with broken quads of pixels, one to four groups of channels, units that a thread does twice, two waves over the columns.
 // <CI, CO, H, W, padding, images, 16-row blocks of a wave, waves over rows, over columns, pixels, width>

@@ -65,10 +65,10 @@ using Conv4 = Conv3x3F32Lds<128, 128, 28, 28, 32, 1, 4>;
 
 // fp32 instantiations of the Llama-3-8B layers (the reference computes every layer in fp32), on the bf16 matrix cores: 256
 // tiles of 128 x 64 for N = 4096 (dense_4, dense_7: 119 -> 93 us, 404 -> 308) and of 256 x 112 for N = 14336 (dense_6: 461 ->
-// 254; two groups of waves over K on 128 x 112 tiles 282).  Before: GemmF32Dma on 64 x 128 tiles.
-using Dense4F32 = GemmSplit<512, 4096, 1, 4096, 1, 1, 2, 4, 1, 2, 64, kPix>;
-using Dense6F32 = GemmSplit<512, 4096, 1, 14336, 1, 1, 2, 8, 1, 1, 112, kPix>;
-using Dense7F32 = GemmSplit<512, 14336, 1, 4096, 1, 1, 2, 4, 1, 2, 64, kPix>;
+// 254; two groups of waves over K on 128 x 112 tiles 282), with the activations taken apart before 95 -> 91, 324 -> 309, 263 -> 259.  Before: GemmF32Dma on 64 x 128 tiles.
+using Dense4F32 = GemmSplit<512, 4096, 1, 4096, 1, 1, 2, 4, 1, 2, 64, kPix, 1, 1, 0, false, true>;
+using Dense6F32 = GemmSplit<512, 4096, 1, 14336, 1, 1, 2, 8, 1, 1, 112, kPix, 1, 1, 0, false, true>;
+using Dense7F32 = GemmSplit<512, 14336, 1, 4096, 1, 1, 2, 4, 1, 2, 64, kPix, 1, 1, 0, false, true>;
 
 // bgemm_4 .. bgemm_17 of llm.yaml (ViT / Swin / small-model attention products: 16 heads x 256 or 208 tokens with
 // head sizes 64 and 80, and single-head products of 512 / 768 / 1024 tokens).  Scores (reductions of 64 and 80) run on

@@ -297,8 +297,10 @@ struct ConvF32Rect {
 // KS waves, which split the channels.  A shared tile like ConvF32Tile, whose place it takes: only what a workgroup does with it differs.
 constexpr int kSplitForm = 32;
 template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int BM, int PB, int KS, int NIMG>
-struct ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, KS, NIMG, kSplitForm> : ConvF32Tile<CI, CO, H, W, KH, KW, S, P, BM, 16 * PB, 1, NIMG> {
-    using Form = SwapOperands<GemmSplit<CO, CI * KH * KW, H, W, S, NIMG, BM / 16 / KS, KS, 1, 1, 16 * PB, kPix, KH, KW, P>>;
+struct ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, KS, NIMG, kSplitForm> : ConvF32Tile<CI, CO, H, W, KH, KW, S, P, BM, PB % 4 == 0 ? 16 * PB : 128, 1, NIMG> {
+    using Form = SwapOperands<GemmSplit<CO, CI * KH * KW, H, W, S, NIMG, BM / 16 / KS, KS, 1, 1, 16 * PB, kPix, KH, KW, P, false, (CI * KH * KW >= 256)>>;
+    using Parts = typename Form::Parts;
+    static constexpr int PARTS_OPERAND = Form::PARTS_OPERAND;
     static constexpr long long TILES = Form::TILES;
     static constexpr bool FITS = Form::FITS;
     static constexpr Dims3 GRID = Form::GRID, BLOCK = Form::BLOCK;
@@ -470,7 +472,11 @@ struct ConvTiling {
     // 1432 -> 1161, 32 -> 64 on 147 x 147 6802 -> 5938, 16 -> 64 at stride 4 1338 -> 865; but at stride 2, where a load of the gather
     // touches twice the lines and the tile's patch was loaded once, 32 -> 64 on 147 x 147 1864 -> 1891.
     static constexpr int SBM = CO % 256 == 0 ? 256 : CO % 128 == 0 ? 128 : CO % 192 == 0 ? 192 : CO % 160 == 0 ? 160 : CO % 96 == 0 ? 96 : 64;
-    using split = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, SBM, SBM == 192 || SBM == 96 ? 4 : 8, SBM == 256 ? 8 : SBM == 160 ? 10 : SBM == 96 ? 2 : 4, NIMG, kSplitForm>;
+    // 256 rows on 112 pixels instead of 128 where that leaves less of the last round over the CUs idle: 256 -> 512 on 14 x 14 at stride 2 is 3.25 rounds (4) of
+    // 128 but 3.7 of 112, 611 -> 585 us; 128 -> 256 on 28 x 28 573 -> 568.
+    static constexpr int ROUNDS8 = (int)(((long long)((OHW + 3) / 4 * 4) * NIMG + 127) / 128 * (CO / 256) + 255) / 256, ROUNDS7 = (int)(((long long)((OHW + 3) / 4 * 4) * NIMG + 111) / 112 * (CO / 256) + 255) / 256;
+    static constexpr int PB256 = 112 * ROUNDS7 < 0.97 * 128 * ROUNDS8 ? 7 : 8;
+    using split = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, SBM, SBM == 256 ? PB256 : SBM == 192 || SBM == 96 ? 4 : 8, SBM == 256 ? 8 : SBM == 160 ? 10 : SBM == 96 ? 2 : 4, NIMG, kSplitForm>;
     static constexpr bool is_split()
     {
         // (the table of taps is made at compile time)
@@ -524,7 +530,7 @@ struct ConvTiling {
             if (c[i] < c[best]) best = i;
         return c[best] < 1e8 ? f[best] : 0;
     }
-    // 1 x 1 filters on 256 and more channels likewise, also on 224 x 128 tiles (seven waves).  us, GemmTile before: 768 -> 192 on
+    // 1 x 1 filters on 256 and more channels likewise, also on 224 x 128 tiles (seven waves).  us, GemmTile before (the filters taken apart by every workgroup; GemmSplit has what it gave to do that once): 768 -> 192 on
     // 17 x 17 641 -> 525 (twelve waves of 16 rows 0.96x that, but no register is left beside twelve waves), 160 573 -> 447, 128 455 -> 344,
     // 1280 -> 448 on 8 x 8 521 -> 378, 384 450 -> 314, 320 377 -> 292, 192 233 -> 179, 2048 -> 448 824 -> 582, 256 -> 256 on 56 x 56
     // 3034 -> 2502, 256 -> 512 at stride 2 145 -> 121.  (160 rows are ten waves on four SIMDs, bound by their LDS reads: 155 TFLOP/s where 256 x
@@ -532,7 +538,7 @@ struct ConvTiling {
     // 152 against 177, 64 -> 128 202 against 218; 64 output channels 394 against 383-410.
     static constexpr int S1BM = CO % 256 == 0 ? 256 : CO % 128 == 0 ? 128 : CO % 224 == 0 ? 224 : CO % 192 == 0 ? 192 : 160;
     static constexpr int S1WR = S1BM == 256 ? 8 : S1BM == 224 ? 7 : S1BM == 160 ? 10 : 4;
-    using split_product = GemmSplit<CO, CI, H, W, S, NIMG, S1BM / 16 / S1WR, S1WR, 1, 1, S1BM == 192 ? 64 : 128, kPix>;
+    using split_product = GemmSplit<CO, CI, H, W, S, NIMG, S1BM / 16 / S1WR, S1WR, 1, 1, S1BM == 256 ? 16 * PB256 : S1BM == 192 ? 64 : 128, kPix, 1, 1, 0, false, true>;
     static constexpr bool is_split_product()
     {
         if constexpr (STREAM && CI >= 256 && CO % S1BM == 0) return split_product::FITS && split_product::TILES >= 512;

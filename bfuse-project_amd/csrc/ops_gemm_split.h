@@ -14,6 +14,12 @@
 //     the fragment reads of a wave are 256 consecutive bytes for each of its four octets: no bank is met twice;
 //   * three LDS buffers and one barrier per stage of 32 k.  While stage s is multiplied, the stage two ahead is taken apart and
 //     written and the A of the next one taken apart, dealt between the MFMAs; the loads are a stage ahead of that;
+//   * PREP: A is taken apart by a kernel that runs before this one (SplitParts), once instead of by every workgroup that has its rows. A
+//     wave's three loads for 16 rows and 32 k go straight into the registers that it multiplies from, a stage ahead; that they are 1.5 times the bytes is what it
+//     costs. Filters, and activations that many column tiles share. us, in turn on one card: 768 -> 192 on 17 x 17 531 -> 472, -> 160 461 -> 447, -> 128 352 ->
+//     340, 1280 -> 384 on 8 x 8 321 -> 309, 2048 -> 192 283 -> 260, 80 -> 192 of 3 x 3 on 73 x 73 7520 -> 6700, 64 -> 192 at stride 2 4186 -> 3650, 288 -> 384 2890 -> 2750, 192 -> 320 382 ->
+//     372, 1024 x 4096 x 14336 (on 112 columns, 512 tiles for 448) 520 -> 505, 512 x 4096 x 4096 94 -> 91: 0.945 in the geometric mean of 26 operators, the same bits.  The
+//     rows' kernel is 5 us for filters and 8 for 1024 x 4096, with its launch 3 more: 1024 x 4096 x 4096 170 -> 173, 1024 x 14336 x 4096 571 -> 574, 1024 x 768 x 3072 33 -> 38, and 16 -> 64 channels (K = 144) 1.01x stay without;
 //   * products with few tiles give two groups of waves the even and the odd stages (KG = 2): two waves per SIMD hide each
 //     other's waits, and the groups' sums meet in LDS at the end.
 // The operands of an MFMA are given in the order (B, A), so that a lane ends up with four consecutive columns of a row.
@@ -61,17 +67,17 @@
 
 namespace bfuse {
 
-// The parts of filters [M, K] of fp32, k = (channel, tap), as a kernel of its own leaves them in a workspace (Prepares, fuse.h) for one that
-// multiplies them (ConvSplit): taps are put behind the channels, 32 of which are a stage's k, stage (channels, tap); for every 16 rows and
-// stage the three parts one after the other, each as the MFMA's operand, 16 bytes a lane.  In front of them: where the filters
-// themselves lie, and a word for every 16 rows and 32 channels that is not zero if a value is more than its parts.
+// The parts of a matrix [M, K] of fp32, as a kernel of its own leaves them in a workspace (Prepares, fuse.h) for one that multiplies it: for
+// every 16 rows and 32 k (a stage) the three parts one after the other, each as the MFMA's operand, 16 bytes a lane.  In front of them: where the matrix
+// itself lies, and a word for every 16 rows and eight stages that is not zero if a value is more than its parts.  TAPS > 1: k counts (channel, tap), and
+// taps are put behind the channels, 32 of which are a stage's k then, stage (channels, tap) (ConvSplit); a word for every 32 channels.
 // One wave takes a stage apart at a time; a lane's values are TAPS apart, so a wave's loads touch 16 rows, of which the other taps' then
 // come from the caches: 256 x 2304 in 5 us.
-template <int M, int K, int TAPS>
+template <int M, int K, int TAPS, bool ON = true>
 struct SplitParts {
-    static_assert(M % 16 == 0 && K % (32 * TAPS) == 0, "parts");
+    static_assert(!ON || (M % 16 == 0 && K % 8 == 0 && (TAPS == 1 || K % (32 * TAPS) == 0)), "parts");
     static constexpr int PARTS_THREADS = 256;
-    static constexpr int STAGES = K / 32, CHUNKS = STAGES / TAPS;
+    static constexpr int STAGES = (K + 31) / 32, CHUNK = TAPS > 1 ? TAPS : 8, CHUNKS = (STAGES + CHUNK - 1) / CHUNK;
     static constexpr int BLOCK_BYTES = STAGES * 3072, HEAD = (64 + M / 16 * CHUNKS * 4 + 1023) / 1024 * 1024;
     static constexpr unsigned PARTS_GRID = M / 16 * CHUNKS;
     static constexpr size_t PARTS_BYTES = (size_t)HEAD + (size_t)(M / 16) * BLOCK_BYTES;
@@ -95,11 +101,11 @@ struct SplitParts {
         if (blockIdx.x == 0 && threadIdx.x == 0) *static_cast<const void**>(parts) = operand;
         __syncthreads();
         unsigned left = 0;
-        for (int s = chunk * TAPS + wave; s < (chunk + 1) * TAPS; s += PARTS_THREADS / 64) {
+        for (int s = chunk * CHUNK + wave; s < (chunk + 1) * CHUNK && s < STAGES; s += PARTS_THREADS / 64) {
             float x[8];
-            const int k = (chunk * 32 + (lane >> 4) * 8) * TAPS + s % TAPS;
+            const int k = TAPS > 1 ? (chunk * 32 + (lane >> 4) * 8) * TAPS + s % TAPS : s * 32 + (lane >> 4) * 8;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] = row[k + e * TAPS];
+            for (int e = 0; e < 8; ++e) x[e] = K % 32 == 0 || k < K ? row[k + e * TAPS] : 0.f;
             unsigned p[3][4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) split2(x[2 * j], x[2 * j + 1], p[0][j], p[1][j], p[2][j], left);
@@ -115,14 +121,17 @@ struct SplitParts {
 
 // M, K, H, W, S, NIMG, LAYOUT: as in GemmTile.  TM 16-row blocks of a wave, WR waves over the rows and WN over the BN columns, KG
 // groups of such waves over the stages.  LEAN: one set of A's parts, taken apart at the top of the stage, instead of the next one's
-// beside this one's: 12 TM registers less for a stage that begins without MFMAs, which other workgroups of the CU fill.
+// beside this one's: 12 TM registers less for a stage that begins without MFMAs, which other workgroups of the CU fill.  PREP: I is A's parts.
 template <int M_, int K_, int H_, int W_, int S_, int NIMG_, int TM_, int WR_, int WN_, int KG_, int BN_, int LAYOUT_, int KH_ = 1, int KW_ = 1, int P_ = 0,
-          bool LEAN_ = (LAYOUT_ == kRows && K_ <= 256)>
+          bool LEAN_ = (LAYOUT_ == kRows && K_ <= 256), bool PREP_ = false>
 struct GemmSplit {
+    using Parts = SplitParts<M_, K_, 1, PREP_>;
+    static constexpr int PARTS_OPERAND = PREP_ ? 0 : -1;
     static constexpr bool MATRIX_CORES = true;   // the inner loop is a stream of MFMAs (what the fusion chooser asks)
     static constexpr int M = M_, K = K_, H = H_, W = W_, S = S_, NIMG = NIMG_, TM = TM_, WR = WR_, WN = WN_, KG = KG_, BN = BN_, LAYOUT = LAYOUT_, KH = KH_, KW = KW_, P = P_;
     static constexpr int T = KH * KW, CI = K / T;                                // kPix: taps, channels of the images
-    static constexpr bool LEAN = LEAN_;
+    static constexpr bool LEAN = LEAN_, PREP = PREP_;
+    static_assert(!PREP || !LEAN, "lean: one set of A's parts");
     static constexpr int NWAVE = WR * WN * KG, THREADS = 64 * NWAVE, GT = 64 * WR * WN, BM = 16 * TM * WR, TN = BN / WN / 16;
     static constexpr int NS = (K + 31) / 32, NIT = NS / KG, TAIL = K % 32;       // stages, those of a group, k of the last one if not 32
     static constexpr int OH = (H - KH + 2 * P) / S + 1, OW = (W - KW + 2 * P) / S + 1, HW = H * W, OHW = OH * OW;
@@ -213,7 +222,7 @@ struct GemmSplit {
     __device__ static __forceinline__ void run(int vblock, int tid, Smem& sm, const void* I, const void* F, void* O, Sync sync)
     {
         static_assert(FITS, "tile too large");
-        const float* A = static_cast<const float*>(I);
+        const float* A = static_cast<const float*>(PREP ? Parts::source(I) : I);
         const float* B = static_cast<const float*>(F);
         float* __restrict__ C = static_cast<float*>(O);
         const int lane = tid & 63, li = lane & 15, kq = lane >> 4;
@@ -266,8 +275,21 @@ struct GemmSplit {
 #pragma unroll
             for (int b = 0; b < TN; ++b) acc[tm][b] = part[tm][b] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-        f32x4 ra[TM][2];
+        f32x4 ra[PREP ? 1 : TM][2];
         float rb[NUJ][8];
+        unsigned pa[LEAN ? 1 : 2][TM][3][4];
+        const auto pr = __builtin_amdgcn_make_buffer_rsrc((void*)(PREP ? Parts::block(I, m0 / 16) : nullptr), 0, PREP ? TM * WR * Parts::BLOCK_BYTES : 0, 0x00020000);
+        // Taken apart before: the parts of stage s, straight into the registers that it is multiplied from.
+        auto load_parts = [&](int set, int s) {
+#pragma unroll
+            for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) {
+                    const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(pr, (unsigned)(lane * 16 + q * 1024), ((wr * TM + tm) * NS + s) * 3072, 0));
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) pa[LEAN ? 0 : set][tm][q][j] = v[j];
+                }
+        };
         auto load_a = [&](int tm, int s) {
             const unsigned v = TAIL != 0 && s == NS - 1 && 8 * kq >= TAIL ? 0x7fffffffu : a_voff;
 #pragma unroll
@@ -300,8 +322,8 @@ struct GemmSplit {
         shared_with_asm(sm.t);
         unsigned char* const base = sm.t + g * NBUF * BUF;
         const unsigned char* const fb = base + (kq * BN + wn * TN * 16 + li) * 16;
-        unsigned pa[LEAN ? 1 : 2][TM][3][4], pb[3][4];
-        unsigned left = 0;                          // see split.h
+        unsigned pb[3][4];
+        unsigned left = PREP ? Parts::inexact(I, m0 / 16 + wr * TM, TM, lane) : 0;   // see split.h
         if (tid == 0) sm.inexact = 0;
         // Two of a unit's eight values: units 0 .. NUJ - 1 are this thread's of B, the others its rows of A.
         auto convert = [&](int part, int to, int off) {
@@ -319,7 +341,7 @@ struct GemmSplit {
                 split2(ra[tm][j / 2][2 * (j % 2)], ra[tm][j / 2][2 * (j % 2) + 1], p[0][j], p[1][j], p[2][j], left);
             }
         };
-        constexpr int NPART = 4 * (LEAN ? NUJ : NUJ + TM);
+        constexpr int NPART = 4 * (LEAN || PREP ? NUJ : NUJ + TM);
         // A partial sum goes to the result between its last stage's MFMAs and the first ones of the next: every other block of columns,
         // over the two stages (2 TN blocks) that this leaves, so that the additions too are dealt between MFMAs (1024 x 4096 x 4096 158 us;
         // all in one stage 164).  Convolutions, whose padding takes registers, add a block right behind its last MFMAs (448 -> 384 channels
@@ -336,7 +358,9 @@ struct GemmSplit {
         for (int i = 0; i < 2 && i < NIT; ++i) {
 #pragma unroll
             for (int j = 0; j < NUJ; ++j) load_b(j, stage_of(i));
-            if (i == 0) {
+            if constexpr (PREP) {
+                if (i == 0) load_parts(0, g);
+            } else if (i == 0) {
 #pragma unroll
                 for (int tm = 0; tm < TM; ++tm) load_a(tm, g);
             }
@@ -354,7 +378,7 @@ struct GemmSplit {
 #pragma unroll
                 for (int tm = 0; tm < TM; ++tm) load_a(tm, stage_of(next));
         };
-        if constexpr (!LEAN) convert_a(1, NIT > 1);
+        if constexpr (!LEAN && !PREP) convert_a(1, NIT > 1);
         u32x4 fr[2][3];
         auto read = [&](int set, int q, int b, int off) { fr[set][q] = *reinterpret_cast<const u32x4*>(fb + off + q * PLANE + b * 256); };
         sync.raw();
@@ -365,11 +389,12 @@ struct GemmSplit {
         // `left`: how many stages follow, if those are less than three: nothing is loaded, taken apart or read past the last one.
         auto stage = [&](int it, auto at, auto left) {
             constexpr int AT = decltype(at)::value, FROM = AT % 2, LEFT = decltype(left)::value;
-            constexpr int FIRST = LEFT >= 2 ? 0 : 4 * NUJ, LAST = LEAN || LEFT >= 1 ? NPART : 4 * NUJ, N = LAST > FIRST ? LAST - FIRST : 0;
+            constexpr int FIRST = LEFT >= 2 ? 0 : 4 * NUJ, LAST = LEAN || PREP || LEFT >= 1 ? NPART : 4 * NUJ, N = LAST > FIRST ? LAST - FIRST : 0;
             constexpr int VPM = (11 * N + (NIT > SUMMED ? 4 * TM * folded(AT) : 0) + 6 * TM * TN - 1) / (6 * TM * TN);
             // Behind the barrier the next stage is in LDS whole, and nobody reads the one before this any more.
             if (it > 0) sync.raw();
             if constexpr (LEAN) convert_a(it + 1, LEFT >= 1);
+            if constexpr (PREP && LEFT >= 1) load_parts(FROM ^ 1, stage_of(it + 1));
 #pragma unroll
             for (int b = 0; b < TN; ++b) {
                 const int set = (b + FROM * (TN & 1)) & 1;
@@ -617,10 +642,10 @@ struct GemmSplit {
 
 // (see Narrow) us, ten waves and five, with twice the rows of a wave: 768 -> 160 channels on 17 x 17 460 and 514, 192 -> 320 at
 // stride 2 385 and 436, 1280 -> 320 on 8 x 8 296 and 324, 2048 -> 320 459 and 500.  (Eight waves of 80 x 32: the 3 x 3 layer spills.)
-template <int M, int K, int H, int W, int S, int NIMG, int TM, int WR, int WN, int KG, int BN, int LAYOUT, int KH, int KW, int P, bool LEAN>
-struct NarrowOf<GemmSplit<M, K, H, W, S, NIMG, TM, WR, WN, KG, BN, LAYOUT, KH, KW, P, LEAN>> {
+template <int M, int K, int H, int W, int S, int NIMG, int TM, int WR, int WN, int KG, int BN, int LAYOUT, int KH, int KW, int P, bool LEAN, bool PREP>
+struct NarrowOf<GemmSplit<M, K, H, W, S, NIMG, TM, WR, WN, KG, BN, LAYOUT, KH, KW, P, LEAN, PREP>> {
     static constexpr int HALVE = 64 * WR * WN * KG > 512 && WR % 2 == 0 ? 2 : 1;
-    using type = GemmSplit<M, K, H, W, S, NIMG, TM * HALVE, WR / HALVE, WN, KG, BN, LAYOUT, KH, KW, P, LEAN>;
+    using type = GemmSplit<M, K, H, W, S, NIMG, TM * HALVE, WR / HALVE, WN, KG, BN, LAYOUT, KH, KW, P, LEAN, PREP>;
 };
 
 }  // namespace bfuse

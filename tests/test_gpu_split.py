@@ -359,3 +359,26 @@ def test_filters_are_taken_apart_for_every_launch_and_side():
         for w in W:
             y = op.run_kernel(0, x, w)
             assert np.array_equal(op.run_fuse(rt, x, w, *P)[0], y)
+
+
+@pytest.mark.parametrize("tag", ["a", "b", "h", "i", "j", "l", "r", "s"])
+@pytest.mark.parametrize("side", [0, 1])
+@pytest.mark.parametrize("value", [1.0, 2.0 ** -120 * 1.2345678, np.inf])
+def test_an_operand_taken_apart_before_gives_the_same_bits(tag, side, value):
+    """The same products of the same parts, whatever values lie in either operand (l: tiles of 112 columns for 64; those with
+    a value that its parts do not hold are done again, so that one compares its ordinary operands alone)."""
+    x, w = _operands(f"selftest_gemm_split_{tag}")
+    if tag == "l" and value != 1.0:
+        return
+    (x, w)[side].reshape(-1)[[7, 1001]] = value
+    with bf.Operation(f"selftest_gemm_split_{tag}", f"selftest_gemm_split_{tag}_p") as op:
+        for i in (0, 1):
+            op.upload(i, x, w)
+        op.zero_outputs()
+        op.launch("serial")
+        a, b = op.download(0), op.download(1)
+    assert np.isfinite(a).any() and np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    if tag == "r":
+        with bf.Operation("selftest_gemm_split_r_p", "layernorm_8x256") as op:
+            P = [fill_normal(21 + i, int(np.prod(op.k[1].shapes[i])), 0, 1) for i in (0, 1)]
+            assert np.array_equal(op.run_fuse(op.fused("bfuse", "_c4"), x, w, *P)[0].view(np.uint32), a.view(np.uint32))
