@@ -33,6 +33,7 @@
 
 #include <numeric>
 #include <type_traits>
+#include <utility>
 
 #include "dispatch.h"
 #include "ops_gemm_split.h"
@@ -91,6 +92,11 @@ struct ConvSplit {
         unsigned inexact;
     };
 
+    template <class Fn, int... t>
+    __device__ static __forceinline__ void each(Fn fn, std::integer_sequence<int, t...>)
+    {
+        (fn(std::integral_constant<int, t>{}), ...);
+    }
     // Has the value here: additions that are needed only behind the loop go there otherwise, and what they add stays in registers.
     __device__ static __forceinline__ void pin(f32x4& v)
     {
@@ -239,12 +245,11 @@ struct ConvSplit {
             }
             if constexpr (LAST) fold(TN - 1);
         };
-        auto taps = [&](auto more, auto... t) { (tap(t, more), ...); };
         auto group = [&](auto more) {
             c_off += 32 * H * W * 4;
 #pragma unroll
             for (int q = 2; q >= 0; --q) read(0, q, 0, 0);
-            [&]<int... t>(std::integer_sequence<int, t...>) { taps(more, std::integral_constant<int, t>{}...); }(std::make_integer_sequence<int, T>{});
+            each([&](auto t) { tap(t, more); }, std::make_integer_sequence<int, T>{});
             if constexpr (decltype(more)::value) {
                 if constexpr (T % 2 != 0)
 #pragma unroll
