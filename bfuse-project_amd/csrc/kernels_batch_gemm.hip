@@ -39,24 +39,24 @@ DENSE_SPLIT(1024, 14336, 4096, 2, 4, 1, 2, 128, kPix)
 // those of 64 - 128, which are mostly ends: 70 - 94 registers instead of 126 - 168, so that three workgroups a CU load, multiply and
 // store at different times.  us on one card, fp32 matrix cores before and now: 1024 products 512 x 64 x 512 360 -> 303 (32-row waves 311-348), 512 x
 // 128 x 512 625 -> 465 (499), 256 x 64 x 256 98 -> 84 (94), 256 x 80 x 256 119 -> 107 (117), 1024 x 64 x 512 705 -> 609 (620), 256 x 256 x
-// 80 134 -> 95 (16-row waves; 32-row 99), 512 x 512 x 128 555 -> 419 (32-row, 128 x 128; 16-row 446), 512 x 512 x 64 334 -> 268 (293), 1024 x
+// 80 134 -> 95 (16-row waves; 32-row 99), 512 x 512 x 128 555 -> 416 (32-row, 128 x 128, lean; not lean 424, 16-row 446), 512 x 512 x 64 334 -> 268 (293), 1024 x
 // 512 x 64 607 -> 518 (573), 256 x 256 x 64 95.6 -> 83 (88).  208 x 208 x 64 gains nothing (75.9 against 74); 208 x 64 x 208, x 80 x 208
 // and x 208 x 80 gain 1.1-1.4x on seven or thirteen waves but keep the one-wave forms, which any operator can take beside it.
 #define BGEMM_F32_SPLIT(B, M, K, N, ...)                                                                         \
-    using Bgemm_##B##x##M##x##K##x##N = GemmSplit<M, K, 1, N, 1, B, __VA_ARGS__, kRows>;                          \
+    using Bgemm_##B##x##M##x##K##x##N = GemmSplit<M, K, 1, N, 1, B, __VA_ARGS__>;                                 \
     BFUSE_KERNEL(bgemm_f32_##B##x##M##x##K##x##N, Bgemm_##B##x##M##x##K##x##N, ({{B, M, K, 1}, 4}), ({{B, N, K, 1}, 4}), ({{B, M, N, 1}, 4}))
-BGEMM_F32_SPLIT(1024, 512, 64, 512, 1, 8, 1, 1, 128)
-BGEMM_F32_SPLIT(1024, 512, 512, 64, 2, 4, 1, 1, 64)
-BGEMM_F32_SPLIT(1024, 512, 128, 512, 1, 8, 1, 1, 128)
-BGEMM_F32_SPLIT(1024, 512, 512, 128, 2, 4, 1, 1, 128)
-BGEMM_F32_SPLIT(1024, 256, 64, 256, 1, 8, 1, 1, 128)
-BGEMM_F32_SPLIT(1024, 256, 256, 64, 2, 4, 1, 1, 64)
-BGEMM_F32_SPLIT(1024, 256, 80, 256, 1, 8, 1, 1, 128)
-BGEMM_F32_SPLIT(1024, 256, 256, 80, 1, 8, 1, 1, 80)
+BGEMM_F32_SPLIT(1024, 512, 64, 512, 1, 8, 1, 1, 128, kRows)
+BGEMM_F32_SPLIT(1024, 512, 512, 64, 2, 4, 1, 1, 64, kRows)
+BGEMM_F32_SPLIT(1024, 512, 128, 512, 1, 8, 1, 1, 128, kRows)
+BGEMM_F32_SPLIT(1024, 512, 512, 128, 2, 4, 1, 1, 128, kRows, 1, 1, 0, true)
+BGEMM_F32_SPLIT(1024, 256, 64, 256, 1, 8, 1, 1, 128, kRows)
+BGEMM_F32_SPLIT(1024, 256, 256, 64, 2, 4, 1, 1, 64, kRows)
+BGEMM_F32_SPLIT(1024, 256, 80, 256, 1, 8, 1, 1, 128, kRows)
+BGEMM_F32_SPLIT(1024, 256, 256, 80, 1, 8, 1, 1, 80, kRows)
 BGEMM_F32_RESERVE(1024, 208, 64, 208, 112, 64, 1, 32768)
 BGEMM_F32_RESERVE(1024, 208, 208, 64, 208, 32, 1, 32768)
 BGEMM_F32_RESERVE(1024, 208, 80, 208, 112, 64, 1, 32768)     // 208 = 112 + 96 rows, 3 x 64 + 16 columns: the last tiles overlap their neighbours
 BGEMM_F32_RESERVE(1024, 208, 208, 80, 64, 80, 1, 32768)
 // tests/interleave_scheduler/config/info.yaml: bgemm_6, bgemm_7
-BGEMM_F32_SPLIT(1024, 1024, 64, 512, 1, 8, 1, 1, 128)
-BGEMM_F32_SPLIT(1024, 1024, 512, 64, 2, 4, 1, 1, 64)
+BGEMM_F32_SPLIT(1024, 1024, 64, 512, 1, 8, 1, 1, 128, kRows)
+BGEMM_F32_SPLIT(1024, 1024, 512, 64, 2, 4, 1, 1, 64, kRows)

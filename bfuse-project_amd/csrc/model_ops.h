@@ -50,12 +50,12 @@ using Dense6 = GemmBf16NTDma<512, 14336, 4096, 128, 224, 3, 4, 4, 2, 2, 11>;
 //            16-row waves (lean 6.05, 11.6, 23.3, 19.4, but 27.6 and 53.3; 128 x 64 of 32-row waves 7.4)
 //   bgemm_2  21.4, 29.2, 42.4, 36.9, 46.1, 73.2 -> 17.4, 22.2, 39.6, 32.6, 37.7, 63.6; 128 x 128 tiles of eight 16-row waves (128 x 64 of four
 //            32-row waves 18.2, 24.1, 36.3, 29.7, 40.2, 65.1)
-//   bgemm_3  20.1 alone, 33.0, 42.5, 67.3 with the last three -> 18.1, 28.1, 35.7, 61.3; 128 x 64 tiles of four 32-row waves, lean: the twelve waves a CU of
-//            a fused kernel with the bf16 gate projection leave 168 registers (not lean 174)
+//   bgemm_3  20.1 alone, 33.0, 42.5, 67.3 with the last three -> 16.4, 27.8, 34.9, 61.1; 128 x 64 tiles of four 32-row waves (lean 17.9, 28.1, 36.6, 62.4, and with the
+//            768 x 768 and 3072 x 768 layers 22.7, 34.9 -> 21.4, 33.9).  The twelve waves a CU of a fused kernel with the bf16 gate projection leave 168 registers: 163
 using Bgemm0 = GemmSplit<512, 64, 1, 512, 1, 12, 1, 4, 1, 1, 64, kRows, 1, 1, 0, false>;      // 8 x 8 tiles x 12 = 768 workgroups
 using Bgemm1 = GemmF32<512, 64, 512, 32, 64, 2, kEpiNone, 2, 1, true, 12>;     // 16 x 1 tiles x 12 = 192 two-wave workgroups
 using Bgemm2 = GemmSplit<512, 128, 1, 512, 1, 32, 1, 8, 1, 1, 128, kRows>;                    // 4 x 4 tiles x 32 = 512
-using Bgemm3 = GemmSplit<512, 512, 1, 128, 1, 32, 2, 4, 1, 1, 64, kRows, 1, 1, 0, true>;      // 4 x 2 tiles x 32 = 256
+using Bgemm3 = GemmSplit<512, 512, 1, 128, 1, 32, 2, 4, 1, 1, 64, kRows, 1, 1, 0, false>;     // 4 x 2 tiles x 32 = 256
 
 // conv2d_1: the convolution of pair 3;  conv2d_4: 128 -> 128 channels on 28 x 28, 32 output channels x 16 pixels
 // per workgroup, four waves take two 16-channel groups each, 49 x 4 = 196 workgroups (eight waves on 16 channels x 32 pixels:
