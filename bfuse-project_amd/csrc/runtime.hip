@@ -78,8 +78,9 @@ struct Side {
     size_t bytes[3] = {0, 0, 0};
     int elem[3] = {4, 4, 4};
     hipStream_t stream = nullptr;                // S1 / S2
-    void* parts = nullptr;                       // workspace of operators that want an operand taken apart: made for the first of them,
-    size_t parts_bytes = 0;                      // never smaller again while the side lives
+    void* parts = nullptr;                       // workspace of operators that want an operand taken apart: made for the first of them, and
+    size_t parts_bytes = 0;                      // anew for one that needs more
+    std::vector<void*> outgrown;                 // smaller ones before, which launches under way may still use: they stay as long as the side
     bool live = false;
 };
 
@@ -207,6 +208,7 @@ int fini_side(int idx)
         s.parts = nullptr;
         s.parts_bytes = 0;
     }
+    for (; !s.outgrown.empty(); s.outgrown.pop_back()) HIP_TRY(hipFree(s.outgrown.back()));
     for (int i = 2; i >= 0; --i) {
         HIP_TRY(hipFree(s.buf[i]));
         s.buf[i] = nullptr;
@@ -331,13 +333,17 @@ int check_buffers(const Launchable& l, int k, int idx)
         if (s.bytes[i] < l.need[k][i])
             return fail(BFUSE_ERR_ARG, "%s needs %zu bytes for tensor %d, side %d holds %zu", l.side[k]->name.c_str(), l.need[k][i], i,
                         idx + 1, s.bytes[i]);
-    if (const size_t need = l.side[k]->parts_bytes; need > s.parts_bytes) {
-        DevBuf made;
-        HIP_TRY(hipMalloc(&made.p, need));
-        if (s.parts) HIP_TRY(hipFree(s.parts));   // waits for the launches that use it
-        s.parts = made.p;
-        made.p = nullptr;
-        s.parts_bytes = need;
+    if (const size_t need = l.side[k]->parts_bytes; need > 0) {
+        static std::mutex m;
+        std::lock_guard<std::mutex> lock(m);
+        if (need > s.parts_bytes) {
+            DevBuf made;
+            HIP_TRY(hipMalloc(&made.p, need));
+            if (s.parts) s.outgrown.push_back(s.parts);
+            s.parts = made.p;
+            made.p = nullptr;
+            s.parts_bytes = need;
+        }
     }
     return BFUSE_OK;
 }
