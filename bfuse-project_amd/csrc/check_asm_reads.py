@@ -21,8 +21,20 @@ compiler produced (`hipcc -save-temps`) and checks it:
 
 The scan is linear over each kernel's text (forward branches are passed straight through), which
 is how the hand-written sequences are laid out; operations the compiler itself has in flight are
-forgotten at basic-block boundaries (see below).  Usage: check_asm_reads.py file.s [...]; exit
-status 1 and one line per finding if anything is wrong.
+forgotten at basic-block boundaries (see below).
+
+Loads whose destination is LDS (`buffer_load_* ... lds`) have the opposite gap: the compiler waits
+neither for them before that place is read nor before something else is written there.  On the
+control-flow graph of every kernel that has such loads,
+
+  * an LDS write reached with one of them in flight is an error (the write could come first);
+  * one in flight behind a wait that says `loads into LDS have landed` is an error: such a wait counts
+    the loads behind them, which the compiler may have dropped or moved.
+
+(`global_load_lds_*`, issued from asm, are not followed: their kernels wait and meet by step numbers,
+which a graph does not show.)
+
+Usage: check_asm_reads.py file.s [...]; exit status 1 and one line per finding if anything is wrong.
 """
 import re
 import sys
@@ -42,6 +54,71 @@ def regs_of(text):
             for i in range(int(m.group(3)), int(m.group(4)) + 1):
                 out.add((kind, i))
     return out
+
+
+VMCNT = re.compile(r"vmcnt\((\d+)\)")
+LANDED = "; loads into LDS have landed"
+VMEM = ("buffer_", "global_", "scratch_", "flat_")
+
+
+def check_lds_loads(path):
+    """Findings on loads into LDS, and how many such loads there are.  The state at an instruction is how many vector
+    memory operations were issued behind the youngest load into LDS that may be in flight (None: there is none), the
+    least of all ways to get there; they retire in order, so `vmcnt(n)` ends it where n or more were."""
+    kernels, func = {}, None
+    for ln, raw in enumerate(open(path, errors="replace"), 1):
+        m = LABEL.match(raw)
+        if m:
+            if not m.group(1).startswith(".L"):
+                func = kernels.setdefault(m.group(1), [])
+            elif func is not None:
+                func.append((ln, "label", m.group(1)))
+            continue
+        s = raw.split(";", 1)[0].strip()
+        if func is None or not s or s.startswith((".", "//")):
+            continue
+        mn, _, ops = s.partition(" ") if " " in s else s.partition("\t")
+        func.append((ln, mn, ops.strip() + (LANDED if LANDED in raw else "")))
+    findings, n_loads = [], 0
+    for name, code in kernels.items():
+        is_load = [mn.startswith("buffer_load") and re.search(r"\blds\b", ops) is not None for _, mn, ops in code]
+        if not any(is_load):
+            continue
+        n_loads += sum(is_load)
+        at = {ops: i for i, (_, mn, ops) in enumerate(code) if mn == "label"}
+        landed = {i for i, (_, _, ops) in enumerate(code) if LANDED in ops}
+        behind = {}                      # instruction -> state on entry
+        todo, bad = [(0, None)], set()
+        while todo:
+            i, y = todo.pop()
+            while i < len(code):
+                if i in behind and (y is None or (behind[i] is not None and behind[i] <= y)):
+                    break
+                y = behind[i] = y if i not in behind or behind[i] is None else min(y, behind[i])
+                ln, mn, ops = code[i]
+                if mn == "s_waitcnt":
+                    m = VMCNT.search(ops)
+                    if m and y is not None and y >= int(m.group(1)):
+                        y = None
+                    if y is not None and i in landed:
+                        bad.add(i)
+                elif mn.startswith("ds_write") and y is not None:
+                    bad.add(i)
+                elif is_load[i]:
+                    y = 0
+                elif mn.startswith(VMEM) and y is not None:
+                    y = min(y + 1, 64)
+                if mn in ("s_endpgm", "s_setpc_b64"):
+                    break
+                if mn.startswith("s_cbranch") or mn == "s_branch":
+                    if ops in at:
+                        todo.append((at[ops], y))
+                    if mn == "s_branch":
+                        break
+                i += 1
+        for i in sorted(bad)[:3]:
+            findings.append(f"{path}:{code[i][0]}: {name}: `{code[i][1]} {code[i][2]}` with a load into LDS in flight")
+    return findings, n_loads
 
 
 def counts_in_lgkm(mn):
@@ -145,10 +222,12 @@ def main():
     bad = 0
     for path in sys.argv[1:]:
         findings, n = check(path)
+        more, n_loads = check_lds_loads(path)
+        findings += more
         for f in findings[:50]:
             print("error:", f)
         bad += len(findings)
-        print(f"{path}: {n} hand-issued LDS reads checked, {len(findings)} findings")
+        print(f"{path}: {n} hand-issued LDS reads and {n_loads} loads into LDS checked, {len(findings)} findings")
     sys.exit(1 if bad else 0)
 
 

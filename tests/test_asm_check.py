@@ -84,15 +84,59 @@ def test_the_compilers_own_reads_are_not_tracked_but_take_a_counter_slot(tmp_pat
     assert n == 1 and findings == []
 
 
+LDS_LOAD = "\tbuffer_load_dwordx4 v5, s[0:3], 0 offen lds\n"
+LOAD = "\tbuffer_load_dwordx4 v[8:11], v6, s[4:7], 0 offen\n"
+WRITE = "\tds_write_b128 v0, v[42:45]\n"
+LANDED = "\t;;#ASMSTART\n\ts_waitcnt vmcnt({n}) ; loads into LDS have landed\n\t;;#ASMEND\n"
+
+
+def _lds(tmp_path, body):
+    p = tmp_path / "k.s"
+    p.write_text("kern:\n" + body + "\ts_endpgm\n.Lfunc_end0:\n")
+    return chk.check_lds_loads(str(p))
+
+
+def test_a_write_to_lds_with_a_load_into_it_in_flight_is_flagged(tmp_path):
+    # what was found: a loop of one stage, whose last loads into LDS nothing waits for before the partial sums go there
+    findings, n = _lds(tmp_path, LDS_LOAD + LOAD * 2 + LANDED.format(n=2) + LDS_LOAD * 2 + "\ts_waitcnt vmcnt(4)\n" + WRITE + "\ts_waitcnt vmcnt(0)\n")
+    assert n == 3 and len(findings) == 1 and "ds_write_b128" in findings[0]
+    findings, _ = _lds(tmp_path, LDS_LOAD + LOAD * 2 + LANDED.format(n=2) + LDS_LOAD * 2 + LANDED.format(n=0) + WRITE)
+    assert findings == []
+    # the compiler's own wait for a register load behind it is as good
+    findings, _ = _lds(tmp_path, LDS_LOAD + LOAD + "\ts_waitcnt vmcnt(1)\n" + WRITE)
+    assert findings == []
+
+
+def test_a_wait_that_counts_loads_that_are_not_there_is_flagged(tmp_path):
+    findings, _ = _lds(tmp_path, LDS_LOAD + LOAD + LANDED.format(n=2))
+    assert len(findings) == 1 and "landed" in findings[0]
+
+
+def test_loads_into_lds_are_followed_round_loops_and_over_branches(tmp_path):
+    findings, _ = _lds(tmp_path, LDS_LOAD + LOAD * 2 + ".LBB0_1:\n" + LANDED.format(n=2) + LDS_LOAD + LOAD * 2 + "\ts_cbranch_scc1 .LBB0_1\n" + LANDED.format(n=0) + WRITE)
+    assert findings == []
+    # one load fewer behind it in the loop than in front of it
+    findings, _ = _lds(tmp_path, LDS_LOAD + LOAD * 2 + ".LBB0_1:\n" + LANDED.format(n=2) + LDS_LOAD + LOAD + "\ts_cbranch_scc1 .LBB0_1\n" + LANDED.format(n=0) + WRITE)
+    assert len(findings) == 1 and "landed" in findings[0]
+    # a branch past the wait
+    findings, _ = _lds(tmp_path, LDS_LOAD + "\ts_cbranch_scc1 .LBB0_2\n" + LANDED.format(n=0) + ".LBB0_2:\n" + WRITE)
+    assert len(findings) == 1 and "ds_write_b128" in findings[0]
+    # another side's code, which no such load leads to
+    findings, _ = _lds(tmp_path, "\ts_cbranch_scc1 .LBB0_2\n" + LDS_LOAD + "\ts_endpgm\n.LBB0_2:\n" + WRITE)
+    assert findings == []
+
+
 def test_the_built_kernels_pass(tmp_path):
     import glob
     files = glob.glob(os.path.join(ROOT, "bfuse-project_amd", "csrc", "obj", "kernels_*-gfx950.s"))
     if not files:
         import pytest
         pytest.skip("device assembly not present (library not built in this tree)")
-    total = 0
+    total = loads = 0
     for f in files:
         findings, n = chk.check(f)
-        assert findings == [], findings[:3]
-        total += n
+        more, m = chk.check_lds_loads(f)
+        assert findings + more == [], (findings + more)[:3]
+        total, loads = total + n, loads + m
     assert total > 1000          # the GEMMs' hand-issued reads were found and followed
+    assert loads > 100           # ... and the loads into LDS
