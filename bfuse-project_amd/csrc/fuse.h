@@ -25,7 +25,9 @@
 //
 // Kernel ABI, as in the reference (macro_h.py:182-198): extern "C", three pointers per
 // operator (input, second operand, output), six for a fused pair (operator 1's three, then
-// operator 2's), 1-D launch, no dynamic shared memory.
+// operator 2's), 1-D launch, no dynamic shared memory.  An operator that wants an operand taken
+// apart first (Prepares, below) has a workspace in that operand's place, which only a kernel of its
+// own in front of this one fills: the library's launches do that, a bare launch of the symbol does not.
 //
 // The reference's emitter fuses a LIST of kernels (horizontal-fuser/src/Algorithms.cc:23-35,
 // 540-566: the maps take any number of grids; Matchers.cc:523-602 concatenates the parameter
@@ -402,7 +404,7 @@ struct KernelEntry {
     const void* parts_func = nullptr;  // single: the kernel that takes operand `parts_operand` apart before a launch (see Prepares)
     int parts_operand = -1;
     unsigned parts_grid = 0, parts_block = 0;
-    size_t parts_bytes = 0;            // the workspace it writes, which the operator then gets in the operand's place
+    size_t parts_bytes = 0;            // the workspace it writes (one for each operator and side), which the operator then gets in the operand's place
 };
 
 // An operator that wants one of its operands taken apart first (PARTS_OPERAND: 0 = I, 1 = F) declares a kernel for that (Parts):

@@ -78,9 +78,12 @@ struct Side {
     size_t bytes[3] = {0, 0, 0};
     int elem[3] = {4, 4, 4};
     hipStream_t stream = nullptr;                // S1 / S2
-    void* parts = nullptr;                       // workspace of operators that want an operand taken apart: made for the first of them, and
-    size_t parts_bytes = 0;                      // anew for one that needs more
-    std::vector<void*> outgrown;                 // smaller ones before, which launches under way may still use: they stay as long as the side
+    // Workspaces of operators that want an operand taken apart, one for each operator (by its handle) that has been launched on this
+    // side, as long as the side.  Such a launch is two kernels, and other threads' launches on the side may come between them: those
+    // of the same operator write the same parts of the same operand there, those of others have their own place.
+    std::unordered_map<const void*, void*> parts;
+    std::mutex parts_mutex;
+    std::atomic<bool> has_parts{false};
     bool live = false;
 };
 
@@ -203,12 +206,14 @@ int fini_side(int idx)
     Side& s = g.side[idx];
     if (!s.live) return fail(BFUSE_ERR_STATE, "kernel%d is not initialized", idx + 1);
     HIP_TRY(hipStreamDestroy(s.stream));
-    if (s.parts) {
-        HIP_TRY(hipFree(s.parts));
-        s.parts = nullptr;
-        s.parts_bytes = 0;
+    {
+        std::lock_guard<std::mutex> lock(s.parts_mutex);
+        while (!s.parts.empty()) {
+            HIP_TRY(hipFree(s.parts.begin()->second));
+            s.parts.erase(s.parts.begin());
+        }
+        s.has_parts = false;
     }
-    for (; !s.outgrown.empty(); s.outgrown.pop_back()) HIP_TRY(hipFree(s.outgrown.back()));
     for (int i = 2; i >= 0; --i) {
         HIP_TRY(hipFree(s.buf[i]));
         s.buf[i] = nullptr;
@@ -324,7 +329,7 @@ int check_launch(const void* func, const unsigned* grid, const unsigned* block, 
 }
 
 // Buffers an operator touches must be at least as large as the shapes its kernel was built for.  The workspace for an operand that is
-// taken apart is made here, by the first check of such an operator and so before any of its launches is enqueued or captured.
+// taken apart is made here, by the operator's first check on this side and so before any of its launches is enqueued or captured.
 int check_buffers(const Launchable& l, int k, int idx)
 {
     Side& s = g.side[idx];
@@ -333,16 +338,18 @@ int check_buffers(const Launchable& l, int k, int idx)
         if (s.bytes[i] < l.need[k][i])
             return fail(BFUSE_ERR_ARG, "%s needs %zu bytes for tensor %d, side %d holds %zu", l.side[k]->name.c_str(), l.need[k][i], i,
                         idx + 1, s.bytes[i]);
-    if (const size_t need = l.side[k]->parts_bytes; need > 0) {
-        static std::mutex m;
-        std::lock_guard<std::mutex> lock(m);
-        if (need > s.parts_bytes) {
+    if (const KernelEntry& e = *l.side[k]; e.parts_func) {
+        std::lock_guard<std::mutex> lock(s.parts_mutex);
+        if (!s.parts.count(e.func)) {
             DevBuf made;
-            HIP_TRY(hipMalloc(&made.p, need));
-            if (s.parts) s.outgrown.push_back(s.parts);
-            s.parts = made.p;
+            HIP_TRY(hipMalloc(&made.p, e.parts_bytes));
+            try {
+                s.parts.emplace(e.func, made.p);
+            } catch (const std::bad_alloc&) {
+                return fail(BFUSE_ERR_HIP, "out of host memory");
+            }
             made.p = nullptr;
-            s.parts_bytes = need;
+            s.has_parts = true;
         }
     }
     return BFUSE_OK;
@@ -366,20 +373,26 @@ int check_fused_fits(const void* func, const int* sides = nullptr)
     return BFUSE_OK;
 }
 
-// Takes an operand of this operator apart if it wants that, and puts the workspace in the operand's place among its three arguments.
-// The first kernel of a launch records its start event.
-int launch_parts(const KernelEntry* e, int idx, void** args, hipStream_t stream, hipEvent_t& ev0)
+// Takes an operand of this operator apart if it wants that, and puts the workspace (kept in `parts`) in the operand's place among its
+// three arguments.  The first kernel of a launch records its start event.
+int launch_parts(const KernelEntry* e, int idx, void** args, void*& parts, hipStream_t stream, hipEvent_t& ev0)
 {
     if (!e || !e->parts_func) return BFUSE_OK;
     Side& s = g.side[idx];
-    void* own[2] = {args[e->parts_operand], &s.parts};
+    {
+        std::lock_guard<std::mutex> lock(s.parts_mutex);
+        auto it = s.parts.find(e->func);
+        if (it == s.parts.end()) return fail(BFUSE_ERR_STATE, "%s: side %d has no workspace for it", e->name.c_str(), idx + 1);
+        parts = it->second;
+    }
+    void* own[2] = {args[e->parts_operand], &parts};
     if (ev0)
         HIP_TRY(hipExtLaunchKernel(e->parts_func, dim3(e->parts_grid), dim3(e->parts_block), own, 0, stream, ev0, nullptr, 0));
     else
         HIP_TRY(hipLaunchKernel(e->parts_func, dim3(e->parts_grid), dim3(e->parts_block), own, 0, stream));
     g_in_flight.add();
     ev0 = nullptr;
-    args[e->parts_operand] = &s.parts;
+    args[e->parts_operand] = &parts;
     return BFUSE_OK;
 }
 
@@ -388,8 +401,9 @@ int launch3(const void* func, const unsigned* grid, const unsigned* block, int i
 {
     Side& s = g.side[idx];
     void* args[3] = {&s.buf[0], &s.buf[1], &s.buf[2]};
-    if (s.parts)   // (a side that has had such an operator)
-        if (int rc = launch_parts(entry_of(func), idx, args, stream, ev0)) return rc;
+    void* parts = nullptr;
+    if (s.has_parts)   // (a side that has had such an operator)
+        if (int rc = launch_parts(entry_of(func), idx, args, parts, stream, ev0)) return rc;
     if (ev0 || ev1)
         HIP_TRY(hipExtLaunchKernel(func, d3(grid), d3(block), args, 0, stream, ev0, ev1, 0));
     else
@@ -405,9 +419,10 @@ int launch_fused(const void* func, const unsigned* grid, const unsigned* block, 
     void* args[3 * kMaxKernels + 1] = {};
     for (int k = 0; k < n; ++k)
         for (int i = 0; i < 3; ++i) args[3 * k + i] = &g.side[sides[k]].buf[i];
+    void* parts[kMaxKernels] = {};
     for (int k = 0; k < n; ++k)
-        if (g.side[sides[k]].parts)
-            if (int rc = launch_parts(launchable(func)->side[k], sides[k], args + 3 * k, stream, ev0)) return rc;
+        if (g.side[sides[k]].has_parts)
+            if (int rc = launch_parts(launchable(func)->side[k], sides[k], args + 3 * k, parts[k], stream, ev0)) return rc;
     // a run-time-plan kernel takes its installed plan by value as its last argument
     auto it = installed_plans().find(func);
     if (it != installed_plans().end()) args[3 * n] = &it->second;

@@ -411,3 +411,14 @@ def test_split_convolution_of_many_taps(tag, s, p, side, scale):
     for part in [(n, slice(None)) for n in range(x.shape[0])] + [(slice(None), m) for m in range(w.shape[0])]:
         ok = np.isfinite(f[part])
         assert np.linalg.norm(y[part][ok] - want[part][ok]) <= u * np.linalg.norm(want[part][ok])
+
+
+def test_a_fused_kernel_of_two_operators_whose_operands_are_taken_apart():
+    a, b = "selftest_conv_split_a", "selftest_gemm_split_r_p"
+    with bf.Operation(a, b) as op:
+        X = [fill_normal(51 + i, int(np.prod(k.shapes[0])), 0, 1) for i, k in enumerate(op.k)]
+        for seed in (61, 71):                          # new filters with every launch
+            W = [fill_normal(seed + i, int(np.prod(k.shapes[1])), 0, 1) for i, k in enumerate(op.k)]
+            want = [op.run_kernel(i, X[i], W[i]) for i in (0, 1)]
+            got = op.run_fuse(op.fused("bfuse", "_c4"), X[0], W[0], X[1], W[1])
+            assert all(np.array_equal(g.view(np.uint32), w.view(np.uint32)) for g, w in zip(got, want))
