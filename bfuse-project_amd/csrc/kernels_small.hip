@@ -273,10 +273,6 @@ PARTS_TEST(i, SwapOperands<PARTS_OF(64, 144, 9, 7, 1, 5, 2, 2, 1, 1, 64, kPix, 3
 PARTS_TEST(j, SwapOperands<PARTS_OF(48, 216, 17, 17, 2, 3, 1, 3, 1, 1, 128, kPix, 3, 3, 0)>, DIMS4(3, 24, 17, 17), DIMS4(48, 24, 3, 3), DIMS4(3, 48, 8, 8))
 PARTS_TEST(l, SwapOperands<PARTS_OF(80, 480, 12, 10, 3, 7, 1, 4, 1, 1, 112, kPix, 5, 6, 2)>, DIMS4(7, 16, 12, 10), DIMS4(80, 16, 5, 6), DIMS4(7, 80, 4, 3))
 PARTS_TEST(r, SwapOperands<PARTS_OF(160, 64, 9, 9, 1, 5, 1, 10, 1, 1, 128, kPix, 1, 1, 0)>, DIMS4(5, 64, 9, 9), DIMS4(160, 64, 1, 1), DIMS4(5, 160, 9, 9))
-// ... and of 31 and more taps: a reduction that is no whole octet, one that is, stride and filter alike.
-PARTS_TEST(u, SwapOperands<PARTS_OF(64, 147, 15, 18, 2, 3, 1, 4, 1, 1, 128, kPix, 7, 7, 3)>, DIMS4(3, 3, 15, 18), DIMS4(64, 3, 7, 7), DIMS4(3, 64, 8, 9))
-CONV_SPLIT_TEST(v, 4, 32, 11, 10, 6, 6, 1, 2, 3, 1, 2, 1, 1, 64)
-CONV_SPLIT_TEST(w, 3, 96, 40, 33, 8, 8, 8, 0, 5, 3, 2, 1, 1, 64)
 BFUSE_BFUSE_KERNEL(selftest_gemm_split_r_p, Narrow<GemmSpP_r>, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
 
 // The convolution from a patch taken apart once: pixels that run on into the next images and past the batch, rectangles past an image's

@@ -297,8 +297,8 @@ struct ConvF32Rect {
 // KS waves, which split the channels.  A shared tile like ConvF32Tile, whose place it takes: only what a workgroup does with it differs.
 constexpr int kSplitForm = 32;
 template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int BM, int PB, int KS, int NIMG>
-struct ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, KS, NIMG, kSplitForm> : ConvF32Tile<(CI + 3) / 4 * 4, CO, H, W, KH, KW, S, P, BM, PB % 4 == 0 ? 16 * PB : 128, 1, NIMG> {
-    using Form = SwapOperands<GemmSplit<CO, CI * KH * KW, H, W, S, NIMG, BM / 16 / KS, KS, 1, 1, 16 * PB, kPix, KH, KW, P, false, (CI * KH * KW >= 256 || CI * KH * KW % 8 != 0)>>;
+struct ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, KS, NIMG, kSplitForm> : ConvF32Tile<CI, CO, H, W, KH, KW, S, P, BM, PB % 4 == 0 ? 16 * PB : 128, 1, NIMG> {
+    using Form = SwapOperands<GemmSplit<CO, CI * KH * KW, H, W, S, NIMG, BM / 16 / KS, KS, 1, 1, 16 * PB, kPix, KH, KW, P, false, (CI * KH * KW >= 256)>>;
     using Parts = typename Form::Parts;
     static constexpr int PARTS_OPERAND = Form::PARTS_OPERAND;
     static constexpr long long TILES = Form::TILES;
@@ -477,16 +477,12 @@ struct ConvTiling {
     static constexpr int ROUNDS8 = (int)(((long long)((OHW + 3) / 4 * 4) * NIMG + 127) / 128 * (CO / 256) + 255) / 256, ROUNDS7 = (int)(((long long)((OHW + 3) / 4 * 4) * NIMG + 111) / 112 * (CO / 256) + 255) / 256;
     static constexpr int PB256 = 112 * ROUNDS7 < 0.97 * 128 * ROUNDS8 ? 7 : 8;
     using split = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, SBM, SBM == 256 ? PB256 : SBM == 192 || SBM == 96 ? 4 : 8, SBM == 256 ? 8 : SBM == 160 ? 10 : SBM == 96 ? 2 : 4, NIMG, kSplitForm>;
+    // Filters of 31 and more taps are left to the per-wave forms: as products 7 x 7 on RGB took 2363 us instead of 3367, but a window with one element that is not
+    // zero came out up to 2.4 u off instead of 1, and one wave without barriers can be thread-fused with any operator.
     static constexpr bool is_split()
     {
         // (the table of taps is made at compile time)
         if constexpr (T > 1 && T < 31 && CI % 16 == 0 && CI * T <= 32768 && CO % SBM == 0 && !(SBM == 64 && S == 2))
-            return split::FITS && split::TILES >= 512;
-        // 31 to 64 taps, whatever the channels: the per-wave forms have a register for every tap and 16 rows, so that a workgroup has 16 of the output channels
-        // and stages the images anew for the next 16.  us, those and these: 3 -> 64 of 7 x 7 at stride 2 on 224 x 224, batch 1024, 3367 -> 2363 (64 columns as fast, two waves of
-        // 32 rows 2684; 103 TFLOP/s: three vector instructions and a load for every element of every window are what bounds it); batch 256: the same 858 -> 613, -> 128 1703 -> 943, at stride 1 on
-        // 112 x 112 1030 -> 573, 3 -> 192 of 8 x 8 at stride 8 1182 -> 154, 16 -> 96 on 35 x 35 575 -> 279, 4 -> 64 of 6 x 6 446 -> 417.
-        if constexpr (T >= 31 && KH <= 8 && KW <= 8 && CI * T >= 128 && CI * T <= 32768 && CI * H * W < 1 << 22 && CO % SBM == 0)
             return split::FITS && split::TILES >= 512;
         return false;
     }

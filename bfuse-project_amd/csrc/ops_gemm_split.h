@@ -77,7 +77,7 @@ namespace bfuse {
 // come from the caches: 256 x 2304 in 5 us.
 template <int M, int K, int TAPS, bool ON = true>
 struct SplitParts {
-    static_assert(!ON || (M % 16 == 0 && (TAPS == 1 || K % (32 * TAPS) == 0)), "parts");
+    static_assert(!ON || (M % 16 == 0 && K % 8 == 0 && (TAPS == 1 || K % (32 * TAPS) == 0)), "parts");
     static constexpr int PARTS_THREADS = 256;
     static constexpr int STAGES = (K + 31) / 32, CHUNK = TAPS > 1 ? TAPS : 8, CHUNKS = (STAGES + CHUNK - 1) / CHUNK;
     static constexpr int BLOCK_BYTES = STAGES * 3072, HEAD = (64 + M / 16 * CHUNKS * 4 + 1023) / 1024 * 1024;
@@ -107,7 +107,7 @@ struct SplitParts {
             float x[8];
             const int k = TAPS > 1 ? (chunk * 32 + (lane >> 4) * 8) * TAPS + s % TAPS : s * 32 + (lane >> 4) * 8;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] = K % 32 == 0 || (K % 8 == 0 ? k : k + e) < K ? row[k + e * TAPS] : 0.f;
+            for (int e = 0; e < 8; ++e) x[e] = K % 32 == 0 || k < K ? row[k + e * TAPS] : 0.f;
             unsigned p[3][4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) split2(x[2 * j], x[2 * j + 1], p[0][j], p[1][j], p[2][j], left);
@@ -149,7 +149,7 @@ struct GemmSplit {
     // one address serves them all
     static constexpr bool EVEN = 4 * BU % GT == 0 && GT % (LAYOUT == kRows ? 4 : BU) == 0;
     static constexpr int NUB = EVEN ? 1 : NUJ;
-    static_assert(BN % (16 * WN) == 0 && (K % 8 == 0 || (PREP && T > 1)) && NS % KG == 0 && M >= BM && (LAYOUT == kPix || (W >= BN && H == 1 && S == 1)), "tile");
+    static_assert(BN % (16 * WN) == 0 && K % 8 == 0 && NS % KG == 0 && M >= BM && (LAYOUT == kPix || (W >= BN && H == 1 && S == 1)), "tile");
     // 31-bit offsets; padding is read through one that lies past the buffer
     static constexpr bool FITS = (long long)BM * K * 4 < (1LL << 31) && (long long)(NIMAGES < NIMG ? NIMAGES : NIMG) * CI * HW * 4 < (1LL << (T == 1 ? 31 : 29));
     static constexpr bool TURNED = LAYOUT == kRows && NS > 2;
@@ -169,30 +169,16 @@ struct GemmSplit {
     };
 
     // Filters larger than 1 x 1: where element k = (channel, row, column) of a window lies from its first one, in bytes, times
-    // eight, and the tap's number in the low five bits; past the last k a tap that no window has.  MANY taps, for whose numbers these bits do not
-    // do: in words, times 2^10, and below that where `outside` has the bits of the tap's column and row.
-    static constexpr bool MANY = T >= 31;
+    // eight, and the tap's number in the low five bits; past the last k a tap that no window has.
     struct Taps {
         unsigned at[T > 1 ? NS * 32 : 1];
         constexpr Taps() : at{}
         {
-            for (int k = 0; T > 1 && k < NS * 32; ++k) {
-                const unsigned words = (unsigned)(k / T * HW + k % T / KW * W + k % KW);
-                if (MANY) at[k] = k < K ? words << 10 | (unsigned)(8 + k % KW) << 5 | (unsigned)(k % T / KW) : 31u << 5 | 31u;
-                else at[k] = k < K ? words * 4 << 3 | (unsigned)(k % T) : 31u;
-            }
+            for (int k = 0; T > 1 && k < NS * 32; ++k) at[k] = k < K ? (unsigned)((k / T * HW + k % T / KW * W + k % KW) * 4) << 3 | (unsigned)(k % T) : 31u;
         }
     };
     __device__ static constexpr Taps TAPS{};
-    static constexpr int bytes_of(unsigned at) { return MANY ? (int)(at >> 10) * 4 : (int)(at >> 5) * 4; }
-    // all ones (past the buffer) if a bit of this tap is set in `outside`
-    __device__ static __forceinline__ unsigned past(unsigned outside, unsigned at)
-    {
-        unsigned o = (unsigned)__builtin_amdgcn_sbfe((int)outside, at, 1);
-        if constexpr (MANY) o |= (unsigned)__builtin_amdgcn_sbfe((int)outside, at >> 5, 1);
-        return o;
-    }
-    static_assert(T == 1 || (LAYOUT == kPix && BN >= 64 && (!MANY || (KH <= 8 && KW <= 8 && CI * HW < 1 << 22)) && K % T == 0), "taps");
+    static_assert(T == 1 || (LAYOUT == kPix && BN >= 64 && T < 31 && K % T == 0), "taps");
 
     // (column tile, row tile), dealt so that the row tiles of one column tile follow each other on one XCD
     template <int NT = GemmSplit::NT>
@@ -221,14 +207,7 @@ struct GemmSplit {
         const int v = v0 + c, img = v / OHWP, p = v % OHWP, y = (p / OW) * S, x = (p % OW) * S;
         const bool in = p < OHW && n_lo + img < NIMG;
         outside = in ? 0x80000000u : ~0u;
-        if constexpr (P > 0 && MANY) {
-#pragma unroll
-            for (int i = 0; i < KH; ++i)
-                if (y + i < P || y + i >= H + P) outside |= 1u << i;
-#pragma unroll
-            for (int i = 0; i < KW; ++i)
-                if (x + i < P || x + i >= W + P) outside |= 256u << i;
-        } else if constexpr (P > 0)
+        if constexpr (P > 0)
 #pragma unroll
             for (int t = 0; t < T; ++t)
                 if (y + t / KW < P || y + t / KW >= H + P || x + t % KW < P || x + t % KW >= W + P) outside |= 1u << t;
@@ -334,8 +313,9 @@ struct GemmSplit {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     const unsigned at = TAPS.at[s * 32 + b_k[i] + (EVEN ? 8 * j * (GT / BU) : 0) + e];
-                    const unsigned o = P > 0 || TAIL != 0 ? past(b_out[i], at) : 0u;   // (without padding only the last stage has such)
-                    rb[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(br, v | o, bytes_of(at), 0));
+                    // all ones (past the buffer) if this tap's bit is set; without padding only the last stage has such
+                    const unsigned o = P > 0 || TAIL != 0 ? (unsigned)__builtin_amdgcn_sbfe((int)b_out[i], at, 1) : 0u;
+                    rb[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(br, v | o, (at >> 5) * 4, 0));
                 }
             } else {
 #pragma unroll
@@ -577,7 +557,7 @@ struct GemmSplit {
                     for (int e = 0; e < 2; ++e)
 #pragma unroll
                         for (int tm = 0; tm < TM; ++tm)
-                            na[e][tm] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ar, K % 8 != 0 && k + eq + 4 * e >= K ? 0x7fffffff : (((wr * TM + tm) * 16 + ei) * K + eq + 4 * e) * 4, k * 4, 0));
+                            na[e][tm] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ar, (((wr * TM + tm) * 16 + ei) * K + eq + 4 * e) * 4, k * 4, 0));
                     unsigned at[2];
                     if constexpr (T > 1) {
                         unsigned t[8];
@@ -592,8 +572,8 @@ struct GemmSplit {
                         for (int b = 0; b < TN; ++b) {
                             unsigned o = bo[b];
                             if constexpr (T > 1) {
-                                o |= past(outside[b], at[e]);
-                                if (o != ~0u) o += bytes_of(at[e]);
+                                o |= (unsigned)__builtin_amdgcn_sbfe((int)outside[b], at[e], 1);
+                                if (o != ~0u) o += (at[e] >> 5) * 4;
                             }
                             nb[e][b] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(br, o, T > 1 ? 0 : (k + 4 * e) * B_K, 0));
                         }

@@ -146,3 +146,12 @@ def test_no_block_fused_pair_of_the_batch_suites_is_left_out_for_registers(i, tm
                         "-Rpass-analysis=kernel-resource-usage", "-I", build_pairs.CSRC, "-c", str(tmp_path / "pairs_0.hip"), "-o", str(tmp_path / "pairs_0.o")], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-2000:]
     assert f"Function Name: {k['name']}" in r.stderr and build_pairs.spilling_kernels(r.stderr) == []
+
+
+@pytest.mark.parametrize("k1,k2", [
+    # one wave without barriers beside operators that synchronise
+    ("conv7x7s2p3_f32_1024x3x224x224_64", "bgemm_f32_1024x512x64x512"), ("conv7x7s2p3_f32_1024x3x224x224_64", "conv1x1s1p0_f32_1024x2048x8x8_320"),
+    ("conv7x7s2p3_f32_1024x3x224x224_64", "conv3x3s2p0_f32_1024x192x17x17_320"), ("conv7x7s2p3_f32_1024x3x224x224_64", "gemm_f32_1024x768x2304")])
+def test_operators_that_one_workgroup_can_hold(k1, k2):
+    reg = {k.name: k for k in bf.list_kernels()}
+    assert build_pairs.hfuse_possible(reg[k1], reg[k2], build_pairs.op_lds(k1), build_pairs.op_lds(k2))

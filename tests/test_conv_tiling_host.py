@@ -122,14 +122,3 @@ def test_places_of_a_patch_against_a_look_at_every_tile(tmp_path):
         static_assert(ConvTiling<256, 256, 14, 14, 3, 3, 1, 1, 64>::patch_form() == 0 && ConvTiling<64, 64, 56, 56, 5, 5, 1, 2, 1024>::patch_form() == 0);   // few tiles; 25 taps
     """
     _compiles(text, tmp_path)
-
-
-def test_filters_of_many_taps_are_products(tmp_path):
-    _compiles("""
-        static_assert(ConvTiling<3, 64, 224, 224, 7, 7, 2, 3, 1024>::is_split() && ConvTiling<16, 96, 35, 35, 7, 7, 1, 3, 256>::is_split() && ConvTiling<3, 192, 224, 224, 8, 8, 8, 0, 256>::is_split());
-        static_assert(!ConvTiling<3, 64, 224, 224, 9, 9, 2, 3, 1024>::is_split() && !ConvTiling<3, 64, 224, 224, 5, 5, 2, 2, 1024>::is_split());    // tap bits; few taps of few channels
-        static_assert(!ConvTiling<64, 64, 256, 256, 7, 7, 1, 3, 1024>::is_split() && !ConvTiling<3, 48, 224, 224, 7, 7, 2, 3, 1024>::is_split());   // an image of 2^22 words; rows that do not divide
-        constexpr auto first = GemmSplit<64, 147, 224, 224, 2, 1024, 1, 4, 1, 1, 128, kPix, 7, 7, 3, false, true>::Taps{};
-        static_assert(GemmSplit<64, 147, 224, 224, 2, 1024, 1, 4, 1, 1, 128, kPix, 7, 7, 3, false, true>::bytes_of(first.at[49 + 7 * 2 + 3]) == (224 * 224 + 2 * 224 + 3) * 4);
-        static_assert((first.at[49 + 7 * 2 + 3] & 31) == 2 && (first.at[49 + 7 * 2 + 3] >> 5 & 31) == 8 + 3 && (first.at[147] & 31) == 31 && (first.at[159] >> 5 & 31) == 31);
-    """, tmp_path)

@@ -384,35 +384,6 @@ def test_an_operand_taken_apart_before_gives_the_same_bits(tag, side, value):
             assert np.array_equal(op.run_fuse(op.fused("bfuse", "_c4"), x, w, *P)[0].view(np.uint32), a.view(np.uint32))
 
 
-@pytest.mark.parametrize("tag,s,p", [("u_p", 2, 3), ("v", 1, 2), ("w", 8, 0)])
-@pytest.mark.parametrize("side", [None, 0, 1])
-@pytest.mark.parametrize("scale", [1.0, 2.0 ** -118, 2.0 ** -140])
-def test_split_convolution_of_many_taps(tag, s, p, side, scale):
-    """31 and more taps: against 64 bits with ordinary values, and with infinite, NaN and tiny ones in an operand, which are in the
-    results that have them in their window or filter and in no others (a filter that is no whole octet ends in the next one's first values)."""
-    name = f"selftest_gemm_split_{tag}"
-    x, w = _operands(name)
-    if side is None:
-        _check(name, lambda a, b: orf.conv2d(a, b, s=s, p=p), "bias_relu_4096", None, "")
-    elif side == 0:
-        w = (np.abs(w) + np.float32(0.5)) * np.float32(2.0 ** 60)
-        x[0, 1, 0, 0], x[1, 2, 4, 3], x[-1, 0, 9, 7] = np.inf, np.nan, -np.inf
-        x[1] *= np.float32(scale)
-    else:
-        x = (np.abs(x) + np.float32(0.5)) * np.float32(2.0 ** 60)
-        w[1, 0, 0, 0], w[5, 2, 3, 3], w[-1, 1, 5, 5] = np.inf, np.nan, -np.inf
-        w[3] *= np.float32(scale)
-    with np.errstate(all="ignore"):
-        want = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(w).double(), stride=s, padding=p).numpy()
-        f = want.astype(np.float32)
-    y = _run(name, x, w)
-    assert np.array_equal(np.isnan(y), np.isnan(f)) and np.array_equal(np.isposinf(y), np.isposinf(f)) and np.array_equal(np.isneginf(y), np.isneginf(f))
-    u = 2.0 ** -24 * np.prod(w.shape[1:]) ** 0.5 * 2     # twice the bound of one sum rounded after every product
-    for part in [(n, slice(None)) for n in range(x.shape[0])] + [(slice(None), m) for m in range(w.shape[0])]:
-        ok = np.isfinite(f[part])
-        assert np.linalg.norm(y[part][ok] - want[part][ok]) <= u * np.linalg.norm(want[part][ok])
-
-
 def test_a_fused_kernel_of_two_operators_whose_operands_are_taken_apart():
     a, b = "selftest_conv_split_a", "selftest_gemm_split_r_p"
     with bf.Operation(a, b) as op:
