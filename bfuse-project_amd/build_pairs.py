@@ -20,8 +20,9 @@ Thread-level fusion is written only where it can work: both workgroups fit one (
 160 KB of LDS together) and at most one side synchronises (config.choose_fusion's rule).
 
 A fused kernel whose sides need more registers than its workgroup leaves them is not built as it stands: if a side
-has more than 512 threads (three waves on a SIMD: 168 registers for both sides) it takes that side's form of fewer
-waves (Narrow: the same tiles, the same bits), and what then still does not fit is left out and named.
+has more than 512 threads (three waves on a SIMD: 168 registers for both sides) it takes the other side's form of fewer
+registers (Slim), or that side's of fewer waves (Narrow: the same tiles, the same bits), and what then still does not
+fit is left out and named.
 """
 import argparse
 import os
@@ -197,18 +198,35 @@ def _edit_spilling(hip_dir: str, edit) -> List[str]:
     return changed
 
 
-def narrow_spilling(hip_dir: str, registry: Dict[str, object]) -> List[str]:
-    """Gives every kernel whose last compilation reported spills its sides of more than 512 threads in their form of
-    fewer waves (csrc/wave.h, Narrow)."""
+def _edit_sides(hip_dir: str, registry: Dict[str, object], edit_side) -> List[str]:
+    """_edit_spilling with `edit_side(type, threads, others, hfuse)` for the type of each side, of so many threads beside another's."""
     def edit(name, line):
         macro, args = line.rstrip(")").split("(", 1)
         a = [x.strip() for x in args.split(",")]
-        for i in (0, 2):
-            k = registry[a[i]]
-            if k.block[0] * k.block[1] * k.block[2] > 512 and not a[i + 1].startswith("Narrow<"):
-                a[i + 1] = f"Narrow<{a[i + 1]}>"
+        threads = [int(registry[a[i]].block[0] * registry[a[i]].block[1] * registry[a[i]].block[2]) for i in (0, 2)]
+        for j in (0, 1):
+            a[2 * j + 1] = edit_side(a[2 * j + 1], threads[j], threads[1 - j], macro == "BFUSE_HFUSE_KERNEL")
         return f"{macro}({', '.join(a)})"
     return _edit_spilling(hip_dir, edit)
+
+
+def slim_spilling(hip_dir: str, registry: Dict[str, object]) -> List[str]:
+    """Gives every kernel whose last compilation reported spills the sides that have only 168 registers because of the
+    other's threads in their form of fewer registers (csrc/wave.h, Slim)."""
+    def edit_side(t, threads, others, hfuse):
+        short = threads <= 512 and (threads + others if hfuse else others) > 512
+        return f"Slim<{t}>" if short and "<" not in t else t
+    return _edit_sides(hip_dir, registry, edit_side)
+
+
+def narrow_spilling(hip_dir: str, registry: Dict[str, object]) -> List[str]:
+    """Gives every kernel whose last compilation reported spills its sides of more than 512 threads in their form of
+    fewer waves (csrc/wave.h, Narrow), which leaves block-fused partners all they need: those are as they were again."""
+    def edit_side(t, threads, others, hfuse):
+        if threads > 512:
+            return t if t.startswith("Narrow<") else f"Narrow<{t}>"
+        return t[len("Slim<"):-1] if others > 512 and not hfuse and t.startswith("Slim<") else t
+    return _edit_sides(hip_dir, registry, edit_side)
 
 
 def drop_spilling(hip_dir: str) -> List[str]:
@@ -287,11 +305,12 @@ def build(suite: str, forms: str = "both", chunk: int = 256, only: Optional[Sequ
         cmd = ["make", "-C", CSRC, f"MODDIR={os.path.abspath(hip)}", f"-j{jobs}", "-k", "module"]
         r = subprocess.run(cmd, capture_output=True, text=True)
         # A fused kernel that needs more registers than its launch bounds leave (a side that already fills the
-        # register file, thread-fused with another) fails the library's no-spill check: its sides of many waves take
-        # their narrow form, then those that still spill are taken out of their translation units; anything else is
-        # an error.
-        if r.returncode != 0 and narrow_spilling(hip, registry):
-            r = subprocess.run(cmd, capture_output=True, text=True)
+        # register file, thread-fused with another) fails the library's no-spill check: the partner of a side of many
+        # waves takes its slim form, or that side its narrow one, then those that still spill are taken out of their
+        # translation units; anything else is an error.
+        for fit in (slim_spilling, narrow_spilling):
+            if r.returncode != 0 and fit(hip, registry):
+                r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             dropped = drop_spilling(hip)
             if dropped:

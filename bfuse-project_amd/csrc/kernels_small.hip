@@ -292,6 +292,10 @@ BFUSE_BFUSE_KERNEL(selftest_conv_split_a, ConvP_a, layernorm_8x256, LayerNormS, 
 BFUSE_HFUSE_KERNEL(selftest_conv_split_b, ConvP_b, bias_relu_4096, BiasReluS)
 BFUSE_HFUSE_KERNEL(selftest_conv_split_d, ConvP_d, conv3x3_f32_32x12x12_32, ConvS2)
 BFUSE_BFUSE_RT_KERNEL(selftest_conv_split_f, ConvP_f, layernorm_8x256, LayerNormS)
+// (beside ten waves: 168 registers)
+BFUSE_BFUSE_KERNEL(selftest_conv_split_a, Slim<ConvP_a>, gemm_bf16_256x448x1792_p2, GemmB9, _c4, bfuse::kChunked, 4, 1)
+BFUSE_BFUSE_KERNEL(selftest_conv_split_b, Slim<ConvP_b>, gemm_bf16_256x448x1792_p2, GemmB9, _c4, bfuse::kChunked, 4, 1)
+BFUSE_BFUSE_KERNEL(selftest_conv_split_d, Slim<ConvP_d>, gemm_bf16_256x448x1792_p2, GemmB9, _c4, bfuse::kChunked, 4, 1)
 BFUSE_BFUSE_KERNEL(selftest_conv_split_a, ConvP_a, selftest_gemm_split_r_p, Narrow<GemmSpP_r>, _c4, bfuse::kChunked, 4, 1)   // operands of both sides are taken apart
 
 // The split-K product on the bf16 matrix cores: a trailing 16-column group and GELU in one round, two waves in two rounds, one stage.

@@ -364,5 +364,9 @@ template <class Op>
 struct NarrowOf<SwapOperands<Op>> {
     using type = SwapOperands<Narrow<Op>>;
 };
+template <class Op>
+struct SlimOf<SwapOperands<Op>> {
+    using type = SwapOperands<Slim<Op>>;
+};
 
 }  // namespace bfuse

@@ -336,6 +336,10 @@ struct ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, TW, NIMG, kPatchForm> : Co
         Form::run(vblock, tid, sm, I, F, O, sync);
     }
 };
+template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int BM, int PB, int TW, int NIMG>
+struct SlimOf<ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, TW, NIMG, kPatchForm>> {
+    using type = Slim<typename ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, TW, NIMG, kPatchForm>::Form>;
+};
 
 // The tiling the library gives a convolution it has no hand-picked one for: as many output channels per
 // workgroup as keep the filter fragments of a wave within ~72 registers (the staged patch is shared by all

@@ -304,4 +304,10 @@ struct ConvSplit {
     }
 };
 
+// (see Slim) Waves of 16 rows, twice as many, read every fragment for half the MFMAs.
+template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int NIMG, int TM, int WR, int WN, int BN, int TW>
+struct SlimOf<ConvSplit<CI, CO, H, W, KH, KW, S, P, NIMG, TM, WR, WN, BN, TW>> {
+    using type = ConvSplit<CI, CO, H, W, KH, KW, S, P, NIMG, 1, TM * WR, WN, BN, TW>;
+};
+
 }  // namespace bfuse

@@ -262,4 +262,13 @@ struct NarrowOf {
 template <class Op>
 using Narrow = typename NarrowOf<Op>::type;
 
+// An operator in at most 168 registers a lane where it has such a form, otherwise itself: again the same tiles and bits, for a side that
+// leaves no more.  (Beside a ten-wave operator this costs less than that one's Narrow.)
+template <class Op>
+struct SlimOf {
+    using type = Op;
+};
+template <class Op>
+using Slim = typename SlimOf<Op>::type;
+
 }  // namespace bfuse

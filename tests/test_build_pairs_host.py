@@ -123,12 +123,47 @@ def test_kernels_that_spill_take_their_narrow_sides_and_are_left_out_only_then(t
     assert [l for l in (d / "pairs_0.hip").read_text().splitlines() if l.startswith("BFUSE_")] == [lines[4]]
 
 
+def test_a_partner_short_of_registers_takes_its_slim_form_first(tmp_path):
+    d = tmp_path / "hip"
+    d.mkdir()
+    reg = {k.name: k for k in (_k("a", 640, True), _k("b", 256, False), _k("c", 384, True))}
+    lines = ["BFUSE_BFUSE_KERNEL(a, Side0, b, Side1, _c256, bfuse::kChunked, 256, 1)", "BFUSE_BFUSE_KERNEL(c, Side2, b, Side1, _c256, bfuse::kChunked, 256, 1)",
+             "BFUSE_HFUSE_KERNEL(c, Side2, b, Side1)", "BFUSE_HFUSE_KERNEL(b, Side1, b, Side1)"]
+    names = ["a_b_fused_bfuse_c256", "c_b_fused_bfuse_c256", "c_b_fused_hfuse", "b_b_fused_hfuse"]
+    (d / "pairs_0.hip").write_text("\n".join(lines) + "\n")
+    (d / "pairs_0.res").write_text("".join(f"remark: Function Name: {n} [-R]\nremark:     ScratchSize [bytes/lane]: 8 [-R]\n" for n in names))
+    assert build_pairs.slim_spilling(str(d), reg) == [names[0], names[2]]           # nobody leaves the others less than 256
+    want = ["BFUSE_BFUSE_KERNEL(a, Side0, b, Slim<Side1>, _c256, bfuse::kChunked, 256, 1)", lines[1], "BFUSE_HFUSE_KERNEL(c, Slim<Side2>, b, Slim<Side1>)", lines[3]]
+    assert (d / "pairs_0.hip").read_text().splitlines() == want
+    assert build_pairs.slim_spilling(str(d), reg) == []
+    assert build_pairs.narrow_spilling(str(d), reg) == names[:1]                     # spilled again: 512 threads instead, and the partner as it was
+    assert (d / "pairs_0.hip").read_text().splitlines()[0] == "BFUSE_BFUSE_KERNEL(a, Narrow<Side0>, b, Side1, _c256, bfuse::kChunked, 256, 1)"
+
+
 def _suite_operators():
     out = set()
     for name in ("benchmark_batch1024", "inception_v3_batch1024", "interleave_scheduler_batch1024"):
         doc = configure.load_user_config(os.path.join(ROOT, "bfuse-project_amd", "examples", f"{name}.yaml"))
         out |= {k.name for k in configure.resolve(doc, {k.name: k for k in bf.list_kernels()}, None)[0].values()}
     return sorted(out)
+
+
+def _compiled(k, src, tmp_path):
+    (tmp_path / "pairs_0.hip").write_text(src)
+    r = subprocess.run(["/opt/rocm/bin/hipcc", "--offload-arch=gfx950", "--cuda-device-only", "-O3", "-std=c++17", "-ffp-contract=off", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                        "-Rpass-analysis=kernel-resource-usage", "-I", build_pairs.CSRC, "-c", str(tmp_path / "pairs_0.hip"), "-o", str(tmp_path / "pairs_0.o")], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    assert f"Function Name: {k['name']}" in r.stderr
+    return build_pairs.spilling_kernels(r.stderr)
+
+
+@pytest.mark.parametrize("k1", ["conv3x3s1p1_f32_1024x32x147x147_64", "conv3x3s1p1_f32_1024x64x56x56_64"])
+def test_patch_convolutions_fit_beside_ten_waves_in_their_slim_form(k1, tmp_path):
+    """... whose own form of five (which the bf16 product does not have) they then do not need."""
+    k = {"k1": k1, "k2": "gemm_bf16_512x4096x14336", "form": "bfuse", "name": f"{k1}_gemm_bf16_512x4096x14336_fused_bfuse_c256"}
+    assert bf.operation.kernel_info(k["k2"]).block[0] > 512
+    src = build_pairs.source_text([k]).replace("Side0, ", "Slim<Side0>, ") + "static_assert(Slim<Side0>::GRID.size() == Side0::GRID.size());\n"
+    assert _compiled(k, src, tmp_path) == []
 
 
 @pytest.mark.parametrize("i", range(4))

@@ -393,3 +393,21 @@ def test_a_fused_kernel_of_two_operators_whose_operands_are_taken_apart():
             want = [op.run_kernel(i, X[i], W[i]) for i in (0, 1)]
             got = op.run_fuse(op.fused("bfuse", "_c4"), X[0], W[0], X[1], W[1])
             assert all(np.array_equal(g.view(np.uint32), w.view(np.uint32)) for g, w in zip(got, want))
+
+
+@pytest.mark.parametrize("tag", ["a", "b", "d"])
+@pytest.mark.parametrize("value", [1.0, 2.0 ** -120 * 1.2345678, np.inf])
+def test_a_patch_convolution_of_twice_the_waves_gives_the_same_bits(tag, value):
+    """Slim, beside ten waves: whatever values lie in either operand."""
+    name = f"selftest_conv_split_{tag}"
+    x, w = _operands(name)
+    with bf.Operation(name, "gemm_bf16_256x448x1792_p2") as op:
+        q = [fill_normal(81 + i, int(np.prod(op.k[1].shapes[i])), 0, 1) for i in (0, 1)]
+        q = [bf.operation.f32_to_bf16(v) for v in q]
+        for side in (0, 1):
+            a, b = x.copy(), w.copy()
+            (a, b)[side].reshape(-1)[[7, 1001]] = value
+            want = op.run_kernel(0, a, b), op.run_kernel(1, *q)
+            got = op.run_fuse(op.fused("bfuse", "_c4"), a, b, *q)
+            assert np.isfinite(want[0]).any()
+            assert np.array_equal(got[0].view(np.uint32), want[0].view(np.uint32)) and np.array_equal(got[1].view(np.uint16), want[1].view(np.uint16))
