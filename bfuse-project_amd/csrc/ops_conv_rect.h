@@ -496,8 +496,9 @@ struct ConvTiling {
     // computes least besides.  Measured: 14 x 14 on 112 900 us, on 96 926; 7 x 7 on 96 972, on 112 (one tile a CU) 1062; 8 x 8 on 128 755, on 64 793; 35 x 35 on 12 x 12
     // 702, on 12 x 8 760, on 36 x 4 806; 56 x 56 on 28 x 4 1242, on 16 x 8 1372; 147 x 147 on 16 x 7 4338, on 12 x 12 4424.  Where
     // none of these does (26 x 26), eight waves on 224 consecutive pixels, one tile a CU (1718 against split's 1887; 28 x 4 of 16 % outside 1766).
-    // 32 output channels: two waves on 224 pixels.
-    static constexpr int QBM = CO % 128 == 0 ? 128 : CO % 96 == 0 ? 96 : CO % 64 == 0 ? 64 : 32;
+    // Tiles have at least 64 of the output channels: a row tile takes its patch apart for itself, and 32 -> 32 on 149 x 149 was on the fp32
+    // instructions before, where a window with one element that is not zero is at most 1 u off and here up to 2.4 (2975 instead of 3479 us).
+    static constexpr int QBM = CO % 128 == 0 ? 128 : CO % 96 == 0 ? 96 : 64;
     template <int PB, int TW> using patch = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, QBM, PB, TW, NIMG, kPatchForm>;
     // what a tile costs a pixel: those outside the image, and a sixteenth part of a wave's columns that every tile takes besides
     template <int PB, int TW>
@@ -512,19 +513,13 @@ struct ConvTiling {
     }
     static constexpr int patch_form()     // 100 TW + PB, or 0
     {
-        if constexpr (KH == 3 && KW == 3 && S == 1 && CI % 32 == 0 && CO % 32 == 0 && CI * T <= 32768 && (long long)OHW * NIMG >= 512LL * 128 * QBM / CO) {
-            if constexpr (QBM == 32) {
-                const int f[] = {14, 1614, 2814};
-                const double c[] = {patch_cost<14, 0>(), patch_cost<14, 16>(), patch_cost<14, 28>()};
-                return least(f, c);
-            } else {
-                const int f[] = {8, 7, 6, 2807, 1607, 1209};
-                const double c[] = {patch_cost<8, 0>(), patch_cost<7, 0>(), patch_cost<6, 0>(), patch_cost<7, 28>(), patch_cost<7, 16>(), patch_cost<9, 12>()};
-                const int best = least(f, c);
-                if constexpr (QBM == 128)
-                    if (best == 0 && patch<14, 0>::FITS) return 14;
-                return best;
-            }
+        if constexpr (KH == 3 && KW == 3 && S == 1 && CI % 32 == 0 && CO % QBM == 0 && CI * T <= 32768 && (long long)OHW * NIMG >= 512LL * 128 * QBM / CO) {
+            const int f[] = {8, 7, 6, 2807, 1607, 1209};
+            const double c[] = {patch_cost<8, 0>(), patch_cost<7, 0>(), patch_cost<6, 0>(), patch_cost<7, 28>(), patch_cost<7, 16>(), patch_cost<9, 12>()};
+            const int best = least(f, c);
+            if constexpr (QBM == 128)
+                if (best == 0 && patch<14, 0>::FITS) return 14;
+            return best;
         }
         return 0;
     }

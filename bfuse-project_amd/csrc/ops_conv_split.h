@@ -19,15 +19,15 @@
 //     images take 945 us, 256 columns on eight waves 1019.  Where consecutive pixels make the patch too large (wide images have whole rows above and below), the tile is a
 //     rectangle of one image; ConvTiling has the choice.
 //
-// Batch 1024, us, GemmSplit (or what the layer had) and now, both in turn on one card, uniform operands: 256 -> 256 on 14 x 14 1109 -> 901, 128 on 28 x 28 1179 -> 945, 512 on 7 x 7
+// Batch 1024, us, GemmSplit and now, both in turn on one card, uniform operands: 256 -> 256 on 14 x 14 1109 -> 901, 128 on 28 x 28 1179 -> 945, 512 on 7 x 7
 // 1227 -> 977, 448 -> 384 on 8 x 8 953 -> 758, 96 on 35 x 35 1228 -> 990, 64 -> 96 909 -> 701, 64 on 56 x 56 1599 -> 1199, 64 -> 128 without padding 2306 ->
-// 1993, 128 -> 256 on 28 x 28 likewise 1833 -> 1681, 32 -> 64 on 147 x 147 6210 -> 4397, 32 on 149 x 149 (rectangles on the fp32 instructions) 3479 -> 2975: 1.24x
-// in the geometric mean.  256 -> 256 is 263 of the 335 TFLOP/s that six bf16 MFMAs for a product leave on random operands.  Of its 900 us the filters' parts
+// 1993, 128 -> 256 on 28 x 28 likewise 1833 -> 1681, 32 -> 64 on 147 x 147 6210 -> 4397: 1.24x in the
+// geometric mean.  256 -> 256 is 263 of the 335 TFLOP/s that six bf16 MFMAs for a product leave on random operands.  Of its 900 us the filters' parts
 // cost 64, the patch 47 and wraps 20; the MFMAs and their LDS reads alone take 758 (650 on constant operands: the clock, 1.9 GHz, is what power allows).
 //
 // Sums: a partial sum of two or three taps (of 32 channels each) is added to the result's; 2-norm errors against 64 bits, GemmSplit's and these, on
-// images after a ReLU: 256 -> 256 1.70e-7 and 1.53e-7, 512 1.92e-7 and 1.78e-7, 128 1.56e-7 and 1.21e-7, 64 on 56 x 56 1.13e-7 and 1.11e-7, 32 on 149 x 149 1.38e-7
-// and 1.02e-7; smaller at all eleven layers.  What three parts do not hold is done again as there.
+// images after a ReLU: 256 -> 256 1.70e-7 and 1.53e-7, 512 1.92e-7 and 1.78e-7, 128 1.56e-7 and 1.21e-7, 64 on 56 x 56 1.13e-7 and 1.11e-7;
+// smaller at all ten layers.  What three parts do not hold is done again as there.
 #pragma once
 #include <hip/hip_runtime.h>
 

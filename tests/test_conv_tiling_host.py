@@ -122,3 +122,11 @@ def test_places_of_a_patch_against_a_look_at_every_tile(tmp_path):
         static_assert(ConvTiling<256, 256, 14, 14, 3, 3, 1, 1, 64>::patch_form() == 0 && ConvTiling<64, 64, 56, 56, 5, 5, 1, 2, 1024>::patch_form() == 0);   // few tiles; 25 taps
     """
     _compiles(text, tmp_path)
+
+
+def test_output_channels_that_no_tall_tile_divides_are_as_without_patches(tmp_path):
+    """32: the fp32 instructions, which round a window's only element once; 160, 224, 352: no five to eleven row tiles with a patch each."""
+    text = ""
+    for ci, co, hw, split in [(32, 32, 149, "false"), (32, 160, 28, "true"), (32, 224, 28, "false"), (32, 352, 28, "false"), (64, 160, 14, "true")]:
+        text += f"static_assert(ConvTiling<{ci}, {co}, {hw}, {hw}, 3, 3, 1, 0, 1024>::patch_form() == 0 && ConvTiling<{ci}, {co}, {hw}, {hw}, 3, 3, 1, 0, 1024>::is_split() == {split});\n"
+    _compiles(text, tmp_path)
