@@ -322,7 +322,7 @@ struct NarrowOf<ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, KS, NIMG, kSplitF
 constexpr int kPatchForm = 33;
 template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int BM, int PB, int TW, int NIMG>
 struct ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, TW, NIMG, kPatchForm> : ConvF32Tile<CI, CO, H, W, KH, KW, S, P, BM, 128, 1, NIMG> {
-    using Form = SwapOperands<ConvSplit<CI, CO, H, W, KH, KW, S, P, NIMG, 2, BM / 32, (PB > 9 ? 2 : 1), 16 * PB, TW>>;
+    using Form = SwapOperands<ConvSplit<CI, CO, H, W, KH, KW, S, P, NIMG, 2, BM / 32, 1, 16 * PB, TW>>;
     using Parts = typename Form::Parts;
     static constexpr int PARTS_OPERAND = Form::PARTS_OPERAND;
     static constexpr long long TILES = Form::TILES;
@@ -492,10 +492,11 @@ struct ConvTiling {
     }
     // 3 x 3 filters at stride 1 on whole groups of 32 channels take the images apart once for all taps (ConvSplit, which has the figures: 0.71-0.92 of
     // split's time on eleven layers, 0.75-0.89 on ten others from 14 x 14 to 14 x 300), where a tile of the most output channels up to 128 that divide theirs fits twice
-    // into a CU's LDS with at most 15 % of it outside the images: of 128, 112 or 96 consecutive pixels, 28 x 4, 16 x 7 and 12 x 12, the one that
+    // into a CU's LDS with at most 15 % of it (tiles of 128 channels: 17) outside the images: of 128, 112 or 96 consecutive pixels, 28 x 4, 16 x 7 and 12 x 12, the one that
     // computes least besides.  Measured: 14 x 14 on 112 900 us, on 96 926; 7 x 7 on 96 972, on 112 (one tile a CU) 1062; 8 x 8 on 128 755, on 64 793; 35 x 35 on 12 x 12
-    // 702, on 12 x 8 760, on 36 x 4 806; 56 x 56 on 28 x 4 1242, on 16 x 8 1372; 147 x 147 on 16 x 7 4338, on 12 x 12 4424.  Where
-    // none of these does (26 x 26), eight waves on 224 consecutive pixels, one tile a CU (1718 against split's 1887; 28 x 4 of 16 % outside 1766).
+    // 702, on 12 x 8 760, on 36 x 4 806; 56 x 56 on 28 x 4 1242, on 16 x 8 1372; 147 x 147 on 16 x 7 4338, on 12 x 12 4424; 26 x 26
+    // on 28 x 4 (16 % outside) 1728, split 1785.  (There 224 consecutive pixels on eight waves, one tile a CU, take 1618, but beside their 150 KB of LDS a
+    // thread-fused partner has 13 KB, and a block-fused one runs only on CUs without such a tile.)
     // Tiles have at least 64 of the output channels: a row tile takes its patch apart for itself, and 32 -> 32 on 149 x 149 was on the fp32
     // instructions before, where a window with one element that is not zero is at most 1 u off and here up to 2.4 (2975 instead of 3479 us).
     static constexpr int QBM = CO % 128 == 0 ? 128 : CO % 96 == 0 ? 96 : 64;
@@ -507,7 +508,7 @@ struct ConvTiling {
         using F = patch<PB, TW>;
         if constexpr (F::FITS && (PB != 9 || CI <= 128)) {   // (nine blocks of columns take all registers there are)
             const double pixels = 16.0 * PB * (double)F::TILES / (CO / QBM) / ((double)OHW * NIMG);
-            if (2 * (int)sizeof(typename F::Smem) <= 163840 && pixels <= 1.15) return pixels * (1 + 1.0 / (PB > 9 ? PB / 2 : PB));
+            if (2 * (int)sizeof(typename F::Smem) <= 163840 && pixels <= (QBM == 128 ? 1.17 : 1.15)) return pixels * (1 + 1.0 / PB);
         }
         return 1e9;
     }
@@ -516,10 +517,7 @@ struct ConvTiling {
         if constexpr (KH == 3 && KW == 3 && S == 1 && CI % 32 == 0 && CO % QBM == 0 && CI * T <= 32768 && (long long)OHW * NIMG >= 512LL * 128 * QBM / CO) {
             const int f[] = {8, 7, 6, 2807, 1607, 1209};
             const double c[] = {patch_cost<8, 0>(), patch_cost<7, 0>(), patch_cost<6, 0>(), patch_cost<7, 28>(), patch_cost<7, 16>(), patch_cost<9, 12>()};
-            const int best = least(f, c);
-            if constexpr (QBM == 128)
-                if (best == 0 && patch<14, 0>::FITS) return 14;
-            return best;
+            return least(f, c);
         }
         return 0;
     }

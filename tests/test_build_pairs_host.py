@@ -186,7 +186,11 @@ def test_no_block_fused_pair_of_the_batch_suites_is_left_out_for_registers(i, tm
 @pytest.mark.parametrize("k1,k2", [
     # one wave without barriers beside operators that synchronise
     ("conv7x7s2p3_f32_1024x3x224x224_64", "bgemm_f32_1024x512x64x512"), ("conv7x7s2p3_f32_1024x3x224x224_64", "conv1x1s1p0_f32_1024x2048x8x8_320"),
-    ("conv7x7s2p3_f32_1024x3x224x224_64", "conv3x3s2p0_f32_1024x192x17x17_320"), ("conv7x7s2p3_f32_1024x3x224x224_64", "gemm_f32_1024x768x2304")])
+    ("conv7x7s2p3_f32_1024x3x224x224_64", "conv3x3s2p0_f32_1024x192x17x17_320"), ("conv7x7s2p3_f32_1024x3x224x224_64", "gemm_f32_1024x768x2304"),
+    # half a CU's LDS beside it
+    ("conv3x3s1p0_f32_1024x128x28x28_256", "bgemm_f32_1024x208x64x208"), ("conv3x3s1p0_f32_1024x128x28x28_256", "bgemm_f32_1024x208x208x64"),
+    ("conv3x3s1p0_f32_1024x128x28x28_256", "bgemm_f32_1024x208x80x208"), ("conv3x3s1p0_f32_1024x128x28x28_256", "bgemm_f32_1024x208x208x80"),
+    ("conv3x3s1p0_f32_1024x128x28x28_256", "conv3x3s2p0_f32_1024x3x299x299_32")])
 def test_operators_that_one_workgroup_can_hold(k1, k2):
     reg = {k.name: k for k in bf.list_kernels()}
     assert build_pairs.hfuse_possible(reg[k1], reg[k2], build_pairs.op_lds(k1), build_pairs.op_lds(k2))
