@@ -21,13 +21,17 @@
 //
 // Batch 1024, us, GemmSplit and now, both in turn on one card, uniform operands: 256 -> 256 on 14 x 14 1109 -> 901, 128 on 28 x 28 1179 -> 945, 512 on 7 x 7
 // 1227 -> 977, 448 -> 384 on 8 x 8 953 -> 758, 96 on 35 x 35 1228 -> 990, 64 -> 96 909 -> 701, 64 on 56 x 56 1599 -> 1199, 64 -> 128 without padding 2306 ->
-// 1993, 128 -> 256 on 28 x 28 likewise 1833 -> 1681, 32 -> 64 on 147 x 147 6210 -> 4397: 1.24x in the
+// 1993, 128 -> 256 on 28 x 28 likewise 1785 -> 1728, 32 -> 64 on 147 x 147 6210 -> 4500: 1.24x in the
 // geometric mean.  256 -> 256 is 263 of the 335 TFLOP/s that six bf16 MFMAs for a product leave on random operands.  Of its 900 us the filters' parts
 // cost 64, the patch 47 and wraps 20; the MFMAs and their LDS reads alone take 758 (650 on constant operands: the clock, 1.9 GHz, is what power allows).
 //
-// Sums: a partial sum of two or three taps (of 32 channels each) is added to the result's; 2-norm errors against 64 bits, GemmSplit's and these, on
-// images after a ReLU: 256 -> 256 1.70e-7 and 1.53e-7, 512 1.92e-7 and 1.78e-7, 128 1.56e-7 and 1.21e-7, 64 on 56 x 56 1.13e-7 and 1.11e-7;
-// smaller at all ten layers.  What three parts do not hold is done again as there.
+// Sums: a partial sum of one, two or three taps (of 32 channels each) is added to the result's: the longer it is the more error it has, the shorter
+// the more of them are added, which large results feel most.  Errors against 64 bits on images after a ReLU, three sets of operands, GemmSplit's and
+// these, 2-norm and largest over the results' rms: 256 -> 256 1.73e-7 -> 1.56e-7 and 1.49e-6 -> 1.60e-6, 512 1.89 -> 1.76 and 1.92 -> 2.00, 448 -> 384 1.85 -> 1.70 and 1.77 ->
+// 1.85, 128 1.61 -> 1.24 and 1.47 -> 1.37, 96 1.55 -> 1.16 and 1.44 -> 1.25, 64 -> 96 1.09 -> 1.08 and 1.13 -> 1.17, 64 on 56 x 56 1.09 -> 1.08 and 1.16 -> 1.20, 64 -> 128 1.10 ->
+// 1.09 and 1.16 -> 1.26, 128 -> 256 1.59 -> 1.24 and 1.46 -> 1.41, 32 -> 64 0.98 -> 0.72 and 1.34 -> 1.05.  So the 2-norm is smaller at all ten layers, the largest
+// up to 1.08 times at six of them.  Other lengths: 32 channels by two taps 0.98 and 1.38 (2.5 % faster), 64 by one 0.92 and 1.33, 128 by three 1.41 and 1.36,
+// 256 by two 1.51 and 1.90.  What three parts do not hold is done again as there.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -80,7 +84,7 @@ struct ConvSplit {
     static constexpr int apart_at(int j) { return 2 * NUJ <= T ? (j + 1) * T / NUJ - 1 : (j + 1) * T / (NUJ + 1); }
     static constexpr int unit_of(bool load, int t) { for (int j = 0; j < NUJ; ++j) if ((load ? load_at(j) : apart_at(j)) == t) return j; return -1; }
     static constexpr int PLANE = UNITS * 16, BUF = 3 * PLANE, NBUF = NG > 1 ? 2 : 1;
-    static constexpr int SUMMED = NG * T <= 36 ? 2 : 3;                              // taps of a partial sum: of both the one that leaves less error
+    static constexpr int SUMMED = NG == 1 ? 1 : NG * T <= 36 ? 2 : 3;                // taps of a partial sum (see Sums)
     static constexpr bool FITS = Form::FITS && CI % 32 == 0 && T > 1 && NBUF * BUF <= 163840 - 256 && (NG > 1 ? NUJ < T : NUJ <= 12) && (long long)BM * CI * T * 6 < (1LL << 31);
     static constexpr long long TILES = (long long)NT * Form::MT;
     static constexpr Dims3 GRID{(int)TILES, 1, 1}, BLOCK = Form::BLOCK;

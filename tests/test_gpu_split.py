@@ -327,6 +327,18 @@ def test_convolution_from_a_patch_is_closer_to_64_bits_than_one_fp32_sum(tag, ch
     assert err <= 2.0 ** -24 * ((steps / 4 + 9) ** 0.5 + 0.5)
 
 
+@pytest.mark.parametrize("tag", ["b", "d"])
+def test_a_convolution_from_a_patch_of_32_channels_adds_up_every_tap(tag):
+    """Nine partial sums, added up: 9 / 2 roundings of the whole in all; each of them rounded six times while it grows, 6 / 2 of a ninth
+    (2-norms squared): 9 * 3 / 9 more.  A rounding is off by u / sqrt(3), evenly spread over half a unit of the last place.  (Sums of two taps
+    are off by 1.6 - 1.7 u.)"""
+    name = f"selftest_conv_split_{tag}"
+    x, w = _operands(name)
+    want = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(w).double(), padding=dict(CONV_PATCHES)[tag]).numpy()
+    err = np.linalg.norm(_run(name, x, w) - want) / np.linalg.norm(want)
+    assert err <= 2.0 ** -24 * ((4.5 + 3) / 3) ** 0.5
+
+
 def test_filters_are_taken_apart_for_every_launch_and_side():
     """The parts are the launch's own filters': new ones, two sides at once on two streams, replays of a graph, a plan at run time."""
     name = "selftest_conv_split_a"
