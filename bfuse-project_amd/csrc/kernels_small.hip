@@ -288,6 +288,7 @@ CONV_PATCH_TEST(d, 32, 32, 20, 33, 1, 2, 2, 1, 2, 224, 16)
 CONV_PATCH_TEST(e, 128, 128, 10, 10, 0, 4, 2, 4, 2, 224, 0)      // 256 pixels of four images
 CONV_PATCH_TEST(f, 64, 64, 9, 9, 2, 3, 2, 2, 1, 112, 16)         // padding of two
 CONV_PATCH_TEST(g, 96, 128, 5, 5, 1, 9, 2, 4, 1, 128, 0)         // a tile of six images
+CONV_PATCH_TEST(h, 160, 64, 7, 7, 1, 5, 2, 2, 1, 96, 0)          // five groups of channels: partial sums of three taps
 BFUSE_BFUSE_KERNEL(selftest_conv_split_a, ConvP_a, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
 BFUSE_HFUSE_KERNEL(selftest_conv_split_b, ConvP_b, bias_relu_4096, BiasReluS)
 BFUSE_HFUSE_KERNEL(selftest_conv_split_d, ConvP_d, conv3x3_f32_32x12x12_32, ConvS2)
@@ -298,13 +299,18 @@ BFUSE_BFUSE_KERNEL(selftest_conv_split_b, Slim<ConvP_b>, gemm_bf16_256x448x1792_
 BFUSE_BFUSE_KERNEL(selftest_conv_split_d, Slim<ConvP_d>, gemm_bf16_256x448x1792_p2, GemmB9, _c4, bfuse::kChunked, 4, 1)
 BFUSE_BFUSE_KERNEL(selftest_conv_split_a, ConvP_a, selftest_gemm_split_r_p, Narrow<GemmSpP_r>, _c4, bfuse::kChunked, 4, 1)   // operands of both sides are taken apart
 
-// The split-K product on the bf16 matrix cores: a trailing 16-column group and GELU in one round, two waves in two rounds, one stage.
+// The split-K product on the bf16 matrix cores: a trailing 16-column group and GELU in one round, two waves in two rounds, one stage; 32
+// and 48 columns past the last group.
 using GemmSpk_a = GemmF32Dma<64, 288, 256, 32, 144, 4, kEpiGeluTanh>;
 using GemmSpk_b = GemmF32Dma<96, 256, 192, 32, 128, 2, kEpiNone, 2>;
 using GemmSpk_c = GemmF32Dma<32, 384, 128, 32, 192, 4, kEpiNone, 2>;
+using GemmSpk_d = GemmSplitK<64, 288, 192, 32, 96, 2, kEpiNone, 1>;
+using GemmSpk_e = GemmSplitK<64, 336, 256, 32, 112, 4, kEpiNone, 2>;
 BFUSE_KERNEL(selftest_gemm_splitk_a, GemmSpk_a, ({{64, 256, 1, 1}, 4}), ({{256, 288, 1, 1}, 4}), ({{64, 288, 1, 1}, 4}))
 BFUSE_KERNEL(selftest_gemm_splitk_b, GemmSpk_b, ({{96, 192, 1, 1}, 4}), ({{192, 256, 1, 1}, 4}), ({{96, 256, 1, 1}, 4}))
 BFUSE_KERNEL(selftest_gemm_splitk_c, GemmSpk_c, ({{32, 128, 1, 1}, 4}), ({{128, 384, 1, 1}, 4}), ({{32, 384, 1, 1}, 4}))
+BFUSE_KERNEL(selftest_gemm_splitk_d, GemmSpk_d, ({{64, 192, 1, 1}, 4}), ({{192, 288, 1, 1}, 4}), ({{64, 288, 1, 1}, 4}))
+BFUSE_KERNEL(selftest_gemm_splitk_e, GemmSpk_e, ({{64, 256, 1, 1}, 4}), ({{256, 336, 1, 1}, 4}), ({{64, 336, 1, 1}, 4}))
 BFUSE_BFUSE_KERNEL(selftest_gemm_splitk_a, GemmSpk_a, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
 BFUSE_HFUSE_KERNEL(selftest_gemm_splitk_b, GemmSpk_b, bias_relu_4096, BiasReluS)
 BFUSE_HFUSE_KERNEL(selftest_gemm_splitk_b, GemmSpk_b, conv3x3_f32_32x12x12_32, ConvS2)

@@ -84,6 +84,7 @@ struct ConvSplit {
     static constexpr int apart_at(int j) { return 2 * NUJ <= T ? (j + 1) * T / NUJ - 1 : (j + 1) * T / (NUJ + 1); }
     static constexpr int unit_of(bool load, int t) { for (int j = 0; j < NUJ; ++j) if ((load ? load_at(j) : apart_at(j)) == t) return j; return -1; }
     static constexpr int PLANE = UNITS * 16, BUF = 3 * PLANE, NBUF = NG > 1 ? 2 : 1;
+    static_assert(TN > 1, "a partial sum is added to the result beside the next block of columns");
     static constexpr int SUMMED = NG == 1 ? 1 : NG * T <= 36 ? 2 : 3;                // taps of a partial sum (see Sums)
     static constexpr bool FITS = Form::FITS && CI % 32 == 0 && T > 1 && NBUF * BUF <= 163840 - 256 && (NG > 1 ? NUJ < T : NUJ <= 12) && (long long)BM * CI * T * 6 < (1LL << 31);
     static constexpr long long TILES = (long long)NT * Form::MT;

@@ -151,7 +151,7 @@ struct GemmSplit {
     static constexpr int NUB = EVEN ? 1 : NUJ;
     static_assert(BN % (16 * WN) == 0 && K % 8 == 0 && NS % KG == 0 && M >= BM && (LAYOUT == kPix || (W >= BN && H == 1 && S == 1)), "tile");
     // 31-bit offsets; padding is read through one that lies past the buffer
-    static constexpr bool FITS = (long long)BM * K * 4 < (1LL << 31) && (long long)(NIMAGES < NIMG ? NIMAGES : NIMG) * CI * HW * 4 < (1LL << (T == 1 ? 31 : 29));
+    static constexpr bool FITS = (long long)BM * (PREP ? NS * 32 * 6 : K * 4) < (1LL << 31) && (long long)(NIMAGES < NIMG ? NIMAGES : NIMG) * CI * HW * 4 < (1LL << (T == 1 ? 31 : 29));
     static constexpr bool TURNED = LAYOUT == kRows && NS > 2;
     static constexpr int PLANE = 4 * BN * 16, BUF = 3 * PLANE, NBUF = NIT < 3 ? NIT : 3;
     static constexpr int SUMMED = NIT > 8 && NIT <= 20 ? 2 : 4;                     // stages of a partial sum (error and time: above)

@@ -32,7 +32,8 @@ def _gelu(x):
 
 
 @pytest.mark.parametrize("tag,partner,kind,suffix", [
-    ("a", "layernorm_8x256", "bfuse", "_c4"), ("b", "bias_relu_4096", "hfuse", ""), ("b", "conv3x3_f32_32x12x12_32", "hfuse", ""), ("c", "bias_relu_4096", None, "")])
+    ("a", "layernorm_8x256", "bfuse", "_c4"), ("b", "bias_relu_4096", "hfuse", ""), ("b", "conv3x3_f32_32x12x12_32", "hfuse", ""), ("c", "bias_relu_4096", None, ""),
+    ("d", "bias_relu_4096", None, ""), ("e", "bias_relu_4096", None, "")])
 def test_split_k_product_against_numpy_and_fused(tag, partner, kind, suffix):
     _check(f"selftest_gemm_splitk_{tag}", lambda a, b: (_gelu if tag == "a" else np.asarray)(_product(a, b)).astype(np.float32), partner, kind, suffix)
 
@@ -95,7 +96,7 @@ def test_split_product_is_closer_to_64_bits_than_one_fp32_sum(tag, steps, groups
     assert err <= 2.0 ** -24 * ((steps / groups / 8 + 12) ** 0.5 + 0.5 + (groups > 1))
 
 
-@pytest.mark.parametrize("tag,steps,groups", [("k_b", 6 * 192 // 32, 2), ("k_c", 6 * 128 // 32, 4)])
+@pytest.mark.parametrize("tag,steps,groups", [("k_b", 6 * 192 // 32, 2), ("k_c", 6 * 128 // 32, 4), ("k_d", 6 * 192 // 32, 2), ("k_e", 6 * 256 // 32, 4)])
 def test_split_k_product_is_closer_to_64_bits_than_one_fp32_sum(tag, steps, groups):
     """One sum a wave, rounded six times for 32 k, `groups` of which are added."""
     name = f"selftest_gemm_split{tag}"
@@ -105,7 +106,7 @@ def test_split_k_product_is_closer_to_64_bits_than_one_fp32_sum(tag, steps, grou
     assert err <= 2.0 ** -24 * ((steps / 2 / groups) ** 0.5 + 0.5 + (groups > 1))
 
 
-@pytest.mark.parametrize("tag", ["_a", "_b", "_e", "k_b", "k_c"])
+@pytest.mark.parametrize("tag", ["_a", "_b", "_e", "k_b", "k_c", "k_d", "k_e"])
 @pytest.mark.parametrize("scale", [2.0 ** -100, 2.0 ** -118, 2.0 ** 100])
 def test_scaled_operands_keep_their_bits(tag, scale):
     """A power of two on an operand is one on the result, however small the operand's own low bits become (whole operand, one
@@ -129,7 +130,7 @@ def test_scaled_operands_keep_their_bits(tag, scale):
         assert np.linalg.norm(y[r] - want[r]) <= u * np.linalg.norm(want[r]), r
 
 
-@pytest.mark.parametrize("tag", ["_a", "_b", "_e", "k_b", "k_c"])
+@pytest.mark.parametrize("tag", ["_a", "_b", "_e", "k_b", "k_c", "k_d", "k_e"])
 @pytest.mark.parametrize("scale", [2.0 ** -112, 2.0 ** -125, 2.0 ** -136, 2.0 ** -145])
 def test_values_with_bits_below_the_parts_keep_them(tag, scale):
     """Operands, or some rows of them, of which one bf16 part or all three are zero or hold less than the value (results are
@@ -172,7 +173,7 @@ def _one_hot(name, x, w, side, values):
     return x, w, _product(x, w)
 
 
-@pytest.mark.parametrize("tag", ["_a", "_b", "_e", "k_b", "k_c"])
+@pytest.mark.parametrize("tag", ["_a", "_b", "_e", "k_b", "k_c", "k_d", "k_e"])
 @pytest.mark.parametrize("scale", [1.0, 2.0 ** -112, 2.0 ** -120, 2.0 ** -126])
 @pytest.mark.parametrize("side", [0, 1])
 def test_a_product_with_a_permutation_is_exact(tag, scale, side):
@@ -184,7 +185,7 @@ def test_a_product_with_a_permutation_is_exact(tag, scale, side):
     assert np.array_equal(_run(name, x, w).reshape(want.shape), want.astype(np.float32))
 
 
-@pytest.mark.parametrize("tag", ["_a", "_b", "_e", "k_b", "k_c"])
+@pytest.mark.parametrize("tag", ["_a", "_b", "_e", "k_b", "k_c", "k_d", "k_e"])
 @pytest.mark.parametrize("side", [0, 1])
 def test_sums_of_one_product(tag, side):
     """One product of two values of 24 bits.  With u = 2^-24, of the product: its sum is rounded (u), after what the smaller partial
@@ -254,7 +255,7 @@ def test_overlapping_tiles_leave_their_neighbours_results_to_them(tag, side, at,
     assert not np.array_equal(out[0], out[1])
 
 
-@pytest.mark.parametrize("tag", ["_a", "_b", "_e", "k_b", "k_c"])
+@pytest.mark.parametrize("tag", ["_a", "_b", "_e", "k_b", "k_c", "k_d", "k_e"])
 def test_infinities_nan_and_the_largest_values(tag):
     """What does not fit three bf16 gives what fp32 arithmetic gives: infinite where it is, NaN where it is, finite elsewhere."""
     name = f"selftest_gemm_split{tag}"
@@ -277,7 +278,7 @@ def test_infinities_nan_and_the_largest_values(tag):
     assert ok.any() and np.all(np.abs(y[ok] - want[ok]) <= 1e-5 * np.maximum(np.abs(want[ok]), np.sqrt(np.float32(x2.shape[1]))))
 
 
-CONV_PATCHES = [("a", 1), ("b", 1), ("c", 0), ("d", 1), ("e", 0), ("f", 2), ("g", 1)]
+CONV_PATCHES = [("a", 1), ("b", 1), ("c", 0), ("d", 1), ("e", 0), ("f", 2), ("g", 1), ("h", 1)]
 
 
 @pytest.mark.parametrize("tag,p", CONV_PATCHES)
@@ -293,7 +294,10 @@ def test_convolution_from_a_patch_against_the_oracle_and_fused(tag, p):
 def test_values_that_parts_do_not_hold_in_a_patch_or_its_filters(tag, p, where, scale):
     """Infinite, NaN and lowest values are in the results that have them in their window (padding and places beside an image
     are not multiplied), and values below bf16's bits keep theirs: what fp32 arithmetic gives."""
-    name = f"selftest_conv_split_{tag}"
+    _values_that_parts_do_not_hold(f"selftest_conv_split_{tag}", 1, p, where, scale)
+
+
+def _values_that_parts_do_not_hold(name, s, p, where, scale):
     x, w = _operands(name)
     w = np.abs(w) + np.float32(0.5)
     if where == "image":
@@ -305,19 +309,20 @@ def test_values_that_parts_do_not_hold_in_a_patch_or_its_filters(tag, p, where, 
         w[2] *= np.float32(scale)
     (w if where == "image" else x)[...] *= np.float32(2.0 ** 60)
     with np.errstate(all="ignore"):
-        want = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(w).double(), padding=p).numpy()
+        want = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(w).double(), stride=s, padding=p).numpy()
         f = want.astype(np.float32)
     y = _run(name, x, w)
     assert np.array_equal(np.isnan(y), np.isnan(f)) and np.array_equal(np.isposinf(y), np.isposinf(f)) and np.array_equal(np.isneginf(y), np.isneginf(f))
-    u = 2.0 ** -24 * (9 * x.shape[1]) ** 0.5 * 2     # twice the bound of one sum rounded after every product
+    u = 2.0 ** -24 * np.prod(w.shape[1:]) ** 0.5 * 2     # twice the bound of one sum rounded after every product
     for part in [(n, slice(None)) for n in range(x.shape[0])] + [(slice(None), m) for m in range(w.shape[0])]:
         ok = np.isfinite(f[part]) & (np.abs(want[part]) < 2.0 ** 120)      # (the lowest value's products drown the others)
         assert np.linalg.norm(y[part][ok] - want[part][ok]) <= u * np.linalg.norm(want[part][ok])
 
 
-@pytest.mark.parametrize("tag,channels", [("a", 64), ("c", 96), ("e", 128), ("g", 96)])
+@pytest.mark.parametrize("tag,channels", [("a", 64), ("c", 96), ("e", 128), ("g", 96), ("h", 160)])
 def test_convolution_from_a_patch_is_closer_to_64_bits_than_one_fp32_sum(tag, channels):
-    """As the products: partial sums of n taps of 32 channels are each rounded 6 n times while they grow, and added once; n is two or three."""
+    """As the products: partial sums of n taps of 32 channels are each rounded 6 n times while they grow, and added once; n is two,
+    or three where more than 128 channels are."""
     name = f"selftest_conv_split_{tag}"
     x, w = _operands(name)
     p = dict(CONV_PATCHES)[tag]
@@ -373,15 +378,12 @@ def test_filters_are_taken_apart_for_every_launch_and_side():
             assert np.array_equal(op.run_fuse(rt, x, w, *P)[0], y)
 
 
-@pytest.mark.parametrize("tag", ["a", "b", "h", "i", "j", "l", "r", "s"])
-@pytest.mark.parametrize("side", [0, 1])
-@pytest.mark.parametrize("value", [1.0, 2.0 ** -120 * 1.2345678, np.inf])
+@pytest.mark.parametrize("tag,side,value", [(tag, side, value) for tag in ("a", "b", "h", "i", "j", "l", "r", "s") for side in (0, 1)
+                                            for value in (1.0, 2.0 ** -120 * 1.2345678, np.inf) if tag != "l" or value == 1.0])
 def test_an_operand_taken_apart_before_gives_the_same_bits(tag, side, value):
     """The same products of the same parts, whatever values lie in either operand (l: tiles of 112 columns for 64; those with
-    a value that its parts do not hold are done again, so that one compares its ordinary operands alone)."""
+    a value that its parts do not hold are done again, so that one compares its ordinary operands alone; the others are the next test's)."""
     x, w = _operands(f"selftest_gemm_split_{tag}")
-    if tag == "l" and value != 1.0:
-        return
     (x, w)[side].reshape(-1)[[7, 1001]] = value
     with bf.Operation(f"selftest_gemm_split_{tag}", f"selftest_gemm_split_{tag}_p") as op:
         for i in (0, 1):
@@ -394,6 +396,12 @@ def test_an_operand_taken_apart_before_gives_the_same_bits(tag, side, value):
         with bf.Operation("selftest_gemm_split_r_p", "layernorm_8x256") as op:
             P = [fill_normal(21 + i, int(np.prod(op.k[1].shapes[i])), 0, 1) for i in (0, 1)]
             assert np.array_equal(op.run_fuse(op.fused("bfuse", "_c4"), x, w, *P)[0].view(np.uint32), a.view(np.uint32))
+
+
+@pytest.mark.parametrize("where", ["image", "filter"])
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** -118, 2.0 ** -140])
+def test_values_that_parts_do_not_hold_in_filters_of_30_taps_taken_apart_before(where, scale):
+    _values_that_parts_do_not_hold("selftest_gemm_split_l_p", 3, 2, where, scale)
 
 
 def test_a_fused_kernel_of_two_operators_whose_operands_are_taken_apart():
