@@ -32,6 +32,7 @@ import yaml
 METHODS = ["kernel1", "kernel2", "parallel", "hfuse", "bfuse"]   # profile_test_suite.py:25
 WARMUP_TRIALS = 3                                                  # profile_test_suite.py:10-11
 TIMED_TRIALS = 30
+TAKE_APART = "bfuse::take_apart<"                                  # csrc/fuse.h
 
 
 # ---- suite description ------------------------------------------------------------------
@@ -143,13 +144,14 @@ def write_trace(path: str, rows: Sequence[dict]) -> None:
 def read_trace(path: str) -> List[dict]:
     """Rows {Name, Start, Duration} (ns) in start order, from this module's own trace files,
     from rocprofv3's `*_kernel_trace.csv` (Kernel_Name, Start_Timestamp, End_Timestamp), or from the
-    reference's nsys export (`Start (ns)`, `Duration (ns)`, `Name`)."""
+    reference's nsys export (`Start (ns)`, `Duration (ns)`, `Name`).  Where rocprofv3 saw an operand taken apart before a
+    launch (csrc/fuse.h, Prepares), that kernel is part of the launch: of the next row of its stream, as in the library's own times."""
     out = []
     with open(path, newline="") as f:
         for r in csv.DictReader(f):
             if "Kernel_Name" in r:
                 s, e = float(r["Start_Timestamp"]), float(r["End_Timestamp"])
-                out.append({"Name": r["Kernel_Name"], "Start": s, "Duration": e - s})
+                out.append({"Name": r["Kernel_Name"], "Start": s, "Duration": e - s, "Stream": (r.get("Queue_Id"), r.get("Stream_Id"))})
             elif "Start (ns)" in r:
                 if not r.get("Duration (ns)"):
                     continue
@@ -157,7 +159,19 @@ def read_trace(path: str) -> List[dict]:
             else:
                 out.append({"Name": r["Name"], "Start": float(r["Start"]), "Duration": float(r["Duration"])})
     out.sort(key=lambda r: r["Start"])
-    return out
+    launches, apart = [], {}
+    for r in out:
+        stream = r.pop("Stream", None)
+        if stream is not None and TAKE_APART in r["Name"]:
+            apart.setdefault(stream, r["Start"])
+            continue
+        if stream in apart:
+            start = apart.pop(stream)
+            r["Duration"] += r["Start"] - start
+            r["Start"] = start
+        launches.append(r)
+    launches.sort(key=lambda r: r["Start"])
+    return launches
 
 
 def _stats(v: Sequence[float]) -> Tuple[float, float, float, float]:

@@ -86,6 +86,14 @@ def test_trace_formats(tmp_path):
     roc.write_text('"Kind","Agent_Id","Queue_Id","Kernel_Name","Start_Timestamp","End_Timestamp"\n'
                    '"KERNEL_DISPATCH",1,1,"k",1000,1800\n"KERNEL_DISPATCH",1,1,"k",3000,3900\n')
     assert [(r["Name"], r["Duration"]) for r in suite.read_trace(str(roc))] == [("k", 800.0), ("k", 900.0)]
+    # an operand taken apart is the beginning of the launch behind it on its stream, two of them that of a fused one
+    apart = '"void bfuse::take_apart<bfuse::SplitParts<64, 576, 9, true> >(void const*, void*)"'
+    roc.write_text('"Kind","Agent_Id","Queue_Id","Stream_Id","Kernel_Name","Start_Timestamp","End_Timestamp"\n' + "".join(
+        f'"KERNEL_DISPATCH",1,{q},{q},{n},{s},{e}\n' for q, n, s, e in [
+            (1, apart, 1000, 1100), (2, '"b"', 1050, 1500), (1, '"a"', 1200, 2000), (1, '"a"', 3000, 3900),
+            (3, apart, 4000, 4100), (3, apart, 4100, 4300), (3, '"a_b_fused_bfuse"', 4400, 6000)]))
+    assert [(r["Name"], r["Start"], r["Duration"]) for r in suite.read_trace(str(roc))] == [
+        ("a", 1000.0, 1000.0), ("b", 1050.0, 450.0), ("a", 3000.0, 900.0), ("a_b_fused_bfuse", 4000.0, 2000.0)]
     # the reference's nsys export: memcpy rows have a duration too, kernels are picked by name later
     nsys = tmp_path / "nsys.csv"
     nsys.write_text("Start (ns),Duration (ns),CorrId,GrdX,Name\n288325122,257825,241,,[CUDA memcpy Host-to-Device]\n"
