@@ -31,8 +31,8 @@ control-flow graph of every kernel that has such loads,
   * one in flight behind a wait that says `loads into LDS have landed` is an error: such a wait counts
     the loads behind them, which the compiler may have dropped or moved.
 
-(`global_load_lds_*`, issued from asm, are not followed: their kernels wait and meet by step numbers,
-which a graph does not show.)
+(Those issued from asm are not followed: their kernels wait and meet by step numbers, which a graph does
+not show.  They count as any other vector memory operation.)
 
 Usage: check_asm_reads.py file.s [...]; exit status 1 and one line per finding if anything is wrong.
 """
@@ -65,7 +65,7 @@ def check_lds_loads(path):
     """Findings on loads into LDS, and how many such loads there are.  The state at an instruction is how many vector
     memory operations were issued behind the youngest load into LDS that may be in flight (None: there is none), the
     least of all ways to get there; they retire in order, so `vmcnt(n)` ends it where n or more were."""
-    kernels, func = {}, None
+    kernels, func, in_asm, by_hand = {}, None, False, set()
     for ln, raw in enumerate(open(path, errors="replace"), 1):
         m = LABEL.match(raw)
         if m:
@@ -74,14 +74,18 @@ def check_lds_loads(path):
             elif func is not None:
                 func.append((ln, "label", m.group(1)))
             continue
+        if ";#ASM" in raw:
+            in_asm = ";#ASMSTART" in raw
         s = raw.split(";", 1)[0].strip()
         if func is None or not s or s.startswith((".", "//")):
             continue
         mn, _, ops = s.partition(" ") if " " in s else s.partition("\t")
+        if in_asm:
+            by_hand.add(ln)
         func.append((ln, mn, ops.strip() + (LANDED if LANDED in raw else "")))
     findings, n_loads = [], 0
     for name, code in kernels.items():
-        is_load = [mn.startswith("buffer_load") and re.search(r"\blds\b", ops) is not None for _, mn, ops in code]
+        is_load = [mn.startswith("buffer_load") and re.search(r"\blds\b", ops) is not None and ln not in by_hand for ln, mn, ops in code]
         if not any(is_load):
             continue
         n_loads += sum(is_load)

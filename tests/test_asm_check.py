@@ -2,6 +2,9 @@
 assembly text: it must accept the intended pattern and flag each way the pattern can break."""
 import importlib.util
 import os
+import subprocess
+
+import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 _spec = importlib.util.spec_from_file_location("check_asm_reads", os.path.join(ROOT, "bfuse-project_amd", "csrc", "check_asm_reads.py"))
@@ -126,11 +129,35 @@ def test_loads_into_lds_are_followed_round_loops_and_over_branches(tmp_path):
     assert findings == []
 
 
+def test_loads_into_lds_from_asm_are_their_kernels_own_affair_and_count_as_others(tmp_path):
+    by_hand = "\t;;#ASMSTART\n\ts_mov_b32 m0, s5\n\ts_nop 0\n\tbuffer_load_dword v5, s[0:3], s4 offen lds\n\t;;#ASMEND\n"
+    assert _lds(tmp_path, by_hand + WRITE) == ([], 0)
+    findings, n = _lds(tmp_path, LDS_LOAD + by_hand * 2 + LANDED.format(n=2) + WRITE)
+    assert (findings, n) == ([], 1)
+    findings, _ = _lds(tmp_path, LDS_LOAD + by_hand + LANDED.format(n=2) + WRITE)
+    assert len(findings) == 2
+
+
+@pytest.mark.parametrize("k1,k2,form", [
+    # loads into LDS from asm on one side, and LDS writes on the other, which the graph reaches past waits and lanes that do not go there
+    ("bgemm_f32_1024x208x64x208", "conv1x1s2p0_f32_1024x128x28x28_256", "hfuse"), ("conv7x7s2p3_f32_1024x3x224x224_64", "conv1x1s2p0_f32_1024x128x28x28_256", "bfuse"),
+    # ... and by the compiler
+    ("gemm_f32_1024x768x2304", "conv1x1s2p0_f32_1024x128x28x28_256", "bfuse")])
+def test_kernels_fused_later_pass(k1, k2, form, tmp_path):
+    from bfuse_project_amd import build_pairs
+    (tmp_path / "pairs_0.hip").write_text(build_pairs.source_text([{"k1": k1, "k2": k2, "form": form, "name": ""}]))
+    r = subprocess.run(["/opt/rocm/bin/hipcc", "--offload-arch=gfx950", "--cuda-device-only", "-S", "-O3", "-std=c++17", "-ffp-contract=off", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                        "-w", "-I", build_pairs.CSRC, str(tmp_path / "pairs_0.hip"), "-o", str(tmp_path / "pairs_0.s")], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    assert chk.check(str(tmp_path / "pairs_0.s"))[0] == []
+    findings, n = chk.check_lds_loads(str(tmp_path / "pairs_0.s"))
+    assert findings == [] and (n > 0) == k1.startswith("gemm")
+
+
 def test_the_built_kernels_pass(tmp_path):
     import glob
     files = glob.glob(os.path.join(ROOT, "bfuse-project_amd", "csrc", "obj", "kernels_*-gfx950.s"))
     if not files:
-        import pytest
         pytest.skip("device assembly not present (library not built in this tree)")
     total = loads = 0
     for f in files:
