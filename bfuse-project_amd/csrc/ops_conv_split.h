@@ -11,7 +11,7 @@
 //     immediates, since a step of a tap is the same number of places everywhere.  1.2 - 1.8 units of eight values for a column where the product takes
 //     nine apart.  A row's wrap inside 16 columns costs a second LDS pass (2 % of the time);
 //   * k counts (32 channels, tap), which is not how filters lie in memory, so they are put in that order by a kernel that runs before
-//     this one (SplitParts: 3 - 8 us) and takes them apart on that occasion: a lane's 48 bytes of a tap and 16 rows are three coalesced loads
+//     this one (SplitParts: 5 - 10 us) and takes them apart on that occasion: a lane's 48 bytes of a tap and 16 rows are three coalesced loads
 //     straight into the registers that are multiplied from, a tap ahead;
 //   * two LDS buffers and one barrier for 32 channels, that is for nine times 12 TN MFMAs of a wave; the units of the next channels are loaded and
 //     taken apart between them, one at a time;
@@ -23,7 +23,9 @@
 // 1227 -> 977, 448 -> 384 on 8 x 8 953 -> 758, 96 on 35 x 35 1228 -> 990, 64 -> 96 909 -> 701, 64 on 56 x 56 1599 -> 1199, 64 -> 128 without padding 2306 ->
 // 1993, 128 -> 256 on 28 x 28 likewise 1785 -> 1728, 32 -> 64 on 147 x 147 6210 -> 4500: 1.24x in the
 // geometric mean.  256 -> 256 is 263 of the 335 TFLOP/s that six bf16 MFMAs for a product leave on random operands.  Of its 900 us the filters' parts
-// cost 64, the patch 47 and wraps 20; the MFMAs and their LDS reads alone take 758 (650 on constant operands: the clock, 1.9 GHz, is what power allows).
+// cost 64, the patch 47 and wraps 20; the MFMAs and their LDS reads alone take 758 (650 on constant operands).
+// The counters have the matrix cores busy 0.82 of the time at 1.73 GHz (GemmSplit: 0.61 at 1.86), so power bounds it; 64 on 56 x 56, with 1.4 vector instructions an
+// MFMA instead of 0.5, 0.54 at 1.98.
 //
 // Sums: a partial sum of one, two or three taps (of 32 channels each) is added to the result's: the longer it is the more error it has, the shorter
 // the more of them are added, which large results feel most.  Errors against 64 bits on images after a ReLU, three sets of operands, GemmSplit's and
