@@ -194,3 +194,22 @@ def test_no_block_fused_pair_of_the_batch_suites_is_left_out_for_registers(i, tm
 def test_operators_that_one_workgroup_can_hold(k1, k2):
     reg = {k.name: k for k in bf.list_kernels()}
     assert build_pairs.hfuse_possible(reg[k1], reg[k2], build_pairs.op_lds(k1), build_pairs.op_lds(k2))
+
+
+def test_an_object_that_failed_a_check_is_not_there_for_the_next_make(tmp_path):
+    """... which otherwise takes it for built and links a kernel that spills."""
+    (tmp_path / "pairs_0.hip").write_text("""
+#include <hip/hip_runtime.h>
+extern "C" __global__ __launch_bounds__(1024) void spills(float* p)
+{
+    float v[160], s = 0.f;
+    for (int i = 0; i < 160; ++i) v[i] = p[i * 1024 + threadIdx.x];
+    for (int i = 0; i < 160; ++i) asm volatile("" : "+v"(v[i]));
+    for (int i = 159; i >= 0; --i) s = s * 1.5f + v[i];
+    p[threadIdx.x] = s;
+}
+""")
+    for _ in range(2):
+        r = subprocess.run(["make", "-C", build_pairs.CSRC, f"MODDIR={tmp_path}", str(tmp_path / "pairs_0.o")], capture_output=True, text=True)
+        assert r.returncode != 0 and "spills registers" in r.stdout + r.stderr, r.stderr[-2000:]
+        assert not (tmp_path / "pairs_0.o").exists() and build_pairs.spilling_kernels((tmp_path / "pairs_0.res").read_text()) == ["spills"]
