@@ -32,15 +32,19 @@
 // multiple of 256 bytes apart read conflict-free).  The loop needs a quarter of the LDS read rate
 // even so, whereas the staging stores, which the shift makes conflict-free, are on the critical path.
 //
-// Measured on the ResNet shape (64 -> 64 channels, 56 x 56, 196 workgroups; in-kernel clocks): filter
-// rows 1.5 us and patch 1.4 us (overlapping), loop 2.2 us (the MFMA pipe rate), reduction and stores
-// 0.85 us, ~1.5 us launch: 6.3-6.9 us.  The lane order of
-// the staging matters as much as the loop: with the chunk index fastest the scattered 4-byte LDS
+// Measured on the ResNet shape (64 -> 64 channels, 56 x 56, 196 workgroups; in-kernel clocks): requests 0.7 us, filter rows to
+// registers (ops_conv_filters.h) and patch to LDS 0.8, loop 2.1 (the MFMA pipe rate), reduction and stores 0.4, launch and arguments ~1.3: 5.3 us
+// queued.  With filter rows loaded as the lanes want them (a line of its own for each), a test and a branch for each load of the patch, five staged rows where a tile
+// touches four, and the whole tile zeroed first it was 6.6; fused with the max-pool 6.8 -> 5.4, with dense layers 1.02 - 1.10x; 128 channels on 28 x 28 8.8 -> 6.2.
+// The lane order of the staging matters as much as the loop: with the chunk index fastest the scattered 4-byte LDS
 // stores were 16-way bank conflicts and the patch alone took 2.9 us.
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <numeric>
+
 #include "dispatch.h"
+#include "ops_conv_filters.h"
 #include "wave.h"
 
 namespace bfuse {
@@ -57,18 +61,20 @@ struct Conv3x3F32Lds {
     static constexpr int GPW = NGROUP / KS;          // groups per wave
     static constexpr int TP = 16 * PB;               // pixels per tile (consecutive in row-major order)
     static constexpr int NPT = HW / TP;
-    static constexpr int SPAN = (TP + W - 2) / W + 1;   // image rows TP consecutive pixels can touch
+    // image rows TP consecutive pixels can touch: a tile starts at a multiple of TP, and so at a multiple of its common divisor with W in a row
+    static constexpr int SPAN = (W - std::gcd(TP, W) + TP - 1) / W + 1;
     static constexpr int R = SPAN + 2, WP = W + 2;      // staged rows / columns, one of padding on each side
     static constexpr int NPOS = R * WP;
     // bytes of one channel quad, [position][4 channels], padded to 16 (mod 256): the four planes then
     // start one 16-byte slot apart in the banks, which is what makes the staging writes below conflict-free
     // (and the tap reads two-way conflicted: the cheaper side of the trade, see the header)
     static constexpr int PLANE = (NPOS * 16 + 255) / 256 * 256 + 16;
-    static constexpr int TILE_BYTES = 4 * PLANE;
+    using Filters = FilterRows<CI, 9, TM>;              // (pass through the tile before the patch is staged)
+    static constexpr int TILE_BYTES = 4 * PLANE > Filters::BYTES ? 4 * PLANE : Filters::BYTES;
     static constexpr int CPR = W / 4;                   // 16-byte chunks per image row
     static constexpr int NCH = R * CPR;                 // 16-byte chunks per channel of the patch (contiguous in memory)
     static constexpr int NLD = (NCH + 3) / 4;           // wave-level loads per group: 16 channels x 4 consecutive chunks each
-    static constexpr int NZ = (TILE_BYTES + 1023) / 1024;
+    static constexpr int NZ = (8 * R + 63) / 64;        // positions of padding (two a row and plane), 64 at a time
     static_assert(CI % 16 == 0 && CO % BM == 0 && BM % 16 == 0, "channel tiling");
     static_assert(HW % TP == 0 && NGROUP % KS == 0 && W % 4 == 0, "pixel / reduction tiling");
     static_assert((2 * WP + 2) * 16 + 3 * PLANE < 65536, "tap offsets are 16-bit immediates");
@@ -130,14 +136,6 @@ struct Conv3x3F32Lds {
         const int li = lane & 15, kq = lane >> 4;
         unsigned char* const tile = sm.t + wave * TILE_BYTES;
 
-        // padding (and rows outside the image) read as zero: 0 * w adds exactly 0, as a border
-        // test would
-#pragma unroll
-        for (int z = 0; z < NZ; ++z) {
-            const int off = z * 1024 + lane * 16;
-            if (off < TILE_BYTES) *reinterpret_cast<f32x4*>(tile + off) = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-
         // this lane's pixel of each block: the top-left tap of its window, plane kq
         const unsigned char* bbase[PB];
 #pragma unroll
@@ -156,35 +154,44 @@ struct Conv3x3F32Lds {
         for (int gi = 0; gi < GPW; ++gi) {
             const int ci0 = (wave + gi * KS) * 16;
             // A operand: Wt[co][ci0 + 4 kq + t][tap], t = 0..3, tap = 0..8 -- 36 consecutive floats
-            f32x4 aw[TM][9];
-#pragma unroll
-            for (int tm = 0; tm < TM; ++tm) {
-                const f32x4* src = reinterpret_cast<const f32x4*>(Wt + ((size_t)(co0 + tm * 16 + li) * CI + ci0 + 4 * kq) * 9);
-#pragma unroll
-                for (int j = 0; j < 9; ++j) aw[tm][j] = src[j];
-            }
+            Filters aw;
+            if (gi > 0) Filters::reads_done();         // of the patch before
+            Filters::request(Wt, co0, ci0, 0, tile, lane);
             // stage the patch: lane = 4 * channel + (chunk % 4), i.e. a wave-level load takes four
             // consecutive 16-byte chunks (64 bytes) of each of the 16 channels.  The four values of a chunk
             // go to four consecutive positions of the channel's plane; with this lane order the 64 lanes of
             // each of those stores fall in 64 different banks (channel % 4 -> word, channel / 4 -> plane,
-            // one slot apart, chunk % 4 -> 64 bytes apart)
+            // one slot apart, chunk % 4 -> 64 bytes apart).  The patch's rows follow each other in memory; the chunks
+            // of rows outside the image are read past the buffer's end and so are zeros: 0 * w adds exactly 0, as a
+            // border test would.
             const int cl = lane >> 2, c4 = lane & 3;
+            const int first = y_lo == 0 ? CPR : 0, end = (H + 1 - y_lo < R ? H + 1 - y_lo : R) * CPR;   // chunks inside it
+            const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(X + (size_t)ci0 * HW), 0, 16 * HW * 4, 0x00020000);
+            const unsigned x_voff = (unsigned)((cl * HW + (y_lo - 1) * W) * 4 + c4 * 16);
             f32x4 v[NLD];
 #pragma unroll
             for (int j = 0; j < NLD; ++j) {
                 const int cc = j * 4 + c4;                 // chunk within the channel's R x W patch
-                const int r = cc / CPR, c = cc % CPR;
-                const int yy = y_lo - 1 + r;
-                const bool ok = cc < NCH && yy >= 0 && yy < H;
-                v[j] = ok ? *reinterpret_cast<const f32x4*>(X + (size_t)(ci0 + cl) * HW + yy * W + 4 * c) : f32x4{0.f, 0.f, 0.f, 0.f};
+                v[j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, cc >= first && cc < end ? x_voff + j * 64 : 0x7fffffffu, 0, 0));
+            }
+            aw.template take<NLD>(0, tile, lane);
+#pragma unroll
+            for (int tm = 1; tm < TM; ++tm) {
+                Filters::request(Wt, co0, ci0, tm, tile, lane);
+                aw.template take<0>(tm, tile, lane);
+            }
+            // the columns beside the image
+#pragma unroll
+            for (int z = 0; z < NZ; ++z) {
+                const int i = z * 64 + lane, r = (i >> 1) % R, q = (i >> 1) / R;
+                if (8 * R % 64 == 0 || q < 4) *reinterpret_cast<f32x4*>(tile + q * PLANE + (r * WP + (i & 1) * (W + 1)) * 16) = f32x4{0.f, 0.f, 0.f, 0.f};
             }
 #pragma unroll
             for (int j = 0; j < NLD; ++j) {
                 const int cc = j * 4 + c4;
-                const int r = cc / CPR, c = cc % CPR;
-                const int yy = y_lo - 1 + r;
-                if (cc < NCH && yy >= 0 && yy < H) {
-                    float* dst = reinterpret_cast<float*>(tile + (cl / 4) * PLANE + (r * WP + 1 + 4 * c) * 16) + cl % 4;
+                if (NCH % 4 == 0 || cc < NCH) {
+                    // row cc / CPR, column 4 (cc % CPR): every row has two positions more than the image's
+                    float* dst = reinterpret_cast<float*>(tile + (cl / 4) * PLANE + (4 * cc + 2 * (cc / CPR) + 1) * 16) + cl % 4;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) dst[4 * e] = v[j][e];
                 }
@@ -207,7 +214,7 @@ struct Conv3x3F32Lds {
                     for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
                         for (int pb = 0; pb < PB; ++pb)
-                            acc[tm][pb] = __builtin_amdgcn_mfma_f32_16x16x4f32(aw[tm][(t * 9 + tap) / 4][(t * 9 + tap) % 4],
+                            acc[tm][pb] = __builtin_amdgcn_mfma_f32_16x16x4f32(aw.w[tm][(t * 9 + tap) / 4][(t * 9 + tap) % 4],
                                                                                b[tap & 1][pb][t], acc[tm][pb], 0, 0, 0);
             }
         }
