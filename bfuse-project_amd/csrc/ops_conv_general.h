@@ -32,7 +32,10 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <numeric>
+
 #include "dispatch.h"
+#include "ops_conv_filters.h"
 #include "wave.h"
 
 namespace bfuse {
@@ -54,19 +57,28 @@ struct ConvF32Lds {
     static constexpr int TM = BM / 16;
     static constexpr int TP = 16 * PB;                  // output pixels per tile (consecutive in row-major order)
     static constexpr int NPT = (OHW + TP - 1) / TP;
-    static constexpr int SPAN0 = (TP + OW - 2) / OW + 1;         // output rows TP consecutive pixels can touch
+    static constexpr int SPAN0 = (OW - std::gcd(TP, OW) + TP - 1) / OW + 1;         // output rows TP consecutive pixels can touch (as in Conv3x3F32Lds)
     static constexpr int SPAN = SPAN0 < OH ? SPAN0 : OH;
     static constexpr int R = (SPAN - 1) * S + KH, WP = W + 2 * P;   // staged rows / columns
     static constexpr int NPOS = R * WP;
     // bytes of one channel quad, [position][4 channels], padded to 16 (mod 256): the planes then start one
     // 16-byte slot apart in the banks (see ops_conv.h)
     static constexpr int PLANE = (NPOS * 16 + 255) / 256 * 256 + 16;
-    static constexpr int TILE_BYTES = NQ * PLANE;
+    // Filters of 2 - 9 taps come to the registers through the wave's tile, before the patch is staged (ops_conv_filters.h); the patch's rows by the buffer
+    // load's own range check instead of a test and a branch for every load.  us alone, 3 x 3 layers of one image: 512 channels on 7 x 7 14.8 -> 8.7, 256 on 14 x 14 8.7 -> 5.7, 256 -> 512 at
+    // stride 2 9.9 -> 6.3, 128 -> 256 6.4 -> 4.5, 64 -> 128 6.0 -> 4.6; 1 x 1 at stride 2 (the rows alone) 5.2 -> 4.3, 3.5 -> 3.0, 3.1 -> 2.8.  (One tap
+    // is 64 bytes of 16 rows as it lies; more than nine would take more LDS than the patch.)
+    static constexpr bool TURNED = CG == 16 && T > 1 && T <= 9;
+    using Filters = FilterRows<CI, T, TM>;
+    static constexpr int TILE_BYTES = TURNED && Filters::BYTES > NQ * PLANE ? Filters::BYTES : NQ * PLANE;
     static constexpr int VW = W % 4 == 0 ? 4 : (W % 2 == 0 ? 2 : 1);   // floats per staging load: image rows start on VW*4-byte boundaries
     static constexpr int LPC = 64 / CG;                 // lanes that share a channel while staging
     static constexpr int NU = R * W / VW;               // staging units per channel
     static constexpr int NLD = (NU + LPC - 1) / LPC;    // wave-level loads per group
-    static constexpr int NZ = (TILE_BYTES + 1023) / 1024;
+    static constexpr int NZ = (NQ * PLANE + 1023) / 1024;
+    // staged straight from the rows; those outside the image are stored as zeros, so that only the columns beside it need zeros of their own
+    static constexpr bool BY_ROWS = VW == 4 || W < 4 || NIMG == 1;
+    static constexpr int NPAD = R * 2 * P * NQ;         // positions of padding
     static_assert(WM_ == 0, "shared tiles have stages of four channels and one or two waves over the output channels");
     static_assert(CG == 16 ? CI % 16 == 0 : CI <= 4, "input channels: a multiple of 16, or at most 4");
     static_assert(CO % BM == 0 && BM % 16 == 0 && NGROUP % KS == 0, "channel tiling");
@@ -142,11 +154,22 @@ struct ConvF32Lds {
         const int li = lane & 15, kq = lane >> 4;
         unsigned char* const tile = sm.t + wave * TILE_BYTES;
 
+        auto zero = [&]() {
+            if constexpr (BY_ROWS) {
 #pragma unroll
-        for (int z = 0; z < NZ; ++z) {
-            const int off = z * 1024 + lane * 16;
-            if (off < TILE_BYTES) *reinterpret_cast<f32x4*>(tile + off) = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
+                for (int z = 0; z < (NPAD + 63) / 64; ++z) {
+                    const int i = z * 64 + lane, c = i % (P > 0 ? 2 * P : 1), r = i / (P > 0 ? 2 * P : 1) % R, q = i / (P > 0 ? 2 * P * R : 1);
+                    if (NPAD % 64 == 0 || i < NPAD) *reinterpret_cast<f32x4*>(tile + q * PLANE + (r * WP + (c < P ? c : W + c)) * 16) = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+            } else {
+#pragma unroll
+                for (int z = 0; z < NZ; ++z) {
+                    const int off = z * 1024 + lane * 16;
+                    if (off < NQ * PLANE) *reinterpret_cast<f32x4*>(tile + off) = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+            }
+        };
+        if constexpr (!TURNED) zero();
 
         // this lane's pixel of each block: the top-left tap of its window; channel quad kq (CG = 16) or
         // channel kq of the only quad (CG = 4)
@@ -172,18 +195,40 @@ struct ConvF32Lds {
             // boundary.  CG = 4: Wt[co][kq][tap], T consecutive floats (zero for a channel the layer does not have).
             constexpr int NA = CG == 16 ? T : (T + 3) / 4;
             f32x4 aw[TM][NA];
-#pragma unroll
-            for (int tm = 0; tm < TM; ++tm) {
-                if constexpr (CG == 16) {
-                    const f32x4* src = reinterpret_cast<const f32x4*>(Wt + ((size_t)(co0 + tm * 16 + li) * CI + ci0 + 4 * kq) * T);
-#pragma unroll
-                    for (int j = 0; j < T; ++j) aw[tm][j] = src[j];
-                } else {
-                    const float* src = Wt + ((size_t)(co0 + tm * 16 + li) * CI + (kq < CI ? kq : 0)) * T;
-#pragma unroll
-                    for (int j = 0; j < 4 * NA; ++j) aw[tm][j / 4][j % 4] = (j < T && kq < CI) ? src[j] : 0.f;
-                }
+            Filters filters;
+            if constexpr (TURNED) {
+                if (gi > 0) Filters::reads_done();         // of the patch before
+                Filters::request(Wt, co0, ci0, 0, tile, lane);
             }
+            // the filters, with BEHIND loads behind the last one's; the tile is the patch's from here on
+            auto take_filters = [&](auto behind) {
+                if constexpr (TURNED) {
+                    filters.template take<decltype(behind)::value>(0, tile, lane);
+#pragma unroll
+                    for (int tm = 1; tm < TM; ++tm) {
+                        Filters::request(Wt, co0, ci0, tm, tile, lane);
+                        filters.template take<0>(tm, tile, lane);
+                    }
+#pragma unroll
+                    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+                        for (int j = 0; j < T; ++j) aw[tm][j] = filters.w[tm][j];
+                    zero();
+                } else {
+#pragma unroll
+                    for (int tm = 0; tm < TM; ++tm) {
+                        if constexpr (CG == 16) {
+                            const f32x4* src = reinterpret_cast<const f32x4*>(Wt + ((size_t)(co0 + tm * 16 + li) * CI + ci0 + 4 * kq) * T);
+#pragma unroll
+                            for (int j = 0; j < T; ++j) aw[tm][j] = src[j];
+                        } else {
+                            const float* src = Wt + ((size_t)(co0 + tm * 16 + li) * CI + (kq < CI ? kq : 0)) * T;
+#pragma unroll
+                            for (int j = 0; j < 4 * NA; ++j) aw[tm][j / 4][j % 4] = (j < T && kq < CI) ? src[j] : 0.f;
+                        }
+                    }
+                }
+            };
             // stage the patch: LPC lanes share a channel and take consecutive units (VW floats) of its R x W
             // rows, which are contiguous in memory
             const int cl = lane / LPC, cu = lane % LPC;
@@ -193,40 +238,43 @@ struct ConvF32Lds {
             // loads straight from their rows (9.9 / 11.4 / 17.0 us against 12.2 / 14.6 / 19.2 for the 14x14 and 7x7
             // layers of ResNet-18); a batch of images (throughput) from aligned 16-byte loads, a quarter of the load
             // instructions (1024 images: 20-45 % faster on 35-, 73-, 147- and 299-wide images, 8-11 % on 14 and 7).
-            if constexpr (VW == 4 || W < 4 || NIMG == 1) {
+            if constexpr (BY_ROWS) {
                 constexpr int JB = NLD < 16 ? NLD : 16;
                 // a single image is in the latency regime: its few batches are unrolled (the next batch's loads go out
                 // under this one's LDS writes); a batch of images keeps the registers for wider tiles and loops
                 constexpr int NBATCH = (NLD + JB - 1) / JB, UNROLL = (NIMG == 1 && NBATCH <= 4) ? NBATCH : 1;
+                // The patch's rows follow each other in memory; units of rows outside the image, and of channels that the layer
+                // does not have, are read past the buffer's end, which gives zeros.
+                const int first = iy_lo < 0 ? -iy_lo * (W / VW) : 0, end = (H - iy_lo < R ? H - iy_lo : R) * (W / VW);
+                const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(X + (size_t)ci0 * HW), 0, (CG < CI ? CG : CI) * HW * 4, 0x00020000);
+                const unsigned x_voff = (unsigned)((cl * HW + iy_lo * W + cu * VW) * 4);
+                if constexpr (NBATCH > 1) take_filters(std::integral_constant<int, 0>{});
 #pragma unroll UNROLL
                 for (int j0 = 0; j0 < NLD; j0 += JB) {
                     float v[JB][VW];
 #pragma unroll
                     for (int jj = 0; jj < JB; ++jj) {
                         const int u = (j0 + jj) * LPC + cu;
-                        const int r = (u * VW) / W, x = (u * VW) % W;
-                        const int iy = iy_lo + r;
-                        const bool ok = j0 + jj < NLD && u < NU && iy >= 0 && iy < H && ci0 + cl < CI;
-                        const float* src = X + (size_t)(ci0 + cl) * HW + iy * W + x;
+                        const unsigned at = u >= first && u < end ? x_voff + (j0 + jj) * (LPC * VW * 4) : 0x7fffffffu;
                         if constexpr (VW == 4) {
-                            const f32x4 q = ok ? *reinterpret_cast<const f32x4*>(src) : f32x4{0.f, 0.f, 0.f, 0.f};
+                            const f32x4 q = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, at, 0, 0));
 #pragma unroll
                             for (int e = 0; e < 4; ++e) v[jj][e] = q[e];
                         } else if constexpr (VW == 2) {
-                            const f32x2 q = ok ? *reinterpret_cast<const f32x2*>(src) : f32x2{0.f, 0.f};
+                            const f32x2 q = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(xr, at, 0, 0));
                             v[jj][0] = q[0];
                             v[jj][1] = q[1];
                         } else {
-                            v[jj][0] = ok ? *src : 0.f;
+                            v[jj][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, at, 0, 0));
                         }
                     }
+                    if constexpr (NBATCH == 1) take_filters(std::integral_constant<int, JB>{});
 #pragma unroll
                     for (int jj = 0; jj < JB; ++jj) {
                         const int u = (j0 + jj) * LPC + cu;
-                        const int r = (u * VW) / W, x = (u * VW) % W;
-                        const int iy = iy_lo + r;
-                        if (j0 + jj < NLD && u < NU && iy >= 0 && iy < H && ci0 + cl < CI) {
-                            float* dst = reinterpret_cast<float*>(tile + (cl / 4) * PLANE + (r * WP + P + x) * 16) + cl % 4;
+                        if (u < NU) {
+                            // row u VW / W: every row has 2 P positions more than the image's
+                            float* dst = reinterpret_cast<float*>(tile + (cl / 4) * PLANE + (u * VW + u * VW / W * (2 * P) + P) * 16) + cl % 4;
 #pragma unroll
                             for (int e = 0; e < VW; ++e) dst[4 * e] = v[jj][e];
                         }
@@ -237,6 +285,7 @@ struct ConvF32Lds {
                 // starts off one): the rows of a channel that lie inside the image are one contiguous span, which
                 // is fetched with ALIGNED 16-byte loads from the boundary below its start; each of a vector's
                 // four floats then finds its own (row, column), and those before and behind the span are dropped.
+                take_filters(std::integral_constant<int, 0>{});
                 const int r_lo = iy_lo < 0 ? -iy_lo : 0;
                 const int r_hi = H - iy_lo < R ? H - iy_lo : R;
                 const int len = (r_hi - r_lo) * W;
