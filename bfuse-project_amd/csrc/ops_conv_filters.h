@@ -57,4 +57,42 @@ struct FilterRows {
     }
 };
 
+// The same for the layers of at most four channels: lane (i, q) gets channel q of filter row i, T consecutive floats (zeros for a channel that there is
+// not).  16 rows are 16 CI T consecutive floats.
+template <int CI, int T, int TM>
+struct FilterFloats {
+    static constexpr int LOADS = (16 * CI * T * 4 + 1023) / 1024, BYTES = 1024 * LOADS;
+    float w[TM][T];
+
+    __device__ static __forceinline__ void request(const float* Wt, int co0, int, int tm, unsigned char* room, int lane)
+    {
+        const auto wr = __builtin_amdgcn_make_buffer_rsrc((void*)(Wt + (size_t)(co0 + 16 * tm) * CI * T), 0, 16 * CI * T * 4, 0x00020000);
+#pragma unroll
+        for (int j = 0; j < LOADS; ++j)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (__attribute__((address_space(3))) void*)(room + j * 1024), 16, (unsigned)(lane * 16), j * 1024, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    template <int BEHIND>
+    __device__ __forceinline__ void take(int tm, const unsigned char* room, int lane)
+    {
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm volatile("s_waitcnt vmcnt(%0) ; loads into LDS have landed" : : "n"(BEHIND) : "memory");
+#endif
+        const int li = lane & 15, kq = lane >> 4;
+        const float* const from = reinterpret_cast<const float*>(room) + (li * CI + (kq < CI ? kq : 0)) * T;
+#pragma unroll
+        for (int j = 0; j < T; ++j) w[tm][j] = from[j];
+#pragma unroll
+        for (int j = 0; j < T; ++j) w[tm][j] = CI == 4 || kq < CI ? w[tm][j] : 0.f;
+        reads_done();
+    }
+    __device__ static __forceinline__ void reads_done()
+    {
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+#endif
+        __builtin_amdgcn_sched_barrier(0);
+    }
+};
+
 }  // namespace bfuse

@@ -10,11 +10,13 @@
 // workgroup holds, which lets more workgroups share a CU.  The MFMA loop is ConvF32Lds's: per lane a base
 // address in the patch plus a compile-time offset per tap.
 //
-// A patch row is a piece of an image row that starts anywhere, so it is fetched with ALIGNED 16-byte loads from
-// the boundary below its start; each float of a vector knows its own column, and those outside the patch or
-// the image are dropped (they stay zero in the tile, which is what padding reads as).  Output columns past
+// A patch row is a piece of an image row that starts anywhere.  It is fetched with 16-byte loads from its start on, whose floats beside the
+// image are made zeros (which is what padding reads as), and is a whole number of them long in LDS, so that every float of a load has its place.  Rows past the
+// image come from past the buffer's end, as zeros.  (With aligned loads each float of a vector has to find its own column and a place, if it has one: six
+// vector instructions a float where this takes two.)  Output columns past
 // the image (OW not a multiple of 16) and rows past it (OH not a multiple of TH) are computed on whatever the
-// patch holds there and not stored.
+// patch holds there and not stored.  us, before and now, with the filters through LDS (ops_conv_filters.h): 7 x 7 on one RGB image 8.8 -> 7.2, on 64 281 -> 216,
+// 3 x 3 at stride 2 on 64 images of 299 x 299 80 -> 63, 64 channels on 56 x 56 6.6 -> 5.8.
 //
 // Replaces the same TVM-generated `conv2d` kernels of the reference as ConvF32Lds
 // (scripts/configure_kernels.py:28-38,60-68); which of the two a shape gets is ConvTiling's choice.
@@ -47,17 +49,20 @@ struct ConvF32Rect {
     static constexpr int TM = BM / 16;
     static constexpr int PB = TH;                       // 16-pixel blocks of the tile: one per output row
     static constexpr int NTX = (OW + 15) / 16, NTY = (OH + TH - 1) / TH, NPT = NTX * NTY;
-    static constexpr int PR = (TH - 1) * S + KH, PC = 15 * S + KW;   // patch rows / columns
+    static constexpr int PR = (TH - 1) * S + KH, PC = (15 * S + KW + 3) / 4 * 4;   // patch rows / columns, whole vectors of four
     static constexpr int NPOS = PR * PC;
     // bytes of one channel quad, [position][4 channels], padded to 16 (mod 256): the planes then start one
     // 16-byte slot apart in the banks (see ops_conv.h)
     static constexpr int PLANE = (NPOS * 16 + 255) / 256 * 256 + 16;
-    static constexpr int TILE_BYTES = NQ * PLANE;
+    // The filters come to the registers through the wave's tile, before the patch is staged (ops_conv_filters.h), where they are not
+    // much more than the patch: up to nine taps of 16 channels, 7 x 7 of three.
+    static constexpr bool TURNED = T > 1 && (CG == 16 ? T <= 9 : CI * T <= 160);
+    using Filters = std::conditional_t<CG == 16, FilterRows<CI, T, BM / 16>, FilterFloats<CI, T, BM / 16>>;
+    static constexpr int TILE_BYTES = TURNED && Filters::BYTES > NQ * PLANE ? Filters::BYTES : NQ * PLANE;
     static constexpr int LPC = 64 / CG;                 // lanes that share a channel while staging
-    static constexpr int NVR = (PC + 3) / 4 + 1;        // aligned 16-byte vectors that can overlap one patch row
+    static constexpr int NVR = PC / 4;                  // vectors of a patch row
     static constexpr int NU = PR * NVR;                 // staging units (row, vector) per channel
     static constexpr int NLD = (NU + LPC - 1) / LPC;    // wave-level loads per group
-    static constexpr int NZ = (TILE_BYTES + 1023) / 1024;
     static_assert(CG == 16 ? CI % 16 == 0 : CI <= 4, "input channels: a multiple of 16, or at most 4");
     static_assert(CO % BM == 0 && BM % 16 == 0 && NGROUP % KS == 0, "channel tiling");
     static_assert(((KH - 1) * PC + KW - 1) * 16 + (NQ - 1) * PLANE + 16 < 65536, "tap offsets are 16-bit immediates");
@@ -131,12 +136,6 @@ struct ConvF32Rect {
         const int li = lane & 15, kq = lane >> 4;
         unsigned char* const tile = sm.t + wave * TILE_BYTES;
 
-#pragma unroll
-        for (int z = 0; z < NZ; ++z) {
-            const int off = z * 1024 + lane * 16;
-            if (off < TILE_BYTES) *reinterpret_cast<f32x4*>(tile + off) = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-
         // this lane's pixel of each block: the top-left tap of its window; channel quad kq (CG = 16) or
         // channel kq of the only quad (CG = 4)
         const unsigned char* bbase[PB];
@@ -149,10 +148,6 @@ struct ConvF32Rect {
 #pragma unroll
             for (int pb = 0; pb < PB; ++pb) acc[tm][pb] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-        // columns of the patch that lie inside the image
-        const int c_lo = ix0 < 0 ? -ix0 : 0;
-        const int c_hi = W - ix0 < PC ? W - ix0 : PC;
-
 #pragma unroll 1
         for (int gi = 0; gi < GPW; ++gi) {
             const int ci0 = (wave + gi * KS) * CG;
@@ -160,66 +155,81 @@ struct ConvF32Rect {
             // boundary.  CG = 4: Wt[co][kq][tap], T consecutive floats (zero for a channel the layer does not have).
             constexpr int NA = CG == 16 ? T : (T + 3) / 4;
             f32x4 aw[TM][NA];
-#pragma unroll
-            for (int tm = 0; tm < TM; ++tm) {
-                if constexpr (CG == 16) {
-                    const f32x4* src = reinterpret_cast<const f32x4*>(Wt + ((size_t)(co0 + tm * 16 + li) * CI + ci0 + 4 * kq) * T);
-#pragma unroll
-                    for (int j = 0; j < T; ++j) aw[tm][j] = src[j];
-                } else {
-                    const float* src = Wt + ((size_t)(co0 + tm * 16 + li) * CI + (kq < CI ? kq : 0)) * T;
-#pragma unroll
-                    for (int j = 0; j < 4 * NA; ++j) aw[tm][j / 4][j % 4] = (j < T && kq < CI) ? src[j] : 0.f;
-                }
+            Filters filters;
+            if constexpr (TURNED) {
+                if (gi > 0) Filters::reads_done();             // of the patch before
+                Filters::request(Wt, co0, ci0, 0, tile, lane);
             }
+            // the filters, with BEHIND loads behind the last one's; the tile is the patch's from here on
+            auto take_filters = [&](auto behind) {
+                constexpr int BEHIND = decltype(behind)::value;
+                if constexpr (TURNED) {
+                    filters.template take<BEHIND>(0, tile, lane);
+#pragma unroll
+                    for (int tm = 1; tm < TM; ++tm) {
+                        Filters::request(Wt, co0, ci0, tm, tile, lane);
+                        filters.template take<0>(tm, tile, lane);
+                    }
+#pragma unroll
+                    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+                        for (int j = 0; j < (CG == 16 ? T : 4 * NA); ++j) {
+                            if constexpr (CG == 16) aw[tm][j] = filters.w[tm][j];
+                            else aw[tm][j / 4][j % 4] = j < T ? filters.w[tm][j < T ? j : 0] : 0.f;
+                        }
+                } else {
+#pragma unroll
+                    for (int tm = 0; tm < TM; ++tm) {
+                        if constexpr (CG == 16) {
+                            const f32x4* src = reinterpret_cast<const f32x4*>(Wt + ((size_t)(co0 + tm * 16 + li) * CI + ci0 + 4 * kq) * T);
+#pragma unroll
+                            for (int j = 0; j < T; ++j) aw[tm][j] = src[j];
+                        } else {
+                            const float* src = Wt + ((size_t)(co0 + tm * 16 + li) * CI + (kq < CI ? kq : 0)) * T;
+#pragma unroll
+                            for (int j = 0; j < 4 * NA; ++j) aw[tm][j / 4][j % 4] = (j < T && kq < CI) ? src[j] : 0.f;
+                        }
+                    }
+                }
+            };
 
-            // stage the patch: LPC lanes share a channel and take the (row, vector) units of its PR patch rows in turn
+            // stage the patch: LPC lanes share a channel and take the (row, vector) units of its PR patch rows in turn.  A vector of a row outside the image, or of
+            // a channel that the layer does not have, is read past the buffer's end; its floats beside the image are made zeros, which is what padding reads as.  (What
+            // a vector has past the buffer's end is zeros float by float; one that begins before the buffer is none at all.  So the vector that begins
+            // before an image row and ends in it is read from the row's first float, and moved.)
             const int cl = lane / LPC;
             int cu = lane % LPC;
             // which positions a lane stages does not change from one channel group to the next, and the compiler would
             // work out every address ahead of the loop and keep them all in registers: hidden from it
             asm volatile("" : "+v"(cu));
-            const bool chan = ci0 + cl < CI;
-            // element index, within the image tensor, of patch position (0, 0) of this lane's channel (32-bit: an image
-            // tensor has fewer than 2^31 elements), and how far the tensor itself starts off a 16-byte boundary
-            const int chan0 = (ci0 + cl) * HW + iy0 * W + ix0;
-            const int xmis = (int)((reinterpret_cast<size_t>(X) >> 2) & 3);
-            // No branches and no lane masks in here: validity is the sign bit of an OR of differences (negative = outside),
-            // spread over the word by an arithmetic shift and used to pick between two addresses.  A vector that lies
-            // outside the image is fetched from the tensor's first 16 bytes instead, and a float that is not part of the
-            // patch is written to the 16 bytes of padding behind the plane.  (With compares, the sixteen loads and
-            // sixty-four stores of a batch each held a 64-bit mask in scalar registers, more than there are.)
+            const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(X + (size_t)ci0 * HW), 0, (CG < CI ? CG : CI) * HW * 4, 0x00020000);
+            const int corner = cl * HW + iy0 * W + ix0;
+            const bool inside = ix0 >= 0 && ix0 + PC <= W;          // no vector reaches beside the image
+            const auto begins_before = [&](int vi) { return P % 4 != 0 && ix0 < 0 && vi == P / 4; };      // (columns begin at a multiple of 16, less P)
             unsigned char* const plane = tile + (cl / 4) * PLANE + (cl % 4) * 4;
-            constexpr int DUMMY = PLANE - 16;
-            const int chan_out = chan ? 0 : -1;
             constexpr int JB = NLD < 16 ? NLD : 16;
             constexpr int NBATCH = (NLD + JB - 1) / JB, UNROLL = (NIMG == 1 && NBATCH <= 4) ? NBATCH : 1;
+            if constexpr (NBATCH > 1 || !TURNED) take_filters(std::integral_constant<int, 0>{});
 #pragma unroll UNROLL
             for (int j0 = 0; j0 < NLD; j0 += JB) {
                 f32x4 v[JB];
 #pragma unroll
                 for (int jj = 0; jj < JB; ++jj) {
                     const int u = (j0 + jj) * LPC + cu;
-                    const int r = u / NVR, vi = u % NVR;
-                    const int iy = iy0 + r;
-                    const int e0 = chan0 + r * W;                            // element index of patch position (r, 0)
-                    const int c0 = 4 * vi - ((e0 + xmis) & 3);               // patch column of the vector's first float
-                    const int out = (chan_out | (NU - 1 - u) | iy | (H - 1 - iy) | (c0 + 3 - c_lo) | (c_hi - 1 - c0)) >> 31;
-                    v[jj] = *reinterpret_cast<const f32x4*>(X + (((e0 + c0) & ~out) | (-xmis & out)));
+                    const int r = u / NVR, vi = u % NVR, iy = iy0 + r;
+                    v[jj] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, iy >= 0 && iy < H && u < NU ? (unsigned)((corner + r * W + 4 * vi + (begins_before(vi) ? P % 4 : 0)) * 4) : 0x7fffffffu, 0, 0));
                 }
+                if constexpr (NBATCH == 1 && TURNED) take_filters(std::integral_constant<int, JB>{});
                 asm volatile("" : "+v"(cu));   // likewise: the stores work their addresses out again, one vector at a time
 #pragma unroll
                 for (int jj = 0; jj < JB; ++jj) {
                     const int u = (j0 + jj) * LPC + cu;
-                    const int r = u / NVR, vi = u % NVR;
-                    const int iy = iy0 + r;
-                    const int c0 = 4 * vi - ((chan0 + r * W + xmis) & 3);
-                    const int row_out = chan_out | (NU - 1 - u) | iy | (H - 1 - iy);
+                    const int vi = u % NVR, x = ix0 + 4 * vi;
+                    const bool moved = begins_before(vi);
+                    if (NU % LPC == 0 || u < NU) {
+                        float* const dst = reinterpret_cast<float*>(plane + u * 64);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int c = c0 + e;
-                        const int out = (row_out | (c - c_lo) | (c_hi - 1 - c)) >> 31;
-                        *reinterpret_cast<float*>(plane + ((((r * PC + c) * 16) & ~out) | (DUMMY & out))) = v[jj][e];
+                        for (int e = 0; e < 4; ++e) dst[4 * e] = inside || (unsigned)(x + e) < (unsigned)W ? moved && e >= P % 4 ? v[jj][e - P % 4 >= 0 ? e - P % 4 : 0] : v[jj][e] : 0.f;
                     }
                 }
             }
