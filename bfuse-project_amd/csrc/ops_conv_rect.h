@@ -382,10 +382,14 @@ struct ConvTiling {
     static constexpr int OHW = OH * OW;
     static constexpr bool RECT = T > 1 && (OW >= 64 || ((OW >= 44 || S > 1) && 6 * OW >= 5 * ((OW + 15) / 16 * 16)));
     static constexpr int patch_bytes(int th) { return ((th - 1) * S + KH) * (15 * S + KW) * (CI >= 16 ? 64 : 16); }
-    static constexpr int TH = patch_bytes(4) <= 12800 ? 4 : patch_bytes(2) <= 12800 ? 2 : 1;
+    // A batch of images of three or four channels: 32 output channels a wave, so that what is staged and read from the patch serves two MFMAs, where the
+    // filters leave registers for that; filters of up to 25 taps on two rows.  us, 64 images, 16 channels x 4 rows / 32 x 4 / 32 x 2: 7 x 7 on 224 216 / 179 / 200, on 113 69.6 / 64.2 / 66.4; 5 x 5 on 149
+    // 36.7 / 32.7 / 31.0; 3 x 3 on 299 at stride 2 63.4 / 64.4 / 56.8, on 150 (96 channels) 49.1 / 49.6 / 42.1, at stride 1 on 112 69 / 57.9 / 55.1, on 150 54.9 / 56.7 / 51.5.  One channel: 32.6 / 35.7 / 34.7, as it was.
+    static constexpr bool FEW = RECT && NIMG > 1 && CI >= 3 && CI < 16 && CO % 32 == 0 && T <= 52;
+    static constexpr int TH = patch_bytes(4) <= 12800 && !(FEW && T <= 25) ? 4 : patch_bytes(2) <= 12800 ? 2 : 1;
     static constexpr int pick_bm()
     {
-        if (CI < 16) return 16;
+        if (CI < 16) return FEW ? 32 : 16;
         if (T == 1)      // a 1x1 filter is one register per row block: as many output channels as divide CO, up to 80
             for (int bm = 80; bm > 16; bm -= 16)     // (96 measured slower than 64 on the 8x8 and 17x17 layers)
                 if (CO % bm == 0) return bm;
