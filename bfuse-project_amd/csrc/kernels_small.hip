@@ -7,6 +7,7 @@
 #include "ops_ceiling.h"
 #include "ops_conv.h"
 #include "ops_conv_1x1.h"
+#include "ops_conv_few.h"
 #include "ops_conv_rect.h"
 #include "ops_conv_split.h"
 #include "ops_conv_tile.h"
@@ -197,18 +198,23 @@ BFUSE_HFUSE_KERNEL(selftest_conv_tile_c, ConvT_c, conv3x3_f32_32x12x12_32, ConvS
     using ConvW_##TAG = __VA_ARGS__;                                                                               \
     BFUSE_KERNEL(selftest_conv_staged_##TAG, ConvW_##TAG, ({{N, CI, H, W}, 4}), ({{CO, CI, KH, KW}, 4}),           \
                  ({{N, CO, (H - KH + 2 * P) / S + 1, (W - KW + 2 * P) / S + 1}, 4}))
-CONV_STAGED_TEST(a, 2, 3, 21, 37, 16, 5, 5, 1, 2, ConvF32Rect<3, 16, 21, 37, 5, 5, 1, 2, 16, 2, 1, 2>)             // a vector begins two floats before the row
+CONV_STAGED_TEST(a, 2, 3, 21, 37, 16, 5, 5, 1, 2, ConvF32Few<3, 16, 21, 37, 5, 5, 1, 2, 16, 2, 1, 2>)             // a vector begins two floats before the row
 CONV_STAGED_TEST(b, 2, 16, 19, 50, 32, 3, 3, 1, 1, ConvF32Rect<16, 32, 19, 50, 3, 3, 1, 1, 32, 4, 1, 2>)          // one float before, two row blocks
-CONV_STAGED_TEST(c, 3, 4, 23, 35, 32, 3, 3, 2, 1, ConvF32Rect<4, 32, 23, 35, 3, 3, 2, 1, 32, 2, 1, 3>)            // four channels, two row blocks
-CONV_STAGED_TEST(d, 1, 2, 30, 30, 16, 11, 11, 1, 5, ConvF32Rect<2, 16, 30, 30, 11, 11, 1, 5, 16, 1, 1, 1>)        // 121 taps; the second vector begins before the row
+CONV_STAGED_TEST(c, 3, 4, 23, 35, 32, 3, 3, 2, 1, ConvF32Few<4, 32, 23, 35, 3, 3, 2, 1, 32, 2, 1, 3>)            // four channels, two row blocks
+CONV_STAGED_TEST(d, 1, 2, 30, 30, 16, 11, 11, 1, 5, ConvF32Few<2, 16, 30, 30, 11, 11, 1, 5, 16, 1, 1, 1>)        // 121 taps; the second vector begins before the row
 CONV_STAGED_TEST(e, 2, 64, 18, 41, 16, 3, 3, 1, 0, ConvF32Rect<64, 16, 18, 41, 3, 3, 1, 0, 16, 4, 2, 2>)          // two waves of two groups, no padding
-CONV_STAGED_TEST(f, 1, 3, 29, 62, 16, 7, 7, 2, 3, ConvF32Rect<3, 16, 29, 62, 7, 7, 2, 3, 16, 4, 1, 1>)            // 9408 bytes of filters, three floats before the row
+CONV_STAGED_TEST(f, 1, 3, 29, 62, 16, 7, 7, 2, 3, ConvF32Few<3, 16, 29, 62, 7, 7, 2, 3, 16, 4, 1, 1>)            // 9408 bytes of filters, three floats before the row
 CONV_STAGED_TEST(g, 1, 32, 9, 10, 32, 3, 3, 1, 1, ConvF32Lds<32, 32, 9, 10, 3, 3, 1, 1, 32, 2, 1, 1>)             // 8-byte loads, two groups, two row blocks
 CONV_STAGED_TEST(h, 1, 48, 7, 7, 16, 3, 3, 2, 1, ConvF32Lds<48, 16, 7, 7, 3, 3, 2, 1, 16, 1, 3, 1>)               // 4-byte loads, three waves
 CONV_STAGED_TEST(i, 3, 16, 13, 11, 16, 5, 5, 1, 2, ConvF32Lds<16, 16, 13, 11, 5, 5, 1, 2, 16, 4, 1, 3>)           // 25 taps, rows as one span
 CONV_STAGED_TEST(j, 3, 32, 15, 13, 16, 3, 3, 1, 1, ConvF32Lds<32, 16, 15, 13, 3, 3, 1, 1, 16, 4, 1, 3>)           // the same, two groups, filters through LDS
 CONV_STAGED_TEST(k, 2, 16, 10, 12, 16, 1, 3, 1, 1, ConvF32Lds<16, 16, 10, 12, 1, 3, 1, 1, 16, 4, 1, 2>)           // three taps
 CONV_STAGED_TEST(l, 1, 32, 8, 12, 32, 3, 3, 1, 1, Conv3x3F32Lds<32, 32, 8, 12, 32, 2, 1>)                        // two groups, two row blocks
+CONV_STAGED_TEST(m, 2, 3, 11, 131, 32, 3, 3, 1, 0, ConvF32Few<3, 32, 11, 131, 3, 3, 1, 0, 32, 2, 4, 2>)            // four columns a lane, 129 of 192: a quad cut after one
+CONV_STAGED_TEST(n, 2, 1, 13, 150, 16, 5, 5, 2, 2, ConvF32Few<1, 16, 13, 150, 5, 5, 2, 2, 16, 2, 4, 2>)            // one channel: a row a lane group and five taps of one that is left; cut after three
+CONV_STAGED_TEST(o, 2, 2, 12, 80, 32, 3, 3, 1, 1, ConvF32Few<2, 32, 12, 80, 3, 3, 1, 1, 32, 2, 4, 2, true>)        // two rows left, six taps; written past the caches
+CONV_STAGED_TEST(p, 1, 3, 40, 66, 16, 7, 7, 2, 3, ConvF32Few<3, 16, 40, 66, 7, 7, 2, 3, 16, 8, 1, 1>)              // eight rows
+BFUSE_HFUSE_KERNEL(selftest_conv_staged_m, ConvW_m, bias_relu_4096, BiasReluS)
 BFUSE_HFUSE_KERNEL(selftest_conv_staged_a, ConvW_a, bias_relu_4096, BiasReluS)
 BFUSE_BFUSE_KERNEL(selftest_conv_staged_g, ConvW_g, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
 BFUSE_HFUSE_KERNEL(selftest_conv_staged_l, ConvW_l, bias_relu_4096, BiasReluS)

@@ -57,44 +57,58 @@ struct FilterRows {
     }
 };
 
-// The same for the layers of at most four channels: lane (i, q) gets channel q of filter row i, T consecutive floats (zeros for a channel that there is
-// not).  16 rows are 16 CI T consecutive floats; lanes behind them load the last ones again.  A workgroup comes here once and has one wave, so the loads are written by hand and
-// everything that is under way is waited for.  (Through registers, which 32 channels of 7 x 7 filters have not enough of for three waves a SIMD: 2827 us instead of 2684 on 1024 images of 224 x 224.)
-template <int CI, int T, int TM>
+// The same for images of at most four channels (ConvF32Few), whose MFMAs have four rows of the window at a tap, or four taps of the rows that are left, for
+// their k: lane (i, q) gets, of filter row i, RPL rows of the window from row q RPL on, which are consecutive floats, and taps q, 4 + q .. of the rest (zeros past the last one).  16 rows
+// are 16 CI KH KW consecutive floats; lanes behind them load the last ones again.  A workgroup comes here once and has one wave, so the loads are written by hand and
+// everything that is under way is waited for.  (Through registers the 7 x 7 layer of 1024 images took 5 % longer: a wave has not enough of them.)
+template <int CI, int KH, int KW, int TM>
 struct FilterFloats {
-    static constexpr int SIZE = 16 * CI * T * 4, LOADS = (SIZE + 1023) / 1024, BYTES = 1024 * LOADS;
+    static constexpr int ROWS = CI * KH, RPL = ROWS / 4, LEFT = ROWS % 4 * KW, NLT = (LEFT + 3) / 4, NM = RPL * KW + NLT, N = ROWS * KW;
+    static constexpr int SIZE = 16 * N * 4, LOADS = (SIZE + 1023) / 1024, BYTES = 1024 * LOADS;
     typedef __attribute__((address_space(3))) unsigned char lds_u8;
-    float w[TM][T];
+    float w[TM][NM];
 
-    __device__ static __forceinline__ void request(const float* Wt, int co0, int, int tm, unsigned char* room, int lane)
+    // The first 16 rows on their way into `room` (BYTES).
+    __device__ static __forceinline__ void request(const float* Wt, int co0, int tm, unsigned char* room, int lane)
     {
 #pragma unroll
         for (int j = 0; j < LOADS; ++j) {
             const unsigned at = (unsigned)(lane * 16 + j * 1024);
-            dma_load_lds_b128(j * 1024 + 1024 <= SIZE || at + 16 <= SIZE ? at : SIZE - 16, Wt + (size_t)(co0 + 16 * tm) * CI * T, (unsigned)(unsigned long long)(lds_u8*)(room + j * 1024));
+            dma_load_lds_b128(j * 1024 + 1024 <= SIZE || at + 16 <= SIZE ? at : SIZE - 16, Wt + (size_t)(co0 + 16 * tm) * N, (unsigned)(unsigned long long)(lds_u8*)(room + j * 1024));
         }
         __builtin_amdgcn_sched_barrier(0);
     }
-    template <int>
-    __device__ __forceinline__ void take(int tm, const unsigned char* room, int lane)
+    __device__ __forceinline__ void pick(int tm, const float* row, int kq)
     {
-#if defined(__HIP_DEVICE_COMPILE__)
-        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-#endif
-        const int li = lane & 15, kq = lane >> 4;
-        const float* const from = reinterpret_cast<const float*>(room) + (li * CI + (kq < CI ? kq : 0)) * T;
 #pragma unroll
-        for (int j = 0; j < T; ++j) w[tm][j] = from[j];
-#pragma unroll
-        for (int j = 0; j < T; ++j) w[tm][j] = CI == 4 || kq < CI ? w[tm][j] : 0.f;
-        reads_done();
+        for (int m = 0; m < NM; ++m) {
+            const int i = m - RPL * KW, k = 4 * RPL * KW + 4 * i + kq;
+            w[tm][m] = i < 0 ? row[kq * RPL * KW + m] : row[k < N ? k : N - 1];
+            if (i >= 0 && 4 * i + 3 >= LEFT) w[tm][m] = k < N ? w[tm][m] : 0.f;
+        }
     }
-    __device__ static __forceinline__ void reads_done()
+    // All of them to registers, `room` is free again.
+    __device__ __forceinline__ void take(const float* Wt, int co0, unsigned char* room, int lane)
     {
+        const int li = lane & 15, kq = lane >> 4;
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm) {
+            if (tm > 0) request(Wt, co0, tm, room, lane);
 #if defined(__HIP_DEVICE_COMPILE__)
-        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+            asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
 #endif
-        __builtin_amdgcn_sched_barrier(0);
+            pick(tm, reinterpret_cast<const float*>(room) + li * N, kq);
+#if defined(__HIP_DEVICE_COMPILE__)
+            asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+#endif
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    // Filters that are too many for that, as they lie in memory.
+    __device__ __forceinline__ void load(const float* Wt, int co0, int lane)
+    {
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm) pick(tm, Wt + (size_t)(co0 + 16 * tm + (lane & 15)) * N, lane >> 4);
     }
 };
 

@@ -1,5 +1,5 @@
 // Convolution on rectangular pixel tiles: the implicit GEMM of ConvF32Lds (ops_conv_general.h: any filter size,
-// stride, padding, image size and batch; channel groups of 16 -- or 4 -- under one filter tap; KS waves over the
+// stride, padding, image size and batch; channel groups of 16 under one filter tap; KS waves over the
 // channel groups, each with a zero-padded LDS patch of its own; partial tiles summed in wave order) with the
 // workgroup's pixels arranged as TH output rows x 16 output columns instead of 64 consecutive pixels.
 //
@@ -15,8 +15,8 @@
 // image come from past the buffer's end, as zeros.  (With aligned loads each float of a vector has to find its own column and a place, if it has one: six
 // vector instructions a float where this takes two.)  Output columns past
 // the image (OW not a multiple of 16) and rows past it (OH not a multiple of TH) are computed on whatever the
-// patch holds there and not stored.  us, before and now, with the filters through LDS (ops_conv_filters.h): 7 x 7 on one RGB image 8.8 -> 7.2, on 64 281 -> 216,
-// 3 x 3 at stride 2 on 64 images of 299 x 299 80 -> 63, 64 channels on 56 x 56 6.6 -> 5.8.
+// patch holds there and not stored.  us, before and now, with the filters through LDS (ops_conv_filters.h): 64
+// channels on 56 x 56 6.6 -> 5.8.  Images of at most four channels have ConvF32Few.
 //
 // Replaces the same TVM-generated `conv2d` kernels of the reference as ConvF32Lds
 // (scripts/configure_kernels.py:28-38,60-68); which of the two a shape gets is ConvTiling's choice.
@@ -27,6 +27,7 @@
 
 #include "dispatch.h"
 #include "ops_conv_1x1.h"
+#include "ops_conv_few.h"
 #include "ops_conv_general.h"
 #include "ops_conv_split.h"
 #include "ops_conv_tile.h"
@@ -42,9 +43,9 @@ struct ConvF32Rect {
     static constexpr int CI = CI_, CO = CO_, H = H_, W = W_, KH = KH_, KW = KW_, S = S_, P = P_, BM = BM_, TH = TH_, KS = KS_, NIMG = NIMG_;
     static constexpr int OH = (H - KH + 2 * P) / S + 1, OW = (W - KW + 2 * P) / S + 1;
     static constexpr int HW = H * W, OHW = OH * OW, T = KH * KW;
-    static constexpr int CG = CI >= 16 ? 16 : 4;        // channels per group
+    static constexpr int CG = 16;                       // channels per group
     static constexpr int NQ = CG / 4;                   // channel quads = planes of the tile = MFMAs per tap
-    static constexpr int NGROUP = CG == 16 ? CI / 16 : 1;
+    static constexpr int NGROUP = CI / 16;
     static constexpr int GPW = NGROUP / KS;             // groups per wave
     static constexpr int TM = BM / 16;
     static constexpr int PB = TH;                       // 16-pixel blocks of the tile: one per output row
@@ -55,15 +56,15 @@ struct ConvF32Rect {
     // 16-byte slot apart in the banks (see ops_conv.h)
     static constexpr int PLANE = (NPOS * 16 + 255) / 256 * 256 + 16;
     // The filters come to the registers through the wave's tile, before the patch is staged (ops_conv_filters.h), where they are not
-    // much more than the patch: up to nine taps of 16 channels, 7 x 7 of three.
-    static constexpr bool TURNED = T > 1 && (CG == 16 ? T <= 9 : CI * T <= 160);
-    using Filters = std::conditional_t<CG == 16, FilterRows<CI, T, BM / 16>, FilterFloats<CI, T, BM / 16>>;
+    // much more than the patch: up to nine taps.
+    static constexpr bool TURNED = T > 1 && T <= 9;
+    using Filters = FilterRows<CI, T, BM / 16>;
     static constexpr int TILE_BYTES = TURNED && Filters::BYTES > NQ * PLANE ? Filters::BYTES : NQ * PLANE;
     static constexpr int LPC = 64 / CG;                 // lanes that share a channel while staging
     static constexpr int NVR = PC / 4;                  // vectors of a patch row
     static constexpr int NU = PR * NVR;                 // staging units (row, vector) per channel
     static constexpr int NLD = (NU + LPC - 1) / LPC;    // wave-level loads per group
-    static_assert(CG == 16 ? CI % 16 == 0 : CI <= 4, "input channels: a multiple of 16, or at most 4");
+    static_assert(CI % 16 == 0, "input channels: a multiple of 16");
     static_assert(CO % BM == 0 && BM % 16 == 0 && NGROUP % KS == 0, "channel tiling");
     static_assert(((KH - 1) * PC + KW - 1) * 16 + (NQ - 1) * PLANE + 16 < 65536, "tap offsets are 16-bit immediates");
     static_assert(S >= 1 && OH >= 1 && OW >= 1 && TH >= 1, "shape");
@@ -136,11 +137,10 @@ struct ConvF32Rect {
         const int li = lane & 15, kq = lane >> 4;
         unsigned char* const tile = sm.t + wave * TILE_BYTES;
 
-        // this lane's pixel of each block: the top-left tap of its window; channel quad kq (CG = 16) or
-        // channel kq of the only quad (CG = 4)
+        // this lane's pixel of each block: the top-left tap of its window; channel quad kq
         const unsigned char* bbase[PB];
 #pragma unroll
-        for (int pb = 0; pb < PB; ++pb) bbase[pb] = tile + ((pb * S) * PC + li * S) * 16 + (CG == 16 ? kq * PLANE : kq * 4);
+        for (int pb = 0; pb < PB; ++pb) bbase[pb] = tile + ((pb * S) * PC + li * S) * 16 + kq * PLANE;
 
         f32x4 acc[TM][PB];
 #pragma unroll
@@ -151,10 +151,8 @@ struct ConvF32Rect {
 #pragma unroll 1
         for (int gi = 0; gi < GPW; ++gi) {
             const int ci0 = (wave + gi * KS) * CG;
-            // A operand.  CG = 16: Wt[co][ci0 + 4 kq + t][tap], t = 0..3: 4*T consecutive floats on a 16-byte
-            // boundary.  CG = 4: Wt[co][kq][tap], T consecutive floats (zero for a channel the layer does not have).
-            constexpr int NA = CG == 16 ? T : (T + 3) / 4;
-            f32x4 aw[TM][NA];
+            // A operand: Wt[co][ci0 + 4 kq + t][tap], t = 0..3: 4*T consecutive floats on a 16-byte boundary.
+            f32x4 aw[TM][T];
             Filters filters;
             if constexpr (TURNED) {
                 if (gi > 0) Filters::reads_done();             // of the patch before
@@ -173,28 +171,18 @@ struct ConvF32Rect {
 #pragma unroll
                     for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
-                        for (int j = 0; j < (CG == 16 ? T : 4 * NA); ++j) {
-                            if constexpr (CG == 16) aw[tm][j] = filters.w[tm][j];
-                            else aw[tm][j / 4][j % 4] = j < T ? filters.w[tm][j < T ? j : 0] : 0.f;
-                        }
+                        for (int j = 0; j < T; ++j) aw[tm][j] = filters.w[tm][j];
                 } else {
 #pragma unroll
                     for (int tm = 0; tm < TM; ++tm) {
-                        if constexpr (CG == 16) {
-                            const f32x4* src = reinterpret_cast<const f32x4*>(Wt + ((size_t)(co0 + tm * 16 + li) * CI + ci0 + 4 * kq) * T);
+                        const f32x4* src = reinterpret_cast<const f32x4*>(Wt + ((size_t)(co0 + tm * 16 + li) * CI + ci0 + 4 * kq) * T);
 #pragma unroll
-                            for (int j = 0; j < T; ++j) aw[tm][j] = src[j];
-                        } else {
-                            const float* src = Wt + ((size_t)(co0 + tm * 16 + li) * CI + (kq < CI ? kq : 0)) * T;
-#pragma unroll
-                            for (int j = 0; j < 4 * NA; ++j) aw[tm][j / 4][j % 4] = (j < T && kq < CI) ? src[j] : 0.f;
-                        }
+                        for (int j = 0; j < T; ++j) aw[tm][j] = src[j];
                     }
                 }
             };
 
-            // stage the patch: LPC lanes share a channel and take the (row, vector) units of its PR patch rows in turn.  A vector of a row outside the image, or of
-            // a channel that the layer does not have, is read past the buffer's end; its floats beside the image are made zeros, which is what padding reads as.  (What
+            // stage the patch: LPC lanes share a channel and take the (row, vector) units of its PR patch rows in turn.  A vector of a row outside the image is read past the buffer's end; its floats beside the image are made zeros, which is what padding reads as.  (What
             // a vector has past the buffer's end is zeros float by float; one that begins before the buffer is none at all.  So the vector that begins
             // before an image row and ends in it is read from the row's first float, and moved.)
             const int cl = lane / LPC;
@@ -202,7 +190,7 @@ struct ConvF32Rect {
             // which positions a lane stages does not change from one channel group to the next, and the compiler would
             // work out every address ahead of the loop and keep them all in registers: hidden from it
             asm volatile("" : "+v"(cu));
-            const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(X + (size_t)ci0 * HW), 0, (CG < CI ? CG : CI) * HW * 4, 0x00020000);
+            const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(X + (size_t)ci0 * HW), 0, CG * HW * 4, 0x00020000);
             const int corner = cl * HW + iy0 * W + ix0;
             const bool inside = ix0 >= 0 && ix0 + PC <= W;          // no vector reaches beside the image
             const auto begins_before = [&](int vi) { return P % 4 != 0 && ix0 < 0 && vi == P / 4; };      // (columns begin at a multiple of 16, less P)
@@ -235,43 +223,24 @@ struct ConvF32Rect {
             }
 
             // the taps: read the next tap's operands while this one multiplies
-            if constexpr (CG == 16) {
-                f32x4 b[2][PB];
+            f32x4 b[2][PB];
 #pragma unroll
-                for (int pb = 0; pb < PB; ++pb) b[0][pb] = *reinterpret_cast<const f32x4*>(bbase[pb]);
+            for (int pb = 0; pb < PB; ++pb) b[0][pb] = *reinterpret_cast<const f32x4*>(bbase[pb]);
 #pragma unroll
-                for (int tap = 0; tap < T; ++tap) {
-                    if (tap + 1 < T) {
-                        const int noff = (((tap + 1) / KW) * PC + (tap + 1) % KW) * 16;
+            for (int tap = 0; tap < T; ++tap) {
+                if (tap + 1 < T) {
+                    const int noff = (((tap + 1) / KW) * PC + (tap + 1) % KW) * 16;
 #pragma unroll
-                        for (int pb = 0; pb < PB; ++pb) b[(tap + 1) & 1][pb] = *reinterpret_cast<const f32x4*>(bbase[pb] + noff);
-                    }
-#pragma unroll
-                    for (int t = 0; t < 4; ++t)
-#pragma unroll
-                        for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-                            for (int pb = 0; pb < PB; ++pb)
-                                acc[tm][pb] = __builtin_amdgcn_mfma_f32_16x16x4f32(aw[tm][(t * T + tap) / 4][(t * T + tap) % 4],
-                                                                                   b[tap & 1][pb][t], acc[tm][pb], 0, 0, 0);
+                    for (int pb = 0; pb < PB; ++pb) b[(tap + 1) & 1][pb] = *reinterpret_cast<const f32x4*>(bbase[pb] + noff);
                 }
-            } else {
-                float b[2][PB];
 #pragma unroll
-                for (int pb = 0; pb < PB; ++pb) b[0][pb] = *reinterpret_cast<const float*>(bbase[pb]);
-#pragma unroll
-                for (int tap = 0; tap < T; ++tap) {
-                    if (tap + 1 < T) {
-                        const int noff = (((tap + 1) / KW) * PC + (tap + 1) % KW) * 16;
-#pragma unroll
-                        for (int pb = 0; pb < PB; ++pb) b[(tap + 1) & 1][pb] = *reinterpret_cast<const float*>(bbase[pb] + noff);
-                    }
+                for (int t = 0; t < 4; ++t)
 #pragma unroll
                     for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
                         for (int pb = 0; pb < PB; ++pb)
-                            acc[tm][pb] = __builtin_amdgcn_mfma_f32_16x16x4f32(aw[tm][tap / 4][tap % 4], b[tap & 1][pb], acc[tm][pb], 0, 0, 0);
-                }
+                            acc[tm][pb] = __builtin_amdgcn_mfma_f32_16x16x4f32(aw[tm][(t * T + tap) / 4][(t * T + tap) % 4],
+                                                                               b[tap & 1][pb][t], acc[tm][pb], 0, 0, 0);
             }
         }
 
@@ -381,15 +350,21 @@ struct ConvTiling {
     static constexpr int OH = (H - KH + 2 * P) / S + 1, OW = (W - KW + 2 * P) / S + 1;
     static constexpr int OHW = OH * OW;
     static constexpr bool RECT = T > 1 && (OW >= 64 || ((OW >= 44 || S > 1) && 6 * OW >= 5 * ((OW + 15) / 16 * 16)));
-    static constexpr int patch_bytes(int th) { return ((th - 1) * S + KH) * (15 * S + KW) * (CI >= 16 ? 64 : 16); }
-    // A batch of images of three or four channels: 32 output channels a wave, so that what is staged and read from the patch serves two MFMAs, where the
-    // filters leave registers for that; filters of up to 25 taps on two rows.  us, 64 images, 16 channels x 4 rows / 32 x 4 / 32 x 2: 7 x 7 on 224 216 / 179 / 200, on 113 69.6 / 64.2 / 66.4; 5 x 5 on 149
-    // 36.7 / 32.7 / 31.0; 3 x 3 on 299 at stride 2 63.4 / 64.4 / 56.8, on 150 (96 channels) 49.1 / 49.6 / 42.1, at stride 1 on 112 69 / 57.9 / 55.1, on 150 54.9 / 56.7 / 51.5.  One channel: 32.6 / 35.7 / 34.7, as it was.
-    static constexpr bool FEW = RECT && NIMG > 1 && CI >= 3 && CI < 16 && CO % 32 == 0 && T <= 52;
-    static constexpr int TH = patch_bytes(4) <= 12800 && !(FEW && T <= 25) ? 4 : patch_bytes(2) <= 12800 ? 2 : 1;
+    static constexpr int patch_bytes(int th) { return ((th - 1) * S + KH) * (15 * S + KW) * 64; }
+    static constexpr int TH = patch_bytes(4) <= 12800 ? 4 : patch_bytes(2) <= 12800 ? 2 : 1;
+    // Images of at most four channels (ConvF32Few).  A batch writes its results 64 columns wide where three quarters of these are the image's, of filters of up to 25 taps (ConvF32Few
+    // has why), on two rows; else 16 columns and eight rows of larger filters, four of smaller ones.  32 output channels a wave for up to nine taps, 16 for more.  us, 256 images, 32 channels x 2 rows x 64 columns / 16 x 2
+    // x 64 / 32 x 4 x 16: 3 x 3 on 299 at stride 2 (1024) 1065 / 1098 / 1338, on 112 181 / - / 340, 5 x 5 on 149 384 / - / 371, on 299 at stride 2 779 / 690 / 763, of one channel on 112 170 / - / 244; on 150 at stride 2, 75 of 128
+    // columns, 264 / - / 229.  7 x 7 on 224 (1024), 16 channels x 8 / 7 / 4 / 12 rows and 32 x 8 / 6 / 4: 2154 / 2154 / 2206 / 2301, 2289 / 2264 / 2509.  One image, 16 x 4 / 16 x 2 / 32 x 2 / 32 x 4: 5.7 / 5.9 / 5.9 / 8.0.
+    static constexpr bool FEW = RECT && CI <= 4;
+    static constexpr int FEW_BM = NIMG > 1 && CO % 32 == 0 && T <= 9 ? 32 : 16;
+    static constexpr int few_bytes(int th, int twb) { return CI * ((th - 1) * S + KH) * ((16 * twb - 1) * S + KW) * 4; }
+    static constexpr int FEW_TWB = NIMG > 1 && T <= 25 && 4 * OW >= 3 * ((OW + 63) / 64 * 64) && few_bytes(2, 4) <= 16384 ? 4 : 1;
+    static constexpr int FEW_TH = FEW_TWB == 4 ? 2 : NIMG > 1 && T > 25 && few_bytes(8, 1) <= 12800 ? 8 : few_bytes(4, 1) <= 25600 ? 4 : few_bytes(2, 1) <= 25600 ? 2 : 1;
+    static constexpr bool FEW_LINES = FEW_TWB == 4 && OW % 16 == 0 && (long long)NIMG * CO * OHW * 4 >= (1LL << 28);
     static constexpr int pick_bm()
     {
-        if (CI < 16) return FEW ? 32 : 16;
+        if (CI < 16) return 16;
         if (T == 1)      // a 1x1 filter is one register per row block: as many output channels as divide CO, up to 80
             for (int bm = 80; bm > 16; bm -= 16)     // (96 measured slower than 64 on the 8x8 and 17x17 layers)
                 if (CO % bm == 0) return bm;
@@ -405,8 +380,9 @@ struct ConvTiling {
     static constexpr int PB = OHW >= 64 ? 4 : (OHW + 15) / 16;
     static constexpr int NGROUP = CI >= 16 ? CI / 16 : 1;
     // (only the chosen form is instantiated: the other may not fit this shape at all)
-    static constexpr int TILE = std::conditional_t<RECT, ConvF32Rect<CI, CO, H, W, KH, KW, S, P, BM, TH, 1, NIMG>,
-                                                   ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, 1, NIMG>>::TILE_BYTES;
+    using few = ConvF32Few<CI, CO, H, W, KH, KW, S, P, FEW_BM, FEW_TH, FEW_TWB, NIMG, FEW_LINES>;
+    static constexpr int TILE = std::conditional_t<FEW, few, std::conditional_t<RECT, ConvF32Rect<CI, CO, H, W, KH, KW, S, P, BM, TH, 1, NIMG>,
+                                                                                ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, 1, NIMG>>>::TILE_BYTES;
     static constexpr int pick_ks()
     {
         // a rectangle gets no more waves than it has rows: the sum of the waves' partial tiles costs the same
@@ -429,12 +405,12 @@ struct ConvTiling {
             if (CO % bm == 0) return bm;
         return 16;
     }
-    using staged = std::conditional_t<RECT, ConvF32Rect<CI, CO, H, W, KH, KW, S, P, BM, TH, KS, NIMG>,
-                                      ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, KS, NIMG>>;
-    // A rectangle on at most four input channels (one wave, a patch of a few KB) is held to twelve workgroups per
-    // CU, three waves per SIMD: the sixteen its registers allow run the 7 x 7 on RGB 1.25x slower (LdsReserve).
-    static constexpr int RESERVE = RECT && CI < 16 && (int)sizeof(typename staged::Smem) < 163840 / 12 - 1024
-                                       ? 163840 / 12 - (int)sizeof(typename staged::Smem) : 0;
+    using staged = std::conditional_t<FEW, few, std::conditional_t<RECT, ConvF32Rect<CI, CO, H, W, KH, KW, S, P, BM, TH, KS, NIMG>,
+                                                                   ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, KS, NIMG>>>;
+    // Those that write most, one wave with a patch of a few KB, are held to eight workgroups per CU, so that fewer rows of results are written at a time
+    // (LdsReserve): 3 x 3 on 299 x 299 at stride 2 1065 -> 985 us, with six 1112; of 5 x 5 filters 714 -> 798.
+    static constexpr int RESERVE = FEW && FEW_TWB == 4 && T <= 9 && (int)sizeof(typename staged::Smem) < 163840 / 8 - 1024
+                                       ? 163840 / 8 - (int)sizeof(typename staged::Smem) : 0;
     using held = std::conditional_t<(RESERVE > 0), LdsReserve<staged, (RESERVE > 0 ? RESERVE : 1)>, staged>;
     // A batch with enough pixels for two workgroups per CU goes to the shared-tile form, with the largest tile whose
     // part of each wave is at least twelve 16 x 16 blocks: measured at batch 1024 over the 3 x 3 and 5 x 5 layers it

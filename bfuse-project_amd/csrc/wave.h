@@ -235,9 +235,8 @@ __device__ __forceinline__ T* opaque_pointer(T* p)
 // streams its operands straight into registers, and the two or three waves per SIMD their registers allow only
 // queue behind each other in the memory pipeline: with 32 KB reserved (four workgroups per CU) the 1024-fold
 // products with 64 x 64 tiles took 461 / 703 / 124 / 147 us instead of 561 / 937 / 131 / 166, and 208 x 208 x 64
-// with 208 x 32 tiles 75 us instead of 94 (24 KB, six per CU: 119; 40 KB, three per CU: 92).  The one-wave
-// convolutions on three input channels want about three waves per SIMD (the 7 x 7 on RGB at batch 1024: 3.53 ms
-// with twelve workgroups per CU, 4.43 with the sixteen its registers allow, 4.2 with six).
+// with 208 x 32 tiles 75 us instead of 94 (24 KB, six per CU: 119; 40 KB, three per CU: 92).  (ConvTiling holds
+// convolutions of few channels that write a lot to eight workgroups per CU.)
 template <class Op, int BYTES>
 struct LdsReserve : Op {
     struct Smem {

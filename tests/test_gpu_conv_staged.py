@@ -1,7 +1,8 @@
-"""The convolutions whose waves stage a patch of their own (csrc/ops_conv.h, ops_conv_general.h, ops_conv_rect.h) and take their filters through
+"""The convolutions whose waves stage a patch of their own (csrc/ops_conv.h, ops_conv_general.h, ops_conv_rect.h, ops_conv_few.h) and take their filters through
 LDS (ops_conv_filters.h), at the edges of images, vectors, row blocks and groups, against the oracle; three of them fused, bit for bit."""
 import numpy as np
 import pytest
+import torch
 
 import bfuse_project_amd as bf
 from bfuse_project_amd.operation import fill_normal
@@ -12,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 FORMS = [("a", 1, 2, "bias_relu_4096", "hfuse", ""), ("b", 1, 1, "bias_relu_4096", None, ""), ("c", 2, 1, "bias_relu_4096", None, ""), ("d", 1, 5, "bias_relu_4096", None, ""),
          ("e", 1, 0, "bias_relu_4096", None, ""), ("f", 2, 3, "bias_relu_4096", None, ""), ("g", 1, 1, "layernorm_8x256", "bfuse", "_c4"), ("h", 2, 1, "bias_relu_4096", None, ""),
-         ("i", 1, 2, "bias_relu_4096", None, ""), ("j", 1, 1, "bias_relu_4096", None, ""), ("k", 1, 1, "bias_relu_4096", None, ""), ("l", 1, 1, "bias_relu_4096", "hfuse", "")]
+         ("i", 1, 2, "bias_relu_4096", None, ""), ("j", 1, 1, "bias_relu_4096", None, ""), ("k", 1, 1, "bias_relu_4096", None, ""), ("l", 1, 1, "bias_relu_4096", "hfuse", ""),
+         ("m", 1, 0, "bias_relu_4096", "hfuse", ""), ("n", 2, 2, "bias_relu_4096", None, ""), ("o", 1, 1, "bias_relu_4096", None, ""), ("p", 2, 3, "bias_relu_4096", None, "")]
 
 
 @pytest.mark.parametrize("tag,s,p,partner,kind,suffix", FORMS)
@@ -31,3 +33,20 @@ def test_staged_convolution_copies_what_a_selector_names(tag, s, p):
         w[c, (5 * c + 1) % ci, (3 * c) % kh, (2 * c + c // kh) % kw] = 1
         y = op.run_kernel(0, x, w.ravel())
     assert np.array_equal(y.ravel(), orf.conv2d(x.reshape(k.shapes[0]), w, s=s, p=p).ravel())
+
+
+@pytest.mark.parametrize("tag,s,p", [f[:3] for f in FORMS if f[0] in "acdfmnop"])
+def test_a_value_that_is_not_finite_is_in_its_own_windows_alone(tag, s, p):
+    """Four k of an MFMA are rows or taps of a window: those that there are not have no part in it, whatever lies in their place."""
+    name = f"selftest_conv_staged_{tag}"
+    with bf.Operation(name, "bias_relu_4096") as op:
+        k = op.k[0]
+        x, w = (fill_normal(8 + i, int(np.prod(k.shapes[i])), 0, 1).reshape(k.shapes[i]) for i in (0, 1))
+        w = np.abs(w) + np.float32(0.5)
+        x[0, 0, 2, 3], x[-1, -1, -1, -1], x[0, -1, 5, 9] = np.inf, np.nan, -np.inf
+        y = op.run_kernel(0, x, w).reshape(k.shapes[2])
+    with np.errstate(all="ignore"):
+        want = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(w).double(), stride=s, padding=p).numpy()
+    assert np.array_equal(np.isnan(y), np.isnan(want)) and np.array_equal(np.isposinf(y), np.isposinf(want)) and np.array_equal(np.isneginf(y), np.isneginf(want))
+    ok = np.isfinite(want)
+    assert ok.any() and np.linalg.norm(y[ok] - want[ok]) <= 1e-5 * np.linalg.norm(want[ok])
