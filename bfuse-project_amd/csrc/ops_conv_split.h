@@ -291,7 +291,7 @@ struct ConvSplit {
             return y < Form::OH && x < OW;
         };
         if constexpr (TW > 0) {
-            Form::template finish<OW % 4 == 0>(acc, sm.inexact != 0, A, B, static_cast<float*>(O), m0, mt, n0, nt, n_lo, wr, wn, el & 15, el >> 4,
+            Form::template finish<OW % 4 == 0, false>(acc, sm.inexact != 0, A, B, static_cast<float*>(O), m0, mt, n0, nt, n_lo, wr, wn, el & 15, el >> 4,
                 [&](int c, unsigned& outside) {
                     int y, x;
                     const bool in = rectangle(c, y, x);

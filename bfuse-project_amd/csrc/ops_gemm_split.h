@@ -162,6 +162,12 @@ struct GemmSplit {
     static constexpr bool LOOP_BARRIERS = true;
     static constexpr int MIN_BARRIERS = NIT;
     static constexpr int RED_BYTES = (KG - 1) * BM * BN * 4;                     // partial sums of the groups
+    // Results that are more than the last-level cache holds (256 MB) and lie in whole lines (two blocks of columns): every line is written at once and past the caches.
+    // Otherwise a store is 64 bytes of sixteen rows, and the results take the place of everything else in the caches.  us, launched again and again / in turn with a layer of 900 MB: 1024 products
+    // 512 x 64 x 512 296 -> 256 / 295 -> 281, 1024 x 64 x 512 588 -> 565 / 587 -> 568, 512 x 128 x 512 453 -> 450 / 459 -> 451, 256 -> 256 channels on 56 x 56 2438 -> 2377 / 2436 -> 2374; 256 x 80 x 256 (268 MB) 105 -> 86 /
+    // 99.5 -> 100.2, 256 x 64 x 256 83 -> 68 / 76.7 -> 77.3: there it is the operands, 134 - 168 MB, that stay in the last-level cache.  Whole lines through the caches gain 0-1 %, 64 bytes past them lose up to 5 %
+    // (512 x 128 x 512).  Smaller results stay in that cache for what reads them (256 x 256 x 64, 67 MB, launched again and again would take 75 us for 81).
+    static constexpr bool LINES_ = TN % 2 == 0 && M % BM == 0 && (LAYOUT == kRows ? W % BN == 0 && W % 32 == 0 : OHW % 32 == 0) && (long long)NIMG * M * (LAYOUT == kRows ? W : OHW) * 4 >= (1LL << 28);
 
     struct Smem {
         __attribute__((aligned(16))) unsigned char t[NBUF * KG * BUF > RED_BYTES ? NBUF * KG * BUF : RED_BYTES];
@@ -493,9 +499,12 @@ struct GemmSplit {
         return img >= NIMG ? 0 : OHW - p < 4 ? OHW - p : 4;
     }
 
+    // Lane (i, q) of 16 gets lane (i ^ 8, q)'s.
+    __device__ static __forceinline__ float swap_halves(float v) { return dpp_mov<0x128>(v); }      // row_ror:8
+
     // What follows the sums of a wave: the results that three parts do not give are done again, and all are stored.
-    // offset(c, outside): as offset_of, for column c of the tile; quad(c, img, p): as quad_at; QUADS: four columns are one image's and aligned.
-    template <bool QUADS = OHW % 4 == 0, class Offset, class Quad>
+    // offset(c, outside): as offset_of, for column c of the tile; quad(c, img, p): as quad_at; QUADS: four columns are one image's and aligned; LINES: as LINES_.
+    template <bool QUADS = OHW % 4 == 0, bool LINES = LINES_, class Offset, class Quad>
     __device__ static __forceinline__ void finish(f32x4 (&acc)[TM][TN], bool again, const float* A, const float* B, float* __restrict__ C, int m0, int mt, long long n0, int nt, int n_lo,
                                                   int wr, int wn, int ei, int eq, Offset offset, Quad quad)
     {
@@ -605,6 +614,30 @@ struct GemmSplit {
                 if (redo[tm])
 #pragma unroll
                     for (int b = 0; b < TN; ++b) acc[tm][b] = re[tm][b];
+        }
+        if constexpr (LINES) {
+            // Two blocks of columns and of eight rows at a time: lanes of rows 8 .. 15 have the second block's columns of the first rows and the other way round, so that
+            // eight lanes write a line.
+#pragma unroll
+            for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+                for (int b = 0; b < TN; b += 2) {
+                    f32x4 o[2];
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const float x = ei < 8 ? acc[tm][b + 1][v] : acc[tm][b][v], y = swap_halves(x);
+                        o[0][v] = ei < 8 ? acc[tm][b][v] : y;
+                        o[1][v] = ei < 8 ? y : acc[tm][b + 1][v];
+                    }
+                    const int row = m0 + (wr * TM + tm) * 16 + (ei & 7), col = (wn * TN + b + (ei >> 3)) * 16 + 4 * eq;
+                    int img = 0, p = 0;
+                    if (LAYOUT == kRows || quad(col, img, p) > 0) {
+                        float* const d = LAYOUT == kRows ? C + (size_t)row * W + n0 + col : C + ((size_t)img * M + row) * OHW + p;
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) __builtin_nontemporal_store(o[h], reinterpret_cast<f32x4*>(d + (size_t)(8 * h) * (LAYOUT == kRows ? W : OHW)));
+                    }
+                }
+            return;
         }
         // lane (i, q): row i of a 16-row block, columns 4q .. 4q + 3 of each 16-column block
         const auto own_row = [&](int m) { return M % BM == 0 || m >= mt * BM; };
