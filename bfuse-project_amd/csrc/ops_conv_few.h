@@ -168,7 +168,7 @@ struct ConvF32Few {
                 }
         }
         // lane (j = column of the tile row, rg) owns output channels 4 rg + v of a block
-                typedef float cols __attribute__((ext_vector_type(TWB), aligned(4)));
+        typedef float cols __attribute__((ext_vector_type(TWB), aligned(4)));
         const int ox = ox0 + li * TWB;
 #pragma unroll
         for (int tm = 0; tm < TM; ++tm)
