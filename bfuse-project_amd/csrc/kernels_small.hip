@@ -214,6 +214,9 @@ CONV_STAGED_TEST(m, 2, 3, 11, 131, 32, 3, 3, 1, 0, ConvF32Few<3, 32, 11, 131, 3,
 CONV_STAGED_TEST(n, 2, 1, 13, 150, 16, 5, 5, 2, 2, ConvF32Few<1, 16, 13, 150, 5, 5, 2, 2, 16, 2, 4, 2>)            // one channel: a row a lane group and five taps of one that is left; cut after three
 CONV_STAGED_TEST(o, 2, 2, 12, 80, 32, 3, 3, 1, 1, ConvF32Few<2, 32, 12, 80, 3, 3, 1, 1, 32, 2, 4, 2, true>)        // two rows left, six taps; written past the caches
 CONV_STAGED_TEST(p, 1, 3, 40, 66, 16, 7, 7, 2, 3, ConvF32Few<3, 16, 40, 66, 7, 7, 2, 3, 16, 8, 1, 1>)              // eight rows
+CONV_STAGED_TEST(q, 2, 4, 20, 64, 16, 14, 14, 1, 7, ConvF32Auto<4, 16, 20, 64, 14, 14, 1, 7, 2>)                   // filters that take most of the registers
+CONV_STAGED_TEST(r, 2, 4, 18, 64, 16, 13, 13, 1, 6, ConvF32Auto<4, 16, 18, 64, 13, 13, 1, 6, 2>)
+CONV_STAGED_TEST(s, 3, 2, 16, 66, 32, 6, 6, 1, 3, ConvF32Auto<2, 32, 16, 66, 6, 6, 1, 3, 3>)                       // half a channel's rows a lane group
 BFUSE_HFUSE_KERNEL(selftest_conv_staged_m, ConvW_m, bias_relu_4096, BiasReluS)
 BFUSE_HFUSE_KERNEL(selftest_conv_staged_a, ConvW_a, bias_relu_4096, BiasReluS)
 BFUSE_BFUSE_KERNEL(selftest_conv_staged_g, ConvW_g, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)

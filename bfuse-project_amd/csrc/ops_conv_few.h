@@ -133,18 +133,20 @@ struct ConvF32Few {
         }
 
         // Where this lane's rows of the window begin for its column, and its taps of the rows that are left.
-        const unsigned char* row[RPL > 0 ? RPL : 1];
+        // (A quarter that stays in one channel has its rows one after the other, a constant apart.)
+        constexpr bool RUN = RPL > 0 && KH % (RPL > 0 ? RPL : 1) == 0;
+        const unsigned char* row[RPL > 0 && !RUN ? RPL : 1];
         const unsigned char* last[NLT > 0 ? NLT : 1];
         const auto at = [&](int r, int kw) { return tile + ((r / KH * PR + r % KH) * PC + kw + li * S * TWB) * 4; };
 #pragma unroll
-        for (int r = 0; r < RPL; ++r) row[r] = at(kq * RPL + r, 0);
+        for (int r = 0; r < (RUN ? 1 : RPL); ++r) row[r] = at(kq * RPL + r, 0);
 #pragma unroll
         for (int i = 0; i < NLT; ++i) {
             const int t = 4 * i + kq < LEFT ? 4 * i + kq : 0;
             last[i] = at(4 * RPL + t / KW, t % KW);
         }
         auto value = [&](int m, int pb) {
-            const unsigned char* const from = m < RPL * KW ? row[m / KW < RPL ? m / KW : 0] + m % KW * 4 : last[m - RPL * KW >= 0 ? m - RPL * KW : 0];
+            const unsigned char* const from = m < RPL * KW ? row[RUN || m / KW >= RPL ? 0 : m / KW] + ((RUN ? m / KW * PC : 0) + m % KW) * 4 : last[m - RPL * KW >= 0 ? m - RPL * KW : 0];
             const float f = *reinterpret_cast<const float*>(from + (pb / TWB * PC + pb % TWB) * S * 4);
             return m == NM - 1 && LEFT % 4 != 0 && kq >= LEFT % 4 ? 0.f : f;
         };

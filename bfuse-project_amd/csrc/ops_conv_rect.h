@@ -360,7 +360,11 @@ struct ConvTiling {
     static constexpr int FEW_BM = NIMG > 1 && CO % 32 == 0 && T <= 9 ? 32 : 16;
     static constexpr int few_bytes(int th, int twb) { return CI * ((th - 1) * S + KH) * ((16 * twb - 1) * S + KW) * 4; }
     static constexpr int FEW_TWB = NIMG > 1 && T <= 25 && 4 * OW >= 3 * ((OW + 63) / 64 * 64) && few_bytes(2, 4) <= 16384 ? 4 : 1;
-    static constexpr int FEW_TH = FEW_TWB == 4 ? 2 : NIMG > 1 && T > 25 && few_bytes(8, 1) <= 12800 ? 8 : few_bytes(4, 1) <= 25600 ? 4 : few_bytes(2, 1) <= 25600 ? 2 : 1;
+    // Filters of many taps leave registers for fewer rows: eight with 144 of them spill 210, four with 196 do not fit 256.  us before (four rows of ConvF32Rect) and now, 64 images of four channels, 96 wide,
+    // to 32: 12 x 12 221 -> 212, 13 x 13 204 -> 204, 9 x 9 108 -> 103, 14 x 14 289 -> 287; of two, 12 x 12 293 -> 135, of three 337 -> 154; 11 x 11 at stride 4 on 224, three channels to 64, 426 -> 118.
+    static constexpr int FEW_NM = FilterFloats<(CI <= 4 ? CI : 4), KH, KW, 1>::NM, FEW_MOST = FEW_NM <= 64 ? 8 : FEW_NM <= 176 ? 4 : FEW_NM <= 200 ? 3 : 1;
+    static constexpr int few_rows(int th) { return th > FEW_MOST ? FEW_MOST : th; }
+    static constexpr int FEW_TH = FEW_TWB == 4 ? 2 : few_rows(NIMG > 1 && T > 25 && few_bytes(8, 1) <= 12800 ? 8 : few_bytes(4, 1) <= 25600 ? 4 : few_bytes(2, 1) <= 25600 ? 2 : 1);
     static constexpr bool FEW_LINES = FEW_TWB == 4 && OW % 16 == 0 && (long long)NIMG * CO * OHW * 4 >= (1LL << 28);
     static constexpr int pick_bm()
     {
