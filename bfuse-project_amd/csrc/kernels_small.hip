@@ -217,6 +217,11 @@ CONV_STAGED_TEST(p, 1, 3, 40, 66, 16, 7, 7, 2, 3, ConvF32Few<3, 16, 40, 66, 7, 7
 CONV_STAGED_TEST(q, 2, 4, 20, 64, 16, 14, 14, 1, 7, ConvF32Auto<4, 16, 20, 64, 14, 14, 1, 7, 2>)                   // filters that take most of the registers
 CONV_STAGED_TEST(r, 2, 4, 18, 64, 16, 13, 13, 1, 6, ConvF32Auto<4, 16, 18, 64, 13, 13, 1, 6, 2>)
 CONV_STAGED_TEST(s, 3, 2, 16, 66, 32, 6, 6, 1, 3, ConvF32Auto<2, 32, 16, 66, 6, 6, 1, 3, 3>)                       // half a channel's rows a lane group
+// More loads than are under way at a time, the last batch of them shorter than the others though every lane has a unit in each (25 loads, 16 at a time).
+CONV_STAGED_TEST(t, 2, 32, 15, 170, 16, 5, 5, 5, 0, ConvF32Rect<32, 16, 15, 170, 5, 5, 5, 0, 16, 1, 2, 2>)         // a second wave's tile behind the patch
+CONV_STAGED_TEST(u, 1, 32, 15, 165, 16, 5, 5, 5, 2, ConvF32Rect<32, 16, 15, 165, 5, 5, 5, 2, 16, 1, 1, 1>)         // a partner's behind it, and a second group's; unrolled
+BFUSE_HFUSE_KERNEL(selftest_conv_staged_t, ConvW_t, bias_relu_4096, BiasReluS)
+BFUSE_HFUSE_KERNEL(selftest_conv_staged_u, ConvW_u, conv3x3_f32_32x12x12_32, ConvS2)
 BFUSE_HFUSE_KERNEL(selftest_conv_staged_m, ConvW_m, bias_relu_4096, BiasReluS)
 BFUSE_HFUSE_KERNEL(selftest_conv_staged_a, ConvW_a, bias_relu_4096, BiasReluS)
 BFUSE_BFUSE_KERNEL(selftest_conv_staged_g, ConvW_g, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)

@@ -29,6 +29,7 @@
 #include "ops_conv_1x1.h"
 #include "ops_conv_few.h"
 #include "ops_conv_general.h"
+#include "ops_conv_patch.h"
 #include "ops_conv_split.h"
 #include "ops_conv_tile.h"
 #include "ops_gemm_split.h"
@@ -63,7 +64,8 @@ struct ConvF32Rect {
     static constexpr int LPC = 64 / CG;                 // lanes that share a channel while staging
     static constexpr int NVR = PC / 4;                  // vectors of a patch row
     static constexpr int NU = PR * NVR;                 // staging units (row, vector) per channel
-    static constexpr int NLD = (NU + LPC - 1) / LPC;    // wave-level loads per group
+    using Units = PatchUnits<NU, LPC>;
+    static constexpr int NLD = Units::NLD;              // wave-level loads per group
     static_assert(CI % 16 == 0, "input channels: a multiple of 16");
     static_assert(CO % BM == 0 && BM % 16 == 0 && NGROUP % KS == 0, "channel tiling");
     static_assert(((KH - 1) * PC + KW - 1) * 16 + (NQ - 1) * PLANE + 16 < 65536, "tap offsets are 16-bit immediates");
@@ -195,8 +197,7 @@ struct ConvF32Rect {
             const bool inside = ix0 >= 0 && ix0 + PC <= W;          // no vector reaches beside the image
             const auto begins_before = [&](int vi) { return P % 4 != 0 && ix0 < 0 && vi == P / 4; };      // (columns begin at a multiple of 16, less P)
             unsigned char* const plane = tile + (cl / 4) * PLANE + (cl % 4) * 4;
-            constexpr int JB = NLD < 16 ? NLD : 16;
-            constexpr int NBATCH = (NLD + JB - 1) / JB, UNROLL = (NIMG == 1 && NBATCH <= 4) ? NBATCH : 1;
+            constexpr int JB = Units::JB, NBATCH = Units::NBATCH, UNROLL = (NIMG == 1 && NBATCH <= 4) ? NBATCH : 1;
             if constexpr (NBATCH > 1 || !TURNED) take_filters(std::integral_constant<int, 0>{});
 #pragma unroll UNROLL
             for (int j0 = 0; j0 < NLD; j0 += JB) {
@@ -214,7 +215,7 @@ struct ConvF32Rect {
                     const int u = (j0 + jj) * LPC + cu;
                     const int vi = u % NVR, x = ix0 + 4 * vi;
                     const bool moved = begins_before(vi);
-                    if (NU % LPC == 0 || u < NU) {
+                    if (Units::there(j0 + jj, u)) {
                         float* const dst = reinterpret_cast<float*>(plane + u * 64);
 #pragma unroll
                         for (int e = 0; e < 4; ++e) dst[4 * e] = inside || (unsigned)(x + e) < (unsigned)W ? moved && e >= P % 4 ? v[jj][e - P % 4 >= 0 ? e - P % 4 : 0] : v[jj][e] : 0.f;

@@ -130,3 +130,28 @@ def test_output_channels_that_no_tall_tile_divides_are_as_without_patches(tmp_pa
     for ci, co, hw, split in [(32, 32, 149, "false"), (32, 160, 28, "true"), (32, 224, 28, "false"), (32, 352, 28, "false"), (64, 160, 14, "true")]:
         text += f"static_assert(ConvTiling<{ci}, {co}, {hw}, {hw}, 3, 3, 1, 0, 1024>::patch_form() == 0 && ConvTiling<{ci}, {co}, {hw}, {hw}, 3, 3, 1, 0, 1024>::is_split() == {split});\n"
     _compiles(text, tmp_path)
+
+
+UNITS = """
+        template <class C> constexpr bool units_are_right()
+        {
+            int stored = 0;
+            for (int j = 0; j < C::Units::NBATCH * C::Units::JB; ++j)
+                for (int lane = 0; lane < LANES; ++lane) {
+                    const int u = j * LANES + lane;
+                    if (C::Units::there(j, u) != (u < C::NU)) return false;
+                    stored += C::Units::there(j, u);
+                }
+            return stored == C::NU;
+        }
+"""
+
+
+def test_a_rectangle_stores_the_units_of_its_patch_and_no_others(tmp_path):
+    """... also where the last batch of loads is shorter than the others: what it would store lies in the next plane, and behind the last one in a neighbour's LDS."""
+    text = UNITS.replace("LANES", "4")
+    for ci, h, w, kh, kw, s, p in [(16, 160, 160, 5, 5, 5, 0), (16, 160, 160, 4, 4, 5, 0), (16, 160, 160, 4, 4, 6, 1), (16, 224, 224, 4, 4, 7, 0), (32, 192, 192, 6, 6, 6, 0), (16, 224, 224, 7, 7, 7, 0), (16, 90, 130, 5, 3, 3, 1),
+                                   (64, 56, 56, 3, 3, 1, 1), (16, 227, 227, 3, 3, 4, 1), (16, 128, 128, 7, 5, 2, 3)]:
+        for n in (1, 8):
+            text += f"static_assert(units_are_right<ConvTiling<{ci}, 16, {h}, {w}, {kh}, {kw}, {s}, {p}, {n}>::staged>());\n"
+    _compiles(text, tmp_path)

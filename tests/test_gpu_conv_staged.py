@@ -15,7 +15,8 @@ FORMS = [("a", 1, 2, "bias_relu_4096", "hfuse", ""), ("b", 1, 1, "bias_relu_4096
          ("e", 1, 0, "bias_relu_4096", None, ""), ("f", 2, 3, "bias_relu_4096", None, ""), ("g", 1, 1, "layernorm_8x256", "bfuse", "_c4"), ("h", 2, 1, "bias_relu_4096", None, ""),
          ("i", 1, 2, "bias_relu_4096", None, ""), ("j", 1, 1, "bias_relu_4096", None, ""), ("k", 1, 1, "bias_relu_4096", None, ""), ("l", 1, 1, "bias_relu_4096", "hfuse", ""),
          ("m", 1, 0, "bias_relu_4096", "hfuse", ""), ("n", 2, 2, "bias_relu_4096", None, ""), ("o", 1, 1, "bias_relu_4096", None, ""), ("p", 2, 3, "bias_relu_4096", None, ""),
-         ("q", 1, 7, "bias_relu_4096", None, ""), ("r", 1, 6, "bias_relu_4096", None, ""), ("s", 1, 3, "bias_relu_4096", None, "")]
+         ("q", 1, 7, "bias_relu_4096", None, ""), ("r", 1, 6, "bias_relu_4096", None, ""), ("s", 1, 3, "bias_relu_4096", None, ""),
+         ("t", 5, 0, "bias_relu_4096", "hfuse", ""), ("u", 5, 2, "conv3x3_f32_32x12x12_32", "hfuse", "")]
 
 
 @pytest.mark.parametrize("tag,s,p,partner,kind,suffix", FORMS)
