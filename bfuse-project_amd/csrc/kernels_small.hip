@@ -220,6 +220,9 @@ CONV_STAGED_TEST(s, 3, 2, 16, 66, 32, 6, 6, 1, 3, ConvF32Auto<2, 32, 16, 66, 6, 
 // More loads than are under way at a time, the last batch of them shorter than the others though every lane has a unit in each (25 loads, 16 at a time).
 CONV_STAGED_TEST(t, 2, 32, 15, 170, 16, 5, 5, 5, 0, ConvF32Rect<32, 16, 15, 170, 5, 5, 5, 0, 16, 1, 2, 2>)         // a second wave's tile behind the patch
 CONV_STAGED_TEST(u, 1, 32, 15, 165, 16, 5, 5, 5, 2, ConvF32Rect<32, 16, 15, 165, 5, 5, 5, 2, 16, 1, 1, 1>)         // a partner's behind it, and a second group's; unrolled
+CONV_STAGED_TEST(v, 2, 3, 40, 264, 16, 8, 8, 8, 0, ConvF32Few<3, 16, 40, 264, 8, 8, 8, 0, 16, 2, 1, 2>)            // 24 loads, 16 at a time
+CONV_STAGED_TEST(w, 2, 3, 21, 281, 32, 4, 4, 4, 1, ConvF32Few<3, 32, 21, 281, 4, 4, 4, 1, 32, 2, 4, 2>)             // the same with four columns a lane, 70 of 128
+BFUSE_HFUSE_KERNEL(selftest_conv_staged_v, ConvW_v, conv3x3_f32_32x12x12_32, ConvS2)
 BFUSE_HFUSE_KERNEL(selftest_conv_staged_t, ConvW_t, bias_relu_4096, BiasReluS)
 BFUSE_HFUSE_KERNEL(selftest_conv_staged_u, ConvW_u, conv3x3_f32_32x12x12_32, ConvS2)
 BFUSE_HFUSE_KERNEL(selftest_conv_staged_m, ConvW_m, bias_relu_4096, BiasReluS)

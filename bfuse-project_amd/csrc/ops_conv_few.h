@@ -20,6 +20,7 @@
 
 #include "dispatch.h"
 #include "ops_conv_filters.h"
+#include "ops_conv_patch.h"
 #include "wave.h"
 
 namespace bfuse {
@@ -44,7 +45,8 @@ struct ConvF32Few {
     static constexpr int TILE_BYTES = TURNED && Filters::BYTES > PATCH_BYTES ? Filters::BYTES : PATCH_BYTES;
     static constexpr int NVR = PC / 4;                  // vectors of a patch row
     static constexpr int NU = CI * PR * NVR;            // staging units (channel, row, vector)
-    static constexpr int NLD = (NU + 63) / 64;          // wave-level loads
+    using Units = PatchUnits<NU, 64>;
+    static constexpr int NLD = Units::NLD;              // wave-level loads
     static_assert(CI >= 1 && CI <= 4 && CO % BM == 0 && BM % 16 == 0, "channels");
     static_assert(S >= 1 && OH >= 1 && OW >= 1 && TH >= 1 && (PR * PC + KW) * 4 < 65536, "shape; offsets of rows and taps are 16-bit immediates");
 
@@ -103,7 +105,7 @@ struct ConvF32Few {
         const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)X, 0, CI * HW * 4, 0x00020000);
         const bool inside = ix0 >= 0 && ix0 + PC <= W;          // no vector reaches beside the image
         const auto begins_before = [&](int vi) { return P % 4 != 0 && ix0 < 0 && vi == P / 4; };      // (columns begin at a multiple of 16, less P)
-        constexpr int JB = NLD < 16 ? NLD : 16;
+        constexpr int JB = Units::JB;
         if constexpr (!TURNED) filters.load(Wt, co0, lane);
         else if constexpr (NLD > JB) filters.take(Wt, co0, tile, lane);
 #pragma unroll 1
@@ -128,7 +130,7 @@ struct ConvF32Few {
 #pragma unroll
             for (int jj = 0; jj < JB; ++jj) {
                 const int u = (j0 + jj) * 64 + lane;
-                if (NU % 64 == 0 || u < NU) *reinterpret_cast<f32x4*>(tile + u * 16) = v[jj];
+                if (Units::there(j0 + jj, u)) *reinterpret_cast<f32x4*>(tile + u * 16) = v[jj];
             }
         }
 

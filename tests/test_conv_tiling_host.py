@@ -155,3 +155,11 @@ def test_a_rectangle_stores_the_units_of_its_patch_and_no_others(tmp_path):
         for n in (1, 8):
             text += f"static_assert(units_are_right<ConvTiling<{ci}, 16, {h}, {w}, {kh}, {kw}, {s}, {p}, {n}>::staged>());\n"
     _compiles(text, tmp_path)
+
+
+def test_a_patch_of_few_channels_stores_its_units_and_no_others(tmp_path):
+    text = UNITS.replace("LANES", "64")
+    for ci, h, w, k, s, p in [(3, 224, 224, 8, 8, 0), (3, 224, 224, 16, 16, 0), (4, 224, 224, 8, 8, 0), (1, 448, 448, 16, 16, 0), (3, 224, 224, 7, 2, 3), (3, 299, 299, 3, 2, 0), (2, 448, 448, 12, 8, 2), (4, 300, 300, 6, 4, 1)]:
+        for n in (1, 8):
+            text += f"static_assert(units_are_right<ConvTiling<{ci}, 32, {h}, {w}, {k}, {k}, {s}, {p}, {n}>::staged>());\n"
+    _compiles(text, tmp_path)
