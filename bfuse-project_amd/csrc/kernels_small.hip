@@ -217,6 +217,11 @@ CONV_STAGED_TEST(p, 1, 3, 40, 66, 16, 7, 7, 2, 3, ConvF32Few<3, 16, 40, 66, 7, 7
 CONV_STAGED_TEST(q, 2, 4, 20, 64, 16, 14, 14, 1, 7, ConvF32Auto<4, 16, 20, 64, 14, 14, 1, 7, 2>)                   // filters that take most of the registers
 CONV_STAGED_TEST(r, 2, 4, 18, 64, 16, 13, 13, 1, 6, ConvF32Auto<4, 16, 18, 64, 13, 13, 1, 6, 2>)
 CONV_STAGED_TEST(s, 3, 2, 16, 66, 32, 6, 6, 1, 3, ConvF32Auto<2, 32, 16, 66, 6, 6, 1, 3, 3>)                       // half a channel's rows a lane group
+// Padding that is wider than a tile: a second and a third tile of a row begin before column 0, inside another vector of theirs.
+CONV_STAGED_TEST(x, 2, 16, 7, 62, 16, 3, 3, 1, 17, ConvF32Rect<16, 16, 7, 62, 3, 3, 1, 17, 16, 2, 1, 2>)
+CONV_STAGED_TEST(y, 1, 16, 5, 70, 32, 3, 3, 1, 35, ConvF32Rect<16, 32, 5, 70, 3, 3, 1, 35, 32, 4, 1, 1>)
+CONV_STAGED_TEST(z, 2, 3, 9, 61, 16, 3, 3, 1, 18, ConvF32Few<3, 16, 9, 61, 3, 3, 1, 18, 16, 4, 1, 2>)
+CONV_STAGED_TEST(aa, 1, 4, 12, 64, 32, 3, 3, 1, 67, ConvF32Few<4, 32, 12, 64, 3, 3, 1, 67, 32, 2, 4, 1>)
 // More loads than are under way at a time, the last batch of them shorter than the others though every lane has a unit in each (25 loads, 16 at a time).
 CONV_STAGED_TEST(t, 2, 32, 15, 170, 16, 5, 5, 5, 0, ConvF32Rect<32, 16, 15, 170, 5, 5, 5, 0, 16, 1, 2, 2>)         // a second wave's tile behind the patch
 CONV_STAGED_TEST(u, 1, 32, 15, 165, 16, 5, 5, 5, 2, ConvF32Rect<32, 16, 15, 165, 5, 5, 5, 2, 16, 1, 1, 1>)         // a partner's behind it, and a second group's; unrolled

@@ -46,6 +46,7 @@ struct ConvF32Few {
     static constexpr int NVR = PC / 4;                  // vectors of a patch row
     static constexpr int NU = CI * PR * NVR;            // staging units (channel, row, vector)
     using Units = PatchUnits<NU, 64>;
+    using Columns = PatchColumns<W, P, 16 * TWB * S>;
     static constexpr int NLD = Units::NLD;              // wave-level loads
     static_assert(CI >= 1 && CI <= 4 && CO % BM == 0 && BM % 16 == 0, "channels");
     static_assert(S >= 1 && OH >= 1 && OW >= 1 && TH >= 1 && (PR * PC + KW) * 4 < 65536, "shape; offsets of rows and taps are 16-bit immediates");
@@ -100,11 +101,9 @@ struct ConvF32Few {
         if constexpr (TURNED) Filters::request(Wt, co0, 0, tile, lane);
 
         // Stage the patch, [channel][row][PC floats]: the lanes take its vectors in turn, which follow each other in LDS.  A vector of a row outside the image is
-        // read past the buffer's end; floats beside the image are made zeros.  (What a vector has past the buffer's end is zeros float by float; one that
-        // begins before the buffer is none at all.  So the vector that begins before an image row and ends in it is read from the row's first float, and moved.)
+        // read past the buffer's end; floats beside the image are made zeros (PatchColumns).
         const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)X, 0, CI * HW * 4, 0x00020000);
         const bool inside = ix0 >= 0 && ix0 + PC <= W;          // no vector reaches beside the image
-        const auto begins_before = [&](int vi) { return P % 4 != 0 && ix0 < 0 && vi == P / 4; };      // (columns begin at a multiple of 16, less P)
         constexpr int JB = Units::JB;
         if constexpr (!TURNED) filters.load(Wt, co0, lane);
         else if constexpr (NLD > JB) filters.take(Wt, co0, tile, lane);
@@ -114,17 +113,16 @@ struct ConvF32Few {
 #pragma unroll
             for (int jj = 0; jj < JB; ++jj) {
                 const int u = (j0 + jj) * 64 + lane, r = u / NVR, vi = u % NVR, c = r / PR, iy = iy0 + r - c * PR;
-                v[jj] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, iy >= 0 && iy < H && u < NU ? (unsigned)((c * HW + iy * W + ix0 + 4 * vi + (begins_before(vi) ? P % 4 : 0)) * 4) : 0x7fffffffu, 0, 0));
+                v[jj] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, iy >= 0 && iy < H && u < NU ? (unsigned)((c * HW + iy * W + Columns::from(ix0, vi)) * 4) : 0x7fffffffu, 0, 0));
             }
             if constexpr (NLD <= JB && TURNED) filters.take(Wt, co0, tile, lane);
             if (!inside) {
 #pragma unroll
                 for (int jj = 0; jj < JB; ++jj) {
-                    const int u = (j0 + jj) * 64 + lane, vi = u % NVR, x = ix0 + 4 * vi;
-                    const bool moved = begins_before(vi);
+                    const int u = (j0 + jj) * 64 + lane;
                     const f32x4 f = v[jj];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) v[jj][e] = (unsigned)(x + e) < (unsigned)W ? moved && e >= P % 4 ? f[e - P % 4 >= 0 ? e - P % 4 : 0] : f[e] : 0.f;
+                    for (int e = 0; e < 4; ++e) v[jj][e] = Columns::at(f, e, ix0, u % NVR, false);
                 }
             }
 #pragma unroll

@@ -65,6 +65,7 @@ struct ConvF32Rect {
     static constexpr int NVR = PC / 4;                  // vectors of a patch row
     static constexpr int NU = PR * NVR;                 // staging units (row, vector) per channel
     using Units = PatchUnits<NU, LPC>;
+    using Columns = PatchColumns<W, P, 16 * S>;
     static constexpr int NLD = Units::NLD;              // wave-level loads per group
     static_assert(CI % 16 == 0, "input channels: a multiple of 16");
     static_assert(CO % BM == 0 && BM % 16 == 0 && NGROUP % KS == 0, "channel tiling");
@@ -184,18 +185,16 @@ struct ConvF32Rect {
                 }
             };
 
-            // stage the patch: LPC lanes share a channel and take the (row, vector) units of its PR patch rows in turn.  A vector of a row outside the image is read past the buffer's end; its floats beside the image are made zeros, which is what padding reads as.  (What
-            // a vector has past the buffer's end is zeros float by float; one that begins before the buffer is none at all.  So the vector that begins
-            // before an image row and ends in it is read from the row's first float, and moved.)
+            // stage the patch: LPC lanes share a channel and take the (row, vector) units of its PR patch rows in turn.  A vector of a row outside the image
+            // is read past the buffer's end; floats beside the image are made zeros, which is what padding reads as (PatchColumns).
             const int cl = lane / LPC;
             int cu = lane % LPC;
             // which positions a lane stages does not change from one channel group to the next, and the compiler would
             // work out every address ahead of the loop and keep them all in registers: hidden from it
             asm volatile("" : "+v"(cu));
             const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(X + (size_t)ci0 * HW), 0, CG * HW * 4, 0x00020000);
-            const int corner = cl * HW + iy0 * W + ix0;
+            const int corner = cl * HW + iy0 * W;
             const bool inside = ix0 >= 0 && ix0 + PC <= W;          // no vector reaches beside the image
-            const auto begins_before = [&](int vi) { return P % 4 != 0 && ix0 < 0 && vi == P / 4; };      // (columns begin at a multiple of 16, less P)
             unsigned char* const plane = tile + (cl / 4) * PLANE + (cl % 4) * 4;
             constexpr int JB = Units::JB, NBATCH = Units::NBATCH, UNROLL = (NIMG == 1 && NBATCH <= 4) ? NBATCH : 1;
             if constexpr (NBATCH > 1 || !TURNED) take_filters(std::integral_constant<int, 0>{});
@@ -206,19 +205,18 @@ struct ConvF32Rect {
                 for (int jj = 0; jj < JB; ++jj) {
                     const int u = (j0 + jj) * LPC + cu;
                     const int r = u / NVR, vi = u % NVR, iy = iy0 + r;
-                    v[jj] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, iy >= 0 && iy < H && u < NU ? (unsigned)((corner + r * W + 4 * vi + (begins_before(vi) ? P % 4 : 0)) * 4) : 0x7fffffffu, 0, 0));
+                    v[jj] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, iy >= 0 && iy < H && u < NU ? (unsigned)((corner + r * W + Columns::from(ix0, vi)) * 4) : 0x7fffffffu, 0, 0));
                 }
                 if constexpr (NBATCH == 1 && TURNED) take_filters(std::integral_constant<int, JB>{});
                 asm volatile("" : "+v"(cu));   // likewise: the stores work their addresses out again, one vector at a time
 #pragma unroll
                 for (int jj = 0; jj < JB; ++jj) {
                     const int u = (j0 + jj) * LPC + cu;
-                    const int vi = u % NVR, x = ix0 + 4 * vi;
-                    const bool moved = begins_before(vi);
+                    const int vi = u % NVR;
                     if (Units::there(j0 + jj, u)) {
                         float* const dst = reinterpret_cast<float*>(plane + u * 64);
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) dst[4 * e] = inside || (unsigned)(x + e) < (unsigned)W ? moved && e >= P % 4 ? v[jj][e - P % 4 >= 0 ? e - P % 4 : 0] : v[jj][e] : 0.f;
+                        for (int e = 0; e < 4; ++e) dst[4 * e] = Columns::at(v[jj], e, ix0, vi, inside);
                     }
                 }
             }

@@ -163,3 +163,34 @@ def test_a_patch_of_few_channels_stores_its_units_and_no_others(tmp_path):
         for n in (1, 8):
             text += f"static_assert(units_are_right<ConvTiling<{ci}, 32, {h}, {w}, {k}, {k}, {s}, {p}, {n}>::staged>());\n"
     _compiles(text, tmp_path)
+
+
+def test_columns_of_a_patch_against_the_padded_image(tmp_path):
+    """A row of a buffer of two rows (the first begins the buffer), loaded and moved as the rectangles do: every column of every tile's patch is the image's, or zero."""
+    text = """
+        template <int W, int P, int STEP, int NVR> constexpr bool columns_are_right(int tiles)
+        {
+            using C = PatchColumns<W, P, STEP>;
+            for (int t = 0; t < tiles; ++t)
+                for (int y = 0; y < 2; ++y) {
+                    const int ix0 = t * STEP - P;
+                    const bool inside = ix0 >= 0 && ix0 + 4 * NVR <= W;
+                    for (int vi = 0; vi < NVR; ++vi) {
+                        const int at = y * W + C::from(ix0, vi);
+                        float came[4] = {};
+                        for (int e = 0; e < 4; ++e) came[e] = at >= 0 && at + e < 2 * W ? at + e + 1 : 0;    // a vector before the buffer is none at all
+                        for (int e = 0; e < 4; ++e) {
+                            const int x = ix0 + 4 * vi + e;
+                            const float want = x >= 0 && x < W ? y * W + x + 1 : 0;
+                            if (C::at(came, e, ix0, vi, inside) != want || (inside && C::at(came, e, ix0, vi, false) != want)) return false;
+                        }
+                    }
+                }
+            return true;
+        }
+    """
+    for w in (1, 2, 3, 5, 16, 33, 60, 64):
+        for step, nvr in ((16, 5), (32, 9), (64, 17)):
+            for p in (0, 1, 2, 3, 5, 14, 15, 16, 17, 18, 19, 20, 31, 33, 34, 47, 49, 65, 66, 67, 130):
+                text += f"static_assert(columns_are_right<{w}, {p}, {step}, {nvr}>({(w + 2 * p) // step + 1}));\n"
+    _compiles(text, tmp_path)
