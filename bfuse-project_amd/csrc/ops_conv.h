@@ -45,6 +45,7 @@
 
 #include "dispatch.h"
 #include "ops_conv_filters.h"
+#include "ops_conv_patch.h"
 #include "wave.h"
 
 namespace bfuse {
@@ -69,6 +70,7 @@ struct Conv3x3F32Lds {
     // start one 16-byte slot apart in the banks, which is what makes the staging writes below conflict-free
     // (and the tap reads two-way conflicted: the cheaper side of the trade, see the header)
     static constexpr int PLANE = (NPOS * 16 + 255) / 256 * 256 + 16;
+    using Source = PatchSource<16LL * HW>;
     using Filters = FilterRows<CI, 9, TM>;              // (pass through the tile before the patch is staged)
     static constexpr int TILE_BYTES = 4 * PLANE > Filters::BYTES ? 4 * PLANE : Filters::BYTES;
     static constexpr int CPR = W / 4;                   // 16-byte chunks per image row
@@ -131,7 +133,8 @@ struct Conv3x3F32Lds {
         int pt, ct;
         tile_of(vblock, pt, ct);
         const int p0 = pt * TP, co0 = ct * BM;
-        const int y_lo = p0 / W;                       // first image row of the tile; staged row 0 is y_lo - 1
+        int y_lo = p0 / W;                             // first image row of the tile; staged row 0 is y_lo - 1
+        opaque_uniform(y_lo);
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;   // wave-uniform: addresses built on it stay in scalar registers
         const int li = lane & 15, kq = lane >> 4;
         unsigned char* const tile = sm.t + wave * TILE_BYTES;
@@ -166,13 +169,13 @@ struct Conv3x3F32Lds {
             // border test would.
             const int cl = lane >> 2, c4 = lane & 3;
             const int first = y_lo == 0 ? CPR : 0, end = (H + 1 - y_lo < R ? H + 1 - y_lo : R) * CPR;   // chunks inside it
-            const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(X + (size_t)ci0 * HW), 0, 16 * HW * 4, 0x00020000);
-            const unsigned x_voff = (unsigned)((cl * HW + (y_lo - 1) * W) * 4 + c4 * 16);
+            const auto xr = Source::open(opaque_pointer(X + (size_t)ci0 * HW));
+            const int corner = cl * HW + (y_lo - 1) * W + c4 * 4;
             f32x4 v[NLD];
 #pragma unroll
             for (int j = 0; j < NLD; ++j) {
                 const int cc = j * 4 + c4;                 // chunk within the channel's R x W patch
-                v[j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, cc >= first && cc < end ? x_voff + j * 64 : 0x7fffffffu, 0, 0));
+                v[j] = Source::template load<4>(xr, cc >= first && cc < end ? Source::place(corner + j * 16) : Source::outside());
             }
             aw.template take<NLD>(0, tile, lane);
 #pragma unroll

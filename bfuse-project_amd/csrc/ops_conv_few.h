@@ -47,6 +47,7 @@ struct ConvF32Few {
     static constexpr int NU = CI * PR * NVR;            // staging units (channel, row, vector)
     using Units = PatchUnits<NU, 64>;
     using Columns = PatchColumns<W, P, 16 * TWB * S>;
+    using Source = PatchSource<(long long)CI * HW>;
     static constexpr int NLD = Units::NLD;              // wave-level loads
     static_assert(CI >= 1 && CI <= 4 && CO % BM == 0 && BM % 16 == 0, "channels");
     static_assert(S >= 1 && OH >= 1 && OW >= 1 && TH >= 1 && (PR * PC + KW) * 4 < 65536, "shape; offsets of rows and taps are 16-bit immediates");
@@ -102,7 +103,7 @@ struct ConvF32Few {
 
         // Stage the patch, [channel][row][PC floats]: the lanes take its vectors in turn, which follow each other in LDS.  A vector of a row outside the image is
         // read past the buffer's end; floats beside the image are made zeros (PatchColumns).
-        const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)X, 0, CI * HW * 4, 0x00020000);
+        const auto xr = Source::open(X);
         const bool inside = ix0 >= 0 && ix0 + PC <= W;          // no vector reaches beside the image
         constexpr int JB = Units::JB;
         if constexpr (!TURNED) filters.load(Wt, co0, lane);
@@ -113,7 +114,7 @@ struct ConvF32Few {
 #pragma unroll
             for (int jj = 0; jj < JB; ++jj) {
                 const int u = (j0 + jj) * 64 + lane, r = u / NVR, vi = u % NVR, c = r / PR, iy = iy0 + r - c * PR;
-                v[jj] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, iy >= 0 && iy < H && u < NU ? (unsigned)((c * HW + iy * W + Columns::from(ix0, vi)) * 4) : 0x7fffffffu, 0, 0));
+                v[jj] = Source::template load<4>(xr, iy >= 0 && iy < H && u < NU ? Source::place(c * HW + iy * W + Columns::from(ix0, vi)) : Source::outside());
             }
             if constexpr (NLD <= JB && TURNED) filters.take(Wt, co0, tile, lane);
             if (!inside) {

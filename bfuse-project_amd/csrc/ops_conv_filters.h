@@ -37,7 +37,7 @@ struct FilterRows {
     __device__ __forceinline__ void take(int tm, const unsigned char* room, int lane)
     {
 #if defined(__HIP_DEVICE_COMPILE__)
-        asm volatile("s_waitcnt vmcnt(%0) ; loads into LDS have landed" : : "n"(BEHIND) : "memory");
+        asm volatile("s_waitcnt vmcnt(%0) ; loads into LDS have landed" : : "n"(BEHIND < 63 ? BEHIND : 63) : "memory");
 #endif
         const int li = lane & 15, kq = lane >> 4;
 #pragma unroll

@@ -36,6 +36,7 @@
 
 #include "dispatch.h"
 #include "ops_conv_filters.h"
+#include "ops_conv_patch.h"
 #include "wave.h"
 
 namespace bfuse {
@@ -76,6 +77,7 @@ struct ConvF32Lds {
     static constexpr int NU = R * W / VW;               // staging units per channel
     static constexpr int NLD = (NU + LPC - 1) / LPC;    // wave-level loads per group
     static constexpr int NZ = (NQ * PLANE + 1023) / 1024;
+    using Source = PatchSource<(long long)(CG < CI ? CG : CI) * HW>;
     // staged straight from the rows; those outside the image are stored as zeros, so that only the columns beside it need zeros of their own
     static constexpr bool BY_ROWS = VW == 4 || W < 4 || NIMG == 1;
     static constexpr int NPAD = R * 2 * P * NQ;         // positions of padding
@@ -149,7 +151,8 @@ struct ConvF32Lds {
         }
         const int p0 = pt * TP, co0 = ct * BM;
         const int oy_lo = p0 / OW;                     // first output row of the tile
-        const int iy_lo = oy_lo * S - P;               // image row of staged row 0
+        int iy_lo = oy_lo * S - P;                     // image row of staged row 0
+        if constexpr (TURNED && BY_ROWS) opaque_uniform(iy_lo);
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
         const int li = lane & 15, kq = lane >> 4;
         unsigned char* const tile = sm.t + wave * TILE_BYTES;
@@ -246,27 +249,16 @@ struct ConvF32Lds {
                 // The patch's rows follow each other in memory; units of rows outside the image, and of channels that the layer
                 // does not have, are read past the buffer's end, which gives zeros.
                 const int first = iy_lo < 0 ? -iy_lo * (W / VW) : 0, end = (H - iy_lo < R ? H - iy_lo : R) * (W / VW);
-                const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(X + (size_t)ci0 * HW), 0, (CG < CI ? CG : CI) * HW * 4, 0x00020000);
-                const unsigned x_voff = (unsigned)((cl * HW + iy_lo * W + cu * VW) * 4);
+                const auto xr = Source::open(opaque_pointer(X + (size_t)ci0 * HW));
+                const int corner = cl * HW + iy_lo * W + cu * VW;
                 if constexpr (NBATCH > 1) take_filters(std::integral_constant<int, 0>{});
 #pragma unroll UNROLL
                 for (int j0 = 0; j0 < NLD; j0 += JB) {
-                    float v[JB][VW];
+                    decltype(Source::template load<VW>(xr, 0)) v[JB];
 #pragma unroll
                     for (int jj = 0; jj < JB; ++jj) {
                         const int u = (j0 + jj) * LPC + cu;
-                        const unsigned at = u >= first && u < end ? x_voff + (j0 + jj) * (LPC * VW * 4) : 0x7fffffffu;
-                        if constexpr (VW == 4) {
-                            const f32x4 q = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, at, 0, 0));
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) v[jj][e] = q[e];
-                        } else if constexpr (VW == 2) {
-                            const f32x2 q = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(xr, at, 0, 0));
-                            v[jj][0] = q[0];
-                            v[jj][1] = q[1];
-                        } else {
-                            v[jj][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, at, 0, 0));
-                        }
+                        v[jj] = Source::template load<VW>(xr, u >= first && u < end ? Source::place(corner + (j0 + jj) * (LPC * VW)) : Source::outside());
                     }
                     if constexpr (NBATCH == 1) take_filters(std::integral_constant<int, JB>{});
 #pragma unroll

@@ -1,9 +1,35 @@
-// A patch of an image in whole vectors of four floats, as the convolutions on rectangles (ConvF32Rect, ConvF32Few) stage it: which of them a lane takes, and
-// what becomes of one that reaches beside the image.
+// How the per-wave convolutions (Conv3x3F32Lds, ConvF32Lds, ConvF32Rect, ConvF32Few) load the patches that they stage, and which whole vectors of four floats
+// a lane takes on rectangles, and what becomes of one that reaches beside the image.
 #pragma once
 #include <hip/hip_runtime.h>
 
 namespace bfuse {
+
+// The patch's loads, from a buffer of FLOATS floats with its own range check.
+// Where a wait for the filters counts the loads behind them (FilterRows::take), all of these have to be made and to stay ahead of it, whatever the compiler
+// knows of them.  So the pointer is opaque there (a memory clobber orders nothing against a `__restrict__` argument: a load that is used under a condition only was moved
+// behind the wait, into it), and so is the first row (of two loads known to lie outside the image one was made).
+template <long long FLOATS>
+struct PatchSource {
+    __device__ static __forceinline__ auto open(const float* x)
+    {
+        return __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, (int)(FLOATS * 4), 0x00020000);
+    }
+    // Float `at` of them, and a place outside the image.
+    __device__ static constexpr __forceinline__ unsigned place(int at) { return (unsigned)(at * 4); }
+    __device__ static constexpr __forceinline__ unsigned outside() { return 0x7fffffffu; }
+    // N floats from there on; those outside are zeros.
+    template <int N, class Source>
+    __device__ static __forceinline__ auto load(Source from, unsigned at)
+    {
+        typedef float vec __attribute__((ext_vector_type(N)));
+        vec v;
+        if constexpr (N == 4) v = __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b128(from, at, 0, 0));
+        else if constexpr (N == 2) v = __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b64(from, at, 0, 0));
+        else v[0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(from, at, 0, 0));
+        return v;
+    }
+};
 
 // NU units for LANES lanes, one a load, up to sixteen loads under way at a time.
 template <int NU, int LANES>

@@ -66,6 +66,7 @@ struct ConvF32Rect {
     static constexpr int NU = PR * NVR;                 // staging units (row, vector) per channel
     using Units = PatchUnits<NU, LPC>;
     using Columns = PatchColumns<W, P, 16 * S>;
+    using Source = PatchSource<(long long)CG * HW>;
     static constexpr int NLD = Units::NLD;              // wave-level loads per group
     static_assert(CI % 16 == 0, "input channels: a multiple of 16");
     static_assert(CO % BM == 0 && BM % 16 == 0 && NGROUP % KS == 0, "channel tiling");
@@ -192,7 +193,7 @@ struct ConvF32Rect {
             // which positions a lane stages does not change from one channel group to the next, and the compiler would
             // work out every address ahead of the loop and keep them all in registers: hidden from it
             asm volatile("" : "+v"(cu));
-            const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(X + (size_t)ci0 * HW), 0, CG * HW * 4, 0x00020000);
+            const auto xr = Source::open(opaque_pointer(X + (size_t)ci0 * HW));
             const int corner = cl * HW + iy0 * W;
             const bool inside = ix0 >= 0 && ix0 + PC <= W;          // no vector reaches beside the image
             unsigned char* const plane = tile + (cl / 4) * PLANE + (cl % 4) * 4;
@@ -205,7 +206,7 @@ struct ConvF32Rect {
                 for (int jj = 0; jj < JB; ++jj) {
                     const int u = (j0 + jj) * LPC + cu;
                     const int r = u / NVR, vi = u % NVR, iy = iy0 + r;
-                    v[jj] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, iy >= 0 && iy < H && u < NU ? (unsigned)((corner + r * W + Columns::from(ix0, vi)) * 4) : 0x7fffffffu, 0, 0));
+                    v[jj] = Source::template load<4>(xr, iy >= 0 && iy < H && u < NU ? Source::place(corner + r * W + Columns::from(ix0, vi)) : Source::outside());
                 }
                 if constexpr (NBATCH == 1 && TURNED) take_filters(std::integral_constant<int, JB>{});
                 asm volatile("" : "+v"(cu));   // likewise: the stores work their addresses out again, one vector at a time

@@ -214,6 +214,15 @@ __device__ __forceinline__ void opaque_value(V& v)
 #endif
 }
 
+// Likewise a wave-uniform one.
+template <class V>
+__device__ __forceinline__ void opaque_uniform(V& v)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(v));
+#endif
+}
+
 // A kernel-argument pointer (wave-uniform, `__restrict__`) as the compiler sees an unknown pointer
 // into device memory.  The memory clobbers in JoinSync::yield() order nothing against memory that
 // is only reachable through a noalias argument (an asm without pointer operands cannot touch it, so

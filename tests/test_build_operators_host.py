@@ -2,12 +2,14 @@
 scripts/configure_kernels.py:40-69): which ids the templates take, the tiling rule, the text of the translation unit,
 and `configure --build-missing` over the in-tree example (compiled by the build step)."""
 import os
+import subprocess
+import sys
 
 import pytest
 import yaml
 
 from bfuse_project_amd import build_operators as bo
-from bfuse_project_amd import configure
+from bfuse_project_amd import build_pairs, configure
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -90,3 +92,21 @@ def test_missing_ids_are_refused_reported_or_built(tmp_path):
     assert info["FusionSet"][1]["Set"] == ["bgemm_f32_6x96x48x80", "bgemm_f32_5x100x32x72", "gemm_f32_48x160x96_nk", "gemm_f32_512x768x768"]
     with open(os.path.join(built, "modules.yaml")) as f:
         assert yaml.safe_load(f) == ["hip/operators/libbfuse_pairs.so", "hip/libbfuse_pairs.so"]
+
+
+def _findings(ids, tmp_path):
+    """What the build's checks (no spills, no instruction ahead of the wait for what it needs) find in the operators of `ids`."""
+    (tmp_path / "unit.hip").write_text(bo.source_text(ids))
+    r = subprocess.run(["/opt/rocm/bin/hipcc", "--offload-arch=gfx950", "--cuda-device-only", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                        "-Rpass-analysis=kernel-resource-usage", "-I", bo.CSRC, "-S", str(tmp_path / "unit.hip"), "-o", str(tmp_path / "unit.s")], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    c = subprocess.run([sys.executable, os.path.join(bo.CSRC, "check_asm_reads.py"), str(tmp_path / "unit.s")], capture_output=True, text=True)
+    return build_pairs.spilling_kernels(r.stderr) + [line for line in c.stdout.splitlines() if line.startswith("error:")]
+
+
+def test_loads_that_a_wait_counts_are_made_and_stay_ahead_of_it(tmp_path):
+    """Filters on their way into LDS are waited for by the number of patch loads behind them.  The compiler moved a load that only some lanes use behind the wait, and made one of two
+    that it knew to lie outside the image (all rows of an image in one tile); kernels of fewer loads than the wait says are refused by the build."""
+    shapes = [[64, 35, 36, 16, 128, 3, 3, 1, 0], [1024, 12, 12, 32, 16, 7, 1, 2, 3], [1, 8, 7, 256, 16, 3, 3, 3, 0], [1, 10, 10, 128, 16, 1, 2, 3, 0], [1, 12, 12, 16, 128, 3, 3, 1, 0],
+              [2, 12, 12, 128, 16, 3, 2, 3, 4], [256, 12, 12, 160, 16, 2, 1, 2, 2], [1, 30, 30, 16, 64, 4, 1, 2, 2], [8, 64, 64, 48, 16, 3, 3, 1, 1]]
+    assert _findings({f"conv2d_{i}": a for i, a in enumerate(shapes)}, tmp_path) == []
