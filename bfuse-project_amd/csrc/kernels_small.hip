@@ -222,6 +222,22 @@ CONV_STAGED_TEST(x, 2, 16, 7, 62, 16, 3, 3, 1, 17, ConvF32Rect<16, 16, 7, 62, 3,
 CONV_STAGED_TEST(y, 1, 16, 5, 70, 32, 3, 3, 1, 35, ConvF32Rect<16, 32, 5, 70, 3, 3, 1, 35, 32, 4, 1, 1>)
 CONV_STAGED_TEST(z, 2, 3, 9, 61, 16, 3, 3, 1, 18, ConvF32Few<3, 16, 9, 61, 3, 3, 1, 18, 16, 4, 1, 2>)
 CONV_STAGED_TEST(aa, 1, 4, 12, 64, 32, 3, 3, 1, 67, ConvF32Few<4, 32, 12, 64, 3, 3, 1, 67, 32, 2, 4, 1>)
+// Images too large for a buffer: their loads on small ones, then 2 GiB of 16 channels and of four (the last floats lie beyond 2^31 bytes; results 16 or 64 times fewer).
+template <> inline constexpr bool bfuse::kFarPatch<16 * 11 * 77> = true;
+template <> inline constexpr bool bfuse::kFarPatch<3 * 13 * 83> = true;
+template <> inline constexpr bool bfuse::kFarPatch<16 * 9 * 15> = true;
+template <> inline constexpr bool bfuse::kFarPatch<16 * 10 * 14> = true;
+template <> inline constexpr bool bfuse::kFarPatch<16 * 8 * 20> = true;
+CONV_STAGED_TEST(ba, 2, 32, 11, 77, 32, 3, 3, 1, 2, ConvF32Rect<32, 32, 11, 77, 3, 3, 1, 2, 32, 4, 2, 2>)
+CONV_STAGED_TEST(bb, 2, 3, 13, 83, 16, 5, 5, 1, 2, ConvF32Few<3, 16, 13, 83, 5, 5, 1, 2, 16, 2, 1, 2>)
+CONV_STAGED_TEST(bc, 1, 32, 9, 15, 16, 3, 3, 1, 1, ConvF32Lds<32, 16, 9, 15, 3, 3, 1, 1, 16, 2, 1, 1>)
+CONV_STAGED_TEST(bd, 1, 16, 10, 14, 16, 5, 3, 2, 1, ConvF32Lds<16, 16, 10, 14, 5, 3, 2, 1, 16, 2, 1, 1>)
+CONV_STAGED_TEST(be, 1, 32, 8, 20, 32, 3, 3, 1, 1, Conv3x3F32Lds<32, 32, 8, 20, 32, 2, 2>)
+CONV_STAGED_TEST(huge_a, 1, 16, 8192, 4100, 16, 5, 5, 4, 2, ConvF32Auto<16, 16, 8192, 4100, 5, 5, 4, 2, 1>)
+CONV_STAGED_TEST(huge_b, 1, 4, 11600, 11601, 16, 8, 8, 8, 1, ConvF32Auto<4, 16, 11600, 11601, 8, 8, 8, 1, 1>)
+CONV_STAGED_TEST(huge_c, 1, 16, 1048580, 36, 16, 3, 3, 4, 1, ConvF32Auto<16, 16, 1048580, 36, 3, 3, 4, 1, 1>)
+static_assert(ConvTiling<16, 16, 8192, 4100, 5, 5, 4, 2, 1>::RECT && ConvW_huge_a::Source::FAR && ConvW_huge_b::Source::FAR && ConvTiling<4, 16, 11600, 11601, 8, 8, 8, 1, 1>::FEW);
+static_assert(!ConvTiling<16, 16, 1048580, 36, 3, 3, 4, 1, 1>::RECT && ConvW_huge_c::Source::FAR && ConvW_ba::Source::FAR && ConvW_be::Source::FAR && !ConvW_x::Source::FAR);
 // More loads than are under way at a time, the last batch of them shorter than the others though every lane has a unit in each (25 loads, 16 at a time).
 CONV_STAGED_TEST(t, 2, 32, 15, 170, 16, 5, 5, 5, 0, ConvF32Rect<32, 16, 15, 170, 5, 5, 5, 0, 16, 1, 2, 2>)         // a second wave's tile behind the patch
 CONV_STAGED_TEST(u, 1, 32, 15, 165, 16, 5, 5, 5, 2, ConvF32Rect<32, 16, 15, 165, 5, 5, 5, 2, 16, 1, 1, 1>)         // a partner's behind it, and a second group's; unrolled

@@ -170,14 +170,14 @@ struct Conv3x3F32Lds {
             const int cl = lane >> 2, c4 = lane & 3;
             const int first = y_lo == 0 ? CPR : 0, end = (H + 1 - y_lo < R ? H + 1 - y_lo : R) * CPR;   // chunks inside it
             const auto xr = Source::open(opaque_pointer(X + (size_t)ci0 * HW));
-            const int corner = cl * HW + (y_lo - 1) * W + c4 * 4;
+            const typename Source::Index corner = (typename Source::Index)cl * HW + (y_lo - 1) * W + c4 * 4;
             f32x4 v[NLD];
 #pragma unroll
             for (int j = 0; j < NLD; ++j) {
                 const int cc = j * 4 + c4;                 // chunk within the channel's R x W patch
                 v[j] = Source::template load<4>(xr, cc >= first && cc < end ? Source::place(corner + j * 16) : Source::outside());
             }
-            aw.template take<NLD>(0, tile, lane);
+            aw.template take<Source::template Behind<NLD>::value>(0, tile, lane);
 #pragma unroll
             for (int tm = 1; tm < TM; ++tm) {
                 Filters::request(Wt, co0, ci0, tm, tile, lane);

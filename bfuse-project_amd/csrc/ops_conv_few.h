@@ -114,7 +114,7 @@ struct ConvF32Few {
 #pragma unroll
             for (int jj = 0; jj < JB; ++jj) {
                 const int u = (j0 + jj) * 64 + lane, r = u / NVR, vi = u % NVR, c = r / PR, iy = iy0 + r - c * PR;
-                v[jj] = Source::template load<4>(xr, iy >= 0 && iy < H && u < NU ? Source::place(c * HW + iy * W + Columns::from(ix0, vi)) : Source::outside());
+                v[jj] = Source::template load<4>(xr, iy >= 0 && iy < H && u < NU ? Source::place((typename Source::Index)c * HW + iy * W + Columns::from(ix0, vi)) : Source::outside());
             }
             if constexpr (NLD <= JB && TURNED) filters.take(Wt, co0, tile, lane);
             if (!inside) {

@@ -250,7 +250,7 @@ struct ConvF32Lds {
                 // does not have, are read past the buffer's end, which gives zeros.
                 const int first = iy_lo < 0 ? -iy_lo * (W / VW) : 0, end = (H - iy_lo < R ? H - iy_lo : R) * (W / VW);
                 const auto xr = Source::open(opaque_pointer(X + (size_t)ci0 * HW));
-                const int corner = cl * HW + iy_lo * W + cu * VW;
+                const typename Source::Index corner = (typename Source::Index)cl * HW + iy_lo * W + cu * VW;
                 if constexpr (NBATCH > 1) take_filters(std::integral_constant<int, 0>{});
 #pragma unroll UNROLL
                 for (int j0 = 0; j0 < NLD; j0 += JB) {
@@ -260,7 +260,7 @@ struct ConvF32Lds {
                         const int u = (j0 + jj) * LPC + cu;
                         v[jj] = Source::template load<VW>(xr, u >= first && u < end ? Source::place(corner + (j0 + jj) * (LPC * VW)) : Source::outside());
                     }
-                    if constexpr (NBATCH == 1) take_filters(std::integral_constant<int, JB>{});
+                    if constexpr (NBATCH == 1) take_filters(typename Source::template Behind<JB>{});
 #pragma unroll
                     for (int jj = 0; jj < JB; ++jj) {
                         const int u = (j0 + jj) * LPC + cu;

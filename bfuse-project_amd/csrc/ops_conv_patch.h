@@ -3,28 +3,46 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 namespace bfuse {
 
-// The patch's loads, from a buffer of FLOATS floats with its own range check.
+// Whether the FLOATS floats that a patch's loads can reach are too many for a buffer: the place outside the image, byte 2^31 - 1, has to lie past its end.
+// (Self-tests say so of small ones.)
+template <long long FLOATS>
+inline constexpr bool kFarPatch = FLOATS * 4 > 0x7fffffffLL;
+
+// The patch's loads: a buffer with its own range check, or, for images of 2 GiB and more (of the channels of a group), a test of every float.
 // Where a wait for the filters counts the loads behind them (FilterRows::take), all of these have to be made and to stay ahead of it, whatever the compiler
 // knows of them.  So the pointer is opaque there (a memory clobber orders nothing against a `__restrict__` argument: a load that is used under a condition only was moved
 // behind the wait, into it), and so is the first row (of two loads known to lie outside the image one was made).
 template <long long FLOATS>
 struct PatchSource {
+    static constexpr bool FAR = kFarPatch<FLOATS>;
+    using Index = std::conditional_t<FAR, long long, int>;
+    using Place = std::conditional_t<FAR, long long, unsigned>;
+    // How many loads are under way behind the filters' where LOADS were written down.
+    template <int LOADS>
+    using Behind = std::integral_constant<int, FAR ? 0 : LOADS>;
+
     __device__ static __forceinline__ auto open(const float* x)
     {
-        return __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, (int)(FLOATS * 4), 0x00020000);
+        if constexpr (FAR) return x;
+        else return __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, (int)(FLOATS * 4), 0x00020000);
     }
     // Float `at` of them, and a place outside the image.
-    __device__ static constexpr __forceinline__ unsigned place(int at) { return (unsigned)(at * 4); }
-    __device__ static constexpr __forceinline__ unsigned outside() { return 0x7fffffffu; }
+    __device__ static constexpr __forceinline__ Place place(Index at) { return FAR ? (Place)at : (Place)(at * 4); }
+    __device__ static constexpr __forceinline__ Place outside() { return FAR ? (Place)-4096 : (Place)0x7fffffff; }
     // N floats from there on; those outside are zeros.
     template <int N, class Source>
-    __device__ static __forceinline__ auto load(Source from, unsigned at)
+    __device__ static __forceinline__ auto load(Source from, Place at)
     {
         typedef float vec __attribute__((ext_vector_type(N)));
         vec v;
-        if constexpr (N == 4) v = __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b128(from, at, 0, 0));
+        if constexpr (FAR) {
+#pragma unroll
+            for (int e = 0; e < N; ++e) v[e] = (unsigned long long)(at + e) < (unsigned long long)FLOATS ? from[at + e] : 0.f;
+        } else if constexpr (N == 4) v = __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b128(from, at, 0, 0));
         else if constexpr (N == 2) v = __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b64(from, at, 0, 0));
         else v[0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(from, at, 0, 0));
         return v;

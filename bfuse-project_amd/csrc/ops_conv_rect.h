@@ -194,7 +194,7 @@ struct ConvF32Rect {
             // work out every address ahead of the loop and keep them all in registers: hidden from it
             asm volatile("" : "+v"(cu));
             const auto xr = Source::open(opaque_pointer(X + (size_t)ci0 * HW));
-            const int corner = cl * HW + iy0 * W;
+            const typename Source::Index corner = (typename Source::Index)cl * HW + iy0 * W;
             const bool inside = ix0 >= 0 && ix0 + PC <= W;          // no vector reaches beside the image
             unsigned char* const plane = tile + (cl / 4) * PLANE + (cl % 4) * 4;
             constexpr int JB = Units::JB, NBATCH = Units::NBATCH, UNROLL = (NIMG == 1 && NBATCH <= 4) ? NBATCH : 1;
@@ -208,7 +208,7 @@ struct ConvF32Rect {
                     const int r = u / NVR, vi = u % NVR, iy = iy0 + r;
                     v[jj] = Source::template load<4>(xr, iy >= 0 && iy < H && u < NU ? Source::place(corner + r * W + Columns::from(ix0, vi)) : Source::outside());
                 }
-                if constexpr (NBATCH == 1 && TURNED) take_filters(std::integral_constant<int, JB>{});
+                if constexpr (NBATCH == 1 && TURNED) take_filters(typename Source::template Behind<JB>{});
                 asm volatile("" : "+v"(cu));   // likewise: the stores work their addresses out again, one vector at a time
 #pragma unroll
                 for (int jj = 0; jj < JB; ++jj) {

@@ -8,6 +8,7 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 
 PROLOGUE = """
 #include <type_traits>
+#include "ops_conv.h"
 #include "ops_conv_1x1.h"
 #include "ops_conv_rect.h"
 using namespace bfuse;
@@ -194,3 +195,14 @@ def test_columns_of_a_patch_against_the_padded_image(tmp_path):
             for p in (0, 1, 2, 3, 5, 14, 15, 16, 17, 18, 19, 20, 31, 33, 34, 47, 49, 65, 66, 67, 130):
                 text += f"static_assert(columns_are_right<{w}, {p}, {step}, {nvr}>({(w + 2 * p) // step + 1}));\n"
     _compiles(text, tmp_path)
+
+
+def test_images_that_no_buffer_holds_are_loaded_otherwise(tmp_path):
+    """2^31 - 1 bytes is the offset of what lies outside an image: images (of the 16 channels of a group, or all of few) of that many are not behind a buffer."""
+    _compiles("""
+        static_assert(ConvF32Rect<16, 16, 8192, 4096, 3, 3, 1, 1, 16, 4, 1, 1>::Source::FAR && !ConvF32Rect<64, 16, 8191, 4096, 3, 3, 1, 1, 16, 4, 1, 1>::Source::FAR);
+        static_assert(ConvF32Few<4, 16, 16384, 8192, 3, 3, 1, 1, 16, 4, 1, 1>::Source::FAR && !ConvF32Few<3, 16, 16384, 8192, 3, 3, 1, 1, 16, 4, 1, 1>::Source::FAR);
+        static_assert(ConvF32Lds<16, 16, 1048576, 32, 3, 3, 4, 1, 16, 4, 1, 1>::Source::FAR && !ConvF32Lds<16, 16, 1048575, 32, 3, 3, 4, 1, 16, 4, 1, 1>::Source::FAR);
+        static_assert(Conv3x3F32Lds<16, 16, 1048576, 32, 16, 2, 1>::Source::FAR && !Conv3x3F32Lds<16, 16, 1048574, 32, 16, 2, 1>::Source::FAR);
+        static_assert(sizeof(ConvF32Rect<16, 16, 8192, 4096, 3, 3, 1, 1, 16, 4, 1, 1>::Source::Index) == 8);
+    """, tmp_path)

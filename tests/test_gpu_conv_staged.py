@@ -18,7 +18,8 @@ FORMS = [("a", 1, 2, "bias_relu_4096", "hfuse", ""), ("b", 1, 1, "bias_relu_4096
          ("q", 1, 7, "bias_relu_4096", None, ""), ("r", 1, 6, "bias_relu_4096", None, ""), ("s", 1, 3, "bias_relu_4096", None, ""),
          ("t", 5, 0, "bias_relu_4096", "hfuse", ""), ("u", 5, 2, "conv3x3_f32_32x12x12_32", "hfuse", ""), ("v", 8, 0, "conv3x3_f32_32x12x12_32", "hfuse", ""),
          ("w", 4, 1, "bias_relu_4096", None, ""), ("x", 1, 17, "bias_relu_4096", None, ""), ("y", 1, 35, "bias_relu_4096", None, ""), ("z", 1, 18, "bias_relu_4096", None, ""),
-         ("aa", 1, 67, "bias_relu_4096", None, "")]
+         ("aa", 1, 67, "bias_relu_4096", None, ""), ("ba", 1, 2, "bias_relu_4096", None, ""), ("bb", 1, 2, "bias_relu_4096", None, ""), ("bc", 1, 1, "bias_relu_4096", None, ""),
+         ("bd", 2, 1, "bias_relu_4096", None, ""), ("be", 1, 1, "bias_relu_4096", None, "")]
 
 
 @pytest.mark.parametrize("tag,s,p,partner,kind,suffix", FORMS)
@@ -39,7 +40,7 @@ def test_staged_convolution_copies_what_a_selector_names(tag, s, p):
     assert np.array_equal(y.ravel(), orf.conv2d(x.reshape(k.shapes[0]), w, s=s, p=p).ravel())
 
 
-@pytest.mark.parametrize("tag,s,p", [f[:3] for f in FORMS if f[0] in (*"acdfmnopqrsvwz", "aa")])
+@pytest.mark.parametrize("tag,s,p", [f[:3] for f in FORMS if f[0] in (*"acdfmnopqrsvwz", "aa", "bb")])
 def test_a_value_that_is_not_finite_is_in_its_own_windows_alone(tag, s, p):
     """Four k of an MFMA are rows or taps of a window: those that there are not have no part in it, whatever lies in their place."""
     name = f"selftest_conv_staged_{tag}"
@@ -54,3 +55,26 @@ def test_a_value_that_is_not_finite_is_in_its_own_windows_alone(tag, s, p):
     assert np.array_equal(np.isnan(y), np.isnan(want)) and np.array_equal(np.isposinf(y), np.isposinf(want)) and np.array_equal(np.isneginf(y), np.isneginf(want))
     ok = np.isfinite(want)
     assert ok.any() and np.linalg.norm(y[ok] - want[ok]) <= 1e-5 * np.linalg.norm(want[ok])
+
+
+@pytest.mark.parametrize("tag,s,p", [("huge_a", 4, 2), ("huge_b", 8, 1), ("huge_c", 4, 1)])
+def test_images_of_two_gigabytes(tag, s, p):
+    """An image of zeros but for its corners and a few other elements, each alone in its windows: every result is a product, exactly, or zero."""
+    with bf.Operation(f"selftest_conv_staged_{tag}", "bias_relu_4096") as op:
+        k = op.k[0]
+        (_, ci, h, wd), (co, _, kh, kw), (oh, ow) = k.shapes[0], k.shapes[1], k.shapes[2][2:]
+        assert ci * h * wd * 4 >= 2 ** 31
+        w = fill_normal(9, co * ci * kh * kw, 0, 1).reshape(co, ci, kh, kw)
+        x, want, rng = np.zeros((ci, h, wd), np.float32), np.zeros((co, oh, ow), np.float32), np.random.default_rng(3)
+        places, ys = [], list(range(0, h, h // 64)) + [h - 1]
+        for i, y in enumerate(ys):
+            places += [(int(rng.integers(ci)), y, x0) for x0 in (0, wd // 2 + int(rng.integers(-2, 3)), wd - 1 - (y % 2 if y < h - 1 else 0))]
+        places.append((ci - 1, h - 1, wd - 1 - 2 * kw))
+        for c, y, x0 in places:
+            x[c, y, x0] = v = np.float32(1 + rng.random())
+            for oy in range(max(0, -(-(y + p - kh + 1) // s)), min(oh - 1, (y + p) // s) + 1):
+                for ox in range(max(0, -(-(x0 + p - kw + 1) // s)), min(ow - 1, (x0 + p) // s) + 1):
+                    assert not want[:, oy, ox].any()
+                    want[:, oy, ox] = v * w[:, c, y + p - oy * s, x0 + p - ox * s]
+        y = op.run_kernel(0, x, w)
+        assert np.count_nonzero(want) > 1000 and np.array_equal(y.reshape(want.shape), want)
