@@ -222,6 +222,10 @@ CONV_STAGED_TEST(x, 2, 16, 7, 62, 16, 3, 3, 1, 17, ConvF32Rect<16, 16, 7, 62, 3,
 CONV_STAGED_TEST(y, 1, 16, 5, 70, 32, 3, 3, 1, 35, ConvF32Rect<16, 32, 5, 70, 3, 3, 1, 35, 32, 4, 1, 1>)
 CONV_STAGED_TEST(z, 2, 3, 9, 61, 16, 3, 3, 1, 18, ConvF32Few<3, 16, 9, 61, 3, 3, 1, 18, 16, 4, 1, 2>)
 CONV_STAGED_TEST(aa, 1, 4, 12, 64, 32, 3, 3, 1, 67, ConvF32Few<4, 32, 12, 64, 3, 3, 1, 67, 32, 2, 4, 1>)
+// Eight loads under way at a time beside many taps: three channels at stride 4 (23 loads), rows that are not whole vectors.
+CONV_STAGED_TEST(ca, 1, 3, 30, 190, 16, 13, 13, 4, 6, ConvF32Auto<3, 16, 30, 190, 13, 13, 4, 6, 1>)
+CONV_STAGED_TEST(cb, 2, 2, 19, 50, 16, 14, 14, 1, 0, ConvF32Auto<2, 16, 19, 50, 14, 14, 1, 0, 2>)
+static_assert(ConvW_ca::Units::JB == 8 && !ConvW_ca::Units::WHOLE && ConvW_cb::MOST == 8);
 // Images too large for a buffer: their loads on small ones, then 2 GiB of 16 channels and of four (the last floats lie beyond 2^31 bytes; results 16 or 64 times fewer).
 template <> inline constexpr bool bfuse::kFarPatch<16 * 11 * 77> = true;
 template <> inline constexpr bool bfuse::kFarPatch<3 * 13 * 83> = true;

@@ -45,7 +45,7 @@ struct ConvF32Few {
     static constexpr int TILE_BYTES = TURNED && Filters::BYTES > PATCH_BYTES ? Filters::BYTES : PATCH_BYTES;
     static constexpr int NVR = PC / 4;                  // vectors of a patch row
     static constexpr int NU = CI * PR * NVR;            // staging units (channel, row, vector)
-    using Units = PatchUnits<NU, 64>;
+    using Units = PatchUnits<NU, 64, loads_beside(NM * TM, (NU + 63) / 64)>;
     using Columns = PatchColumns<W, P, 16 * TWB * S>;
     using Source = PatchSource<(long long)CI * HW>;
     static constexpr int NLD = Units::NLD;              // wave-level loads

@@ -80,6 +80,8 @@ struct ConvF32Lds {
     using Source = PatchSource<(long long)(CG < CI ? CG : CI) * HW>;
     // staged straight from the rows; those outside the image are stored as zeros, so that only the columns beside it need zeros of their own
     static constexpr bool BY_ROWS = VW == 4 || W < 4 || NIMG == 1;
+    // loads under way at a time (rows of whole vectors beside filters of groups of 16: sixteen, with eight two of 33 that fit spill)
+    static constexpr int MOST = T > 40 && (CG == 4 || !BY_ROWS) ? loads_beside(4 * (CG == 16 ? T : (T + 3) / 4) * TM, NLD) : 16;
     static constexpr int NPAD = R * 2 * P * NQ;         // positions of padding
     static_assert(WM_ == 0, "shared tiles have stages of four channels and one or two waves over the output channels");
     static_assert(CG == 16 ? CI % 16 == 0 : CI <= 4, "input channels: a multiple of 16, or at most 4");
@@ -242,7 +244,7 @@ struct ConvF32Lds {
             // layers of ResNet-18); a batch of images (throughput) from aligned 16-byte loads, a quarter of the load
             // instructions (1024 images: 20-45 % faster on 35-, 73-, 147- and 299-wide images, 8-11 % on 14 and 7).
             if constexpr (BY_ROWS) {
-                constexpr int JB = NLD < 16 ? NLD : 16;
+                constexpr int JB = NLD < MOST ? NLD : MOST;
                 // a single image is in the latency regime: its few batches are unrolled (the next batch's loads go out
                 // under this one's LDS writes); a batch of images keeps the registers for wider tiles and loops
                 constexpr int NBATCH = (NLD + JB - 1) / JB, UNROLL = (NIMG == 1 && NBATCH <= 4) ? NBATCH : 1;
@@ -287,7 +289,7 @@ struct ConvF32Lds {
                 const bool chan = ci0 + cl < CI;
                 constexpr int NV = (R * W + 3) / 4 + 1;          // aligned vectors that can overlap a span
                 constexpr int NLA = (NV + LPC - 1) / LPC;
-                constexpr int JA = NLA < 16 ? NLA : 16;
+                constexpr int JA = NLA < MOST ? NLA : MOST;
                 constexpr int NBATCH = (NLA + JA - 1) / JA, UNROLL = (NIMG == 1 && NBATCH <= 4) ? NBATCH : 1;
 #pragma unroll UNROLL
                 for (int j0 = 0; j0 < NLA; j0 += JA) {

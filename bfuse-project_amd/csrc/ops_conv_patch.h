@@ -49,11 +49,15 @@ struct PatchSource {
     }
 };
 
-// NU units for LANES lanes, one a load, up to sixteen loads under way at a time.
-template <int NU, int LANES>
+// How many of a patch's loads are under way at a time beside a lane's filters: sixteen take 64 registers, and what their addresses need, out of 256.  (Eight where they would all
+// be one batch are 5 % of the time: 12 x 12 of four channels at stride 2, 13 loads, 484 us and 509.)
+constexpr int loads_beside(int filters, int loads) { return filters > 190 || (filters > 96 && loads >= 16) ? 8 : 16; }
+
+// NU units for LANES lanes, one a load, up to MOST loads under way at a time.
+template <int NU, int LANES, int MOST = 16>
 struct PatchUnits {
     static constexpr int NLD = (NU + LANES - 1) / LANES;         // loads
-    static constexpr int JB = NLD < 16 ? NLD : 16;               // loads of a batch; the last one has fewer, unless
+    static constexpr int JB = NLD < MOST ? NLD : MOST;           // loads of a batch; the last one has fewer, unless
     static constexpr int NBATCH = (NLD + JB - 1) / JB;
     static constexpr bool WHOLE = NLD % JB == 0;
     // Whether load j (of NBATCH JB) brings a unit to the lane whose would be u; what one that does not would store lies past the patch.

@@ -360,9 +360,15 @@ struct ConvTiling {
     static constexpr int FEW_BM = NIMG > 1 && CO % 32 == 0 && T <= 9 ? 32 : 16;
     static constexpr int few_bytes(int th, int twb) { return CI * ((th - 1) * S + KH) * ((16 * twb - 1) * S + KW) * 4; }
     static constexpr int FEW_TWB = NIMG > 1 && T <= 25 && 4 * OW >= 3 * ((OW + 63) / 64 * 64) && few_bytes(2, 4) <= 16384 ? 4 : 1;
-    // Filters of many taps leave registers for fewer rows: eight with 144 of them spill 210, four with 196 do not fit 256.  us before (four rows of ConvF32Rect) and now, 64 images of four channels, 96 wide,
-    // to 32: 12 x 12 221 -> 212, 13 x 13 204 -> 204, 9 x 9 108 -> 103, 14 x 14 289 -> 287; of two, 12 x 12 293 -> 135, of three 337 -> 154; 11 x 11 at stride 4 on 224, three channels to 64, 426 -> 118.
-    static constexpr int FEW_NM = FilterFloats<(CI <= 4 ? CI : 4), KH, KW, 1>::NM, FEW_MOST = FEW_NM <= 64 ? 8 : FEW_NM <= 176 ? 4 : FEW_NM <= 200 ? 3 : 1;
+    // Filters of many taps leave registers for fewer rows.  Eight: up to 64 registers of filters, and not where the rows of a window are many and one after the other for some lane groups
+    // only (13 x 13 and 13 x 11 of one channel, 11 x 11 and 9 x 14 of two spill), or wide at stride 2, where two phases of a row are kept (16 x 13 of one channel).  Four: up to 160 at a stride, 176 without.
+    // us before (four rows of ConvF32Rect) and now, 64 images of four channels, 96 wide,
+    // to 32: 12 x 12 221 -> 212, 13 x 13 204 -> 204, 9 x 9 108 -> 103, 14 x 14 289 -> 287; of two, 12 x 12 293 -> 135, of three 337 -> 154; 11 x 11 at stride 4 on 224, three channels to 64, 426 -> 118;
+    // of one channel, 12 x 12 with eight rows 251 -> 71 (four 76), 10 x 10 of two 204 -> 85 (95).
+    using FewFilters = FilterFloats<(CI <= 4 ? CI : 4), KH, KW, 1>;
+    static constexpr int FEW_NM = FewFilters::NM;
+    static constexpr bool FEW_EIGHT = FEW_NM <= 64 && ((KH <= 10 && KW <= 12) || FewFilters::RPL <= 2 || KH % FewFilters::RPL == 0) && !(S == 2 && KW > 12);
+    static constexpr int FEW_MOST = FEW_EIGHT ? 8 : FEW_NM <= (S == 1 ? 176 : 160) ? 4 : FEW_NM <= 200 ? 3 : 1;
     static constexpr int few_rows(int th) { return th > FEW_MOST ? FEW_MOST : th; }
     static constexpr int FEW_TH = FEW_TWB == 4 ? 2 : few_rows(NIMG > 1 && T > 25 && few_bytes(8, 1) <= 12800 ? 8 : few_bytes(4, 1) <= 25600 ? 4 : few_bytes(2, 1) <= 25600 ? 2 : 1);
     static constexpr bool FEW_LINES = FEW_TWB == 4 && OW % 16 == 0 && (long long)NIMG * CO * OHW * 4 >= (1LL << 28);

@@ -110,3 +110,13 @@ def test_loads_that_a_wait_counts_are_made_and_stay_ahead_of_it(tmp_path):
     shapes = [[64, 35, 36, 16, 128, 3, 3, 1, 0], [1024, 12, 12, 32, 16, 7, 1, 2, 3], [1, 8, 7, 256, 16, 3, 3, 3, 0], [1, 10, 10, 128, 16, 1, 2, 3, 0], [1, 12, 12, 16, 128, 3, 3, 1, 0],
               [2, 12, 12, 128, 16, 3, 2, 3, 4], [256, 12, 12, 160, 16, 2, 1, 2, 2], [1, 30, 30, 16, 64, 4, 1, 2, 2], [8, 64, 64, 48, 16, 3, 3, 1, 1]]
     assert _findings({f"conv2d_{i}": a for i, a in enumerate(shapes)}, tmp_path) == []
+
+
+@pytest.mark.parametrize("shapes", [
+    # one channel, two and more of a batch; at strides; 196 taps where rows are not whole vectors; 49 beside a tile that leaves two waves a SIMD
+    [[64, 96, 96, 32, 1, 13, 13, 1, 6], [8, 14, 200, 32, 1, 13, 12, 1, 6], [64, 224, 224, 32, 1, 13, 11, 1, 6], [64, 96, 96, 32, 2, 11, 11, 1, 5], [256, 50, 50, 64, 2, 11, 11, 1, 3], [8, 160, 160, 64, 2, 11, 10, 1, 5],
+     [64, 200, 200, 16, 1, 16, 13, 2, 8], [8, 160, 131, 64, 2, 9, 14, 1, 8], [8, 200, 200, 96, 2, 10, 11, 2, 5], [64, 160, 160, 96, 2, 12, 10, 2, 0]],
+    [[1, 224, 224, 32, 3, 13, 13, 3, 6], [1024, 224, 224, 32, 3, 13, 13, 4, 6], [1, 224, 224, 32, 4, 12, 12, 4, 6], [8, 160, 160, 32, 4, 12, 12, 4, 6], [64, 96, 96, 32, 4, 13, 13, 3, 6], [1, 224, 224, 32, 4, 13, 13, 4, 6]],
+    [[256, 224, 224, 256, 4, 12, 14, 2, 3], [8, 299, 50, 160, 2, 14, 14, 1, 0], [2, 19, 19, 32, 16, 7, 7, 2, 5], [2, 12, 12, 128, 512, 7, 7, 1, 3], [8, 12, 12, 160, 16, 7, 7, 1, 1], [64, 96, 96, 32, 4, 14, 14, 1, 7]]])
+def test_filters_of_many_taps_leave_room_for_what_they_are_staged_beside(shapes, tmp_path):
+    assert _findings({f"conv2d_{i}": a for i, a in enumerate(shapes)}, tmp_path) == []

@@ -19,7 +19,7 @@ FORMS = [("a", 1, 2, "bias_relu_4096", "hfuse", ""), ("b", 1, 1, "bias_relu_4096
          ("t", 5, 0, "bias_relu_4096", "hfuse", ""), ("u", 5, 2, "conv3x3_f32_32x12x12_32", "hfuse", ""), ("v", 8, 0, "conv3x3_f32_32x12x12_32", "hfuse", ""),
          ("w", 4, 1, "bias_relu_4096", None, ""), ("x", 1, 17, "bias_relu_4096", None, ""), ("y", 1, 35, "bias_relu_4096", None, ""), ("z", 1, 18, "bias_relu_4096", None, ""),
          ("aa", 1, 67, "bias_relu_4096", None, ""), ("ba", 1, 2, "bias_relu_4096", None, ""), ("bb", 1, 2, "bias_relu_4096", None, ""), ("bc", 1, 1, "bias_relu_4096", None, ""),
-         ("bd", 2, 1, "bias_relu_4096", None, ""), ("be", 1, 1, "bias_relu_4096", None, "")]
+         ("bd", 2, 1, "bias_relu_4096", None, ""), ("be", 1, 1, "bias_relu_4096", None, ""), ("ca", 4, 6, "bias_relu_4096", None, ""), ("cb", 1, 0, "bias_relu_4096", None, "")]
 
 
 @pytest.mark.parametrize("tag,s,p,partner,kind,suffix", FORMS)
@@ -40,7 +40,7 @@ def test_staged_convolution_copies_what_a_selector_names(tag, s, p):
     assert np.array_equal(y.ravel(), orf.conv2d(x.reshape(k.shapes[0]), w, s=s, p=p).ravel())
 
 
-@pytest.mark.parametrize("tag,s,p", [f[:3] for f in FORMS if f[0] in (*"acdfmnopqrsvwz", "aa", "bb")])
+@pytest.mark.parametrize("tag,s,p", [f[:3] for f in FORMS if f[0] in (*"acdfmnopqrsvwz", "aa", "bb", "ca", "cb")])
 def test_a_value_that_is_not_finite_is_in_its_own_windows_alone(tag, s, p):
     """Four k of an MFMA are rows or taps of a window: those that there are not have no part in it, whatever lies in their place."""
     name = f"selftest_conv_staged_{tag}"
