@@ -226,6 +226,16 @@ CONV_STAGED_TEST(aa, 1, 4, 12, 64, 32, 3, 3, 1, 67, ConvF32Few<4, 32, 12, 64, 3,
 CONV_STAGED_TEST(ca, 1, 3, 30, 190, 16, 13, 13, 4, 6, ConvF32Auto<3, 16, 30, 190, 13, 13, 4, 6, 1>)
 CONV_STAGED_TEST(cb, 2, 2, 19, 50, 16, 14, 14, 1, 0, ConvF32Auto<2, 16, 19, 50, 14, 14, 1, 0, 2>)
 static_assert(ConvW_ca::Units::JB == 8 && !ConvW_ca::Units::WHOLE && ConvW_cb::MOST == 8);
+// Forms of fewer registers beside ten waves: channels and rows one part after the other, fewer loads under way.
+CONV_STAGED_TEST(da, 2, 3, 11, 131, 32, 3, 3, 1, 0, LdsReserve<ConvF32Few<3, 32, 11, 131, 3, 3, 1, 0, 32, 2, 4, 2>, 1024>)
+CONV_STAGED_TEST(db, 2, 3, 23, 70, 16, 8, 8, 1, 4, ConvF32Auto<3, 16, 23, 70, 8, 8, 1, 4, 2>)                     // eight rows in two parts
+CONV_STAGED_TEST(dc, 1, 4, 31, 188, 16, 9, 9, 3, 4, ConvF32Auto<4, 16, 31, 188, 9, 9, 3, 4, 1>)                   // four rows, one at a time
+CONV_STAGED_TEST(dd, 1, 32, 14, 22, 16, 3, 3, 1, 1, ConvF32Lds<32, 16, 14, 22, 3, 3, 1, 1, 16, 4, 1, 1>)          // four of the loads that one batch was
+BFUSE_BFUSE_KERNEL(selftest_conv_staged_da, Slim<ConvW_da>, gemm_bf16_256x448x1792_p2, GemmB9, _c4, bfuse::kChunked, 4, 1)
+BFUSE_BFUSE_KERNEL(selftest_conv_staged_db, Slim<ConvW_db>, gemm_bf16_256x448x1792_p2, GemmB9, _c4, bfuse::kChunked, 4, 1)
+BFUSE_BFUSE_KERNEL(selftest_conv_staged_dc, Slim<ConvW_dc>, gemm_bf16_256x448x1792_p2, GemmB9, _c4, bfuse::kChunked, 4, 1)
+BFUSE_BFUSE_KERNEL(selftest_conv_staged_dd, Slim<ConvW_dd>, gemm_bf16_256x448x1792_p2, GemmB9, _c4, bfuse::kChunked, 4, 1)
+static_assert(Slim<ConvW_da>::TMP == 1 && Slim<ConvW_db>::THP == 4 && ConvW_db::TH == 8 && Slim<ConvW_dc>::THP == 1 && ConvW_dc::TH == 4 && Slim<ConvW_dd>::MOST == 4);
 // Images too large for a buffer: their loads on small ones, then 2 GiB of 16 channels and of four (the last floats lie beyond 2^31 bytes; results 16 or 64 times fewer).
 template <> inline constexpr bool bfuse::kFarPatch<16 * 11 * 77> = true;
 template <> inline constexpr bool bfuse::kFarPatch<3 * 13 * 83> = true;

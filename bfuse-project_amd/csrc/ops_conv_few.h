@@ -25,7 +25,7 @@
 
 namespace bfuse {
 
-template <int CI_, int CO_, int H_, int W_, int KH_, int KW_, int S_, int P_, int BM_, int TH_, int TWB_, int NIMG_ = 1, bool LINES_ = false>
+template <int CI_, int CO_, int H_, int W_, int KH_, int KW_, int S_, int P_, int BM_, int TH_, int TWB_, int NIMG_ = 1, bool LINES_ = false, bool SLIM_ = false>
 struct ConvF32Few {
     static constexpr bool MATRIX_CORES = true;   // the inner loop is a stream of MFMAs (what the fusion chooser asks)
     static constexpr int CI = CI_, CO = CO_, H = H_, W = W_, KH = KH_, KW = KW_, S = S_, P = P_, BM = BM_, TH = TH_, TWB = TWB_, NIMG = NIMG_;
@@ -34,18 +34,19 @@ struct ConvF32Few {
     static_assert(!LINES || OW % 16 == 0, "rows of whole pieces of lines");
     static constexpr int HW = H * W, OHW = OH * OW;
     static constexpr int TM = BM / 16;
-    static constexpr int PB = TH * TWB;                 // 16-pixel blocks of the tile
     static constexpr int NTX = (OW + 16 * TWB - 1) / (16 * TWB), NTY = (OH + TH - 1) / TH, NPT = NTX * NTY;
     static constexpr int PR = (TH - 1) * S + KH, PC = ((16 * TWB - 1) * S + KW + 3) / 4 * 4;   // patch rows / columns, whole vectors of four
     using Filters = FilterFloats<CI, KH, KW, TM>;
     static constexpr int RPL = Filters::RPL, NLT = Filters::NLT, NM = Filters::NM, LEFT = Filters::LEFT, HALF = (NM + 1) / 2;
+    // 16-channel blocks and rows that are summed up at a time, and the 16-pixel blocks of these
+    static constexpr int TMP = SLIM_ ? 1 : TM, THP = !SLIM_ ? TH : NM > 72 ? 1 : TH % 4 == 0 ? 4 : TH, PB = THP * TWB;
     // The filters come to the registers through the wave's tile, before the patch is staged, where they are not much more than the patch.
     static constexpr bool TURNED = CI * KH * KW <= 160;
     static constexpr int PATCH_BYTES = CI * PR * PC * 4;
     static constexpr int TILE_BYTES = TURNED && Filters::BYTES > PATCH_BYTES ? Filters::BYTES : PATCH_BYTES;
     static constexpr int NVR = PC / 4;                  // vectors of a patch row
     static constexpr int NU = CI * PR * NVR;            // staging units (channel, row, vector)
-    using Units = PatchUnits<NU, 64, loads_beside(NM * TM, (NU + 63) / 64)>;
+    using Units = PatchUnits<NU, 64, (!SLIM_ ? loads_beside(NM * TM, (NU + 63) / 64) : NM > 72 ? 4 : 8)>;
     using Columns = PatchColumns<W, P, 16 * TWB * S>;
     using Source = PatchSource<(long long)CI * HW>;
     static constexpr int NLD = Units::NLD;              // wave-level loads
@@ -146,55 +147,69 @@ struct ConvF32Few {
             const int t = 4 * i + kq < LEFT ? 4 * i + kq : 0;
             last[i] = at(4 * RPL + t / KW, t % KW);
         }
-        auto value = [&](int m, int pb) {
+        auto value = [&](int m, int y0, int pb) {
             const unsigned char* const from = m < RPL * KW ? row[RUN || m / KW >= RPL ? 0 : m / KW] + ((RUN ? m / KW * PC : 0) + m % KW) * 4 : last[m - RPL * KW >= 0 ? m - RPL * KW : 0];
-            const float f = *reinterpret_cast<const float*>(from + (pb / TWB * PC + pb % TWB) * S * 4);
+            const float f = *reinterpret_cast<const float*>(from + ((y0 + pb / TWB) * PC + pb % TWB) * S * 4);
             return m == NM - 1 && LEFT % 4 != 0 && kq >= LEFT % 4 ? 0.f : f;
         };
-        f32x4 acc[2][TM][PB];                               // the sums of the first and of the second half
-        // read the next operands while these multiply
-        float b[2][PB];
-#pragma unroll
-        for (int pb = 0; pb < PB; ++pb) b[0][pb] = value(0, pb);
-#pragma unroll
-        for (int m = 0; m < NM; ++m) {
-            if (m + 1 < NM) {
-#pragma unroll
-                for (int pb = 0; pb < PB; ++pb) b[(m + 1) & 1][pb] = value(m + 1, pb);
-            }
-#pragma unroll
-            for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-                for (int pb = 0; pb < PB; ++pb) {
-                    f32x4& sum = acc[m >= HALF][tm][pb];
-                    sum = __builtin_amdgcn_mfma_f32_16x16x4f32(filters.w[tm][m], b[m & 1][pb], m % HALF == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : sum, 0, 0, 0);
-                }
-        }
-        // lane (j = column of the tile row, rg) owns output channels 4 rg + v of a block
         typedef float cols __attribute__((ext_vector_type(TWB), aligned(4)));
         const int ox = ox0 + li * TWB;
 #pragma unroll
-        for (int tm = 0; tm < TM; ++tm)
+        for (int pass = 0; pass < TM / TMP * (TH / THP); ++pass) {
+            const int t0 = pass / (TH / THP) * TMP, y0 = pass % (TH / THP) * THP;
+#if defined(__HIP_DEVICE_COMPILE__)
+            if (pass > 0) asm volatile("" : : : "memory");   // the patch is read again, not kept
+#endif
+            f32x4 acc[2][TMP][PB];                              // the sums of the first and of the second half
+            // read the next operands while these multiply
+            float b[2][PB];
 #pragma unroll
-            for (int y = 0; y < TH; ++y)
-                if (oy0 + y < OH) {
+            for (int pb = 0; pb < PB; ++pb) b[0][pb] = value(0, y0, pb);
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        float* const to = Y + (size_t)(co0 + tm * 16 + 4 * kq + v) * OHW + (oy0 + y) * OW + ox;
-                        cols c;
+            for (int m = 0; m < NM; ++m) {
+                if (m + 1 < NM) {
 #pragma unroll
-                        for (int b = 0; b < TWB; ++b) c[b] = NM > 1 ? acc[0][tm][y * TWB + b][v] + acc[1][tm][y * TWB + b][v] : acc[0][tm][y * TWB + b][v];
-                        if (ox + TWB <= OW) {
-                            if constexpr (LINES) __builtin_nontemporal_store(c, reinterpret_cast<cols*>(to));
-                            else *reinterpret_cast<cols*>(to) = c;
-                        } else {
+                    for (int pb = 0; pb < PB; ++pb) b[(m + 1) & 1][pb] = value(m + 1, y0, pb);
+                }
 #pragma unroll
-                            for (int b = 0; b + 1 < TWB; ++b)
-                                if (ox + b < OW) to[b] = c[b];
+                for (int tm = 0; tm < TMP; ++tm)
+#pragma unroll
+                    for (int pb = 0; pb < PB; ++pb) {
+                        f32x4& sum = acc[m >= HALF][tm][pb];
+                        sum = __builtin_amdgcn_mfma_f32_16x16x4f32(filters.w[t0 + tm][m], b[m & 1][pb], m % HALF == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : sum, 0, 0, 0);
+                    }
+            }
+            // lane (j = column of the tile row, rg) owns output channels 4 rg + v of a block
+#pragma unroll
+            for (int tm = 0; tm < TMP; ++tm)
+#pragma unroll
+                for (int y = 0; y < THP; ++y)
+                    if (oy0 + y0 + y < OH) {
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) {
+                            float* const to = Y + (size_t)(co0 + (t0 + tm) * 16 + 4 * kq + v) * OHW + (oy0 + y0 + y) * OW + ox;
+                            cols c;
+#pragma unroll
+                            for (int b = 0; b < TWB; ++b) c[b] = NM > 1 ? acc[0][tm][y * TWB + b][v] + acc[1][tm][y * TWB + b][v] : acc[0][tm][y * TWB + b][v];
+                            if (ox + TWB <= OW) {
+                                if constexpr (LINES) __builtin_nontemporal_store(c, reinterpret_cast<cols*>(to));
+                                else *reinterpret_cast<cols*>(to) = c;
+                            } else {
+#pragma unroll
+                                for (int b = 0; b + 1 < TWB; ++b)
+                                    if (ox + b < OW) to[b] = c[b];
+                            }
                         }
                     }
-                }
+        }
     }
+};
+
+// (see Slim) Sixteen channels and four rows at a time, or one beside many taps, and fewer loads under way: 32 channels with 64 columns of two rows, or 16 with eight rows, are 128 or 64 registers of sums, with which 3 x 3 layers (169
+// in all) and larger filters do not fit beside ten waves.  The patch is read again for each.
+template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int BM, int TH, int TWB, int NIMG, bool LINES>
+struct SlimOf<ConvF32Few<CI, CO, H, W, KH, KW, S, P, BM, TH, TWB, NIMG, LINES>> {
+    using type = ConvF32Few<CI, CO, H, W, KH, KW, S, P, BM, TH, TWB, NIMG, LINES, true>;
 };
 
 }  // namespace bfuse

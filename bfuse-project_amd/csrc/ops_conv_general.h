@@ -44,7 +44,7 @@ namespace bfuse {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
-// WM_ = 0: this form.  WM_ = 1 or 2 (ops_conv_tile.h): large tiles that the waves of a workgroup share.
+// WM_ = 0: this form; -n: with at most n of a patch's loads under way (Slim).  WM_ = 1 or 2 (ops_conv_tile.h): large tiles that the waves of a workgroup share.
 template <int CI_, int CO_, int H_, int W_, int KH_, int KW_, int S_, int P_, int BM_, int PB_, int KS_, int NIMG_ = 1, int WM_ = 0>
 struct ConvF32Lds {
     static constexpr bool MATRIX_CORES = true;   // the inner loop is a stream of MFMAs (what the fusion chooser asks)
@@ -81,9 +81,9 @@ struct ConvF32Lds {
     // staged straight from the rows; those outside the image are stored as zeros, so that only the columns beside it need zeros of their own
     static constexpr bool BY_ROWS = VW == 4 || W < 4 || NIMG == 1;
     // loads under way at a time (rows of whole vectors beside filters of groups of 16: sixteen, with eight two of 33 that fit spill)
-    static constexpr int MOST = T > 40 && (CG == 4 || !BY_ROWS) ? loads_beside(4 * (CG == 16 ? T : (T + 3) / 4) * TM, NLD) : 16;
+    static constexpr int MOST = WM_ < 0 ? -WM_ : T > 40 && (CG == 4 || !BY_ROWS) ? loads_beside(4 * (CG == 16 ? T : (T + 3) / 4) * TM, NLD) : 16;
     static constexpr int NPAD = R * 2 * P * NQ;         // positions of padding
-    static_assert(WM_ == 0, "shared tiles have stages of four channels and one or two waves over the output channels");
+    static_assert(WM_ <= 0, "shared tiles have stages of four channels and one or two waves over the output channels");
     static_assert(CG == 16 ? CI % 16 == 0 : CI <= 4, "input channels: a multiple of 16, or at most 4");
     static_assert(CO % BM == 0 && BM % 16 == 0 && NGROUP % KS == 0, "channel tiling");
     static_assert(((KH - 1) * WP + KW - 1) * 16 + (NQ - 1) * PLANE + 16 < 65536, "tap offsets are 16-bit immediates");
@@ -410,6 +410,11 @@ struct NarrowOf<SwapOperands<Op>> {
 template <class Op>
 struct SlimOf<SwapOperands<Op>> {
     using type = SwapOperands<Slim<Op>>;
+};
+
+template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int BM, int PB, int KS, int NIMG>
+struct SlimOf<ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, KS, NIMG, 0>> {
+    using type = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, BM, PB, KS, NIMG, -4>;
 };
 
 }  // namespace bfuse

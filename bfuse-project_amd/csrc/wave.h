@@ -278,5 +278,9 @@ struct SlimOf {
 };
 template <class Op>
 using Slim = typename SlimOf<Op>::type;
+template <class Op, int BYTES>
+struct SlimOf<LdsReserve<Op, BYTES>> {
+    using type = LdsReserve<Slim<Op>, BYTES>;
+};
 
 }  // namespace bfuse

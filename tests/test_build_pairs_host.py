@@ -166,6 +166,15 @@ def test_patch_convolutions_fit_beside_ten_waves_in_their_slim_form(k1, tmp_path
     assert _compiled(k, src, tmp_path) == []
 
 
+@pytest.mark.parametrize("form,k2", [("bfuse", "gemm_bf16_512x4096x14336"), ("hfuse", "conv1x1s1p0_f32_1024x768x17x17_160"), ("hfuse", "conv3x3s2p0_f32_1024x192x17x17_320")])
+def test_rgb_layers_fit_beside_ten_waves_in_their_slim_form(form, k2, tmp_path):
+    """Their own form takes 169 registers of the 168 that are left; with the products that have no form of fewer waves the pair would not be built."""
+    k1 = "conv3x3s2p0_f32_1024x3x299x299_32"
+    k = {"k1": k1, "k2": k2, "form": form, "name": f"{k1}_{k2}_fused_{'bfuse_c256' if form == 'bfuse' else 'hfuse'}"}
+    src = build_pairs.source_text([k]).replace("Side0, ", "Slim<Side0>, ") + "static_assert(Slim<Side0>::GRID.size() == Side0::GRID.size() && sizeof(Slim<Side0>::Smem) == sizeof(Side0::Smem));\n"
+    assert _compiled(k, src, tmp_path) == []
+
+
 @pytest.mark.parametrize("i", range(4))
 def test_no_block_fused_pair_of_the_batch_suites_is_left_out_for_registers(i, tmp_path):
     """A side of at most 512 threads is compiled for 256 registers a lane, as many as a fused workgroup of two such sides has.  The

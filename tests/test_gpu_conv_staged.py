@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import bfuse_project_amd as bf
-from bfuse_project_amd.operation import fill_normal
+from bfuse_project_amd.operation import f32_to_bf16, fill_normal
 from oracle import oracle as orf
 from tests.test_gpu_conv_tile import _check
 
@@ -19,7 +19,8 @@ FORMS = [("a", 1, 2, "bias_relu_4096", "hfuse", ""), ("b", 1, 1, "bias_relu_4096
          ("t", 5, 0, "bias_relu_4096", "hfuse", ""), ("u", 5, 2, "conv3x3_f32_32x12x12_32", "hfuse", ""), ("v", 8, 0, "conv3x3_f32_32x12x12_32", "hfuse", ""),
          ("w", 4, 1, "bias_relu_4096", None, ""), ("x", 1, 17, "bias_relu_4096", None, ""), ("y", 1, 35, "bias_relu_4096", None, ""), ("z", 1, 18, "bias_relu_4096", None, ""),
          ("aa", 1, 67, "bias_relu_4096", None, ""), ("ba", 1, 2, "bias_relu_4096", None, ""), ("bb", 1, 2, "bias_relu_4096", None, ""), ("bc", 1, 1, "bias_relu_4096", None, ""),
-         ("bd", 2, 1, "bias_relu_4096", None, ""), ("be", 1, 1, "bias_relu_4096", None, ""), ("ca", 4, 6, "bias_relu_4096", None, ""), ("cb", 1, 0, "bias_relu_4096", None, "")]
+         ("bd", 2, 1, "bias_relu_4096", None, ""), ("be", 1, 1, "bias_relu_4096", None, ""), ("ca", 4, 6, "bias_relu_4096", None, ""), ("cb", 1, 0, "bias_relu_4096", None, ""),
+         ("da", 1, 0, "bias_relu_4096", None, ""), ("db", 1, 4, "bias_relu_4096", None, ""), ("dc", 3, 4, "bias_relu_4096", None, ""), ("dd", 1, 1, "bias_relu_4096", None, "")]
 
 
 @pytest.mark.parametrize("tag,s,p,partner,kind,suffix", FORMS)
@@ -55,6 +56,22 @@ def test_a_value_that_is_not_finite_is_in_its_own_windows_alone(tag, s, p):
     assert np.array_equal(np.isnan(y), np.isnan(want)) and np.array_equal(np.isposinf(y), np.isposinf(want)) and np.array_equal(np.isneginf(y), np.isneginf(want))
     ok = np.isfinite(want)
     assert ok.any() and np.linalg.norm(y[ok] - want[ok]) <= 1e-5 * np.linalg.norm(want[ok])
+
+
+@pytest.mark.parametrize("tag", ["da", "db", "dc", "dd"])
+def test_forms_of_fewer_registers_give_the_same_bits_beside_ten_waves(tag):
+    with bf.Operation(f"selftest_conv_staged_{tag}", "gemm_bf16_256x448x1792_p2") as op:
+        for side, k in enumerate(op.k):
+            x, w = (fill_normal(11 + 2 * side + i, int(np.prod(k.shapes[i])), 0, 1) for i in (0, 1))
+            op.upload(side, *((x, w) if side == 0 else (f32_to_bf16(x), f32_to_bf16(w))))
+        op.zero_outputs()
+        op.launch("serial")
+        want = [op.download(side).copy() for side in (0, 1)]
+        op.zero_outputs()
+        op.launch("bfuse", op.fused("bfuse", "_c4"))
+        for side in (0, 1):
+            got = op.download(side)
+            assert np.any(got.view(np.uint8)) and np.array_equal(got.view(np.uint8), want[side].view(np.uint8))
 
 
 @pytest.mark.parametrize("tag,s,p", [("huge_a", 4, 2), ("huge_b", 8, 1), ("huge_c", 4, 1)])
