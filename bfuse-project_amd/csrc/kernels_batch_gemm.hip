@@ -40,8 +40,8 @@ DENSE_SPLIT(1024, 14336, 4096, 2, 4, 1, 2, 128, kPix)
 // store at different times.  us on one card, fp32 matrix cores before and now: 1024 products 512 x 64 x 512 360 -> 303 (32-row waves 311-348), 512 x
 // 128 x 512 625 -> 465 (499), 256 x 64 x 256 98 -> 84 (94), 256 x 80 x 256 119 -> 107 (117), 1024 x 64 x 512 705 -> 609 (620), 256 x 256 x
 // 80 134 -> 95 (16-row waves; 32-row 99), 512 x 512 x 128 555 -> 416 (32-row, 128 x 128, lean; not lean 424, 16-row 446), 512 x 512 x 64 334 -> 268 (293), 1024 x
-// 512 x 64 607 -> 518 (573), 256 x 256 x 64 95.6 -> 83 (88).  Results of 256 MB and more since go past the caches in whole lines (GemmSplit, LINES_): 512 x 64 x 512 308 -> 270, 512 x 128 x 512
-// 468 -> 458, 1024 x 64 x 512 602 -> 579, 256 x 64 x 256 84 -> 70, 256 x 80 x 256 107 -> 86, the last two only while their operands stay in the last-level cache.  208 x 208 x 64 gains nothing (75.9 against 74); 208 x 64 x 208, x 80 x 208
+// 512 x 64 607 -> 518 (573), 256 x 256 x 64 95.6 -> 83 (88).  Results of more than 256 MB
+// since go past the caches in whole lines (GemmSplit, LINES): 512 x 64 x 512 308 -> 270, 512 x 128 x 512 468 -> 458, 1024 x 64 x 512 602 -> 579.  208 x 208 x 64 gains nothing (75.9 against 74); 208 x 64 x 208, x 80 x 208
 // and x 208 x 80 gain 1.1-1.4x on seven or thirteen waves but keep the one-wave forms, which any operator can take beside it.
 #define BGEMM_F32_SPLIT(B, M, K, N, ...)                                                                         \
     using Bgemm_##B##x##M##x##K##x##N = GemmSplit<M, K, 1, N, 1, B, __VA_ARGS__>;                                 \

@@ -351,6 +351,22 @@ PARTS_TEST(l, SwapOperands<PARTS_OF(80, 480, 12, 10, 3, 7, 1, 4, 1, 1, 112, kPix
 PARTS_TEST(r, SwapOperands<PARTS_OF(160, 64, 9, 9, 1, 5, 1, 10, 1, 1, 128, kPix, 1, 1, 0)>, DIMS4(5, 64, 9, 9), DIMS4(160, 64, 1, 1), DIMS4(5, 160, 9, 9))
 BFUSE_BFUSE_KERNEL(selftest_gemm_split_r_p, Narrow<GemmSpP_r>, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
 
+// Results a line at a time, past the caches, which large ones are (_w): two and six blocks of columns, 16-row blocks, waves over the columns, groups over K, images whose last
+// tile is cut, operands taken apart before.
+#define LINES_TEST(TAG, I, F, O, WRAP, ...)                                                                         \
+    using GemmSpL_##TAG = WRAP<GemmSplit<__VA_ARGS__, 0>>;                                                          \
+    using GemmSpW_##TAG = WRAP<GemmSplit<__VA_ARGS__, 1>>;                                                          \
+    BFUSE_KERNEL(selftest_gemm_lines_##TAG, GemmSpL_##TAG, (I), (F), (O))                                           \
+    BFUSE_KERNEL(selftest_gemm_lines_##TAG##_w, GemmSpW_##TAG, (I), (F), (O))
+template <class Op>
+using AsItIs = Op;
+LINES_TEST(a, DIMS4(3, 128, 72, 1), DIMS4(3, 192, 72, 1), DIMS4(3, 128, 192, 1), AsItIs, 128, 72, 1, 192, 1, 3, 2, 2, 1, 1, 96, kRows, 1, 1, 0, true, false)
+LINES_TEST(b, DIMS4(2, 64, 128, 1), DIMS4(2, 128, 128, 1), DIMS4(2, 64, 128, 1), AsItIs, 64, 128, 1, 128, 1, 2, 1, 2, 2, 2, 128, kRows, 1, 1, 0, false, false)
+LINES_TEST(c, DIMS4(5, 48, 8, 12), DIMS4(64, 48, 1, 1), DIMS4(5, 64, 8, 12), SwapOperands, 64, 48, 8, 12, 1, 5, 2, 2, 1, 1, 128, kPix, 1, 1, 0, false, false)
+LINES_TEST(d, DIMS4(3, 32, 8, 8), DIMS4(160, 32, 3, 3), DIMS4(3, 160, 8, 8), SwapOperands, 160, 288, 8, 8, 1, 3, 1, 10, 1, 1, 128, kPix, 3, 3, 1, false, true)
+BFUSE_BFUSE_KERNEL(selftest_gemm_lines_a_w, GemmSpW_a, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
+BFUSE_BFUSE_KERNEL(selftest_gemm_lines_d_w, Narrow<GemmSpW_d>, layernorm_8x256, LayerNormS, _c4, bfuse::kChunked, 4, 1)
+
 // The convolution from a patch taken apart once: pixels that run on into the next images and past the batch, rectangles past an image's
 // edges with whole and with broken quads of pixels, one to four groups of channels, units that a thread does twice, two waves over the columns.
 // <CI, CO, H, W, padding, images, 16-row blocks of a wave, waves over rows, over columns, pixels, width>

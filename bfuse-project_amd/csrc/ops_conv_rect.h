@@ -371,7 +371,7 @@ struct ConvTiling {
     static constexpr int FEW_MOST = FEW_EIGHT ? 8 : FEW_NM <= (S == 1 ? 176 : 160) ? 4 : FEW_NM <= 200 ? 3 : 1;
     static constexpr int few_rows(int th) { return th > FEW_MOST ? FEW_MOST : th; }
     static constexpr int FEW_TH = FEW_TWB == 4 ? 2 : few_rows(NIMG > 1 && T > 25 && few_bytes(8, 1) <= 12800 ? 8 : few_bytes(4, 1) <= 25600 ? 4 : few_bytes(2, 1) <= 25600 ? 2 : 1);
-    static constexpr bool FEW_LINES = FEW_TWB == 4 && OW % 16 == 0 && (long long)NIMG * CO * OHW * 4 >= (1LL << 28);
+    static constexpr bool FEW_LINES = FEW_TWB == 4 && OW % 16 == 0 && (long long)NIMG * CO * OHW * 4 > (1LL << 28);
     static constexpr int pick_bm()
     {
         if (CI < 16) return 16;

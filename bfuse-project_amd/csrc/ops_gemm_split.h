@@ -124,8 +124,9 @@ struct SplitParts {
 // M, K, H, W, S, NIMG, LAYOUT: as in GemmTile.  TM 16-row blocks of a wave, WR waves over the rows and WN over the BN columns, KG
 // groups of such waves over the stages.  LEAN: one set of A's parts, taken apart at the top of the stage, instead of the next one's
 // beside this one's: 12 TM registers less for a stage that begins without MFMAs, which other workgroups of the CU fill.  PREP: I is A's parts.
+// LINES_: whether results are written a line at a time and past the caches (-1: by their size).
 template <int M_, int K_, int H_, int W_, int S_, int NIMG_, int TM_, int WR_, int WN_, int KG_, int BN_, int LAYOUT_, int KH_ = 1, int KW_ = 1, int P_ = 0,
-          bool LEAN_ = (LAYOUT_ == kRows && K_ <= 256), bool PREP_ = false>
+          bool LEAN_ = (LAYOUT_ == kRows && K_ <= 256), bool PREP_ = false, int LINES_ = -1>
 struct GemmSplit {
     using Parts = SplitParts<M_, K_, 1, PREP_>;
     static constexpr int PARTS_OPERAND = PREP_ ? 0 : -1;
@@ -164,10 +165,13 @@ struct GemmSplit {
     static constexpr int RED_BYTES = (KG - 1) * BM * BN * 4;                     // partial sums of the groups
     // Results that are more than the last-level cache holds (256 MB) and lie in whole lines (two blocks of columns): every line is written at once and past the caches.
     // Otherwise a store is 64 bytes of sixteen rows, and the results take the place of everything else in the caches.  us, launched again and again / in turn with a layer of 900 MB: 1024 products
-    // 512 x 64 x 512 296 -> 256 / 295 -> 281, 1024 x 64 x 512 588 -> 565 / 587 -> 568, 512 x 128 x 512 453 -> 450 / 459 -> 451, 256 -> 256 channels on 56 x 56 2438 -> 2377 / 2436 -> 2374; 256 x 80 x 256 (268 MB) 105 -> 86 /
-    // 99.5 -> 100.2, 256 x 64 x 256 83 -> 68 / 76.7 -> 77.3: there it is the operands, 134 - 168 MB, that stay in the last-level cache.  Whole lines through the caches gain 0-1 %, 64 bytes past them lose up to 5 %
-    // (512 x 128 x 512).  Smaller results stay in that cache for what reads them (256 x 256 x 64, 67 MB, launched again and again would take 75 us for 81).
-    static constexpr bool LINES_ = TN % 2 == 0 && M % BM == 0 && (LAYOUT == kRows ? W % BN == 0 && W % 32 == 0 : OHW % 32 == 0) && (long long)NIMG * M * (LAYOUT == kRows ? W : OHW) * 4 >= (1LL << 28);
+    // 512 x 64 x 512 296 -> 256 / 295 -> 281, 1024 x 64 x 512 588 -> 565 / 587 -> 568, 512 x 128 x 512 453 -> 450 / 459 -> 451, 256 -> 256 channels on 56 x 56 2438 -> 2377 / 2436 -> 2374.  Not 256 MB themselves: 256 x 80 x 256
+    // 105 -> 86 / 99.5 -> 100.2, 256 x 64 x 256 83 -> 68 / 76.7 -> 77.3, where the gain is that operands of 134 - 168 MB stay in the last-level cache for the next launch over the same ones.
+    // Whole lines through the caches gain 0-1 %, 64 bytes past them lose up to 5 % (512 x 128 x 512).  Smaller results stay in that cache for what reads them
+    // (256 x 256 x 64, 67 MB, launched again and again would take 75 us for 81).
+    static constexpr bool IN_LINES = TN % 2 == 0 && M % BM == 0 && (LAYOUT == kRows ? W % BN == 0 && W % 32 == 0 : OHW % 32 == 0);
+    static constexpr bool LINES = IN_LINES && (LINES_ >= 0 ? LINES_ > 0 : (long long)NIMG * M * (LAYOUT == kRows ? W : OHW) * 4 > (1LL << 28));
+    static_assert(LINES_ <= 0 || LINES, "whole lines");
 
     struct Smem {
         __attribute__((aligned(16))) unsigned char t[NBUF * KG * BUF > RED_BYTES ? NBUF * KG * BUF : RED_BYTES];
@@ -503,8 +507,8 @@ struct GemmSplit {
     __device__ static __forceinline__ float swap_halves(float v) { return dpp_mov<0x128>(v); }      // row_ror:8
 
     // What follows the sums of a wave: the results that three parts do not give are done again, and all are stored.
-    // offset(c, outside): as offset_of, for column c of the tile; quad(c, img, p): as quad_at; QUADS: four columns are one image's and aligned; LINES: as LINES_.
-    template <bool QUADS = OHW % 4 == 0, bool LINES = LINES_, class Offset, class Quad>
+    // offset(c, outside): as offset_of, for column c of the tile; quad(c, img, p): as quad_at; QUADS: four columns are one image's and aligned; WHOLE: as LINES.
+    template <bool QUADS = OHW % 4 == 0, bool WHOLE = LINES, class Offset, class Quad>
     __device__ static __forceinline__ void finish(f32x4 (&acc)[TM][TN], bool again, const float* A, const float* B, float* __restrict__ C, int m0, int mt, long long n0, int nt, int n_lo,
                                                   int wr, int wn, int ei, int eq, Offset offset, Quad quad)
     {
@@ -615,7 +619,7 @@ struct GemmSplit {
 #pragma unroll
                     for (int b = 0; b < TN; ++b) acc[tm][b] = re[tm][b];
         }
-        if constexpr (LINES) {
+        if constexpr (WHOLE) {
             // Two blocks of columns and of eight rows at a time: lanes of rows 8 .. 15 have the second block's columns of the first rows and the other way round, so that
             // eight lanes write a line.
 #pragma unroll
@@ -678,10 +682,10 @@ struct GemmSplit {
 
 // (see Narrow) us, ten waves and five, with twice the rows of a wave: 768 -> 160 channels on 17 x 17 460 and 514, 192 -> 320 at
 // stride 2 385 and 436, 1280 -> 320 on 8 x 8 296 and 324, 2048 -> 320 459 and 500.  (Eight waves of 80 x 32: the 3 x 3 layer spills.)
-template <int M, int K, int H, int W, int S, int NIMG, int TM, int WR, int WN, int KG, int BN, int LAYOUT, int KH, int KW, int P, bool LEAN, bool PREP>
-struct NarrowOf<GemmSplit<M, K, H, W, S, NIMG, TM, WR, WN, KG, BN, LAYOUT, KH, KW, P, LEAN, PREP>> {
+template <int M, int K, int H, int W, int S, int NIMG, int TM, int WR, int WN, int KG, int BN, int LAYOUT, int KH, int KW, int P, bool LEAN, bool PREP, int LINES>
+struct NarrowOf<GemmSplit<M, K, H, W, S, NIMG, TM, WR, WN, KG, BN, LAYOUT, KH, KW, P, LEAN, PREP, LINES>> {
     static constexpr int HALVE = 64 * WR * WN * KG > 512 && WR % 2 == 0 ? 2 : 1;
-    using type = GemmSplit<M, K, H, W, S, NIMG, TM * HALVE, WR / HALVE, WN, KG, BN, LAYOUT, KH, KW, P, LEAN, PREP>;
+    using type = GemmSplit<M, K, H, W, S, NIMG, TM * HALVE, WR / HALVE, WN, KG, BN, LAYOUT, KH, KW, P, LEAN, PREP, LINES>;
 };
 
 }  // namespace bfuse

@@ -206,3 +206,10 @@ def test_images_that_no_buffer_holds_are_loaded_otherwise(tmp_path):
         static_assert(Conv3x3F32Lds<16, 16, 1048576, 32, 16, 2, 1>::Source::FAR && !Conv3x3F32Lds<16, 16, 1048574, 32, 16, 2, 1>::Source::FAR);
         static_assert(sizeof(ConvF32Rect<16, 16, 8192, 4096, 3, 3, 1, 1, 16, 4, 1, 1>::Source::Index) == 8);
     """, tmp_path)
+
+
+def test_results_past_the_caches_are_more_than_the_last_level_cache_holds(tmp_path):
+    _compiles("""
+        static_assert(!GemmSplit<256, 80, 1, 256, 1, 1024, 2, 4, 1, 1, 64, kRows>::LINES && GemmSplit<256, 80, 1, 256, 1, 1025, 2, 4, 1, 1, 64, kRows>::LINES);
+        static_assert(GemmSplit<512, 64, 1, 512, 1, 1024, 2, 4, 1, 1, 64, kRows>::LINES && !GemmSplit<208, 64, 1, 208, 1, 4096, 1, 13, 1, 1, 16, kRows>::IN_LINES);
+    """, tmp_path)

@@ -431,3 +431,22 @@ def test_a_patch_convolution_of_twice_the_waves_gives_the_same_bits(tag, value):
             got = op.run_fuse(op.fused("bfuse", "_c4"), a, b, *q)
             assert np.isfinite(want[0]).any()
             assert np.array_equal(got[0].view(np.uint32), want[0].view(np.uint32)) and np.array_equal(got[1].view(np.uint16), want[1].view(np.uint16))
+
+
+@pytest.mark.parametrize("tag", ["a", "b", "c", "d"])
+@pytest.mark.parametrize("value", [1.0, 2.0 ** -120 * 1.2345678, np.inf])
+@pytest.mark.parametrize("side", [0, 1])
+def test_results_in_whole_lines_are_the_same_bits(tag, value, side):
+    """... also those that are done again where three parts do not hold an operand, of an ordinary one, one tiny row or column among others and one infinity, alone and fused."""
+    name = f"selftest_gemm_lines_{tag}"
+    ops = _operands(name)
+    ops[side].reshape(ops[side].shape[0], -1)[-1, 5::7] *= np.float32(value)
+    want = _run(name, *ops)
+    assert np.any(want) and np.array_equal(_run(name + "_w", *ops).view(np.uint32), want.view(np.uint32))
+    if tag in "ad":
+        with bf.Operation(name + "_w", "layernorm_8x256") as op:
+            op.upload(0, *ops)
+            op.upload(1, *(fill_normal(21 + i, int(np.prod(op.k[1].shapes[i])), 0, 1) for i in (0, 1)))
+            op.zero_outputs()
+            op.launch("bfuse", op.fused("bfuse", "_c4"))
+            assert np.array_equal(op.download(0).view(np.uint32).ravel(), want.view(np.uint32).ravel())
