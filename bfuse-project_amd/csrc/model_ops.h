@@ -96,12 +96,13 @@ using Bgemm17 = GemmF32<1024, 64, 512, 16, 64, 4, kEpiNone, 2, 1, true, 1>;     
 // The other ResNet-18 layers (test-utils/examples/resnet-18.yaml) on the general convolution:
 // <CI, CO, H, W, KH, KW, stride, padding, output channels per workgroup, 16-pixel blocks, waves>
 // One image has 128 - 208 tiles of 16 x 16 results and a reduction of 576 - 4608 for each: staging and the chain of MFMAs
-// of a wave are what takes the time, so the 3x3 layers of 128 channels and more split it over eight waves: 17.1 -> 14.7 us on
-// 7x7 (sixteen waves 14.5, but fused with the LayerNorm 16.4 against 14.9), 10.0 -> 8.9 on 14x14, 11.4 -> 9.9 and 6.8 -> 6.5 at
-// stride 2; fused with the LayerNorm 1.05-1.3x.  The 1x1 layers gain 1.1-1.2x alone and lose 0.74-0.84x fused: four waves.
+// of a wave are what takes the time, so the 3x3 layers of 128 channels and more split it over eight waves.  us with eight: 512 channels on 7x7 8.6, 256 on
+// 14x14 5.5, 256 -> 512 and 128 -> 256 at stride 2 6.1 and 4.3.  (Against four waves, measured while filters came as the lanes want them and these took
+// 14.7, 8.9, 9.9 and 6.5: 1.16x, 1.12x, 1.15x and 1.05x, sixteen waves on 7x7 1.01x more, but 0.91x fused with the LayerNorm; the 1x1 layers gained 1.1-1.2x
+// alone and lost 0.74-0.84x fused: four waves.)
 using Conv0 = ConvF32Few<3, 64, 224, 224, 7, 7, 2, 3, 16, 4, 1>;          // 7x7 stride 2 on RGB: 4 x 16-pixel rectangles (13 x 37 patch instead of 9 x 230), 196 x 4 = 784 one-wave workgroups
 using Conv2 = SwapOperands<GemmF32<64, 3136, 64, 16, 64, 1>>;            // 1x1 stride 1 = Wt[64,64] . X[64,3136]: 4 x 49 = 196
-using Conv3 = ConvF32Lds<64, 128, 56, 56, 3, 3, 2, 1, 16, 2, 4>;          // 25 x 8 = 200 workgroups; 32 channels x 16 pixels 6.4 against 6.1 us, fused 10.8 against 8.0
+using Conv3 = ConvF32Lds<64, 128, 56, 56, 3, 3, 2, 1, 16, 2, 4>;          // 25 x 8 = 200 workgroups; 32 channels x 16 pixels 1.05x the time, fused 1.35x
 using Conv5 = ConvF32Lds<64, 128, 56, 56, 1, 1, 2, 0, 32, 1, 4>;
 using Conv6 = ConvF32Lds<128, 256, 28, 28, 3, 3, 2, 1, 16, 1, 8>;         // 13 x 16 = 208
 using Conv7 = ConvF32Lds<256, 256, 14, 14, 3, 3, 1, 1, 16, 1, 8>;

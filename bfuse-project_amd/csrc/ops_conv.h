@@ -134,7 +134,7 @@ struct Conv3x3F32Lds {
         tile_of(vblock, pt, ct);
         const int p0 = pt * TP, co0 = ct * BM;
         int y_lo = p0 / W;                             // first image row of the tile; staged row 0 is y_lo - 1
-        opaque_uniform(y_lo);
+        if constexpr (NPT == 1) opaque_uniform(y_lo);
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;   // wave-uniform: addresses built on it stay in scalar registers
         const int li = lane & 15, kq = lane >> 4;
         unsigned char* const tile = sm.t + wave * TILE_BYTES;
@@ -169,7 +169,7 @@ struct Conv3x3F32Lds {
             // border test would.
             const int cl = lane >> 2, c4 = lane & 3;
             const int first = y_lo == 0 ? CPR : 0, end = (H + 1 - y_lo < R ? H + 1 - y_lo : R) * CPR;   // chunks inside it
-            const auto xr = Source::open(opaque_pointer(X + (size_t)ci0 * HW));
+            const auto xr = Source::template open<(NCH % 4 != 0)>(X + (size_t)ci0 * HW);
             const typename Source::Index corner = (typename Source::Index)cl * HW + (y_lo - 1) * W + c4 * 4;
             f32x4 v[NLD];
 #pragma unroll

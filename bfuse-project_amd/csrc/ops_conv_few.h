@@ -14,7 +14,8 @@
 //   * a sum is two halves, added up at the end: as one it is off by 1.00 - 1.02 times what the sum over taps of all channels was (2-norm), as two by 0.75 times; 3 % of
 //     the time of 7 x 7, none elsewhere.
 //
-// us, before (ConvF32Rect) and now: 7 x 7 on 1024 RGB images of 224 x 224 2688 -> 2154, on one 7.26 -> 5.72, with the LayerNorm 10.5 -> 8.2, 3 x 3 at stride 2 on 1024 of 299 x 299 1338 -> 985.
+// us, with the channels as k, every float staged by itself and filters as the lanes want them (ConvF32Rect as it was), and now: 7 x 7 on 1024 RGB images of 224 x 224 3371 -> 2154, on one 8.75 -> 5.72, with the LayerNorm
+// 12.2 -> 8.2, 3 x 3 at stride 2 on 1024 of 299 x 299 1484 -> 985.  (With filters through LDS and 32 channels a wave alone 2688, 7.26, 10.5 and 1338.)
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -104,7 +105,7 @@ struct ConvF32Few {
 
         // Stage the patch, [channel][row][PC floats]: the lanes take its vectors in turn, which follow each other in LDS.  A vector of a row outside the image is
         // read past the buffer's end; floats beside the image are made zeros (PatchColumns).
-        const auto xr = Source::open(X);
+        const auto xr = Source::template open<false>(X);
         const bool inside = ix0 >= 0 && ix0 + PC <= W;          // no vector reaches beside the image
         constexpr int JB = Units::JB;
         if constexpr (!TURNED) filters.load(Wt, co0, lane);
@@ -205,8 +206,8 @@ struct ConvF32Few {
     }
 };
 
-// (see Slim) Sixteen channels and four rows at a time, or one beside many taps, and fewer loads under way: 32 channels with 64 columns of two rows, or 16 with eight rows, are 128 or 64 registers of sums, with which 3 x 3 layers (169
-// in all) and larger filters do not fit beside ten waves.  The patch is read again for each.
+// (see Slim) Sixteen channels and four rows at a time, or one beside many taps, and fewer loads under way: 32 channels with 64 columns of two rows, or 16 with
+// eight rows, are 128 or 64 registers of sums, with which 3 x 3 layers (169 in all) and larger filters do not fit beside ten waves.  The patch is read again for each.
 template <int CI, int CO, int H, int W, int KH, int KW, int S, int P, int BM, int TH, int TWB, int NIMG, bool LINES>
 struct SlimOf<ConvF32Few<CI, CO, H, W, KH, KW, S, P, BM, TH, TWB, NIMG, LINES>> {
     using type = ConvF32Few<CI, CO, H, W, KH, KW, S, P, BM, TH, TWB, NIMG, LINES, true>;

@@ -154,7 +154,7 @@ struct ConvF32Lds {
         const int p0 = pt * TP, co0 = ct * BM;
         const int oy_lo = p0 / OW;                     // first output row of the tile
         int iy_lo = oy_lo * S - P;                     // image row of staged row 0
-        if constexpr (TURNED && BY_ROWS) opaque_uniform(iy_lo);
+        if constexpr (TURNED && BY_ROWS && NPT == 1) opaque_uniform(iy_lo);
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
         const int li = lane & 15, kq = lane >> 4;
         unsigned char* const tile = sm.t + wave * TILE_BYTES;
@@ -240,8 +240,8 @@ struct ConvF32Lds {
             // in batches of JB loads, so that a large patch (7x7 filters on 224-wide rows) does not need a
             // register per element
             // Rows that are not whole 16-byte chunks: a single image (latency regime) takes them with 8- or 4-byte
-            // loads straight from their rows (9.9 / 11.4 / 17.0 us against 12.2 / 14.6 / 19.2 for the 14x14 and 7x7
-            // layers of ResNet-18); a batch of images (throughput) from aligned 16-byte loads, a quarter of the load
+            // loads straight from their rows (1.23x, 1.28x and 1.13x for the 14x14 and 7x7 layers of ResNet-18 when they
+            // took 9.9, 11.4 and 17.0 us; with filters through LDS they take 5.5, 6.1 and 8.6); a batch of images (throughput) from aligned 16-byte loads, a quarter of the load
             // instructions (1024 images: 20-45 % faster on 35-, 73-, 147- and 299-wide images, 8-11 % on 14 and 7).
             if constexpr (BY_ROWS) {
                 constexpr int JB = NLD < MOST ? NLD : MOST;
@@ -251,7 +251,7 @@ struct ConvF32Lds {
                 // The patch's rows follow each other in memory; units of rows outside the image, and of channels that the layer
                 // does not have, are read past the buffer's end, which gives zeros.
                 const int first = iy_lo < 0 ? -iy_lo * (W / VW) : 0, end = (H - iy_lo < R ? H - iy_lo : R) * (W / VW);
-                const auto xr = Source::open(opaque_pointer(X + (size_t)ci0 * HW));
+                const auto xr = Source::template open<(NU % LPC != 0)>(X + (size_t)ci0 * HW);
                 const typename Source::Index corner = (typename Source::Index)cl * HW + iy_lo * W + cu * VW;
                 if constexpr (NBATCH > 1) take_filters(std::integral_constant<int, 0>{});
 #pragma unroll UNROLL

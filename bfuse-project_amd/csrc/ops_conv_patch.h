@@ -5,6 +5,8 @@
 
 #include <type_traits>
 
+#include "wave.h"
+
 namespace bfuse {
 
 // Whether the FLOATS floats that a patch's loads can reach are too many for a buffer: the place outside the image, byte 2^31 - 1, has to lie past its end.
@@ -14,8 +16,8 @@ inline constexpr bool kFarPatch = FLOATS * 4 > 0x7fffffffLL;
 
 // The patch's loads: a buffer with its own range check, or, for images of 2 GiB and more (of the channels of a group), a test of every float.
 // Where a wait for the filters counts the loads behind them (FilterRows::take), all of these have to be made and to stay ahead of it, whatever the compiler
-// knows of them.  So the pointer is opaque there (a memory clobber orders nothing against a `__restrict__` argument: a load that is used under a condition only was moved
-// behind the wait, into it), and so is the first row (of two loads known to lie outside the image one was made).
+// knows of them.  So where the last one is used by some lanes only the pointer is opaque (a memory clobber orders nothing against a `__restrict__` argument: that load was
+// moved behind the wait, into the condition), and where one tile has all rows so is the first (of two loads known to lie outside the image one was made).
 template <long long FLOATS>
 struct PatchSource {
     static constexpr bool FAR = kFarPatch<FLOATS>;
@@ -25,8 +27,11 @@ struct PatchSource {
     template <int LOADS>
     using Behind = std::integral_constant<int, FAR ? 0 : LOADS>;
 
+    // HIDDEN: the pointer is opaque.
+    template <bool HIDDEN>
     __device__ static __forceinline__ auto open(const float* x)
     {
+        if constexpr (HIDDEN) x = opaque_pointer(x);
         if constexpr (FAR) return x;
         else return __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, (int)(FLOATS * 4), 0x00020000);
     }

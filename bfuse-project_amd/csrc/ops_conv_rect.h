@@ -193,7 +193,7 @@ struct ConvF32Rect {
             // which positions a lane stages does not change from one channel group to the next, and the compiler would
             // work out every address ahead of the loop and keep them all in registers: hidden from it
             asm volatile("" : "+v"(cu));
-            const auto xr = Source::open(opaque_pointer(X + (size_t)ci0 * HW));
+            const auto xr = Source::template open<(NU % LPC != 0)>(X + (size_t)ci0 * HW);
             const typename Source::Index corner = (typename Source::Index)cl * HW + iy0 * W;
             const bool inside = ix0 >= 0 && ix0 + PC <= W;          // no vector reaches beside the image
             unsigned char* const plane = tile + (cl / 4) * PLANE + (cl % 4) * 4;
@@ -352,19 +352,21 @@ struct ConvTiling {
     static constexpr bool RECT = T > 1 && (OW >= 64 || ((OW >= 44 || S > 1) && 6 * OW >= 5 * ((OW + 15) / 16 * 16)));
     static constexpr int patch_bytes(int th) { return ((th - 1) * S + KH) * (15 * S + KW) * 64; }
     static constexpr int TH = patch_bytes(4) <= 12800 ? 4 : patch_bytes(2) <= 12800 ? 2 : 1;
-    // Images of at most four channels (ConvF32Few).  A batch writes its results 64 columns wide where three quarters of these are the image's, of filters of up to 25 taps (ConvF32Few
-    // has why), on two rows; else 16 columns and eight rows of larger filters, four of smaller ones.  32 output channels a wave for up to nine taps, 16 for more.  us, 256 images, 32 channels x 2 rows x 64 columns / 16 x 2
-    // x 64 / 32 x 4 x 16: 3 x 3 on 299 at stride 2 (1024) 1065 / 1098 / 1338, on 112 181 / - / 340, 5 x 5 on 149 384 / - / 371, on 299 at stride 2 779 / 690 / 763, of one channel on 112 170 / - / 244; on 150 at stride 2, 75 of 128
-    // columns, 264 / - / 229.  7 x 7 on 224 (1024), 16 channels x 8 / 7 / 4 / 12 rows and 32 x 8 / 6 / 4: 2154 / 2154 / 2206 / 2301, 2289 / 2264 / 2509.  One image, 16 x 4 / 16 x 2 / 32 x 2 / 32 x 4: 5.7 / 5.9 / 5.9 / 8.0.
+    // Images of at most four channels (ConvF32Few).  A batch writes its results 64 columns wide where three quarters of these are the image's, of filters of up to
+    // 25 taps (ConvF32Few has why), on two rows; else 16 columns and eight rows of larger filters, four of smaller ones.  32 output channels a wave for up to nine
+    // taps, 16 for more.  us, 256 images, 32 channels x 2 rows x 64 columns / 16 x 2 x 64 / 32 x 4 x 16: 3 x 3 on 299 at stride 2 (1024) 1065 / 1098 / 1338, on 112
+    // 181 / - / 340, 5 x 5 on 149 384 / - / 371, on 299 at stride 2 779 / 690 / 763, of one channel on 112 170 / - / 244; on 150 at stride 2, 75 of 128 columns,
+    // 264 / - / 229.  7 x 7 on 224 (1024), 16 channels x 8 / 7 / 4 / 12 rows and 32 x 8 / 6 / 4: 2154 / 2154 / 2206 / 2301, 2289 / 2264 / 2509.  One image,
+    // 16 x 4 / 16 x 2 / 32 x 2 / 32 x 4: 5.7 / 5.9 / 5.9 / 8.0.
     static constexpr bool FEW = RECT && CI <= 4;
     static constexpr int FEW_BM = NIMG > 1 && CO % 32 == 0 && T <= 9 ? 32 : 16;
     static constexpr int few_bytes(int th, int twb) { return CI * ((th - 1) * S + KH) * ((16 * twb - 1) * S + KW) * 4; }
     static constexpr int FEW_TWB = NIMG > 1 && T <= 25 && 4 * OW >= 3 * ((OW + 63) / 64 * 64) && few_bytes(2, 4) <= 16384 ? 4 : 1;
-    // Filters of many taps leave registers for fewer rows.  Eight: up to 64 registers of filters, and not where the rows of a window are many and one after the other for some lane groups
-    // only (13 x 13 and 13 x 11 of one channel, 11 x 11 and 9 x 14 of two spill), or wide at stride 2, where two phases of a row are kept (16 x 13 of one channel).  Four: up to 160 at a stride, 176 without.
-    // us before (four rows of ConvF32Rect) and now, 64 images of four channels, 96 wide,
-    // to 32: 12 x 12 221 -> 212, 13 x 13 204 -> 204, 9 x 9 108 -> 103, 14 x 14 289 -> 287; of two, 12 x 12 293 -> 135, of three 337 -> 154; 11 x 11 at stride 4 on 224, three channels to 64, 426 -> 118;
-    // of one channel, 12 x 12 with eight rows 251 -> 71 (four 76), 10 x 10 of two 204 -> 85 (95).
+    // Filters of many taps leave registers for fewer rows.  Eight: up to 64 registers of filters, and not where the rows of a window are many and one after the
+    // other for some lane groups only (13 x 13 and 13 x 11 of one channel, 11 x 11 and 9 x 14 of two spill), or wide at stride 2, where two phases of a row are
+    // kept (16 x 13 of one channel).  Four: up to 160 at a stride, 176 without.  us, four rows of ConvF32Rect as it was and now, 64 images 96 wide of four channels to 32:
+    // 12 x 12 222 -> 212, 13 x 13 205 -> 204, 14 x 14 290 -> 288, 13 x 13 at stride 2 73 -> 62; of three 12 x 12 338 -> 154; of two 10 x 10 203 -> 85 (with four rows 95); of one
+    // 12 x 12 250 -> 72 (76), 10 x 10 167 -> 54, 9 x 9 125 -> 39; on 224 11 x 11 at stride 4 of three to 64 427 -> 118, 12 x 12 at stride 2 of four 524 -> 483.
     using FewFilters = FilterFloats<(CI <= 4 ? CI : 4), KH, KW, 1>;
     static constexpr int FEW_NM = FewFilters::NM;
     static constexpr bool FEW_EIGHT = FEW_NM <= 64 && ((KH <= 10 && KW <= 12) || FewFilters::RPL <= 2 || KH % FewFilters::RPL == 0) && !(S == 2 && KW > 12);
@@ -467,7 +469,8 @@ struct ConvTiling {
     // Filters larger than 1 x 1: as a product on the bf16 matrix cores whose second operand is gathered from the images (GemmSplit),
     // on at least two rounds of tiles over the CUs.  The tile is the largest of 256 x 128 (eight waves), 128 x 128, 192 x 64 (four
     // waves, two workgroups a CU), 160 x 128 (ten waves of 16 rows), 96 x 64 (two waves) and 64 x 128 (four of 16 rows) whose rows
-    // divide the channels.  (Those at stride 1 have since gone on to the patch above, except channels that are no groups of 32.)  Batch 1024, us, shared tiles before (all on one card; others hold 0.93-1.00 of the clock): 256 -> 256 on 14 x 14 1712 -> 1033 (128 x 128: 1.09x that), 512 on 7 x 7
+    // divide the channels.  (Those at stride 1 have since gone on to the patch above, except channels that are no groups of 32.)  Batch 1024, us, shared tiles before
+    // (all on one card; others hold 0.93-1.00 of the clock): 256 -> 256 on 14 x 14 1712 -> 1033 (128 x 128: 1.09x that), 512 on 7 x 7
     // 1720 -> 1136, 128 on 28 x 28 1692 -> 1122, 448 -> 384 on 8 x 8 1381 -> 882 (192 x 64: 1.08x), 288 -> 384 at stride 2 4153 -> 2838
     // (192 x 128 and x 64: 1.10x), 80 -> 192 on 73 x 73 10209 -> 7393, 192 -> 320 at stride 2 521 -> 378 (128 x 128 on 2.5 tiles: 433; five
     // waves of 32 rows twice 477).  Few channels
@@ -481,8 +484,8 @@ struct ConvTiling {
     static constexpr int ROUNDS8 = (int)(((long long)((OHW + 3) / 4 * 4) * NIMG + 127) / 128 * (CO / 256) + 255) / 256, ROUNDS7 = (int)(((long long)((OHW + 3) / 4 * 4) * NIMG + 111) / 112 * (CO / 256) + 255) / 256;
     static constexpr int PB256 = 112 * ROUNDS7 < 0.97 * 128 * ROUNDS8 ? 7 : 8;
     using split = ConvF32Lds<CI, CO, H, W, KH, KW, S, P, SBM, SBM == 256 ? PB256 : SBM == 192 || SBM == 96 ? 4 : 8, SBM == 256 ? 8 : SBM == 160 ? 10 : SBM == 96 ? 2 : 4, NIMG, kSplitForm>;
-    // Filters of 31 and more taps are left to the per-wave forms: as products 7 x 7 on RGB took 2363 us instead of 3367, but a window with one element that is not
-    // zero came out up to 2.4 u off instead of 1, and one wave without barriers can be thread-fused with any operator.
+    // Filters of 31 and more taps are left to the per-wave forms: 7 x 7 on RGB takes 2154 us there and took 2363 as a product, a window with one element that is
+    // not zero came out up to 2.4 u off instead of 1 as a product, and one wave without barriers can be thread-fused with any operator.
     static constexpr bool is_split()
     {
         // (the table of taps is made at compile time)

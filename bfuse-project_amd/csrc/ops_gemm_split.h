@@ -163,12 +163,13 @@ struct GemmSplit {
     static constexpr bool LOOP_BARRIERS = true;
     static constexpr int MIN_BARRIERS = NIT;
     static constexpr int RED_BYTES = (KG - 1) * BM * BN * 4;                     // partial sums of the groups
-    // Results that are more than the last-level cache holds (256 MB) and lie in whole lines (two blocks of columns): every line is written at once and past the caches.
-    // Otherwise a store is 64 bytes of sixteen rows, and the results take the place of everything else in the caches.  us, launched again and again / in turn with a layer of 900 MB: 1024 products
-    // 512 x 64 x 512 296 -> 256 / 295 -> 281, 1024 x 64 x 512 588 -> 565 / 587 -> 568, 512 x 128 x 512 453 -> 450 / 459 -> 451, 256 -> 256 channels on 56 x 56 2438 -> 2377 / 2436 -> 2374.  Not 256 MB themselves: 256 x 80 x 256
-    // 105 -> 86 / 99.5 -> 100.2, 256 x 64 x 256 83 -> 68 / 76.7 -> 77.3, where the gain is that operands of 134 - 168 MB stay in the last-level cache for the next launch over the same ones.
-    // Whole lines through the caches gain 0-1 %, 64 bytes past them lose up to 5 % (512 x 128 x 512).  Smaller results stay in that cache for what reads them
-    // (256 x 256 x 64, 67 MB, launched again and again would take 75 us for 81).
+    // Results that are more than the last-level cache holds (256 MB) and lie in whole lines (two blocks of columns): every line is written at once and past the
+    // caches.  Otherwise a store is 64 bytes of sixteen rows, and the results take the place of everything else in the caches.  us, launched again and again / in turn
+    // with a layer of 900 MB: 1024 products 512 x 64 x 512 296 -> 256 / 295 -> 281, 1024 x 64 x 512 588 -> 565 / 587 -> 568, 512 x 128 x 512 453 -> 450 / 459 -> 451,
+    // 256 -> 256 channels on 56 x 56 2438 -> 2377 / 2436 -> 2374.  Not 256 MB themselves: 256 x 80 x 256 105 -> 86 / 99.5 -> 100.2, 256 x 64 x 256 83 -> 68 / 76.7 -> 77.3,
+    // where the gain is that operands of 134 - 168 MB stay in the last-level cache for the next launch over the same ones.  Whole lines through the caches gain 0-1 %,
+    // 64 bytes past them lose up to 5 % (512 x 128 x 512).  Smaller results stay in that cache for what reads them (256 x 256 x 64, 67 MB, launched again and again
+    // would take 75 us for 81).
     static constexpr bool IN_LINES = TN % 2 == 0 && M % BM == 0 && (LAYOUT == kRows ? W % BN == 0 && W % 32 == 0 : OHW % 32 == 0);
     static constexpr bool LINES = IN_LINES && (LINES_ >= 0 ? LINES_ > 0 : (long long)NIMG * M * (LAYOUT == kRows ? W : OHW) * 4 > (1LL << 28));
     static_assert(LINES_ <= 0 || LINES, "whole lines");
